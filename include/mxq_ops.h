@@ -60,7 +60,13 @@ int mxq_node_infer_type(void* node, int num_in, int* in_type, int num_out, int* 
 /* bytes of ResourceRequest::kTempSpace the node will ask for (0 if none) */
 int mxq_node_temp_bytes(void* node, int num_in, const mxq_blob* in, int num_out,
                         const mxq_blob* out, size_t* bytes);
-/* runs FCompute<gpu> or FCreateOpState + FStatefulCompute<gpu> on `stream` */
+/* The three calls above for complete inputs in one: shapes and types of the outputs (at most
+ * max_out; `data` is left alone, ndim -1 says that a shape stays unknown) and the temp-space
+ * bytes.  `in` needs shapes and types only. */
+int mxq_node_describe(void* node, int num_in, const mxq_blob* in, int max_out, mxq_blob* out,
+                      int* num_out, size_t* temp_bytes);
+/* runs FCompute<gpu> or FCreateOpState + FStatefulCompute<gpu> on `stream`; one node may be
+ * run from several threads */
 int mxq_node_forward(void* node, void* stream, int dev_id, int num_in, const mxq_blob* in,
                      int num_out, const mxq_blob* out, void* temp_space, size_t temp_bytes);
 

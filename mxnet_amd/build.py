@@ -102,7 +102,34 @@ def build_ops(verbose=False):
     return OPS_LIB
 
 
+FRONTEND_LIB = os.path.join(HERE, "_frontend.so")
+FRONTEND_SOURCES = ["mxq_frontend.cc"]
+
+
+def build_frontend(verbose=False):
+    """_frontend.so: the Python package's call path as an extension module over torch's C++
+    tensors (allocation, current stream) and the two libraries above."""
+    import sysconfig
+
+    from torch.utils import cpp_extension
+    cxx = os.environ.get("CXX", "g++")
+    cmd = [cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-ffp-contract=off", "-Wall",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-o", FRONTEND_LIB]
+    cmd += [os.path.join(CSRC, "host", s) for s in FRONTEND_SOURCES]
+    cmd += ["-isystem" + d for d in cpp_extension.include_paths(device_type="cuda")]
+    cmd += ["-I" + sysconfig.get_paths()["include"], "-L" + HERE, "-lmxq_ops", "-lmxq_hip",
+            "-Wl,-rpath,$ORIGIN"]
+    for d in cpp_extension.library_paths(device_type="cuda"):
+        cmd += ["-L" + d]
+    cmd += ["-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    subprocess.check_call(cmd)
+    return FRONTEND_LIB
+
+
 if __name__ == "__main__":
     print(build(verbose="-v" in sys.argv))
     print(build_ops(verbose="-v" in sys.argv))
+    print(build_frontend(verbose="-v" in sys.argv))
     print(build_probe(verbose="-v" in sys.argv))

@@ -5,7 +5,7 @@ import ctypes
 
 import torch
 
-from . import _lib
+from . import _frontend, _lib
 from ._lib import INT8, UINT8, check, lib
 
 _TYPE_CODE = {torch.int8: INT8, torch.uint8: UINT8}
@@ -96,6 +96,9 @@ def quantized_fc(data, weight, bias, min_data, max_data, min_weight, max_weight,
     """data int8 [M,K], weight int8 [N,K], bias int8 [N] or None.
     Returns dict(out32, omin, omax[, out8, rmin, rmax]).  `force` = (cfg, splits,
     stream_groups) goes through the test-only entry point that pins the kernel variant."""
+    if force is None:
+        return _frontend.quantized_fc(data, weight, bias, min_data, max_data, min_weight,
+                                      max_weight, min_bias, max_bias, want_int32, calib, relu)
     M, K = data.shape
     N, K2 = weight.shape
     assert K == K2
@@ -112,15 +115,10 @@ def quantized_fc(data, weight, bias, min_data, max_data, min_weight, max_weight,
             _ptr(max_data), _ptr(min_weight), _ptr(max_weight), _ptr(min_bias), _ptr(max_bias),
             _ptr(out32), _ptr(res["omin"]), _ptr(res["omax"]), _ptr(out8), _ptr(rmin),
             _ptr(rmax), int(relu), lo, hi]
-    if force is None:
-        wsb = lib.mxq_quantized_fc_workspace(M, N, K, int(not want_int32))
-        ws = _workspace(wsb, dev) if wsb else None
-        check(lib.mxq_quantized_fc(*args, _ptr(ws), wsb))
-    else:
-        cfg, splits, groups = force
-        wsb = _SPLIT_WS_BYTES if splits > 1 else 0
-        ws = _workspace(wsb, dev) if wsb else None
-        check(lib.mxq_test_quantized_fc(*args, _ptr(ws), wsb, cfg, splits, groups))
+    cfg, splits, groups = force
+    wsb = _SPLIT_WS_BYTES if splits > 1 else 0
+    ws = _workspace(wsb, dev) if wsb else None
+    check(lib.mxq_test_quantized_fc(*args, _ptr(ws), wsb, cfg, splits, groups))
     res.update(out32=out32, out8=out8, rmin=rmin, rmax=rmax)
     return res
 
@@ -187,6 +185,10 @@ def quantized_conv_nhwc(data, weight, bias, min_data, max_data, min_weight, max_
                         want_int32=True, calib=None, relu=False, force=None):
     """data int8 [N,H,W,C], weight int8 [O,KH,KW,C] -> out [N,OH,OW,O].  `force` = (cfg,
     splits) goes through the test-only entry point that pins the kernel variant."""
+    if force is None:
+        return _frontend.quantized_conv_nhwc(data, weight, bias, min_data, max_data, min_weight,
+                                             max_weight, min_bias, max_bias, stride, pad, dilate,
+                                             want_int32, calib, relu)
     N, H, W, C = data.shape
     O, KH, KW, C2 = weight.shape
     assert C == C2
@@ -206,15 +208,10 @@ def quantized_conv_nhwc(data, weight, bias, min_data, max_data, min_weight, max_
         _ptr(min_data), _ptr(max_data), _ptr(min_weight), _ptr(max_weight), _ptr(min_bias),
         _ptr(max_bias), _ptr(out32), _ptr(res["omin"]), _ptr(res["omax"]), _ptr(out8),
         _ptr(rmin), _ptr(rmax), int(relu), lo, hi]
-    if force is None:
-        wsb = lib.mxq_quantized_conv_workspace(*geo, int(not want_int32))
-        ws = _workspace(wsb, dev) if wsb else None
-        check(lib.mxq_quantized_conv_nhwc(*args, _ptr(ws), wsb))
-    else:
-        cfg, splits = force
-        wsb = _SPLIT_WS_BYTES if splits > 1 else 0
-        ws = _workspace(wsb, dev) if wsb else None
-        check(lib.mxq_test_quantized_conv_nhwc(*args, _ptr(ws), wsb, cfg, splits))
+    cfg, splits = force
+    wsb = _SPLIT_WS_BYTES if splits > 1 else 0
+    ws = _workspace(wsb, dev) if wsb else None
+    check(lib.mxq_test_quantized_conv_nhwc(*args, _ptr(ws), wsb, cfg, splits))
     res.update(out32=out32, out8=out8, rmin=rmin, rmax=rmax)
     return res
 

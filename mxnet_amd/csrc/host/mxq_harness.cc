@@ -3,6 +3,8 @@
 // (src/imperative/imperative.cc:51-139, imperative_utils.h:653-712), reduced to
 // parse -> infer -> build TBlobs / OpContext -> call the registered gpu function.
 #include <cstring>
+#include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -21,11 +23,37 @@ namespace {
 
 thread_local std::string tl_error;
 
+// The operator's registered functions are looked up once, when the node is made: the
+// registry is complete then and never changes, and a lookup by attribute name costs a few
+// hundred nanoseconds, more than the whole unpacking of a small call.
 struct Node {
   nnvm::NodeAttrs attrs;
+  std::once_flag state_once;  // a node may be run by several threads
   mxnet::OpStatePtr state;
   std::string in_names, out_names, grad_names;
+  const mxnet::FInferShape* infer_shape = nullptr;
+  const nnvm::FInferType* infer_type = nullptr;
+  const mxnet::FCompute* compute = nullptr;
+  const mxnet::FCreateOpState* create_state = nullptr;
+  const mxnet::FStatefulCompute* stateful = nullptr;
+  std::vector<mxnet::ResourceRequest> resources;
 };
+
+template <typename F>
+const F* find_attr(const char* key, const nnvm::Op* op) {
+  const auto map = nnvm::Op::GetAttr<F>(key);
+  return map.count(op) ? &map[op] : nullptr;
+}
+
+void infer_shapes(const Node* n, mxnet::ShapeVector* in, mxnet::ShapeVector* out) {
+  if (n->infer_shape == nullptr) throw dmlc::Error("op has no FInferShape");
+  (*n->infer_shape)(n->attrs, in, out);
+}
+
+void infer_types(const Node* n, std::vector<int>* in, std::vector<int>* out) {
+  if (n->infer_type == nullptr) throw dmlc::Error("op has no FInferType");
+  (*n->infer_type)(n->attrs, in, out);
+}
 
 #define OPS_API_BEGIN() try {
 #define OPS_API_END()                 \
@@ -94,6 +122,13 @@ int mxq_node_create(const char* op, const char* node_name, int num_attrs, const 
   if (in_names.count(n->attrs.op)) n->in_names = join(in_names[n->attrs.op](n->attrs));
   auto out_names = nnvm::Op::GetAttr<nnvm::FListOutputNames>("FListOutputNames");
   if (out_names.count(n->attrs.op)) n->out_names = join(out_names[n->attrs.op](n->attrs));
+  n->infer_shape = find_attr<mxnet::FInferShape>("FInferShape", n->attrs.op);
+  n->infer_type = find_attr<nnvm::FInferType>("FInferType", n->attrs.op);
+  n->compute = find_attr<mxnet::FCompute>("FCompute<gpu>", n->attrs.op);
+  n->create_state = find_attr<mxnet::FCreateOpState>("FCreateOpState", n->attrs.op);
+  n->stateful = find_attr<mxnet::FStatefulCompute>("FStatefulCompute<gpu>", n->attrs.op);
+  if (const auto* request = find_attr<mxnet::FResourceRequest>("FResourceRequest", n->attrs.op))
+    n->resources = (*request)(n->attrs);
   *out_node = n.release();
   OPS_API_END();
 }
@@ -152,9 +187,7 @@ int mxq_node_infer_shape(void* node, int num_in, int* in_ndim, int64_t* in_shape
   mxnet::ShapeVector in(num_in), out(num_out);
   for (int i = 0; i < num_in; ++i) in[i] = to_shape(in_ndim[i], in_shape + i * MXQ_MAX_NDIM);
   for (int i = 0; i < num_out; ++i) out[i] = to_shape(out_ndim[i], out_shape + i * MXQ_MAX_NDIM);
-  auto fmap = nnvm::Op::GetAttr<mxnet::FInferShape>("FInferShape");
-  if (!fmap.count(n->attrs.op)) throw dmlc::Error("op has no FInferShape");
-  fmap[n->attrs.op](n->attrs, &in, &out);
+  infer_shapes(n, &in, &out);
   auto write = [](const mxnet::TShape& s, int* nd, int64_t* dims) {
     *nd = s.ndim();
     if (s.ndim() > MXQ_MAX_NDIM) throw dmlc::Error("too many dimensions");
@@ -170,9 +203,7 @@ int mxq_node_infer_type(void* node, int num_in, int* in_type, int num_out, int* 
   OPS_API_BEGIN();
   Node* n = static_cast<Node*>(node);
   std::vector<int> in(in_type, in_type + num_in), out(out_type, out_type + num_out);
-  auto fmap = nnvm::Op::GetAttr<nnvm::FInferType>("FInferType");
-  if (!fmap.count(n->attrs.op)) throw dmlc::Error("op has no FInferType");
-  fmap[n->attrs.op](n->attrs, &in, &out);
+  infer_types(n, &in, &out);
   std::copy(in.begin(), in.end(), in_type);
   std::copy(out.begin(), out.end(), out_type);
   OPS_API_END();
@@ -183,12 +214,37 @@ int mxq_node_temp_bytes(void* node, int num_in, const mxq_blob* in, int num_out,
   OPS_API_BEGIN();
   Node* n = static_cast<Node*>(node);
   *bytes = 0;
-  auto fres = nnvm::Op::GetAttr<mxnet::FResourceRequest>("FResourceRequest");
-  if (!fres.count(n->attrs.op) || fres[n->attrs.op](n->attrs).empty()) return 0;
+  if (n->resources.empty()) return 0;
   mxnet::ShapeVector si(num_in), so(num_out);
   for (int i = 0; i < num_in; ++i) si[i] = to_shape(in[i].ndim, in[i].shape);
   for (int i = 0; i < num_out; ++i) so[i] = to_shape(out[i].ndim, out[i].shape);
   *bytes = mxnet::op::MXQTempSpaceBytes(n->attrs, si, so);
+  OPS_API_END();
+}
+
+int mxq_node_describe(void* node, int num_in, const mxq_blob* in, int max_out, mxq_blob* out,
+                      int* num_out, size_t* temp_bytes) {
+  OPS_API_BEGIN();
+  Node* n = static_cast<Node*>(node);
+  const int count = static_cast<int>(n->attrs.op->NumOutputs(n->attrs));
+  if (count > max_out) throw dmlc::Error("too many outputs");
+  mxnet::ShapeVector si(num_in), so(count);
+  std::vector<int> ti(num_in), to(count, -1);
+  for (int i = 0; i < num_in; ++i) {
+    si[i] = to_shape(in[i].ndim, in[i].shape);
+    ti[i] = in[i].dtype;
+  }
+  infer_shapes(n, &si, &so);
+  infer_types(n, &ti, &to);
+  if (static_cast<int>(so.size()) != count) throw dmlc::Error("output count changed");
+  for (int i = 0; i < count; ++i) {
+    if (so[i].ndim() > MXQ_MAX_NDIM) throw dmlc::Error("too many dimensions");
+    out[i].ndim = mxnet::shape_is_known(so[i]) ? so[i].ndim() : -1;
+    for (int d = 0; d < out[i].ndim; ++d) out[i].shape[d] = so[i][d];
+    out[i].dtype = to[i];
+  }
+  *num_out = count;
+  *temp_bytes = n->resources.empty() ? 0 : mxnet::op::MXQTempSpaceBytes(n->attrs, si, so);
   OPS_API_END();
 }
 
@@ -202,14 +258,11 @@ int mxq_node_forward(void* node, void* stream, int dev_id, int num_in, const mxq
   if (num_out != static_cast<int>(op->NumOutputs(n->attrs)))
     throw dmlc::Error("wrong number of outputs for " + op->name);
   std::vector<mxnet::TBlob> ins, outs;
-  mxnet::ShapeVector in_shapes;
-  std::vector<int> in_types;
-  for (int i = 0; i < num_in; ++i) {
+  ins.reserve(num_in);
+  outs.reserve(num_out);
+  for (int i = 0; i < num_in; ++i)
     ins.emplace_back(in[i].data, to_shape(in[i].ndim, in[i].shape), mshadow::gpu::kDevMask,
                      in[i].dtype, dev_id);
-    in_shapes.push_back(ins.back().shape_);
-    in_types.push_back(in[i].dtype);
-  }
   for (int i = 0; i < num_out; ++i)
     outs.emplace_back(out[i].data, to_shape(out[i].ndim, out[i].shape), mshadow::gpu::kDevMask,
                       out[i].dtype, dev_id);
@@ -221,28 +274,30 @@ int mxq_node_forward(void* node, void* stream, int dev_id, int num_in, const mxq
   ctx.run_ctx.ctx.dev_type = mxnet::Context::kGPU;
   ctx.run_ctx.ctx.dev_id = dev_id;
   ctx.run_ctx.stream = &s;
-  auto fres = nnvm::Op::GetAttr<mxnet::FResourceRequest>("FResourceRequest");
-  if (fres.count(op)) {
-    for (const auto& r : fres[op](n->attrs)) {
-      mxnet::Resource res;
-      res.req = r;
-      res.ptr_ = temp_space;
-      res.capacity = temp_bytes;
-      ctx.requested.push_back(res);
-    }
+  for (const auto& r : n->resources) {
+    mxnet::Resource res;
+    res.req = r;
+    res.ptr_ = temp_space;
+    res.capacity = temp_bytes;
+    ctx.requested.push_back(res);
   }
 
   // dispatch order of Imperative::InvokeOp: FCompute, else stateful
-  auto fcompute = nnvm::Op::GetAttr<mxnet::FCompute>("FCompute<gpu>");
-  if (fcompute.count(op)) {
-    fcompute[op](n->attrs, ctx, ins, req, outs);
+  if (n->compute != nullptr) {
+    (*n->compute)(n->attrs, ctx, ins, req, outs);
     return 0;
   }
-  auto fcreate = nnvm::Op::GetAttr<mxnet::FCreateOpState>("FCreateOpState");
-  auto fstate = nnvm::Op::GetAttr<mxnet::FStatefulCompute>("FStatefulCompute<gpu>");
-  if (fcreate.count(op) && fstate.count(op)) {
-    if (!n->state) n->state = fcreate[op](n->attrs, ctx.run_ctx.ctx, in_shapes, in_types);
-    fstate[op](n->state, ctx, ins, req, outs);
+  if (n->create_state != nullptr && n->stateful != nullptr) {
+    std::call_once(n->state_once, [&] {
+      mxnet::ShapeVector in_shapes;
+      std::vector<int> in_types;
+      for (const mxnet::TBlob& b : ins) {
+        in_shapes.push_back(b.shape_);
+        in_types.push_back(b.type_flag_);
+      }
+      n->state = (*n->create_state)(n->attrs, ctx.run_ctx.ctx, in_shapes, in_types);
+    });
+    (*n->stateful)(n->state, ctx, ins, req, outs);
     return 0;
   }
   throw dmlc::Error("Operator " + op->name + " is not implemented for GPU.");

@@ -3,13 +3,15 @@ the registry with the reference's operator names, attribute parsing, shape/type
 inference and FCompute<gpu>.  `invoke()` does what `mx.nd.contrib.<op>(...)` does
 in MXNet: attributes are stringified into the node dict exactly as MXNet's frontend
 does, outputs are allocated from the inferred shapes/types, the registered gpu
-function runs on the current stream.  Torch only owns the device memory."""
+function runs on the current stream.  Torch only owns the device memory.  Calls run in
+the extension module `_frontend`; the rest of the host's interface is bound with ctypes."""
 import ctypes
 import os
 
 import torch
 
 from . import _lib  # loads libmxq_hip.so first (libmxq_ops.so links against it)
+from . import _frontend
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 OPS_LIB_PATH = os.path.join(_HERE, "libmxq_ops.so")
@@ -46,6 +48,7 @@ OPS_SIGNATURES = {
     "mxq_node_infer_shape": (_i, [_p, _i, _pi, _pl, _i, _pi, _pl]),
     "mxq_node_infer_type": (_i, [_p, _i, _pi, _i, _pi]),
     "mxq_node_temp_bytes": (_i, [_p, _i, _pb, _i, _pb, ctypes.POINTER(_sz)]),
+    "mxq_node_describe": (_i, [_p, _i, _pb, _i, _pb, _pi, ctypes.POINTER(_sz)]),
     "mxq_node_forward": (_i, [_p, _p, _i, _i, _pb, _i, _pb, _p, _sz]),
     "mxq_quantize_symbol": (_i, [ctypes.c_char_p, _i, _i, _pps, _i, _pps, _i, _pps,
                                  ctypes.c_char_p, ctypes.c_char_p, ctypes.c_char_p, _pps, _pi,
@@ -75,6 +78,9 @@ _DTYPE_OF = {v: k for k, v in _FLAG_OF.items()}
 
 class MXNetError(RuntimeError):
     """What MXNet raises when an operator's CHECK fails (dmlc::Error)."""
+
+
+_frontend.init(MXNetError, _lib.MXQError)
 
 
 def _check(rc):
@@ -116,6 +122,7 @@ class Node:
         _check(ops.mxq_node_create(op.encode(), name.encode(), len(self.attrs), keys, vals,
                                    ctypes.byref(h)))
         self._h = h
+        self._call = _frontend.node(h.value, op)
 
     def __del__(self):
         h = getattr(self, "_h", None)
@@ -188,44 +195,9 @@ class Node:
                 [None if x < 0 else _DTYPE_OF[x] for x in ot])
 
     def __call__(self, *inputs):
-        inputs = [x for x in inputs if x is not None]
-        if len(inputs) != self.num_inputs:
-            raise MXNetError("%s expects %d inputs %s, got %d" % (
-                self.op, self.num_inputs, self.list_inputs(), len(inputs)))
-        for x in inputs:
-            if not (x.is_cuda and x.is_contiguous()):
-                raise MXNetError("inputs must be contiguous device tensors")
-        dev = inputs[0].device
-        _, out_shapes = self.infer_shape([tuple(x.shape) for x in inputs])
-        _, out_types = self.infer_type([x.dtype for x in inputs])
-        outputs = [torch.empty(s, dtype=t, device=dev) for s, t in zip(out_shapes, out_types)]
-
-        def blobs(ts):
-            arr = (Blob * len(ts))()
-            for b, t in zip(arr, ts):
-                b.data = t.data_ptr()
-                b.ndim = t.dim()
-                for d, x in enumerate(t.shape):
-                    b.shape[d] = x
-                b.dtype = _FLAG_OF[t.dtype]
-            return arr
-
-        bi, bo = blobs(inputs), blobs(outputs)
-        nbytes = _sz()
-        _check(ops.mxq_node_temp_bytes(self._h, len(inputs), bi, len(outputs), bo,
-                                       ctypes.byref(nbytes)))
-        temp = None
-        if nbytes.value:
-            temp = torch.empty(nbytes.value, dtype=torch.uint8, device=dev)
-        stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
-        _check(ops.mxq_node_forward(self._h, stream, dev.index or 0, len(inputs), bi,
-                                    len(outputs), bo,
-                                    ctypes.c_void_p(temp.data_ptr()) if temp is not None else None,
-                                    nbytes.value))
-        return outputs[0] if len(outputs) == 1 else tuple(outputs)
+        return _frontend.forward(self._call, *inputs)
 
 
 def invoke(op, *inputs, **attrs):
     """mx.nd.contrib-style call: tensors positionally, attributes by keyword."""
-    attrs = {k: v for k, v in attrs.items() if v is not None}
-    return Node(op, **attrs)(*inputs)
+    return _frontend.invoke(op, *inputs, **attrs)
