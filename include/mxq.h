@@ -404,6 +404,20 @@ int mxq_quantized_conv_nchw(void* stream, const int8_t* data, const int8_t* weig
                             const float* min_bias, const float* max_bias, int32_t* out32,
                             float* omin, float* omax, void* workspace, size_t workspace_bytes);
 
+/* ---- calibration -----------------------------------------------------------
+ * What the calibration collectors take of a float tensor
+ * (python/mxnet/contrib/quantization.py:269-361, numpy on the host in the reference).
+ * mxq_minmax_f32: smallest and largest value into two device floats, both NaN if there is a
+ * NaN; workspace as for mxq_quantize_v2.
+ * mxq_histogram_f32: counts[k] of the values with edges[k] <= x < edges[k + 1] (the last bin
+ * includes its upper edge), `bins` + 1 increasing edges and `bins` counts on the device;
+ * values outside and NaN are not counted; n < 2^32. */
+size_t mxq_minmax_f32_workspace(size_t n);
+int mxq_minmax_f32(void* stream, const float* in, size_t n, float* out_min, float* out_max,
+                   void* workspace, size_t workspace_bytes);
+int mxq_histogram_f32(void* stream, const float* in, size_t n, const float* edges, int bins,
+                      uint32_t* counts);
+
 /* [N,C,H,W] int8 -> [N,H,W,C] int8 (also OIHW -> OHWI for the weight). */
 int mxq_nchw_to_nhwc_i8(void* stream, const int8_t* in, int8_t* out, int N, int C, int H, int W);
 /* The same with the channel extent of the output padded to C_padded >= C with zeros

@@ -94,6 +94,11 @@ int mxq_symbol_normalize(const char* symbol_json, const char** out_symbol_json);
  * arrays: hist[num_bins] (num_bins odd), hist_edges[num_bins + 1]. */
 int mxq_calibrate_entropy(const float* hist, const float* hist_edges, size_t num_bins,
                           int num_quantized_bins, float* out_threshold, float* out_divergence);
+/* The same for `count` histograms in one call, which share the threads it starts. */
+int mxq_calibrate_entropy_many(int count, const float* const* hist,
+                               const float* const* hist_edges, const size_t* num_bins,
+                               const int* num_quantized_bins, float* out_thresholds,
+                               float* out_divergences);
 
 /* ---- NDArray list files (`.params`, mx.nd.save / mx.nd.load) ------------------------
  * src/ndarray/ndarray.cc:1856-2146: dense arrays of the V2 / V3 record layouts plus the

@@ -72,6 +72,9 @@ SIGNATURES = {
     "mxq_quantized_conv_nchw_workspace": (_sz, [_i] * 14),
     "mxq_quantized_conv_nchw": (_i, [_p, _p, _p, _p] + [_i] * 13 + [_p] * 6 +
                                 [_p, _p, _p, _p, _sz]),
+    "mxq_minmax_f32_workspace": (_sz, [_sz]),
+    "mxq_minmax_f32": (_i, [_p, _p, _sz, _p, _p, _p, _sz]),
+    "mxq_histogram_f32": (_i, [_p, _p, _sz, _p, _i, _p]),
     "mxq_nchw_to_nhwc_i8": (_i, [_p, _p, _p, _i, _i, _i, _i]),
     "mxq_nchw_to_nhwc_pad_i8": (_i, [_p, _p, _p, _i, _i, _i, _i, _i]),
     "mxq_nchw_to_s2d_nhwc_i8": (_i, [_p, _p, _p, _i, _i, _i, _i, _i, _i, _i]),

@@ -9,7 +9,7 @@ LIB = os.path.join(HERE, "libmxq_hip.so")
 
 HIP_SOURCES = ["mxq_capi.hip", "mxq_cast.hip", "mxq_fc.hip", "mxq_fc_plain.hip", "mxq_fc_f32.hip",
                "mxq_fc_sum.hip", "mxq_conv.hip", "mxq_conv_nchw.hip", "mxq_pool.hip",
-               "mxq_eltwise.hip", "mxq_layout.hip"]
+               "mxq_eltwise.hip", "mxq_layout.hip", "mxq_histogram.hip"]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",
@@ -94,7 +94,7 @@ def build_ops(verbose=False):
     cxx = os.environ.get("CXX", "g++")
     srcs = [os.path.join(CSRC, "host", s) for s in HOST_SOURCES]
     cmd = [cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-ffp-contract=off", "-Wall", "-Wextra",
-           "-Wno-unused-parameter", "-o", OPS_LIB] + srcs + \
+           "-Wno-unused-parameter", "-pthread", "-o", OPS_LIB] + srcs + \
           ["-L" + HERE, "-lmxq_hip", "-Wl,-rpath,$ORIGIN"]
     if verbose:
         print(" ".join(cmd), flush=True)

@@ -258,3 +258,25 @@ def nhwc_to_nchw(x):
     out = torch.empty((N, C, H, W), dtype=x.dtype, device=x.device)
     check(lib.mxq_nhwc_to_nchw(_stream(), _ptr(x), _ptr(out), N, C, H, W, x.element_size()))
     return out
+
+
+def minmax(data):
+    """Smallest and largest value of a float32 tensor as one device tensor of two."""
+    assert data.dtype == torch.float32
+    out = torch.empty(2, dtype=torch.float32, device=data.device)
+    n = data.numel()
+    wsb = lib.mxq_minmax_f32_workspace(n)
+    ws = _workspace(wsb, data.device)
+    check(lib.mxq_minmax_f32(_stream(), _ptr(data), n, _ptr(out), _ptr(out[1:]), _ptr(ws), wsb))
+    return out
+
+
+def histogram(data, edges):
+    """Counts (int32, on the device) of a float32 tensor's values between consecutive `edges`
+    (increasing, on the device); the last bin includes its upper edge."""
+    assert data.dtype == torch.float32 and edges.dtype == torch.float32
+    bins = edges.numel() - 1
+    counts = torch.empty(bins, dtype=torch.int32, device=data.device)
+    check(lib.mxq_histogram_f32(_stream(), _ptr(data), data.numel(), _ptr(edges), bins,
+                                _ptr(counts)))
+    return counts

@@ -370,4 +370,17 @@ int mxq_calibrate_entropy(const float* hist, const float* hist_edges, size_t num
   OPS_API_END();
 }
 
+int mxq_calibrate_entropy_many(int count, const float* const* hist,
+                               const float* const* hist_edges, const size_t* num_bins,
+                               const int* num_quantized_bins, float* out_thresholds,
+                               float* out_divergences) {
+  OPS_API_BEGIN();
+  CHECK(count >= 0) << "negative count";
+  CHECK(hist && hist_edges && num_bins && num_quantized_bins && out_thresholds && out_divergences)
+      << "null argument";
+  mxq_graph::CalibrateEntropyMany(static_cast<size_t>(count), hist, hist_edges, num_bins,
+                                  num_quantized_bins, out_thresholds, out_divergences);
+  OPS_API_END();
+}
+
 }  // extern "C"

@@ -796,6 +796,17 @@ __global__ __launch_bounds__(kThreads) void relu_chunk_kernel(const int8_t* __re
   }
 }
 
+// The partials of minmax_f32_kernel as two floats; both NaN where the tensor holds one.
+__global__ __launch_bounds__(kThreads) void minmax_result_kernel(
+    const uint32_t* __restrict__ parts, int nparts, float* out_min, float* out_max) {
+  float lo, hi;
+  load_range_f32(parts, nparts, lo, hi);
+  if (threadIdx.x == 0) {
+    *out_min = lo;
+    *out_max = hi;
+  }
+}
+
 __global__ void passthrough_range_kernel(float* omin, float* omax, float lo, float hi) {
   *omin = lo;
   *omax = hi;
@@ -933,6 +944,26 @@ int mxq_quantize(void* stream, const float* in, const float* imin, const float* 
   if (n == 0) return 0;
   launch_quantize(static_cast<hipStream_t>(stream), in, out, omin, omax, n, out_type, 0.f, 0.f,
                   imin, imax, nullptr, 0);
+  MXQ_API_END();
+}
+
+size_t mxq_minmax_f32_workspace(size_t) { return kWsBytes; }
+
+int mxq_minmax_f32(void* stream, const float* in, size_t n, float* out_min, float* out_max,
+                   void* workspace, size_t workspace_bytes) {
+  MXQ_API_BEGIN();
+  MXQ_CHECK(n > 0 && in != nullptr, "no data");
+  MXQ_CHECK(out_min != nullptr && out_max != nullptr, "null output");
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  uint32_t* parts = carve(workspace, workspace_bytes);
+  const int grid = reduce_grid(n);
+  if (aligned16(in))
+    hipLaunchKernelGGL((minmax_f32_kernel<true>), dim3(grid), dim3(kThreads), 0, s, in, n, parts);
+  else
+    hipLaunchKernelGGL((minmax_f32_kernel<false>), dim3(grid), dim3(kThreads), 0, s, in, n, parts);
+  hipLaunchKernelGGL(minmax_result_kernel, dim3(1), dim3(kThreads), 0, s, parts, grid, out_min,
+                     out_max);
+  MXQ_LAUNCH_CHECK();
   MXQ_API_END();
 }
 

@@ -1,0 +1,95 @@
+"""The entropy search against a plain restatement of its definition
+(src/operator/quantization/calibrate.cc:33-186) in binary32, bin by bin: the same threshold and
+divergence to the last bit, on histograms with long empty runs, with more than 2^24 counts and
+with none outside the kept bins."""
+import ctypes
+import ctypes.util
+
+import numpy as np
+import pytest
+
+from mxnet_amd import quantization as Q
+
+f32 = np.float32
+_libm = ctypes.CDLL(ctypes.util.find_library("m"))
+_libm.logf.restype = ctypes.c_float
+_libm.logf.argtypes = [ctypes.c_float]
+
+
+def running_sum(values, first=f32(0)):
+    return f32(np.cumsum(np.concatenate([[first], values]).astype(f32), dtype=f32)[-1])
+
+
+def smooth(p):
+    zero = p == 0
+    nz = int((~zero).sum())
+    if nz == 0:
+        return None
+    take = f32(f32(0.0001) * f32(zero.sum()) / f32(nz))
+    return None if take >= 1 else np.where(zero, f32(0.0001), p - take).astype(f32)
+
+
+def restated(hist, edges, nq):
+    n, zero, half = len(hist), len(hist) // 2, nq // 2
+    best = (np.finfo(f32).max, 0)
+    for i in range(half, zero + 1):
+        start, stop = zero - i, zero + i + 1
+        p = hist[start:stop].astype(f32).copy()
+        sliced = hist[start:stop].astype(np.int64)
+        sliced[0] = 0
+        p[0] = running_sum(hist[:start + 1])
+        p[-1] = running_sum(hist[stop:], p[-1])
+        merged = len(p) // nq
+        q = np.zeros(len(p), f32)
+        for j in range(nq):
+            lo, hi = j * merged, len(p) if j == nq - 1 else (j + 1) * merged
+            level = f32(sliced[lo:lo + merged].sum())
+            if j == nq - 1:
+                level = f32(level + f32(sliced[lo + merged:].sum()))
+            filled = int((sliced[lo:hi] != 0).sum())
+            if filled:
+                q[lo:hi] = np.where(p[lo:hi] != 0, level / f32(filled), 0)
+        ps, qs = smooth(p), smooth(q)
+        if qs is None:
+            continue
+        ps, qs = ps / running_sum(ps), qs / running_sum(qs)
+        terms = ps * np.array([_libm.logf(r) for r in (ps / qs).astype(f32)], f32)
+        kl = running_sum(terms)
+        if kl < best[0]:
+            best = (kl, i)
+    return edges[zero + best[1] + 1], best[0]
+
+
+@pytest.mark.parametrize("kind", ["normal", "outliers", "one_sided", "sparse", "huge", "empty"])
+@pytest.mark.parametrize("bins,nq", [(61, 15), (255, 255), (1001, 31)])
+def test_entropy_search_is_the_definition_bit_for_bit(kind, bins, nq):
+    rng = np.random.default_rng(bins + nq)
+    x = rng.standard_normal(20000)
+    hist = np.histogram(x, bins=bins, range=(-5, 5))[0].astype(f32)
+    if kind == "outliers":  # empty runs of hundreds of bins
+        hist = np.histogram(np.where(rng.random(20000) < 1e-3, np.sign(x) * 39, x), bins=bins,
+                            range=(-40, 40))[0].astype(f32)
+    elif kind == "one_sided":
+        hist = np.histogram(np.maximum(x, 0), bins=bins, range=(-5, 5))[0].astype(f32)
+    elif kind == "sparse":
+        hist = np.where(rng.random(bins) < 0.1, rng.integers(1, 900, bins), 0).astype(f32)
+        hist[bins // 2] = 5
+    elif kind == "huge":  # partial sums round
+        hist = (hist * f32(100003)).astype(f32)
+    elif kind == "empty":
+        hist = np.zeros(bins, f32)
+        hist[bins // 2] = 7
+    edges = np.linspace(-1, 1, bins + 1).astype(f32)
+    got = Q.calibrate_entropy(hist, edges, nq)
+    want = restated(hist, edges, nq)
+    assert (got[0], got[1]) == (f32(want[0]), f32(want[1]))
+
+
+def test_several_histograms_at_once():
+    rng = np.random.default_rng(0)
+    problems = []
+    for bins, nq in ((401, 63), (8001, 255), (1201, 31)):
+        hist = np.histogram(rng.standard_normal(5000), bins=bins, range=(-4, 4))[0]
+        problems.append((hist, np.linspace(-4, 4, bins + 1), nq))
+    assert Q._calibrate_entropy_many(problems) == [Q.calibrate_entropy(*p) for p in problems]
+    assert Q._calibrate_entropy_many([]) == []

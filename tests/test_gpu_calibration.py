@@ -1,0 +1,59 @@
+"""The calibration collectors' device reductions against numpy: extreme values and histogram
+counts are the same numbers, at the edges of the vector loads, of the LDS bins and of the bins
+themselves."""
+import numpy as np
+import pytest
+import torch
+
+from mxnet_amd import capi
+from mxnet_amd import quantization as Q
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 1023, 4097, 100003])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_minmax(n, offset):
+    x = np.random.default_rng(n).standard_normal(n + offset).astype(np.float32)
+    got = capi.minmax(torch.from_numpy(x).cuda()[offset:]).cpu().numpy()
+    assert tuple(got) == (x[offset:].min(), x[offset:].max())
+
+
+def test_minmax_nan():
+    x = torch.randn(1000, device="cuda")
+    x[777] = float("nan")
+    assert torch.isnan(capi.minmax(x)).all()
+
+
+@pytest.mark.parametrize("n", [1, 511, 513, 70001, 1 << 20])
+@pytest.mark.parametrize("bins", [1, 2, 255, 8001, 16384, 16385, 30001])
+def test_histogram_counts_as_numpy(n, bins):
+    rng = np.random.default_rng(n + bins)
+    x = rng.standard_normal(n).astype(np.float32)
+    x[:: 3] = np.maximum(x[:: 3], 0)
+    th = np.max(np.abs(x)) * np.float32(0.9 if n % 2 else 1.0)  # values outside, too
+    got = Q._Values(torch.from_numpy(x).cuda()).counts(bins, th)
+    assert np.array_equal(got, np.histogram(x, bins=bins, range=(-th, th))[0])
+
+
+def test_histogram_of_values_on_the_edges():
+    edges = np.linspace(-2, 2, 8002).astype(np.float32)
+    x = np.concatenate([edges, np.nextafter(edges, np.float32(9)),
+                        np.nextafter(edges, np.float32(-9)), [np.nan]]).astype(np.float32)
+    got = capi.histogram(torch.from_numpy(x).cuda(), torch.from_numpy(edges).cuda())
+    inside = x[(x >= edges[0]) & (x <= edges[-1])]
+    at = np.minimum(np.searchsorted(edges, inside, side="right") - 1, 8000)
+    assert np.array_equal(got.cpu().numpy(), np.bincount(at, minlength=8001))
+
+
+def test_collector_on_device_tensors_is_the_host_collector():
+    rng = np.random.default_rng(1)
+    batches = [rng.standard_normal((64, 33)).astype(np.float32) * s for s in (1.0, 3.0, 0.5)]
+    on_host, on_device = (Q._LayerHistogramCollector("int8", include_layers=["t"])
+                          for _ in range(2))
+    for b in batches:
+        on_host.collect("t", "op", b)
+        on_device.collect("t", "op", torch.from_numpy(b).cuda())
+    for h, d in zip(on_host.hist_dict["t"], on_device.hist_dict["t"]):
+        assert np.array_equal(h, d)
+    assert on_host.post_collect() == on_device.post_collect()
