@@ -343,6 +343,24 @@ int mxq_quantized_fc_sum(void* stream, const int8_t* data, const int8_t* weight,
                          float max_calib, float sum_min_calib, float sum_max_calib, int sum_relu,
                          void* workspace, size_t workspace_bytes);
 
+/* mxq_quantized_fc_sum for a sum that is calibrated behind the operator: the layer's
+ * requantized int8 output and the residual are added in int32 over the sum's own range
+ * (_contrib_quantized_elemwise_add without a calibrated range) and that sum is requantized
+ * over (sum_min_calib, sum_max_calib) (_contrib_requantize), which is the graph QuantizeGraph
+ * makes of an elemwise_add between two layers; sum_relu != 0 clamps at zero.  out8 is
+ * bit-identical to the operators one after the other; rmin / rmax receive the requantized
+ * range. */
+int mxq_quantized_fc_sum_requant(void* stream, const int8_t* data, const int8_t* weight,
+                                 const int8_t* bias, int M, int N, int K, const float* min_data,
+                                 const float* max_data, const float* min_weight,
+                                 const float* max_weight, const float* min_bias,
+                                 const float* max_bias, const int8_t* residual,
+                                 const float* min_residual, const float* max_residual,
+                                 int8_t* out8, float* omin, float* omax, float* rmin, float* rmax,
+                                 float min_calib, float max_calib, float sum_min_calib,
+                                 float sum_max_calib, int sum_relu, void* workspace,
+                                 size_t workspace_bytes);
+
 /* ---- _contrib_quantized_conv ----------------------------------------------
  * Replaces QuantizedCuDNNConvOp::Forward
  * (src/operator/quantization/quantized_conv.cu:101-219): the NHWC int8
@@ -403,6 +421,29 @@ int mxq_quantized_conv_nchw(void* stream, const int8_t* data, const int8_t* weig
                             const float* min_weight, const float* max_weight,
                             const float* min_bias, const float* max_bias, int32_t* out32,
                             float* omin, float* omax, void* workspace, size_t workspace_bytes);
+
+/* ---- networks held as NHWC ---------------------------------------------------
+ * For a caller that keeps int8 activations as [N,H,W,C_padded] between the layers, C_padded
+ * the channel count rounded up to 16 and the channels past C zero (zero weights and a zero
+ * bias keep them zero through every layer).
+ * mxq_quantize_to_nhwc: calibrated quantize_v2 (int8) of a float NCHW image straight into that
+ * layout; space_to_depth != 0 into the layout of mxq_nchw_to_s2d_nhwc_i8.
+ * mxq_quantized_pooling_nhwc: mxq_quantized_pooling_nchw's windows and rounding on int8 of that
+ * layout (C a multiple of 16); the range passes through and is left to the caller.
+ * mxq_pack_weight: OIHW int8 -> [O_padded,KH,KW,C_padded] with zeros, or the weight of the
+ * space-to-depth form ([O_padded,(KH+1)/2,(KW+1)/2,C_padded]).
+ * mxq_nhwc_pad_to_nchw_i8: back to [N,C,H,W]. */
+int mxq_quantize_to_nhwc(void* stream, const float* in, int8_t* out, float* omin, float* omax,
+                         int N, int C, int H, int W, int C_padded, int space_to_depth, int off_h,
+                         int off_w, float min_calib, float max_calib);
+int mxq_quantized_pooling_nhwc(void* stream, const int8_t* in, int N, int H, int W, int C,
+                               int kernel_h, int kernel_w, int stride_h, int stride_w, int pad_h,
+                               int pad_w, int OH, int OW, int pool_type, int count_include_pad,
+                               int8_t* out);
+int mxq_pack_weight(void* stream, const int8_t* in, int8_t* out, int O, int C, int KH, int KW,
+                    int O_padded, int C_padded, int space_to_depth);
+int mxq_nhwc_pad_to_nchw_i8(void* stream, const int8_t* in, int8_t* out, int N, int C, int H,
+                            int W, int C_padded);
 
 /* ---- calibration -----------------------------------------------------------
  * What the calibration collectors take of a float tensor

@@ -3,6 +3,9 @@ missing or a symbol is absent the import raises."""
 import ctypes
 import os
 
+# before the library below: the HIP runtime torch brings has to be the process's only one
+import torch  # noqa: F401
+
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libmxq_hip.so")
 
@@ -64,6 +67,8 @@ SIGNATURES = {
                                   _i, _f, _f, _p, _sz]),
     "mxq_quantized_fc_sum": (_i, [_p, _p, _p, _p, _i, _i, _i] + [_p] * 6 + [_p, _p, _p] +
                              [_p, _p, _p, _p, _p, _f, _f, _f, _f, _i, _p, _sz]),
+    "mxq_quantized_fc_sum_requant": (_i, [_p, _p, _p, _p, _i, _i, _i] + [_p] * 6 + [_p, _p, _p] +
+                                     [_p, _p, _p, _p, _p, _f, _f, _f, _f, _i, _p, _sz]),
     "mxq_quantized_conv_workspace": (_sz, [_i] * 14),
     "mxq_quantized_conv_nhwc": (_i, [_p, _p, _p, _p] + [_i] * 13 + [_p] * 6 +
                                 [_p, _p, _p, _p, _p, _p, _i, _f, _f, _p, _sz]),
@@ -72,6 +77,10 @@ SIGNATURES = {
     "mxq_quantized_conv_nchw_workspace": (_sz, [_i] * 14),
     "mxq_quantized_conv_nchw": (_i, [_p, _p, _p, _p] + [_i] * 13 + [_p] * 6 +
                                 [_p, _p, _p, _p, _sz]),
+    "mxq_quantize_to_nhwc": (_i, [_p] * 5 + [_i] * 8 + [_f, _f]),
+    "mxq_quantized_pooling_nhwc": (_i, [_p, _p] + [_i] * 14 + [_p]),
+    "mxq_pack_weight": (_i, [_p, _p, _p] + [_i] * 7),
+    "mxq_nhwc_pad_to_nchw_i8": (_i, [_p, _p, _p] + [_i] * 5),
     "mxq_minmax_f32_workspace": (_sz, [_sz]),
     "mxq_minmax_f32": (_i, [_p, _p, _sz, _p, _p, _p, _sz]),
     "mxq_histogram_f32": (_i, [_p, _p, _sz, _p, _i, _p]),

@@ -8,8 +8,9 @@ CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libmxq_hip.so")
 
 HIP_SOURCES = ["mxq_capi.hip", "mxq_cast.hip", "mxq_fc.hip", "mxq_fc_plain.hip", "mxq_fc_f32.hip",
-               "mxq_fc_sum.hip", "mxq_conv.hip", "mxq_conv_nchw.hip", "mxq_pool.hip",
-               "mxq_eltwise.hip", "mxq_layout.hip", "mxq_histogram.hip"]
+               "mxq_fc_sum.hip", "mxq_fc_sum_requant.hip", "mxq_conv.hip", "mxq_conv_nchw.hip", "mxq_pool.hip",
+               "mxq_eltwise.hip", "mxq_layout.hip", "mxq_histogram.hip",
+               "mxq_nhwc.hip"]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",
@@ -103,7 +104,7 @@ def build_ops(verbose=False):
 
 
 FRONTEND_LIB = os.path.join(HERE, "_frontend.so")
-FRONTEND_SOURCES = ["mxq_frontend.cc"]
+FRONTEND_SOURCES = ["mxq_frontend.cc", "mxq_plan.cc"]
 
 
 def build_frontend(verbose=False):

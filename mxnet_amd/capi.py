@@ -152,10 +152,11 @@ def quantized_fc_f32(data, weight, bias, min_data, max_data, min_weight, max_wei
 
 def quantized_fc_sum(data, weight, bias, residual, min_data, max_data, min_weight, max_weight,
                      min_bias, max_bias, min_residual, max_residual, calib, sum_calib,
-                     sum_relu=False, force=None):
+                     sum_relu=False, force=None, requant=False):
     """quantized_fc -> requantize over `calib` -> elemwise_add with `residual` over `sum_calib`
-    (-> relu) in one launch.  Returns dict(out8, omin, omax, rmin, rmax).  `force` = (cfg,
-    splits, stream_groups) pins the kernel variant through the test-only entry point."""
+    (-> relu) in one launch.  Returns dict(out8, omin, omax, rmin, rmax).  `requant`: the sum is
+    taken in int32 over its own range and requantized over `sum_calib`.  `force` = (cfg, splits,
+    stream_groups) pins the kernel variant through the test-only entry point."""
     M, K = data.shape
     N, K2 = weight.shape
     assert K == K2 and tuple(residual.shape) == (M, N) and residual.dtype == torch.int8
@@ -171,7 +172,8 @@ def quantized_fc_sum(data, weight, bias, residual, min_data, max_data, min_weigh
     if force is None:
         wsb = lib.mxq_quantized_fc_workspace(M, N, K, 1)
         ws = _workspace(wsb, dev) if wsb else None
-        check(lib.mxq_quantized_fc_sum(*args, _ptr(ws), wsb))
+        call = lib.mxq_quantized_fc_sum_requant if requant else lib.mxq_quantized_fc_sum
+        check(call(*args, _ptr(ws), wsb))
     else:
         cfg, splits, groups = force
         wsb = _SPLIT_WS_BYTES if splits > 1 else 0

@@ -20,6 +20,7 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <cstdlib>
 #include <cstring>
 #include <memory>
 #include <string>
@@ -28,6 +29,7 @@
 
 #include "../../../include/mxq.h"
 #include "../../../include/mxq_ops.h"
+#include "mxq_plan.h"
 
 namespace {
 
@@ -625,6 +627,223 @@ PyObject* py_quantized_conv_nhwc(PyObject*, PyObject* const* args, Py_ssize_t na
   END_HANDLE_TH_ERRORS
 }
 
+// ---- plans (mxq_plan.h) ------------------------------------------------------------------------
+
+// describe(node, ((type flag, shape), ...)) -> ([(type flag, shape), ...], temp-space bytes)
+PyObject* py_describe(PyObject*, PyObject* args) {
+  HANDLE_TH_ERRORS
+  PyObject *capsule, *given;
+  if (!PyArg_ParseTuple(args, "OO!", &capsule, &PyTuple_Type, &given)) return nullptr;
+  OpNode* n = static_cast<OpNode*>(PyCapsule_GetPointer(capsule, kNodeCapsule));
+  if (n == nullptr) return nullptr;
+  mxq_blob in[kMaxInputs];
+  const Py_ssize_t num_in = PyTuple_GET_SIZE(given);
+  if (num_in != n->num_inputs || num_in > kMaxInputs) {
+    wrong_count(*n, num_in);
+    return nullptr;
+  }
+  for (Py_ssize_t i = 0; i < num_in; ++i) {
+    PyObject* shape;
+    if (!PyArg_ParseTuple(PyTuple_GET_ITEM(given, i), "iO!", &in[i].dtype, &PyTuple_Type, &shape))
+      return nullptr;
+    in[i].ndim = static_cast<int>(PyTuple_GET_SIZE(shape));
+    if (in[i].ndim > MXQ_MAX_NDIM) {
+      PyErr_SetString(PyExc_IndexError, "too many dimensions");
+      return nullptr;
+    }
+    for (int d = 0; d < in[i].ndim; ++d)
+      in[i].shape[d] = PyLong_AsLongLong(PyTuple_GET_ITEM(shape, d));
+  }
+  if (PyErr_Occurred()) return nullptr;
+  const auto sig = signature_of(n, in, static_cast<int>(num_in));
+  if (sig == nullptr) return nullptr;
+  PyObject* outs = PyList_New(0);
+  for (const OutMeta& m : sig->outs) {
+    PyObject* shape = PyTuple_New(m.ndim);
+    for (int d = 0; d < m.ndim; ++d) PyTuple_SET_ITEM(shape, d, PyLong_FromLongLong(m.shape[d]));
+    PyObject* one = Py_BuildValue("(iN)", m.flag, shape);
+    if (one == nullptr || PyList_Append(outs, one) != 0) {
+      Py_XDECREF(one);
+      Py_DECREF(outs);
+      return nullptr;
+    }
+    Py_DECREF(one);
+  }
+  return Py_BuildValue("(NK)", outs, static_cast<unsigned long long>(sig->temp_bytes));
+  END_HANDLE_TH_ERRORS
+}
+
+constexpr const char* kPlanCapsule = "mxnet_amd.plan";
+
+void free_plan(PyObject* capsule) {
+  delete static_cast<mxq_plan::Plan*>(PyCapsule_GetPointer(capsule, kPlanCapsule));
+}
+
+bool int_list(PyObject* tuple, std::vector<int64_t>* out) {
+  if (!PyTuple_Check(tuple)) {
+    PyErr_SetString(PyExc_TypeError, "expected a tuple");
+    return false;
+  }
+  for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(tuple); ++i)
+    out->push_back(PyLong_AsLongLong(PyTuple_GET_ITEM(tuple, i)));
+  return !PyErr_Occurred();
+}
+
+// step tuple: (kind, ints, floats, ((base, index, offset), ...)[, node, (num_in, ((flag, shape), ...))])
+bool parse_step(PyObject* item, mxq_plan::Step* s) {
+  int kind;
+  PyObject *ints, *floats, *refs, *node = nullptr, *blobs = nullptr;
+  if (!PyArg_ParseTuple(item, "iOO!O!|OO!", &kind, &ints, &PyTuple_Type, &floats, &PyTuple_Type,
+                        &refs, &node, &PyTuple_Type, &blobs))
+    return false;
+  s->kind = static_cast<mxq_plan::Kind>(kind);
+  if (!int_list(ints, &s->ints)) return false;
+  for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(floats); ++i)
+    s->floats.push_back(static_cast<float>(PyFloat_AsDouble(PyTuple_GET_ITEM(floats, i))));
+  for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(refs); ++i) {
+    mxq_plan::Ref r;
+    long long offset;
+    if (!PyArg_ParseTuple(PyTuple_GET_ITEM(refs, i), "iiL", &r.base, &r.index, &offset))
+      return false;
+    r.offset = offset;
+    s->refs.push_back(r);
+  }
+  if (node != nullptr) {
+    const OpNode* n = static_cast<OpNode*>(PyCapsule_GetPointer(node, kNodeCapsule));
+    if (n == nullptr) return false;
+    s->node = n->handle;
+    PyObject* list;
+    if (!PyArg_ParseTuple(blobs, "iO!", &s->num_in, &PyTuple_Type, &list)) return false;
+    for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(list); ++i) {
+      mxq_blob b = {};
+      PyObject* shape;
+      if (!PyArg_ParseTuple(PyTuple_GET_ITEM(list, i), "iO!", &b.dtype, &PyTuple_Type, &shape))
+        return false;
+      b.ndim = static_cast<int>(PyTuple_GET_SIZE(shape));
+      if (b.ndim > MXQ_MAX_NDIM) {
+        PyErr_SetString(PyExc_IndexError, "too many dimensions");
+        return false;
+      }
+      for (int d = 0; d < b.ndim; ++d)
+        b.shape[d] = PyLong_AsLongLong(PyTuple_GET_ITEM(shape, d));
+      s->blobs.push_back(b);
+    }
+    if (s->refs.size() != s->blobs.size() + 1) {
+      PyErr_SetString(PyExc_ValueError, "a node step has one reference per tensor and a workspace");
+      return false;
+    }
+  }
+  return !PyErr_Occurred();
+}
+
+// plan(arena bytes, [held tensors], [steps], [(type flag, shape) of the outputs])
+PyObject* py_plan(PyObject*, PyObject* args) {
+  HANDLE_TH_ERRORS
+  long long arena;
+  PyObject *held, *steps, *outputs;
+  if (!PyArg_ParseTuple(args, "LO!O!O!", &arena, &PyList_Type, &held, &PyList_Type, &steps,
+                        &PyList_Type, &outputs))
+    return nullptr;
+  std::unique_ptr<mxq_plan::Plan> plan(new mxq_plan::Plan());
+  plan->arena_bytes = arena;
+  for (Py_ssize_t i = 0; i < PyList_GET_SIZE(held); ++i) {
+    at::Tensor t;
+    if (!tensor_arg(PyList_GET_ITEM(held, i), &t)) return nullptr;
+    plan->held.push_back(t);
+  }
+  for (Py_ssize_t i = 0; i < PyList_GET_SIZE(steps); ++i) {
+    mxq_plan::Step s;
+    if (!parse_step(PyList_GET_ITEM(steps, i), &s)) return nullptr;
+    plan->steps.push_back(std::move(s));
+  }
+  for (Py_ssize_t i = 0; i < PyList_GET_SIZE(outputs); ++i) {
+    int flag;
+    PyObject* shape;
+    if (!PyArg_ParseTuple(PyList_GET_ITEM(outputs, i), "iO!", &flag, &PyTuple_Type, &shape))
+      return nullptr;
+    mxq_plan::Output o;
+    if (!dtype_of(flag, &o.type) || !int_list(shape, &o.shape)) return nullptr;
+    plan->outputs.push_back(o);
+  }
+  PyObject* capsule = PyCapsule_New(plan.get(), kPlanCapsule, free_plan);
+  if (capsule != nullptr) plan.release();
+  return capsule;
+  END_HANDLE_TH_ERRORS
+}
+
+// run_plan(plan, *feeds) -> [outputs]
+PyObject* py_run_plan(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  if (nargs < 2) {
+    PyErr_SetString(PyExc_TypeError, "run_plan(plan, *feeds)");
+    return nullptr;
+  }
+  const auto* plan = static_cast<mxq_plan::Plan*>(PyCapsule_GetPointer(args[0], kPlanCapsule));
+  if (plan == nullptr) return nullptr;
+  std::vector<at::Tensor> feeds(nargs - 1), outs;
+  for (Py_ssize_t i = 1; i < nargs; ++i)
+    if (!tensor_arg(args[i], &feeds[i - 1])) return nullptr;
+  const at::Device dev = feeds[0].device();
+  for (const auto& o : plan->outputs) outs.push_back(empty_on(o.shape, o.type, dev));
+  at::Tensor arena;
+  if (plan->arena_bytes != 0) arena = workspace(static_cast<size_t>(plan->arena_bytes), dev);
+  void* stream = current_stream();
+  std::string error;
+  bool ok;
+  Py_BEGIN_ALLOW_THREADS;
+  ok = plan->run(stream, feeds, outs, arena, &error);
+  Py_END_ALLOW_THREADS;
+  if (!ok) {
+    PyErr_SetString(g_op_error, error.c_str());
+    return nullptr;
+  }
+  PyObject* list = PyList_New(static_cast<Py_ssize_t>(outs.size()));
+  for (size_t i = 0; i < outs.size(); ++i) {
+    PyObject* o = THPVariable_Wrap(std::move(outs[i]));
+    if (o == nullptr) {
+      Py_DECREF(list);
+      return nullptr;
+    }
+    PyList_SET_ITEM(list, static_cast<Py_ssize_t>(i), o);
+  }
+  return list;
+  END_HANDLE_TH_ERRORS
+}
+
+// same_params(dict, ((name, tensor, version), ...)): the dict still holds these tensors, unwritten
+PyObject* py_same_params(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  if (nargs != 2 || !PyDict_Check(args[0]) || !PyTuple_Check(args[1])) {
+    PyErr_SetString(PyExc_TypeError, "same_params(dict, entries)");
+    return nullptr;
+  }
+  for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(args[1]); ++i) {
+    PyObject* entry = PyTuple_GET_ITEM(args[1], i);
+    PyObject* now = PyDict_GetItemWithError(args[0], PyTuple_GET_ITEM(entry, 0));
+    PyObject* was = PyTuple_GET_ITEM(entry, 1);
+    if (now == nullptr && PyErr_Occurred()) return nullptr;
+    if (now != was) Py_RETURN_FALSE;
+    const at::Tensor& t = THPVariable_Unpack(was);
+    if (static_cast<long>(t._version()) != PyLong_AsLong(PyTuple_GET_ITEM(entry, 2)))
+      Py_RETURN_FALSE;
+  }
+  Py_RETURN_TRUE;
+  END_HANDLE_TH_ERRORS
+}
+
+// float_of(text): an attribute's value as the operators parse it
+PyObject* py_float_of(PyObject*, PyObject* text) {
+  const char* s = PyUnicode_AsUTF8(text);
+  if (s == nullptr) return nullptr;
+  char* end = nullptr;
+  const float v = std::strtof(s, &end);
+  if (end == s) {
+    PyErr_SetString(PyExc_ValueError, "not a number");
+    return nullptr;
+  }
+  return PyFloat_FromDouble(v);
+}
+
 // init(MXNetError, MXQError)
 PyObject* py_init(PyObject*, PyObject* args) {
   PyObject *op_error, *lib_error;
@@ -649,6 +868,11 @@ PyMethodDef methods[] = {
     {"forward", as_cfunction(py_forward), METH_FASTCALL, "One call of an existing node."},
     {"quantized_fc", as_cfunction(py_quantized_fc), METH_FASTCALL, nullptr},
     {"quantized_conv_nhwc", as_cfunction(py_quantized_conv_nhwc), METH_FASTCALL, nullptr},
+    {"describe", py_describe, METH_VARARGS, nullptr},
+    {"plan", py_plan, METH_VARARGS, nullptr},
+    {"run_plan", as_cfunction(py_run_plan), METH_FASTCALL, nullptr},
+    {"same_params", as_cfunction(py_same_params), METH_FASTCALL, nullptr},
+    {"float_of", py_float_of, METH_O, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_frontend", nullptr, -1, methods, nullptr, nullptr,

@@ -218,7 +218,7 @@ __global__ __launch_bounds__(Cfg::kThreads, NS <= 2 ? Cfg::kMinWaves : 1) void c
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 
   // what the epilogue needs is fetched while the first operand stages are in flight
-  EpiPre pre;
+  EpiPreOf<kEpiPlain> pre;
   auto prefetch = [&]() { pre = epi_prefetch<Cfg>(p.epi, n0, p.O); };
   // this work-group's K slice: stages [kt0, kt0 + KT) (all of them without a split)
   const int kt_all = (p.K + Cfg::BK - 1) / Cfg::BK;
@@ -556,7 +556,7 @@ __global__ __launch_bounds__(512, 2) void conv3x3_patch_kernel(ConvArgs p) {
 #pragma unroll
   for (int st = 0; st < NS - 1; ++st) issue(st);
   MXQ_STAMP(5);
-  EpiPre pre = epi_prefetch<Cfg>(p.epi, n0, p.O);
+  EpiPreOf<kEpiPlain> pre = epi_prefetch<Cfg>(p.epi, n0, p.O);
   MXQ_STAMP(6);
 
   // this lane's output pixel and its patch pixel under tap (0, 0)
@@ -1199,7 +1199,7 @@ void conv_nhwc(void* stream, const int8_t* data, const int8_t* weight, const int
   e.min_bias = min_bias; e.max_bias = max_bias;
   e.out32 = out32; e.out8 = out8; e.outf = nullptr;
   e.res = nullptr; e.res_min = nullptr; e.res_max = nullptr;
-  e.sum_min_calib = 0.f; e.sum_max_calib = 0.f; e.sum_relu = 0; e.with_sum = 0;
+  e.sum_min_calib = 0.f; e.sum_max_calib = 0.f; e.sum_relu = 0; e.sum_requant = 0; e.with_sum = 0;
   e.omin = omin; e.omax = omax; e.rmin = rmin; e.rmax = rmax;
   e.relu = relu;
   float x = fabsf(min_calib), y = fabsf(max_calib);

@@ -188,6 +188,7 @@ void launch_fc(hipStream_t s, const int8_t* data, const int8_t* weight, int M, i
   switch (epi_mode(a.epi)) {
     case kEpiF32: fc_launch_f32(s, a, how, ws); break;
     case kEpiSum: fc_launch_sum(s, a, how, ws); break;
+    case kEpiSumRq: fc_launch_sum_requant(s, a, how, ws); break;
     default: fc_launch_plain(s, a, how, ws);
   }
 }
@@ -219,6 +220,7 @@ struct SumArgs {
   const float* res_max;
   float min_calib, max_calib;
   int relu;
+  int requant;
 };
 
 void fc_entry(void* stream, const int8_t* data, const int8_t* weight, const int8_t* bias, int M,
@@ -253,6 +255,7 @@ void fc_entry(void* stream, const int8_t* data, const int8_t* weight, const int8
   e.res_min = e.res_max = nullptr;
   e.sum_min_calib = e.sum_max_calib = 0.f;
   e.sum_relu = 0;
+  e.sum_requant = 0;
   e.with_sum = 0;
   if (sum != nullptr) {
     MXQ_CHECK((M == 0 || N == 0 || out8 != nullptr) && out32 == nullptr && out_f32 == nullptr,
@@ -267,6 +270,7 @@ void fc_entry(void* stream, const int8_t* data, const int8_t* weight, const int8
     e.sum_min_calib = sum->min_calib;
     e.sum_max_calib = sum->max_calib;
     e.sum_relu = sum->relu;
+    e.sum_requant = sum->requant;
     e.with_sum = 1;
   }
   e.omin = omin;
@@ -358,7 +362,26 @@ int mxq_quantized_fc_sum(void* stream, const int8_t* data, const int8_t* weight,
                          void* workspace, size_t workspace_bytes) {
   MXQ_API_BEGIN();
   const SumArgs sum = {residual, min_residual, max_residual, sum_min_calib, sum_max_calib,
-                       sum_relu};
+                       sum_relu, 0};
+  fc_entry(stream, data, weight, bias, M, N, K, min_data, max_data, min_weight, max_weight,
+           min_bias, max_bias, nullptr, omin, omax, out8, nullptr, rmin, rmax, 0, min_calib,
+           max_calib, workspace, workspace_bytes, GemmForce(), &sum);
+  MXQ_API_END();
+}
+
+int mxq_quantized_fc_sum_requant(void* stream, const int8_t* data, const int8_t* weight,
+                                 const int8_t* bias, int M, int N, int K, const float* min_data,
+                                 const float* max_data, const float* min_weight,
+                                 const float* max_weight, const float* min_bias,
+                                 const float* max_bias, const int8_t* residual,
+                                 const float* min_residual, const float* max_residual,
+                                 int8_t* out8, float* omin, float* omax, float* rmin, float* rmax,
+                                 float min_calib, float max_calib, float sum_min_calib,
+                                 float sum_max_calib, int sum_relu, void* workspace,
+                                 size_t workspace_bytes) {
+  MXQ_API_BEGIN();
+  const SumArgs sum = {residual, min_residual, max_residual, sum_min_calib, sum_max_calib,
+                       sum_relu, 1};
   fc_entry(stream, data, weight, bias, M, N, K, min_data, max_data, min_weight, max_weight,
            min_bias, max_bias, nullptr, omin, omax, out8, nullptr, rmin, rmax, 0, min_calib,
            max_calib, workspace, workspace_bytes, GemmForce(), &sum);
@@ -380,7 +403,7 @@ int mxq_test_quantized_fc_sum(void* stream, const int8_t* data, const int8_t* we
                               size_t workspace_bytes, int cfg, int splits, int stream_groups) {
   MXQ_API_BEGIN();
   const SumArgs sum = {residual, min_residual, max_residual, sum_min_calib, sum_max_calib,
-                       sum_relu};
+                       sum_relu, 0};
   GemmForce force;
   force.cfg = cfg;
   force.splits = splits;

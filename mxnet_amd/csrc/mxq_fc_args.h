@@ -1,6 +1,6 @@
-// What the fully-connected launcher hands to its kernels, and the three entry points of the
+// What the fully-connected launcher hands to its kernels, and the entry points of the
 // kernel translation units: the kernels are built once per epilogue mode (mxq_gemm.h:
-// kEpiPlain / kEpiF32 / kEpiSum), each mode in a file of its own so that they compile side
+// kEpiPlain ... kEpiSumRq), each mode in a file of its own so that they compile side
 // by side.
 #ifndef MXQ_FC_ARGS_H_
 #define MXQ_FC_ARGS_H_
@@ -34,10 +34,12 @@ struct FcLaunch {
 };
 
 // Launch the kernel of `how.cfg` built for the mode (mxq_fc_plain.hip, mxq_fc_f32.hip,
-// mxq_fc_sum.hip).  The caller has checked that the shape qualifies for the configuration.
+// mxq_fc_sum.hip, mxq_fc_sum_requant.hip).  The caller has checked that the shape qualifies for the configuration.
 void fc_launch_plain(hipStream_t s, const FcArgs& a, const FcLaunch& how, const Workspace& ws);
 void fc_launch_f32(hipStream_t s, const FcArgs& a, const FcLaunch& how, const Workspace& ws);
 void fc_launch_sum(hipStream_t s, const FcArgs& a, const FcLaunch& how, const Workspace& ws);
+void fc_launch_sum_requant(hipStream_t s, const FcArgs& a, const FcLaunch& how,
+                           const Workspace& ws);
 
 }  // namespace mxq
 #endif  // MXQ_FC_ARGS_H_

@@ -64,7 +64,7 @@ __global__ __launch_bounds__(Cfg::kThreads, NS <= 2 ? Cfg::kMinWaves : 1) void f
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 
   // what the epilogue needs is fetched while the first operand stages are in flight
-  EpiPre pre;
+  EpiPreOf<MODE> pre;
   auto prefetch = [&]() { pre = epi_prefetch<Cfg, MODE>(p.epi, n0, p.N); };
   v16i acc[Cfg::MI][Cfg::NI];
   // this work-group's K slice: stages [kt0, kt0 + KT) (all of them without a split)
@@ -118,9 +118,10 @@ typedef GemmCfg<256, 192, 128, 4, 2> CfgW192K; // 8 waves, wave tile 64 x 96
 // the next item's fragment requested before the current one is multiplied, weights read from
 // LDS, then the fused epilogue and a transpose of the int8 tile through the wave's own LDS
 // scratch.  No barrier after the weights are staged; waves only meet the memory system.
-// SUM: the residual operand FcArgs::epi.res is added to the int8 tile on its way out.
-template <int KS, int NI, bool SUM>
+// A sum MODE: the residual operand FcArgs::epi.res is added to the int8 tile on its way out.
+template <int KS, int NI, int MODE>
 __global__ __launch_bounds__(256, 2) void fc_stream_kernel(FcArgs p, int bn, int strips) {
+  constexpr bool SUM = epi_sums(MODE);
   constexpr int K = 32 * KS, CH = 2 * KS;  // bytes and 16-byte chunks per row
   constexpr int TN = 32 * NI, LD = TN + 16;
   constexpr int LPR = TN / 16, RPI = 64 / LPR;
@@ -138,11 +139,12 @@ __global__ __launch_bounds__(256, 2) void fc_stream_kernel(FcArgs p, int bn, int
         p.weight + static_cast<size_t>(n_begin + r) * K + c * 16);
   }
   const EpiScalars s = epi_scalars(p.epi);
-  SumRule rule = {0.0f, 0.0f, 1};
-  if (SUM)
-    rule = sum_rule(dev_maxabs(-p.epi.real_range, p.epi.real_range),
-                    dev_maxabs(*p.epi.res_min, *p.epi.res_max), p.epi.sum_min_calib,
-                    p.epi.sum_max_calib);
+  EpiPreOf<SUM ? MODE : kEpiSum> rules;
+  if constexpr (SUM)
+    rules.sum = epi_sum_rule<MODE>(p.epi);
+  else
+    rules.sum = SumRule{0.0f, 0.0f, 1};
+  const auto& rule = rules.sum;
   if (tid < cols) sbias[tid] = epi_bias32(p.epi, s, n_begin + tid);
   __syncthreads();
 
@@ -230,10 +232,16 @@ __global__ __launch_bounds__(256, 2) void fc_stream_kernel(FcArgs p, int bn, int
         v4i val = *reinterpret_cast<const v4i*>(stage + rr * LD + c16 * 16);
         if (SUM) {
 #pragma unroll
-          for (int w = 0; w < 4; ++w)
-            val[w] = static_cast<int>(
-                sum4<decltype(sum_relu)::value, decltype(sum_fast)::value>(
-                    static_cast<uint32_t>(val[w]), static_cast<uint32_t>(resv[it][w]), rule));
+          for (int w = 0; w < 4; ++w) {
+            constexpr bool kRelu = decltype(sum_relu)::value, kFast = decltype(sum_fast)::value;
+            const uint32_t x = static_cast<uint32_t>(val[w]);
+            const uint32_t y = static_cast<uint32_t>(resv[it][w]);
+            if constexpr (MODE == kEpiSumRq)
+              val[w] = static_cast<int>(kFast ? sum_requant4<kRelu>(x, y, rule)
+                                              : sum_requant4_general<kRelu>(x, y, rule));
+            else
+              val[w] = static_cast<int>(sum4<kRelu, kFast>(x, y, rule));
+          }
         }
         const int m = m_base + rr;
         if (m < p.M)
@@ -264,10 +272,10 @@ __global__ __launch_bounds__(256, 2) void fc_stream_kernel(FcArgs p, int bn, int
       for (int ks = 0; ks < KS; ++ks) fa[ks] = fa_next[ks];
     }
   }
-  if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) epilogue_ranges<SUM ? kEpiSum : kEpiPlain>(p.epi);
+  if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) epilogue_ranges<MODE>(p.epi);
 }
 
-template <int KS, int NI, bool SUM>
+template <int KS, int NI, int MODE>
 void launch_stream(hipStream_t s, const FcArgs& a, long cus, int groups_per_cu) {
   // the residual operand is read in 16-byte pieces, like the output is written
   MXQ_CHECK(a.epi.res == nullptr || aligned16(a.epi.res), "unaligned residual operand");
@@ -280,7 +288,7 @@ void launch_stream(hipStream_t s, const FcArgs& a, long cus, int groups_per_cu) 
   long gx = cus * groups_per_cu / ny;
   if (gx < 1) gx = 1;
   if (gx * 4 > items) gx = (items + 3) / 4;
-  hipLaunchKernelGGL((fc_stream_kernel<KS, NI, SUM>), dim3(static_cast<unsigned>(gx), ny),
+  hipLaunchKernelGGL((fc_stream_kernel<KS, NI, MODE>), dim3(static_cast<unsigned>(gx), ny),
                      dim3(256), 0, s, a, bn, strips);
   MXQ_LAUNCH_CHECK();
 }
@@ -314,14 +322,13 @@ void fc_launch_mode(hipStream_t s, const FcArgs& a, const FcLaunch& how, const W
     if constexpr (MODE == kEpiF32) {
       MXQ_CHECK(false, "the short-K streaming kernel has no float-output form");
     } else {
-      constexpr bool SUM = MODE == kEpiSum;
       const long cus = num_cus();
 #define MXQ_STREAM(NI)                                                             \
   do {                                                                             \
-    if (a.K == 32) launch_stream<1, NI, SUM>(s, a, cus, how.stream_groups);        \
-    else if (a.K == 64) launch_stream<2, NI, SUM>(s, a, cus, how.stream_groups);   \
-    else if (a.K == 128) launch_stream<4, NI, SUM>(s, a, cus, how.stream_groups);  \
-    else launch_stream<8, NI, SUM>(s, a, cus, how.stream_groups);                  \
+    if (a.K == 32) launch_stream<1, NI, MODE>(s, a, cus, how.stream_groups);        \
+    else if (a.K == 64) launch_stream<2, NI, MODE>(s, a, cus, how.stream_groups);   \
+    else if (a.K == 128) launch_stream<4, NI, MODE>(s, a, cus, how.stream_groups);  \
+    else launch_stream<8, NI, MODE>(s, a, cus, how.stream_groups);                  \
   } while (0)
       if (cfg == 61) MXQ_STREAM(2); else MXQ_STREAM(4);
 #undef MXQ_STREAM

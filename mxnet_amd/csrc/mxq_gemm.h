@@ -66,6 +66,7 @@ struct Epilogue {
   const float* res_max;
   float sum_min_calib, sum_max_calib;
   int sum_relu;
+  int sum_requant;         // the sum in int32 over its own range, then requantized (RequantRule)
   int with_sum;            // rmin / rmax report the sum's range (also for an empty output)
   float* omin;             // int32 output range
   float* omax;
@@ -188,15 +189,8 @@ __device__ __forceinline__ uint32_t pack_bytes(int a, int b, int c, int d) {
 // Four requantized outputs as one dword (first in byte 0).  (Converting the relu'd values as
 // unsigned and or-ing them without byte masks saves a quarter instruction per output and
 // measures the same: 19-layer stack 261.7 against 260.3 us.)
-// With the relu the four values are in [0, 127] and v_cvt_pk_u8_f32 can take the place of
-// the clamp's lower side, the truncating convert and the pack: it saturates at 0, writes
-// byte k of its destination, and rounds as the wave's float rounding mode says.  The mode
-// is switched to round-toward-zero for exactly the four converts (one asm statement, so
-// that no multiply or add of the requantization can be scheduled into the stretch) and
-// back: u = f * s + 0.5 itself is computed in round-to-nearest as before, only its
-// truncation changes hands.  6.25 VALU instructions per output instead of 7.
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
+// With the relu pack4_truncated takes the place of the clamp's lower side, the truncating
+// convert and the pack: 6.25 VALU instructions per output instead of 7.
 __device__ __forceinline__ uint32_t epi_requant_relu_pack(int a0, int a1, int a2, int a3,
                                                           const EpiScalars& s) {
   auto level = [&](int a) {
@@ -204,20 +198,8 @@ __device__ __forceinline__ uint32_t epi_requant_relu_pack(int a0, int a1, int a2
     const float u = f * s.qscale + 0.5f;
     return (u < 127.0f) ? u : 127.0f;   // the reference's min(|f| * s + 0.5, 127)
   };
-  const float u0 = level(a0), u1 = level(a1), u2 = level(a2), u3 = level(a3);
-  uint32_t w;
-  asm volatile(
-      "s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 3\n\t"
-      "v_cvt_pk_u8_f32 %0, %1, 0, 0\n\t"
-      "v_cvt_pk_u8_f32 %0, %2, 1, %0\n\t"
-      "v_cvt_pk_u8_f32 %0, %3, 2, %0\n\t"
-      "v_cvt_pk_u8_f32 %0, %4, 3, %0\n\t"
-      "s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 0"
-      : "=&v"(w)
-      : "v"(u0), "v"(u1), "v"(u2), "v"(u3));
-  return w;
+  return pack4_truncated(level(a0), level(a1), level(a2), level(a3));
 }
-#pragma clang diagnostic pop
 
 template <bool RELU>
 __device__ __forceinline__ uint32_t epi_requant_pack(int a0, int a1, int a2, int a3,
@@ -716,9 +698,23 @@ __device__ __forceinline__ void gemm_mainloop_dma(v16i (&acc)[Cfg::MI][Cfg::NI],
 constexpr int kEpiPlain = 0;  // out32 and / or out8
 constexpr int kEpiF32 = 1;    // Epilogue::outf
 constexpr int kEpiSum = 2;    // out8 with Epilogue::res added
+constexpr int kEpiSumRq = 3;  // ... in int32, then requantized
+constexpr bool epi_sums(int mode) { return mode == kEpiSum || mode == kEpiSumRq; }
 
 inline int epi_mode(const Epilogue& e) {
-  return e.outf != nullptr ? kEpiF32 : (e.res != nullptr ? kEpiSum : kEpiPlain);
+  if (e.res != nullptr) return e.sum_requant ? kEpiSumRq : kEpiSum;
+  return e.outf != nullptr ? kEpiF32 : kEpiPlain;
+}
+
+// The rule of a sum mode: a RequantRule for kEpiSumRq, else a SumRule.
+template <int MODE>
+__device__ __forceinline__ auto epi_sum_rule(const Epilogue& e) {
+  const float a = dev_maxabs(-e.real_range, e.real_range);
+  const float b = dev_maxabs(*e.res_min, *e.res_max);
+  if constexpr (MODE == kEpiSumRq)
+    return sum_requant_rule(a, b, e.sum_min_calib, e.sum_max_calib);
+  else
+    return sum_rule(a, b, e.sum_min_calib, e.sum_max_calib);
 }
 
 template <class Cfg, int MODE = kEpiPlain>
@@ -770,17 +766,20 @@ __device__ __forceinline__ void gemm_epilogue(v16i (&acc)[Cfg::MI][Cfg::NI], con
           for (int i = 0; i < 4; ++i) {
             q[i] = epi_requant(v[i], s, e.relu ? 0.0f : -127.0f);
           }
-          if (MODE == kEpiSum && e.res != nullptr && e.out8 != nullptr) {
-            const SumRule r = sum_rule(dev_maxabs(-e.real_range, e.real_range),
-                                       dev_maxabs(*e.res_min, *e.res_max), e.sum_min_calib,
-                                       e.sum_max_calib);
+          if (epi_sums(MODE) && e.res != nullptr && e.out8 != nullptr) {
+            const auto r = epi_sum_rule<MODE>(e);
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
               if (n + i < N) {
                 // the overflow-safe form serves every rule on this rarely taken path
                 const int b = static_cast<int>(e.res[off + i]);
-                const uint32_t v8 = e.sum_relu ? sum_one<true, false>(q[i], b, r)
-                                               : sum_one<false, false>(q[i], b, r);
+                uint32_t v8;
+                if constexpr (MODE == kEpiSumRq)
+                  v8 = static_cast<uint32_t>(e.sum_relu ? sum_requant_one<true>(q[i], b, r)
+                                                        : sum_requant_one<false>(q[i], b, r));
+                else
+                  v8 = e.sum_relu ? sum_one<true, false>(q[i], b, r)
+                                  : sum_one<false, false>(q[i], b, r);
                 e.out8[off + i] = static_cast<int8_t>(v8 & 0xffu);
               }
             }
@@ -823,17 +822,39 @@ __device__ __forceinline__ void gemm_epilogue(v16i (&acc)[Cfg::MI][Cfg::NI], con
 struct EpiPre {
   EpiScalars s;
   int bias32;
-  SumRule sum;  // the residual sum's scales (kernels built for it)
 };
+// with the residual sum's scales, for the kernels built for it
+template <int MODE>
+struct EpiPreOf : EpiPre {};
+template <>
+struct EpiPreOf<kEpiSum> : EpiPre {
+  SumRule sum;
+};
+template <>
+struct EpiPreOf<kEpiSumRq> : EpiPre {
+  RequantRule sum;
+};
+// four elements of the sum under a fast rule
+template <bool RELU>
+__device__ __forceinline__ uint32_t epi_sum4(uint32_t x, uint32_t, const EpiPre&) {
+  return x;
+}
+template <bool RELU>
+__device__ __forceinline__ uint32_t epi_sum4(uint32_t x, uint32_t y,
+                                             const EpiPreOf<kEpiSum>& pre) {
+  return sum4<RELU, true>(x, y, pre.sum);
+}
+template <bool RELU>
+__device__ __forceinline__ uint32_t epi_sum4(uint32_t x, uint32_t y,
+                                             const EpiPreOf<kEpiSumRq>& pre) {
+  return sum_requant4<RELU>(x, y, pre.sum);
+}
 template <class Cfg, int MODE = kEpiPlain>
-__device__ __forceinline__ EpiPre epi_prefetch(const Epilogue& e, int n0, int N) {
+__device__ __forceinline__ EpiPreOf<MODE> epi_prefetch(const Epilogue& e, int n0, int N) {
   static_assert(Cfg::kThreads >= Cfg::BN, "one thread per tile column");
-  EpiPre p;
+  EpiPreOf<MODE> p;
   p.s = epi_scalars(e);
-  p.sum = SumRule{0.0f, 0.0f, 1};
-  if (MODE == kEpiSum && e.res != nullptr)
-    p.sum = sum_rule(dev_maxabs(-e.real_range, e.real_range),
-                     dev_maxabs(*e.res_min, *e.res_max), e.sum_min_calib, e.sum_max_calib);
+  if constexpr (epi_sums(MODE)) p.sum = epi_sum_rule<MODE>(e);
   const int t = threadIdx.x;
   p.bias32 = (t < Cfg::BN && n0 + t < N) ? epi_bias32(e, p.s, n0 + t) : 0;
   return p;
@@ -856,8 +877,8 @@ struct EpiScratch {
 
 template <class Cfg, int RING_BYTES, int MODE = kEpiPlain>
 __device__ __forceinline__ void gemm_epilogue_lds(v16i (&acc)[Cfg::MI][Cfg::NI],
-                                                  const Epilogue& e, const EpiPre& pre, int m0,
-                                                  int n0, int M, int N, size_t ldo,
+                                                  const Epilogue& e, const EpiPreOf<MODE>& pre,
+                                                  int m0, int n0, int M, int N, size_t ldo,
                                                   v4i* lds_v) {
   typedef EpiScratch<Cfg> Scratch;
   static_assert(RING_BYTES >= Scratch::kNeed8, "stage ring too small for the epilogue transpose");
@@ -879,9 +900,9 @@ __device__ __forceinline__ void gemm_epilogue_lds(v16i (&acc)[Cfg::MI][Cfg::NI],
                        ((reinterpret_cast<uintptr_t>(e.out32) & 15u) == 0));
   // the sum's scales; a rule whose products could overflow goes the general way with the
   // unaligned outputs
-  const SumRule rule = pre.sum;
-  const bool fasts = MODE != kEpiSum || e.res == nullptr ||
-                     (((reinterpret_cast<uintptr_t>(e.res) & 15u) == 0) && rule.fast);
+  bool fasts = true;
+  if constexpr (epi_sums(MODE))
+    fasts = ((reinterpret_cast<uintptr_t>(e.res) & 15u) == 0) && pre.sum.fast;
   const bool fastf = MODE != kEpiF32 || e.outf == nullptr ||
                      ((N % 4 == 0) && (ldo % 4 == 0) &&
                       ((reinterpret_cast<uintptr_t>(e.outf) & 15u) == 0));
@@ -1076,9 +1097,9 @@ __device__ __forceinline__ void gemm_epilogue_lds(v16i (&acc)[Cfg::MI][Cfg::NI],
     constexpr int kPieces = TM * LPR;
     constexpr int kIters = (kPieces + 63) / 64;
     // the residual operand's pieces are fetched now, behind the requantization's arithmetic
-    v4i resv[MODE == kEpiSum ? kIters : 1];
-    if constexpr (MODE == kEpiSum) {
-      if (e.res != nullptr) {
+    v4i resv[epi_sums(MODE) ? kIters : 1];
+    if constexpr (epi_sums(MODE)) {
+      {
 #pragma unroll
         for (int it = 0; it < kIters; ++it) {
           const int piece = it * 64 + lane;
@@ -1125,35 +1146,34 @@ __device__ __forceinline__ void gemm_epilogue_lds(v16i (&acc)[Cfg::MI][Cfg::NI],
         v4i val = *reinterpret_cast<const v4i*>(stage + rr * LD + c16 * 16);
         if constexpr (SM != 0) {
 #pragma unroll
-          for (int w = 0; w < 4; ++w)
-            val[w] = static_cast<int>(sum4<SM == 2, true>(
-                static_cast<uint32_t>(val[w]), static_cast<uint32_t>(resv[it][w]), rule));
+          for (int w = 0; w < 4; ++w) {
+            const uint32_t x = static_cast<uint32_t>(val[w]);
+            const uint32_t y = static_cast<uint32_t>(resv[it][w]);
+            val[w] = static_cast<int>(epi_sum4<SM == 2>(x, y, pre));
+          }
         }
         const int m = m_base + rr, n = n_base + c16 * 16;
         if (m < M && n < N)
           epi_store16<decltype(stream)::value>(val, e.out8 + static_cast<size_t>(m) * ldo + n);
       }
     };
-    if constexpr (MODE == kEpiSum) {
-      if (e.res != nullptr) {
-        if (e.stream8) {
-          if (e.sum_relu)
-            store_tile(std::true_type(), std::integral_constant<int, 2>());
-          else
-            store_tile(std::true_type(), std::integral_constant<int, 1>());
-        } else {
-          if (e.sum_relu)
-            store_tile(std::false_type(), std::integral_constant<int, 2>());
-          else
-            store_tile(std::false_type(), std::integral_constant<int, 1>());
-        }
-        return;
+    if constexpr (epi_sums(MODE)) {
+      if (e.stream8) {
+        if (e.sum_relu)
+          store_tile(std::true_type(), std::integral_constant<int, 2>());
+        else
+          store_tile(std::true_type(), std::integral_constant<int, 1>());
+      } else {
+        if (e.sum_relu)
+          store_tile(std::false_type(), std::integral_constant<int, 2>());
+        else
+          store_tile(std::false_type(), std::integral_constant<int, 1>());
       }
-    }
-    if (e.stream8)
+    } else if (e.stream8) {
       store_tile(std::true_type(), std::integral_constant<int, 0>());
-    else
+    } else {
       store_tile(std::false_type(), std::integral_constant<int, 0>());
+    }
   }
 }
 
@@ -1294,9 +1314,15 @@ __device__ __forceinline__ void epilogue_ranges(const Epilogue& e) {
   *e.omax = s.max_out;
   // also for an output without elements, whose buffer pointer may be null
   if (e.rmin != nullptr && e.rmax != nullptr) {
-    if (MODE == kEpiSum && e.with_sum) {  // the sum's calibrated range, as quantized_elemwise_add reports it
-      *e.rmin = e.sum_min_calib;
-      *e.rmax = e.sum_max_calib;
+    if (epi_sums(MODE) && e.with_sum) {
+      if (e.sum_requant) {  // the requantized range
+        const float r = dev_maxabs(e.sum_min_calib, e.sum_max_calib);
+        *e.rmin = -r;
+        *e.rmax = r;
+      } else {  // the sum's calibrated range, as quantized_elemwise_add reports it
+        *e.rmin = e.sum_min_calib;
+        *e.rmax = e.sum_max_calib;
+      }
     } else {
       *e.rmin = -e.real_range;
       *e.rmax = e.real_range;

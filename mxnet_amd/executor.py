@@ -10,10 +10,16 @@ the way `SymbolBlock.register_op_hook(collector.collect, monitor_all=True)` does
 sees every operator output as `<node>_<output name>` and, with monitor_all, every
 operator input as `<node>_<argument name>`; operators without registered names get
 the decimal output index and `input<i>` (src/common/utils.cc:53-107).
+
+Without a hook, a graph of quantized operators runs as a plan (_plan.py): one native call per
+forward pass, the same outputs.
 """
 import torch
 
+from . import _frontend, _plan
 from . import operator as _operator
+
+_MAX_PLANS = 8  # input shape combinations an executor keeps a plan for
 
 
 def _tuple(text, n=2, default=None):
@@ -139,6 +145,8 @@ class Executor:
         self.monitor = None
         self.monitor_all = False
         self._nodes = {}
+        self._graph = None   # (symbol, its nodes, its heads)
+        self._plans = {}     # feed names, shapes and types -> (plan, parameters it read) or None
 
     def register_op_hook(self, callback, monitor_all=False):
         """callback(name, op_name, array) as in Block.register_op_hook."""
@@ -151,14 +159,50 @@ class Executor:
             node = self._nodes[i] = _operator.Node(op, name, **attrs)
         return node
 
+    def _structure(self):
+        if self._graph is None or self._graph[0] is not self.symbol:
+            self._graph = (self.symbol, self.symbol.nodes(), self.symbol.heads())
+            self._nodes, self._plans = {}, {}
+        return self._graph[1:]
+
+    def _plan_for(self, feed):
+        """The plan for these inputs, None where the graph has to be walked.  A plan holds
+        parameters in its own layout, so it lives as long as `params` holds the tensors it read,
+        unwritten."""
+        nodes, heads = self._structure()
+        key = tuple((name, v.shape, v.dtype, v.device) for name, v in feed.items())
+        if key in self._plans:
+            entry = self._plans[key]
+            if entry is None or _frontend.same_params(self.params, entry[1]):
+                return entry and entry[0]
+        if torch.cuda.is_current_stream_capturing():
+            return None
+        stream = torch.cuda.current_stream()
+        try:
+            entry = _plan.build(self, nodes, heads, feed, stream.cuda_stream)
+        except _operator.MXNetError:
+            entry = None  # the walk reports it
+        if entry is not None:
+            stream.synchronize()  # the laid-out weights may be read on any stream from here on
+        while len(self._plans) >= _MAX_PLANS:
+            self._plans.pop(next(iter(self._plans)))
+        self._plans[key] = entry
+        return entry and entry[0]
+
     def forward(self, **feed):
+        feed = {name: (v if isinstance(v, torch.Tensor) else torch.as_tensor(v)).to(self.device)
+                for name, v in feed.items()}
+        if self.monitor is None and feed:
+            tensors = {name: v.contiguous() for name, v in feed.items()}
+            plan = self._plan_for(tensors)
+            if plan is not None:
+                return _frontend.run_plan(plan, *tensors.values())
         values = []
-        nodes = self.symbol.nodes()
+        nodes, heads = self._structure()
         for i, (op, name, attrs, inputs) in enumerate(nodes):
             if op == "null":
                 if name in feed:
                     v = feed[name]
-                    v = (v if isinstance(v, torch.Tensor) else torch.as_tensor(v)).to(self.device)
                 elif name in self.params:
                     v = self.params[name]
                 else:
@@ -191,4 +235,4 @@ class Executor:
                 for k, arr in enumerate(outs):
                     out_name = out_names[k] if k < len(out_names) else str(k)
                     self.monitor("%s_%s" % (name, out_name), op, arr)
-        return [values[j][k] for j, k in self.symbol.heads()]
+        return [values[j][k] for j, k in heads]
