@@ -178,7 +178,9 @@ def quantized_fc_sum(data, weight, bias, residual, min_data, max_data, min_weigh
         cfg, splits, groups = force
         wsb = _SPLIT_WS_BYTES if splits > 1 else 0
         ws = _workspace(wsb, dev) if wsb else None
-        check(lib.mxq_test_quantized_fc_sum(*args, _ptr(ws), wsb, cfg, splits, groups))
+        call = (lib.mxq_test_quantized_fc_sum_requant if requant else
+                lib.mxq_test_quantized_fc_sum)
+        check(call(*args, _ptr(ws), wsb, cfg, splits, groups))
     return res
 
 

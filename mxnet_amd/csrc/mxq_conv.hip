@@ -16,6 +16,7 @@
 
 #include "../../include/mxq.h"
 #include "mxq_common.h"
+#include "mxq_few_tiles.h"
 #include "mxq_thin_transpose.h"
 #include "mxq_gemm.h"
 #include "mxq_tiles.h"
@@ -1123,6 +1124,11 @@ ConvPlan plan_conv(const ConvGeometry& g, bool aligned, const GemmForce& force) 
       return static_cast<long>((M + bm - 1) / bm) * ((O + bn - 1) / bn);
     };
     int auto_splits = 1;
+    if (dma_ok && few_tiles_wins(M, O, K, cus) && few_tiles_conv_ok(g.C, K, g.KH, g.KW)) {
+      plan.cfg = 63;
+      plan.splits = 1;
+      return plan;
+    }
     if (dma_ok) {
       switch (choose_tile(M, O, K, cus, true, &auto_splits)) {
         case Tile::kL8: plan.cfg = 11; break;
@@ -1153,6 +1159,25 @@ ConvPlan plan_conv(const ConvGeometry& g, bool aligned, const GemmForce& force) 
   }
   if (plan.splits <= 0) plan.splits = 1;
   return plan;
+}
+
+// Channels that are no multiple of 16: copies of both operands with the channels padded, where
+// the caller brought room for them (the loader of the register-staged kernels fetches such
+// channels byte by byte: 21 x 29 x 29 x 17 -> 64, 7 x 7, 690 us against 14).
+int conv_padded_c(const ConvGeometry& g) {
+  const int Cp = (g.C + 15) / 16 * 16;
+  const bool wanted = Cp != g.C && static_cast<long long>(g.N) * g.H * g.W * Cp < (1LL << 31) &&
+                      static_cast<long long>(g.O) * g.KH * g.KW * Cp < (1LL << 31) &&
+                      static_cast<long long>(g.N) * g.H * g.W * g.C >= 16 &&
+                      static_cast<long long>(g.O) * g.K >= 16;
+  return wanted ? Cp : 0;
+}
+size_t conv_padded_data(const ConvGeometry& g, int Cp) {
+  return (static_cast<size_t>(g.N) * g.H * g.W * Cp + 255) / 256 * 256;
+}
+size_t conv_padded_bytes(const ConvGeometry& g, int Cp) {
+  return conv_padded_data(g, Cp) +
+         (static_cast<size_t>(g.O) * g.KH * g.KW * Cp + 255) / 256 * 256;
 }
 
 size_t conv_plan_workspace(const ConvPlan& plan, const ConvGeometry& g) {
@@ -1218,6 +1243,23 @@ void conv_nhwc(void* stream, const int8_t* data, const int8_t* weight, const int
     launch_fc(s, data, weight, a.M, O, C, O, e, force, ws);
     return;
   }
+  if (const int Cp = force.cfg == 0 && C % 16 != 0 ? conv_padded_c(g) : 0) {
+    const size_t copies = conv_padded_bytes(g, Cp);
+    if (ws.ptr != nullptr && aligned16(ws.ptr) && ws.bytes >= copies) {
+      int8_t* d = static_cast<int8_t*>(ws.ptr);
+      int8_t* w = d + conv_padded_data(g, Cp);
+      launch_pad_rows(s, data, static_cast<long long>(N) * H * W, d, weight,
+                      static_cast<long long>(O) * KH * KW, w, C, Cp);
+      Workspace rest;
+      rest.ptr = d + copies;
+      rest.bytes = ws.bytes - copies;
+      conv_nhwc(stream, d, w, bias, N, H, W, Cp, O, KH, KW, stride_h, stride_w, pad_h, pad_w,
+                dilate_h, dilate_w, min_data, max_data, min_weight, max_weight, min_bias,
+                max_bias, out32, omin, omax, out8, rmin, rmax, relu, min_calib, max_calib, planar,
+                force, rest);
+      return;
+    }
+  }
   const bool aligned = (C % 16 == 0) && aligned16(data) && aligned16(weight);
   const long long data_bytes = static_cast<long long>(N) * H * W * C;
   const bool dma_ok = aligned && data_bytes < (1LL << 31) &&
@@ -1250,6 +1292,17 @@ void conv_nhwc(void* stream, const int8_t* data, const int8_t* weight, const int
     return;
   }
   const int cfg = plan.cfg, sp = plan.splits;
+  if (cfg == 63) {  // the few-tiles kernel; `splits` is the number of waves per tile
+    MXQ_CHECK(dma_ok && few_tiles_conv_ok(C, a.K, KH, KW),
+              "shape does not qualify for the few-tiles kernel");
+    FewTilesArgs f = {};
+    f.data = data; f.weight = weight; f.M = a.M; f.N = O; f.K = a.K; f.ldo = O; f.epi = e;
+    f.images = N; f.H = H; f.W = W; f.C = C; f.KW = KW; f.sh = a.sh; f.sw = a.sw; f.ph = a.ph;
+    f.pw = a.pw; f.dh = a.dh; f.dw = a.dw; f.OH = a.OH; f.OW = a.OW;
+    launch_few_tiles_conv(s, f,
+                          force.splits > 0 ? force.splits : few_tiles_waves(a.M, O, a.K, true));
+    return;
+  }
   if (cfg > 10) MXQ_CHECK(dma_ok, "shape does not qualify for the direct-to-LDS conv kernels");
   if (cfg <= 10) MXQ_CHECK(sp <= 1, "the register-staged kernels have no split-K form");
   switch (cfg) {
@@ -1317,6 +1370,10 @@ size_t mxq_quantized_conv_workspace(int N, int H, int W, int C, int O, int KH, i
     if (g.M == 0) return 0;
     if (g.is_fc)
       return fc_workspace_bytes(static_cast<int>(g.M), O, C, fused_int8_only != 0 && O % 16 == 0);
+    if (const int Cp = C % 16 != 0 ? conv_padded_c(g) : 0)
+      return conv_padded_bytes(g, Cp) +
+             mxq_quantized_conv_workspace(N, H, W, Cp, O, KH, KW, stride_h, stride_w, pad_h,
+                                          pad_w, dilate_h, dilate_w, fused_int8_only);
     return conv_plan_workspace(plan_conv(g, C % 16 == 0, GemmForce()), g);
   } catch (...) {
     return 0;

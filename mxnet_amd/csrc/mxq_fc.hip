@@ -12,6 +12,7 @@
 #include "../../include/mxq.h"
 #include "mxq_common.h"
 #include "mxq_fc_args.h"
+#include "mxq_few_tiles.h"
 #include "mxq_gemm.h"
 #include "mxq_tiles.h"
 
@@ -28,6 +29,7 @@ namespace mxq {
 //   57..59  128x64 and 64x128 with 128-byte stages, 64x64 with 256-byte stages
 //   60      256x192 with 128-byte stages (outputs whose width is a multiple of 192)
 //   61, 62  the short-K streaming kernel with 64- / 128-column strips
+//   71      the few-tiles kernel (any shape; here `splits` is the number of waves per tile)
 // Output tile of a direct-to-LDS configuration (what a split-K work-group leaves in the
 // workspace); false for every other configuration.
 bool fc_cfg_tile(int cfg, int& bm, int& bn) {
@@ -55,7 +57,8 @@ struct FcPlan {
 // multiple of 16 (what the streaming kernel stores).
 // `sum`: the residual-sum form, whose epilogue does twice the arithmetic per output.
 FcPlan plan_fc(int M, int N, int K, bool aligned, bool fused8, const GemmForce& force,
-               bool sum = false) {
+               bool sum = false,
+               bool requant = false) {
   FcPlan plan = {force.cfg, force.splits, force.stream_groups > 0 ? force.stream_groups : 2};
   const bool buf_ok = aligned && K >= 16 && static_cast<long long>(M) * K < (1LL << 31) &&
                       static_cast<long long>(N) * K < (1LL << 31);
@@ -66,6 +69,13 @@ FcPlan plan_fc(int M, int N, int K, bool aligned, bool fused8, const GemmForce& 
       return static_cast<long>((M + bm - 1) / bm) * ((N + bn - 1) / bn);
     };
     int auto_splits = 1;
+    if ((buf_ok && few_tiles_wins(M, N, K, cus)) ||
+        (!aligned && few_tiles_count(M, N) < (1L << 31) && static_cast<long long>(M) * K >= 16 &&
+         static_cast<long long>(N) * K >= 16)) {
+      plan.cfg = 71;
+      plan.splits = 0;
+      return plan;
+    }
     if (buf_ok) {
       switch (choose_tile(M, N, K, cus, false, &auto_splits)) {
         case Tile::kL8: plan.cfg = glb_ok ? 12 : 31; break;
@@ -95,8 +105,10 @@ FcPlan plan_fc(int M, int N, int K, bool aligned, bool fused8, const GemmForce& 
     // 256 x 128 tiles on 64-byte stages, 256 x 256 tiles on 128-byte stages are ahead once
     // they cover 0.56 of the CUs (12544 x 256 -> 1024: -1.9 us per layer) and 128 x 128
     // tiles otherwise (50176 x 128 -> 512: -1.2 us per layer).
+    // The requantized sum is another third of arithmetic: 128 x 128 tiles throughout (12544 x 256
+    // -> 1024 15.8 us against 16.8, 50176 x 128 -> 512 22.6 against 27.7).
     if (sum && plan.cfg == 41) {
-      if (K >= 256 && N > 128 && 16 * tiles(256, 256) >= 9 * cus)
+      if (!requant && K >= 256 && N > 128 && 16 * tiles(256, 256) >= 9 * cus)
         plan.cfg = 55;
       else
         plan.cfg = 43;
@@ -115,12 +127,28 @@ FcPlan plan_fc(int M, int N, int K, bool aligned, bool fused8, const GemmForce& 
       // groups in flight (200704 x 64 -> 256 inside the chain: -7 us per layer)
       if (sum && K <= 64) {
         plan.cfg = 61;
-        if (force.stream_groups <= 0) plan.stream_groups = 5;
+        if (force.stream_groups <= 0) plan.stream_groups = requant ? 4 : 5;
       }
     }
   }
-  if (plan.splits <= 0) plan.splits = 1;
+  if (plan.splits <= 0 && plan.cfg != 71) plan.splits = 1;
   return plan;
+}
+
+// Rows that are no multiple of 16 bytes: the few-tiles kernel reads them as they are, but a
+// shape of many tiles is better copied into padded rows and given to the tiled kernels, where the
+// caller brought room for the copies (K = 1237: 1024 x 1024 13.5 us against 11.2 with the copies,
+// 256 x 2048 9.2 against 10.6).
+int fc_padded_k(int M, int N, int K) {
+  const int Kp = (K + 15) / 16 * 16;
+  const bool wanted = Kp != K && K >= 64 && few_tiles_count(M, N) > 3L * num_cus() &&
+                      static_cast<long long>(M) * Kp < (1LL << 31) &&
+                      static_cast<long long>(N) * Kp < (1LL << 31);
+  return wanted ? Kp : 0;
+}
+size_t up256(long long x) { return static_cast<size_t>((x + 255) / 256 * 256); }
+size_t fc_padded_bytes(int M, int N, int Kp) {
+  return up256(static_cast<long long>(M) * Kp) + up256(static_cast<long long>(N) * Kp);
 }
 
 size_t fc_plan_workspace(const FcPlan& plan, int M, int N) {
@@ -163,13 +191,26 @@ void launch_fc(hipStream_t s, const int8_t* data, const int8_t* weight, int M, i
                       ldo % 16 == 0 && aligned16(epi.out8) &&
                       (epi.res == nullptr || aligned16(epi.res));
   const bool sum = epi.res != nullptr;
-  FcPlan plan = plan_fc(M, N, K, aligned, fused8, force, sum);
+  if (const int Kp = force.cfg == 0 && K % 16 != 0 ? fc_padded_k(M, N, K) : 0) {
+    const size_t copies = fc_padded_bytes(M, N, Kp);
+    if (ws.ptr != nullptr && aligned16(ws.ptr) && ws.bytes >= copies) {
+      int8_t* d = static_cast<int8_t*>(ws.ptr);
+      int8_t* w = d + up256(static_cast<long long>(M) * Kp);
+      launch_pad_rows(s, data, M, d, weight, N, w, K, Kp);
+      Workspace rest;
+      rest.ptr = d + copies;
+      rest.bytes = ws.bytes - copies;
+      launch_fc(s, d, w, M, N, Kp, ldo, epi, force, rest);
+      return;
+    }
+  }
+  FcPlan plan = plan_fc(M, N, K, aligned, fused8, force, sum, epi.sum_requant != 0);
   // a split the chooser proposed is dropped when the caller brought no room for it
   if (force.splits == 0 && plan.splits > 1 &&
       (ws.ptr == nullptr || !aligned16(ws.ptr) || ws.bytes < fc_plan_workspace(plan, M, N))) {
     GemmForce unsplit = force;
     unsplit.splits = 1;
-    plan = plan_fc(M, N, K, aligned, fused8, unsplit, sum);
+    plan = plan_fc(M, N, K, aligned, fused8, unsplit, sum, epi.sum_requant != 0);
   }
   const int cfg = plan.cfg;
   if (cfg >= 11 && cfg <= 16) MXQ_CHECK(glb_ok, "shape does not qualify for the DMA kernels");
@@ -183,6 +224,19 @@ void launch_fc(hipStream_t s, const int8_t* data, const int8_t* weight, int M, i
   }
   if (cfg >= 21 && cfg < 61)
     MXQ_CHECK(buf_ok, "shape does not qualify for the buffer-load DMA kernels");
+  if (cfg == 71) {
+    FewTilesArgs f = {};
+    f.data = data;
+    f.weight = weight;
+    f.M = M;
+    f.N = N;
+    f.K = K;
+    f.ldo = ldo;
+    f.epi = a.epi;
+    launch_few_tiles_fc(s, f, buf_ok,
+                        plan.splits > 0 ? plan.splits : few_tiles_waves(M, N, K, buf_ok));
+    return;
+  }
   if (cfg < 11) MXQ_CHECK(plan.splits <= 1, "the register-staged kernels have no split-K form");
   const FcLaunch how = {cfg, plan.splits, plan.stream_groups, aligned};
   switch (epi_mode(a.epi)) {
@@ -199,6 +253,8 @@ void launch_fc(hipStream_t s, const int8_t* data, const int8_t* weight, int M, i
 // sized by this query serves mxq_quantized_fc and mxq_quantized_fc_sum alike.
 size_t fc_workspace_bytes(int M, int N, int K, bool fused8) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
+  if (const int Kp = K % 16 != 0 ? fc_padded_k(M, N, K) : 0)
+    return fc_padded_bytes(M, N, Kp) + fc_workspace_bytes(M, N, Kp, fused8);
   const size_t plain =
       fc_plan_workspace(plan_fc(M, N, K, K % 16 == 0, fused8, GemmForce(), false), M, N);
   if (!fused8) return plain;
@@ -389,7 +445,7 @@ int mxq_quantized_fc_sum_requant(void* stream, const int8_t* data, const int8_t*
 }
 
 #ifdef MXQ_TEST_HOOKS
-// Test-only twin of mxq_quantized_fc_sum with the kernel variant pinned
+// Test-only twins of the two residual-sum entry points with the kernel variant pinned
 // (tests/mxq_test_hooks.h).
 int mxq_test_quantized_fc_sum(void* stream, const int8_t* data, const int8_t* weight,
                               const int8_t* bias, int M, int N, int K, const float* min_data,
@@ -404,6 +460,29 @@ int mxq_test_quantized_fc_sum(void* stream, const int8_t* data, const int8_t* we
   MXQ_API_BEGIN();
   const SumArgs sum = {residual, min_residual, max_residual, sum_min_calib, sum_max_calib,
                        sum_relu, 0};
+  GemmForce force;
+  force.cfg = cfg;
+  force.splits = splits;
+  force.stream_groups = stream_groups;
+  fc_entry(stream, data, weight, bias, M, N, K, min_data, max_data, min_weight, max_weight,
+           min_bias, max_bias, nullptr, omin, omax, out8, nullptr, rmin, rmax, 0, min_calib,
+           max_calib, workspace, workspace_bytes, force, &sum);
+  MXQ_API_END();
+}
+
+int mxq_test_quantized_fc_sum_requant(void* stream, const int8_t* data, const int8_t* weight,
+                              const int8_t* bias, int M, int N, int K, const float* min_data,
+                              const float* max_data, const float* min_weight,
+                              const float* max_weight, const float* min_bias,
+                              const float* max_bias, const int8_t* residual,
+                              const float* min_residual, const float* max_residual,
+                              int8_t* out8, float* omin, float* omax, float* rmin, float* rmax,
+                              float min_calib, float max_calib, float sum_min_calib,
+                              float sum_max_calib, int sum_relu, void* workspace,
+                              size_t workspace_bytes, int cfg, int splits, int stream_groups) {
+  MXQ_API_BEGIN();
+  const SumArgs sum = {residual, min_residual, max_residual, sum_min_calib, sum_max_calib,
+                       sum_relu, 1};
   GemmForce force;
   force.cfg = cfg;
   force.splits = splits;

@@ -849,12 +849,96 @@ __device__ __forceinline__ uint32_t epi_sum4(uint32_t x, uint32_t y,
                                              const EpiPreOf<kEpiSumRq>& pre) {
   return sum_requant4<RELU>(x, y, pre.sum);
 }
+// one element of the sum under any rule
+__device__ __forceinline__ int8_t epi_sum_one(int a, int, bool, const EpiPre&) {
+  return static_cast<int8_t>(a);
+}
+__device__ __forceinline__ int8_t epi_sum_one(int a, int b, bool relu,
+                                              const EpiPreOf<kEpiSum>& pre) {
+  const uint32_t v = relu ? sum_one<true, false>(a, b, pre.sum) : sum_one<false, false>(a, b, pre.sum);
+  return static_cast<int8_t>(v & 0xffu);
+}
+__device__ __forceinline__ int8_t epi_sum_one(int a, int b, bool relu,
+                                              const EpiPreOf<kEpiSumRq>& pre) {
+  return static_cast<int8_t>(relu ? sum_requant_one<true>(a, b, pre.sum)
+                                  : sum_requant_one<false>(a, b, pre.sum));
+}
+template <int MODE>
+__device__ __forceinline__ EpiPreOf<MODE> epi_prefetch_scalars(const Epilogue& e) {
+  EpiPreOf<MODE> p;
+  p.s = epi_scalars(e);
+  p.bias32 = 0;
+  if constexpr (epi_sums(MODE)) p.sum = epi_sum_rule<MODE>(e);
+  return p;
+}
+
+// One lane's four adjacent columns n ... n + 3 of row m, bias included, into every output the
+// launch has: vector stores where the row pitch allows them, element by element elsewhere.
+template <int MODE>
+__device__ __forceinline__ void epi_store_quad(const Epilogue& e, const EpiPreOf<MODE>& pre,
+                                               const int (&v)[4], int m, int n, int N,
+                                               size_t ldo) {
+  const bool full = (N & 3) == 0 && (ldo & 3) == 0;  // then n + 3 < N as well
+  const size_t off = static_cast<size_t>(m) * ldo + n;
+  if (MODE == kEpiPlain && e.out32 != nullptr) {
+    if (e.plane > 0) {
+      const int img = m / e.plane, pix = m - img * e.plane;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (n + i < N) e.out32[(static_cast<size_t>(img) * N + (n + i)) * e.plane + pix] = v[i];
+    } else if (full && (reinterpret_cast<uintptr_t>(e.out32) & 15u) == 0) {
+      *reinterpret_cast<v4i*>(e.out32 + off) = v4i{v[0], v[1], v[2], v[3]};
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (n + i < N) e.out32[off + i] = v[i];
+    }
+  }
+  if (MODE == kEpiPlain && e.out8 == nullptr) return;
+  const float lo = e.relu ? 0.0f : -127.0f;
+  int q[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) q[i] = epi_requant(v[i], pre.s, lo);
+  if (MODE == kEpiF32) {
+    int* of = reinterpret_cast<int*>(e.outf);
+    if (full && (reinterpret_cast<uintptr_t>(e.outf) & 15u) == 0) {
+      *reinterpret_cast<v4i*>(of + off) =
+          v4i{epi_dequant_bits(q[0], pre.s), epi_dequant_bits(q[1], pre.s),
+              epi_dequant_bits(q[2], pre.s), epi_dequant_bits(q[3], pre.s)};
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (n + i < N) of[off + i] = epi_dequant_bits(q[i], pre.s);
+    }
+    return;
+  }
+  const bool dwords = full && (reinterpret_cast<uintptr_t>(e.out8) & 3u) == 0 &&
+                      (!epi_sums(MODE) || (reinterpret_cast<uintptr_t>(e.res) & 3u) == 0);
+  if (dwords) {
+    if (epi_sums(MODE)) {
+      const uint32_t r = *reinterpret_cast<const uint32_t*>(e.res + off);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        q[i] = epi_sum_one(q[i], static_cast<int8_t>((r >> (8 * i)) & 0xffu), e.sum_relu != 0,
+                           pre);
+    }
+    *reinterpret_cast<uint32_t*>(e.out8 + off) = pack_bytes(q[0], q[1], q[2], q[3]);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if (n + i >= N) continue;
+      int x = q[i];
+      if (epi_sums(MODE))
+        x = epi_sum_one(x, static_cast<int>(e.res[off + i]), e.sum_relu != 0, pre);
+      e.out8[off + i] = static_cast<int8_t>(x);
+    }
+  }
+}
+
 template <class Cfg, int MODE = kEpiPlain>
 __device__ __forceinline__ EpiPreOf<MODE> epi_prefetch(const Epilogue& e, int n0, int N) {
   static_assert(Cfg::kThreads >= Cfg::BN, "one thread per tile column");
-  EpiPreOf<MODE> p;
-  p.s = epi_scalars(e);
-  if constexpr (epi_sums(MODE)) p.sum = epi_sum_rule<MODE>(e);
+  EpiPreOf<MODE> p = epi_prefetch_scalars<MODE>(e);
   const int t = threadIdx.x;
   p.bias32 = (t < Cfg::BN && n0 + t < N) ? epi_bias32(e, p.s, n0 + t) : 0;
   return p;
@@ -906,9 +990,15 @@ __device__ __forceinline__ void gemm_epilogue_lds(v16i (&acc)[Cfg::MI][Cfg::NI],
   const bool fastf = MODE != kEpiF32 || e.outf == nullptr ||
                      ((N % 4 == 0) && (ldo % 4 == 0) &&
                       ((reinterpret_cast<uintptr_t>(e.outf) & 15u) == 0));
-  if (__builtin_expect(!(fast8 && fast32 && fastf && fasts), 0)) {
-    gemm_epilogue<Cfg, MODE>(acc, e, m_base, n_base, M, N, ldo);
-    return;
+  // A kernel of a sum mode writes nothing but the int8 tile: where that cannot leave in 16-byte
+  // pieces, it leaves byte by byte from the staged copy below.  Without the element-wise
+  // epilogue in it the 256 x 256 tile keeps its accumulators in registers (with it 768 bytes of
+  // scratch per lane: 12544 x 256 -> 1024 43 us).
+  if constexpr (!epi_sums(MODE)) {
+    if (__builtin_expect(!(fast8 && fast32 && fastf), 0)) {
+      gemm_epilogue<Cfg, MODE>(acc, e, m_base, n_base, M, N, ldo);
+      return;
+    }
   }
   char* lds = reinterpret_cast<char*>(lds_v);
   int* sbias = reinterpret_cast<int*>(lds);
@@ -1099,7 +1189,7 @@ __device__ __forceinline__ void gemm_epilogue_lds(v16i (&acc)[Cfg::MI][Cfg::NI],
     // the residual operand's pieces are fetched now, behind the requantization's arithmetic
     v4i resv[epi_sums(MODE) ? kIters : 1];
     if constexpr (epi_sums(MODE)) {
-      {
+      if (fast8 && fasts) {
 #pragma unroll
         for (int it = 0; it < kIters; ++it) {
           const int piece = it * 64 + lane;
@@ -1158,6 +1248,18 @@ __device__ __forceinline__ void gemm_epilogue_lds(v16i (&acc)[Cfg::MI][Cfg::NI],
       }
     };
     if constexpr (epi_sums(MODE)) {
+      if (__builtin_expect(!(fast8 && fasts), 0)) {
+#pragma unroll 1
+        for (int i = lane; i < TM * TN; i += 64) {
+          const int rr = i / TN, c = i - rr * TN;
+          const int m = m_base + rr, n = n_base + c;
+          if (m >= M || n >= N) continue;
+          const size_t off = static_cast<size_t>(m) * ldo + n;
+          const int a = static_cast<int8_t>(stage[rr * LD + c]);
+          e.out8[off] = epi_sum_one(a, static_cast<int>(e.res[off]), e.sum_relu != 0, pre);
+        }
+        return;
+      }
       if (e.stream8) {
         if (e.sum_relu)
           store_tile(std::true_type(), std::integral_constant<int, 2>());
