@@ -2,7 +2,8 @@
 reads like `mx.nd.contrib.quantize_v2(...)` (and the `_npx_*` aliases like
 `mx.npx.requantize`).  Same positional tensors, same keyword attributes, same
 outputs; everything runs through the C++ operator host."""
-from .operator import invoke
+from . import operator  # noqa: F401  (registers the exception classes of the call path)
+from ._frontend import invoke
 
 
 def quantize(data, min_range, max_range, out_type="uint8"):

@@ -70,7 +70,7 @@ void infer_types(const Node* n, std::vector<int>* in, std::vector<int>* out) {
 
 mxnet::TShape to_shape(int ndim, const int64_t* dims) {
   if (ndim < 0) return mxnet::TShape();
-  return mxnet::TShape(std::vector<mxnet::index_t>(dims, dims + ndim));
+  return mxnet::TShape(dims, dims + ndim);
 }
 
 std::string join(const std::vector<std::string>& v) {

@@ -141,32 +141,55 @@ typedef int64_t index_t;
 
 // Shape with numpy semantics: ndim() == -1 is an unknown shape, a dimension of
 // -1 an unknown extent (include/mxnet/tuple.h).
+// Up to kInline extents lie in the object itself: a call of an operator makes a dozen of these.
 class TShape {
  public:
   TShape() : ndim_(-1) {}
-  TShape(int ndim, index_t value) : ndim_(ndim), d_(ndim > 0 ? ndim : 0, value) {}
-  TShape(std::initializer_list<index_t> l) : ndim_(static_cast<int>(l.size())), d_(l) {}
-  explicit TShape(const std::vector<index_t>& v) : ndim_(static_cast<int>(v.size())), d_(v) {}
+  TShape(int ndim, index_t value) : ndim_(ndim) {
+    reserve();
+    for (int i = 0; i < ndim_; ++i) begin()[i] = value;
+  }
+  TShape(std::initializer_list<index_t> l) : TShape(l.begin(), l.end()) {}
+  explicit TShape(const std::vector<index_t>& v) : TShape(v.data(), v.data() + v.size()) {}
+  TShape(const index_t* first, const index_t* last) : ndim_(static_cast<int>(last - first)) {
+    reserve();
+    for (int i = 0; i < ndim_; ++i) begin()[i] = first[i];
+  }
   int ndim() const { return ndim_; }
-  index_t& operator[](int i) { return d_.at(i); }
-  const index_t& operator[](int i) const { return d_.at(i); }
+  index_t& operator[](int i) { return begin()[check(i)]; }
+  const index_t& operator[](int i) const { return begin()[check(i)]; }
   size_t Size() const {
     size_t s = 1;
-    for (int i = 0; i < ndim_; ++i) s *= static_cast<size_t>(d_[i]);
+    for (int i = 0; i < ndim_; ++i) s *= static_cast<size_t>(begin()[i]);
     return ndim_ < 0 ? 0 : s;
   }
   index_t ProdShape(int b, int e) const {
     index_t s = 1;
-    for (int i = b; i < e; ++i) s *= d_[i];
+    for (int i = b; i < e; ++i) s *= (*this)[i];
     return s;
   }
-  bool operator==(const TShape& o) const { return ndim_ == o.ndim_ && d_ == o.d_; }
+  bool operator==(const TShape& o) const {
+    if (ndim_ != o.ndim_) return false;
+    for (int i = 0; i < ndim_; ++i)
+      if (begin()[i] != o.begin()[i]) return false;
+    return true;
+  }
   bool operator!=(const TShape& o) const { return !(*this == o); }
-  const std::vector<index_t>& data() const { return d_; }
 
  private:
+  static constexpr int kInline = 6;
+  index_t* begin() { return ndim_ > kInline ? more_.data() : few_; }
+  const index_t* begin() const { return ndim_ > kInline ? more_.data() : few_; }
+  void reserve() {
+    if (ndim_ > kInline) more_.resize(ndim_);
+  }
+  int check(int i) const {
+    if (i < 0 || i >= ndim_) throw std::out_of_range("TShape index");
+    return i;
+  }
   int ndim_;
-  std::vector<index_t> d_;
+  index_t few_[kInline] = {};
+  std::vector<index_t> more_;
 };
 inline std::ostream& operator<<(std::ostream& os, const TShape& s) {
   if (s.ndim() < 0) return os << "None";
