@@ -458,6 +458,219 @@ void launch_conv3x3_rows(hipStream_t s, const ConvArgs& a) {
   MXQ_LAUNCH_CHECK();
 }
 
+// ---- few-tap convolution over 16 channels, straight from memory -------------------------
+// An image's first layer (16 channels, usually 12 real ones in space-to-depth form) has a
+// reduction of one 16-byte piece per tap: 256 bytes for a 7 x 7 stride-2 stem.  As tiles of the
+// implicit GEMM that is 12544 work-groups of four stages, each with its own prologue, im2col
+// gather through LDS and epilogue (batch 64, 224 x 224: 57 us).  Consecutive output pixels of a
+// row read consecutive 16-byte pixels, so the MFMA's activation fragment (32 pixels by two taps)
+// is one coalesced load per lane and needs no LDS at all.  A work-group parks the weights in LDS
+// once and walks a contiguous run of pixels, 32 at a time per wave, the next 32 pixels' fragments
+// requested before the current ones are multiplied: 27 us, of which the matrix products, the
+// requantization's arithmetic and the 64 MB of memory traffic need 11 to 12 each.
+// int8 output with the fused requantize; `strips` groups of 32 * NI output channels.
+struct TapArgs {
+  ConvArgs c;
+  int items_per_group;  // 32-pixel tiles times strips that one work-group walks
+  int strips;
+};
+
+template <int KS, int NI>
+__global__ __launch_bounds__(256, KS > 5 ? 3 : 4) void conv_taps_kernel(TapArgs t) {
+  const ConvArgs& p = t.c;
+  constexpr int TN = 32 * NI, LD = TN + 16, LPR = TN / 16, RPI = 64 / LPR;
+  constexpr int CH = 2 * KS, PITCH = CH | 1;  // 16-byte pieces per weight row; odd against banks
+  extern __shared__ __attribute__((aligned(16))) char taps_lds[];
+  const int rows = t.strips * TN;
+  v4i* wl = reinterpret_cast<v4i*>(taps_lds);                                   // [rows][PITCH]
+  int* sbias = reinterpret_cast<int*>(wl + rows * PITCH);                       // [rows]
+  char* stage_all = reinterpret_cast<char*>(sbias + rows);                      // [4][32 * LD]
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lrow = lane & 31, lgrp = lane >> 5;
+  const int taps = p.KH * p.KW;
+  for (int i = tid; i < rows * CH; i += 256) {
+    const int o = i / CH, c = i - o * CH;
+    v4i w = {0, 0, 0, 0};
+    if (o < p.O && c < taps)
+      w = *reinterpret_cast<const v4i*>(p.weight + (static_cast<size_t>(o) * taps + c) * 16);
+    wl[o * PITCH + c] = w;
+  }
+  const EpiScalars s = epi_scalars(p.epi);
+  for (int i = tid; i < rows; i += 256) sbias[i] = i < p.O ? epi_bias32(p.epi, s, i) : 0;
+  __syncthreads();
+
+  // this lane's taps: 2 * ks + lane / 32 (taps past the last one meet zero weights; they re-read
+  // the window's first pixel)
+  int dih[KS], diw[KS], toff[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    const int tap = 2 * ks + lgrp < taps ? 2 * ks + lgrp : 0;
+    const int kh = tap / p.KW, kw = tap - kh * p.KW;
+    dih[ks] = kh * p.dh;
+    diw[ks] = kw * p.dw;
+    toff[ks] = (dih[ks] * p.W + diw[ks]) * 16;
+  }
+  const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<int8_t*>(p.data), 0, static_cast<uint32_t>(p.N) * p.H * p.W * 16, 0x00020000);
+  const int reach_h = (p.KH - 1) * p.dh, reach_w = (p.KW - 1) * p.dw;
+  const int tiles = (p.M + 31) / 32, items = tiles * t.strips;
+  int item = blockIdx.x * t.items_per_group + wave;
+  const int end = (blockIdx.x + 1) * t.items_per_group < items
+                      ? (blockIdx.x + 1) * t.items_per_group : items;
+  // the lane's output pixel, moved on from item to item without a division
+  const int plane = p.OH * p.OW;
+  int tile = item / t.strips, strip = item - tile * t.strips;
+  int n, oh, ow;
+  {
+    const int m = tile * 32 + lrow;
+    n = m / plane;
+    const int rem = m - n * plane;
+    oh = rem / p.OW;
+    ow = rem - oh * p.OW;
+  }
+  auto advance = [&](int by) {  // by tiles
+    if (by == 0) return;
+    ow += by * 32;
+    while (ow >= p.OW) {
+      ow -= p.OW;
+      if (++oh == p.OH) {
+        oh = 0;
+        ++n;
+      }
+    }
+  };
+  auto load_a = [&](v4i (&f)[KS]) {
+    const int ih0 = oh * p.sh - p.ph, iw0 = ow * p.sw - p.pw;
+    const int base = ((n * p.H + ih0) * p.W + iw0) * 16;
+    const bool live = n < p.N;
+    const bool inside = live && ih0 >= 0 && iw0 >= 0 && ih0 + reach_h < p.H && iw0 + reach_w < p.W;
+    if (__all(inside)) {
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+        f[ks] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(
+                                            rsrc, static_cast<uint32_t>(base + toff[ks]), 0, 0));
+    } else {
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        const bool ok = live &&
+                        static_cast<unsigned>(ih0 + dih[ks]) < static_cast<unsigned>(p.H) &&
+                        static_cast<unsigned>(iw0 + diw[ks]) < static_cast<unsigned>(p.W);
+        f[ks] = __builtin_bit_cast(
+            v4i, __builtin_amdgcn_raw_buffer_load_b128(
+                     rsrc, ok ? static_cast<uint32_t>(base + toff[ks]) : kOutOfRange, 0, 0));
+      }
+    }
+  };
+  char* stage = stage_all + wave * 32 * LD;
+  const bool relu = p.epi.relu != 0, stream8 = p.epi.stream8 != 0;
+  v4i fa[KS];
+  if (item < end) load_a(fa);
+  for (; item < end; item += 4) {
+    const int m_base = tile * 32, s0 = strip * TN;
+    v4i fa_next[KS];
+    const bool more = item + 4 < end;
+    if (more) {
+      const int next = (item + 4) / t.strips;
+      advance(next - tile);
+      strip = item + 4 - next * t.strips;
+      tile = next;
+      load_a(fa_next);
+    }
+    v16i acc[NI];
+#pragma unroll
+    for (int ni = 0; ni < NI; ++ni)
+#pragma unroll
+      for (int vq = 0; vq < 4; ++vq) {
+        const v4i b = *reinterpret_cast<const v4i*>(sbias + s0 + ni * 32 + 8 * vq + 4 * lgrp);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[ni][4 * vq + i] = b[i];
+      }
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+      for (int ni = 0; ni < NI; ++ni)
+        acc[ni] = __builtin_amdgcn_mfma_i32_32x32x32_i8(
+            wl[(s0 + ni * 32 + lrow) * PITCH + 2 * ks + lgrp], fa[ks], acc[ni], 0, 0, 0);
+    auto requantize_tile = [&](auto with_relu) {
+#pragma unroll
+      for (int ni = 0; ni < NI; ++ni)
+#pragma unroll
+        for (int vq = 0; vq < 4; ++vq)
+          *reinterpret_cast<uint32_t*>(stage + lrow * LD + ni * 32 + 8 * vq + 4 * lgrp) =
+              epi_requant_pack<decltype(with_relu)::value>(acc[ni][4 * vq], acc[ni][4 * vq + 1],
+                                                           acc[ni][4 * vq + 2],
+                                                           acc[ni][4 * vq + 3], s);
+    };
+    if (relu)
+      requantize_tile(std::true_type());
+    else
+      requantize_tile(std::false_type());
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_wave_barrier();
+    auto store_tile = [&](auto stream) {
+#pragma unroll
+      for (int it = 0; it < 32 / RPI; ++it) {
+        const int rr = it * RPI + lane / LPR, c16 = lane % LPR;
+        const v4i val = *reinterpret_cast<const v4i*>(stage + rr * LD + c16 * 16);
+        const int m = m_base + rr, o = s0 + c16 * 16;
+        if (m < p.M && o < p.O)
+          epi_store16<decltype(stream)::value>(val,
+                                               p.epi.out8 + static_cast<size_t>(m) * p.O + o);
+      }
+    };
+    if (stream8)
+      store_tile(std::true_type());
+    else
+      store_tile(std::false_type());
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_wave_barrier();
+    if (more) {
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) fa[ks] = fa_next[ks];
+    }
+  }
+  if (blockIdx.x == 0 && tid == 0) epilogue_ranges(p.epi);
+}
+
+bool conv_taps_ok(const ConvArgs& a) {
+  const long long data_bytes = static_cast<long long>(a.N) * a.H * a.W * a.C;
+  return a.C == 16 && a.KH * a.KW <= 16 && a.KH * a.KW > 1 && a.O % 16 == 0 && a.O <= 128 &&
+         a.epi.out32 == nullptr && a.epi.out8 != nullptr && aligned16(a.data) &&
+         aligned16(a.weight) && aligned16(a.epi.out8) && data_bytes < (1LL << 31);
+}
+
+template <int KS, int NI>
+void launch_taps(hipStream_t s, const ConvArgs& a) {
+  TapArgs t;
+  t.c = a;
+  t.strips = (a.O + 32 * NI - 1) / (32 * NI);
+  const int rows = t.strips * 32 * NI;
+  const long items = static_cast<long>((a.M + 31) / 32) * t.strips;
+  // as many work-groups as the CUs hold at once; runs of whole rounds of the four waves
+  const long groups = (KS > 5 ? 3L : 4L) * num_cus();
+  long per = ((items + groups - 1) / groups + 3) / 4 * 4;
+  t.items_per_group = static_cast<int>(per);
+  const size_t lds = static_cast<size_t>(rows) * ((2 * KS) | 1) * 16 + rows * 4 +
+                     4 * 32 * (32 * NI + 16);
+  hipLaunchKernelGGL((conv_taps_kernel<KS, NI>),
+                     dim3(static_cast<unsigned>((items + per - 1) / per)), dim3(256), lds, s, t);
+  MXQ_LAUNCH_CHECK();
+}
+
+void launch_conv_taps(hipStream_t s, const ConvArgs& a) {
+  const int ks = (a.KH * a.KW + 1) / 2;
+#define MXQ_TAPS(KS)                  \
+  do {                                \
+    if (a.O <= 32)                    \
+      launch_taps<KS, 1>(s, a);       \
+    else                              \
+      launch_taps<KS, 2>(s, a);       \
+  } while (0)
+  if (ks <= 2) MXQ_TAPS(2); else if (ks <= 5) MXQ_TAPS(5); else MXQ_TAPS(8);
+#undef MXQ_TAPS
+}
+
 // ---- 3 x 3 convolution with the input patch resident in LDS -------------------------
 // The implicit GEMM above stages every input pixel nine times, once per tap, through the
 // CU's 64 bytes per clock from L1 into LDS, which is what bounds every tile below 256 x 256.
@@ -1279,6 +1492,14 @@ void conv_nhwc(void* stream, const int8_t* data, const int8_t* weight, const int
     MXQ_CHECK(conv3x3_rows_ok(a), "shape does not qualify for the parked-weights 3x3 kernel");
     MXQ_CHECK(plan.splits <= 1 || force.splits == 0, "the 3x3 row kernel has no split-K form");
     launch_conv3x3_rows(s, a);
+    return;
+  }
+  // 64: the few-tap kernel; chosen once two waves of every SIMD have an item (4 x 4 taps, 64
+  // outputs: 25088 pixels 5.6 us tiled and 5.1 here, 12544 pixels 5.1 both)
+  if (plan.cfg == 64 || (force.cfg == 0 && plan.splits <= 1 && conv_taps_ok(a) &&
+                         a.M >= 64L * num_cus())) {
+    MXQ_CHECK(conv_taps_ok(a), "shape does not qualify for the few-tap kernel");
+    launch_conv_taps(s, a);
     return;
   }
   // 62: the resident-patch 3 x 3 kernel; chosen where it was measured ahead of the tiled

@@ -3,10 +3,12 @@ can go wrong: rows and columns around the 32 x 32 tile, reductions around the 12
 the 16-byte piece, operands off every mark up to the last byte of their buffer.  Products are
 exact in float64, so the int32 output is compared with one; the other outputs with the operators
 behind it."""
+import ctypes
+
 import pytest
 import torch
 
-from mxnet_amd import capi
+from mxnet_amd import _lib, capi
 
 pytestmark = pytest.mark.gpu
 
@@ -114,3 +116,43 @@ def test_convolutions_over_unaligned_channels(n, h, w, c, o, k, stride, off):
     assert torch.equal(got["out32"], want)
     q = capi.requantize(got["out32"], got["omin"], got["omax"], -20.0, 20.0)[0]
     assert torch.equal(got["out8"], q)
+
+
+@pytest.mark.parametrize("n,h,w,o,k,stride,pad,dilate", [
+    (3, 13, 11, 64, (4, 4), 1, 1, 1), (2, 9, 40, 48, (3, 3), 1, 1, 1), (1, 33, 1, 16, (2, 1), 1, 0, 1),
+    (5, 7, 6, 128, (4, 4), 2, 3, 1), (2, 21, 19, 112, (3, 2), 1, 2, 3), (4, 1, 16, 32, (1, 16), 1, 5, 1),
+    (7, 1, 1, 96, (3, 3), 1, 1, 1), (6, 80, 77, 64, (4, 4), 1, 1, 1)])
+def test_convolutions_of_few_taps(n, h, w, o, k, stride, pad, dilate):
+    g = torch.Generator(device="cuda").manual_seed(h * w + o)
+    x, wt, b = int8(g, 0, n, h, w, 16), int8(g, 0, o, *k, 16), int8(g, 0, o)
+    args = scalars(*RANGES, -0.5, 0.5)
+    conv = dict(stride=(stride,) * 2, pad=(pad,) * 2, dilate=(dilate,) * 2, calib=(-30.0, 20.0))
+    ref = capi.quantized_conv_nhwc(x, wt, None, *args[:4], **conv)
+    assert torch.equal(ref["out32"], conv_exact(x, wt, *(conv[a] for a in ("stride", "pad", "dilate"))))
+    for bias, relu in ((None, True), (b, False), (b, True)):
+        a = args if bias is not None else args[:4]
+        ref = capi.quantized_conv_nhwc(x, wt, bias, *a, relu=relu, force=(4, 1), **conv)
+        got = capi.quantized_conv_nhwc(x, wt, bias, *a, relu=relu, want_int32=False, force=(64, 1),
+                                       **conv)
+        for key in ("out8", "omin", "omax", "rmin", "rmax"):
+            assert torch.equal(got[key], ref[key]), key
+
+
+@pytest.mark.parametrize("c", [1, 2, 3, 4, 5])
+@pytest.mark.parametrize("n,h,w,off", [(2, 7, 6, 1), (1, 8, 8, 0), (3, 5, 9, 1), (1, 1, 1, 0)])
+def test_quantize_with_space_to_depth(c, n, h, w, off):
+    g = torch.Generator(device="cuda").manual_seed(c * h * w)
+    x = torch.randn(n, c, h, w, device="cuda", generator=g) * 2
+    q = capi.quantize_v2(x, "int8", -3.0, 3.0)[0]
+    cp = (4 * c + 15) // 16 * 16
+    oh, ow = (h + off + 1) // 2, (w + off + 1) // 2
+    out = torch.empty(n, oh, ow, cp, dtype=torch.int8, device="cuda")
+    ranges = torch.empty(2, device="cuda")
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    _lib.check(_lib.lib.mxq_quantize_to_nhwc(
+        stream, x.data_ptr(), out.data_ptr(), ranges.data_ptr(), ranges.data_ptr() + 4, n, c, h, w,
+        cp, 1, off, off, -3.0, 3.0))
+    want = torch.empty_like(out)
+    _lib.check(_lib.lib.mxq_nchw_to_s2d_nhwc_i8(stream, q.data_ptr(), want.data_ptr(), n, c, h, w,
+                                                off, off, cp))
+    assert torch.equal(out, want)
