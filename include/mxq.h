@@ -349,7 +349,8 @@ int mxq_quantized_fc_sum(void* stream, const int8_t* data, const int8_t* weight,
  * over (sum_min_calib, sum_max_calib) (_contrib_requantize), which is the graph QuantizeGraph
  * makes of an elemwise_add between two layers; sum_relu != 0 clamps at zero.  out8 is
  * bit-identical to the operators one after the other; rmin / rmax receive the requantized
- * range. */
+ * range.
+ * `pairs` is null, or what mxq_sum_requant_pairs left on the device for these very ranges. */
 int mxq_quantized_fc_sum_requant(void* stream, const int8_t* data, const int8_t* weight,
                                  const int8_t* bias, int M, int N, int K, const float* min_data,
                                  const float* max_data, const float* min_weight,
@@ -358,8 +359,16 @@ int mxq_quantized_fc_sum_requant(void* stream, const int8_t* data, const int8_t*
                                  const float* min_residual, const float* max_residual,
                                  int8_t* out8, float* omin, float* omax, float* rmin, float* rmax,
                                  float min_calib, float max_calib, float sum_min_calib,
-                                 float sum_max_calib, int sum_relu, void* workspace,
-                                 size_t workspace_bytes);
+                                 float sum_max_calib, int sum_relu, const void* pairs,
+                                 void* workspace, size_t workspace_bytes);
+
+/* Looks for a short form of that sum with sum_relu != 0 over ranges that stay: two products and
+ * one rounding that give the same int8 for every pair of int8 operands, which is tried out on
+ * the device.  Writes 12 bytes to `pairs` (device, 4-byte aligned), among them whether one was
+ * found; the fused launch takes it from there, without it the result is the same. */
+int mxq_sum_requant_pairs(void* stream, float min_calib, float max_calib,
+                          float min_residual, float max_residual, float sum_min_calib,
+                          float sum_max_calib, void* pairs);
 
 /* ---- _contrib_quantized_conv ----------------------------------------------
  * Replaces QuantizedCuDNNConvOp::Forward

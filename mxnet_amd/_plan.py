@@ -504,10 +504,22 @@ class _Builder:
                   [x.at, self.dense_weight(weight, o, c, 1, 1, o_padded, x.channels),
                    self.bias_of(bias, o, o_padded)] + [self.bare(r) for r in ranges] +
                   [self.scratch_range(), out, self.buffer(ws) if ws else None, residual.at] +
-                  residual_range)
+                  residual_range +
+                  ([] if j is None else [self.pairs(layer, residual_range, total, relu)]))
         self.close(last, relu, _Value(_INT8, (n, o, h, w), out, o_padded),
                    self.constant_range(*total) if j is None else self.symmetric(*total))
         return True
+
+    def pairs(self, layer, residual, total, relu):
+        """What mxq_sum_requant_pairs finds for a sum with a relu behind it whose ranges are the
+        plan's constants; None for any other."""
+        if relu is None or not all(getattr(r, "in_table", False) for r in residual):
+            return None
+        lo, hi = (self.constants[r.place[2] // 4] for r in residual)
+        found = torch.empty(3, dtype=torch.int32, device=self.device)
+        _lib.check(_lib.lib.mxq_sum_requant_pairs(self.stream, *layer, lo, hi, *total,
+                                                  found.data_ptr()))
+        return self.hold(found)
 
     def act(self, i, attrs, inputs):
         x = self.values[inputs[0]]

@@ -152,10 +152,11 @@ def quantized_fc_f32(data, weight, bias, min_data, max_data, min_weight, max_wei
 
 def quantized_fc_sum(data, weight, bias, residual, min_data, max_data, min_weight, max_weight,
                      min_bias, max_bias, min_residual, max_residual, calib, sum_calib,
-                     sum_relu=False, force=None, requant=False):
+                     sum_relu=False, force=None, requant=False, pairs=None):
     """quantized_fc -> requantize over `calib` -> elemwise_add with `residual` over `sum_calib`
     (-> relu) in one launch.  Returns dict(out8, omin, omax, rmin, rmax).  `requant`: the sum is
-    taken in int32 over its own range and requantized over `sum_calib`.  `force` = (cfg, splits,
+    taken in int32 over its own range and requantized over `sum_calib`, `pairs` is then what
+    sum_requant_pairs gave for these ranges, or None.  `force` = (cfg, splits,
     stream_groups) pins the kernel variant through the test-only entry point."""
     M, K = data.shape
     N, K2 = weight.shape
@@ -172,16 +173,29 @@ def quantized_fc_sum(data, weight, bias, residual, min_data, max_data, min_weigh
     if force is None:
         wsb = lib.mxq_quantized_fc_workspace(M, N, K, 1)
         ws = _workspace(wsb, dev) if wsb else None
-        call = lib.mxq_quantized_fc_sum_requant if requant else lib.mxq_quantized_fc_sum
-        check(call(*args, _ptr(ws), wsb))
+        if requant:
+            check(lib.mxq_quantized_fc_sum_requant(*args, _ptr(pairs), _ptr(ws), wsb))
+        else:
+            check(lib.mxq_quantized_fc_sum(*args, _ptr(ws), wsb))
     else:
         cfg, splits, groups = force
         wsb = _SPLIT_WS_BYTES if splits > 1 else 0
         ws = _workspace(wsb, dev) if wsb else None
-        call = (lib.mxq_test_quantized_fc_sum_requant if requant else
-                lib.mxq_test_quantized_fc_sum)
-        check(call(*args, _ptr(ws), wsb, cfg, splits, groups))
+        rest = [_ptr(ws), wsb, cfg, splits, groups]
+        if requant:
+            check(lib.mxq_test_quantized_fc_sum_requant(*args, _ptr(pairs), *rest))
+        else:
+            check(lib.mxq_test_quantized_fc_sum(*args, *rest))
     return res
+
+
+def sum_requant_pairs(calib, residual_range, sum_calib):
+    """The short form of a requantized sum with a relu over these ranges, as an opaque device
+    tensor for quantized_fc_sum: its third word is 1 where there is one."""
+    found = torch.empty(3, dtype=torch.int32, device="cuda")
+    check(lib.mxq_sum_requant_pairs(_stream(), *(float(v) for v in (*calib, *residual_range,
+                                                                    *sum_calib)), _ptr(found)))
+    return found
 
 
 def quantized_conv_nhwc(data, weight, bias, min_data, max_data, min_weight, max_weight,

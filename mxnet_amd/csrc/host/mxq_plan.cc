@@ -40,7 +40,7 @@ bool Plan::run(void* stream, const std::vector<at::Tensor>& feeds,
         }
         continue;
       }
-      // refs: data, weight, bias, six ranges, scratch, output, workspace[, residual, its range]
+      // refs: data, weight, bias, six ranges, scratch, output, workspace[, residual, its range[, pairs]]
       case Kind::kConv:
         rc = mxq_quantized_conv_nhwc(stream, q(0), q(1), q(2), i(0), i(1), i(2), i(3), i(4), i(5),
                                      i(6), i(7), i(8), i(9), i(10), i(11), i(12), v(3), v(4), v(5),
@@ -59,14 +59,17 @@ bool Plan::run(void* stream, const std::vector<at::Tensor>& feeds,
                                   i(3), f[0], f[1], p(11), static_cast<size_t>(n[4]));
         break;
       case Kind::kFcSum:
-      case Kind::kFcSumRq: {
-        const auto call =
-            s.kind == Kind::kFcSum ? mxq_quantized_fc_sum : mxq_quantized_fc_sum_requant;
-        rc = call(stream, q(0), q(1), q(2), i(0), i(1), i(2), v(3), v(4), v(5), v(6), v(7), v(8),
-                  q(12), v(13), v(14), q(10), v(9), v(9) + 1, v(9) + 2, v(9) + 3, f[0], f[1],
-                  f[2], f[3], i(3), p(11), static_cast<size_t>(n[4]));
+        rc = mxq_quantized_fc_sum(stream, q(0), q(1), q(2), i(0), i(1), i(2), v(3), v(4), v(5),
+                                  v(6), v(7), v(8), q(12), v(13), v(14), q(10), v(9), v(9) + 1,
+                                  v(9) + 2, v(9) + 3, f[0], f[1], f[2], f[3], i(3), p(11),
+                                  static_cast<size_t>(n[4]));
         break;
-      }
+      case Kind::kFcSumRq:
+        rc = mxq_quantized_fc_sum_requant(stream, q(0), q(1), q(2), i(0), i(1), i(2), v(3), v(4),
+                                          v(5), v(6), v(7), v(8), q(12), v(13), v(14), q(10),
+                                          v(9), v(9) + 1, v(9) + 2, v(9) + 3, f[0], f[1], f[2],
+                                          f[3], i(3), p(15), p(11), static_cast<size_t>(n[4]));
+        break;
       case Kind::kQuantNhwc:
         rc = mxq_quantize_to_nhwc(stream, v(0), q(1), v(2), v(2) + 1, i(0), i(1), i(2), i(3),
                                   i(4), i(5), i(6), i(7), f[0], f[1]);

@@ -1438,6 +1438,7 @@ void conv_nhwc(void* stream, const int8_t* data, const int8_t* weight, const int
   e.out32 = out32; e.out8 = out8; e.outf = nullptr;
   e.res = nullptr; e.res_min = nullptr; e.res_max = nullptr;
   e.sum_min_calib = 0.f; e.sum_max_calib = 0.f; e.sum_relu = 0; e.sum_requant = 0; e.with_sum = 0;
+  e.sum_pairs = nullptr;
   e.omin = omin; e.omax = omax; e.rmin = rmin; e.rmax = rmax;
   e.relu = relu;
   float x = fabsf(min_calib), y = fabsf(max_calib);

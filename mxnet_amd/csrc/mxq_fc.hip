@@ -113,22 +113,25 @@ FcPlan plan_fc(int M, int N, int K, bool aligned, bool fused8, const GemmForce& 
       else
         plan.cfg = 43;
     }
-    // the short-K streaming kernel: chosen for tall outputs of at most 256 columns
-    // (200704 x 64 -> 64: 8.5 us against 10.2; -> 256: 18.5 against 21.9; 200704 x 128 ->
-    // 128: 15.3 against 17.1); from 512 columns on the tiled kernels are level or ahead
+    // The short-K streaming kernel, from 3 M outputs on (8192 x 64 -> 512 4.8 us against 5.4 on
+    // tiles, 50176 x 128 -> 512 11.0 against 13.6, 50176 x 64 -> 1024 18.4 against 22.8; below,
+    // the strips a work-group parks cost more than they save: 4096 x 128 -> 512 4.9 against 4.2,
+    // 2048 x 128 -> 256 4.4 against 3.6).  128-column strips, three work-groups per CU, where an
+    // output of 6 M gives every wave a few of them (50176 x 64 -> 256: 7.1 us against 7.2 on
+    // 64-column strips, 50176 x 128 -> 512 11.0 against 11.9, 8192 x 64 -> 512 5.1 against 4.8).
+    // With a sum the wide strips need the registers of two groups at K = 128 (50176 x 128 -> 512
+    // 20.0 us, 21.4 on narrow ones, 21.2 on tiles), and at K <= 64 an output of 32 M (200704 x 64
+    // -> 256 28.7 against 31.8 on narrow strips; 50176 rows 11.8 against 10.9).
     const int stream_rows = K == 256 ? 128 : 256;
     const bool stream_ok = aligned && fused8 && (K == 32 || K == 64 || K == 128 || K == 256) &&
                            N % 64 == 0 && (N <= stream_rows || N % stream_rows == 0);
-    if (stream_ok && N <= 256 && K <= 128 && M >= 32768) {
-      plan.cfg = (N % 128 == 0) ? 62 : 61;
+    const long long outputs = static_cast<long long>(M) * N;
+    if (stream_ok && K <= 128 && outputs >= 3LL << 20) {
+      const bool wide = N % 128 == 0 && outputs >= (sum && K <= 64 ? 32LL << 20 : 6LL << 20);
+      plan.cfg = wide ? 62 : 61;
       plan.splits = 1;
-      if (force.stream_groups <= 0) plan.stream_groups = K <= 64 ? 4 : 3;
-      // the sum's extra registers and arithmetic favour the 64-column strips with more
-      // groups in flight (200704 x 64 -> 256 inside the chain: -7 us per layer)
-      if (sum && K <= 64) {
-        plan.cfg = 61;
-        if (force.stream_groups <= 0) plan.stream_groups = requant ? 4 : 5;
-      }
+      if (force.stream_groups <= 0)
+        plan.stream_groups = sum ? (wide && K > 64 ? 2 : 3) : (wide || K > 64 ? 3 : 4);
     }
   }
   if (plan.splits <= 0 && plan.cfg != 71) plan.splits = 1;
@@ -156,6 +159,46 @@ size_t fc_plan_workspace(const FcPlan& plan, int M, int N) {
   if (plan.splits <= 1 || !fc_cfg_tile(plan.cfg, bm, bn)) return 0;
   const long tiles = static_cast<long>((M + bm - 1) / bm) * ((N + bn - 1) / bn);
   return splitk_workspace_bytes(tiles, plan.splits, bm, bn);
+}
+
+// Looks for a short form of the requantized sum over given ranges (SumPairs): the products of the
+// rule's scales, each moved by up to three last places, the nearest first, until one gives the
+// definition's result for every pair of int8 operands.  One work-group; 8 to 10 us where the
+// first candidate holds, 0.3 ms where none does.  It runs when a plan is made, not per pass.
+__global__ __launch_bounds__(1024) void sum_pairs_kernel(float layer_range,
+                                                         float res_min, float res_max,
+                                                         float min_calib, float max_calib,
+                                                         SumPairs* out) {
+  RequantRule r = sum_requant_rule(dev_maxabs(-layer_range, layer_range),
+                                   dev_maxabs(res_min, res_max), min_calib, max_calib);
+  const double level = static_cast<double>(r.in_scale) * static_cast<double>(r.qscale);
+  const float ta = static_cast<float>(r.s0 * level), tb = static_cast<float>(r.s1 * level);
+  auto moved = [](float v, int c) {  // c = 0, 1, 2, ...: 0, +1, -1, +2, ... last places
+    return __int_as_float(__float_as_int(v) + ((c & 1) ? (c + 1) / 2 : -(c / 2)));
+  };
+  bool found = false;
+  // no denormal, infinity or NaN among the candidates
+  if (r.fast && ta > 1e-30f && tb > 1e-30f && ta < 1e30f && tb < 1e30f) {
+    for (int c = 0; c < 49 && !found; ++c) {
+      r.ta = moved(ta, c % 7);
+      r.tb = moved(tb, c / 7);
+      bool differs = false;
+      for (int i = threadIdx.x; i < 64 * 256; i += 1024) {
+        const int a0 = 4 * (i >> 8) - 127, b = (i & 255) - 128;  // a0 ... a0 + 3
+        uint32_t x = 0;
+        for (int k = 0; k < 4; ++k)  // -127 ... 127, the last quad one short
+          x |= (static_cast<uint32_t>(a0 + k < 127 ? a0 + k : 127) & 0xffu) << (8 * k);
+        const uint32_t y = (static_cast<uint32_t>(b) & 0xffu) * 0x01010101u;
+        differs |= sum_pairs4(x, y, r) != sum_requant4_general<true>(x, y, r);
+      }
+      found = __syncthreads_or(differs) == 0;
+    }
+  }
+  if (threadIdx.x == 0) {
+    out->ta = r.ta;
+    out->tb = r.tb;
+    out->ok = found;
+  }
 }
 
 // an output without elements still owes its range scalars
@@ -277,6 +320,7 @@ struct SumArgs {
   float min_calib, max_calib;
   int relu;
   int requant;
+  const SumPairs* pairs;
 };
 
 void fc_entry(void* stream, const int8_t* data, const int8_t* weight, const int8_t* bias, int M,
@@ -312,6 +356,7 @@ void fc_entry(void* stream, const int8_t* data, const int8_t* weight, const int8
   e.sum_min_calib = e.sum_max_calib = 0.f;
   e.sum_relu = 0;
   e.sum_requant = 0;
+  e.sum_pairs = nullptr;
   e.with_sum = 0;
   if (sum != nullptr) {
     MXQ_CHECK((M == 0 || N == 0 || out8 != nullptr) && out32 == nullptr && out_f32 == nullptr,
@@ -327,6 +372,7 @@ void fc_entry(void* stream, const int8_t* data, const int8_t* weight, const int8
     e.sum_max_calib = sum->max_calib;
     e.sum_relu = sum->relu;
     e.sum_requant = sum->requant;
+    e.sum_pairs = sum->pairs;
     e.with_sum = 1;
   }
   e.omin = omin;
@@ -418,7 +464,7 @@ int mxq_quantized_fc_sum(void* stream, const int8_t* data, const int8_t* weight,
                          void* workspace, size_t workspace_bytes) {
   MXQ_API_BEGIN();
   const SumArgs sum = {residual, min_residual, max_residual, sum_min_calib, sum_max_calib,
-                       sum_relu, 0};
+                       sum_relu, 0, nullptr};
   fc_entry(stream, data, weight, bias, M, N, K, min_data, max_data, min_weight, max_weight,
            min_bias, max_bias, nullptr, omin, omax, out8, nullptr, rmin, rmax, 0, min_calib,
            max_calib, workspace, workspace_bytes, GemmForce(), &sum);
@@ -433,14 +479,29 @@ int mxq_quantized_fc_sum_requant(void* stream, const int8_t* data, const int8_t*
                                  const float* min_residual, const float* max_residual,
                                  int8_t* out8, float* omin, float* omax, float* rmin, float* rmax,
                                  float min_calib, float max_calib, float sum_min_calib,
-                                 float sum_max_calib, int sum_relu, void* workspace,
-                                 size_t workspace_bytes) {
+                                 float sum_max_calib, int sum_relu, const void* pairs,
+                                 void* workspace, size_t workspace_bytes) {
   MXQ_API_BEGIN();
+  MXQ_CHECK((reinterpret_cast<uintptr_t>(pairs) & 3u) == 0, "unaligned pairs");
   const SumArgs sum = {residual, min_residual, max_residual, sum_min_calib, sum_max_calib,
-                       sum_relu, 1};
+                       sum_relu, 1, static_cast<const SumPairs*>(pairs)};
   fc_entry(stream, data, weight, bias, M, N, K, min_data, max_data, min_weight, max_weight,
            min_bias, max_bias, nullptr, omin, omax, out8, nullptr, rmin, rmax, 0, min_calib,
            max_calib, workspace, workspace_bytes, GemmForce(), &sum);
+  MXQ_API_END();
+}
+
+int mxq_sum_requant_pairs(void* stream, float min_calib, float max_calib,
+                          float min_residual, float max_residual, float sum_min_calib,
+                          float sum_max_calib, void* pairs) {
+  MXQ_API_BEGIN();
+  MXQ_CHECK(pairs != nullptr, "null pointer");
+  MXQ_CHECK((reinterpret_cast<uintptr_t>(pairs) & 3u) == 0, "unaligned pairs");
+  const float a = fabsf(min_calib), b = fabsf(max_calib);
+  hipLaunchKernelGGL(sum_pairs_kernel, dim3(1), dim3(1024), 0, static_cast<hipStream_t>(stream),
+                     (a < b) ? b : a, min_residual, max_residual, sum_min_calib, sum_max_calib,
+                     static_cast<SumPairs*>(pairs));
+  MXQ_LAUNCH_CHECK();
   MXQ_API_END();
 }
 
@@ -459,7 +520,7 @@ int mxq_test_quantized_fc_sum(void* stream, const int8_t* data, const int8_t* we
                               size_t workspace_bytes, int cfg, int splits, int stream_groups) {
   MXQ_API_BEGIN();
   const SumArgs sum = {residual, min_residual, max_residual, sum_min_calib, sum_max_calib,
-                       sum_relu, 0};
+                       sum_relu, 0, nullptr};
   GemmForce force;
   force.cfg = cfg;
   force.splits = splits;
@@ -478,11 +539,11 @@ int mxq_test_quantized_fc_sum_requant(void* stream, const int8_t* data, const in
                               const float* min_residual, const float* max_residual,
                               int8_t* out8, float* omin, float* omax, float* rmin, float* rmax,
                               float min_calib, float max_calib, float sum_min_calib,
-                              float sum_max_calib, int sum_relu, void* workspace,
-                              size_t workspace_bytes, int cfg, int splits, int stream_groups) {
+                              float sum_max_calib, int sum_relu, const void* pairs,
+                              void* workspace, size_t workspace_bytes, int cfg, int splits, int stream_groups) {
   MXQ_API_BEGIN();
   const SumArgs sum = {residual, min_residual, max_residual, sum_min_calib, sum_max_calib,
-                       sum_relu, 1};
+                       sum_relu, 1, static_cast<const SumPairs*>(pairs)};
   GemmForce force;
   force.cfg = cfg;
   force.splits = splits;

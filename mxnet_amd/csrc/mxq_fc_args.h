@@ -34,7 +34,8 @@ struct FcLaunch {
 };
 
 // Launch the kernel of `how.cfg` built for the mode (mxq_fc_plain.hip, mxq_fc_f32.hip,
-// mxq_fc_sum.hip, mxq_fc_sum_requant.hip).  The caller has checked that the shape qualifies for the configuration.
+// mxq_fc_sum.hip, mxq_fc_sum_requant.hip).  The caller has checked that the shape
+// qualifies for the configuration.
 void fc_launch_plain(hipStream_t s, const FcArgs& a, const FcLaunch& how, const Workspace& ws);
 void fc_launch_f32(hipStream_t s, const FcArgs& a, const FcLaunch& how, const Workspace& ws);
 void fc_launch_sum(hipStream_t s, const FcArgs& a, const FcLaunch& how, const Workspace& ws);

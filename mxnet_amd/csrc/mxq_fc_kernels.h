@@ -119,6 +119,11 @@ typedef GemmCfg<256, 192, 128, 4, 2> CfgW192K; // 8 waves, wave tile 64 x 96
 // LDS, then the fused epilogue and a transpose of the int8 tile through the wave's own LDS
 // scratch.  No barrier after the weights are staged; waves only meet the memory system.
 // A sum MODE: the residual operand FcArgs::epi.res is added to the int8 tile on its way out.
+constexpr int kNonTemporal = 2;  // the buffer instructions' nt bit
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t stream_rsrc(const int8_t* p, int bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(p), 0, bytes, 0x00020000);
+}
+
 template <int KS, int NI, int MODE>
 __global__ __launch_bounds__(256, 2) void fc_stream_kernel(FcArgs p, int bn, int strips) {
   constexpr bool SUM = epi_sums(MODE);
@@ -153,39 +158,46 @@ __global__ __launch_bounds__(256, 2) void fc_stream_kernel(FcArgs p, int bn, int
   const int tiles_m = (p.M + 31) / 32;
   const int items = tiles_m * strips;
   const int step = gridDim.x * 4;
-  auto load_a = [&](int item, v4i (&f)[KS]) {
-    const int m = (item / strips) * 32 + lrow;
-    const bool ok = m < p.M;
-    const int8_t* row = p.data + static_cast<size_t>(ok ? m : 0) * K + lgrp * 16;
+  // Both streams of an item come through a buffer descriptor of its own: what lies past the last
+  // row, or past the last item (the loads of the last turn), arrives as zeros without being
+  // fetched.  No branch around a load and nothing that looks at one before the next turn: with
+  // either the compiler makes every turn wait for its own prefetch, and memory and arithmetic
+  // take turns (200704 x 64 -> 256 20.4 us, 17.2 now at 3.7 TB/s; with the requantized sum 37.7,
+  // 28.2 now, 4.1 TB/s, the VALU busy for two thirds of it).
+  constexpr int kRes = SUM ? 32 / RPI : 1;
+  struct Item {
+    v4i a[KS];
+    v4i res[kRes];  // the residual operand's pieces, in the layout the tile leaves in
+  };
+  auto load = [&](int item, Item& f) {
+    const int tile = item / strips;
+    const int rows = item < items ? (p.M - tile * 32 < 32 ? p.M - tile * 32 : 32) : 0;
+    const int first = rows > 0 ? tile * 32 : 0;
+    const auto a = stream_rsrc(p.data + static_cast<size_t>(first) * K, rows * K);
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      f[ks] = *reinterpret_cast<const v4i*>(row + ks * 32);
-      if (!ok) f[ks] = v4i{0, 0, 0, 0};
+    for (int ks = 0; ks < KS; ++ks)
+      f.a[ks] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(
+                                            a, lrow * K + lgrp * 16 + ks * 32, 0, 0));
+    if constexpr (SUM) {
+      const auto r = stream_rsrc(p.epi.res + static_cast<size_t>(first) * p.ldo, rows * p.ldo);
+      const int col = n_begin + (item - tile * strips) * TN + (lane % LPR) * 16;
+#pragma unroll
+      for (int it = 0; it < kRes; ++it)
+        f.res[it] = __builtin_bit_cast(
+            v4i, __builtin_amdgcn_raw_buffer_load_b128(
+                     r, (it * RPI + lane / LPR) * p.ldo + col, 0, kNonTemporal));
     }
   };
-  int item = blockIdx.x * 4 + wave;
-  v4i fa[KS];
-  if (item < items) load_a(item, fa);
-  const bool relu = p.epi.relu != 0, stream8 = p.epi.stream8 != 0;
-  for (; item < items; item += step) {
-    v4i fa_next[KS];
-    const bool more = item + step < items;
-    if (more) load_a(item + step, fa_next);
+  // One item: the next one's loads go out, this one is multiplied, finished and stored.
+  // SM: 0 no sum, 1 sum, 2 sum + relu, 3 sum + relu in its short form, 4 / 5 as 1 / 2 where the
+  // products could overflow
+  auto turn = [&](int item, const Item& now, Item& next, auto stream, auto sum_mode,
+                  auto with_relu) {
+    constexpr int SM = decltype(sum_mode)::value;
+    load(item + step, next);
     const int tile = item / strips;
     const int s0 = (item - tile * strips) * TN;  // first column of the strip inside the group's
     const int m_base = tile * 32;
-    // the residual operand's pieces of this tile, in the layout the tile leaves in
-    v4i resv[32 / RPI];
-    if (SUM) {
-#pragma unroll
-      for (int it = 0; it < 32 / RPI; ++it) {
-        const int m = m_base + it * RPI + lane / LPR;
-        resv[it] = v4i{0, 0, 0, 0};
-        if (m < p.M)
-          resv[it] = __builtin_nontemporal_load(reinterpret_cast<const v4i*>(
-              p.epi.res + static_cast<size_t>(m) * p.ldo + n_begin + s0 + (lane % LPR) * 16));
-      }
-    }
     // the accumulators start at the int32 bias of their columns (read from LDS straight
     // into the registers the MFMAs add to): the epilogue has no bias add left
     v16i acc[NI];
@@ -203,75 +215,87 @@ __global__ __launch_bounds__(256, 2) void fc_stream_kernel(FcArgs p, int bn, int
       for (int ni = 0; ni < NI; ++ni) {
         const int r = s0 + ni * 32 + lrow;
         const v4i fb = ldsB[r * CH + ((ks * 2 + lgrp) ^ swz<CH>(r))];
-        acc[ni] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fb, fa[ks], acc[ni], 0, 0, 0);
+        acc[ni] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fb, now.a[ks], acc[ni], 0, 0, 0);
       }
-    auto requantize_tile = [&](auto with_relu) {
 #pragma unroll
-      for (int ni = 0; ni < NI; ++ni)
+    for (int ni = 0; ni < NI; ++ni)
 #pragma unroll
-        for (int vq = 0; vq < 4; ++vq) {
-          const int nl = ni * 32 + 8 * vq + 4 * lgrp;
-          *reinterpret_cast<uint32_t*>(stage + lrow * LD + nl) =
-              epi_requant_pack<decltype(with_relu)::value>(acc[ni][4 * vq], acc[ni][4 * vq + 1],
-                                                           acc[ni][4 * vq + 2],
-                                                           acc[ni][4 * vq + 3], s);
-        }
-    };
-    if (relu)
-      requantize_tile(std::true_type());
-    else
-      requantize_tile(std::false_type());
+      for (int vq = 0; vq < 4; ++vq) {
+        const int nl = ni * 32 + 8 * vq + 4 * lgrp;
+        *reinterpret_cast<uint32_t*>(stage + lrow * LD + nl) =
+            epi_requant_pack<decltype(with_relu)::value>(acc[ni][4 * vq], acc[ni][4 * vq + 1],
+                                                         acc[ni][4 * vq + 2],
+                                                         acc[ni][4 * vq + 3], s);
+      }
     // the wave reads back what its own lanes wrote: LDS executes a wave's instructions in
     // order, the wait makes the writes complete first
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_wave_barrier();
-    auto store_tile = [&](auto stream, auto sum_relu, auto sum_fast) {
+    const int rows = p.M - m_base < 32 ? p.M - m_base : 32;
+    const auto out = stream_rsrc(p.epi.out8 + static_cast<size_t>(m_base) * p.ldo, rows * p.ldo);
 #pragma unroll
-      for (int it = 0; it < 32 / RPI; ++it) {
-        const int rr = it * RPI + lane / LPR, c16 = lane % LPR;
-        v4i val = *reinterpret_cast<const v4i*>(stage + rr * LD + c16 * 16);
-        if (SUM) {
+    for (int it = 0; it < 32 / RPI; ++it) {
+      const int rr = it * RPI + lane / LPR, c16 = lane % LPR;
+      v4i val = *reinterpret_cast<const v4i*>(stage + rr * LD + c16 * 16);
+      if constexpr (SM != 0) {
 #pragma unroll
-          for (int w = 0; w < 4; ++w) {
-            constexpr bool kRelu = decltype(sum_relu)::value, kFast = decltype(sum_fast)::value;
-            const uint32_t x = static_cast<uint32_t>(val[w]);
-            const uint32_t y = static_cast<uint32_t>(resv[it][w]);
-            if constexpr (MODE == kEpiSumRq)
-              val[w] = static_cast<int>(kFast ? sum_requant4<kRelu>(x, y, rule)
-                                              : sum_requant4_general<kRelu>(x, y, rule));
-            else
-              val[w] = static_cast<int>(sum4<kRelu, kFast>(x, y, rule));
-          }
+        for (int w = 0; w < 4; ++w) {
+          constexpr bool kRelu = SM == 2 || SM == 5, kFast = SM < 4;
+          const uint32_t x = static_cast<uint32_t>(val[w]);
+          const uint32_t y = static_cast<uint32_t>(now.res[it][w]);
+          if constexpr (SM == 3)
+            val[w] = static_cast<int>(epi_sum_pairs4(x, y, rules));
+          else if constexpr (MODE == kEpiSumRq)
+            val[w] = static_cast<int>(kFast ? sum_requant4<kRelu>(x, y, rule)
+                                            : sum_requant4_general<kRelu>(x, y, rule));
+          else
+            val[w] = static_cast<int>(sum4<kRelu, kFast>(x, y, rule));
         }
-        const int m = m_base + rr;
-        if (m < p.M)
-          epi_store16<decltype(stream)::value>(
-              val, p.epi.out8 + static_cast<size_t>(m) * p.ldo + n_begin + s0 + c16 * 16);
       }
-    };
-    auto store_flavour = [&](auto sum_relu, auto sum_fast) {
-      if (stream8)
-        store_tile(std::true_type(), sum_relu, sum_fast);
-      else
-        store_tile(std::false_type(), sum_relu, sum_fast);
-    };
-    if (SUM && !rule.fast) {
-      if (p.epi.sum_relu)
-        store_flavour(std::true_type(), std::integral_constant<bool, !SUM>());
-      else
-        store_flavour(std::false_type(), std::integral_constant<bool, !SUM>());
-    } else if (SUM && p.epi.sum_relu) {
-      store_flavour(std::true_type(), std::true_type());
-    } else {
-      store_flavour(std::false_type(), std::true_type());
+      __builtin_amdgcn_raw_buffer_store_b128(val, out, rr * p.ldo + n_begin + s0 + c16 * 16, 0,
+                                             decltype(stream)::value ? kNonTemporal : 0);
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_wave_barrier();
-    if (more) {
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) fa[ks] = fa_next[ks];
+  };
+  // Two items change places instead of registers being copied: a copy would wait for its loads,
+  // and for the stores in front of them.
+  auto run = [&](auto stream, auto sum_mode, auto with_relu) {
+    int item = blockIdx.x * 4 + wave;
+    Item x, y;
+    load(item, x);
+    while (item < items) {
+      turn(item, x, y, stream, sum_mode, with_relu);
+      item += step;
+      if (item >= items) break;
+      turn(item, y, x, stream, sum_mode, with_relu);
+      item += step;
     }
-  }
+  };
+  auto run_flavour = [&](auto stream) {
+    typedef std::false_type No;
+    if constexpr (!SUM) {
+      if (p.epi.relu)
+        run(stream, std::integral_constant<int, 0>(), std::true_type());
+      else
+        run(stream, std::integral_constant<int, 0>(), No());
+    } else {  // a layer in front of a sum has no relu of its own
+      if (MODE == kEpiSumRq && epi_sum_pairs(rules))
+        run(stream, std::integral_constant<int, MODE == kEpiSumRq ? 3 : 2>(), No());
+      else if (rule.fast && p.epi.sum_relu)
+        run(stream, std::integral_constant<int, 2>(), No());
+      else if (rule.fast)
+        run(stream, std::integral_constant<int, 1>(), No());
+      else if (p.epi.sum_relu)
+        run(stream, std::integral_constant<int, 5>(), No());
+      else
+        run(stream, std::integral_constant<int, 4>(), No());
+    }
+  };
+  if (p.epi.stream8)
+    run_flavour(std::true_type());
+  else
+    run_flavour(std::false_type());
   if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) epilogue_ranges<MODE>(p.epi);
 }
 
@@ -279,6 +303,8 @@ template <int KS, int NI, int MODE>
 void launch_stream(hipStream_t s, const FcArgs& a, long cus, int groups_per_cu) {
   // the residual operand is read in 16-byte pieces, like the output is written
   MXQ_CHECK(a.epi.res == nullptr || aligned16(a.epi.res), "unaligned residual operand");
+  // 32 rows of the output are addressed with 32-bit byte offsets
+  MXQ_CHECK(a.ldo < (1 << 25), "row pitch too large for the short-K streaming kernel");
   constexpr int TN = 32 * NI;
   const int max_rows = KS <= 4 ? 256 : 128;
   const int bn = a.N < max_rows ? a.N : max_rows;

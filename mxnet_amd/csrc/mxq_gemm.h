@@ -67,6 +67,7 @@ struct Epilogue {
   float sum_min_calib, sum_max_calib;
   int sum_relu;
   int sum_requant;         // the sum in int32 over its own range, then requantized (RequantRule)
+  const SumPairs* sum_pairs;  // device, or null: the short form of that rule
   int with_sum;            // rmin / rmax report the sum's range (also for an empty output)
   float* omin;             // int32 output range
   float* omax;
@@ -711,9 +712,15 @@ template <int MODE>
 __device__ __forceinline__ auto epi_sum_rule(const Epilogue& e) {
   const float a = dev_maxabs(-e.real_range, e.real_range);
   const float b = dev_maxabs(*e.res_min, *e.res_max);
-  if constexpr (MODE == kEpiSumRq)
-    return sum_requant_rule(a, b, e.sum_min_calib, e.sum_max_calib);
-  else
+  if constexpr (MODE == kEpiSumRq) {
+    RequantRule r = sum_requant_rule(a, b, e.sum_min_calib, e.sum_max_calib);
+    if (e.sum_pairs != nullptr && e.sum_relu && r.fast) {
+      r.ta = e.sum_pairs->ta;
+      r.tb = e.sum_pairs->tb;
+      r.pairs = e.sum_pairs->ok;
+    }
+    return r;
+  } else
     return sum_rule(a, b, e.sum_min_calib, e.sum_max_calib);
 }
 
@@ -848,6 +855,18 @@ template <bool RELU>
 __device__ __forceinline__ uint32_t epi_sum4(uint32_t x, uint32_t y,
                                              const EpiPreOf<kEpiSumRq>& pre) {
   return sum_requant4<RELU>(x, y, pre.sum);
+}
+// whether the rule has the short form, and four elements under it
+__device__ __forceinline__ bool epi_sum_pairs(const EpiPre&) { return false; }
+__device__ __forceinline__ bool epi_sum_pairs(const EpiPreOf<kEpiSumRq>& pre) {
+  return pre.sum.pairs != 0;
+}
+__device__ __forceinline__ uint32_t epi_sum_pairs4(uint32_t x, uint32_t, const EpiPre&) {
+  return x;
+}
+__device__ __forceinline__ uint32_t epi_sum_pairs4(uint32_t x, uint32_t y,
+                                                   const EpiPreOf<kEpiSumRq>& pre) {
+  return sum_pairs4(x, y, pre.sum);
 }
 // one element of the sum under any rule
 __device__ __forceinline__ int8_t epi_sum_one(int a, int, bool, const EpiPre&) {
@@ -1186,7 +1205,9 @@ __device__ __forceinline__ void gemm_epilogue_lds(v16i (&acc)[Cfg::MI][Cfg::NI],
     // (a wave tile of 96 columns has 6 pieces per row: the last instruction is then partial)
     constexpr int kPieces = TM * LPR;
     constexpr int kIters = (kPieces + 63) / 64;
-    // the residual operand's pieces are fetched now, behind the requantization's arithmetic
+    // the residual operand's pieces are fetched now, behind the requantization's arithmetic (asked
+    // for with the first operand stage instead, all of a launch's residual traffic stands in front
+    // of its first K step: 12544 x 256 -> 1024 16.9 us against 13.8)
     v4i resv[epi_sums(MODE) ? kIters : 1];
     if constexpr (epi_sums(MODE)) {
       if (fast8 && fasts) {
@@ -1226,7 +1247,7 @@ __device__ __forceinline__ void gemm_epilogue_lds(v16i (&acc)[Cfg::MI][Cfg::NI],
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_wave_barrier();
     auto store_tile = [&](auto stream, auto sum_mode) {
-      constexpr int SM = decltype(sum_mode)::value;  // 0 no sum, 1 sum, 2 sum + relu
+      constexpr int SM = decltype(sum_mode)::value;  // 0 no sum, 1 sum, 2 + relu, 3 short form
 #pragma unroll
       for (int it = 0; it < kIters; ++it) {
         const int piece = it * 64 + lane;
@@ -1239,7 +1260,8 @@ __device__ __forceinline__ void gemm_epilogue_lds(v16i (&acc)[Cfg::MI][Cfg::NI],
           for (int w = 0; w < 4; ++w) {
             const uint32_t x = static_cast<uint32_t>(val[w]);
             const uint32_t y = static_cast<uint32_t>(resv[it][w]);
-            val[w] = static_cast<int>(epi_sum4<SM == 2>(x, y, pre));
+            val[w] = static_cast<int>(SM == 3 ? epi_sum_pairs4(x, y, pre)
+                                              : epi_sum4<SM == 2>(x, y, pre));
           }
         }
         const int m = m_base + rr, n = n_base + c16 * 16;
@@ -1260,17 +1282,18 @@ __device__ __forceinline__ void gemm_epilogue_lds(v16i (&acc)[Cfg::MI][Cfg::NI],
         }
         return;
       }
-      if (e.stream8) {
-        if (e.sum_relu)
-          store_tile(std::true_type(), std::integral_constant<int, 2>());
+      auto store_sums = [&](auto stream) {
+        if (MODE == kEpiSumRq && epi_sum_pairs(pre))
+          store_tile(stream, std::integral_constant<int, MODE == kEpiSumRq ? 3 : 2>());
+        else if (e.sum_relu)
+          store_tile(stream, std::integral_constant<int, 2>());
         else
-          store_tile(std::true_type(), std::integral_constant<int, 1>());
-      } else {
-        if (e.sum_relu)
-          store_tile(std::false_type(), std::integral_constant<int, 2>());
-        else
-          store_tile(std::false_type(), std::integral_constant<int, 1>());
-      }
+          store_tile(stream, std::integral_constant<int, 1>());
+      };
+      if (e.stream8)
+        store_sums(std::true_type());
+      else
+        store_sums(std::false_type());
     } else if (e.stream8) {
       store_tile(std::true_type(), std::integral_constant<int, 0>());
     } else {

@@ -70,6 +70,20 @@ struct RequantRule {
   float in_scale;  // float per int32 level
   float qscale;    // int8 levels per float
   int fast;        // no product overflows and nothing is NaN: the sum needs no saturation
+  float ta, tb;    // the short form, where `pairs` says that it holds (SumPairs)
+  int pairs;
+};
+
+// The short form of a RequantRule with the relu behind it: nearest-even(a * ta + b * tb) clamped
+// to [0, 127], one rounding per product and one for the sum instead of seven.  Both operands are
+// int8, so it either gives the definition's result for all 255 x 256 pairs or it does not, and
+// that is found out by trying them: sum_pairs_kernel (mxq_fc.hip) does so once for ranges that
+// stay (a plan's constants).  What it may be off by is a last place of a value near a tie, so the
+// products of the rule's scales hold as they are for most ranges and within three last places of
+// them for nearly all others.
+struct SumPairs {
+  float ta, tb;
+  int ok;
 };
 
 __device__ __forceinline__ RequantRule sum_requant_rule(float a_absmax, float b_absmax,
@@ -86,7 +100,23 @@ __device__ __forceinline__ RequantRule sum_requant_rule(float a_absmax, float b_
   r.qscale = 127.0f / ((x < y) ? y : x);
   r.fast = fabsf(r.s0) < 1e30f && fabsf(r.s1) < 1e30f && fabsf(r.qscale) < 1e30f &&
            r.in_scale > 0.0f;
+  r.ta = r.tb = 0.0f;
+  r.pairs = 0;
   return r;
+}
+
+// Four pairs under the short form: 6 instructions a pair instead of 11.5.
+__device__ __forceinline__ uint32_t sum_pairs4(uint32_t x, uint32_t y, const RequantRule& r) {
+  uint32_t w = 0;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int a = static_cast<int>(static_cast<int8_t>((x >> (8 * k)) & 0xffu));
+    const int b = static_cast<int>(static_cast<int8_t>((y >> (8 * k)) & 0xffu));
+    const float u = __builtin_fmaf(static_cast<float>(a), r.ta, static_cast<float>(b) * r.tb);
+    // rounds to nearest even, what is below zero becomes 0
+    w = __builtin_amdgcn_cvt_pk_u8_f32(u < 127.0f ? u : 127.0f, k, w);
+  }
+  return w;
 }
 
 // One element, as the two operators compute it one after the other.

@@ -60,8 +60,9 @@ int mxq_test_quantized_fc_sum_requant(void* stream, const int8_t* data, const in
                               const float* min_residual, const float* max_residual,
                               int8_t* out8, float* omin, float* omax, float* rmin, float* rmax,
                               float min_calib, float max_calib, float sum_min_calib,
-                              float sum_max_calib, int sum_relu, void* workspace,
-                              size_t workspace_bytes, int cfg, int splits, int stream_groups);
+                              float sum_max_calib, int sum_relu, const void* pairs,
+                              void* workspace, size_t workspace_bytes, int cfg, int splits,
+                              int stream_groups);
 
 /* mxq_quantized_conv_nhwc with the tile configuration (mxq_conv.hip lists them) and the
  * split-K factor pinned. */
