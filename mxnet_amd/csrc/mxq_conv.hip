@@ -1522,7 +1522,7 @@ void conv_nhwc(void* stream, const int8_t* data, const int8_t* weight, const int
     f.images = N; f.H = H; f.W = W; f.C = C; f.KW = KW; f.sh = a.sh; f.sw = a.sw; f.ph = a.ph;
     f.pw = a.pw; f.dh = a.dh; f.dw = a.dw; f.OH = a.OH; f.OW = a.OW;
     launch_few_tiles_conv(s, f,
-                          force.splits > 0 ? force.splits : few_tiles_waves(a.M, O, a.K, true));
+                          force.splits != 0 ? force.splits : few_tiles_waves(a.M, O, a.K, true));
     return;
   }
   if (cfg > 10) MXQ_CHECK(dma_ok, "shape does not qualify for the direct-to-LDS conv kernels");

@@ -29,7 +29,8 @@ namespace mxq {
 //   57..59  128x64 and 64x128 with 128-byte stages, 64x64 with 256-byte stages
 //   60      256x192 with 128-byte stages (outputs whose width is a multiple of 192)
 //   61, 62  the short-K streaming kernel with 64- / 128-column strips
-//   71      the few-tiles kernel (any shape; here `splits` is the number of waves per tile)
+//   71      the few-tiles kernel (any shape; here `splits` is the number of waves per
+//           32 x 32 tile, negative for 16 x 16 tiles)
 // Output tile of a direct-to-LDS configuration (what a split-K work-group leaves in the
 // workspace); false for every other configuration.
 bool fc_cfg_tile(int cfg, int& bm, int& bn) {
@@ -277,7 +278,7 @@ void launch_fc(hipStream_t s, const int8_t* data, const int8_t* weight, int M, i
     f.ldo = ldo;
     f.epi = a.epi;
     launch_few_tiles_fc(s, f, buf_ok,
-                        plan.splits > 0 ? plan.splits : few_tiles_waves(M, N, K, buf_ok));
+                        plan.splits != 0 ? plan.splits : few_tiles_waves(M, N, K, buf_ok));
     return;
   }
   if (cfg < 11) MXQ_CHECK(plan.splits <= 1, "the register-staged kernels have no split-K form");

@@ -33,7 +33,8 @@ inline bool few_tiles_wins(long M, long N, long K, long cus) {
   return K >= 256 && few_tiles_count(M, N) <= (K < 8192 ? cus : cus / 4);
 }
 
-// Waves that share one tile's reduction of K bytes.
+// Waves that share one tile's reduction of K bytes: 2, 4, 8 or 16 for a 32 x 32 tile, -4 or -8
+// for a 16 x 16 one.
 int few_tiles_waves(int M, int N, int K, bool aligned);
 // `aligned`: 16 | K, 16-byte aligned operands below 2 GiB.
 void launch_few_tiles_fc(hipStream_t s, const FewTilesArgs& a, bool aligned, int waves);

@@ -3,11 +3,11 @@
 // a barrier per stage: a 3 x 3 convolution over 512 channels of one 7 x 7 plane is 8 work-groups
 // of 18 stages, 15-17 us, nearly all of it waiting for memory.
 //
-// Here a work-group owns a 32 x 32 output tile and its waves share the reduction: wave w takes
+// Here a work-group owns a 32 x 32 or 16 x 16 output tile and its waves share the reduction: wave w takes
 // the 128-byte blocks w, w + W, ... of the K axis, loads both operands' fragments straight from
 // memory into the MFMA layout (no LDS, no barrier, two or three blocks in flight per wave), and the
 // W partial tiles meet in LDS once at the end.  Integer addition is associative: the result is the
-// tiled kernels' bit for bit.  The same convolution: 4.6 us.
+// tiled kernels' bit for bit.  The same convolution: 5.4 us, of which an empty launch is 3.0.
 //
 // Four consecutive lanes load 64 consecutive bytes of one row, which is what the address unit
 // handles in one step; the MFMA wants consecutive lanes to hold consecutive rows, so the pieces
@@ -29,12 +29,11 @@
 namespace mxq {
 namespace {
 
-constexpr int kTile = 32;       // rows and columns of an output tile
 constexpr int kBlockK = 128;    // bytes of the reduction a wave takes at a time: a cache line
 constexpr int kSteps = kBlockK / 64;
-// blocks in flight per wave: three, two where 16 waves leave a lane 128 registers
-constexpr int depth_of(int waves) { return waves == 16 ? 2 : 3; }
-constexpr int kPitch = 36;      // ints per row of a partial tile in LDS
+// blocks in flight per wave: three, two where 16 waves leave a lane 128 registers and a block of
+// a 32 x 32 tile takes 32 of them
+constexpr int depth_of(int waves, int tile) { return waves == 16 && tile == 32 ? 2 : 3; }
 
 // 16-byte pieces of row-major rows of K bytes, aligned: pieces past the row, rows past the
 // operand and blocks past the reduction come back as zeros without being fetched.
@@ -124,9 +123,11 @@ struct ConvRows {
 
 enum Operands { kAligned, kAny, kConv };
 
-template <int W, int OPERANDS, int MODE>
+// T: rows and columns of an output tile, 32 or 16
+template <int W, int T, int OPERANDS, int MODE>
 __global__ __launch_bounds__(64 * W) void few_tiles_kernel(FewTilesArgs p) {
-  constexpr int kDepth = depth_of(W);
+  constexpr int kDepth = depth_of(W, T), kTile = T, F = T / 16;
+  constexpr int kPitch = T + 4;  // ints per row of a partial tile in LDS
   __shared__ __attribute__((aligned(16))) int part[W][kTile * kPitch];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -143,12 +144,12 @@ __global__ __launch_bounds__(64 * W) void few_tiles_kernel(FewTilesArgs p) {
     return v;
   };
 
-  typename std::conditional<OPERANDS == kAny, AnyRows, AlignedRows>::type b[2];
+  typename std::conditional<OPERANDS == kAny, AnyRows, AlignedRows>::type b[F];
   typename std::conditional<
       OPERANDS == kAny, AnyRows,
-      typename std::conditional<OPERANDS == kConv, ConvRows, AlignedRows>::type>::type a[2];
+      typename std::conditional<OPERANDS == kConv, ConvRows, AlignedRows>::type>::type a[F];
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
+  for (int i = 0; i < F; ++i) {
     if constexpr (OPERANDS == kConv)
       a[i].init(p, m0 + 16 * i + load_row);
     else
@@ -156,13 +157,13 @@ __global__ __launch_bounds__(64 * W) void few_tiles_kernel(FewTilesArgs p) {
     b[i].init(p.weight, n0 + 16 * i + load_row, p.N, p.K);
   }
 
-  v4i fa[kDepth][kSteps][2], fb[kDepth][kSteps][2];
-  auto fetch = [&](int block, v4i (&x)[kSteps][2], v4i (&y)[kSteps][2]) {
+  v4i fa[kDepth][kSteps][F], fb[kDepth][kSteps][F];
+  auto fetch = [&](int block, v4i (&x)[kSteps][F], v4i (&y)[kSteps][F]) {
 #pragma unroll
     for (int s = 0; s < kSteps; ++s) {
       const int k0 = block * kBlockK + s * 64 + load_piece * 16;
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
+      for (int i = 0; i < F; ++i) {
         x[s][i] = a[i].load(k0);
         y[s][i] = b[i].load(k0);
       }
@@ -174,39 +175,39 @@ __global__ __launch_bounds__(64 * W) void few_tiles_kernel(FewTilesArgs p) {
   for (int d = 0; d < kDepth; ++d)
     if (d < rounds) fetch(wave + d * W, fa[d], fb[d]);
 
-  // what the epilogue needs, behind the first loads: thread t finishes columns 4 * (t % 8) ... of
-  // row t / 8 (and of row t / 8 + 64 * W / 8 with few waves)
-  constexpr int kQuads = kTile * kTile / 4, kThreads = 64 * W;
+  // what the epilogue needs, behind the first loads: thread t finishes columns 4 * (t % Q) ... of
+  // row t / Q, Q = T / 4 (and of row t / Q + 64 * W / Q with few waves)
+  constexpr int Q = T / 4, kQuads = T * Q, kThreads = 64 * W;
   constexpr int kPer = (kQuads + kThreads - 1) / kThreads;
   const EpiPreOf<MODE> pre = epi_prefetch_scalars<MODE>(p.epi);
-  const int n = n0 + 4 * (tid & 7);
+  const int n = n0 + 4 * (tid % Q);
   int bias[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i)
     bias[i] = (tid < kQuads && n + i < p.N) ? epi_bias32(p.epi, pre.s, n + i) : 0;
 
   // lane: activation row lane % 16, output columns 4 * (lane / 16) ... + 3
-  v4i acc[2][2];
+  v4i acc[F][F];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < F; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = v4i{0, 0, 0, 0};
+    for (int j = 0; j < F; ++j) acc[i][j] = v4i{0, 0, 0, 0};
   for (int r = 0; r < rounds; r += kDepth) {
 #pragma unroll
     for (int d = 0; d < kDepth; ++d) {
       if (r + d < rounds) {
 #pragma unroll
         for (int s = 0; s < kSteps; ++s) {
-          v4i x[2], y[2];
+          v4i x[F], y[F];
 #pragma unroll
-          for (int i = 0; i < 2; ++i) {
+          for (int i = 0; i < F; ++i) {
             x[i] = to_mfma(fa[d][s][i]);
             y[i] = to_mfma(fb[d][s][i]);
           }
 #pragma unroll
-          for (int i = 0; i < 2; ++i)
+          for (int i = 0; i < F; ++i)
 #pragma unroll
-            for (int j = 0; j < 2; ++j)
+            for (int j = 0; j < F; ++j)
               acc[i][j] =
                   __builtin_amdgcn_mfma_i32_16x16x64_i8(y[j], x[i], acc[i][j], 0, 0, 0);
         }
@@ -215,9 +216,9 @@ __global__ __launch_bounds__(64 * W) void few_tiles_kernel(FewTilesArgs p) {
     }
   }
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < F; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < F; ++j)
       *reinterpret_cast<v4i*>(&part[wave][(16 * i + lrow) * kPitch + 16 * j + 4 * lgrp]) =
           acc[i][j];
   __syncthreads();
@@ -227,11 +228,11 @@ __global__ __launch_bounds__(64 * W) void few_tiles_kernel(FewTilesArgs p) {
   for (int j = 0; j < kPer; ++j) {
     const int q = tid + j * kThreads;
     if (kQuads % kThreads != 0 && q >= kQuads) break;
-    const int row = q >> 3, m = m0 + row;
+    const int row = q / Q, m = m0 + row;
     uint32_t sum[4] = {};
 #pragma unroll
     for (int w = 0; w < W; ++w) {
-      const v4i x = *reinterpret_cast<const v4i*>(&part[w][row * kPitch + 4 * (tid & 7)]);
+      const v4i x = *reinterpret_cast<const v4i*>(&part[w][row * kPitch + 4 * (tid % Q)]);
 #pragma unroll
       for (int i = 0; i < 4; ++i) sum[i] += static_cast<uint32_t>(x[i]);
     }
@@ -271,20 +272,26 @@ __global__ __launch_bounds__(256) void pad_rows_kernel(PadJob x, PadJob y, int K
 
 template <int OPERANDS, int MODE>
 void launch(hipStream_t s, const FewTilesArgs& a, int waves) {
-  const long tiles = few_tiles_count(a.M, a.N);
-  const dim3 grid(static_cast<unsigned>(tiles));
+  const long side = waves == -4 || waves == -8 ? 16 : 32;
+  const dim3 grid(static_cast<unsigned>((a.M + side - 1) / side * ((a.N + side - 1) / side)));
   switch (waves) {
+    case -4:
+      hipLaunchKernelGGL((few_tiles_kernel<4, 16, OPERANDS, MODE>), grid, dim3(256), 0, s, a);
+      break;
+    case -8:
+      hipLaunchKernelGGL((few_tiles_kernel<8, 16, OPERANDS, MODE>), grid, dim3(512), 0, s, a);
+      break;
     case 2:
-      hipLaunchKernelGGL((few_tiles_kernel<2, OPERANDS, MODE>), grid, dim3(128), 0, s, a);
+      hipLaunchKernelGGL((few_tiles_kernel<2, 32, OPERANDS, MODE>), grid, dim3(128), 0, s, a);
       break;
     case 4:
-      hipLaunchKernelGGL((few_tiles_kernel<4, OPERANDS, MODE>), grid, dim3(256), 0, s, a);
+      hipLaunchKernelGGL((few_tiles_kernel<4, 32, OPERANDS, MODE>), grid, dim3(256), 0, s, a);
       break;
     case 8:
-      hipLaunchKernelGGL((few_tiles_kernel<8, OPERANDS, MODE>), grid, dim3(512), 0, s, a);
+      hipLaunchKernelGGL((few_tiles_kernel<8, 32, OPERANDS, MODE>), grid, dim3(512), 0, s, a);
       break;
     default:
-      hipLaunchKernelGGL((few_tiles_kernel<16, OPERANDS, MODE>), grid, dim3(1024), 0, s, a);
+      hipLaunchKernelGGL((few_tiles_kernel<16, 32, OPERANDS, MODE>), grid, dim3(1024), 0, s, a);
   }
   MXQ_LAUNCH_CHECK();
 }
@@ -299,13 +306,18 @@ void launch_rows(hipStream_t s, const FewTilesArgs& a, bool aligned, int waves) 
 
 }  // namespace
 
-// A wave per block of the reduction up to 8; up to 16 where the pieces are masked on their way in
-// (16 x 1237 -> 43: 5.8 us against 6.3) or the reduction has 16 blocks, which is level at worst.
-// With more tiles than the chip has CUs the tiles themselves fill it and splitting a reduction
-// further only adds partial tiles (1024 x 435 -> 1024: 7.7 us on 2 waves, 14.3 on 8).
+// 16 x 16 tiles (negative) where 32 x 32 ones would occupy half of the CUs or fewer: a CU then takes
+// in half the bytes and four times as many of them do (3 x 3 over 512 channels of one 7 x 7 plane
+// 8.5 us -> 5.4, over 256 channels of 14 x 14 6.9 -> 4.5, 64 x 2048 -> 1000 5.0 -> 3.75; an empty
+// launch is 3.0).  Between half and all of them the narrow tiles read too much twice (784 x 512 ->
+// 256 5.0 us against 3.9).  There a wave per block of the reduction up to 8, up to 16 where the
+// pieces are masked on their way in or the reduction has 16 blocks, which is level at worst.  With more tiles than the chip has CUs the
+// tiles themselves fill it and splitting a reduction further only adds partial tiles (1024 x 435 ->
+// 1024: 7.7 us on 2 waves, 14.3 on 8).
 int few_tiles_waves(int M, int N, int K, bool aligned) {
   const int blocks = (K + kBlockK - 1) / kBlockK;
   const long tiles = few_tiles_count(M, N), cus = num_cus();
+  if (2 * tiles <= cus && blocks > 1) return K >= 512 ? -8 : -4;
   if (tiles > 2 * cus || blocks <= 2) return 2;
   if (tiles > cus || blocks <= 4) return 4;
   return blocks > (aligned ? 15 : 8) ? 16 : 8;

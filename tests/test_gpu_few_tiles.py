@@ -33,7 +33,7 @@ def exact(x, w):
 RANGES = (-1.0, 1.0, -2.0, 2.0)
 
 
-@pytest.mark.parametrize("waves", [0, 2, 4, 8, 16])
+@pytest.mark.parametrize("waves", [0, 2, 4, 8, 16, -4, -8])
 @pytest.mark.parametrize("m,n,k,off", [
     (1, 1, 16, 0), (1, 16, 17, 0), (31, 33, 127, 0), (32, 32, 128, 0), (33, 31, 129, 1),
     (65, 48, 256, 0), (3, 70, 45, 3), (17, 20, 1237, 5), (49, 64, 4096, 0), (64, 5, 2049, 2),
@@ -92,7 +92,7 @@ def conv_exact(x, w, stride, pad, dilate):
 @pytest.mark.parametrize("n,h,w,c,o,k,stride,pad,dilate", [
     (1, 7, 7, 512, 64, 3, 1, 1, 1), (1, 14, 13, 48, 33, 3, 2, 1, 1), (2, 9, 9, 16, 20, 5, 1, 2, 2),
     (1, 5, 6, 32, 17, 1, 2, 0, 1), (3, 4, 4, 64, 40, 4, 1, 2, 1), (1, 1, 1, 272, 32, 1, 1, 1, 1)])
-@pytest.mark.parametrize("waves", [0, 2, 4, 8, 16])
+@pytest.mark.parametrize("waves", [0, 2, 4, 8, 16, -4, -8])
 def test_convolutions(n, h, w, c, o, k, stride, pad, dilate, waves):
     g = torch.Generator(device="cuda").manual_seed(c + k)
     x, wt = int8(g, 0, n, h, w, c), int8(g, 0, o, k, k, c)
