@@ -540,10 +540,12 @@ __global__ __launch_bounds__(256, KS > 5 ? 3 : 4) void conv_taps_kernel(TapArgs 
       }
     }
   };
-  auto load_a = [&](v4i (&f)[KS]) {
+  // `more` == false: nothing is fetched, but the loads are issued all the same (kOutOfRange): a
+  // branch around them would make every turn of the loop wait for its own prefetch
+  auto load_a = [&](v4i (&f)[KS], bool more) {
     const int ih0 = oh * p.sh - p.ph, iw0 = ow * p.sw - p.pw;
     const int base = ((n * p.H + ih0) * p.W + iw0) * 16;
-    const bool live = n < p.N;
+    const bool live = more && n < p.N;
     const bool inside = live && ih0 >= 0 && iw0 >= 0 && ih0 + reach_h < p.H && iw0 + reach_w < p.W;
     if (__all(inside)) {
 #pragma unroll
@@ -563,20 +565,16 @@ __global__ __launch_bounds__(256, KS > 5 ? 3 : 4) void conv_taps_kernel(TapArgs 
     }
   };
   char* stage = stage_all + wave * 32 * LD;
-  const bool relu = p.epi.relu != 0, stream8 = p.epi.stream8 != 0;
-  v4i fa[KS];
-  if (item < end) load_a(fa);
-  for (; item < end; item += 4) {
+  auto turn = [&](const v4i (&fa)[KS], v4i (&fa_next)[KS], auto with_relu, auto stream) {
     const int m_base = tile * 32, s0 = strip * TN;
-    v4i fa_next[KS];
     const bool more = item + 4 < end;
     if (more) {
       const int next = (item + 4) / t.strips;
       advance(next - tile);
       strip = item + 4 - next * t.strips;
       tile = next;
-      load_a(fa_next);
     }
+    load_a(fa_next, more);
     v16i acc[NI];
 #pragma unroll
     for (int ni = 0; ni < NI; ++ni)
@@ -592,43 +590,51 @@ __global__ __launch_bounds__(256, KS > 5 ? 3 : 4) void conv_taps_kernel(TapArgs 
       for (int ni = 0; ni < NI; ++ni)
         acc[ni] = __builtin_amdgcn_mfma_i32_32x32x32_i8(
             wl[(s0 + ni * 32 + lrow) * PITCH + 2 * ks + lgrp], fa[ks], acc[ni], 0, 0, 0);
-    auto requantize_tile = [&](auto with_relu) {
 #pragma unroll
-      for (int ni = 0; ni < NI; ++ni)
+    for (int ni = 0; ni < NI; ++ni)
 #pragma unroll
-        for (int vq = 0; vq < 4; ++vq)
-          *reinterpret_cast<uint32_t*>(stage + lrow * LD + ni * 32 + 8 * vq + 4 * lgrp) =
-              epi_requant_pack<decltype(with_relu)::value>(acc[ni][4 * vq], acc[ni][4 * vq + 1],
-                                                           acc[ni][4 * vq + 2],
-                                                           acc[ni][4 * vq + 3], s);
-    };
-    if (relu)
-      requantize_tile(std::true_type());
-    else
-      requantize_tile(std::false_type());
+      for (int vq = 0; vq < 4; ++vq)
+        *reinterpret_cast<uint32_t*>(stage + lrow * LD + ni * 32 + 8 * vq + 4 * lgrp) =
+            epi_requant_pack<decltype(with_relu)::value>(acc[ni][4 * vq], acc[ni][4 * vq + 1],
+                                                         acc[ni][4 * vq + 2],
+                                                         acc[ni][4 * vq + 3], s);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_wave_barrier();
-    auto store_tile = [&](auto stream) {
+    // rows past the last pixel lie past the descriptor's end and are dropped
+    const int left = p.M - m_base < 32 ? p.M - m_base : 32;
+    const __amdgpu_buffer_rsrc_t out = __builtin_amdgcn_make_buffer_rsrc(
+        p.epi.out8 + static_cast<size_t>(m_base) * p.O, 0, left * p.O, 0x00020000);
 #pragma unroll
-      for (int it = 0; it < 32 / RPI; ++it) {
-        const int rr = it * RPI + lane / LPR, c16 = lane % LPR;
-        const v4i val = *reinterpret_cast<const v4i*>(stage + rr * LD + c16 * 16);
-        const int m = m_base + rr, o = s0 + c16 * 16;
-        if (m < p.M && o < p.O)
-          epi_store16<decltype(stream)::value>(val,
-                                               p.epi.out8 + static_cast<size_t>(m) * p.O + o);
-      }
-    };
-    if (stream8)
-      store_tile(std::true_type());
-    else
-      store_tile(std::false_type());
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_wave_barrier();
-    if (more) {
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) fa[ks] = fa_next[ks];
+    for (int it = 0; it < 32 / RPI; ++it) {
+      const int rr = it * RPI + lane / LPR, c16 = lane % LPR, o = s0 + c16 * 16;
+      const v4i val = *reinterpret_cast<const v4i*>(stage + rr * LD + c16 * 16);
+      __builtin_amdgcn_raw_buffer_store_b128(
+          val, out, o < p.O ? static_cast<uint32_t>(rr * p.O + o) : kOutOfRange, 0,
+          decltype(stream)::value ? 2 /* nt */ : 0);
     }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_wave_barrier();
+    item += 4;
+  };
+  // two sets of fragments change places instead of being copied: a copy would wait for its loads
+  auto run = [&](auto with_relu, auto stream) {
+    v4i x[KS], y[KS];
+    load_a(x, item < end);
+    while (item < end) {
+      turn(x, y, with_relu, stream);
+      if (item >= end) break;
+      turn(y, x, with_relu, stream);
+    }
+  };
+  if (p.epi.stream8) {
+    if (p.epi.relu)
+      run(std::true_type(), std::true_type());
+    else
+      run(std::false_type(), std::true_type());
+  } else if (p.epi.relu) {
+    run(std::true_type(), std::false_type());
+  } else {
+    run(std::false_type(), std::false_type());
   }
   if (blockIdx.x == 0 && tid == 0) epilogue_ranges(p.epi);
 }

@@ -205,6 +205,41 @@ __global__ __launch_bounds__(kThreads) void pool_nhwc_kernel(PoolNhwcArgs a) {
   a.out[i] = out;
 }
 
+// The maximum over 3 x 3 windows (a network's stem).  With the window's extents known all nine
+// loads are on their way at once; a row or column outside the image reads the window's nearest one
+// again, which a maximum does not notice.
+__global__ __launch_bounds__(kThreads) void max3x3_nhwc_kernel(PoolNhwcArgs a) {
+  const size_t i = size_t(blockIdx.x) * kThreads + threadIdx.x;
+  if (i >= a.pieces) return;
+  const int o = static_cast<int>(i / a.chunks);
+  const int chunk = static_cast<int>(i - static_cast<size_t>(o) * a.chunks);
+  const int t = o / a.OW, ow = o - t * a.OW;
+  const int n = t / a.OH, oh = t - n * a.OH;
+  const Window win = window_of(a, oh, ow);
+  v4i out;
+  if (win.h0 < win.h1 && win.w0 < win.w1) {
+    const v4i* img = a.in + static_cast<size_t>(n) * a.H * a.W * a.chunks + chunk;
+    v4i v[9];
+#pragma unroll
+    for (int h = 0; h < 3; ++h)
+#pragma unroll
+      for (int w = 0; w < 3; ++w)
+        v[3 * h + w] = img[(static_cast<size_t>(min(win.h0 + h, win.h1 - 1)) * a.W +
+                            min(win.w0 + w, win.w1 - 1)) * a.chunks];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      s2 even = s2{-32768, -32768}, odd = even;
+#pragma unroll
+      for (int k = 0; k < 9; ++k) max_bytes(static_cast<uint32_t>(v[k][q]), even, odd);
+      out[q] = static_cast<int>((__builtin_bit_cast(uint32_t, even) >> 8) |
+                                __builtin_bit_cast(uint32_t, odd));
+    }
+  } else {
+    out = v4i{1, 1, 1, 1} * static_cast<int>(0x80808080u);
+  }
+  a.out[i] = out;
+}
+
 // Averages over large windows (global pooling: one window per image and channel): 16 lanes take
 // 16 pieces of a pixel, 16 such groups the pixels of the window in turn, and the 16 partial sums
 // meet in LDS.  One lane walking a 7 x 7 window alone is 49 dependent round trips to memory.
@@ -373,6 +408,8 @@ int mxq_quantized_pooling_nhwc(void* stream, const int8_t* in, int N, int H, int
   } else if (pool_type == MXQ_POOL_AVG) {
     hipLaunchKernelGGL((pool_nhwc_kernel<true>), dim3(blocks_for(a.pieces)), dim3(kThreads), 0, s,
                        a);
+  } else if (kernel_h == 3 && kernel_w == 3) {
+    hipLaunchKernelGGL(max3x3_nhwc_kernel, dim3(blocks_for(a.pieces)), dim3(kThreads), 0, s, a);
   } else {
     hipLaunchKernelGGL((pool_nhwc_kernel<false>), dim3(blocks_for(a.pieces)), dim3(kThreads), 0,
                        s, a);

@@ -4,6 +4,7 @@ the layers that stay registered operators between them."""
 import pytest
 import torch
 
+from mxnet_amd import _lib, contrib
 from mxnet_amd import quantization as Q
 from mxnet_amd import symbol as S
 from mxnet_amd.executor import Executor
@@ -192,3 +193,24 @@ def test_graphs_that_are_walked():
     sym = S.softmax(S.FullyConnected(data, num_hidden=7, name="f"), name="s")
     check(quantized(sym, {"f_weight": (7, 16), "f_bias": (7,)}), plan=False,
           data=torch.randn(4, 16, device="cuda"))
+
+
+@pytest.mark.parametrize("n,c,h,w,stride,pad,convention", [
+    (1, 16, 1, 1, 1, 1, "valid"), (2, 48, 7, 9, 2, 1, "valid"), (3, 16, 8, 5, 3, 2, "valid"),
+    (1, 64, 33, 20, 1, 0, "valid"), (2, 32, 10, 11, 2, 1, "full"), (1, 16, 4, 4, 3, 1, "full")])
+def test_nhwc_max_over_3x3_windows(n, c, h, w, stride, pad, convention):
+    """The NHWC kernel of the plans against the NCHW operator, -128 and the image's borders among
+    the windows' contents."""
+    g = torch.Generator(device="cuda").manual_seed(h * w)
+    x = torch.randint(-128, -100, (n, c, h, w), device="cuda", generator=g, dtype=torch.int8)
+    lo, hi = (torch.tensor([v], dtype=torch.float32, device="cuda") for v in (-1.0, 1.0))
+    want = contrib.quantized_pooling(x, lo, hi, kernel=(3, 3), stride=(stride,) * 2,
+                                     pad=(pad,) * 2, pool_type="max",
+                                     pooling_convention=convention)[0]
+    oh, ow = want.shape[2:]
+    nhwc = x.permute(0, 2, 3, 1).contiguous()
+    out = torch.empty((n, oh, ow, c), dtype=torch.int8, device="cuda")
+    _lib.check(_lib.lib.mxq_quantized_pooling_nhwc(
+        torch.cuda.current_stream().cuda_stream, nhwc.data_ptr(), n, h, w, c, 3, 3, stride, stride,
+        pad, pad, oh, ow, 0, 1, out.data_ptr()))
+    assert torch.equal(out.permute(0, 3, 1, 2), want)
