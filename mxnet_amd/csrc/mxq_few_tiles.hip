@@ -186,6 +186,19 @@ __global__ __launch_bounds__(64 * W) void few_tiles_kernel(FewTilesArgs p) {
   for (int i = 0; i < 4; ++i)
     bias[i] = (tid < kQuads && n + i < p.N) ? epi_bias32(p.epi, pre.s, n + i) : 0;
 
+  uint32_t residual[kPer];
+  if constexpr (epi_sums(MODE)) {
+    const bool dwords = epi_quad_dwords<MODE>(p.epi, p.N, static_cast<size_t>(p.ldo));
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+      const int q = tid + j * kThreads, m = m0 + q / Q;
+      residual[j] = 0;
+      if (dwords && q < kQuads && m < p.M && n < p.N)
+        residual[j] = *reinterpret_cast<const uint32_t*>(p.epi.res +
+                                                         static_cast<size_t>(m) * p.ldo + n);
+    }
+  }
+
   // lane: activation row lane % 16, output columns 4 * (lane / 16) ... + 3
   v4i acc[F][F];
 #pragma unroll
@@ -240,7 +253,8 @@ __global__ __launch_bounds__(64 * W) void few_tiles_kernel(FewTilesArgs p) {
     int v[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) v[i] = static_cast<int>(sum[i] + static_cast<uint32_t>(bias[i]));
-    epi_store_quad<MODE>(p.epi, pre, v, m, n, p.N, static_cast<size_t>(p.ldo));
+    epi_store_quad<MODE>(p.epi, pre, v, m, n, p.N, static_cast<size_t>(p.ldo),
+                         epi_sums(MODE) ? residual[j] : 0);
   }
 }
 

@@ -713,15 +713,18 @@ __device__ __forceinline__ auto epi_sum_rule(const Epilogue& e) {
   const float a = dev_maxabs(-e.real_range, e.real_range);
   const float b = dev_maxabs(*e.res_min, *e.res_max);
   if constexpr (MODE == kEpiSumRq) {
-    RequantRule r = sum_requant_rule(a, b, e.sum_min_calib, e.sum_max_calib);
-    if (e.sum_pairs != nullptr && e.sum_relu && r.fast) {
+    // a short form exists for fast rules only, and every path takes it before it looks at the scales
+    if (e.sum_pairs != nullptr && e.sum_relu && e.sum_pairs->ok) {
+      RequantRule r = {};
+      r.fast = r.pairs = 1;
       r.ta = e.sum_pairs->ta;
       r.tb = e.sum_pairs->tb;
-      r.pairs = e.sum_pairs->ok;
+      return r;
     }
-    return r;
-  } else
+    return sum_requant_rule(a, b, e.sum_min_calib, e.sum_max_calib);
+  } else {
     return sum_rule(a, b, e.sum_min_calib, e.sum_max_calib);
+  }
 }
 
 template <class Cfg, int MODE = kEpiPlain>
@@ -782,8 +785,7 @@ __device__ __forceinline__ void gemm_epilogue(v16i (&acc)[Cfg::MI][Cfg::NI], con
                 const int b = static_cast<int>(e.res[off + i]);
                 uint32_t v8;
                 if constexpr (MODE == kEpiSumRq)
-                  v8 = static_cast<uint32_t>(e.sum_relu ? sum_requant_one<true>(q[i], b, r)
-                                                        : sum_requant_one<false>(q[i], b, r));
+                  v8 = static_cast<uint32_t>(sum_requant_any(q[i], b, e.sum_relu != 0, r));
                 else
                   v8 = e.sum_relu ? sum_one<true, false>(q[i], b, r)
                                   : sum_one<false, false>(q[i], b, r);
@@ -879,8 +881,7 @@ __device__ __forceinline__ int8_t epi_sum_one(int a, int b, bool relu,
 }
 __device__ __forceinline__ int8_t epi_sum_one(int a, int b, bool relu,
                                               const EpiPreOf<kEpiSumRq>& pre) {
-  return static_cast<int8_t>(relu ? sum_requant_one<true>(a, b, pre.sum)
-                                  : sum_requant_one<false>(a, b, pre.sum));
+  return static_cast<int8_t>(sum_requant_any(a, b, relu, pre.sum));
 }
 template <int MODE>
 __device__ __forceinline__ EpiPreOf<MODE> epi_prefetch_scalars(const Epilogue& e) {
@@ -891,12 +892,20 @@ __device__ __forceinline__ EpiPreOf<MODE> epi_prefetch_scalars(const Epilogue& e
   return p;
 }
 
+// Whether epi_store_quad moves the int8 output, and a sum's residual operand, in dwords.
+template <int MODE>
+__device__ __forceinline__ bool epi_quad_dwords(const Epilogue& e, int N, size_t ldo) {
+  return (N & 3) == 0 && (ldo & 3) == 0 && (reinterpret_cast<uintptr_t>(e.out8) & 3u) == 0 &&
+         (!epi_sums(MODE) || (reinterpret_cast<uintptr_t>(e.res) & 3u) == 0);
+}
+
 // One lane's four adjacent columns n ... n + 3 of row m, bias included, into every output the
 // launch has: vector stores where the row pitch allows them, element by element elsewhere.
+// `residual`: those four bytes of a sum's residual operand where epi_quad_dwords.
 template <int MODE>
 __device__ __forceinline__ void epi_store_quad(const Epilogue& e, const EpiPreOf<MODE>& pre,
                                                const int (&v)[4], int m, int n, int N,
-                                               size_t ldo) {
+                                               size_t ldo, uint32_t residual) {
   const bool full = (N & 3) == 0 && (ldo & 3) == 0;  // then n + 3 < N as well
   const size_t off = static_cast<size_t>(m) * ldo + n;
   if (MODE == kEpiPlain && e.out32 != nullptr) {
@@ -931,17 +940,20 @@ __device__ __forceinline__ void epi_store_quad(const Epilogue& e, const EpiPreOf
     }
     return;
   }
-  const bool dwords = full && (reinterpret_cast<uintptr_t>(e.out8) & 3u) == 0 &&
-                      (!epi_sums(MODE) || (reinterpret_cast<uintptr_t>(e.res) & 3u) == 0);
-  if (dwords) {
-    if (epi_sums(MODE)) {
-      const uint32_t r = *reinterpret_cast<const uint32_t*>(e.res + off);
+  if (epi_quad_dwords<MODE>(e, N, ldo)) {
+    uint32_t w = pack_bytes(q[0], q[1], q[2], q[3]);
+    if constexpr (epi_sums(MODE)) {
+      if (epi_sum_pairs(pre)) {
+        w = epi_sum_pairs4(w, residual, pre);
+      } else {
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        q[i] = epi_sum_one(q[i], static_cast<int8_t>((r >> (8 * i)) & 0xffu), e.sum_relu != 0,
-                           pre);
+        for (int i = 0; i < 4; ++i)
+          q[i] = epi_sum_one(q[i], static_cast<int8_t>((residual >> (8 * i)) & 0xffu),
+                             e.sum_relu != 0, pre);
+        w = pack_bytes(q[0], q[1], q[2], q[3]);
+      }
     }
-    *reinterpret_cast<uint32_t*>(e.out8 + off) = pack_bytes(q[0], q[1], q[2], q[3]);
+    *reinterpret_cast<uint32_t*>(e.out8 + off) = w;
   } else {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {

@@ -70,7 +70,8 @@ struct RequantRule {
   float in_scale;  // float per int32 level
   float qscale;    // int8 levels per float
   int fast;        // no product overflows and nothing is NaN: the sum needs no saturation
-  float ta, tb;    // the short form, where `pairs` says that it holds (SumPairs)
+  float ta, tb;    // the short form, where `pairs` says that it holds (SumPairs): the scales
+                   // above are then left out
   int pairs;
 };
 
@@ -137,6 +138,14 @@ __device__ __forceinline__ int sum_requant_one(int a, int b, const RequantRule& 
   const int v = static_cast<int>(u);
   const int s = f < 0.0f ? -v : (f > 0.0f ? v : 0);
   return RELU && s < 0 ? 0 : s;
+}
+
+// One element under whatever form the rule has.
+__device__ __forceinline__ int sum_requant_any(int a, int b, bool relu, const RequantRule& r) {
+  if (r.pairs)
+    return static_cast<int>(sum_pairs4(static_cast<uint32_t>(a) & 0xffu,
+                                       static_cast<uint32_t>(b) & 0xffu, r) & 0xffu);
+  return relu ? sum_requant_one<true>(a, b, r) : sum_requant_one<false>(a, b, r);
 }
 
 // One element: saturate, round to nearest even, NaN -> 0; with RELU the negative results

@@ -66,6 +66,25 @@ def test_short_form_is_the_sum(m, k, n, ranges):
     assert torch.equal(call(pairs), want)
 
 
+@pytest.mark.parametrize("m,k,n", [(33, 64, 64), (130, 96, 132), (65, 128, 37), (40, 256, 128)])
+@pytest.mark.parametrize("force", [(1, 1, 0), (3, 1, 0), (4, 1, 0), (43, 1, 0), (44, 1, 0),
+                                   (55, 1, 0), (71, 4, 0), (71, -8, 0)])
+def test_short_form_on_every_kind_of_kernel(m, k, n, force):
+    """Register-staged, direct-to-LDS and few-tiles kernels, rows on and off the 4- and 16-byte
+    marks."""
+    g = torch.Generator(device="cuda").manual_seed(m + k + n)
+    draw = lambda *s: torch.randint(-128, 128, s, device="cuda", generator=g, dtype=torch.int8)
+    data, weight, bias, res = draw(m, k), draw(n, k), draw(n), draw(m, n)
+    args = [scalar(v) for v in (-1.0, 1.0, -2.0, 2.0, -0.5, 0.5, -2.0, 2.0)]
+    reach = 3.0 * k ** 0.5
+    pairs = capi.sum_requant_pairs((-reach, reach), (-2.0, 2.0), (-4.0, 4.0))
+    assert int(pairs[2]) == 1
+    got, want = (capi.quantized_fc_sum(data, weight, bias, res, *args, (-reach, reach),
+                                       (-4.0, 4.0), sum_relu=True, requant=True, force=force,
+                                       pairs=p)["out8"] for p in (pairs, None))
+    assert torch.equal(got, want)
+
+
 def test_short_form_is_found_for_most_ranges():
     g = torch.Generator().manual_seed(0)
     found = [capi.sum_requant_pairs(*((-v, v) for v in (0.5 + 4 * torch.rand(3, generator=g))
