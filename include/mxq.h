@@ -362,6 +362,32 @@ int mxq_quantized_fc_sum_requant(void* stream, const int8_t* data, const int8_t*
                                  float sum_max_calib, int sum_relu, const void* pairs,
                                  void* workspace, size_t workspace_bytes);
 
+/* The layers above, and mxq_quantized_conv_nhwc, for ranges that stay: mxq_prepare_layer computes
+ * what a launch derives from the six ranges, the calibrated range and the bias once, into
+ * 64 + 4 * N bytes on the device (16-byte aligned); the _prepared entries take it instead of them,
+ * write the same int8 (or dequantized float) output and no ranges. */
+int mxq_prepare_layer(void* stream, const int8_t* bias, int N, const float* min_data,
+                      const float* max_data, const float* min_weight, const float* max_weight,
+                      const float* min_bias, const float* max_bias, float min_calib,
+                      float max_calib, void* prepared);
+int mxq_quantized_fc_prepared(void* stream, const int8_t* data, const int8_t* weight,
+                              const void* prepared, int M, int N, int K, int8_t* out8,
+                              float* out_f32, int relu, float min_calib, float max_calib,
+                              void* workspace, size_t workspace_bytes);
+int mxq_quantized_fc_sum_prepared(void* stream, const int8_t* data, const int8_t* weight,
+                                  const void* prepared, int M, int N, int K,
+                                  const int8_t* residual, const float* min_residual,
+                                  const float* max_residual, int8_t* out8, float min_calib,
+                                  float max_calib, float sum_min_calib, float sum_max_calib,
+                                  int sum_relu, int requant, const void* pairs, void* workspace,
+                                  size_t workspace_bytes);
+int mxq_quantized_conv_nhwc_prepared(void* stream, const int8_t* data, const int8_t* weight,
+                                     const void* prepared, int N, int H, int W, int C, int O,
+                                     int KH, int KW, int stride_h, int stride_w, int pad_h,
+                                     int pad_w, int dilate_h, int dilate_w, int8_t* out8, int relu,
+                                     float min_calib, float max_calib, void* workspace,
+                                     size_t workspace_bytes);
+
 /* Looks for a short form of that sum with sum_relu != 0 over ranges that stay: two products and
  * one rounding that give the same int8 for every pair of int8 operands, which is tried out on
  * the device.  Writes 12 bytes to `pairs` (device, 4-byte aligned), among them whether one was

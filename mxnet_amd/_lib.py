@@ -69,6 +69,12 @@ SIGNATURES = {
                              [_p, _p, _p, _p, _p, _f, _f, _f, _f, _i, _p, _sz]),
     "mxq_quantized_fc_sum_requant": (_i, [_p, _p, _p, _p, _i, _i, _i] + [_p] * 6 + [_p, _p, _p] +
                                      [_p, _p, _p, _p, _p, _f, _f, _f, _f, _i, _p, _p, _sz]),
+    "mxq_prepare_layer": (_i, [_p, _p, _i] + [_p] * 6 + [_f, _f, _p]),
+    "mxq_quantized_fc_prepared": (_i, [_p] * 4 + [_i] * 3 + [_p, _p, _i, _f, _f, _p, _sz]),
+    "mxq_quantized_fc_sum_prepared": (_i, [_p] * 4 + [_i] * 3 + [_p] * 4 + [_f] * 4 +
+                                      [_i, _i, _p, _p, _sz]),
+    "mxq_quantized_conv_nhwc_prepared": (_i, [_p] * 4 + [_i] * 13 +
+                                         [_p, _i, _f, _f, _p, _sz]),
     "mxq_sum_requant_pairs": (_i, [_p, _f, _f, _f, _f, _f, _f, _p]),
     "mxq_quantized_conv_workspace": (_sz, [_i] * 14),
     "mxq_quantized_conv_nhwc": (_i, [_p, _p, _p, _p] + [_i] * 13 + [_p] * 6 +

@@ -652,11 +652,27 @@ class _Builder:
 
         steps = []
         for kind, ints, floats, refs, node, blobs in self.steps:
+            places = [place(r) for r in refs]
+            if kind in (_CONV, _FC, _FC_F32, _FC_SUM, _FC_SUM_RQ):
+                places.append(self.prepared(ints[4 if kind == _CONV else 1], floats, places))
             step = (kind, tuple(int(v) for v in ints), tuple(float(v) for v in floats),
-                    tuple(place(r) for r in refs))
+                    tuple(places))
             steps.append(step if node is None else step + (node._call, blobs))
         plan = _frontend.plan(size, self.held, steps, [(f, tuple(s)) for f, s in outputs])
         return plan, tuple((name, t, t._version) for name, t in self.params.items())
+
+
+    def prepared(self, columns, calib, places):
+        """What mxq_prepare_layer makes of a layer's bias and six ranges, if they stay."""
+        given = places[2:9]
+        if any(base not in (_HELD, _NULL) for base, _, _ in given):
+            return (_NULL, 0, 0)
+        at = [None if base == _NULL else self.held[i].data_ptr() + offset
+              for base, i, offset in given]
+        out = torch.empty(64 + 4 * columns, dtype=torch.int8, device=self.device)
+        _lib.check(_lib.lib.mxq_prepare_layer(self.stream, at[0], int(columns), *at[1:],
+                                              float(calib[0]), float(calib[1]), out.data_ptr()))
+        return self.hold(out).place
 
 
 class _Offset:

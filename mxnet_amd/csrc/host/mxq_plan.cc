@@ -40,36 +40,57 @@ bool Plan::run(void* stream, const std::vector<at::Tensor>& feeds,
         }
         continue;
       }
-      // refs: data, weight, bias, six ranges, scratch, output, workspace[, residual, its range[, pairs]]
+      // refs: data, weight, bias, six ranges, scratch, output, workspace[, residual, its
+      // range[, pairs]], what mxq_prepare_layer made of bias and ranges where those stay
       case Kind::kConv:
-        rc = mxq_quantized_conv_nhwc(stream, q(0), q(1), q(2), i(0), i(1), i(2), i(3), i(4), i(5),
-                                     i(6), i(7), i(8), i(9), i(10), i(11), i(12), v(3), v(4), v(5),
-                                     v(6), v(7), v(8), nullptr, v(9), v(9) + 1, q(10), v(9) + 2,
-                                     v(9) + 3, i(13), f[0], f[1], p(11),
-                                     static_cast<size_t>(n[14]));
+        if (const void* prepared = at(s.refs.back()))
+          rc = mxq_quantized_conv_nhwc_prepared(
+              stream, q(0), q(1), prepared, i(0), i(1), i(2), i(3), i(4), i(5), i(6), i(7), i(8),
+              i(9), i(10), i(11), i(12), q(10), i(13), f[0], f[1], p(11),
+              static_cast<size_t>(n[14]));
+        else
+          rc = mxq_quantized_conv_nhwc(
+              stream, q(0), q(1), q(2), i(0), i(1), i(2), i(3), i(4), i(5), i(6), i(7), i(8), i(9),
+              i(10), i(11), i(12), v(3), v(4), v(5), v(6), v(7), v(8), nullptr, v(9), v(9) + 1,
+              q(10), v(9) + 2, v(9) + 3, i(13), f[0], f[1], p(11), static_cast<size_t>(n[14]));
         break;
       case Kind::kFc:
-        rc = mxq_quantized_fc(stream, q(0), q(1), q(2), i(0), i(1), i(2), v(3), v(4), v(5), v(6),
-                              v(7), v(8), nullptr, v(9), v(9) + 1, q(10), v(9) + 2, v(9) + 3,
-                              i(3), f[0], f[1], p(11), static_cast<size_t>(n[4]));
+      case Kind::kFcF32: {
+        const bool floats = s.kind == Kind::kFcF32;
+        if (const void* prepared = at(s.refs.back()))
+          rc = mxq_quantized_fc_prepared(stream, q(0), q(1), prepared, i(0), i(1), i(2),
+                                         floats ? nullptr : q(10), floats ? v(10) : nullptr, i(3),
+                                         f[0], f[1], p(11), static_cast<size_t>(n[4]));
+        else if (floats)
+          rc = mxq_quantized_fc_f32(stream, q(0), q(1), q(2), i(0), i(1), i(2), v(3), v(4), v(5),
+                                    v(6), v(7), v(8), v(10), v(9), v(9) + 1, v(9) + 2, v(9) + 3,
+                                    i(3), f[0], f[1], p(11), static_cast<size_t>(n[4]));
+        else
+          rc = mxq_quantized_fc(stream, q(0), q(1), q(2), i(0), i(1), i(2), v(3), v(4), v(5), v(6),
+                                v(7), v(8), nullptr, v(9), v(9) + 1, q(10), v(9) + 2, v(9) + 3,
+                                i(3), f[0], f[1], p(11), static_cast<size_t>(n[4]));
         break;
-      case Kind::kFcF32:
-        rc = mxq_quantized_fc_f32(stream, q(0), q(1), q(2), i(0), i(1), i(2), v(3), v(4), v(5),
-                                  v(6), v(7), v(8), v(10), v(9), v(9) + 1, v(9) + 2, v(9) + 3,
-                                  i(3), f[0], f[1], p(11), static_cast<size_t>(n[4]));
-        break;
+      }
       case Kind::kFcSum:
-        rc = mxq_quantized_fc_sum(stream, q(0), q(1), q(2), i(0), i(1), i(2), v(3), v(4), v(5),
-                                  v(6), v(7), v(8), q(12), v(13), v(14), q(10), v(9), v(9) + 1,
-                                  v(9) + 2, v(9) + 3, f[0], f[1], f[2], f[3], i(3), p(11),
-                                  static_cast<size_t>(n[4]));
+      case Kind::kFcSumRq: {
+        const bool requant = s.kind == Kind::kFcSumRq;
+        const void* pairs = requant ? p(15) : nullptr;
+        if (const void* prepared = at(s.refs.back()))
+          rc = mxq_quantized_fc_sum_prepared(
+              stream, q(0), q(1), prepared, i(0), i(1), i(2), q(12), v(13), v(14), q(10), f[0],
+              f[1], f[2], f[3], i(3), requant, pairs, p(11), static_cast<size_t>(n[4]));
+        else if (requant)
+          rc = mxq_quantized_fc_sum_requant(
+              stream, q(0), q(1), q(2), i(0), i(1), i(2), v(3), v(4), v(5), v(6), v(7), v(8),
+              q(12), v(13), v(14), q(10), v(9), v(9) + 1, v(9) + 2, v(9) + 3, f[0], f[1], f[2],
+              f[3], i(3), pairs, p(11), static_cast<size_t>(n[4]));
+        else
+          rc = mxq_quantized_fc_sum(stream, q(0), q(1), q(2), i(0), i(1), i(2), v(3), v(4), v(5),
+                                    v(6), v(7), v(8), q(12), v(13), v(14), q(10), v(9), v(9) + 1,
+                                    v(9) + 2, v(9) + 3, f[0], f[1], f[2], f[3], i(3), p(11),
+                                    static_cast<size_t>(n[4]));
         break;
-      case Kind::kFcSumRq:
-        rc = mxq_quantized_fc_sum_requant(stream, q(0), q(1), q(2), i(0), i(1), i(2), v(3), v(4),
-                                          v(5), v(6), v(7), v(8), q(12), v(13), v(14), q(10),
-                                          v(9), v(9) + 1, v(9) + 2, v(9) + 3, f[0], f[1], f[2],
-                                          f[3], i(3), p(15), p(11), static_cast<size_t>(n[4]));
-        break;
+      }
       case Kind::kQuantNhwc:
         rc = mxq_quantize_to_nhwc(stream, v(0), q(1), v(2), v(2) + 1, i(0), i(1), i(2), i(3),
                                   i(4), i(5), i(6), i(7), f[0], f[1]);

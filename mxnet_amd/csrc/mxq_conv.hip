@@ -1413,14 +1413,17 @@ void conv_nhwc(void* stream, const int8_t* data, const int8_t* weight, const int
                const float* max_data, const float* min_weight, const float* max_weight,
                const float* min_bias, const float* max_bias, int32_t* out32, float* omin,
                float* omax, int8_t* out8, float* rmin, float* rmax, int relu, float min_calib,
-               float max_calib, bool planar, const GemmForce& force, const Workspace& ws) {
+               float max_calib, bool planar, const GemmForce& force, const Workspace& ws,
+               const void* prepared = nullptr) {
   const ConvGeometry g = conv_geometry(N, H, W, C, O, KH, KW, stride_h, stride_w, pad_h, pad_w,
                                        dilate_h, dilate_w);
-  MXQ_CHECK(min_data && max_data && min_weight && max_weight, "null input range pointer");
-  MXQ_CHECK(omin && omax, "null output range pointer");
-  MXQ_CHECK(bias == nullptr || (min_bias && max_bias), "bias given without its range");
+  if (prepared == nullptr) {
+    MXQ_CHECK(min_data && max_data && min_weight && max_weight, "null input range pointer");
+    MXQ_CHECK(omin && omax, "null output range pointer");
+    MXQ_CHECK(bias == nullptr || (min_bias && max_bias), "bias given without its range");
+    MXQ_CHECK(out8 == nullptr || (rmin && rmax), "fused requantize needs rmin/rmax");
+  }
   MXQ_CHECK(N == 0 || out32 != nullptr || out8 != nullptr, "no output buffer");
-  MXQ_CHECK(out8 == nullptr || (rmin && rmax), "fused requantize needs rmin/rmax");
   ConvArgs a;
   a.data = data;
   a.weight = weight;
@@ -1445,6 +1448,7 @@ void conv_nhwc(void* stream, const int8_t* data, const int8_t* weight, const int
   e.res = nullptr; e.res_min = nullptr; e.res_max = nullptr;
   e.sum_min_calib = 0.f; e.sum_max_calib = 0.f; e.sum_relu = 0; e.sum_requant = 0; e.with_sum = 0;
   e.sum_pairs = nullptr;
+  e.prepared = static_cast<const char*>(prepared);
   e.omin = omin; e.omax = omax; e.rmin = rmin; e.rmax = rmax;
   e.relu = relu;
   float x = fabsf(min_calib), y = fabsf(max_calib);
@@ -1476,7 +1480,7 @@ void conv_nhwc(void* stream, const int8_t* data, const int8_t* weight, const int
       conv_nhwc(stream, d, w, bias, N, H, W, Cp, O, KH, KW, stride_h, stride_w, pad_h, pad_w,
                 dilate_h, dilate_w, min_data, max_data, min_weight, max_weight, min_bias,
                 max_bias, out32, omin, omax, out8, rmin, rmax, relu, min_calib, max_calib, planar,
-                force, rest);
+                force, rest, prepared);
       return;
     }
   }
@@ -1606,6 +1610,24 @@ size_t mxq_quantized_conv_workspace(int N, int H, int W, int C, int O, int KH, i
   } catch (...) {
     return 0;
   }
+}
+
+int mxq_quantized_conv_nhwc_prepared(void* stream, const int8_t* data, const int8_t* weight,
+                                     const void* prepared, int N, int H, int W, int C, int O,
+                                     int KH, int KW, int stride_h, int stride_w, int pad_h,
+                                     int pad_w, int dilate_h, int dilate_w, int8_t* out8, int relu,
+                                     float min_calib, float max_calib, void* workspace,
+                                     size_t workspace_bytes) {
+  MXQ_API_BEGIN();
+  MXQ_CHECK(prepared != nullptr && aligned16(prepared), "null or unaligned pointer");
+  Workspace ws;
+  ws.ptr = workspace;
+  ws.bytes = workspace_bytes;
+  conv_nhwc(stream, data, weight, nullptr, N, H, W, C, O, KH, KW, stride_h, stride_w, pad_h, pad_w,
+            dilate_h, dilate_w, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr,
+            nullptr, nullptr, out8, nullptr, nullptr, relu, min_calib, max_calib, false,
+            GemmForce(), ws, prepared);
+  MXQ_API_END();
 }
 
 int mxq_quantized_conv_nhwc(void* stream, const int8_t* data, const int8_t* weight,

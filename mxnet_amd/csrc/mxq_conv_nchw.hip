@@ -322,8 +322,8 @@ __global__ __launch_bounds__(Cfg::kThreads, 2) void conv1x1_planes_kernel(PlaneA
     issue(0);
   }
   // what the epilogue needs, behind the first operand fetch
-  const EpiScalars es = epi_scalars(p.epi);
-  if (tid < Cfg::BO) sbias[tid] = (o0 + tid < p.O) ? epi_bias32(p.epi, es, o0 + tid) : 0;
+  const EpiScalars es = epi_scalars_computed(p.epi);
+  if (tid < Cfg::BO) sbias[tid] = (o0 + tid < p.O) ? epi_bias32_computed(p.epi, es, o0 + tid) : 0;
 
   PLANE_STAMP(1);
   if constexpr (!gathered) {

@@ -202,6 +202,14 @@ __global__ __launch_bounds__(1024) void sum_pairs_kernel(float layer_range,
   }
 }
 
+// The scalars and the int32 bias of a layer whose ranges stay, the bits a launch computes itself.
+__global__ __launch_bounds__(256) void prepare_layer_kernel(Epilogue e, int N, char* out) {
+  const EpiScalars s = epi_scalars(e);
+  const int n = blockIdx.x * 256 + threadIdx.x;
+  if (n == 0) *reinterpret_cast<EpiScalars*>(out) = s;
+  if (n < N) reinterpret_cast<int*>(out + kPreparedBias)[n] = epi_bias32(e, s, n);
+}
+
 // an output without elements still owes its range scalars
 __global__ void gemm_ranges_kernel(Epilogue e) { epilogue_ranges<kEpiSum>(e); }
 
@@ -330,15 +338,17 @@ void fc_entry(void* stream, const int8_t* data, const int8_t* weight, const int8
               const float* max_bias, int32_t* out32, float* omin, float* omax, int8_t* out8,
               float* out_f32, float* rmin, float* rmax, int relu, float min_calib,
               float max_calib, void* workspace, size_t workspace_bytes, const GemmForce& force,
-              const SumArgs* sum = nullptr) {
+              const SumArgs* sum = nullptr, const void* prepared = nullptr) {
   MXQ_CHECK(M >= 0 && N >= 0 && K >= 0, "negative dimension");
-  MXQ_CHECK(min_data && max_data && min_weight && max_weight, "null input range pointer");
-  MXQ_CHECK(omin && omax, "null output range pointer");
-  MXQ_CHECK(bias == nullptr || (min_bias && max_bias), "bias given without its range");
+  if (prepared == nullptr) {
+    MXQ_CHECK(min_data && max_data && min_weight && max_weight, "null input range pointer");
+    MXQ_CHECK(omin && omax, "null output range pointer");
+    MXQ_CHECK(bias == nullptr || (min_bias && max_bias), "bias given without its range");
+    MXQ_CHECK((out8 == nullptr && out_f32 == nullptr) || (rmin && rmax),
+              "fused requantize needs rmin/rmax");
+  }
   MXQ_CHECK(M == 0 || N == 0 || out32 != nullptr || out8 != nullptr || out_f32 != nullptr,
             "no output buffer");
-  MXQ_CHECK((out8 == nullptr && out_f32 == nullptr) || (rmin && rmax),
-            "fused requantize needs rmin/rmax");
   MXQ_CHECK(M == 0 || N == 0 || K == 0 || (data != nullptr && weight != nullptr),
             "null operand pointer");
   Epilogue e;
@@ -376,6 +386,7 @@ void fc_entry(void* stream, const int8_t* data, const int8_t* weight, const int8
     e.sum_pairs = sum->pairs;
     e.with_sum = 1;
   }
+  e.prepared = static_cast<const char*>(prepared);
   e.omin = omin;
   e.omax = omax;
   e.rmin = rmin;
@@ -489,6 +500,62 @@ int mxq_quantized_fc_sum_requant(void* stream, const int8_t* data, const int8_t*
   fc_entry(stream, data, weight, bias, M, N, K, min_data, max_data, min_weight, max_weight,
            min_bias, max_bias, nullptr, omin, omax, out8, nullptr, rmin, rmax, 0, min_calib,
            max_calib, workspace, workspace_bytes, GemmForce(), &sum);
+  MXQ_API_END();
+}
+
+int mxq_prepare_layer(void* stream, const int8_t* bias, int N, const float* min_data,
+                      const float* max_data, const float* min_weight, const float* max_weight,
+                      const float* min_bias, const float* max_bias, float min_calib,
+                      float max_calib, void* prepared) {
+  MXQ_API_BEGIN();
+  MXQ_CHECK(N >= 0, "negative dimension");
+  MXQ_CHECK(min_data && max_data && min_weight && max_weight, "null input range pointer");
+  MXQ_CHECK(bias == nullptr || (min_bias && max_bias), "bias given without its range");
+  MXQ_CHECK(prepared != nullptr && aligned16(prepared), "null or unaligned pointer");
+  Epilogue e = {};
+  e.bias = bias;
+  e.min_data = min_data;
+  e.max_data = max_data;
+  e.min_weight = min_weight;
+  e.max_weight = max_weight;
+  e.min_bias = min_bias;
+  e.max_bias = max_bias;
+  const float a = fabsf(min_calib), b = fabsf(max_calib);
+  e.real_range = (a < b) ? b : a;
+  hipLaunchKernelGGL(prepare_layer_kernel, dim3(static_cast<unsigned>(N / 256 + 1)), dim3(256), 0,
+                     static_cast<hipStream_t>(stream), e, N, static_cast<char*>(prepared));
+  MXQ_LAUNCH_CHECK();
+  MXQ_API_END();
+}
+
+int mxq_quantized_fc_prepared(void* stream, const int8_t* data, const int8_t* weight,
+                              const void* prepared, int M, int N, int K, int8_t* out8,
+                              float* out_f32, int relu, float min_calib, float max_calib,
+                              void* workspace, size_t workspace_bytes) {
+  MXQ_API_BEGIN();
+  MXQ_CHECK(prepared != nullptr && aligned16(prepared), "null or unaligned pointer");
+  MXQ_CHECK((out8 == nullptr) != (out_f32 == nullptr), "one output buffer");
+  fc_entry(stream, data, weight, nullptr, M, N, K, nullptr, nullptr, nullptr, nullptr, nullptr,
+           nullptr, nullptr, nullptr, nullptr, out8, out_f32, nullptr, nullptr, relu, min_calib,
+           max_calib, workspace, workspace_bytes, GemmForce(), nullptr, prepared);
+  MXQ_API_END();
+}
+
+int mxq_quantized_fc_sum_prepared(void* stream, const int8_t* data, const int8_t* weight,
+                                  const void* prepared, int M, int N, int K,
+                                  const int8_t* residual, const float* min_residual,
+                                  const float* max_residual, int8_t* out8, float min_calib,
+                                  float max_calib, float sum_min_calib, float sum_max_calib,
+                                  int sum_relu, int requant, const void* pairs, void* workspace,
+                                  size_t workspace_bytes) {
+  MXQ_API_BEGIN();
+  MXQ_CHECK(prepared != nullptr && aligned16(prepared), "null or unaligned pointer");
+  MXQ_CHECK((reinterpret_cast<uintptr_t>(pairs) & 3u) == 0, "unaligned pairs");
+  const SumArgs sum = {residual, min_residual, max_residual, sum_min_calib, sum_max_calib,
+                       sum_relu, requant, requant ? static_cast<const SumPairs*>(pairs) : nullptr};
+  fc_entry(stream, data, weight, nullptr, M, N, K, nullptr, nullptr, nullptr, nullptr, nullptr,
+           nullptr, nullptr, nullptr, nullptr, out8, nullptr, nullptr, nullptr, 0, min_calib,
+           max_calib, workspace, workspace_bytes, GemmForce(), &sum, prepared);
   MXQ_API_END();
 }
 

@@ -44,6 +44,21 @@ namespace mxq {
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 
+// Scalars every thread needs in the epilogue.
+struct EpiScalars {
+  float max_out;   // QuantizationRangeForMultiplication, quantization_utils.h:141-157
+  float foq, fbq;  // float per int32 level / per int8 bias level
+  float in_scale;  // max_out / 2^31
+  float qscale;    // 127 / R
+  float dqscale;   // R / 127: float per int8 level of the requantized output
+};
+
+// A layer whose ranges stay (a plan's constants): its scalars, and behind them the int32 bias of
+// every output column, computed once by prepare_layer_kernel (mxq_fc.hip).  Computing them is a
+// chain of loads and eleven divisions, two of them in double, in front of every launch's epilogue:
+// quantized ResNet-50 on one image 263 us with it, 240 without.
+constexpr int kPreparedBias = 64;  // bytes in front of the bias
+
 struct Epilogue {
   const int8_t* bias;      // int8 [N] or null
   const float* min_data;   // device scalars
@@ -69,6 +84,7 @@ struct Epilogue {
   int sum_requant;         // the sum in int32 over its own range, then requantized (RequantRule)
   const SumPairs* sum_pairs;  // device, or null: the short form of that rule
   int with_sum;            // rmin / rmax report the sum's range (also for an empty output)
+  const char* prepared;    // device, or null: EpiScalars and the int32 bias (kPreparedBias)
   float* omin;             // int32 output range
   float* omax;
   float* rmin;             // requantized range (only with out8)
@@ -117,16 +133,7 @@ __device__ __forceinline__ float dev_maxabs(float a, float b) {
   return (x < y) ? y : x;
 }
 
-// Scalars every thread needs in the epilogue.
-struct EpiScalars {
-  float max_out;   // QuantizationRangeForMultiplication, quantization_utils.h:141-157
-  float foq, fbq;  // float per int32 level / per int8 bias level
-  float in_scale;  // max_out / 2^31
-  float qscale;    // 127 / R
-  float dqscale;   // R / 127: float per int8 level of the requantized output
-};
-
-__device__ __forceinline__ EpiScalars epi_scalars(const Epilogue& e) {
+__device__ __forceinline__ EpiScalars epi_scalars_computed(const Epilogue& e) {
   EpiScalars s;
   const float la = dev_maxabs(*e.min_data, *e.max_data) / 127.0f;
   const float lb = dev_maxabs(*e.min_weight, *e.max_weight) / 127.0f;
@@ -143,10 +150,23 @@ __device__ __forceinline__ EpiScalars epi_scalars(const Epilogue& e) {
   return s;
 }
 
-__device__ __forceinline__ int epi_bias32(const Epilogue& e, const EpiScalars& s, int n) {
+__device__ __forceinline__ int epi_bias32_computed(const Epilogue& e, const EpiScalars& s, int n) {
   if (e.bias == nullptr || s.foq == 0.0f) return 0;
   float p = static_cast<float>(static_cast<int>(e.bias[n])) * s.fbq;
   return static_cast<int>(p / s.foq);
+}
+
+// The same where the launch may have them ready (unlikely to the compiler: a launch that computes
+// them keeps its straight code).
+__device__ __forceinline__ EpiScalars epi_scalars(const Epilogue& e) {
+  if (__builtin_expect(e.prepared != nullptr, 0))
+    return *reinterpret_cast<const EpiScalars*>(e.prepared);
+  return epi_scalars_computed(e);
+}
+__device__ __forceinline__ int epi_bias32(const Epilogue& e, const EpiScalars& s, int n) {
+  if (__builtin_expect(e.prepared != nullptr, 0))
+    return reinterpret_cast<const int*>(e.prepared + kPreparedBias)[n];
+  return epi_bias32_computed(e, s, n);
 }
 
 // FloatToQuantized<int8>(float(acc) * in_scale): trunc(sign(f) * min(|f|*s + 0.5, 127)),
@@ -1446,7 +1466,8 @@ __device__ __forceinline__ bool splitk_gather(v16i (&acc)[Cfg::MI][Cfg::NI], con
 // (three more scalar registers, which some of the tiled kernels do not have to spare).
 template <int MODE = kEpiPlain>
 __device__ __forceinline__ void epilogue_ranges(const Epilogue& e) {
-  const EpiScalars s = epi_scalars(e);
+  if (__builtin_expect(e.prepared != nullptr, 0)) return;  // the caller knows them
+  const EpiScalars s = epi_scalars_computed(e);
   *e.omin = -s.max_out;
   *e.omax = s.max_out;
   // also for an output without elements, whose buffer pointer may be null
