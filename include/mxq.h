@@ -480,6 +480,36 @@ int mxq_pack_weight(void* stream, const int8_t* in, int8_t* out, int O, int C, i
 int mxq_nhwc_pad_to_nchw_i8(void* stream, const int8_t* in, int8_t* out, int N, int C, int H,
                             int W, int C_padded);
 
+/* The tail of a residual block over NHWC activations as one launch (channel counts multiples of
+ * 16, ranges that stay): 3 x 3 convolution (stride and pad 1) C -> C_mid, requantize, relu if
+ * relu_first; 1 x 1 convolution C_mid -> C_out and the sum with `residual` as
+ * mxq_quantized_fc_sum_prepared with requant and sum_relu computes it, into `out`; and, unless
+ * C_next is 0, the 1 x 1 convolution C_out -> C_next that reads that sum, requantize, relu if
+ * relu_third, into `next`.  All three layers' int8 results are those of the launches one by one;
+ * the two that only this launch reads are not stored.
+ * mxq_quantized_block_fits: whether a block of this shape can run that way and is faster for it.
+ * mxq_pack_block_weights: the layers' NHWC weights [C_mid,3,3,C], [C_out,C_mid], [C_next,C_out]
+ * into the mxq_quantized_block_weights() bytes that the launch reads (16-byte aligned).
+ * mxq_prepare_block: from what mxq_prepare_layer made of the layers (their scales; the launch
+ * takes their bias from there), the residual's range and the calibrated ranges of the second
+ * layer and of the sum, the mxq_quantized_block_forms() bytes that the launch reads (16-byte
+ * aligned). */
+int mxq_quantized_block_fits(int N, int H, int W, int C, int C_mid, int C_out, int C_next);
+size_t mxq_quantized_block_weights(int C, int C_mid, int C_out, int C_next);
+int mxq_pack_block_weights(void* stream, const int8_t* first, const int8_t* second,
+                           const int8_t* third, int C, int C_mid, int C_out, int C_next,
+                           int8_t* out);
+size_t mxq_quantized_block_forms(void);
+int mxq_prepare_block(void* stream, const void* prepared_first, const void* prepared_second,
+                      const void* prepared_third, const float* min_residual,
+                      const float* max_residual, float min_calib, float max_calib,
+                      float sum_min_calib, float sum_max_calib, void* forms);
+int mxq_quantized_block(void* stream, const int8_t* data, const int8_t* weights,
+                        const void* forms, const void* prepared_first,
+                        const void* prepared_second, const void* prepared_third, int N, int H,
+                        int W, int C, int C_mid, int C_out, int C_next, const int8_t* residual,
+                        int8_t* out, int8_t* next, int relu_first, int relu_third);
+
 /* ---- calibration -----------------------------------------------------------
  * What the calibration collectors take of a float tensor
  * (python/mxnet/contrib/quantization.py:269-361, numpy on the host in the reference).

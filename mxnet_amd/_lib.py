@@ -87,6 +87,12 @@ SIGNATURES = {
     "mxq_quantize_to_nhwc": (_i, [_p] * 5 + [_i] * 8 + [_f, _f]),
     "mxq_quantized_pooling_nhwc": (_i, [_p, _p] + [_i] * 14 + [_p]),
     "mxq_pack_weight": (_i, [_p, _p, _p] + [_i] * 7),
+    "mxq_quantized_block_fits": (_i, [_i] * 7),
+    "mxq_quantized_block_weights": (_sz, [_i] * 4),
+    "mxq_pack_block_weights": (_i, [_p] * 4 + [_i] * 4 + [_p]),
+    "mxq_quantized_block_forms": (_sz, []),
+    "mxq_prepare_block": (_i, [_p] * 6 + [_f] * 4 + [_p]),
+    "mxq_quantized_block": (_i, [_p] * 7 + [_i] * 7 + [_p] * 3 + [_i, _i]),
     "mxq_nhwc_pad_to_nchw_i8": (_i, [_p, _p, _p] + [_i] * 5),
     "mxq_minmax_f32_workspace": (_sz, [_sz]),
     "mxq_minmax_f32": (_i, [_p, _p, _sz, _p, _p, _p, _sz]),

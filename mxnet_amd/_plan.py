@@ -7,6 +7,8 @@ keeps the graph's results and drops that traffic:
   * convolution -> requantize (-> relu), fully connected -> requantize (-> relu, -> dequantize)
     and convolution -> requantize -> sum (-> requantize) (-> relu) become one launch each (the
     fused epilogues of include/mxq.h, bit-identical to the operators one after the other);
+  * the tail of a residual block (3 x 3 convolution, 1 x 1 convolution, sum, the next block's first
+    1 x 1 convolution) becomes one launch where its ranges stay (fuse_blocks);
   * activations between convolutions and pooling stay NHWC with the channels padded to a multiple
     of 16; weights are laid out once, when the plan is made;
   * every range that a calibrated operator hands on is a constant of the plan;
@@ -28,7 +30,7 @@ _FLAG_OF = {torch.float32: 0, torch.float64: 1, torch.float16: 2, torch.uint8: 3
 _SIZE_OF = {0: 4, 1: 8, 2: 2, 3: 1, 4: 4, 5: 1, 6: 8, 7: 1, 12: 2}
 _FLOAT32, _INT32, _INT8 = 0, 4, 5
 (_NODE, _CONV, _FC, _FC_F32, _FC_SUM, _FC_SUM_RQ, _QUANT_NHWC, _TO_NHWC, _FROM_NHWC, _POOL, _RELU,
- _ADD, _REQUANTIZE) = range(13)
+ _ADD, _REQUANTIZE, _BLOCK) = range(14)
 _NULL, _ARENA, _HELD, _FEED, _OUTPUT = range(5)
 
 
@@ -679,6 +681,7 @@ class _Builder:
                 raise _Unsupported("a head that is an input, or the same as another head")
             v.at.place = (_OUTPUT, len(outputs), 0)
             outputs.append((v.flag, v.shape))
+        self.fuse_blocks()
         # offsets: first fit over the buffers alive at the same steps
         taken, size = [], 0
         for b in sorted((b for b in self.buffers if b.place is None and b.first is not None),
@@ -710,6 +713,14 @@ class _Builder:
         steps = []
         for kind, ints, floats, refs, node, blobs in self.steps:
             places = [place(r) for r in refs]
+            if kind == _BLOCK:
+                layers, blobs = blobs, None
+                layers = [(columns, calib, [place(r) for r in refs])
+                          for columns, calib, refs in layers]
+                places[1] = self.block_weights(ints, layers)
+                places[3:6] = [self.prepared(*layer) if layer[2] else (_NULL, 0, 0)
+                               for layer in layers]
+                places[2] = self.block_forms(floats, layers, places[3:6])
             if kind in (_CONV, _FC, _FC_F32, _FC_SUM, _FC_SUM_RQ):
                 places.append(self.prepared(ints[4 if kind == _CONV else 1], floats, places))
             step = (kind, tuple(int(v) for v in ints), tuple(float(v) for v in floats),
@@ -718,13 +729,106 @@ class _Builder:
         plan = _frontend.plan(size, self.held, steps, [(f, tuple(s)) for f, s in outputs])
         return plan, tuple(self.params.values()), self.made
 
-    def prepared(self, columns, calib, places):
-        """What mxq_prepare_layer makes of a layer's bias and six ranges, if they stay."""
-        given = places[2:9]
-        if any(base not in (_HELD, _NULL) for base, _, _ in given):
-            return (_NULL, 0, 0)
-        key, names = ["prepared", int(columns), _bits(calib[0]), _bits(calib[1])], []
-        for base, i, offset in given:
+    def fuse_blocks(self):
+        """The tail of a residual block as one step: a 3 x 3 convolution that only the sum's 1 x 1
+        convolution reads, that convolution with the sum, and a 1 x 1 convolution that reads the
+        sum."""
+        users = {}  # id of a buffer -> the steps that read or write it
+        for at, step in enumerate(self.steps):
+            for r in step[3]:
+                b = r.buffer if isinstance(r, _Offset) else r
+                if isinstance(b, _Buffer):
+                    users.setdefault(id(b), []).append(at)
+        gone = set()
+        for at, (kind, ints, floats, refs, _, _) in enumerate(self.steps):
+            if kind != _FC_SUM_RQ or not ints[3] or not self.stays(refs):
+                continue
+            mid = refs[0]
+            first = users[id(mid)][0] if isinstance(mid, _Buffer) else at
+            if len(users.get(id(mid), ())) != 2 or first >= at or mid.place is not None:
+                continue
+            kind, geo, calib, conv, _, _ = self.steps[first]
+            n, h, w, c, c_mid = geo[:5]
+            if (kind != _CONV or conv[10] is not mid or geo[5:13] != (3, 3, 1, 1, 1, 1, 1, 1) or
+                    not self.stays(conv) or c_mid != ints[2] or n * h * w != ints[0]):
+                continue
+            layers = [(c_mid, calib, conv), (ints[1], floats, refs)]
+            shape, relu, out, third = (n, h, w, c, c_mid, ints[1]), 0, None, None
+            for j in users[id(refs[10])]:
+                kind, geo, calib, after, _, _ = self.steps[j]
+                if (j > at and kind == _CONV and j not in gone and after[0] is refs[10] and
+                        geo[:4] == (n, h, w, ints[1]) and self.stays(after) and
+                        geo[5:13] == (1, 1, 1, 1, 0, 0, 1, 1) and
+                        _lib.lib.mxq_quantized_block_fits(*shape, geo[4])):
+                    layers.append((geo[4], calib, after))
+                    relu, out, third = geo[13], after[10], j
+                    break
+            if third is None:
+                if not _lib.lib.mxq_quantized_block_fits(*shape, 0):
+                    continue
+                layers.append((0, (), ()))
+            gone.update((first, third))
+            self.steps[at] = (_BLOCK, shape + (layers[2][0], self.steps[first][1][13], relu),
+                              floats, [conv[0], None, None, None, None, None, refs[12],
+                                       refs[10], out], None, layers)
+        if gone:
+            self.steps = [s for at, s in enumerate(self.steps) if at not in gone]
+            for b in self.buffers:
+                b.first = b.last = None
+            for at, step in enumerate(self.steps):
+                for r in step[3]:
+                    b = r.buffer if isinstance(r, _Offset) else r
+                    if isinstance(b, _Buffer):
+                        b.first = at if b.first is None else b.first
+                        b.last = at
+
+    @staticmethod
+    def stays(refs):
+        """Whether a layer's bias and six ranges are constants of the plan."""
+        return all(r is None or (isinstance(r, _Place) and r.place[0] == _HELD)
+                   for r in refs[2:9] + refs[13:15])
+
+    def block_weights(self, ints, layers):
+        """[where the weights of a _BLOCK step lie]"""
+        places = [refs[1] if refs else None for _, _, refs in layers]
+        names = sum((self.origin[p[1]][1] for p in places if p), ())
+
+        def make():
+            out = torch.empty(int(_lib.lib.mxq_quantized_block_weights(*ints[3:7])),
+                              dtype=torch.int8, device=self.device)
+            _lib.check(_lib.lib.mxq_pack_block_weights(
+                self.stream, *[self.held[p[1]].data_ptr() if p else None for p in places],
+                *ints[3:7], out.data_ptr()))
+            return out
+
+        key = ("block",) + tuple(self.origin[p[1]][0] if p else None for p in places)
+        return self.laid(key, names, make).place
+
+    def block_forms(self, floats, layers, prepared):
+        """Where what mxq_prepare_block makes of a _BLOCK step's scales and sum lies."""
+        residual = layers[1][2][13:15]
+        key, names = self.constants_key(residual)
+        for _, calib, refs in layers:  # whatever the bias is, its scale is one of the ranges
+            more, read = self.constants_key(refs[3:9])
+            key += [len(more), refs[2:3] != [(_NULL, 0, 0)]] + more + [_bits(f) for f in calib]
+            names += read
+
+        def make():
+            out = torch.empty(int(_lib.lib.mxq_quantized_block_forms()), dtype=torch.int8,
+                              device=self.device)
+            _lib.check(_lib.lib.mxq_prepare_block(
+                self.stream, *[None if base == _NULL else self.held[i].data_ptr()
+                               for base, i, _ in prepared],
+                *[self.held[i].data_ptr() + offset for _, i, offset in residual],
+                *[float(f) for f in floats], out.data_ptr()))
+            return out
+
+        return self.laid(("forms",) + tuple(key), tuple(names), make).place
+
+    def constants_key(self, places):
+        """Operands that stay as part of a layout's key, and the parameters among them."""
+        key, names = [], []
+        for base, i, offset in places:
             if base == _NULL:
                 key.append(None)
             elif i == self.table_index:
@@ -733,6 +837,15 @@ class _Builder:
                 what, read = self.origin[i]
                 key += [what, offset]
                 names += read
+        return key, names
+
+    def prepared(self, columns, calib, places):
+        """What mxq_prepare_layer makes of a layer's bias and six ranges, if they stay."""
+        given = places[2:9]
+        if any(base not in (_HELD, _NULL) for base, _, _ in given):
+            return (_NULL, 0, 0)
+        key, names = self.constants_key(given)
+        key = ["prepared", int(columns), _bits(calib[0]), _bits(calib[1])] + key
 
         def make():
             at = [None if base == _NULL else self.held[i].data_ptr() + offset

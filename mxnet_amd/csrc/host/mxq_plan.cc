@@ -124,6 +124,11 @@ bool Plan::run(void* stream, const std::vector<at::Tensor>& feeds,
                                         v(6), p(2), i(1), v(7), v(7) + 1,
                                         static_cast<size_t>(n[0]), i(2), f[0], f[1]);
         break;
+      case Kind::kBlock:  // refs: data, weights, what mxq_prepare_block made, what
+                          // mxq_prepare_layer made of three layers, residual, sum, third output
+        rc = mxq_quantized_block(stream, q(0), q(1), p(2), p(3), p(4), p(5), i(0), i(1), i(2),
+                                 i(3), i(4), i(5), i(6), q(6), q(7), q(8), i(7), i(8));
+        break;
       case Kind::kRequantize:
         rc = mxq_requantize(stream, static_cast<int32_t*>(p(0)), v(2), v(3), q(1), v(4), v(4) + 1,
                             static_cast<size_t>(n[0]), 1, f[0], f[1], nullptr, 0);

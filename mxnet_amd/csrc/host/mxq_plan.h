@@ -42,6 +42,7 @@ enum class Kind : int {
   kRelu,         // int8 relu
   kAdd,          // int8 sum, int32 or calibrated int8
   kRequantize,   // calibrated
+  kBlock,        // 3 x 3 convolution -> 1 x 1 -> sum (-> 1 x 1), each requantized
 };
 
 struct Step {

@@ -1,0 +1,836 @@
+// The tail of a residual block as one launch: 3 x 3 convolution, 1 x 1 convolution, the sum with
+// the shortcut, and the next block's first 1 x 1 convolution, each with its requantize and relu.
+//
+// Layer by layer every one of these is a launch of 10 to 30 us around 2 to 6 us of matrix work:
+// its operands come through memory, its K loop waits for a stage at every barrier, its epilogue
+// leaves the matrix cores idle.  The 1 x 1 layers need nothing but the pixels of the layer in
+// front of them, so a work-group that owns whole pixels (all channels of TM consecutive ones)
+// keeps them in LDS from the 3 x 3 layer's input to the last layer's output:
+//
+//   patch   the input rows its pixels touch, halo included          [rows][W + 2][C]
+//           then the 3 x 3 layer's int8 result                      [TM][Cm]
+//           then the next block's first layer                       [TM][Ca]
+//   wide    the shortcut, which the sum overwrites in place         [TM][Co]
+//
+// What moves through memory is the patch, the shortcut, the block's output (both contiguous:
+// whole pixels), the last layer's output, and the weights.  Those come straight into registers:
+// they were laid out beforehand in the order a wave consumes them (mxq_pack_block_weights: 1 KB
+// per 32 x 32 MFMA operand), so a load is one contiguous KB, no LDS ring and no barrier stands
+// between a wave and its next operand, and five barriers per tile are all that is left.  A CU
+// takes in 64 bytes of weights per clock and multiplies them with the 64 pixels in the same time,
+// which is why TM is no smaller.
+//
+// Rows in LDS are an odd number of 16-byte chunks apart: 16 consecutive rows' fragments hit
+// distinct bank groups without a permutation, for any channel count.
+//
+// What bounds it: a tile's own chain.  Of the 42000 clocks of a tile of 14 x 14 x 256 -> 1024 -> 256
+// (one per CU) 5000 go by until the patch is there, 15000 in the 3 x 3 layer (9200 of matrix work),
+// 14000 in the sum's layer (8000 of vector and 4000 of matrix work that overlap little: two waves of
+// a SIMD run in step from the barrier on), 8000 behind it.  Measured at batch 64 against the three
+// launches: 22.0 us against 38.3 there, 30.3 / 45.3 for 28 x 28 x 128, 44.4 / 59.4 for 56 x 56 x 64.
+// A quantized ResNet-50 at batch 64 takes 716 us with it, 867 without.  Measured and not kept: four
+// row tiles' products made while the tile before is finished (level, 100 registers more), the second
+// layer's operand held in registers (level), wave priorities (level).
+#include <hip/hip_runtime.h>
+
+#include <cstdint>
+
+#include "../../include/mxq.h"
+#include "mxq_common.h"
+#include "mxq_gemm.h"
+
+namespace mxq {
+namespace {
+
+// a lambda that is called rather than inlined would keep what it captures in scratch memory
+#define MXQ_INLINE __attribute__((always_inline))
+
+constexpr int kBlockLds = 160 * 1024;
+
+// Short forms.  The definition of a requantize is four float operations with a rounding each, then
+// a clamp, a truncation and a relu: 6.5 vector instructions per output with the packing, 7.75
+// without the relu, and 6 more for the sum, together several times what the matrix cores take for
+// a 1 x 1 layer.  Each of them is a function with few steps of an integer: a requantize has 127
+// thresholds (its negative half mirrors the positive one), the sum is defined on 255 x 256 pairs.
+// So whether one multiplication and one addition give the same int8 everywhere is found out by
+// looking at every threshold from both sides, or at every pair; the factor may move by some last
+// places until they do (it holds for nearly all ranges, the others keep the definition).
+//   with the relu   cvt_pk_u8(fma(acc, 2t, c)) / 2 with c = 0.5, or some 2^-18 beside it: twice the
+//                   level, rounded, in [0, 255]; the halving drops what the rounding of twice the
+//                   level and a half is off by
+//   without         fma(acc, t, 2^23 + 128) clamped to 2^23 + [1, 255]: its rounding is the
+//                   level's, and the low byte is the level + 128
+//   the sum         as the first, over fma(level, 2ta, fma(residual, 2tb, c)).  Both operands are
+//                   small integers in 16 bits, which read as half floats are that many times
+//                   2^-24: v_fma_mix_f32 takes them as they are, without a conversion
+// 3.25 instructions per output of a layer with a relu, 7 instead of 13.75 for the sum.
+constexpr float kRound = 8388608.0f + 128.0f;
+__device__ __forceinline__ uint32_t halve4(uint32_t w) { return __builtin_amdgcn_lerp(w, 0u, 0u); }
+__device__ __forceinline__ uint32_t short_relu4(int a0, int a1, int a2, int a3, float t, float c) {
+  uint32_t w = 0;
+  w = __builtin_amdgcn_cvt_pk_u8_f32(__builtin_fmaf(static_cast<float>(a0), t, c), 0, w);
+  w = __builtin_amdgcn_cvt_pk_u8_f32(__builtin_fmaf(static_cast<float>(a1), t, c), 1, w);
+  w = __builtin_amdgcn_cvt_pk_u8_f32(__builtin_fmaf(static_cast<float>(a2), t, c), 2, w);
+  w = __builtin_amdgcn_cvt_pk_u8_f32(__builtin_fmaf(static_cast<float>(a3), t, c), 3, w);
+  return halve4(w);
+}
+// the level + 128, in the low 16 bits
+__device__ __forceinline__ uint32_t short_level(int a, float t) {
+  return __float_as_uint(
+      __builtin_amdgcn_fmed3f(__builtin_fmaf(static_cast<float>(a), t, kRound), kRound - 127.0f,
+                              kRound + 127.0f));
+}
+struct SumForm {
+  float ta, tb, c;  // for levels and residuals + 128, times 2^-24
+};
+__host__ __device__ inline SumForm sum_form(float ta, float tb) {  // ta, tb doubled
+  return SumForm{ta * 16777216.0f, tb * 16777216.0f, 0.5f - 128.0f * (ta + tb)};
+}
+__device__ __forceinline__ float half_of(uint32_t w, int k) {
+  typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+  return static_cast<float>(__builtin_bit_cast(h2, w)[k]);
+}
+__device__ __forceinline__ uint32_t short_sum4(uint32_t a0, uint32_t a1, uint32_t a2, uint32_t a3,
+                                               uint32_t y, const SumForm& f) {
+  const uint32_t a[4] = {a0, a1, a2, a3};
+  y ^= 0x80808080u;
+  const uint32_t b[2] = {__builtin_amdgcn_perm(0u, y, 0x0c010c00u),
+                         __builtin_amdgcn_perm(0u, y, 0x0c030c02u)};
+  uint32_t w = 0;
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+    w = __builtin_amdgcn_cvt_pk_u8_f32(
+        __builtin_fmaf(half_of(a[k], 0), f.ta, __builtin_fmaf(half_of(b[k >> 1], k & 1), f.tb, f.c)),
+        k, w);
+  return halve4(w);
+}
+
+// What a launch needs to know of its three layers' scales and of the sum, prepared once
+// (mxq_prepare_block).
+struct BlockForms {
+  EpiScalars s[3];
+  RequantRule rule;
+  float t[3], c[3];  // factor and constant of the layers' short forms
+  SumForm sum;
+  int has;       // bit i: layer i has one; bit 3: the sum has
+  int pair;      // which of the tried ones that is
+};
+constexpr size_t kBlockForms = 192;
+static_assert(sizeof(BlockForms) <= kBlockForms, "room for the forms");
+
+struct BlockArgs {
+  const int8_t* data;     // [N][H][W][C]
+  const int8_t* weights;  // fragments of the three layers, one behind the other
+  const BlockForms* forms;
+  const char* prepared[3];  // the layers' int32 bias, kPreparedBias bytes in
+  const int8_t* res;      // [M][Co]
+  int8_t* out;            // [M][Co]
+  int8_t* next;           // [M][Ca]
+  int N, H, W, C, Cm, Co, Ca, M;
+  int kb, ksb;            // MFMA steps of the 3 x 3 layer, and of one tap of it
+  int ka;                 // ... of the last layer
+  int at_c, at_a, kb_all; // where the second and third layer's fragments begin (KB), and all end
+  int off_patch, off_bias, off_table;  // bytes in LDS
+  int parts, row_pitch;   // load instructions and bytes per row of the patch
+  uint32_t magic_plane, magic_w, magic_pixel, magic_image, magic_res, magic_wide,
+      magic_next, magic_tap;
+  int relu_b, relu_a, stream, tiles;
+};
+
+__host__ __device__ constexpr int odd(int chunks) { return chunks | 1; }
+// ... of rows that are written in whole column tiles of 32 channels
+__host__ __device__ constexpr int odd_tiles(int chunks) { return ((chunks + 1) & ~1) | 1; }
+
+// floor(n / d) for n * d < 2^30, magic = 2^31 / d + 1: (2n + 1) / 2d is never an integer, and no
+// case (d = 1) needs a branch, behind which the compiler would load the next argument
+__device__ __forceinline__ int quotient(int n, uint32_t magic) {
+  return static_cast<int>(__umulhi(2u * static_cast<uint32_t>(n) + 1u, magic));
+}
+// floor(n / d) for any 0 <= n < 2^31: the product above is at most one too large there
+__device__ __forceinline__ int quotient_any(int n, int d, uint32_t magic) {
+  const int q = quotient(n, magic);
+  return q - (static_cast<uint32_t>(q) * static_cast<uint32_t>(d) > static_cast<uint32_t>(n));
+}
+uint32_t magic_of(int d) { return static_cast<uint32_t>((1ULL << 31) / static_cast<unsigned>(d) + 1); }
+
+// WM x WN waves, each RT row tiles of 32 pixels by one column tile of 32 channels at a time.
+// GB, GC: MFMA steps whose weights a wave requests together (the 3 x 3 layer's, and the whole
+// reduction of the second layer).
+template <int WM, int WN, int RT, int GB, int GC>
+__global__ __launch_bounds__(64 * WM * WN, GC < 8 ? 4 : 2) void block_kernel(BlockArgs p) {
+  constexpr int NW = WM * WN, TM = 32 * WM * RT, GA = 8;
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  // every argument at once: left alone the compiler loads each of them where it is first used, a
+  // round trip at a time, 3000 clocks before the first pixels are requested
+  asm volatile("" ::"s"(p.data), "s"(p.weights), "s"(p.forms), "s"(p.prepared[0]),
+               "s"(p.prepared[1]), "s"(p.prepared[2]), "s"(p.res), "s"(p.N), "s"(p.H), "s"(p.W),
+               "s"(p.C), "s"(p.Cm), "s"(p.Co), "s"(p.Ca), "s"(p.M), "s"(p.kb), "s"(p.ksb),
+               "s"(p.at_c), "s"(p.kb_all), "s"(p.off_patch), "s"(p.off_bias), "s"(p.off_table),
+               "s"(p.magic_plane), "s"(p.magic_w), "s"(p.magic_pixel), "s"(p.parts), "s"(p.row_pitch),
+               "s"(p.magic_image), "s"(p.magic_res), "s"(p.magic_tap), "s"(p.tiles));
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave / WN, wn = wave % WN;
+  // an XCD takes a run of neighbouring tiles: they share halo rows in its L2
+  const int per = (p.tiles + 7) >> 3;
+  const int tile = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  if (tile >= p.tiles) return;
+  const int m0 = tile * TM;
+  const int CH = p.C >> 4, PP = odd(CH), H2 = p.H + 2;
+  const int row_pitch = p.row_pitch;  // bytes of a patch row
+  const int PM = odd_tiles(p.Cm >> 4), CO = p.Co >> 4, PO = odd_tiles(CO);
+  const int CA = p.Ca >> 4, PA = odd_tiles(CA);
+  const int plane = p.H * p.W;
+  const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(smem));
+  // 64 pieces of 16 bytes to `to` and on in LDS
+  auto fetch = [&](int to, uint32_t from, v4i rsrc) MXQ_INLINE {
+    dma_buffer(__builtin_amdgcn_readfirstlane(lds0 + to), from, rsrc);
+  };
+
+  const auto weights = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(p.weights), 0,
+                                                         p.kb_all * 1024, 0x00020000);
+  // fragment number k; zeros, and nothing is fetched, from kNone on
+  constexpr int kNone = 0x100000;
+  auto fragment = [&](int k) MXQ_INLINE {
+    return __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(
+                                       weights, k * 1024 + lane * 16, 0, 0));
+  };
+  const int tiles_b = (p.Cm + 31) >> 5, tiles_c = (p.Co + 31) >> 5, tiles_a = (p.Ca + 31) >> 5;
+  const bool has_b = wn < tiles_b;
+  v4i wb[GB];
+  const int first_b = (has_b ? wn : 0) * p.kb;
+#pragma unroll
+  for (int i = 0; i < GB; ++i) wb[i] = fragment(first_b + i);
+
+  // the patch: virtual rows n * (H + 2) + ih + 1, so that the zero rows above and below an image
+  // are rows like any other
+  const int mb = (m0 + TM - 1 < p.M) ? m0 + TM - 1 : p.M - 1;
+  const int na = quotient_any(m0, plane, p.magic_plane);
+  const int oha = quotient(m0 - na * plane, p.magic_w);
+  const int nb = quotient_any(mb, plane, p.magic_plane);
+  const int ohb = quotient(mb - nb * plane, p.magic_w);
+  const int vr0 = na * H2 + oha, rows = nb * H2 + ohb + 2 - vr0 + 1;
+  {
+    const v4i rsrc = make_rsrc(p.data, static_cast<uint32_t>(p.N) * plane * p.C);
+    // A row of the patch is a whole number of load instructions: a lane's place in the row stays as
+    // the wave goes down the rows, and a row is one scalar offset.  (A lane that finds its pixel
+    // anew for every piece, by divisions or by carries, costs 300 clocks per instruction.)
+    int j = lane, iw = -1;
+    const int row_bytes = p.W * p.C;
+    int carry = quotient(j, p.magic_pixel);
+    j -= carry * PP;
+    iw += carry;
+    const int step = quotient(64, p.magic_pixel), rest = 64 - step * PP;
+    for (int part = 0; part < p.parts; ++part) {
+      const bool ok = j < CH && static_cast<unsigned>(iw) < static_cast<unsigned>(p.W);
+      const uint32_t place = ok ? static_cast<uint32_t>(iw * p.C + 16 * j) : kOutOfRange;
+      for (int r = wave; r < rows; r += NW) {
+        const int v = vr0 + r, n = quotient(v, p.magic_image), ih = v - n * H2 - 1;
+        const bool inside = n < p.N && static_cast<unsigned>(ih) < static_cast<unsigned>(p.H);
+        fetch(p.off_patch + r * row_pitch + part * 1024,
+              inside ? place + static_cast<uint32_t>((n * p.H + ih) * row_bytes) : kOutOfRange,
+              rsrc);
+      }
+      j += rest;
+      iw += step;
+      if (j >= PP) {
+        j -= PP;
+        ++iw;
+      }
+    }
+  }
+  const int* const sbias = reinterpret_cast<const int*>(smem + p.off_bias);
+  const int bias_c = (p.Cm + 255) & ~255, bias_a = bias_c + ((p.Co + 255) & ~255);
+#pragma unroll
+  for (int layer = 0; layer < 3; ++layer) {
+    const int columns = layer == 0 ? p.Cm : layer == 1 ? p.Co : p.Ca;
+    const int at = layer == 0 ? 0 : layer == 1 ? bias_c : bias_a;
+    if (columns != 0) {  // whole load instructions, zeros behind the last column
+      const v4i rsrc = make_rsrc(p.prepared[layer] + kPreparedBias, 4u * columns);
+      for (int it = wave; it * 256 < columns; it += NW)
+        fetch(p.off_bias + at * 4 + it * 1024, it * 1024 + lane * 16, rsrc);
+    }
+  }
+  const EpiScalars s_b = p.forms->s[0], s_c = p.forms->s[1], s_a = p.forms->s[2];
+  const RequantRule rule = p.forms->rule;
+  const float t_b = p.forms->t[0], t_c = p.forms->t[1], t_a = p.forms->t[2];
+  const float c_b = p.forms->c[0], c_a = p.forms->c[2];
+  const SumForm form = p.forms->sum;
+  const int has = p.forms->has;
+  // where step k of the 3 x 3 layer reads, from the pixel's place under the first tap; steps behind
+  // the last one have zero weights
+  for (int k = tid; k < p.kb + 2 * GB; k += 64 * NW) {
+    const int last = 9 * p.ksb - 1, at = k < last ? k : last;
+    const int tap = quotient(at, p.magic_tap), kh = tap / 3;
+    reinterpret_cast<int*>(smem + p.off_table)[k] =
+        kh * row_pitch + (tap - 3 * kh) * PP * 16 + (at - tap * p.ksb) * 32;
+  }
+  // The shortcut, a share of it at a time while the 3 x 3 layer runs.
+  const v4i res_rsrc = make_rsrc(p.res, static_cast<uint32_t>(p.M) * p.Co);
+  const int res_slots = TM * PO;
+  int res_at = wave;
+  auto fetch_shortcut = [&]() MXQ_INLINE {
+    if (res_at * 64 < res_slots) {
+      const int q = res_at * 64 + lane;
+      const int row = quotient(q, p.magic_res), j = q - row * PO;
+      const bool ok = j < CO && row < TM && m0 + row < p.M;
+      fetch(res_at * 1024,
+                 ok ? static_cast<uint32_t>((m0 + row) * p.Co + 16 * j) : kOutOfRange, res_rsrc);
+      res_at += NW;
+    }
+  };
+
+  // this lane's rows: where they begin in each of the three
+  const int frow = lane & 31, fgrp = lane >> 5;
+  const int row0 = wm * RT * 32 + frow;
+  int in_patch[RT];
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) {
+    int m = m0 + row0 + 32 * rt;
+    m = m < p.M ? m : p.M - 1;  // rows past the end repeat the last pixel; never stored
+    const int n = quotient_any(m, plane, p.magic_plane), rem = m - n * plane;
+    const int oh = quotient(rem, p.magic_w), ow = rem - oh * p.W;
+    in_patch[rt] = p.off_patch + (n * H2 + oh - vr0) * row_pitch + ow * PP * 16 + fgrp * 16;
+  }
+  v16i acc[RT];
+  auto read_bias = [&](const int* bias, v4i (&b)[4]) MXQ_INLINE {
+#pragma unroll
+    for (int vq = 0; vq < 4; ++vq)
+      b[vq] = *reinterpret_cast<const v4i*>(bias + 8 * vq + 4 * fgrp);
+  };
+  auto start = [&](v16i (&acc)[RT], const v4i (&b)[4]) MXQ_INLINE {
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[rt][i] = b[i / 4][i % 4];
+  };
+  // One group of G steps.  The pixels of a step are read kAhead steps before they are multiplied,
+  // and a step's weights make room for those of the same step of the next group (fragments from
+  // `from` on) as soon as they are used: G KB per wave are always on their way.  Requested all at
+  // once, at the start of a group, the CU's 64 KB arrive in 1024 clocks and a latency, which is 1700
+  // of the 1024 that eight steps should take.  The order is pinned: left alone the compiler sinks
+  // the requests to the end of the group and reads each step's pixels right in front of its MFMAs.
+  constexpr int kRing = NW * RT >= 16 && GC == 8 ? 4 : 2, kAhead = kRing - 1;
+  v4i px[kRing][RT];
+  auto read_pixels = [&](v4i (&x)[RT], const int (&base)[RT], int offset) MXQ_INLINE {
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+      x[rt] = *reinterpret_cast<const v4i*>(smem + base[rt] + offset);
+  };
+  // offset_of(i): where step i of the group reads, for i up to G + kAhead - 1
+  auto first_pixels = [&](const int (&base)[RT], auto offset_of) MXQ_INLINE {
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) read_pixels(px[i], base, offset_of(i));
+  };
+  auto multiply = [&](v16i (&acc)[RT], v4i w, const v4i (&x)[RT]) MXQ_INLINE {
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+      acc[rt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(w, x[rt], acc[rt], 0, 0, 0);
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) asm volatile("" : "+v"(acc[rt]));
+  };
+  auto run_group = [&](auto& w, int from, const int (&base)[RT], auto offset_of) MXQ_INLINE {
+    constexpr int G = sizeof(w) / sizeof(v4i);
+    static_assert(G % kRing == 0, "the sets of pixels take turns");
+#pragma unroll
+    for (int i = 0; i < G; ++i) {
+      read_pixels(px[(i + kAhead) % kRing], base, offset_of(i + kAhead));
+      multiply(acc, w[i], px[i % kRing]);
+      w[i] = fragment(from + i);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  auto publish = [&]() MXQ_INLINE {  // what this wave wrote to LDS or had written there, to all of them
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  publish();
+
+  // ---- 3 x 3 ------------------------------------------------------------------------------
+  const int groups = p.kb / GB;
+  if (has_b) {
+    v4i bias[4];
+    read_bias(sbias + 32 * wn, bias);
+    start(acc, bias);
+    const int* const table = reinterpret_cast<const int*>(smem + p.off_table);
+    auto read_offsets = [&](int g, int (&o)[GB]) MXQ_INLINE {
+#pragma unroll
+      for (int i = 0; i < GB; ++i) o[i] = __builtin_amdgcn_readfirstlane(table[g * GB + i]);
+    };
+    int now[GB], later[GB];
+    read_offsets(0, now);
+    read_offsets(1, later);
+    auto offset_of = [&](int i) MXQ_INLINE { return i < GB ? now[i] : later[i - GB]; };
+    first_pixels(in_patch, offset_of);
+    for (int g = 0; g < groups; ++g) {
+      fetch_shortcut();
+      run_group(wb, g + 1 < groups ? first_b + (g + 1) * GB : kNone, in_patch, offset_of);
+#pragma unroll
+      for (int i = 0; i < GB; ++i) now[i] = later[i];
+      read_offsets(g + 2, later);
+    }
+  }
+  while (res_at * 64 < res_slots) fetch_shortcut();
+  v4i wc[GC];
+#pragma unroll
+  for (int i = 0; i < GC; ++i) wc[i] = fragment(p.at_c + wn * GC + i);
+  // column tile t of a layer's int8 result into rows of `pitch` chunks at the patch's place
+  auto finish = [&](int t, int pitch, auto pack) MXQ_INLINE {
+#pragma unroll
+    for (int vq = 0; vq < 4; ++vq)
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt)
+        *reinterpret_cast<uint32_t*>(smem + p.off_patch + (row0 + 32 * rt) * pitch * 16 + 32 * t +
+                                     8 * vq + 4 * fgrp) =
+            pack(acc[rt][4 * vq], acc[rt][4 * vq + 1], acc[rt][4 * vq + 2], acc[rt][4 * vq + 3]);
+  };
+  auto finish_layer = [&](const EpiScalars s, const float factor, const float constant, bool has,
+                          int relu, int t, int pitch) MXQ_INLINE {
+    if (relu && has)
+      finish(t, pitch,
+             [&](int a, int b, int c, int d) { return short_relu4(a, b, c, d, factor, constant); });
+    else if (relu)
+      finish(t, pitch,
+             [&](int a, int b, int c, int d) { return epi_requant_pack<true>(a, b, c, d, s); });
+    else
+      finish(t, pitch,
+             [&](int a, int b, int c, int d) { return epi_requant_pack<false>(a, b, c, d, s); });
+  };
+  __builtin_amdgcn_s_barrier();  // every wave is through with the patch
+  asm volatile("" ::: "memory");
+  if (has_b) finish_layer(s_b, t_b, c_b, (has & 1) != 0, p.relu_b, wn, PM);
+  publish();
+
+  // ---- 1 x 1 and the sum ------------------------------------------------------------------
+  // where this lane's rows are read as an operand, and where its outputs of a column tile lie
+  int in_mid[RT], in_wide[RT], at_wide[RT];
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) {
+    in_mid[rt] = p.off_patch + (row0 + 32 * rt) * PM * 16 + fgrp * 16;
+    in_wide[rt] = (row0 + 32 * rt) * PO * 16 + fgrp * 16;
+    at_wide[rt] = (row0 + 32 * rt) * PO * 16 + fgrp * 4;
+  }
+  auto widen = [&](auto how) MXQ_INLINE {
+    constexpr int F = decltype(how)::value;
+    for (int t = wn; t < tiles_c; t += WN) {
+      const int from = t + WN < tiles_c ? p.at_c + (t + WN) * GC : kNone;
+      v4i bias[4];
+      uint32_t shortcut[RT][4];
+      read_bias(sbias + bias_c + 32 * t, bias);
+      read_pixels(px[0], in_mid, 0);
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+        for (int vq = 0; vq < 4; ++vq)
+          shortcut[rt][vq] =
+              *reinterpret_cast<const uint32_t*>(smem + at_wide[rt] + 32 * t + 8 * vq);
+      start(acc, bias);
+#pragma unroll
+      for (int i = 0; i < GC; ++i) {
+        if (i + 1 < GC) read_pixels(px[(i + 1) & 1], in_mid, 32 * (i + 1));
+        multiply(acc, wc[i], px[i & 1]);
+        wc[i] = fragment(from + i);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int vq = 0; vq < 4; ++vq)
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+          const int a = acc[rt][4 * vq], b = acc[rt][4 * vq + 1], c = acc[rt][4 * vq + 2],
+                    d = acc[rt][4 * vq + 3];
+          const uint32_t y = shortcut[rt][vq];
+          uint32_t w;
+          if constexpr (F == 2) {
+            w = short_sum4(short_level(a, t_c), short_level(b, t_c), short_level(c, t_c),
+                           short_level(d, t_c), y, form);
+          } else {
+            const uint32_t x = epi_requant_pack<false>(a, b, c, d, s_c);
+            w = F == 1 ? sum_requant4<true>(x, y, rule) : sum_requant4_general<true>(x, y, rule);
+          }
+          *reinterpret_cast<uint32_t*>(smem + at_wide[rt] + 32 * t + 8 * vq) = w;
+        }
+    }
+  };
+  if ((has & 10) == 10)
+    widen(std::integral_constant<int, 2>());
+  else if (rule.fast)
+    widen(std::integral_constant<int, 1>());
+  else
+    widen(std::integral_constant<int, 0>());
+  v4i wa[GA];
+  if (p.Ca != 0) {
+#pragma unroll
+    for (int i = 0; i < GA; ++i) wa[i] = fragment(p.at_a + wn * p.ka + i);
+  }
+  publish();
+
+  // rows of `chunks` pieces, `pitch` apart in LDS, to consecutive memory
+  const int rows_left = p.M - m0 < TM ? p.M - m0 : TM;
+  auto leave = [&](int at, int chunks, int pitch, uint32_t magic, int8_t* out, auto stream) MXQ_INLINE {
+    for (int i = tid; i < rows_left * chunks; i += 64 * NW) {
+      const int row = quotient(i, magic);
+      epi_store16<decltype(stream)::value>(
+          *reinterpret_cast<const v4i*>(smem + at + (row * pitch + i - row * chunks) * 16),
+          out + static_cast<size_t>(m0) * chunks * 16 + static_cast<size_t>(i) * 16);
+    }
+  };
+  if (p.stream)
+    leave(0, CO, PO, p.magic_wide, p.out, std::true_type());
+  else
+    leave(0, CO, PO, p.magic_wide, p.out, std::false_type());
+  if (p.Ca == 0) return;
+
+  // ---- the next block's first 1 x 1 ---------------------------------------------------------
+  const int groups_a = p.ka / GA;
+  for (int t = wn; t < tiles_a; t += WN) {
+    v4i bias[4];
+    read_bias(sbias + bias_a + 32 * t, bias);
+    start(acc, bias);
+    first_pixels(in_wide, [](int i) { return 32 * i; });
+    for (int g = 0; g < groups_a; ++g)
+      run_group(wa,
+                g + 1 < groups_a ? p.at_a + t * p.ka + (g + 1) * GA
+                : t + WN < tiles_a ? p.at_a + (t + WN) * p.ka : kNone,
+                in_wide, [&](int i) { return (g * GA + i) * 32; });
+    finish_layer(s_a, t_a, c_a, (has & 4) != 0, p.relu_a, t, PA);
+  }
+  publish();
+  leave(p.off_patch, CA, PA, p.magic_next, p.next, std::false_type());
+}
+
+// [O][taps][C] rows -> fragments [ceil(O / 32)][steps][64 lanes][16 bytes]: lane l of step
+// tap * per_tap + s holds bytes 32 * s + 16 * (l / 32) ... + 15 of tap `tap` of row l % 32 of the
+// column tile, zeros where there are none.
+__global__ __launch_bounds__(256) void pack_fragments_kernel(const v4i* in, v4i* out, int O,
+                                                             int taps, int chunks, int per_tap,
+                                                             int steps, unsigned pieces) {
+  const unsigned i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= pieces) return;
+  const int lane = i & 63;
+  const unsigned f = i >> 6;
+  const int t = f / steps, k = f - t * steps;
+  const int tap = k / per_tap, c = 2 * (k - tap * per_tap) + (lane >> 5);
+  const int n = 32 * t + (lane & 31);
+  const bool ok = n < O && tap < taps && c < chunks;
+  out[i] = ok ? in[(static_cast<size_t>(n) * taps + tap) * chunks + c] : v4i{0, 0, 0, 0};
+}
+
+// The search for the forms, in three launches: nothing found yet; work-groups 0 ... 2 each try
+// every factor and constant for a layer (layers 0 and 2 with the relu, 1 without), one per thread,
+// and the others one pair of factors each for the sum; then what the sum's found.
+struct PrepareArgs {
+  const char* prepared[3];
+  const float* res_min;
+  const float* res_max;
+  float layer_range, sum_min, sum_max;
+  BlockForms* out;
+};
+constexpr int kFactors = 64, kConstants = 16, kPairs = 49;
+__device__ __forceinline__ float moved(float v, int c) {  // 0, +1, -1, +2, ... last places away
+  return __int_as_float(__float_as_int(v) + ((c & 1) ? (c + 1) / 2 : -(c / 2)));
+}
+__device__ __forceinline__ float constant(int k) {  // likewise around 0.5, in steps of 2^-18
+  return 0.5f + static_cast<float>((k & 1) ? (k + 1) / 2 : -(k / 2)) * (1.0f / 262144.0f);
+}
+__device__ __forceinline__ RequantRule block_rule(const PrepareArgs& p) {
+  return sum_requant_rule(dev_maxabs(-p.layer_range, p.layer_range),
+                          dev_maxabs(*p.res_min, *p.res_max), p.sum_min, p.sum_max);
+}
+// doubled factors number c of the rule, where they can be used
+__device__ __forceinline__ bool pair_of_factors(const RequantRule& r, int c, float* a, float* b) {
+  const double level = 2.0 * static_cast<double>(r.in_scale) * static_cast<double>(r.qscale);
+  const float ta = static_cast<float>(r.s0 * level), tb = static_cast<float>(r.s1 * level);
+  *a = moved(ta, c % 7);
+  *b = moved(tb, c / 7);
+  return r.fast && ta > 1e-30f && tb > 1e-30f && ta < 1e30f && tb < 1e30f;
+}
+__global__ void clear_forms_kernel(BlockForms* out) {
+  out->has = 0;
+  out->pair = kPairs;
+}
+__global__ void finish_forms_kernel(PrepareArgs p) {
+  BlockForms* const out = p.out;
+  out->rule = block_rule(p);
+  float a, b;
+  pair_of_factors(out->rule, out->pair % kPairs, &a, &b);
+  out->sum = sum_form(a, b);
+  if (out->pair < kPairs) out->has |= 8;
+}
+__global__ __launch_bounds__(1024) void prepare_block_kernel(PrepareArgs p) {
+  const int tid = threadIdx.x;
+  __shared__ int threshold[128], first;
+  BlockForms* const out = p.out;
+  if (blockIdx.x < 3) {
+    const int layer = blockIdx.x;
+    if (p.prepared[layer] == nullptr) return;
+    const EpiScalars s = *reinterpret_cast<const EpiScalars*>(p.prepared[layer]);
+    // the smallest accumulator of level tid, or the largest int where none reaches it
+    if (tid < 128) {
+      int lo = 0, hi = 0x7fffffff;  // level(lo) < tid, unless tid is 0
+      while (tid > 0 && hi - lo > 1) {
+        const int at = lo + (hi - lo) / 2;
+        (epi_requant(at, s, -127.0f) >= tid ? hi : lo) = at;
+      }
+      threshold[tid] = hi;
+    }
+    if (tid == 0) first = kFactors * kConstants;
+    __syncthreads();
+    const float unit = s.in_scale * s.qscale * (layer == 1 ? 1.0f : 2.0f);
+    if (unit > 1e-30f && unit < 1e30f) {
+      const float t = moved(unit, tid / kConstants), c = constant(tid % kConstants);
+      bool same = true;
+      for (int v = 1; v < 128 && same; ++v) {
+        const int a = threshold[v];
+        for (int d = 0; d < 2; ++d) {  // the definition gives v from a on (unless a is the end)
+          const bool reached = d == 0 && epi_requant(a, s, -127.0f) >= v;
+          const int level = layer == 1
+                                ? static_cast<int>(short_level(a - d, t) & 0xffu) - 128
+                                : static_cast<int>(short_relu4(a - d, 0, 0, 0, t, c) & 0xffu);
+          same = same && (level >= v) == reached;
+        }
+      }
+      if (same) atomicMin(&first, tid);
+    }
+    __syncthreads();
+    if (tid == 0) {
+      const int at = first % (kFactors * kConstants);
+      out->s[layer] = s;
+      out->t[layer] = moved(unit, at / kConstants);
+      out->c[layer] = constant(at % kConstants);
+      if (first < kFactors * kConstants) atomicOr(&out->has, 1 << layer);
+    }
+  } else {
+    const RequantRule r = block_rule(p);
+    float a, b;
+    if (!pair_of_factors(r, blockIdx.x - 3, &a, &b)) return;
+    bool differs = false;
+    for (int i = tid; i < 64 * 256; i += 1024) {
+      const int a0 = 4 * (i >> 8) - 127, y0 = (i & 255) - 128;  // a0 ... a0 + 3
+      int x[4];
+      uint32_t packed = 0;
+      for (int k = 0; k < 4; ++k) {
+        x[k] = a0 + k < 127 ? a0 + k : 127;  // the last quad is one short
+        packed |= (static_cast<uint32_t>(x[k]) & 0xffu) << (8 * k);
+      }
+      const uint32_t y = (static_cast<uint32_t>(y0) & 0xffu) * 0x01010101u;
+      differs |= short_sum4(x[0] + 128, x[1] + 128, x[2] + 128, x[3] + 128, y, sum_form(a, b)) !=
+                 sum_requant4_general<true>(packed, y, r);
+    }
+    if (__syncthreads_or(differs) == 0 && tid == 0)
+      atomicMin(&out->pair, static_cast<int>(blockIdx.x) - 3);
+  }
+}
+
+int up(int n, int unit) { return (n + unit - 1) / unit * unit; }
+
+// How a block of this shape is laid out; `tiles` is 0 where it does not fit.
+struct BlockPlan {
+  int variant = 0;  // 64, 128 or 256: the channels in the middle, at most
+  int tm = 0, tiles = 0;
+  int steps[3] = {0, 0, 0};
+  size_t fragments[3] = {0, 0, 0};  // KB
+  int parts = 0, row_pitch = 0, off_patch = 0, off_bias = 0, off_table = 0, lds = 0;
+};
+// Tile and fragments of a block over these channels; false where no kernel takes them.
+bool plan_layers(int C, int Cm, int Co, int Ca, BlockPlan* b) {
+  for (int v : {C, Cm, Co})
+    if (v <= 0 || v % 16 != 0 || v > 8192) return false;
+  if (Ca < 0 || Ca % 16 != 0 || Ca > 8192 || Cm > 256) return false;
+  b->variant = Cm <= 64 ? 64 : Cm <= 128 ? 128 : 256;
+  b->tm = b->variant == 64 ? 128 : 64;
+  b->steps[0] = up(9 * ((C + 31) / 32), b->variant == 256 ? 8 : 6);
+  b->steps[1] = b->variant / 32;
+  b->steps[2] = up((Co + 31) / 32, 8);
+  const int columns[3] = {Cm, Co, Ca};
+  size_t kb = 0;
+  for (int i = 0; i < 3; ++i) {
+    b->fragments[i] = static_cast<size_t>((columns[i] + 31) / 32) * b->steps[i];
+    kb += b->fragments[i];
+  }
+  return kb < 0x100000;  // offsets in KB below 1 GiB
+}
+BlockPlan plan_block(int N, int H, int W, int C, int Cm, int Co, int Ca) {
+  BlockPlan b;
+  if (!plan_layers(C, Cm, Co, Ca, &b)) return b;
+  if (N <= 0 || H <= 0 || W <= 0 || W > 8192 || H > 8192) return b;
+  const long long M = static_cast<long long>(N) * H * W;
+  const long long widest = Co > C ? Co : C;
+  if (M * (widest > Ca ? widest : Ca) >= (1LL << 31) ||
+      (static_cast<long long>(N) + 1) * (H + 2) * (H + 2) >= (1LL << 30) ||
+      static_cast<long long>(H) * W * W >= (1LL << 30))
+    return b;
+  // virtual rows a tile's pixels can touch: their own, one above and below, two more for every
+  // image boundary inside the tile
+  const int rows = (b.tm + W - 2) / W + 1 + 2 + 2 * ((b.tm + H * W - 2) / (H * W));
+  b.parts = up((W + 2) * odd(C / 16), 64) / 64;
+  // a row begins where the bank group of the pixel behind the last output pixel of the row before
+  // it would be, so that 16 output pixels in a row hit distinct ones across the end of a row as well
+  b.row_pitch = b.parts * 1024 + W * odd(C / 16) % 16 * 16;
+  const int first = rows * b.row_pitch;
+  // whole load instructions of the shortcut and of the bias; what a row's padded steps read past
+  // the end of their part lies in the next one
+  const int wide = up(b.tm * odd_tiles(Co / 16), 64) * 16;
+  const int mid = b.tm * odd_tiles((Cm > Ca ? Cm : Ca) / 16) * 16;
+  const int patch = first > mid ? first : mid;
+  const int bias = 4 * (up(Cm, 256) + up(Co, 256) + up(Ca, 256));
+  const int table = 4 * (b.steps[0] + 2 * 8);
+  const long long lds = static_cast<long long>(wide) + patch + bias + table;
+  if (lds > kBlockLds) return b;
+  b.off_patch = wide;
+  b.off_bias = wide + patch;
+  b.off_table = b.off_bias + bias;
+  b.lds = static_cast<int>(lds);
+  b.tiles = static_cast<int>((M + b.tm - 1) / b.tm);
+  return b;
+}
+
+template <int WM, int WN, int RT, int GB, int GC>
+void launch_block(hipStream_t s, const BlockArgs& a, int lds) {
+  const unsigned grid = static_cast<unsigned>((a.tiles + 7) / 8 * 8);
+  hipLaunchKernelGGL((block_kernel<WM, WN, RT, GB, GC>), dim3(grid), dim3(64 * WM * WN),
+                     static_cast<size_t>(lds), s, a);
+  MXQ_LAUNCH_CHECK();
+}
+
+}  // namespace
+}  // namespace mxq
+
+using namespace mxq;
+
+extern "C" {
+
+// Whether it is also the faster way.  It is from one image on with up to 128 channels in the middle
+// (56 x 56 x 64: 10.3 us against 15.0 in three launches on one image, 44.4 against 59.4 on 64;
+// 28 x 28 x 128 10.3 / 14.5 and 30.3 / 45.3).  Above that a tile alone takes 18 us, most of it the
+// 1.1 MB of weights that a CU takes in: 13 tiles (14 x 14 x 256 on 4 images) 18.9 us against 16.4,
+// 25 tiles 19.1 against 20.4, 196 tiles 22.0 against 38.3.
+int mxq_quantized_block_fits(int N, int H, int W, int C, int C_mid, int C_out, int C_next) {
+  const BlockPlan b = plan_block(N, H, W, C, C_mid, C_out, C_next);
+  return b.tiles > 0 && (b.variant < 256 || b.tiles >= 20) ? 1 : 0;
+}
+
+size_t mxq_quantized_block_weights(int C, int C_mid, int C_out, int C_next) {
+  BlockPlan b;
+  if (!plan_layers(C, C_mid, C_out, C_next, &b)) return 0;
+  return 1024 * (b.fragments[0] + b.fragments[1] + b.fragments[2]);
+}
+
+int mxq_pack_block_weights(void* stream, const int8_t* first, const int8_t* second,
+                           const int8_t* third, int C, int C_mid, int C_out, int C_next,
+                           int8_t* out) {
+  MXQ_API_BEGIN();
+  BlockPlan b;
+  MXQ_CHECK(plan_layers(C, C_mid, C_out, C_next, &b), "bad channel counts");
+  const int8_t* const in[3] = {first, second, third};
+  const int rows[3] = {C_mid, C_out, C_next}, columns[3] = {C, C_mid, C_out};
+  MXQ_CHECK(out != nullptr && aligned16(out), "null or unaligned pointer");
+  for (int i = 0; i < 3; ++i) {
+    if (rows[i] == 0) continue;
+    MXQ_CHECK(in[i] != nullptr && aligned16(in[i]), "null or unaligned pointer");
+    const unsigned pieces = static_cast<unsigned>(b.fragments[i] * 64);
+    hipLaunchKernelGGL(pack_fragments_kernel, dim3((pieces + 255) / 256), dim3(256), 0,
+                       static_cast<hipStream_t>(stream), reinterpret_cast<const v4i*>(in[i]),
+                       reinterpret_cast<v4i*>(out), rows[i], i == 0 ? 9 : 1, columns[i] / 16,
+                       (columns[i] + 31) / 32, b.steps[i], pieces);
+    MXQ_LAUNCH_CHECK();
+    out += b.fragments[i] * 1024;
+  }
+  MXQ_API_END();
+}
+
+size_t mxq_quantized_block_forms(void) { return kBlockForms; }
+
+int mxq_prepare_block(void* stream, const void* prepared_first, const void* prepared_second,
+                      const void* prepared_third, const float* min_residual,
+                      const float* max_residual, float min_calib, float max_calib,
+                      float sum_min_calib, float sum_max_calib, void* forms) {
+  MXQ_API_BEGIN();
+  MXQ_CHECK(prepared_first && prepared_second && min_residual && max_residual && forms,
+            "null pointer");
+  for (const void* v : {prepared_first, prepared_second, prepared_third,
+                        static_cast<const void*>(forms)})
+    MXQ_CHECK(aligned16(v), "unaligned pointer");
+  PrepareArgs a = {};
+  a.prepared[0] = static_cast<const char*>(prepared_first);
+  a.prepared[1] = static_cast<const char*>(prepared_second);
+  a.prepared[2] = static_cast<const char*>(prepared_third);
+  a.res_min = min_residual;
+  a.res_max = max_residual;
+  const float x = fabsf(min_calib), y = fabsf(max_calib);
+  a.layer_range = (x < y) ? y : x;
+  a.sum_min = sum_min_calib;
+  a.sum_max = sum_max_calib;
+  a.out = static_cast<BlockForms*>(forms);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  hipLaunchKernelGGL(clear_forms_kernel, dim3(1), dim3(1), 0, s, a.out);
+  MXQ_LAUNCH_CHECK();
+  hipLaunchKernelGGL(prepare_block_kernel, dim3(3 + kPairs), dim3(1024), 0, s, a);
+  MXQ_LAUNCH_CHECK();
+  hipLaunchKernelGGL(finish_forms_kernel, dim3(1), dim3(1), 0, s, a);
+  MXQ_LAUNCH_CHECK();
+  MXQ_API_END();
+}
+
+int mxq_quantized_block(void* stream, const int8_t* data, const int8_t* weights,
+                        const void* forms, const void* prepared_first,
+                        const void* prepared_second, const void* prepared_third, int N, int H,
+                        int W, int C, int C_mid, int C_out, int C_next, const int8_t* residual, int8_t* out, int8_t* next,
+                        int relu_first, int relu_third) {
+  MXQ_API_BEGIN();
+  const BlockPlan b = plan_block(N, H, W, C, C_mid, C_out, C_next);
+  MXQ_CHECK(b.tiles > 0, "a block of this shape does not fit");
+  MXQ_CHECK(data && weights && forms && residual && out && prepared_first && prepared_second &&
+                (C_next == 0 || (next && prepared_third)),
+            "null pointer");
+  for (const void* v : {static_cast<const void*>(data), static_cast<const void*>(weights), forms,
+                        prepared_first, prepared_second, prepared_third,
+                        static_cast<const void*>(residual), static_cast<const void*>(out),
+                        static_cast<const void*>(next)})
+    MXQ_CHECK(aligned16(v), "unaligned pointer");
+  BlockArgs a = {};
+  a.data = data;
+  a.weights = weights;
+  a.forms = static_cast<const BlockForms*>(forms);
+  a.prepared[0] = static_cast<const char*>(prepared_first);
+  a.prepared[1] = static_cast<const char*>(prepared_second);
+  a.prepared[2] = static_cast<const char*>(prepared_third);
+  a.res = residual;
+  a.out = out;
+  a.next = next;
+  a.N = N; a.H = H; a.W = W; a.C = C; a.Cm = C_mid; a.Co = C_out; a.Ca = C_next;
+  a.M = N * H * W;
+  a.kb = b.steps[0];
+  a.ksb = (C + 31) / 32;
+  a.ka = b.steps[2];
+  a.at_c = static_cast<int>(b.fragments[0]);
+  a.at_a = static_cast<int>(b.fragments[0] + b.fragments[1]);
+  a.kb_all = static_cast<int>(a.at_a + b.fragments[2]);
+  a.off_patch = b.off_patch;
+  a.off_bias = b.off_bias;
+  a.off_table = b.off_table;
+  a.magic_plane = magic_of(H * W);
+  a.magic_w = magic_of(W);
+  a.magic_pixel = magic_of(odd(C / 16));
+  a.parts = b.parts;
+  a.row_pitch = b.row_pitch;
+  a.magic_image = magic_of(H + 2);
+  a.magic_res = magic_of(odd_tiles(C_out / 16));
+  a.magic_wide = magic_of(C_out / 16);
+  a.magic_tap = magic_of(a.ksb);
+  a.magic_next = C_next ? magic_of(C_next / 16) : 0;
+  a.relu_b = relu_first != 0;
+  a.relu_a = relu_third != 0;
+  a.stream = epi_stream_rows(a.M);
+  a.tiles = b.tiles;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (b.variant == 64)
+    launch_block<2, 4, 2, 6, 2>(s, a, b.lds);
+  else if (b.variant == 128)
+    launch_block<1, 8, 2, 6, 4>(s, a, b.lds);
+  else
+    launch_block<1, 8, 2, 8, 8>(s, a, b.lds);
+  MXQ_API_END();
+}
+
+}  // extern "C"
