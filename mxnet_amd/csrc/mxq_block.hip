@@ -23,14 +23,14 @@
 // Rows in LDS are an odd number of 16-byte chunks apart: 16 consecutive rows' fragments hit
 // distinct bank groups without a permutation, for any channel count.
 //
-// What bounds it: a tile's own chain.  Of the 42000 clocks of a tile of 14 x 14 x 256 -> 1024 -> 256
-// (one per CU) 5000 go by until the patch is there, 15000 in the 3 x 3 layer (9200 of matrix work),
-// 14000 in the sum's layer (8000 of vector and 4000 of matrix work that overlap little: two waves of
-// a SIMD run in step from the barrier on), 8000 behind it.  Measured at batch 64 against the three
-// launches: 22.0 us against 38.3 there, 30.3 / 45.3 for 28 x 28 x 128, 44.4 / 59.4 for 56 x 56 x 64.
-// A quantized ResNet-50 at batch 64 takes 716 us with it, 867 without.  Measured and not kept: four
-// row tiles' products made while the tile before is finished (level, 100 registers more), the second
-// layer's operand held in registers (level), wave priorities (level).
+// What bounds it: a tile's own chain.  Of the 42000 clocks of a tile of 14 x 14 x 256 -> 1024 ->
+// 256 (one per CU) 5000 go by until the patch is there, 15000 in the 3 x 3 layer (9200 of matrix
+// work), 14000 in the sum's layer (8000 of vector and 4000 of matrix work that overlap little: two
+// waves of a SIMD run in step from the barrier on), 8000 behind it.  Measured at batch 64 against
+// the three launches: 22.8 us against 38.3 there, 31 / 45 for 28 x 28 x 128, 38.6 / 60 for 56 x 56 x
+// 64.  A quantized ResNet-50 at batch 64 takes 667 us with it, 867 without, one image 234 and 241.
+// Measured and not kept: a column tile's products made while the one before is finished (level, 100
+// registers more), the second layer's operand held in registers (level), wave priorities (level).
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -126,15 +126,18 @@ struct BlockArgs {
   const int8_t* res;      // [M][Co]
   int8_t* out;            // [M][Co]
   int8_t* next;           // [M][Ca]
-  int N, H, W, C, Cm, Co, Ca, M;
+  int N, H, W, C, Cm, Co, Ca;
   int kb, ksb;            // MFMA steps of the 3 x 3 layer, and of one tap of it
   int ka;                 // ... of the last layer
   int at_c, at_a, kb_all; // where the second and third layer's fragments begin (KB), and all end
-  int off_patch, off_bias, off_table;  // bytes in LDS
+  int run;                // whether tiles are runs of pixels; else of tn images, th rows, tw columns
+  int tn, th, tw, tiles_h, tiles_w;  // tiles down and across an image
+  int area, across, count, rows;     // (above) and pixels of a tile, rows of its patch
+  int off_patch, off_bias, off_table, off_pixel;  // bytes in LDS
   int parts, row_pitch;   // load instructions and bytes per row of the patch
-  uint32_t magic_plane, magic_w, magic_pixel, magic_image, magic_res, magic_wide,
-      magic_next, magic_tap;
-  int relu_b, relu_a, stream, tiles;
+  uint32_t magic_tiles_w, magic_tiles_h, magic_area, magic_across, magic_h2, magic_pixel, magic_res,
+      magic_wide, magic_next, magic_tap;
+  int relu_b, relu_a, tiles;
 };
 
 __host__ __device__ constexpr int odd(int chunks) { return chunks | 1; }
@@ -164,10 +167,12 @@ __global__ __launch_bounds__(64 * WM * WN, GC < 8 ? 4 : 2) void block_kernel(Blo
   // round trip at a time, 3000 clocks before the first pixels are requested
   asm volatile("" ::"s"(p.data), "s"(p.weights), "s"(p.forms), "s"(p.prepared[0]),
                "s"(p.prepared[1]), "s"(p.prepared[2]), "s"(p.res), "s"(p.N), "s"(p.H), "s"(p.W),
-               "s"(p.C), "s"(p.Cm), "s"(p.Co), "s"(p.Ca), "s"(p.M), "s"(p.kb), "s"(p.ksb),
+               "s"(p.C), "s"(p.Cm), "s"(p.Co), "s"(p.Ca), "s"(p.kb), "s"(p.ksb),
                "s"(p.at_c), "s"(p.kb_all), "s"(p.off_patch), "s"(p.off_bias), "s"(p.off_table),
-               "s"(p.magic_plane), "s"(p.magic_w), "s"(p.magic_pixel), "s"(p.parts), "s"(p.row_pitch),
-               "s"(p.magic_image), "s"(p.magic_res), "s"(p.magic_tap), "s"(p.tiles));
+               "s"(p.run), "s"(p.area), "s"(p.across), "s"(p.count), "s"(p.rows), "s"(p.off_pixel),
+               "s"(p.magic_area), "s"(p.magic_across), "s"(p.magic_h2),
+               "s"(p.magic_pixel), "s"(p.parts), "s"(p.row_pitch), "s"(p.magic_res),
+               "s"(p.magic_tap), "s"(p.tiles));
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WN, wn = wave % WN;
@@ -175,12 +180,24 @@ __global__ __launch_bounds__(64 * WM * WN, GC < 8 ? 4 : 2) void block_kernel(Blo
   const int per = (p.tiles + 7) >> 3;
   const int tile = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
   if (tile >= p.tiles) return;
-  const int m0 = tile * TM;
-  const int CH = p.C >> 4, PP = odd(CH), H2 = p.H + 2;
+  // The tile's pixel i is pixel (h0, w0) + place start + i of rows of `across` in images of `area`
+  // pixels, from image n0 on: a rectangle, whole images, or a run of pixels in the tensor's order.
+  int n0, h0 = 0, w0 = 0, start_at = 0;
+  if (p.run) {
+    n0 = quotient_any(tile * TM, p.area, p.magic_area);
+    start_at = tile * TM - n0 * p.area;
+  } else {
+    const int down = quotient(tile, p.magic_tiles_w), batch = quotient(down, p.magic_tiles_h);
+    n0 = batch * p.tn;
+    h0 = (down - batch * p.tiles_h) * p.th;
+    w0 = (tile - down * p.tiles_w) * p.tw;
+  }
+  // rows of the patch are rows of the images one below the other, each with one more above and below
+  const int H2 = p.H + 2, v0 = n0 * H2 + h0 + quotient(start_at, p.magic_across);
+  const int CH = p.C >> 4, PP = odd(CH);
   const int row_pitch = p.row_pitch;  // bytes of a patch row
   const int PM = odd_tiles(p.Cm >> 4), CO = p.Co >> 4, PO = odd_tiles(CO);
   const int CA = p.Ca >> 4, PA = odd_tiles(CA);
-  const int plane = p.H * p.W;
   const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(smem));
   // 64 pieces of 16 bytes to `to` and on in LDS
   auto fetch = [&](int to, uint32_t from, v4i rsrc) MXQ_INLINE {
@@ -202,42 +219,47 @@ __global__ __launch_bounds__(64 * WM * WN, GC < 8 ? 4 : 2) void block_kernel(Blo
 #pragma unroll
   for (int i = 0; i < GB; ++i) wb[i] = fragment(first_b + i);
 
-  // the patch: virtual rows n * (H + 2) + ih + 1, so that the zero rows above and below an image
-  // are rows like any other
-  const int mb = (m0 + TM - 1 < p.M) ? m0 + TM - 1 : p.M - 1;
-  const int na = quotient_any(m0, plane, p.magic_plane);
-  const int oha = quotient(m0 - na * plane, p.magic_w);
-  const int nb = quotient_any(mb, plane, p.magic_plane);
-  const int ohb = quotient(mb - nb * plane, p.magic_w);
-  const int vr0 = na * H2 + oha, rows = nb * H2 + ohb + 2 - vr0 + 1;
+  // the patch: the tile's rows of every one of its images and one above and below, a column on
+  // either side; zeros where they leave the image
   {
-    const v4i rsrc = make_rsrc(p.data, static_cast<uint32_t>(p.N) * plane * p.C);
+    const v4i rsrc = make_rsrc(p.data, static_cast<uint32_t>(p.N) * p.H * p.W * p.C);
     // A row of the patch is a whole number of load instructions: a lane's place in the row stays as
     // the wave goes down the rows, and a row is one scalar offset.  (A lane that finds its pixel
     // anew for every piece, by divisions or by carries, costs 300 clocks per instruction.)
-    int j = lane, iw = -1;
+    int j = lane, px = 0;
     const int row_bytes = p.W * p.C;
     int carry = quotient(j, p.magic_pixel);
     j -= carry * PP;
-    iw += carry;
+    px += carry;
     const int step = quotient(64, p.magic_pixel), rest = 64 - step * PP;
     for (int part = 0; part < p.parts; ++part) {
-      const bool ok = j < CH && static_cast<unsigned>(iw) < static_cast<unsigned>(p.W);
+      const int iw = w0 + px - 1;
+      const bool ok = j < CH && px < p.across + 2 &&
+                      static_cast<unsigned>(iw) < static_cast<unsigned>(p.W);
       const uint32_t place = ok ? static_cast<uint32_t>(iw * p.C + 16 * j) : kOutOfRange;
-      for (int r = wave; r < rows; r += NW) {
-        const int v = vr0 + r, n = quotient(v, p.magic_image), ih = v - n * H2 - 1;
+      for (int r = wave; r < p.rows; r += NW) {
+        const int n = quotient_any(v0 + r, H2, p.magic_h2), ih = v0 + r - n * H2 - 1;
         const bool inside = n < p.N && static_cast<unsigned>(ih) < static_cast<unsigned>(p.H);
         fetch(p.off_patch + r * row_pitch + part * 1024,
               inside ? place + static_cast<uint32_t>((n * p.H + ih) * row_bytes) : kOutOfRange,
               rsrc);
       }
       j += rest;
-      iw += step;
+      px += step;
       if (j >= PP) {
         j -= PP;
-        ++iw;
+        ++px;
       }
     }
+  }
+  // which pixel of the tensor each of the tile's is, -1 past the edges
+  int* const pixel_of = reinterpret_cast<int*>(smem + p.off_pixel);
+  if (tid < TM) {
+    const int img = quotient_any(start_at + tid, p.area, p.magic_area), rem = start_at + tid - img * p.area;
+    const int ty = quotient(rem, p.magic_across), tx = rem - ty * p.across;
+    const int n = n0 + img, h = h0 + ty, w = w0 + tx;
+    const bool ok = tid < p.count && n < p.N && h < p.H && w < p.W;
+    pixel_of[tid] = ok ? (n * p.H + h) * p.W + w : -1;
   }
   const int* const sbias = reinterpret_cast<const int*>(smem + p.off_bias);
   const int bias_c = (p.Cm + 255) & ~255, bias_a = bias_c + ((p.Co + 255) & ~255);
@@ -266,16 +288,16 @@ __global__ __launch_bounds__(64 * WM * WN, GC < 8 ? 4 : 2) void block_kernel(Blo
         kh * row_pitch + (tap - 3 * kh) * PP * 16 + (at - tap * p.ksb) * 32;
   }
   // The shortcut, a share of it at a time while the 3 x 3 layer runs.
-  const v4i res_rsrc = make_rsrc(p.res, static_cast<uint32_t>(p.M) * p.Co);
+  const v4i res_rsrc = make_rsrc(p.res, static_cast<uint32_t>(p.N) * p.H * p.W * p.Co);
   const int res_slots = TM * PO;
   int res_at = wave;
   auto fetch_shortcut = [&]() MXQ_INLINE {
     if (res_at * 64 < res_slots) {
       const int q = res_at * 64 + lane;
       const int row = quotient(q, p.magic_res), j = q - row * PO;
-      const bool ok = j < CO && row < TM && m0 + row < p.M;
-      fetch(res_at * 1024,
-                 ok ? static_cast<uint32_t>((m0 + row) * p.Co + 16 * j) : kOutOfRange, res_rsrc);
+      const int pixel = row < TM && j < CO ? pixel_of[row] : -1;
+      fetch(res_at * 1024, pixel >= 0 ? static_cast<uint32_t>(pixel * p.Co + 16 * j) : kOutOfRange,
+            res_rsrc);
       res_at += NW;
     }
   };
@@ -286,11 +308,13 @@ __global__ __launch_bounds__(64 * WM * WN, GC < 8 ? 4 : 2) void block_kernel(Blo
   int in_patch[RT];
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) {
-    int m = m0 + row0 + 32 * rt;
-    m = m < p.M ? m : p.M - 1;  // rows past the end repeat the last pixel; never stored
-    const int n = quotient_any(m, plane, p.magic_plane), rem = m - n * plane;
-    const int oh = quotient(rem, p.magic_w), ow = rem - oh * p.W;
-    in_patch[rt] = p.off_patch + (n * H2 + oh - vr0) * row_pitch + ow * PP * 16 + fgrp * 16;
+    int i = row0 + 32 * rt;
+    // rows without a pixel read the first one's; never stored
+    i = start_at + (i < p.count ? i : 0);
+    const int img = quotient_any(i, p.area, p.magic_area), rem = i - img * p.area;
+    const int ty = quotient(rem, p.magic_across), tx = rem - ty * p.across;
+    in_patch[rt] = p.off_patch + ((n0 + img) * H2 + h0 + ty - v0) * row_pitch + tx * PP * 16 +
+                   fgrp * 16;
   }
   v16i acc[RT];
   auto read_bias = [&](const int* bias, v4i (&b)[4]) MXQ_INLINE {
@@ -465,20 +489,18 @@ __global__ __launch_bounds__(64 * WM * WN, GC < 8 ? 4 : 2) void block_kernel(Blo
   }
   publish();
 
-  // rows of `chunks` pieces, `pitch` apart in LDS, to consecutive memory
-  const int rows_left = p.M - m0 < TM ? p.M - m0 : TM;
-  auto leave = [&](int at, int chunks, int pitch, uint32_t magic, int8_t* out, auto stream) MXQ_INLINE {
-    for (int i = tid; i < rows_left * chunks; i += 64 * NW) {
-      const int row = quotient(i, magic);
-      epi_store16<decltype(stream)::value>(
-          *reinterpret_cast<const v4i*>(smem + at + (row * pitch + i - row * chunks) * 16),
-          out + static_cast<size_t>(m0) * chunks * 16 + static_cast<size_t>(i) * 16);
+  // Rows of `chunks` pieces, `pitch` apart in LDS, to their pixels.  Plain stores: the next block
+  // reads both outputs, and what it finds in the memory-side cache it does not fetch from memory
+  // (quantized ResNet-50 at batch 64, all blocks with streaming stores / plain ones: 680 / 651 us).
+  auto leave = [&](int at, int chunks, int pitch, uint32_t magic, int8_t* out) MXQ_INLINE {
+    for (int i = tid; i < TM * chunks; i += 64 * NW) {
+      const int row = quotient(i, magic), j = i - row * chunks, pixel = pixel_of[row];
+      if (pixel >= 0)
+        *reinterpret_cast<v4i*>(out + (static_cast<size_t>(pixel) * chunks + j) * 16) =
+            *reinterpret_cast<const v4i*>(smem + at + (row * pitch + j) * 16);
     }
   };
-  if (p.stream)
-    leave(0, CO, PO, p.magic_wide, p.out, std::true_type());
-  else
-    leave(0, CO, PO, p.magic_wide, p.out, std::false_type());
+  leave(0, CO, PO, p.magic_wide, p.out);
   if (p.Ca == 0) return;
 
   // ---- the next block's first 1 x 1 ---------------------------------------------------------
@@ -496,7 +518,7 @@ __global__ __launch_bounds__(64 * WM * WN, GC < 8 ? 4 : 2) void block_kernel(Blo
     finish_layer(s_a, t_a, c_a, (has & 4) != 0, p.relu_a, t, PA);
   }
   publish();
-  leave(p.off_patch, CA, PA, p.magic_next, p.next, std::false_type());
+  leave(p.off_patch, CA, PA, p.magic_next, p.next);
 }
 
 // [O][taps][C] rows -> fragments [ceil(O / 32)][steps][64 lanes][16 bytes]: lane l of step
@@ -630,7 +652,8 @@ struct BlockPlan {
   int tm = 0, tiles = 0;
   int steps[3] = {0, 0, 0};
   size_t fragments[3] = {0, 0, 0};  // KB
-  int parts = 0, row_pitch = 0, off_patch = 0, off_bias = 0, off_table = 0, lds = 0;
+  int run = 0, tn = 1, th = 1, tw = 1, tiles_h = 1, tiles_w = 1, rows = 0;
+  int parts = 0, row_pitch = 0, off_patch = 0, off_bias = 0, off_table = 0, off_pixel = 0, lds = 0;
 };
 // Tile and fragments of a block over these channels; false where no kernel takes them.
 bool plan_layers(int C, int Cm, int Co, int Ca, BlockPlan* b) {
@@ -638,7 +661,7 @@ bool plan_layers(int C, int Cm, int Co, int Ca, BlockPlan* b) {
     if (v <= 0 || v % 16 != 0 || v > 8192) return false;
   if (Ca < 0 || Ca % 16 != 0 || Ca > 8192 || Cm > 256) return false;
   b->variant = Cm <= 64 ? 64 : Cm <= 128 ? 128 : 256;
-  b->tm = b->variant == 64 ? 128 : 64;
+  b->tm = 64;
   b->steps[0] = up(9 * ((C + 31) / 32), b->variant == 256 ? 8 : 6);
   b->steps[1] = b->variant / 32;
   b->steps[2] = up((Co + 31) / 32, 8);
@@ -650,38 +673,84 @@ bool plan_layers(int C, int Cm, int Co, int Ca, BlockPlan* b) {
   }
   return kb < 0x100000;  // offsets in KB below 1 GiB
 }
+// The parts of LDS for a patch of b->rows rows of b->tw + 2 pixels; whether they fit.
+bool fit_lds(BlockPlan* b, int C, int Cm, int Co, int Ca) {
+  b->parts = up((b->tw + 2) * odd(C / 16), 64) / 64;
+  // a row begins where the bank group of the pixel behind the last output pixel of the row before
+  // it would be, so that 16 output pixels in a row hit distinct ones across the end of a row as well
+  b->row_pitch = b->parts * 1024 + b->tw * odd(C / 16) % 16 * 16;
+  const long long first = static_cast<long long>(b->rows) * b->row_pitch;
+  if (first > kBlockLds) return false;
+  // whole load instructions of the shortcut and of the bias; what a row's padded steps read past
+  // the end of their part lies in the next one
+  const int wide = up(b->tm * odd_tiles(Co / 16), 64) * 16;
+  const int mid = b->tm * odd_tiles((Cm > Ca ? Cm : Ca) / 16) * 16;
+  const int patch = first > mid ? static_cast<int>(first) : mid;
+  const int bias = 4 * (up(Cm, 256) + up(Co, 256) + up(Ca, 256));
+  const int table = 4 * (b->steps[0] + 2 * 8);
+  const long long lds = static_cast<long long>(wide) + patch + bias + table + 4 * b->tm;
+  b->off_patch = wide;
+  b->off_bias = wide + patch;
+  b->off_table = b->off_bias + bias;
+  b->off_pixel = b->off_table + table;
+  b->lds = static_cast<int>(lds);
+  return lds <= kBlockLds;
+}
 BlockPlan plan_block(int N, int H, int W, int C, int Cm, int Co, int Ca) {
   BlockPlan b;
   if (!plan_layers(C, Cm, Co, Ca, &b)) return b;
   if (N <= 0 || H <= 0 || W <= 0 || W > 8192 || H > 8192) return b;
   const long long M = static_cast<long long>(N) * H * W;
   const long long widest = Co > C ? Co : C;
-  if (M * (widest > Ca ? widest : Ca) >= (1LL << 31) ||
-      (static_cast<long long>(N) + 1) * (H + 2) * (H + 2) >= (1LL << 30) ||
-      static_cast<long long>(H) * W * W >= (1LL << 30))
+  if (M * (widest > Ca ? widest : Ca) >= (1LL << 31) || (M + 64) * 2 >= (1LL << 31) ||
+      (static_cast<long long>(H) * W + 64) * W >= (1LL << 30) ||
+      (N + 1LL) * (H + 2) + 256 >= (1LL << 30))
     return b;
-  // virtual rows a tile's pixels can touch: their own, one above and below, two more for every
-  // image boundary inside the tile
-  const int rows = (b.tm + W - 2) / W + 1 + 2 + 2 * ((b.tm + H * W - 2) / (H * W));
-  b.parts = up((W + 2) * odd(C / 16), 64) / 64;
-  // a row begins where the bank group of the pixel behind the last output pixel of the row before
-  // it would be, so that 16 output pixels in a row hit distinct ones across the end of a row as well
-  b.row_pitch = b.parts * 1024 + W * odd(C / 16) % 16 * 16;
-  const int first = rows * b.row_pitch;
-  // whole load instructions of the shortcut and of the bias; what a row's padded steps read past
-  // the end of their part lies in the next one
-  const int wide = up(b.tm * odd_tiles(Co / 16), 64) * 16;
-  const int mid = b.tm * odd_tiles((Cm > Ca ? Cm : Ca) / 16) * 16;
-  const int patch = first > mid ? first : mid;
-  const int bias = 4 * (up(Cm, 256) + up(Co, 256) + up(Ca, 256));
-  const int table = 4 * (b.steps[0] + 2 * 8);
-  const long long lds = static_cast<long long>(wide) + patch + bias + table;
-  if (lds > kBlockLds) return b;
-  b.off_patch = wide;
-  b.off_bias = wide + patch;
-  b.off_table = b.off_bias + bias;
-  b.lds = static_cast<int>(lds);
-  b.tiles = static_cast<int>((M + b.tm - 1) / b.tm);
+  // A run of pixels in the tensor's order wastes no row of a tile, but its patch is three to five
+  // times the tile: 36 KB for 64 pixels of a 56 x 56 plane over 64 channels where 8 x 8 of them need
+  // 10, and LDS is what limits the work-groups a CU holds.  So runs where a CU holds one anyway or
+  // where it still holds two; rectangles elsewhere.  (Batch 64, runs / rectangles: 56 x 56 x 64 43.4 /
+  // 39.0 us, 28 x 28 x 128 31.6 / 32.0, 14 x 14 x 256 23.2 / 24.6.)
+  if (b.variant > 64) {
+    b.run = 1;
+    // its rows, one above and below, two more for every image boundary inside
+    b.rows = (b.tm + W - 2) / W + 1 + 2 + 2 * ((b.tm + H * W - 2) / (H * W));
+    b.tw = W;
+    const long long tiles = (M + b.tm - 1) / b.tm;
+    if (fit_lds(&b, C, Cm, Co, Ca) && (b.variant == 256 || 2 * b.lds <= kBlockLds)) {
+      b.tiles = static_cast<int>(tiles);
+      return b;
+    }
+    b.run = 0;
+  }
+  // Whole images where one is no larger than a tile; else the rectangle that wastes least, a pixel
+  // of the halo counted as a quarter of a row of the tile.
+  if (H * W <= b.tm) {
+    b.tn = b.tm / (H * W) < N ? b.tm / (H * W) : N;
+    b.th = H;
+    b.tw = W;
+  } else {
+    long long best = -1;
+    for (int across = (W + b.tm - 1) / b.tm; across <= W; ++across) {
+      const int tw = (W + across - 1) / across;
+      if ((W + tw - 1) / tw != across) continue;
+      const int most = b.tm / tw < H ? b.tm / tw : H, down = (H + most - 1) / most;
+      const int th = (H + down - 1) / down;
+      const long long cost = static_cast<long long>(across) * down * (4 * b.tm + (th + 2) * (tw + 2));
+      if (best < 0 || cost < best) {
+        best = cost;
+        b.th = th;
+        b.tw = tw;
+        b.tiles_h = down;
+        b.tiles_w = across;
+      }
+    }
+  }
+  b.rows = b.tn * (b.th + 2);
+  const long long tiles = static_cast<long long>((N + b.tn - 1) / b.tn) * b.tiles_h * b.tiles_w;
+  if (fit_lds(&b, C, Cm, Co, Ca) &&
+      tiles * (b.tiles_w > b.tiles_h ? b.tiles_w : b.tiles_h) < (1 << 30))
+    b.tiles = static_cast<int>(tiles);
   return b;
 }
 
@@ -701,8 +770,8 @@ using namespace mxq;
 extern "C" {
 
 // Whether it is also the faster way.  It is from one image on with up to 128 channels in the middle
-// (56 x 56 x 64: 10.3 us against 15.0 in three launches on one image, 44.4 against 59.4 on 64;
-// 28 x 28 x 128 10.3 / 14.5 and 30.3 / 45.3).  Above that a tile alone takes 18 us, most of it the
+// (56 x 56 x 64: 7.8 us against 14.1 in three launches on one image, 38.6 against 60.2 on 64;
+// 28 x 28 x 128 10.7 / 13.3 and 30.4 / 45.2).  Above that a tile alone takes 18 us, most of it the
 // 1.1 MB of weights that a CU takes in: 13 tiles (14 x 14 x 256 on 4 images) 18.9 us against 16.4,
 // 25 tiles 19.1 against 20.4, 196 tiles 22.0 against 38.3.
 int mxq_quantized_block_fits(int N, int H, int W, int C, int C_mid, int C_out, int C_next) {
@@ -799,7 +868,7 @@ int mxq_quantized_block(void* stream, const int8_t* data, const int8_t* weights,
   a.out = out;
   a.next = next;
   a.N = N; a.H = H; a.W = W; a.C = C; a.Cm = C_mid; a.Co = C_out; a.Ca = C_next;
-  a.M = N * H * W;
+  
   a.kb = b.steps[0];
   a.ksb = (C + 31) / 32;
   a.ka = b.steps[2];
@@ -809,23 +878,30 @@ int mxq_quantized_block(void* stream, const int8_t* data, const int8_t* weights,
   a.off_patch = b.off_patch;
   a.off_bias = b.off_bias;
   a.off_table = b.off_table;
-  a.magic_plane = magic_of(H * W);
-  a.magic_w = magic_of(W);
+  a.run = b.run; a.tn = b.tn; a.th = b.th; a.tw = b.tw; a.tiles_h = b.tiles_h; a.tiles_w = b.tiles_w;
+  a.area = b.run ? H * W : b.th * b.tw;
+  a.across = b.tw;
+  a.count = b.run ? b.tm : b.tn * b.th * b.tw;
+  a.rows = b.rows;
+  a.off_pixel = b.off_pixel;
+  a.magic_tiles_w = magic_of(b.tiles_w);
+  a.magic_tiles_h = magic_of(b.tiles_h);
+  a.magic_area = magic_of(a.area);
+  a.magic_across = magic_of(b.tw);
+  a.magic_h2 = magic_of(H + 2);
   a.magic_pixel = magic_of(odd(C / 16));
   a.parts = b.parts;
   a.row_pitch = b.row_pitch;
-  a.magic_image = magic_of(H + 2);
   a.magic_res = magic_of(odd_tiles(C_out / 16));
   a.magic_wide = magic_of(C_out / 16);
   a.magic_tap = magic_of(a.ksb);
   a.magic_next = C_next ? magic_of(C_next / 16) : 0;
   a.relu_b = relu_first != 0;
   a.relu_a = relu_third != 0;
-  a.stream = epi_stream_rows(a.M);
   a.tiles = b.tiles;
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (b.variant == 64)
-    launch_block<2, 4, 2, 6, 2>(s, a, b.lds);
+    launch_block<2, 2, 1, 6, 2>(s, a, b.lds);
   else if (b.variant == 128)
     launch_block<1, 8, 2, 6, 4>(s, a, b.lds);
   else
