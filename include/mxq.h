@@ -524,6 +524,16 @@ int mxq_minmax_f32(void* stream, const float* in, size_t n, float* out_min, floa
 int mxq_histogram_f32(void* stream, const float* in, size_t n, const float* edges, int bins,
                       uint32_t* counts);
 
+/* Entropy calibration: bounds [lower, upper] of what mxq_calibrate_entropy's float sums give for
+ * every candidate threshold, narrowest first, of up to 16 histograms (`hist`, on the device, one
+ * behind the other, finite, none negative, less than 2^31 counts each; `bins` odd, up to 32767, and
+ * `levels` of 3 and more, on the host), as doubles on the device; (-inf, inf) where none are known,
+ * (inf, inf) for a candidate without a quantized distribution. */
+size_t mxq_entropy_bounds_workspace(int count, const int* bins, const int* levels);
+int mxq_entropy_bounds(void* stream, int count, const float* hist, const int* bins,
+                       const int* levels, double* bounds, void* workspace,
+                       size_t workspace_bytes);
+
 /* [N,C,H,W] int8 -> [N,H,W,C] int8 (also OIHW -> OHWI for the weight). */
 int mxq_nchw_to_nhwc_i8(void* stream, const int8_t* in, int8_t* out, int N, int C, int H, int W);
 /* The same with the channel extent of the output padded to C_padded >= C with zeros

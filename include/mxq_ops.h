@@ -99,6 +99,12 @@ int mxq_calibrate_entropy_many(int count, const float* const* hist,
                                const float* const* hist_edges, const size_t* num_bins,
                                const int* num_quantized_bins, float* out_thresholds,
                                float* out_divergences);
+/* With bounds of the candidates' divergences (mxq_entropy_bounds, copied to the host, the
+ * histograms' one behind the other): only the candidates that can be the smallest are summed up. */
+int mxq_calibrate_entropy_bounded(int count, const float* const* hist,
+                                  const float* const* hist_edges, const size_t* num_bins,
+                                  const int* num_quantized_bins, const double* bounds,
+                                  float* out_thresholds, float* out_divergences);
 
 /* ---- NDArray list files (`.params`, mx.nd.save / mx.nd.load) ------------------------
  * src/ndarray/ndarray.cc:1856-2146: dense arrays of the V2 / V3 record layouts plus the

@@ -3,6 +3,7 @@ Tensors must be contiguous CUDA(HIP) tensors; outputs are allocated with torch
 and the calls are enqueued on torch's current stream."""
 import ctypes
 
+import numpy as np
 import torch
 
 from . import _frontend, _lib
@@ -287,6 +288,25 @@ def minmax(data):
     ws = _workspace(wsb, data.device)
     check(lib.mxq_minmax_f32(_stream(), _ptr(data), n, _ptr(out), _ptr(out[1:]), _ptr(ws), wsb))
     return out
+
+
+def entropy_bounds(hists, levels):
+    """float64 [candidate, 2] on the host: bounds of what the entropy calibration's float sums give
+    for every candidate of numpy histograms, one behind the other; taken on the current device."""
+    dev = torch.device("cuda", torch.cuda.current_device())
+    found = []
+    for at in range(0, len(hists), 16):  # as many as a call takes
+        h, n = hists[at:at + 16], levels[at:at + 16]
+        bins, quantized = (ctypes.c_int * len(h))(*[x.size for x in h]), (ctypes.c_int * len(h))(*n)
+        data = torch.from_numpy(np.concatenate(h)).to(dev)
+        out = torch.empty(sum(b // 2 + 1 - q // 2 for b, q in zip(bins, quantized)), 2,
+                          dtype=torch.float64, device=dev)
+        wsb = lib.mxq_entropy_bounds_workspace(len(h), bins, quantized)
+        ws = _workspace(wsb, dev)
+        check(lib.mxq_entropy_bounds(_stream(), len(h), _ptr(data), bins, quantized, _ptr(out),
+                                     _ptr(ws), wsb))
+        found.append(out)
+    return torch.cat(found).cpu().numpy() if len(found) > 1 else found[0].cpu().numpy()
 
 
 def histogram(data, edges):

@@ -37,10 +37,11 @@ Graph SetCalibTable(const Graph& g, const std::map<std::string, std::pair<float,
 // observed one.  hist has an odd number of bins, hist_edges one more entry.
 void CalibrateEntropy(const float* hist, const float* hist_edges, size_t num_bins,
                       int num_quantized_bins, float* threshold, float* divergence);
-// The same for `count` histograms at once: their candidates share one set of threads.
+// The same for `count` histograms at once: their candidates share one set of threads.  `bounds`,
+// unless it is null: [lower, upper] of every candidate, the narrowest of a histogram first.
 void CalibrateEntropyMany(size_t count, const float* const* hist, const float* const* hist_edges,
                           const size_t* num_bins, const int* num_quantized_bins,
-                          float* thresholds, float* divergences);
+                          const double* bounds, float* thresholds, float* divergences);
 
 }  // namespace mxq_graph
 

@@ -379,7 +379,21 @@ int mxq_calibrate_entropy_many(int count, const float* const* hist,
   CHECK(hist && hist_edges && num_bins && num_quantized_bins && out_thresholds && out_divergences)
       << "null argument";
   mxq_graph::CalibrateEntropyMany(static_cast<size_t>(count), hist, hist_edges, num_bins,
-                                  num_quantized_bins, out_thresholds, out_divergences);
+                                  num_quantized_bins, nullptr, out_thresholds, out_divergences);
+  OPS_API_END();
+}
+
+int mxq_calibrate_entropy_bounded(int count, const float* const* hist,
+                                  const float* const* hist_edges, const size_t* num_bins,
+                                  const int* num_quantized_bins, const double* bounds,
+                                  float* out_thresholds, float* out_divergences) {
+  OPS_API_BEGIN();
+  CHECK(count >= 0) << "negative count";
+  CHECK(hist && hist_edges && num_bins && num_quantized_bins && bounds && out_thresholds &&
+        out_divergences)
+      << "null argument";
+  mxq_graph::CalibrateEntropyMany(static_cast<size_t>(count), hist, hist_edges, num_bins,
+                                  num_quantized_bins, bounds, out_thresholds, out_divergences);
   OPS_API_END();
 }
 

@@ -1,0 +1,406 @@
+// Bounds of every candidate's divergence in the entropy calibration (_contrib_calibrate_entropy,
+// src/operator/quantization/calibrate.cc:33-186), from which the host picks the few candidates it
+// has to sum up in float itself (host/mxq_calibrate.cc, which defines a candidate, its levels, its
+// two smoothed distributions and the order of the sums).
+//
+// What the divergence depends on in float are the two normalisations: chains of up to `bins`
+// additions, taken here in the same order, a lane per candidate (thousands of chains side by side:
+// what 16 host threads need 4 ms for).  The terms themselves are then summed up in double from the
+// same float quotients, a wave per candidate, 256 bins at a time with their running sums: what the
+// float chain can differ from that by is bounded by the roundings of its terms and of its additions,
+// each one of the running sum it rounds.  Any bounds a few times wider cost the host a multiple of
+// the candidates (its own, from sums of magnitudes only, leave 10 % of them).
+//
+// Three histograms of 8001 bins, 11622 candidates, with 16 host threads: 7.5 ms of search become 0.4
+// of launches and 0.4 of sums on the host.
+#include <hip/hip_runtime.h>
+
+#include <cmath>
+#include <cstdint>
+
+#include "../../include/mxq.h"
+#include "mxq_common.h"
+
+namespace mxq {
+namespace {
+
+constexpr float kEps = 0.0001f;
+constexpr int kMaxBins = 32767;     // a histogram in LDS
+constexpr int kMaxProblems = 16;    // of one set of launches: their descriptions are an argument
+
+struct Problem {
+  int hist;       // where its bins begin
+  int bins, levels, half, zero, candidates;
+  int prefix;     // where its prefix sums begin
+  int candidate;  // where its candidates begin
+  long long level;  // where their levels begin
+};
+struct Info {     // of a candidate
+  float first, last, p_take, q_take, p_sum, q_sum;
+  int state;      // 0: bounded, 1: infinite, 2: unknown (the host's chain reports what is wrong)
+};
+struct Args {
+  Problem p[kMaxProblems];
+  const float* hist;
+  int *counts, *filled, *seen;  // prefix sums of the integer parts, of them that are not 0, of bins
+  float* head;                  // float sums from the first bin on
+  int* exact;                   // per problem: every partial sum of counts is exact
+  float* levels;                // [candidate][level], not smoothed
+  Info* info;
+  double* bounds;               // [candidate][2]
+};
+
+// Prefix sums of one histogram, a contiguous run of bins per thread.
+__global__ __launch_bounds__(1024) void entropy_prefix_kernel(Args a) {
+  const Problem p = a.p[blockIdx.x];
+  const float* const h = a.hist + p.hist;
+  const int tid = threadIdx.x, per = (p.bins + 1023) / 1024;
+  const int from = tid * per < p.bins ? tid * per : p.bins;
+  const int to = from + per < p.bins ? from + per : p.bins;
+  __shared__ int sums[3][1024];
+  int s[3] = {0, 0, 0};
+  bool whole = true;
+  for (int j = from; j < to; ++j) {
+    const int n = static_cast<int>(h[j]);
+    whole = whole && static_cast<float>(n) == h[j];
+    s[0] += n;
+    s[1] += n != 0;
+    s[2] += h[j] != 0.0f;
+  }
+  for (int k = 0; k < 3; ++k) sums[k][tid] = s[k];
+  whole = __syncthreads_and(whole) != 0;
+  for (int step = 1; step < 1024; step *= 2) {
+    int add[3];
+    for (int k = 0; k < 3; ++k) add[k] = tid >= step ? sums[k][tid - step] : 0;
+    __syncthreads();
+    for (int k = 0; k < 3; ++k) sums[k][tid] += add[k];
+    __syncthreads();
+  }
+  const int total = sums[0][1023];
+  const bool exact = whole && total < (1 << 24);
+  int at[3];
+  for (int k = 0; k < 3; ++k) at[k] = sums[k][tid] - s[k];
+  int* const out[3] = {a.counts + p.prefix, a.filled + p.prefix, a.seen + p.prefix};
+  for (int j = from; j < to; ++j) {
+    for (int k = 0; k < 3; ++k) out[k][j] = at[k];
+    const int n = static_cast<int>(h[j]);
+    at[0] += n;
+    at[1] += n != 0;
+    at[2] += h[j] != 0.0f;
+    if (exact) a.head[p.prefix + j] = static_cast<float>(at[0]);
+  }
+  if (tid == 1023)
+    for (int k = 0; k < 3; ++k) out[k][p.bins] = sums[k][1023];
+  if (tid == 0) {
+    a.exact[blockIdx.x] = exact;
+    if (!exact) {
+      float sum = 0.0f;
+      for (int j = 0; j < p.bins; ++j) a.head[p.prefix + j] = sum += h[j];
+    }
+  }
+}
+
+__device__ __forceinline__ int wave_sum(int v) {
+  for (int d = 1; d < 64; d *= 2) v += __shfl_xor(v, d);
+  return v;
+}
+
+// Correction of a smoothed distribution; false: all entries are zero, or so many that it reaches 1.
+__device__ __forceinline__ bool smoothing(int width, int nonzeros, float* take) {
+  if (nonzeros == 0) return false;
+  *take = kEps * static_cast<float>(width - nonzeros) / static_cast<float>(nonzeros);
+  return !(*take >= 1.0f);
+}
+
+// Levels, edge entries and smoothing of a candidate: a wave each, a level per lane.
+__global__ __launch_bounds__(256) void entropy_levels_kernel(Args a) {
+  const Problem p = a.p[blockIdx.y];
+  const int lane = threadIdx.x & 63, s = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (s >= p.candidates) return;
+  const int i = p.half + s, start = p.zero - i, stop = p.zero + i + 1;
+  const int width = stop - start, merged = width / p.levels, inner = start + 1;
+  const int* const counts = a.counts + p.prefix;
+  const int* const filled = a.filled + p.prefix;
+  const int* const seen = a.seen + p.prefix;
+  const float first = a.head[p.prefix + start];
+  float last;
+  if (a.exact[blockIdx.y]) {
+    last = static_cast<float>(counts[p.bins] - counts[stop - 1]);
+  } else {
+    const float* const h = a.hist + p.hist;
+    last = h[stop - 1];
+    for (int j = stop; j < p.bins; ++j) last += h[j];
+  }
+  auto between = [&](const int* sum, int lo, int hi) {
+    return lo < hi ? sum[hi] - sum[lo] : 0;
+  };
+  int p_entries = 0, q_entries = 0;
+  float* const levels = a.levels + p.level + static_cast<long long>(s) * p.levels;
+  for (int j = lane; j < p.levels; j += 64) {
+    const int lo = j * merged, end = j + 1 == p.levels ? width : lo + merged;
+    const int from = lo + start > inner ? lo + start : inner;
+    float level = static_cast<float>(between(counts, from, lo + merged + start));
+    if (j + 1 == p.levels) {
+      const int rest = lo + merged + start > inner ? lo + merged + start : inner;
+      level += static_cast<float>(between(counts, rest, stop));
+    }
+    const int nonempty = between(filled, from, end + start);
+    level = nonempty != 0 ? level / static_cast<float>(nonempty) : 0.0f;
+    levels[j] = level;
+    const int to = end + start < stop - 1 ? end + start : stop - 1;
+    const int entries = between(seen, from, to);
+    p_entries += entries;
+    if (level != 0.0f)
+      q_entries += entries + (j == 0 && first != 0.0f) + (j + 1 == p.levels && last != 0.0f);
+  }
+  p_entries = wave_sum(p_entries) + (first != 0.0f) + (last != 0.0f);
+  q_entries = wave_sum(q_entries);
+  if (lane == 0) {
+    Info r = {};
+    r.first = first;
+    r.last = last;
+    if (!smoothing(width, q_entries, &r.q_take))
+      r.state = 1;
+    else if (!smoothing(width, p_entries, &r.p_take))
+      r.state = 2;
+    a.info[p.candidate + s] = r;
+  }
+}
+
+// The two float chains of a candidate, a lane each, of two waves; the histogram in LDS.
+// Neighbouring candidates step through their bins side by side, one bin apart.  A chain's pace is
+// what one wave issues and what it waits for LDS: 195 us for the three histograms above (both
+// chains in one wave, 4 bins read at a time: 264).
+__global__ __launch_bounds__(128) void entropy_chains_kernel(Args a) {
+  extern __shared__ float hist[];
+  const Problem p = a.p[blockIdx.y];
+  if (static_cast<int>(blockIdx.x) * 64 >= p.candidates) return;
+  for (int j = threadIdx.x; j < p.bins; j += 128) hist[j] = a.hist[p.hist + j];
+  __syncthreads();
+  // the widest first: a wave of them takes longest
+  const int s = p.candidates - 1 - (blockIdx.x * 64 + (threadIdx.x & 63));
+  if (s < 0) return;
+  Info* const info = a.info + p.candidate + s;
+  if (info->state != 0) return;
+  const int i = p.half + s, width = 2 * i + 1, merged = width / p.levels;
+  const float* const h = hist + p.zero - i;
+  const float first = info->first, last = info->last;
+  float sum = 0.0f;
+  if (threadIdx.x < 64) {
+    const float take = info->p_take;
+    auto add = [&](float v) { sum += v != 0.0f ? v - take : kEps; };
+    add(first);
+    int o = 1;
+    for (; o + 16 < width; o += 16) {
+      float v[16];
+#pragma unroll
+      for (int k = 0; k < 16; ++k) v[k] = h[o + k];
+#pragma unroll
+      for (int k = 0; k < 16; ++k) add(v[k]);
+    }
+    for (; o + 1 < width; ++o) add(h[o]);
+    add(last);
+    info->p_sum = sum;
+    return;
+  }
+  const float take = info->q_take;
+  const float* const levels = a.levels + p.level + static_cast<long long>(s) * p.levels;
+  float level = levels[0];
+  auto smoothed = [&](float v) { return v != 0.0f ? v - take : kEps; };
+  auto add = [&](float v, float q) { sum += v != 0.0f ? q : kEps; };
+  add(first, smoothed(level));
+  for (int j = 0; j < p.levels; ++j) {
+    const float q = smoothed(level);
+    const bool end = j + 1 == p.levels;
+    if (!end) level = levels[j + 1];
+    const int to = end ? width - 1 : (j + 1) * merged;
+    int o = j == 0 ? 1 : j * merged;
+    for (; o + 8 <= to; o += 8) {
+      float v[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[k] = h[o + k];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) add(v[k], q);
+    }
+    if (o < to) {  // fewer than 8, read in one go as well
+      float v[7];
+#pragma unroll
+      for (int k = 0; k < 7; ++k) v[k] = h[o + k < to ? o + k : o];
+#pragma unroll
+      for (int k = 0; k < 7; ++k)
+        if (o + k < to) add(v[k], q);
+    }
+    if (end) add(last, q);
+  }
+  info->q_sum = sum;
+}
+
+// The bounds, a wave per candidate, 4 bins in a row per lane.  With u = 2^-24, a term of the float
+// chain carries a logarithm of at most a last place (2u) and a product's rounding, a term here a
+// logarithm of at most two (4u) and an exact product; a sum of the chain carries u of itself.
+// (135 us for the three histograms above; with logarithms in double and a bin per lane 314.)
+__global__ __launch_bounds__(256) void entropy_bounds_kernel(Args a) {
+  const Problem p = a.p[blockIdx.y];
+  const int lane = threadIdx.x & 63, s = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (s >= p.candidates) return;
+  double* const out = a.bounds + 2 * static_cast<long long>(p.candidate + s);
+  const Info r = a.info[p.candidate + s];
+  if (r.state != 0) {
+    if (lane < 2) out[lane] = r.state == 1 || lane == 1 ? INFINITY : -INFINITY;
+    return;
+  }
+  const int i = p.half + s, start = p.zero - i, width = 2 * i + 1, merged = width / p.levels;
+  const float* const h = a.hist + p.hist + start;
+  const float* const levels = a.levels + p.level + static_cast<long long>(s) * p.levels;
+  const float p_zero = kEps / r.p_sum, q_zero = kEps / r.q_sum;
+  const double zero_term = static_cast<double>(p_zero) * static_cast<double>(logf(p_zero / q_zero));
+  double sum = 0.0, magnitude = 0.0, sums = 0.0;  // the first the same in every lane
+  bool bad = false;
+  for (int base = 0; base < width; base += 256) {
+    const int from = base + 4 * lane;
+    int j = from / merged, rest = from - j * merged;
+    double t[4], all = 0.0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int o = from + k;
+      t[k] = 0.0;
+      if (o < width) {
+        const float v = o == 0 ? r.first : o + 1 == width ? r.last : h[o];
+        t[k] = zero_term;
+        if (v != 0.0f) {
+          const float level = levels[j < p.levels ? j : p.levels - 1];
+          const float q = level != 0.0f ? level - r.q_take : kEps;
+          const float pn = (v - r.p_take) / r.p_sum, qn = q / r.q_sum;
+          bad = bad || !(pn > 0.0f) || !(qn > 0.0f);
+          t[k] = static_cast<double>(pn) * static_cast<double>(logf(pn / qn));
+        }
+      }
+      magnitude += fabs(t[k]);
+      all += t[k];
+      if (++rest == merged) {
+        ++j;
+        rest = 0;
+      }
+    }
+    double before = all;
+    for (int d = 1; d < 64; d *= 2) {
+      const double other = __shfl_up(before, d);
+      before += lane >= d ? other : 0.0;
+    }
+    before += sum;
+    sum = __shfl(before, 63);
+    before -= all;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      before += t[k];
+      sums += from + k < width ? fabs(before) : 0.0;
+    }
+  }
+  for (int d = 1; d < 64; d *= 2) {
+    magnitude += __shfl_xor(magnitude, d);
+    sums += __shfl_xor(sums, d);
+  }
+  bad = __any(bad);
+  const double u = 1.0 / 16777216.0;
+  const double margin = 1.05 * u * (8 * magnitude + sums) + 1e-12;
+  if (lane == 0) {
+    const bool known = !bad && isfinite(sum) && isfinite(margin);
+    out[0] = known ? sum - margin : -INFINITY;
+    out[1] = known ? sum + margin : INFINITY;
+  }
+}
+
+size_t up256(size_t x) { return (x + 255) / 256 * 256; }
+
+// Where the parts of the workspace lie, and the problems' descriptions.
+struct Layout {
+  size_t prefix = 0, candidates = 0, levels = 0, hist = 0;  // elements
+  size_t bytes = 0, at[7];
+  Layout(int count, const int* bins, const int* num_levels, Problem* out) {
+    for (int i = 0; i < count; ++i) {
+      MXQ_CHECK(bins[i] % 2 == 1 && bins[i] <= kMaxBins && num_levels[i] >= 3 &&
+                    num_levels[i] <= bins[i],
+                "bins or levels out of range");
+      Problem p;
+      p.bins = bins[i];
+      p.levels = num_levels[i];
+      p.half = num_levels[i] / 2;
+      p.zero = bins[i] / 2;
+      p.candidates = p.zero + 1 - p.half;
+      p.hist = static_cast<int>(hist);
+      p.prefix = static_cast<int>(prefix);
+      p.candidate = static_cast<int>(candidates);
+      p.level = static_cast<long long>(levels);
+      hist += bins[i];
+      prefix += bins[i] + 1;
+      candidates += p.candidates;
+      levels += static_cast<size_t>(p.candidates) * p.levels;
+      if (out != nullptr) out[i] = p;
+    }
+    const size_t parts[7] = {prefix * 4, prefix * 4, prefix * 4, prefix * 4, kMaxProblems * 4,
+                             levels * 4, candidates * sizeof(Info)};
+    for (int k = 0; k < 7; ++k) {
+      at[k] = bytes;
+      bytes += up256(parts[k]);
+    }
+  }
+};
+
+}  // namespace
+}  // namespace mxq
+
+using namespace mxq;
+
+extern "C" {
+
+size_t mxq_entropy_bounds_workspace(int count, const int* bins, const int* levels) {
+  try {
+    if (count <= 0 || count > kMaxProblems || bins == nullptr || levels == nullptr) return 0;
+    return Layout(count, bins, levels, nullptr).bytes;
+  } catch (const std::exception& e) {
+    set_last_error(e.what());
+    return 0;
+  }
+}
+
+int mxq_entropy_bounds(void* stream, int count, const float* hist, const int* bins,
+                       const int* levels, double* bounds, void* workspace,
+                       size_t workspace_bytes) {
+  MXQ_API_BEGIN();
+  MXQ_CHECK(count >= 0 && count <= kMaxProblems, "too many histograms");
+  if (count == 0) return 0;
+  MXQ_CHECK(hist && bins && levels && bounds && workspace, "null pointer");
+  Args a;
+  const Layout l(count, bins, levels, a.p);
+  MXQ_CHECK(workspace_bytes >= l.bytes && (reinterpret_cast<uintptr_t>(workspace) & 15u) == 0,
+            "workspace too small or unaligned");
+  char* const ws = static_cast<char*>(workspace);
+  a.hist = hist;
+  a.counts = reinterpret_cast<int*>(ws + l.at[0]);
+  a.filled = reinterpret_cast<int*>(ws + l.at[1]);
+  a.seen = reinterpret_cast<int*>(ws + l.at[2]);
+  a.head = reinterpret_cast<float*>(ws + l.at[3]);
+  a.exact = reinterpret_cast<int*>(ws + l.at[4]);
+  a.levels = reinterpret_cast<float*>(ws + l.at[5]);
+  a.info = reinterpret_cast<Info*>(ws + l.at[6]);
+  a.bounds = bounds;
+  int most = 0, widest = 0;
+  for (int i = 0; i < count; ++i) {
+    most = a.p[i].candidates > most ? a.p[i].candidates : most;
+    widest = bins[i] > widest ? bins[i] : widest;
+  }
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const unsigned n = static_cast<unsigned>(count);
+  hipLaunchKernelGGL(entropy_prefix_kernel, dim3(n), dim3(1024), 0, s, a);
+  MXQ_LAUNCH_CHECK();
+  hipLaunchKernelGGL(entropy_levels_kernel, dim3((most + 3) / 4, n), dim3(256), 0, s, a);
+  MXQ_LAUNCH_CHECK();
+  hipLaunchKernelGGL(entropy_chains_kernel, dim3((most + 63) / 64, n), dim3(128),
+                     static_cast<size_t>(widest) * 4, s, a);
+  MXQ_LAUNCH_CHECK();
+  hipLaunchKernelGGL(entropy_bounds_kernel, dim3((most + 3) / 4, n), dim3(256), 0, s, a);
+  MXQ_LAUNCH_CHECK();
+  MXQ_API_END();
+}
+
+}  // extern "C"

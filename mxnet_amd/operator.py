@@ -67,6 +67,10 @@ OPS_SIGNATURES = {
     "mxq_calibrate_entropy_many": (_i, [_i, ctypes.POINTER(_p), ctypes.POINTER(_p),
                                         ctypes.POINTER(_sz), _pi, ctypes.POINTER(ctypes.c_float),
                                         ctypes.POINTER(ctypes.c_float)]),
+    "mxq_calibrate_entropy_bounded": (_i, [_i, ctypes.POINTER(_p), ctypes.POINTER(_p),
+                                           ctypes.POINTER(_sz), _pi, _p,
+                                           ctypes.POINTER(ctypes.c_float),
+                                           ctypes.POINTER(ctypes.c_float)]),
 }
 for _name, (_res, _args) in OPS_SIGNATURES.items():
     _fn = getattr(ops, _name)

@@ -168,6 +168,20 @@ def calibrate_entropy(hist, hist_edges, num_quantized_bins=255):
     return _calibrate_entropy_many([(hist, hist_edges, num_quantized_bins)])[0]
 
 
+def _entropy_bounds(hists, levels):
+    """Bounds of the candidates' divergences, taken on the GPU where one is in use already: 16 host
+    threads need ten times as long for them.  None: the search takes its own."""
+    if not hists or not torch.cuda.is_initialized() or torch.cuda.is_current_stream_capturing():
+        return None
+    for h, n in zip(hists, levels):
+        # what the kernels are made for: counts that int32 sums hold, a histogram that LDS holds
+        if h.ndim != 1 or h.size % 2 == 0 or h.size > 32767 or not 3 <= n <= h.size:
+            return None
+        if not (h.min() >= 0 and h.sum(dtype=np.float64) < 2 ** 31):  # neither for a NaN
+            return None
+    return capi.entropy_bounds(hists, levels)
+
+
 def _calibrate_entropy_many(problems):
     """[(threshold, divergence)] of (hist, hist_edges, num_quantized_bins) entries."""
     n = len(problems)
@@ -175,12 +189,17 @@ def _calibrate_entropy_many(problems):
     edges = [np.ascontiguousarray(p[1], dtype=np.float32) for p in problems]
     if any(e.size != h.size + 1 for h, e in zip(hists, edges)):
         raise ValueError("hist_edges needs one more entry than hist")
+    levels = [int(p[2]) for p in problems]
+    bounds = _entropy_bounds(hists, levels)
     th, div = (ctypes.c_float * n)(), (ctypes.c_float * n)()
-    _operator._check(_operator.ops.mxq_calibrate_entropy_many(
-        n, (ctypes.c_void_p * n)(*[h.ctypes.data for h in hists]),
-        (ctypes.c_void_p * n)(*[e.ctypes.data for e in edges]),
-        (ctypes.c_size_t * n)(*[h.size for h in hists]),
-        (ctypes.c_int * n)(*[int(p[2]) for p in problems]), th, div))
+    args = [n, (ctypes.c_void_p * n)(*[h.ctypes.data for h in hists]),
+            (ctypes.c_void_p * n)(*[e.ctypes.data for e in edges]),
+            (ctypes.c_size_t * n)(*[h.size for h in hists]), (ctypes.c_int * n)(*levels)]
+    if bounds is None:
+        _operator._check(_operator.ops.mxq_calibrate_entropy_many(*args, th, div))
+    else:
+        _operator._check(_operator.ops.mxq_calibrate_entropy_bounded(
+            *args, bounds.ctypes.data, th, div))
     return [(np.float32(t), np.float32(d)) for t, d in zip(th, div)]
 
 
