@@ -796,6 +796,130 @@ __global__ __launch_bounds__(kThreads) void relu_chunk_kernel(const int8_t* __re
   }
 }
 
+// ---- uncalibrated casts of small tensors ---------------------------------------------------
+// One work-group holds the whole tensor in registers: it takes the range, then casts what it
+// has, in one launch instead of a reduction and a cast: 16 instructions an element (fold and
+// conversion) on one CU's four SIMDs against the second launch and the hand-over of the partials.
+// In a chain of calls, fp32 -> int8, two launches / one, us: 100 elements 3.7 / 1.8, 1000 3.8 / 2.1,
+// 4096 4.4 / 2.8, 8192 4.3 / 3.4, 16384 4.6 / 4.0, 32768 4.5 / 5.8, 78540 4.6 / 11.8; on the host
+// one launch of 3 us less.  So up to 16384 elements.
+enum WholeKind { kWholeI8, kWholeU8, kWholeAsym, kWholeRequant };
+constexpr int kWholeThreads = 1024;
+constexpr int kWholePieces = 4;  // 16-byte pieces of a lane
+constexpr size_t kWholeMaxElements = size_t(kWholeThreads) * kWholePieces * 4;
+
+template <int KIND, int PIECES>
+__global__ __launch_bounds__(kWholeThreads) void whole_cast_kernel(
+    const void* __restrict__ in, uint8_t* __restrict__ out, float* __restrict__ omin,
+    float* __restrict__ omax, int n, const float* __restrict__ imin,
+    const float* __restrict__ imax) {
+  constexpr bool INT = KIND == kWholeRequant;
+  typedef std::conditional_t<INT, int, float> T;
+  typedef T Vec4 __attribute__((ext_vector_type(4)));
+  const T* const src = static_cast<const T*>(in);
+  const Vec4* const src4 = static_cast<const Vec4*>(in);
+  const int nquad = n >> 2, threads = blockDim.x, tid = threadIdx.x;
+  float in_scale = 0.0f;
+  if (INT) in_scale = maxabs(*imin, *imax) / 2147483648.0f;
+  Vec4 x[PIECES];
+  if (nquad != 0) {
+#pragma unroll
+    for (int j = 0; j < PIECES; ++j) {  // past the end: the last one again
+      const int q = j * threads + tid;
+      x[j] = src4[q < nquad ? q : nquad - 1];
+    }
+  }
+  const int tail = (nquad << 2) + tid;
+  const T last = src[tail < n ? tail : n - 1];
+
+  T mn = last, mx = last;
+  uint32_t amax = 0;
+  auto fold = [&](T v) {
+    if constexpr (INT) {
+      mn = v < mn ? v : mn;
+      mx = v > mx ? v : mx;
+    } else {
+      mn = fminf(mn, v);
+      mx = fmaxf(mx, v);
+      const uint32_t a = __builtin_bit_cast(uint32_t, v) & 0x7fffffffu;
+      amax = a > amax ? a : amax;
+    }
+  };
+  fold(last);
+  if (nquad != 0) {
+#pragma unroll
+    for (int j = 0; j < PIECES; ++j) {
+      fold(x[j].x);
+      fold(x[j].y);
+      fold(x[j].z);
+      fold(x[j].w);
+    }
+  }
+  // unsigned words in the order of the values, as the partials of the two-launch form
+  __shared__ uint32_t part[3][kWholeThreads / 64];
+  uint32_t low, high;
+  if constexpr (INT) {
+    low = static_cast<uint32_t>(wave_reduce(mn, MinI())) ^ 0x80000000u;
+    high = static_cast<uint32_t>(wave_reduce(mx, MaxI())) ^ 0x80000000u;
+  } else {
+    low = f2ord(wave_reduce(mn, MinF()));
+    high = f2ord(wave_reduce(mx, MaxF()));
+    amax = wave_reduce(amax, MaxU());
+  }
+  if ((tid & 63) == 0) {
+    part[0][tid >> 6] = low;
+    part[1][tid >> 6] = high;
+    part[2][tid >> 6] = amax;
+  }
+  __syncthreads();
+  for (int w = 0; w < threads / 64; ++w) {
+    low = part[0][w] < low ? part[0][w] : low;
+    high = part[1][w] > high ? part[1][w] : high;
+    amax = part[2][w] > amax ? part[2][w] : amax;
+  }
+
+  auto write = [&](auto rule) {
+    auto one = [&](T v) { return rule(INT ? to_float(v) * in_scale : to_float(v)); };
+    uint32_t* const out4 = reinterpret_cast<uint32_t*>(out);
+#pragma unroll
+    for (int j = 0; j < PIECES; ++j) {
+      const int q = j * threads + tid;
+      if (q < nquad) out4[q] = pack4(one(x[j].x), one(x[j].y), one(x[j].z), one(x[j].w));
+    }
+    if (tail < n) out[tail] = static_cast<uint8_t>(one(last));
+  };
+  float lo, hi, first, second;
+  if constexpr (INT) {
+    lo = static_cast<float>(static_cast<int>(low ^ 0x80000000u)) * in_scale;
+    hi = static_cast<float>(static_cast<int>(high ^ 0x80000000u)) * in_scale;
+  } else {
+    lo = ord2f(low);
+    hi = ord2f(high);
+    if (amax > 0x7f800000u) lo = hi = NAN;
+  }
+  if constexpr (KIND == kWholeI8) {
+    second = maxabs(lo, hi);
+    first = -second;
+    write(QuantI8{127.0f / second});
+  } else if constexpr (KIND == kWholeU8) {
+    first = lo;
+    second = hi;
+    write(QuantU8{lo, static_cast<float>((255.0 - 0.0) / static_cast<double>(hi - lo))});
+  } else if constexpr (KIND == kWholeAsym) {
+    first = 255.0f / (hi - lo);
+    second = 255.0f - hi * first;
+    write(QuantAsym{first, second});
+  } else {
+    second = maxabs(lo, hi);
+    first = -second;
+    write(QuantI8{127.0f / maxabs(first, second)});
+  }
+  if (tid == 0) {
+    *omin = first;
+    *omax = second;
+  }
+}
+
 // The partials of minmax_f32_kernel as two floats; both NaN where the tensor holds one.
 __global__ __launch_bounds__(kThreads) void minmax_result_kernel(
     const uint32_t* __restrict__ parts, int nparts, float* out_min, float* out_max) {
@@ -857,6 +981,28 @@ uint32_t* carve(void* workspace, size_t bytes) {
   return static_cast<uint32_t*>(workspace);
 }
 
+bool fits_whole(const void* in, const void* out, size_t n) {
+  return n <= kWholeMaxElements && aligned16(in) && (reinterpret_cast<uintptr_t>(out) & 3u) == 0;
+}
+
+template <int KIND>
+void launch_whole(hipStream_t s, const void* in, uint8_t* out, float* omin, float* omax, size_t n,
+                  const float* imin, const float* imax) {
+  const size_t quads = (n + 3) / 4;
+  const unsigned threads =
+      quads < kWholeThreads ? static_cast<unsigned>((quads + 63) / 64 * 64) : kWholeThreads;
+  const int count = static_cast<int>(n);
+#define MXQ_W(PIECES)                                                                             \
+  hipLaunchKernelGGL((whole_cast_kernel<KIND, PIECES>), dim3(1), dim3(threads), 0, s, in, out,   \
+                     omin, omax, count, imin, imax)
+  if (quads <= kWholeThreads)
+    MXQ_W(1);
+  else
+    MXQ_W(kWholePieces);
+#undef MXQ_W
+  MXQ_LAUNCH_CHECK();
+}
+
 void launch_quantize(hipStream_t s, const float* in, void* out, float* omin, float* omax,
                      size_t n, int out_type, float lo, float hi, const float* dlo,
                      const float* dhi, const uint32_t* parts, int nparts) {
@@ -905,6 +1051,14 @@ int mxq_quantize_v2(void* stream, const float* in, void* out, float* omin, float
   } else {
     if (n == 0) return 0;
     uint32_t* parts = carve(workspace, workspace_bytes);
+    if (fits_whole(in, out, n)) {
+      uint8_t* o = static_cast<uint8_t*>(out);
+      if (out_type == MXQ_UINT8)
+        launch_whole<kWholeU8>(s, in, o, omin, omax, n, nullptr, nullptr);
+      else
+        launch_whole<kWholeI8>(s, in, o, omin, omax, n, nullptr, nullptr);
+      return 0;
+    }
     const int grid = reduce_grid(n);
     if (aligned16(in))
       hipLaunchKernelGGL((minmax_f32_kernel<true>), dim3(grid), dim3(kThreads), 0, s, in, n,
@@ -998,6 +1152,10 @@ int mxq_quantize_asym(void* stream, const void* in, int in_type, uint8_t* out, f
   int nparts = 0;
   if (!calibrated) {
     uint32_t* ws = carve(workspace, workspace_bytes);
+    if (fits_whole(in, out, n)) {
+      launch_whole<kWholeAsym>(s, in, out, oscale, oshift, n, nullptr, nullptr);
+      return 0;
+    }
     nparts = reduce_grid(n);
     if (aligned16(in))
       hipLaunchKernelGGL((minmax_f32_kernel<true>), dim3(nparts), dim3(kThreads), 0, s, f, n, ws);
@@ -1065,6 +1223,10 @@ int mxq_requantize(void* stream, const int32_t* in, const float* imin, const flo
     real_range = (a < b) ? b : a;
   } else {
     uint32_t* ws = carve(workspace, workspace_bytes);
+    if (fits_whole(in, out, n)) {
+      launch_whole<kWholeRequant>(s, in, o, omin, omax, n, imin, imax);
+      return 0;
+    }
     nparts = reduce_grid(n);
     if (aligned16(in))
       hipLaunchKernelGGL((minmax_i32_kernel<true>), dim3(nparts), dim3(kThreads), 0, s, in, n,
