@@ -17,6 +17,7 @@
 #include "../../include/mxq.h"
 #include "mxq_common.h"
 #include "mxq_few_tiles.h"
+#include "mxq_resident.h"
 #include "mxq_thin_transpose.h"
 #include "mxq_gemm.h"
 #include "mxq_tiles.h"
@@ -1488,6 +1489,25 @@ void conv_nhwc(void* stream, const int8_t* data, const int8_t* weight, const int
   const long long data_bytes = static_cast<long long>(N) * H * W * C;
   const bool dma_ok = aligned && data_bytes < (1LL << 31) &&
                       static_cast<long long>(O) * a.K < (1LL << 31);
+  if (force.cfg == 0 && KH == 1 && KW == 1 && pad_h == 0 && pad_w == 0) {
+    ResidentArgs r = {};
+    r.data = data;
+    r.weight = weight;
+    r.M = a.M;
+    r.N = r.ldo = O;
+    r.K = C;
+    r.epi = e;
+    r.area = a.OH * a.OW;
+    r.OW = a.OW;
+    r.image = static_cast<long long>(H) * W * C;
+    r.down = stride_h * W * C;
+    r.right = stride_w * C;
+    r.images = N;
+    if (resident_wins(r, aligned && aligned16(out8))) {
+      launch_resident(s, r);
+      return;
+    }
+  }
   ConvPlan plan = plan_conv(g, aligned, force);
   // a split the chooser proposed is dropped when the caller brought no room for it
   if (force.splits == 0 && plan.splits > 1 &&

@@ -13,6 +13,7 @@
 #include "mxq_common.h"
 #include "mxq_fc_args.h"
 #include "mxq_few_tiles.h"
+#include "mxq_resident.h"
 #include "mxq_gemm.h"
 #include "mxq_tiles.h"
 
@@ -253,6 +254,20 @@ void launch_fc(hipStream_t s, const int8_t* data, const int8_t* weight, int M, i
       rest.ptr = d + copies;
       rest.bytes = ws.bytes - copies;
       launch_fc(s, d, w, M, N, Kp, ldo, epi, force, rest);
+      return;
+    }
+  }
+  if (force.cfg == 0) {
+    ResidentArgs r = {};
+    r.data = data;
+    r.weight = weight;
+    r.M = M;
+    r.N = N;
+    r.K = K;
+    r.ldo = ldo;
+    r.epi = a.epi;
+    if (resident_wins(r, aligned && fused8)) {
+      launch_resident(s, r);
       return;
     }
   }
