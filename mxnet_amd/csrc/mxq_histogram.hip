@@ -4,6 +4,7 @@
 // a copy to the host.
 #include <hip/hip_runtime.h>
 
+#include <cmath>
 #include <cstdint>
 
 #include "../../include/mxq.h"
@@ -13,7 +14,9 @@ namespace mxq {
 namespace {
 
 constexpr int kThreads = 512;
-// bins a work-group counts in LDS (64 KB); more are counted in memory directly
+constexpr int kCountThreads = 1024;
+constexpr int kValues = 8;  // of a lane in flight
+// bins a work-group counts in LDS (64 KB, and their edges); more are counted in memory directly
 constexpr int kMaxLdsBins = 16384;
 
 __global__ __launch_bounds__(kThreads) void zero_counts_kernel(uint32_t* counts, int bins) {
@@ -25,34 +28,66 @@ __global__ __launch_bounds__(kThreads) void zero_counts_kernel(uint32_t* counts,
 // edges[k] <= x < edges[k + 1], the last one its upper edge as well, values outside the edges
 // and NaN are left out (numpy corrects its own guess against the edges the same way, so the
 // counts agree with it exactly).
-// Bound by the LDS atomics and, at the end, one memory atomic per bin that a work-group filled:
-// hence few work-groups with many values each (393216 values in 8001 bins: 1.45 ms on the host,
-// copy included, 12 us here).
+// Bound by latency: a value's load, its edges, its atomic.  So the edges lie in LDS beside the
+// counts and a lane has eight values on their way; at the end there is one memory atomic per bin
+// that a work-group filled, hence few work-groups with many values each.  196608 values in 8001
+// bins 10 us; with the edges in memory and one value at a time 36, on the host 700.
 template <bool LDS>
-__global__ __launch_bounds__(kThreads) void histogram_kernel(const float* __restrict__ in,
-                                                             size_t n,
-                                                             const float* __restrict__ edges,
-                                                             int bins, uint32_t* counts) {
+__global__ __launch_bounds__(kCountThreads) void histogram_kernel(const float* __restrict__ in,
+                                                                  size_t n,
+                                                                  const float* __restrict__ edges,
+                                                                  int bins, uint32_t* counts) {
   extern __shared__ uint32_t local[];
+  float* const edge_lds = reinterpret_cast<float*>(local + bins);
+  const size_t stride = size_t(gridDim.x) * kCountThreads;
+  size_t at = size_t(blockIdx.x) * kCountThreads + threadIdx.x;
+  float x[kValues];
+  auto load = [&]() {
+#pragma unroll
+    for (int j = 0; j < kValues; ++j) {
+      const size_t i = at + j * stride;
+      x[j] = i < n ? in[i] : NAN;
+    }
+    at += kValues * stride;
+  };
+  load();
   if (LDS) {
-    for (int i = threadIdx.x; i < bins; i += kThreads) local[i] = 0;
+    for (int i = threadIdx.x; i <= bins; i += kCountThreads) {
+      if (i < bins) local[i] = 0;
+      edge_lds[i] = edges[i];
+    }
     __syncthreads();
   }
-  const float lo = edges[0], hi = edges[bins];
+  const float* const e = LDS ? edge_lds : edges;
+  const float lo = e[0], hi = e[bins];
   const float per_unit = static_cast<float>(bins) / (hi - lo);
-  const size_t stride = size_t(gridDim.x) * kThreads;
-  for (size_t i = size_t(blockIdx.x) * kThreads + threadIdx.x; i < n; i += stride) {
-    const float x = in[i];
-    if (!(x >= lo && x <= hi)) continue;
-    int k = static_cast<int>((x - lo) * per_unit);
-    k = k < 0 ? 0 : k > bins - 1 ? bins - 1 : k;
-    while (k > 0 && x < edges[k]) --k;
-    while (k < bins - 1 && x >= edges[k + 1]) ++k;
-    atomicAdd(LDS ? local + k : counts + k, 1u);
+  for (bool more = true; more;) {
+    int k[kValues];
+    float low[kValues], high[kValues];
+#pragma unroll
+    for (int j = 0; j < kValues; ++j) {
+      const int guess = static_cast<int>((x[j] - lo) * per_unit);
+      k[j] = guess < 0 ? 0 : guess > bins - 1 ? bins - 1 : guess;
+      low[j] = e[k[j]];
+      high[j] = e[k[j] + 1];
+    }
+#pragma unroll
+    for (int j = 0; j < kValues; ++j) {
+      const float v = x[j];
+      if (!(v >= lo && v <= hi)) continue;
+      int b = k[j];
+      if (v < low[j])
+        while (b > 0 && v < e[b]) --b;
+      else if (v >= high[j])
+        while (b < bins - 1 && v >= e[b + 1]) ++b;
+      atomicAdd(LDS ? local + b : counts + b, 1u);
+    }
+    more = at < n;
+    if (more) load();
   }
   if (LDS) {
     __syncthreads();
-    for (int i = threadIdx.x; i < bins; i += kThreads)
+    for (int i = threadIdx.x; i < bins; i += kCountThreads)
       if (local[i] != 0) atomicAdd(counts + i, local[i]);
   }
 }
@@ -75,16 +110,15 @@ extern "C" int mxq_histogram_f32(void* stream, const float* in, size_t n, const 
   if (n == 0) return 0;
   const bool lds = bins <= kMaxLdsBins;
   // twice as many values as bins per work-group, so that counting outweighs the final atomics
-  size_t grid = n / (lds ? 2 * static_cast<size_t>(bins) : kThreads) + 1;
-  const size_t cap = static_cast<size_t>(num_cus()) * 2;
+  size_t grid = n / (lds ? 2 * static_cast<size_t>(bins) : kCountThreads) + 1;
+  const size_t cap = static_cast<size_t>(num_cus()) * (bins <= kMaxLdsBins / 2 ? 2 : 1);
   if (grid > cap) grid = cap;
   if (lds)
-    hipLaunchKernelGGL((histogram_kernel<true>), dim3(static_cast<unsigned>(grid)), dim3(kThreads),
-                       static_cast<size_t>(bins) * sizeof(uint32_t), s, in, n, edges, bins,
-                       counts);
+    hipLaunchKernelGGL((histogram_kernel<true>), dim3(static_cast<unsigned>(grid)), dim3(kCountThreads), (2 * static_cast<size_t>(bins) + 1) * sizeof(uint32_t), s, in, n,
+                       edges, bins, counts);
   else
     hipLaunchKernelGGL((histogram_kernel<false>), dim3(static_cast<unsigned>(grid)),
-                       dim3(kThreads), 0, s, in, n, edges, bins, counts);
+                       dim3(kCountThreads), 0, s, in, n, edges, bins, counts);
   MXQ_LAUNCH_CHECK();
   MXQ_API_END();
 }
