@@ -388,6 +388,17 @@ int mxq_quantized_conv_nhwc_prepared(void* stream, const int8_t* data, const int
                                      float min_calib, float max_calib, void* workspace,
                                      size_t workspace_bytes);
 
+/* Two 1 x 1 convolutions of the same images, both prepared, in one launch (two where the operands
+ * are unaligned or _fits is 0). */
+int mxq_quantized_conv_pair_fits(int N, int H, int W, int C, int O1, int O2, int stride_h,
+                                 int stride_w);
+int mxq_quantized_conv_pair_prepared(void* stream, const int8_t* data, int N, int H, int W, int C,
+                                     int stride_h, int stride_w, const int8_t* weight1,
+                                     const void* prepared1, int O1, int8_t* out1, int relu1,
+                                     float min_calib1, float max_calib1, const int8_t* weight2,
+                                     const void* prepared2, int O2, int8_t* out2, int relu2,
+                                     float min_calib2, float max_calib2);
+
 /* Looks for a short form of that sum with sum_relu != 0 over ranges that stay: two products and
  * one rounding that give the same int8 for every pair of int8 operands, which is tried out on
  * the device.  Writes 12 bytes to `pairs` (device, 4-byte aligned), among them whether one was

@@ -73,6 +73,9 @@ SIGNATURES = {
     "mxq_quantized_fc_prepared": (_i, [_p] * 4 + [_i] * 3 + [_p, _p, _i, _f, _f, _p, _sz]),
     "mxq_quantized_fc_sum_prepared": (_i, [_p] * 4 + [_i] * 3 + [_p] * 4 + [_f] * 4 +
                                       [_i, _i, _p, _p, _sz]),
+    "mxq_quantized_conv_pair_fits": (_i, [_i] * 8),
+    "mxq_quantized_conv_pair_prepared": (_i, [_p] * 2 + [_i] * 6 +
+                                         [_p, _p, _i, _p, _i, _f, _f] * 2),
     "mxq_quantized_conv_nhwc_prepared": (_i, [_p] * 4 + [_i] * 13 +
                                          [_p, _i, _f, _f, _p, _sz]),
     "mxq_sum_requant_pairs": (_i, [_p, _f, _f, _f, _f, _f, _f, _p]),

@@ -30,7 +30,7 @@ _FLAG_OF = {torch.float32: 0, torch.float64: 1, torch.float16: 2, torch.uint8: 3
 _SIZE_OF = {0: 4, 1: 8, 2: 2, 3: 1, 4: 4, 5: 1, 6: 8, 7: 1, 12: 2}
 _FLOAT32, _INT32, _INT8 = 0, 4, 5
 (_NODE, _CONV, _FC, _FC_F32, _FC_SUM, _FC_SUM_RQ, _QUANT_NHWC, _TO_NHWC, _FROM_NHWC, _POOL, _RELU,
- _ADD, _REQUANTIZE, _BLOCK) = range(14)
+ _ADD, _REQUANTIZE, _BLOCK, _PAIR) = range(15)
 _NULL, _ARENA, _HELD, _FEED, _OUTPUT = range(5)
 
 
@@ -682,6 +682,7 @@ class _Builder:
             v.at.place = (_OUTPUT, len(outputs), 0)
             outputs.append((v.flag, v.shape))
         self.fuse_blocks()
+        self.pair_convs()
         # offsets: first fit over the buffers alive at the same steps
         taken, size = [], 0
         for b in sorted((b for b in self.buffers if b.place is None and b.first is not None),
@@ -721,6 +722,10 @@ class _Builder:
                 places[3:6] = [self.prepared(*layer) if layer[2] else (_NULL, 0, 0)
                                for layer in layers]
                 places[2] = self.block_forms(floats, layers, places[3:6])
+            if kind == _PAIR:
+                layers, blobs = blobs, None
+                places[5:7] = [self.prepared(columns, calib, [place(r) for r in refs])
+                               for columns, calib, refs in layers]
             if kind in (_CONV, _FC, _FC_F32, _FC_SUM, _FC_SUM_RQ):
                 places.append(self.prepared(ints[4 if kind == _CONV else 1], floats, places))
             step = (kind, tuple(int(v) for v in ints), tuple(float(v) for v in floats),
@@ -771,16 +776,42 @@ class _Builder:
             self.steps[at] = (_BLOCK, shape + (layers[2][0], self.steps[first][1][13], relu),
                               floats, [conv[0], None, None, None, None, None, refs[12],
                                        refs[10], out], None, layers)
-        if gone:
-            self.steps = [s for at, s in enumerate(self.steps) if at not in gone]
-            for b in self.buffers:
-                b.first = b.last = None
-            for at, step in enumerate(self.steps):
-                for r in step[3]:
-                    b = r.buffer if isinstance(r, _Offset) else r
-                    if isinstance(b, _Buffer):
-                        b.first = at if b.first is None else b.first
-                        b.last = at
+        self.drop(gone)
+
+    def pair_convs(self):
+        """Two 1 x 1 convolutions of the same tensor as one step, at the place of the first."""
+        gone = set()
+        for at, (kind, geo, calib, refs, _, _) in enumerate(self.steps):
+            if (kind != _CONV or at in gone or geo[5:7] != (1, 1) or geo[9:11] != (0, 0) or
+                    not self.stays(refs)):
+                continue
+            for j in range(at + 1, len(self.steps)):
+                other, geo2, calib2, refs2, _, _ = self.steps[j]
+                if (other == _CONV and j not in gone and refs2[0] is refs[0] and
+                        geo2[:4] + geo2[5:13] == geo[:4] + geo[5:13] and self.stays(refs2) and
+                        _lib.lib.mxq_quantized_conv_pair_fits(*geo[:5], geo2[4], *geo[7:9])):
+                    self.steps[at] = (
+                        _PAIR, geo[:5] + (geo2[4],) + geo[7:9] + (geo[13], geo2[13]),
+                        tuple(calib) + tuple(calib2),
+                        [refs[0], refs[1], refs2[1], refs[10], refs2[10], None, None], None,
+                        [(geo[4], calib, refs), (geo2[4], calib2, refs2)])
+                    gone.add(j)
+                    break
+        self.drop(gone)
+
+    def drop(self, gone):
+        """Leaves the steps `gone` out; the buffers' lifetimes follow."""
+        if not gone:
+            return
+        self.steps = [s for at, s in enumerate(self.steps) if at not in gone]
+        for b in self.buffers:
+            b.first = b.last = None
+        for at, step in enumerate(self.steps):
+            for r in step[3]:
+                b = r.buffer if isinstance(r, _Offset) else r
+                if isinstance(b, _Buffer):
+                    b.first = at if b.first is None else b.first
+                    b.last = at
 
     @staticmethod
     def stays(refs):

@@ -129,6 +129,11 @@ bool Plan::run(void* stream, const std::vector<at::Tensor>& feeds,
         rc = mxq_quantized_block(stream, q(0), q(1), p(2), p(3), p(4), p(5), i(0), i(1), i(2),
                                  i(3), i(4), i(5), i(6), q(6), q(7), q(8), i(7), i(8));
         break;
+      case Kind::kConvPair:  // refs: data, both weights, outputs, what mxq_prepare_layer made
+        rc = mxq_quantized_conv_pair_prepared(stream, q(0), i(0), i(1), i(2), i(3), i(6), i(7),
+                                              q(1), p(5), i(4), q(3), i(8), f[0], f[1], q(2), p(6),
+                                              i(5), q(4), i(9), f[2], f[3]);
+        break;
       case Kind::kRequantize:
         rc = mxq_requantize(stream, static_cast<int32_t*>(p(0)), v(2), v(3), q(1), v(4), v(4) + 1,
                             static_cast<size_t>(n[0]), 1, f[0], f[1], nullptr, 0);

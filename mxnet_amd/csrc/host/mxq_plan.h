@@ -43,6 +43,7 @@ enum class Kind : int {
   kAdd,          // int8 sum, int32 or calibrated int8
   kRequantize,   // calibrated
   kBlock,        // 3 x 3 convolution -> 1 x 1 -> sum (-> 1 x 1), each requantized
+  kConvPair,     // two 1 x 1 convolutions of one tensor, each requantized (-> relu)
 };
 
 struct Step {

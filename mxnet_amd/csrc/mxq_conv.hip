@@ -207,14 +207,14 @@ struct ConvIssuer {
 };
 
 template <class Cfg, int NS, int PIPE>
-__global__ __launch_bounds__(Cfg::kThreads, NS <= 2 ? Cfg::kMinWaves : 1) void conv_dma_kernel(ConvArgs p) {
+__device__ __forceinline__ void conv_dma(const ConvArgs& p, int block) {
   __shared__ __attribute__((aligned(16))) v4i lds[NS * Cfg::STAGE_SLOTS];
   const int tiles_m = (p.M + Cfg::BM - 1) / Cfg::BM, tiles_n = (p.O + Cfg::BN - 1) / Cfg::BN;
   int tm, tn, tile = 0, z = 0;
   if (__builtin_expect(p.sk.splits > 1, 0))
-    tile_coords_split(blockIdx.x, tiles_m, tiles_n, p.sk.splits, tm, tn, tile, z);
+    tile_coords_split(block, tiles_m, tiles_n, p.sk.splits, tm, tn, tile, z);
   else
-    tile_coords(blockIdx.x, tiles_m, tiles_n, tm, tn);
+    tile_coords(block, tiles_m, tiles_n, tm, tn);
   const int m0 = tm * Cfg::BM, n0 = tn * Cfg::BN;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -235,11 +235,29 @@ __global__ __launch_bounds__(Cfg::kThreads, NS <= 2 ? Cfg::kMinWaves : 1) void c
   v16i acc[Cfg::MI][Cfg::NI];
   gemm_mainloop_dma<Cfg, NS, PIPE>(acc, ai, bi, KT, lds, prefetch);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  if (blockIdx.x == 0 && threadIdx.x == 0) epilogue_ranges(p.epi);
+  if (block == 0 && threadIdx.x == 0) epilogue_ranges(p.epi);
   if (__builtin_expect(p.sk.splits > 1, 0) && !splitk_gather<Cfg>(acc, p.sk, tile, z)) return;
 
   gemm_epilogue_lds<Cfg, NS * Cfg::STAGE_SLOTS * 16>(acc, p.epi, pre, m0, n0, p.M, p.O,
                                                      static_cast<size_t>(p.O), lds);
+}
+
+template <class Cfg, int NS, int PIPE>
+__global__ __launch_bounds__(Cfg::kThreads, NS <= 2 ? Cfg::kMinWaves : 1) void conv_dma_kernel(ConvArgs p) {
+  conv_dma<Cfg, NS, PIPE>(p, blockIdx.x);
+}
+
+// Two convolutions of the same images in one launch.
+struct ConvPair {
+  ConvArgs a, b;
+  int first;  // work-groups of a
+};
+template <class Cfg, int NS>
+__global__ __launch_bounds__(Cfg::kThreads, Cfg::kMinWaves) void conv_pair_kernel(ConvPair p) {
+  const bool second = static_cast<int>(blockIdx.x) >= p.first;
+  ConvArgs a = p.a;
+  if (second) a = p.b;
+  conv_dma<Cfg, NS, 0>(a, static_cast<int>(blockIdx.x) - (second ? p.first : 0));
 }
 
 // ---- 3 x 3 convolution over 64 channels with the weights parked in LDS --------------
@@ -898,6 +916,17 @@ void launch_dma(hipStream_t s, ConvArgs a, int splits, const Workspace& ws) {
   hipLaunchKernelGGL((conv_dma_kernel<Cfg, NS, PIPE>),
                      dim3(static_cast<unsigned>(tiles * a.sk.splits)), dim3(Cfg::kThreads), 0, s,
                      a);
+  MXQ_LAUNCH_CHECK();
+}
+
+template <class Cfg>
+void launch_pair(hipStream_t s, const ConvArgs& a, const ConvArgs& b) {
+  auto tiles = [](const ConvArgs& x) {
+    return static_cast<long>((x.M + Cfg::BM - 1) / Cfg::BM) * ((x.O + Cfg::BN - 1) / Cfg::BN);
+  };
+  const ConvPair p = {a, b, static_cast<int>(tiles(a))};
+  hipLaunchKernelGGL((conv_pair_kernel<Cfg, 2>), dim3(static_cast<unsigned>(tiles(a) + tiles(b))),
+                     dim3(Cfg::kThreads), 0, s, p);
   MXQ_LAUNCH_CHECK();
 }
 
@@ -1588,6 +1617,132 @@ void conv_nhwc(void* stream, const int8_t* data, const int8_t* weight, const int
 
 }  // namespace
 
+namespace {
+
+struct PairLayer {
+  const int8_t* weight;
+  const void* prepared;
+  int O;
+  int8_t* out8;
+  int relu;
+  float min_calib, max_calib;
+};
+
+enum class PairRoute { kNone, kResident, kFewTiles, kTiles64, kTiles64Deep, kTiles128 };
+
+// How two 1 x 1 convolutions of the same images go out as one launch, and whether that is faster
+// than two.
+PairRoute pair_route(const ConvGeometry& g, int O1, int O2) {
+  const long long M = g.M, data = static_cast<long long>(g.N) * g.H * g.W * g.C;
+  const int O = O1 + O2;
+  if (g.M == 0 || O1 % 16 != 0 || O2 % 16 != 0 || g.C % 16 != 0 || data >= (1LL << 31) ||
+      static_cast<long long>(O) * g.C >= (1LL << 31))
+    return PairRoute::kNone;
+  const long cus = num_cus();
+  ResidentArgs a = {}, b;
+  a.M = static_cast<int>(M);
+  a.K = g.C;
+  a.epi.out8 = reinterpret_cast<int8_t*>(16);  // only whether there is one counts
+  a.area = g.OH * g.OW;
+  a.OW = g.OW;
+  a.image = static_cast<long long>(g.H) * g.W * g.C;
+  b = a;
+  a.N = a.ldo = O1;
+  b.N = b.ldo = O2;
+  if (resident_pair_wins(a, b, true)) return PairRoute::kResident;
+  const long few = few_tiles_count(M, O1) + few_tiles_count(M, O2);
+  if (g.C >= 256 && 4 * few <= 5 * cus && few_tiles_conv_ok(g.C, g.C, 1, 1))
+    return PairRoute::kFewTiles;
+  auto tiles = [&](long bm, long bn) {
+    return (M + bm - 1) / bm * ((O1 + bn - 1) / bn + (O2 + bn - 1) / bn);
+  };
+  if (tiles(64, 64) <= 4 * cus) return g.C >= 1024 ? PairRoute::kTiles64Deep : PairRoute::kTiles64;
+  if (g.C >= 1024 && tiles(128, 128) <= 2 * cus) return PairRoute::kTiles128;
+  return PairRoute::kNone;
+}
+
+void conv_pair(void* stream, const int8_t* data, int N, int H, int W, int C, int stride_h,
+               int stride_w, const PairLayer& x, const PairLayer& y) {
+  MXQ_CHECK(x.prepared && aligned16(x.prepared) && y.prepared && aligned16(y.prepared),
+            "null or unaligned pointer");
+  const ConvGeometry g =
+      conv_geometry(N, H, W, C, x.O, 1, 1, stride_h, stride_w, 0, 0, 1, 1);
+  MXQ_CHECK(y.O > 0, "bad shape");
+  MXQ_CHECK(g.M == 0 || (data && x.weight && y.weight), "null operand pointer");
+  MXQ_CHECK(g.M == 0 || (x.out8 && y.out8), "no output buffer");
+  const bool aligned = aligned16(data) && aligned16(x.weight) && aligned16(y.weight) &&
+                       aligned16(x.out8) && aligned16(y.out8);
+  const PairRoute route = aligned ? pair_route(g, x.O, y.O) : PairRoute::kNone;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  auto epilogue = [&](const PairLayer& l) {
+    Epilogue e = {};
+    e.out8 = l.out8;
+    e.prepared = static_cast<const char*>(l.prepared);
+    e.relu = l.relu;
+    const float lo = fabsf(l.min_calib), hi = fabsf(l.max_calib);
+    e.real_range = (lo < hi) ? hi : lo;
+    e.stream8 = epi_stream_rows(g.M);
+    return e;
+  };
+  const int M = static_cast<int>(g.M);
+  if (route == PairRoute::kNone) {
+    for (const PairLayer* l : {&x, &y})
+      conv_nhwc(stream, data, l->weight, nullptr, N, H, W, C, l->O, 1, 1, stride_h, stride_w, 0, 0,
+                1, 1, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr,
+                nullptr, l->out8, nullptr, nullptr, l->relu, l->min_calib, l->max_calib, false,
+                GemmForce(), Workspace(), l->prepared);
+  } else if (route == PairRoute::kResident) {
+    ResidentArgs r[2] = {};
+    for (int i = 0; i < 2; ++i) {
+      const PairLayer& l = i == 0 ? x : y;
+      r[i].data = data;
+      r[i].weight = l.weight;
+      r[i].M = M;
+      r[i].N = r[i].ldo = l.O;
+      r[i].K = C;
+      r[i].epi = epilogue(l);
+      if (!g.is_fc) {
+        r[i].area = g.OH * g.OW;
+        r[i].OW = g.OW;
+        r[i].image = static_cast<long long>(H) * W * C;
+        r[i].down = stride_h * W * C;
+        r[i].right = stride_w * C;
+        r[i].images = N;
+      }
+    }
+    launch_resident_pair(s, r[0], r[1]);
+  } else if (route == PairRoute::kFewTiles) {
+    FewTilesArgs f[2] = {};
+    for (int i = 0; i < 2; ++i) {
+      const PairLayer& l = i == 0 ? x : y;
+      f[i].data = data; f[i].weight = l.weight; f[i].M = M; f[i].N = f[i].ldo = l.O; f[i].K = C;
+      f[i].epi = epilogue(l);
+      f[i].images = N; f[i].H = H; f[i].W = W; f[i].C = C; f[i].KW = 1;
+      f[i].sh = stride_h; f[i].sw = stride_w; f[i].dh = f[i].dw = 1;
+      f[i].OH = g.OH; f[i].OW = g.OW;
+    }
+    const int waves = few_tiles_waves(M, x.O + y.O, C, true);
+    launch_few_tiles_pair(s, f[0], f[1], waves == 16 ? 8 : waves);
+  } else {
+    ConvArgs a[2] = {};
+    for (int i = 0; i < 2; ++i) {
+      const PairLayer& l = i == 0 ? x : y;
+      a[i].data = data; a[i].weight = l.weight;
+      a[i].N = N; a[i].H = H; a[i].W = W; a[i].C = C; a[i].O = l.O; a[i].KH = a[i].KW = 1;
+      a[i].sh = stride_h; a[i].sw = stride_w; a[i].dh = a[i].dw = 1;
+      a[i].OH = g.OH; a[i].OW = g.OW; a[i].M = M; a[i].K = C;
+      a[i].epi = epilogue(l);
+      a[i].sk.splits = 1;
+      a[i].sk.kt_per_split = 1 << 30;
+    }
+    if (route == PairRoute::kTiles128) launch_pair<CfgMK>(s, a[0], a[1]);
+    else if (route == PairRoute::kTiles64Deep) launch_pair<CfgSK2>(s, a[0], a[1]);
+    else launch_pair<CfgS>(s, a[0], a[1]);
+  }
+}
+
+}  // namespace
+
 // Data [N][C][H][W] -> [N][H][W][Cp] and weights [O][C][KH][KW] -> [O][KH][KW][Cp] for the
 // NCHW operator's adapter route, in one launch where the data's kernel can carry the weights.
 void nchw_to_nhwc_pair(hipStream_t s, const int8_t* data, int8_t* d_out, int N, int C, int H,
@@ -1647,6 +1802,29 @@ int mxq_quantized_conv_nhwc_prepared(void* stream, const int8_t* data, const int
             dilate_h, dilate_w, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr,
             nullptr, nullptr, out8, nullptr, nullptr, relu, min_calib, max_calib, false,
             GemmForce(), ws, prepared);
+  MXQ_API_END();
+}
+
+int mxq_quantized_conv_pair_fits(int N, int H, int W, int C, int O1, int O2, int stride_h,
+                                 int stride_w) {
+  try {
+    return pair_route(conv_geometry(N, H, W, C, O1, 1, 1, stride_h, stride_w, 0, 0, 1, 1), O1, O2) !=
+           PairRoute::kNone;
+  } catch (...) {
+    return 0;
+  }
+}
+
+int mxq_quantized_conv_pair_prepared(void* stream, const int8_t* data, int N, int H, int W, int C,
+                                     int stride_h, int stride_w, const int8_t* weight1,
+                                     const void* prepared1, int O1, int8_t* out1, int relu1,
+                                     float min_calib1, float max_calib1, const int8_t* weight2,
+                                     const void* prepared2, int O2, int8_t* out2, int relu2,
+                                     float min_calib2, float max_calib2) {
+  MXQ_API_BEGIN();
+  conv_pair(stream, data, N, H, W, C, stride_h, stride_w,
+            {weight1, prepared1, O1, out1, relu1, min_calib1, max_calib1},
+            {weight2, prepared2, O2, out2, relu2, min_calib2, max_calib2});
   MXQ_API_END();
 }
 

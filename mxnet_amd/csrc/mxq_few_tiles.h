@@ -41,6 +41,8 @@ void launch_few_tiles_fc(hipStream_t s, const FewTilesArgs& a, bool aligned, int
 // Extents the convolution's loader can index; the operands are 16-byte aligned and below 2 GiB.
 bool few_tiles_conv_ok(int C, int K, int KH, int KW);
 void launch_few_tiles_conv(hipStream_t s, FewTilesArgs a, int waves);
+// Two of them of the same images in one launch.
+void launch_few_tiles_pair(hipStream_t s, const FewTilesArgs& a, const FewTilesArgs& b, int waves);
 
 // Copies of two operands with their rows of K bytes padded to Kp (a multiple of 16) with zeros:
 // what brings an operand of any width to the kernels that need aligned rows.

@@ -125,14 +125,14 @@ enum Operands { kAligned, kAny, kConv };
 
 // T: rows and columns of an output tile, 32 or 16
 template <int W, int T, int OPERANDS, int MODE>
-__global__ __launch_bounds__(64 * W) void few_tiles_kernel(FewTilesArgs p) {
+__device__ __forceinline__ void few_tiles(const FewTilesArgs& p, int block) {
   constexpr int kDepth = depth_of(W, T), kTile = T, F = T / 16;
   constexpr int kPitch = T + 4;  // ints per row of a partial tile in LDS
   __shared__ __attribute__((aligned(16))) int part[W][kTile * kPitch];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int tiles_n = (p.N + kTile - 1) / kTile;
-  const int tm = blockIdx.x / tiles_n, tn = blockIdx.x - tm * tiles_n;
+  const int tm = block / tiles_n, tn = block - tm * tiles_n;
   const int m0 = tm * kTile, n0 = tn * kTile;
   // how a lane loads (row, 16-byte piece of the row's 64) and what it multiplies
   const int load_row = lane >> 2, load_piece = lane & 3;
@@ -236,7 +236,7 @@ __global__ __launch_bounds__(64 * W) void few_tiles_kernel(FewTilesArgs p) {
           acc[i][j];
   __syncthreads();
 
-  if (blockIdx.x == 0 && tid == 0) epilogue_ranges<MODE>(p.epi);
+  if (block == 0 && tid == 0) epilogue_ranges<MODE>(p.epi);
 #pragma unroll
   for (int j = 0; j < kPer; ++j) {
     const int q = tid + j * kThreads;
@@ -256,6 +256,24 @@ __global__ __launch_bounds__(64 * W) void few_tiles_kernel(FewTilesArgs p) {
     epi_store_quad<MODE>(p.epi, pre, v, m, n, p.N, static_cast<size_t>(p.ldo),
                          epi_sums(MODE) ? residual[j] : 0);
   }
+}
+
+template <int W, int T, int OPERANDS, int MODE>
+__global__ __launch_bounds__(64 * W) void few_tiles_kernel(FewTilesArgs p) {
+  few_tiles<W, T, OPERANDS, MODE>(p, blockIdx.x);
+}
+
+// Two convolutions of the same images in one launch.
+struct FewTilesPair {
+  FewTilesArgs a, b;
+  int first;  // work-groups of a
+};
+template <int W, int T>
+__global__ __launch_bounds__(64 * W) void few_tiles_pair_kernel(FewTilesPair p) {
+  const bool second = static_cast<int>(blockIdx.x) >= p.first;
+  FewTilesArgs a = p.a;
+  if (second) a = p.b;
+  few_tiles<W, T, kConv, kEpiPlain>(a, static_cast<int>(blockIdx.x) - (second ? p.first : 0));
 }
 
 // Rows of K bytes -> rows of Kp >= K bytes on 16-byte marks, zeros behind: two tensors in one
@@ -369,13 +387,37 @@ bool few_tiles_conv_ok(int C, int K, int KH, int KW) {
          static_cast<long long>(KH) * KW * KW < (1LL << 32);
 }
 
-void launch_few_tiles_conv(hipStream_t s, FewTilesArgs a, int waves) {
+static void conv_magics(FewTilesArgs& a) {
   auto magic = [](int d) {
     return d == 1 ? 0u : static_cast<uint32_t>((1ULL << 32) / static_cast<unsigned>(d) + 1);
   };
   a.magic_c = magic(a.C / 16);
   a.magic_kw = magic(a.KW);
+}
+
+void launch_few_tiles_conv(hipStream_t s, FewTilesArgs a, int waves) {
+  conv_magics(a);
   launch<kConv, kEpiPlain>(s, a, waves);
+}
+
+void launch_few_tiles_pair(hipStream_t s, const FewTilesArgs& a, const FewTilesArgs& b, int waves) {
+  FewTilesPair p = {a, b, 0};
+  conv_magics(p.a);
+  conv_magics(p.b);
+  const long side = waves == -4 || waves == -8 ? 16 : 32;
+  auto tiles = [&](const FewTilesArgs& x) {
+    return static_cast<int>((x.M + side - 1) / side * ((x.N + side - 1) / side));
+  };
+  p.first = tiles(a);
+  const dim3 grid(static_cast<unsigned>(p.first + tiles(b)));
+  switch (waves) {
+    case -4: hipLaunchKernelGGL((few_tiles_pair_kernel<4, 16>), grid, dim3(256), 0, s, p); break;
+    case -8: hipLaunchKernelGGL((few_tiles_pair_kernel<8, 16>), grid, dim3(512), 0, s, p); break;
+    case 2: hipLaunchKernelGGL((few_tiles_pair_kernel<2, 32>), grid, dim3(128), 0, s, p); break;
+    case 4: hipLaunchKernelGGL((few_tiles_pair_kernel<4, 32>), grid, dim3(256), 0, s, p); break;
+    default: hipLaunchKernelGGL((few_tiles_pair_kernel<8, 32>), grid, dim3(512), 0, s, p);
+  }
+  MXQ_LAUNCH_CHECK();
 }
 
 }  // namespace mxq

@@ -28,6 +28,9 @@ struct ResidentArgs {
 // and output.
 bool resident_wins(const ResidentArgs& a, bool aligned);
 void launch_resident(hipStream_t s, const ResidentArgs& a);
+// Two layers over the same rows in one launch.
+bool resident_pair_wins(const ResidentArgs& a, const ResidentArgs& b, bool aligned);
+void launch_resident_pair(hipStream_t s, const ResidentArgs& a, const ResidentArgs& b);
 
 }  // namespace mxq
 #endif  // MXQ_RESIDENT_H_

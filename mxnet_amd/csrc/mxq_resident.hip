@@ -54,14 +54,13 @@ constexpr int kRing = 8192;  // bytes in LDS through which a wave's weights come
 // 4 waves, WN of them side by side, each on 32 rows and NI times 32 columns of a tile; NS tiles of
 // operand rows in LDS, two work-groups per CU.
 template <int KS, int WN, int NI, int NS, bool GATHER>
-__global__ __launch_bounds__(256, 2) void resident_kernel(Args args) {
+__device__ __forceinline__ void resident(const Args& args, const ResidentArgs& p, int group) {
   constexpr int NW = 4, THREADS = 64 * NW, WM = NW / WN, TM = 32 * WM, TN = 32 * NI, NC = WN * TN;
   constexpr int K = 32 * KS, CH = 2 * KS;
   constexpr int D = TM * CH / THREADS;           // DMA instructions of a wave and tile
   constexpr int S = TM * NC / 16 / THREADS;      // stores of a lane and tile
   constexpr int LD = NC + 16, PIECES = NC / 16;
   static_assert(D >= 1 && S >= 1, "tile too small");
-  const ResidentArgs& p = args.r;
   static_assert(2 * TM * LD + NC * 4 <= NW * kRing, "the rings' place is too small");
   static_assert(NS * TM * CH * 16 + NW * kRing <= 80 * 1024, "LDS of two work-groups");
   __shared__ __attribute__((aligned(16))) v4i rows[NS * TM * CH];
@@ -72,7 +71,7 @@ __global__ __launch_bounds__(256, 2) void resident_kernel(Args args) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WN, wn = wave % WN, lrow = lane & 31, lgrp = lane >> 5;
-  const int n0 = blockIdx.y * NC;
+  const int n0 = group * NC;
   const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(rows));
   auto swizzle = [](int r) { return r & 15; };
 
@@ -247,33 +246,70 @@ __global__ __launch_bounds__(256, 2) void resident_kernel(Args args) {
     if (p.epi.relu) run(std::false_type(), std::true_type());
     else run(std::false_type(), std::false_type());
   }
-  if (blockIdx.x == 0 && blockIdx.y == 0 && tid == 0) epilogue_ranges<kEpiPlain>(p.epi);
+  if (blockIdx.x == 0 && group == 0 && tid == 0) epilogue_ranges<kEpiPlain>(p.epi);
+}
+
+template <int KS, int WN, int NI, int NS, bool GATHER>
+__global__ __launch_bounds__(256, 2) void resident_kernel(Args args) {
+  resident<KS, WN, NI, NS, GATHER>(args, args.r, blockIdx.y);
+}
+
+// Two layers over the same rows.
+struct PairArgs {
+  Args a;
+  ResidentArgs b;
+  int first;  // column groups of the first
+};
+template <int KS, int NS, bool GATHER>
+__global__ __launch_bounds__(256, 2) void resident_pair_kernel(PairArgs args) {
+  const bool second = static_cast<int>(blockIdx.y) >= args.first;
+  ResidentArgs r = args.a.r;
+  if (second) r = args.b;
+  resident<KS, 4, 2, NS, GATHER>(args.a, r, static_cast<int>(blockIdx.y) - (second ? args.first : 0));
+}
+
+// Work-groups along the rows, and how a tile's images follow the one before.
+int row_groups(Args& a, int tile, int column_groups) {
+  const ResidentArgs& r = a.r;
+  const int tiles = (r.M + tile - 1) / tile;
+  int gx = 2 * num_cus() / column_groups;
+  if (gx > 8) gx = gx / 8 * 8;  // column groups of the same rows on the same XCD
+  if (gx < 1) gx = 1;
+  if (gx > tiles) gx = tiles;
+  if (r.area != 0) {
+    const long long step = static_cast<long long>(gx) * tile;
+    a.magic_area = magic_of(r.area);
+    a.magic_ow = magic_of(r.OW);
+    a.step_images = static_cast<int>(step / r.area);
+    a.step_rest = static_cast<int>(step % r.area);
+  }
+  return gx;
 }
 
 template <int KS, int WN, int NI, int NS>
 void launch(hipStream_t s, Args& a) {
-  constexpr int TM = 128 / WN, NC = 32 * WN * NI;
-  const ResidentArgs& r = a.r;
-  const int tiles = (r.M + TM - 1) / TM, ny = (r.N + NC - 1) / NC;
-  int gx = 2 * num_cus() / ny;
-  if (gx > 8) gx = gx / 8 * 8;  // column groups of the same rows on the same XCD
-  if (gx < 1) gx = 1;
-  if (gx > tiles) gx = tiles;
-  const dim3 grid(gx, ny), block(256);
-  if (r.area != 0) {
-    const long long step = static_cast<long long>(gx) * TM;
-    a.step_images = static_cast<int>(step / r.area);
-    a.step_rest = static_cast<int>(step % r.area);
-    hipLaunchKernelGGL((resident_kernel<KS, WN, NI, NS, true>), grid, block, 0, s, a);
-  } else {
-    hipLaunchKernelGGL((resident_kernel<KS, WN, NI, NS, false>), grid, block, 0, s, a);
-  }
+  constexpr int NC = 32 * WN * NI;
+  const int ny = (a.r.N + NC - 1) / NC, gx = row_groups(a, 128 / WN, ny);
+  if (a.r.area != 0)
+    hipLaunchKernelGGL((resident_kernel<KS, WN, NI, NS, true>), dim3(gx, ny), dim3(256), 0, s, a);
+  else
+    hipLaunchKernelGGL((resident_kernel<KS, WN, NI, NS, false>), dim3(gx, ny), dim3(256), 0, s, a);
   MXQ_LAUNCH_CHECK();
 }
 
-}  // namespace
+template <int KS, int NS>
+void launch_pair(hipStream_t s, PairArgs& p) {
+  const int first = (p.a.r.N + 255) / 256, ny = first + (p.b.N + 255) / 256;
+  const int gx = row_groups(p.a, 32, ny);
+  p.first = first;
+  if (p.a.r.area != 0)
+    hipLaunchKernelGGL((resident_pair_kernel<KS, NS, true>), dim3(gx, ny), dim3(256), 0, s, p);
+  else
+    hipLaunchKernelGGL((resident_pair_kernel<KS, NS, false>), dim3(gx, ny), dim3(256), 0, s, p);
+  MXQ_LAUNCH_CHECK();
+}
 
-bool resident_wins(const ResidentArgs& a, bool aligned) {
+bool takes(const ResidentArgs& a, bool aligned) {
   if (!aligned || a.epi.out8 == nullptr || a.epi.out32 != nullptr || a.epi.outf != nullptr ||
       a.epi.with_sum)
     return false;
@@ -284,6 +320,13 @@ bool resident_wins(const ResidentArgs& a, bool aligned) {
     const long long span = (128 / a.area + 2) * a.image;
     if (a.area >= 30000 || a.OW >= 30000 || span >= (1LL << 31)) return false;
   }
+  return true;
+}
+
+}  // namespace
+
+bool resident_wins(const ResidentArgs& a, bool aligned) {
+  if (!takes(a, aligned)) return false;
   const int wide = a.K == 256 && a.N <= 64 ? 64 : a.N <= 128 ? 128 : 256;  // columns of a group
   const int high = wide == 64 ? 64 : 32;                                   // rows of a tile
   const long long groups = (a.N + wide - 1) / wide, tiles = (a.M + high - 1LL) / high * groups;
@@ -291,13 +334,24 @@ bool resident_wins(const ResidentArgs& a, bool aligned) {
   return tiles >= (a.K == 256 ? 3 : 6) * num_cus();
 }
 
+bool resident_pair_wins(const ResidentArgs& a, const ResidentArgs& b, bool aligned) {
+  if (!takes(a, aligned) || !takes(b, aligned)) return false;
+  const long long groups = (a.N + 255) / 256 + (b.N + 255) / 256;
+  if (3 * (a.N + b.N) < 2 * groups * 256) return false;
+  return (a.M + 31LL) / 32 * groups >= (a.K == 256 ? 3 : 6) * num_cus();
+}
+
+void launch_resident_pair(hipStream_t s, const ResidentArgs& a, const ResidentArgs& b) {
+  PairArgs p = {};
+  p.a.r = a;
+  p.b = b;
+  if (a.K == 256) launch_pair<8, 4>(s, p);
+  else launch_pair<16, 3>(s, p);
+}
+
 void launch_resident(hipStream_t s, const ResidentArgs& r) {
   Args a = {};
   a.r = r;
-  if (r.area != 0) {
-    a.magic_area = magic_of(r.area);
-    a.magic_ow = magic_of(r.OW);
-  }
   if (r.K == 256) {
     if (r.N <= 64) launch<8, 2, 1, 3>(s, a);
     else if (r.N <= 128) launch<8, 4, 1, 4>(s, a);
