@@ -399,6 +399,15 @@ int mxq_quantized_conv_pair_prepared(void* stream, const int8_t* data, int N, in
                                      const void* prepared2, int O2, int8_t* out2, int relu2,
                                      float min_calib2, float max_calib2);
 
+/* A stem: a 4 x 4 convolution of stride 1 over 16 channels, prepared, and the 3 x 3 maximum of
+ * stride 2 and padding 1 behind it in one launch; out8 is [N][pooled_h][pooled_w][O]. */
+int mxq_quantized_conv_pool_fits(int N, int H, int W, int C, int O, int KH, int KW, int pad_h,
+                                 int pad_w, int pooled_h, int pooled_w);
+int mxq_quantized_conv_pool(void* stream, const int8_t* data, const int8_t* weight,
+                            const void* prepared, int N, int H, int W, int C, int O, int KH,
+                            int KW, int pad_h, int pad_w, int pooled_h, int pooled_w, int8_t* out8,
+                            int relu);
+
 /* Looks for a short form of that sum with sum_relu != 0 over ranges that stay: two products and
  * one rounding that give the same int8 for every pair of int8 operands, which is tried out on
  * the device.  Writes 12 bytes to `pairs` (device, 4-byte aligned), among them whether one was

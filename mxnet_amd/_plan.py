@@ -30,7 +30,7 @@ _FLAG_OF = {torch.float32: 0, torch.float64: 1, torch.float16: 2, torch.uint8: 3
 _SIZE_OF = {0: 4, 1: 8, 2: 2, 3: 1, 4: 4, 5: 1, 6: 8, 7: 1, 12: 2}
 _FLOAT32, _INT32, _INT8 = 0, 4, 5
 (_NODE, _CONV, _FC, _FC_F32, _FC_SUM, _FC_SUM_RQ, _QUANT_NHWC, _TO_NHWC, _FROM_NHWC, _POOL, _RELU,
- _ADD, _REQUANTIZE, _BLOCK, _PAIR) = range(15)
+ _ADD, _REQUANTIZE, _BLOCK, _PAIR, _CONV_POOL) = range(16)
 _NULL, _ARENA, _HELD, _FEED, _OUTPUT = range(5)
 
 
@@ -681,6 +681,7 @@ class _Builder:
                 raise _Unsupported("a head that is an input, or the same as another head")
             v.at.place = (_OUTPUT, len(outputs), 0)
             outputs.append((v.flag, v.shape))
+        self.fuse_stem()
         self.fuse_blocks()
         self.pair_convs()
         # offsets: first fit over the buffers alive at the same steps
@@ -726,6 +727,9 @@ class _Builder:
                 layers, blobs = blobs, None
                 places[5:7] = [self.prepared(columns, calib, [place(r) for r in refs])
                                for columns, calib, refs in layers]
+            if kind == _CONV_POOL:
+                (columns, calib, refs), blobs = blobs, None
+                places[2] = self.prepared(columns, calib, [place(r) for r in refs])
             if kind in (_CONV, _FC, _FC_F32, _FC_SUM, _FC_SUM_RQ):
                 places.append(self.prepared(ints[4 if kind == _CONV else 1], floats, places))
             step = (kind, tuple(int(v) for v in ints), tuple(float(v) for v in floats),
@@ -734,17 +738,42 @@ class _Builder:
         plan = _frontend.plan(size, self.held, steps, [(f, tuple(s)) for f, s in outputs])
         return plan, tuple(self.params.values()), self.made
 
-    def fuse_blocks(self):
-        """The tail of a residual block as one step: a 3 x 3 convolution that only the sum's 1 x 1
-        convolution reads, that convolution with the sum, and a 1 x 1 convolution that reads the
-        sum."""
-        users = {}  # id of a buffer -> the steps that read or write it
+    def touched(self):
+        """id of a buffer -> the steps that read or write it"""
+        users = {}
         for at, step in enumerate(self.steps):
             for r in step[3]:
                 b = r.buffer if isinstance(r, _Offset) else r
                 if isinstance(b, _Buffer):
                     users.setdefault(id(b), []).append(at)
-        gone = set()
+        return users
+
+    def fuse_stem(self):
+        """A 4 x 4 convolution over 16 channels that only a 3 x 3 maximum reads, and that, as one
+        step."""
+        users, gone = self.touched(), set()
+        for at, (kind, geo, _, refs, _, _) in enumerate(self.steps):
+            if kind != _POOL or geo[4:10] != (3, 3, 2, 2, 1, 1) or geo[12]:
+                continue
+            mid = refs[0]
+            if not isinstance(mid, _Buffer) or mid.place is not None or len(users[id(mid)]) != 2:
+                continue
+            first = users[id(mid)][0]
+            kind, conv, calib, layer, _, _ = self.steps[first]
+            if (kind != _CONV or layer[10] is not mid or conv[7:9] != (1, 1) or
+                    conv[11:13] != (1, 1) or geo[3] != conv[4] or not self.stays(layer) or
+                    not _lib.lib.mxq_quantized_conv_pool_fits(*conv[:7], *conv[9:11], *geo[10:12])):
+                continue
+            self.steps[at] = (_CONV_POOL, conv[:7] + conv[9:11] + geo[10:12] + (conv[13],), (),
+                              [layer[0], layer[1], None, refs[1]], None, (conv[4], calib, layer))
+            gone.add(first)
+        self.drop(gone)
+
+    def fuse_blocks(self):
+        """The tail of a residual block as one step: a 3 x 3 convolution that only the sum's 1 x 1
+        convolution reads, that convolution with the sum, and a 1 x 1 convolution that reads the
+        sum."""
+        users, gone = self.touched(), set()
         for at, (kind, ints, floats, refs, _, _) in enumerate(self.steps):
             if kind != _FC_SUM_RQ or not ints[3] or not self.stays(refs):
                 continue

@@ -44,6 +44,7 @@ enum class Kind : int {
   kRequantize,   // calibrated
   kBlock,        // 3 x 3 convolution -> 1 x 1 -> sum (-> 1 x 1), each requantized
   kConvPair,     // two 1 x 1 convolutions of one tensor, each requantized (-> relu)
+  kConvPool,     // 4 x 4 convolution, requantized (-> relu) -> 3 x 3 maximum
 };
 
 struct Step {
