@@ -56,40 +56,7 @@ __global__ __launch_bounds__(kThreads) void quantize_nhwc_kernel(QuantNhwcArgs a
   const float* img = a.in + n * a.C * a.H * a.W;
   const size_t stride = static_cast<size_t>(a.H) * a.W;
   uint32_t w[4] = {0, 0, 0, 0};
-  if (S2D && a.C <= 4 && a.chunks == 1) {
-    // one piece holds the whole pixel: two neighbouring columns of each channel and row, loaded
-    // as one (224 x 224 x 3, the same image again and again, in cache: batch 64 17.5 us by single
-    // elements, 13.2 so; batch 1 7.4 and 4.1; images that come from memory 17.6 and 5.2 us so, the
-    // one image at the head of a network's pass 6.7)
-    const int x = 2 * ow - a.off_w;
-    const bool left = static_cast<unsigned>(x) < static_cast<unsigned>(a.W);
-    const bool right = static_cast<unsigned>(x + 1) < static_cast<unsigned>(a.W);
-    const bool both = left && right;
-#pragma unroll
-    for (int d = 0; d < 2; ++d) {
-      const int h = 2 * oh - a.off_h + d;
-      if (static_cast<unsigned>(h) >= static_cast<unsigned>(a.H)) continue;
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        if (c >= a.C) break;
-        const float* at = img + c * stride + static_cast<size_t>(h) * a.W + x;
-        float v[2] = {0.0f, 0.0f};
-        if (both) {
-          __builtin_memcpy(v, at, 8);
-        } else {
-          if (left) v[0] = at[0];
-          if (right) v[1] = at[1];
-        }
-#pragma unroll
-        for (int e = 0; e < 2; ++e) {
-          const int k = (2 * d + e) * a.C + c;
-          const uint32_t q = quant_byte(v[e], s) << (8 * (k & 3));
-#pragma unroll
-          for (int j = 0; j < 4; ++j) w[j] |= (k >> 2) == j ? q : 0u;
-        }
-      }
-    }
-  } else if (S2D) {
+  if (S2D) {
     int d = chunk * 16 / a.C, c = chunk * 16 - d * a.C;
 #pragma unroll
     for (int k = 0; k < 16; ++k) {
@@ -113,6 +80,59 @@ __global__ __launch_bounds__(kThreads) void quantize_nhwc_kernel(QuantNhwcArgs a
   a.out[(n * plane + pixel) * a.chunks + chunk] =
       v4i{static_cast<int>(w[0]), static_cast<int>(w[1]), static_cast<int>(w[2]),
           static_cast<int>(w[3])};
+}
+
+// The same for an image of up to four channels in space-to-depth form, a pixel of 16 bytes per lane:
+// two neighbouring columns of each channel and row, loaded as one, all of them before the first is
+// looked at (clamped into the image and taken out again where they were outside).  224 x 224 x 3
+// in the head of a network's pass: batch 64 9.9 us, one image 3.2 (with the channels a variable and
+// a branch around each load 13.4 and 6.7).
+constexpr int kS2dThreads = 128;
+template <int C>
+__global__ __launch_bounds__(kS2dThreads) void quantize_s2d_kernel(QuantNhwcArgs a) {
+  const int pixel = blockIdx.x * kS2dThreads + threadIdx.x, plane = a.OH * a.OW;
+  if (pixel == 0 && blockIdx.y == 0) {
+    *a.omin = -a.range;
+    *a.omax = a.range;
+  }
+  if (pixel >= plane) return;
+  const float s = 127.0f / a.range;
+  const int oh = static_cast<int>(static_cast<unsigned>(pixel) / static_cast<unsigned>(a.OW));
+  const int x = 2 * (pixel - oh * a.OW) - a.off_w, y = 2 * oh - a.off_h;
+  const int from = x < 0 ? 0 : x > a.W - 2 ? a.W - 2 : x;
+  const float* const img = a.in + static_cast<size_t>(blockIdx.y) * C * a.H * a.W;
+  float v[2][C][2];
+#pragma unroll
+  for (int d = 0; d < 2; ++d) {
+    const int h = y + d < 0 ? 0 : y + d > a.H - 1 ? a.H - 1 : y + d;
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+      __builtin_memcpy(v[d][c], img + (static_cast<size_t>(c) * a.H + h) * a.W + from, 8);
+  }
+  int q[16];
+#pragma unroll
+  for (int k = 0; k < 16; ++k) q[k] = 0;
+#pragma unroll
+  for (int d = 0; d < 2; ++d) {
+    const bool row = static_cast<unsigned>(y + d) < static_cast<unsigned>(a.H);
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const bool in = row && static_cast<unsigned>(x + e) < static_cast<unsigned>(a.W);
+      const bool high = x + e != from;  // of the pair
+#pragma unroll
+      for (int c = 0; c < C; ++c) {
+        const float f = in ? (high ? v[d][c][1] : v[d][c][0]) : 0.0f;
+        const float t = fabsf(f) * s + 0.5f;
+        // the sign before the conversion: it truncates either side alike
+        q[(2 * d + e) * C + c] = static_cast<int>(copysignf(127.0f < t ? 127.0f : t, f));
+      }
+    }
+  }
+  v4i w;
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    w[j] = static_cast<int>(pack_bytes(q[4 * j], q[4 * j + 1], q[4 * j + 2], q[4 * j + 3]));
+  a.out[static_cast<size_t>(blockIdx.y) * plane + pixel] = w;
 }
 
 struct PoolNhwcArgs {
@@ -368,7 +388,15 @@ int mxq_quantize_to_nhwc(void* stream, const float* in, int8_t* out, float* omin
   if (a.pieces == 0) return 0;
   MXQ_CHECK(in != nullptr && out != nullptr && aligned16(out), "null or unaligned data pointer");
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (space_to_depth)
+  if (space_to_depth && C <= 4 && a.chunks == 1 && W >= 2 && N <= 65535) {
+    const dim3 grid((a.OH * a.OW + kS2dThreads - 1) / kS2dThreads, N), block(kS2dThreads);
+    switch (C) {
+      case 1: hipLaunchKernelGGL(quantize_s2d_kernel<1>, grid, block, 0, s, a); break;
+      case 2: hipLaunchKernelGGL(quantize_s2d_kernel<2>, grid, block, 0, s, a); break;
+      case 3: hipLaunchKernelGGL(quantize_s2d_kernel<3>, grid, block, 0, s, a); break;
+      default: hipLaunchKernelGGL(quantize_s2d_kernel<4>, grid, block, 0, s, a);
+    }
+  } else if (space_to_depth)
     hipLaunchKernelGGL((quantize_nhwc_kernel<true>), dim3(blocks_for(a.pieces)), dim3(kThreads),
                        0, s, a);
   else

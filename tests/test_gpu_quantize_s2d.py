@@ -1,0 +1,40 @@
+"""A float image quantized into space-to-depth form: the bytes of the quantize operator and the
+layout change behind it, with odd extents, both offsets, and one column."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from mxnet_amd import capi
+from mxnet_amd._lib import check, lib
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("c", [1, 2, 3, 4, 5])
+@pytest.mark.parametrize("n,h,w", [(2, 224, 224), (3, 7, 9), (1, 1, 2), (1, 5, 1), (2, 2, 3),
+                                   (1, 33, 130)])
+@pytest.mark.parametrize("off", [(0, 0), (1, 1), (0, 1), (1, 0)])
+def test_image(c, n, h, w, off):
+    rng = np.random.default_rng(h * w + c)
+    x = rng.standard_normal((n, c, h, w)).astype(np.float32) * 2
+    special = [0.0, -0.0, np.nan, np.inf, -np.inf, 3.0, -3.0, 1e-30, -1e-30]
+    at = rng.integers(0, x.size, len(special))
+    x.reshape(-1)[at] = special
+    x = torch.from_numpy(x).cuda()
+    oh, ow = (h + off[0] + 1) // 2, (w + off[1] + 1) // 2
+    padded = (4 * c + 15) // 16 * 16
+    out = torch.full((n * oh * ow * padded + 64,), 99, dtype=torch.int8, device="cuda")
+    lo, hi = torch.zeros(1, device="cuda"), torch.zeros(1, device="cuda")
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    check(lib.mxq_quantize_to_nhwc(stream, x.data_ptr(), out.data_ptr(), lo.data_ptr(),
+                                   hi.data_ptr(), n, c, h, w, padded, 1, *off, -2.5, 3.0))
+    q, qlo, qhi = capi.quantize_v2(x, "int8", min_calib_range=-2.5, max_calib_range=3.0)
+    want = torch.zeros((n, 2 * oh, 2 * ow, c), dtype=torch.int8, device="cuda")
+    want[:, off[0]:off[0] + h, off[1]:off[1] + w] = q.permute(0, 2, 3, 1)
+    want = want.view(n, oh, 2, ow, 2, c).permute(0, 1, 3, 2, 4, 5).reshape(n, oh, ow, 4 * c)
+    got = out[:-64].view(n, oh, ow, padded)
+    assert torch.equal(got[..., :4 * c], want) and not got[..., 4 * c:].any()
+    assert (out[-64:] == 99).all()
+    assert (lo.item(), hi.item()) == (qlo.item(), qhi.item())
