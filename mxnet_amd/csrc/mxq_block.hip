@@ -18,7 +18,7 @@
 // per 32 x 32 MFMA operand), so a load is one contiguous KB, no LDS ring and no barrier stands
 // between a wave and its next operand, and five barriers per tile are all that is left.  A CU
 // takes in 64 bytes of weights per clock and multiplies them with the 64 pixels in the same time,
-// which is why TM is no smaller.
+// which is why TM is no smaller where the tiles fill the chip.
 //
 // Rows in LDS are an odd number of 16-byte chunks apart: 16 consecutive rows' fragments hit
 // distinct bank groups without a permutation, for any channel count.
@@ -696,9 +696,10 @@ bool fit_lds(BlockPlan* b, int C, int Cm, int Co, int Ca) {
   b->lds = static_cast<int>(lds);
   return lds <= kBlockLds;
 }
-BlockPlan plan_block(int N, int H, int W, int C, int Cm, int Co, int Ca) {
+BlockPlan plan_tiles(int N, int H, int W, int C, int Cm, int Co, int Ca, int tm) {
   BlockPlan b;
   if (!plan_layers(C, Cm, Co, Ca, &b)) return b;
+  b.tm = tm;
   if (N <= 0 || H <= 0 || W <= 0 || W > 8192 || H > 8192) return b;
   const long long M = static_cast<long long>(N) * H * W;
   const long long widest = Co > C ? Co : C;
@@ -754,6 +755,17 @@ BlockPlan plan_block(int N, int H, int W, int C, int Cm, int Co, int Ca) {
   return b;
 }
 
+// Tiles of 64 pixels: a CU then multiplies a weight as long as it takes in the next one.  Where they
+// would leave half of the CUs idle, of 32: a tile's chain is shorter by half of its products and its
+// vector work (28 x 28 x 128 on one image 10.7 us -> 9.2, on 8 images 13 -> 9.6; 14 x 14 x 256 on
+// 4 images 18.9 -> 15.6).
+BlockPlan plan_block(int N, int H, int W, int C, int Cm, int Co, int Ca) {
+  const BlockPlan b = plan_tiles(N, H, W, C, Cm, Co, Ca, 64);
+  if (b.tiles == 0 || 2 * b.tiles > num_cus()) return b;
+  const BlockPlan half = plan_tiles(N, H, W, C, Cm, Co, Ca, 32);
+  return half.tiles > 0 ? half : b;
+}
+
 template <int WM, int WN, int RT, int GB, int GC>
 void launch_block(hipStream_t s, const BlockArgs& a, int lds) {
   const unsigned grid = static_cast<unsigned>((a.tiles + 7) / 8 * 8);
@@ -770,10 +782,10 @@ using namespace mxq;
 extern "C" {
 
 // Whether it is also the faster way.  It is from one image on with up to 128 channels in the middle
-// (56 x 56 x 64: 7.8 us against 14.1 in three launches on one image, 38.6 against 60.2 on 64;
-// 28 x 28 x 128 10.7 / 13.3 and 30.4 / 45.2).  Above that a tile alone takes 18 us, most of it the
-// 1.1 MB of weights that a CU takes in: 13 tiles (14 x 14 x 256 on 4 images) 18.9 us against 16.4,
-// 25 tiles 19.1 against 20.4, 196 tiles 22.0 against 38.3.
+// (56 x 56 x 64: 7.4 us against 14.1 in three launches on one image, 38.6 against 60.2 on 64;
+// 28 x 28 x 128 9.2 / 14.0 and 30.4 / 45.2).  Above that a tile alone takes 15 us, most of it the
+// 1.1 MB of weights that a CU takes in: 19 tiles (14 x 14 x 256 on 3 images) 15.6 us against 16.0,
+// 25 tiles 15.6 against 16.5, 98 of 32 pixels 16.6 against 23.3, 196 of 64 22.0 against 38.3.
 int mxq_quantized_block_fits(int N, int H, int W, int C, int C_mid, int C_out, int C_next) {
   const BlockPlan b = plan_block(N, H, W, C, C_mid, C_out, C_next);
   return b.tiles > 0 && (b.variant < 256 || b.tiles >= 20) ? 1 : 0;
@@ -900,12 +912,20 @@ int mxq_quantized_block(void* stream, const int8_t* data, const int8_t* weights,
   a.relu_a = relu_third != 0;
   a.tiles = b.tiles;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (b.variant == 64)
+  if (b.tm == 32) {
+    if (b.variant == 64)
+      launch_block<1, 4, 1, 6, 2>(s, a, b.lds);
+    else if (b.variant == 128)
+      launch_block<1, 8, 1, 6, 4>(s, a, b.lds);
+    else
+      launch_block<1, 8, 1, 8, 8>(s, a, b.lds);
+  } else if (b.variant == 64) {
     launch_block<2, 2, 1, 6, 2>(s, a, b.lds);
-  else if (b.variant == 128)
+  } else if (b.variant == 128) {
     launch_block<1, 8, 2, 6, 4>(s, a, b.lds);
-  else
+  } else {
     launch_block<1, 8, 2, 8, 8>(s, a, b.lds);
+  }
   MXQ_API_END();
 }
 

@@ -85,16 +85,36 @@ def blocks(n, h, w, c, mid, out, after, relu1=1, relu3=1, residual=(-3.0, 3.0), 
     return have, want, int(forms[:192].view(torch.int32)[35])
 
 
-@pytest.mark.parametrize("n,h,w,c,mid,out,after", [
+SHAPES = [
     (1, 4, 4, 16, 16, 16, 16), (1, 8, 8, 32, 64, 256, 64), (1, 5, 13, 48, 48, 80, 0),
     (2, 7, 9, 64, 64, 256, 48), (3, 13, 5, 16, 32, 144, 16), (1, 3, 43, 80, 16, 16, 272),
     (2, 56, 56, 64, 64, 256, 64), (1, 112, 9, 16, 32, 48, 16),          # up to 64 in the middle
     (2, 14, 14, 128, 128, 512, 128), (1, 9, 7, 96, 80, 336, 80), (5, 28, 28, 128, 112, 64, 0),
     (3, 7, 5, 144, 96, 32, 160),                                         # up to 128
     (1, 14, 14, 256, 256, 1024, 256), (4, 14, 13, 256, 144, 592, 144), (2, 9, 31, 160, 256, 16, 0),
-    (1, 1, 65, 16, 176, 48, 512)])                                       # up to 256
+    (1, 1, 65, 16, 176, 48, 512)]                                        # up to 256
+
+
+@pytest.mark.parametrize("n,h,w,c,mid,out,after", SHAPES)
 def test_block(n, h, w, c, mid, out, after):
     have, want, _ = blocks(n, h, w, c, mid, out, after)
+    for a, b in zip(have, want):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("n,h,w,c,mid,out,after", SHAPES)
+def test_block_on_whole_tiles(n, h, w, c, mid, out, after):
+    """Enough pixels for tiles of 64, which fewer images than fill half of the chip do not take."""
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    have, want, _ = blocks(n + cus * 32 // (h * w) + 1, h, w, c, mid, out, after)
+    for a, b in zip(have, want):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("relu1,relu3", [(0, 0), (1, 0), (0, 1)])
+@pytest.mark.parametrize("mid,spread", [(48, 0.02), (128, 40.0), (160, 1.0)])
+def test_block_ranges_on_whole_tiles(mid, spread, relu1, relu3):
+    have, want, _ = blocks(90, 10, 11, 64, mid, 96, 32, relu1, relu3, spread=spread)
     for a, b in zip(have, want):
         assert torch.equal(a, b)
 
