@@ -159,8 +159,9 @@ uint32_t magic_of(int d) { return static_cast<uint32_t>((1ULL << 31) / static_ca
 // WM x WN waves, each RT row tiles of 32 pixels by one column tile of 32 channels at a time.
 // GB, GC: MFMA steps whose weights a wave requests together (the 3 x 3 layer's, and the whole
 // reduction of the second layer).
+// `tile` is one of p.tiles; or, of runs, the one that begins at pixel `first`.
 template <int WM, int WN, int RT, int GB, int GC>
-__global__ __launch_bounds__(64 * WM * WN, GC < 8 ? 4 : 2) void block_kernel(BlockArgs p) {
+__device__ __forceinline__ void block_tile(const BlockArgs& p, int tile, int first) {
   constexpr int NW = WM * WN, TM = 32 * WM * RT, GA = 8;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   // every argument at once: left alone the compiler loads each of them where it is first used, a
@@ -176,16 +177,12 @@ __global__ __launch_bounds__(64 * WM * WN, GC < 8 ? 4 : 2) void block_kernel(Blo
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WN, wn = wave % WN;
-  // an XCD takes a run of neighbouring tiles: they share halo rows in its L2
-  const int per = (p.tiles + 7) >> 3;
-  const int tile = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
-  if (tile >= p.tiles) return;
   // The tile's pixel i is pixel (h0, w0) + place start + i of rows of `across` in images of `area`
   // pixels, from image n0 on: a rectangle, whole images, or a run of pixels in the tensor's order.
   int n0, h0 = 0, w0 = 0, start_at = 0;
   if (p.run) {
-    n0 = quotient_any(tile * TM, p.area, p.magic_area);
-    start_at = tile * TM - n0 * p.area;
+    n0 = quotient_any(first, p.area, p.magic_area);
+    start_at = first - n0 * p.area;
   } else {
     const int down = quotient(tile, p.magic_tiles_w), batch = quotient(down, p.magic_tiles_h);
     n0 = batch * p.tn;
@@ -521,6 +518,24 @@ __global__ __launch_bounds__(64 * WM * WN, GC < 8 ? 4 : 2) void block_kernel(Blo
   leave(p.off_patch, CA, PA, p.magic_next, p.next);
 }
 
+template <int WM, int WN, int RT, int GB, int GC>
+__global__ __launch_bounds__(64 * WM * WN, GC < 8 ? 4 : 2) void block_kernel(BlockArgs p) {
+  // an XCD takes a run of neighbouring tiles: they share halo rows in its L2
+  const int per = (p.tiles + 7) >> 3;
+  const int tile = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  if (tile < p.tiles) block_tile<WM, WN, RT, GB, GC>(p, tile, tile * 32 * WM * RT);
+}
+
+// Runs of pixels: p.tiles (a multiple of 8) of 64 and the rest in halves behind them.
+template <int GB, int GC>
+__global__ __launch_bounds__(512, GC < 8 ? 4 : 2) void block_halves_kernel(BlockArgs p) {
+  const int block = blockIdx.x;
+  if (block < p.tiles)
+    block_tile<1, 8, 2, GB, GC>(p, 0, 64 * ((block & 7) * (p.tiles >> 3) + (block >> 3)));
+  else
+    block_tile<1, 8, 1, GB, GC>(p, 0, 64 * p.tiles + 32 * (block - p.tiles));
+}
+
 // [O][taps][C] rows -> fragments [ceil(O / 32)][steps][64 lanes][16 bytes]: lane l of step
 // tap * per_tap + s holds bytes 32 * s + 16 * (l / 32) ... + 15 of tap `tap` of row l % 32 of the
 // column tile, zeros where there are none.
@@ -650,6 +665,7 @@ int up(int n, int unit) { return (n + unit - 1) / unit * unit; }
 struct BlockPlan {
   int variant = 0;  // 64, 128 or 256: the channels in the middle, at most
   int tm = 0, tiles = 0;
+  int halves = 0;  // tiles of half the size behind them
   int steps[3] = {0, 0, 0};
   size_t fragments[3] = {0, 0, 0};  // KB
   int run = 0, tn = 1, th = 1, tw = 1, tiles_h = 1, tiles_w = 1, rows = 0;
@@ -758,10 +774,17 @@ BlockPlan plan_tiles(int N, int H, int W, int C, int Cm, int Co, int Ca, int tm)
 // Tiles of 64 pixels: a CU then multiplies a weight as long as it takes in the next one.  Where they
 // would leave half of the CUs idle, of 32: a tile's chain is shorter by half of its products and its
 // vector work (28 x 28 x 128 on one image 10.7 us -> 9.2, on 8 images 13 -> 9.6; 14 x 14 x 256 on
-// 4 images 18.9 -> 15.6).
+// 4 images 18.9 -> 15.6).  And where a few runs are left over when every CU has had as many, those
+// go in halves, so that fewer CUs end with a whole tile more than the others (784 tiles of 28 x 28 x
+// 128 on 256 CUs, four blocks in a network's pass: 2 us less each).
 BlockPlan plan_block(int N, int H, int W, int C, int Cm, int Co, int Ca) {
-  const BlockPlan b = plan_tiles(N, H, W, C, Cm, Co, Ca, 64);
-  if (b.tiles == 0 || 2 * b.tiles > num_cus()) return b;
+  BlockPlan b = plan_tiles(N, H, W, C, Cm, Co, Ca, 64);
+  const int cus = num_cus(), over = b.tiles % cus;
+  if (b.run && b.variant > 64 && b.tiles > cus && over != 0 && 2 * over <= cus && cus % 8 == 0) {
+    b.tiles -= over;
+    b.halves = static_cast<int>((static_cast<long long>(N) * H * W - 64LL * b.tiles + 31) / 32);
+  }
+  if (b.tiles == 0 || 2 * b.tiles > cus) return b;
   const BlockPlan half = plan_tiles(N, H, W, C, Cm, Co, Ca, 32);
   return half.tiles > 0 ? half : b;
 }
@@ -912,7 +935,14 @@ int mxq_quantized_block(void* stream, const int8_t* data, const int8_t* weights,
   a.relu_a = relu_third != 0;
   a.tiles = b.tiles;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (b.tm == 32) {
+  if (b.halves != 0) {
+    const dim3 grid(static_cast<unsigned>(b.tiles + b.halves));
+    if (b.variant == 128)
+      hipLaunchKernelGGL((block_halves_kernel<6, 4>), grid, dim3(512), b.lds, s, a);
+    else
+      hipLaunchKernelGGL((block_halves_kernel<8, 8>), grid, dim3(512), b.lds, s, a);
+    MXQ_LAUNCH_CHECK();
+  } else if (b.tm == 32) {
     if (b.variant == 64)
       launch_block<1, 4, 1, 6, 2>(s, a, b.lds);
     else if (b.variant == 128)

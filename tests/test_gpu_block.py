@@ -111,6 +111,16 @@ def test_block_on_whole_tiles(n, h, w, c, mid, out, after):
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("n,h,w,c,mid,out,after", SHAPES[8:])
+@pytest.mark.parametrize("more", [1, 700, 5000])
+def test_block_that_ends_in_halves(n, h, w, c, mid, out, after, more):
+    """A few tiles more than the chip has CUs: what is left over goes in tiles of 32."""
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    have, want, _ = blocks((cus * 64 + more) // (h * w) + 1, h, w, c, mid, out, after)
+    for a, b in zip(have, want):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("relu1,relu3", [(0, 0), (1, 0), (0, 1)])
 @pytest.mark.parametrize("mid,spread", [(48, 0.02), (128, 40.0), (160, 1.0)])
 def test_block_ranges_on_whole_tiles(mid, spread, relu1, relu3):
