@@ -180,6 +180,9 @@ __global__ __launch_bounds__(256, 2) void conv_pool_kernel(StemArgs p) {
   take(window[0]);
   take(window[1]);
   take(window[2]);
+  // Row 0 sends for the row that takes the first one's slot, and a row outside the image is zeros
+  // at once: they must not overtake the read.  (From here on a slot's rows have been multiplied.)
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 
   int above[NI][7];  // the maxima of the window's upper row
   // The horizontal maxima of convolution row r of the walk, R = r mod 4.

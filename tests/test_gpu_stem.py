@@ -56,6 +56,33 @@ def test_stem_is_convolution_and_pooling(shape, relu, full, far):
     assert torch.equal(got, want)
 
 
+def test_rows_outside_the_image_do_not_overtake():
+    """Bands of one pooled row at the image's lower edge, where the rows sent for ahead are zeros
+    that arrive at once: the same bytes every time."""
+    n, h, w, o, p_h, p_w = 64, 33, 33, 64, 16, 16
+    g = torch.Generator(device="cuda").manual_seed(5)
+    draw = lambda s: torch.randint(-127, 128, s, device="cuda", generator=g, dtype=torch.int8)
+    data, weight, bias = draw((n, h, w, 16)), draw((o, 4, 4, 16)), draw((o,))
+    ranges = [torch.tensor([v], device="cuda") for v in (-3.0, 2.5, -0.5, 0.75, -1.0, 1.0)]
+    prepared = torch.empty(64 + 4 * o, dtype=torch.int8, device="cuda")
+    stream = torch.cuda.current_stream().cuda_stream
+    check(lib.mxq_prepare_layer(stream, bias.data_ptr(), o, *[r.data_ptr() for r in ranges], -20.0,
+                                18.0, prepared.data_ptr()))
+    conv = torch.empty((n, 32, 32, o), dtype=torch.int8, device="cuda")
+    check(lib.mxq_quantized_conv_nhwc_prepared(
+        stream, data.data_ptr(), weight.data_ptr(), prepared.data_ptr(), n, h, w, 16, o, 4, 4, 1, 1,
+        1, 1, 1, 1, conv.data_ptr(), 1, -20.0, 18.0, None, 0))
+    want = torch.empty((n, p_h, p_w, o), dtype=torch.int8, device="cuda")
+    check(lib.mxq_quantized_pooling_nhwc(stream, conv.data_ptr(), n, 32, 32, o, 3, 3, 2, 2, 1, 1,
+                                         p_h, p_w, 0, 1, want.data_ptr()))
+    for _ in range(100):
+        got = torch.empty_like(want)
+        check(lib.mxq_quantized_conv_pool(stream, data.data_ptr(), weight.data_ptr(),
+                                          prepared.data_ptr(), n, h, w, 16, o, 4, 4, 1, 1, p_h, p_w,
+                                          got.data_ptr(), 1))
+        assert torch.equal(got, want)
+
+
 def test_what_does_not_fit():
     fits = lib.mxq_quantized_conv_pool_fits
     assert fits(1, 115, 115, 16, 64, 4, 4, 0, 0, 56, 56)
