@@ -370,6 +370,9 @@ int mxq_prepare_layer(void* stream, const int8_t* bias, int N, const float* min_
                       const float* max_data, const float* min_weight, const float* max_weight,
                       const float* min_bias, const float* max_bias, float min_calib,
                       float max_calib, void* prepared);
+/* Looks for short forms of the layer's requantize that give the same int8 for every accumulator and
+ * notes them in what mxq_prepare_layer wrote, for the launches that use them. */
+int mxq_prepare_forms(void* stream, void* prepared);
 int mxq_quantized_fc_prepared(void* stream, const int8_t* data, const int8_t* weight,
                               const void* prepared, int M, int N, int K, int8_t* out8,
                               float* out_f32, int relu, float min_calib, float max_calib,

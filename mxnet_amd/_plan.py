@@ -567,7 +567,7 @@ class _Builder:
 
     def pairs(self, layer, residual, total, relu):
         """What mxq_sum_requant_pairs finds for a sum with a relu behind it whose ranges are the
-        plan's constants; None for any other."""
+        plan's constants, once the step turns out to be one of the plan; None for any other."""
         if relu is None or not all(getattr(r, "in_table", False) for r in residual):
             return None
         ranges = (*layer, *(self.constants[r.place[2] // 4] for r in residual), *total)
@@ -577,7 +577,7 @@ class _Builder:
             _lib.check(_lib.lib.mxq_sum_requant_pairs(self.stream, *ranges, found.data_ptr()))
             return found
 
-        return self.laid(("pairs",) + tuple(map(_bits, ranges)), (), make)
+        return _Later(lambda: self.laid(("pairs",) + tuple(map(_bits, ranges)), (), make).place)
 
     def act(self, i, attrs, inputs):
         x = self.values[inputs[0]]
@@ -681,9 +681,7 @@ class _Builder:
                 raise _Unsupported("a head that is an input, or the same as another head")
             v.at.place = (_OUTPUT, len(outputs), 0)
             outputs.append((v.flag, v.shape))
-        self.fuse_stem()
-        self.fuse_blocks()
-        self.pair_convs()
+        self.fuse()
         # offsets: first fit over the buffers alive at the same steps
         taken, size = [], 0
         for b in sorted((b for b in self.buffers if b.place is None and b.first is not None),
@@ -708,6 +706,8 @@ class _Builder:
             if isinstance(r, _Offset):
                 base, at, offset = r.buffer.place
                 return (base, at, offset + r.offset)
+            if isinstance(r, _Later):
+                return r.find()
             if getattr(r, "in_table", False):
                 return (_HELD, self.table_index, r.place[2])
             return r.place
@@ -725,7 +725,7 @@ class _Builder:
                 places[2] = self.block_forms(floats, layers, places[3:6])
             if kind == _PAIR:
                 layers, blobs = blobs, None
-                places[5:7] = [self.prepared(columns, calib, [place(r) for r in refs])
+                places[5:7] = [self.prepared(columns, calib, [place(r) for r in refs], True)
                                for columns, calib, refs in layers]
             if kind == _CONV_POOL:
                 (columns, calib, refs), blobs = blobs, None
@@ -738,20 +738,33 @@ class _Builder:
         plan = _frontend.plan(size, self.held, steps, [(f, tuple(s)) for f, s in outputs])
         return plan, tuple(self.params.values()), self.made
 
-    def touched(self):
-        """id of a buffer -> the steps that read or write it"""
-        users = {}
+    def fuse(self):
+        """Steps that go out together as one; the buffers' lifetimes follow."""
+        users = {}  # id of a buffer -> the steps that read or write it
         for at, step in enumerate(self.steps):
             for r in step[3]:
-                b = r.buffer if isinstance(r, _Offset) else r
-                if isinstance(b, _Buffer):
+                b = r.buffer if type(r) is _Offset else r
+                if type(b) is _Buffer:
                     users.setdefault(id(b), []).append(at)
-        return users
+        gone = set()
+        self.fuse_stem(users, gone)
+        self.fuse_blocks(users, gone)
+        self.pair_convs(gone)
+        if not gone:
+            return
+        self.steps = [s for at, s in enumerate(self.steps) if at not in gone]
+        for b in self.buffers:
+            b.first = b.last = None
+        for at, step in enumerate(self.steps):
+            for r in step[3]:
+                b = r.buffer if type(r) is _Offset else r
+                if type(b) is _Buffer:
+                    b.first = at if b.first is None else b.first
+                    b.last = at
 
-    def fuse_stem(self):
+    def fuse_stem(self, users, gone):
         """A 4 x 4 convolution over 16 channels that only a 3 x 3 maximum reads, and that, as one
         step."""
-        users, gone = self.touched(), set()
         for at, (kind, geo, _, refs, _, _) in enumerate(self.steps):
             if kind != _POOL or geo[4:10] != (3, 3, 2, 2, 1, 1) or geo[12]:
                 continue
@@ -767,13 +780,11 @@ class _Builder:
             self.steps[at] = (_CONV_POOL, conv[:7] + conv[9:11] + geo[10:12] + (conv[13],), (),
                               [layer[0], layer[1], None, refs[1]], None, (conv[4], calib, layer))
             gone.add(first)
-        self.drop(gone)
 
-    def fuse_blocks(self):
+    def fuse_blocks(self, users, gone):
         """The tail of a residual block as one step: a 3 x 3 convolution that only the sum's 1 x 1
         convolution reads, that convolution with the sum, and a 1 x 1 convolution that reads the
         sum."""
-        users, gone = self.touched(), set()
         for at, (kind, ints, floats, refs, _, _) in enumerate(self.steps):
             if kind != _FC_SUM_RQ or not ints[3] or not self.stays(refs):
                 continue
@@ -805,42 +816,26 @@ class _Builder:
             self.steps[at] = (_BLOCK, shape + (layers[2][0], self.steps[first][1][13], relu),
                               floats, [conv[0], None, None, None, None, None, refs[12],
                                        refs[10], out], None, layers)
-        self.drop(gone)
 
-    def pair_convs(self):
+    def pair_convs(self, gone):
         """Two 1 x 1 convolutions of the same tensor as one step, at the place of the first."""
-        gone = set()
-        for at, (kind, geo, calib, refs, _, _) in enumerate(self.steps):
-            if (kind != _CONV or at in gone or geo[5:7] != (1, 1) or geo[9:11] != (0, 0) or
-                    not self.stays(refs)):
+        first = {}  # id of the tensor -> a convolution of it that has no partner yet
+        for j, (kind, geo2, calib2, refs2, _, _) in enumerate(self.steps):
+            if (kind != _CONV or j in gone or geo2[5:7] != (1, 1) or geo2[9:11] != (0, 0) or
+                    not self.stays(refs2)):
                 continue
-            for j in range(at + 1, len(self.steps)):
-                other, geo2, calib2, refs2, _, _ = self.steps[j]
-                if (other == _CONV and j not in gone and refs2[0] is refs[0] and
-                        geo2[:4] + geo2[5:13] == geo[:4] + geo[5:13] and self.stays(refs2) and
-                        _lib.lib.mxq_quantized_conv_pair_fits(*geo[:5], geo2[4], *geo[7:9])):
-                    self.steps[at] = (
-                        _PAIR, geo[:5] + (geo2[4],) + geo[7:9] + (geo[13], geo2[13]),
-                        tuple(calib) + tuple(calib2),
-                        [refs[0], refs[1], refs2[1], refs[10], refs2[10], None, None], None,
-                        [(geo[4], calib, refs), (geo2[4], calib2, refs2)])
-                    gone.add(j)
-                    break
-        self.drop(gone)
-
-    def drop(self, gone):
-        """Leaves the steps `gone` out; the buffers' lifetimes follow."""
-        if not gone:
-            return
-        self.steps = [s for at, s in enumerate(self.steps) if at not in gone]
-        for b in self.buffers:
-            b.first = b.last = None
-        for at, step in enumerate(self.steps):
-            for r in step[3]:
-                b = r.buffer if isinstance(r, _Offset) else r
-                if isinstance(b, _Buffer):
-                    b.first = at if b.first is None else b.first
-                    b.last = at
+            at = first.setdefault(id(refs2[0]), j)
+            _, geo, calib, refs, _, _ = self.steps[at]
+            if (at == j or geo2[:4] + geo2[5:13] != geo[:4] + geo[5:13] or
+                    not _lib.lib.mxq_quantized_conv_pair_fits(*geo[:5], geo2[4], *geo[7:9])):
+                first[id(refs2[0])] = j
+                continue
+            self.steps[at] = (_PAIR, geo[:5] + (geo2[4],) + geo[7:9] + (geo[13], geo2[13]),
+                              tuple(calib) + tuple(calib2),
+                              [refs[0], refs[1], refs2[1], refs[10], refs2[10], None, None], None,
+                              [(geo[4], calib, refs), (geo2[4], calib2, refs2)])
+            gone.add(j)
+            del first[id(refs2[0])]
 
     @staticmethod
     def stays(refs):
@@ -899,13 +894,14 @@ class _Builder:
                 names += read
         return key, names
 
-    def prepared(self, columns, calib, places):
-        """What mxq_prepare_layer makes of a layer's bias and six ranges, if they stay."""
+    def prepared(self, columns, calib, places, forms=False):
+        """What mxq_prepare_layer makes of a layer's bias and six ranges, if they stay; with the
+        short forms that mxq_prepare_forms finds."""
         given = places[2:9]
         if any(base not in (_HELD, _NULL) for base, _, _ in given):
             return (_NULL, 0, 0)
         key, names = self.constants_key(given)
-        key = ["prepared", int(columns), _bits(calib[0]), _bits(calib[1])] + key
+        key = ["prepared", forms, int(columns), _bits(calib[0]), _bits(calib[1])] + key
 
         def make():
             at = [None if base == _NULL else self.held[i].data_ptr() + offset
@@ -914,9 +910,18 @@ class _Builder:
             _lib.check(_lib.lib.mxq_prepare_layer(self.stream, at[0], int(columns), *at[1:],
                                                   float(calib[0]), float(calib[1]),
                                                   out.data_ptr()))
+            if forms:
+                _lib.check(_lib.lib.mxq_prepare_forms(self.stream, out.data_ptr()))
             return out
 
         return self.laid(tuple(key), tuple(names), make).place
+
+
+class _Later:
+    """An operand that is laid out when its step is assembled."""
+
+    def __init__(self, find):
+        self.find = find
 
 
 class _Offset:

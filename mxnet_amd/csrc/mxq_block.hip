@@ -37,6 +37,7 @@
 
 #include "../../include/mxq.h"
 #include "mxq_common.h"
+#include "mxq_forms.h"
 #include "mxq_gemm.h"
 
 namespace mxq {
@@ -47,39 +48,11 @@ namespace {
 
 constexpr int kBlockLds = 160 * 1024;
 
-// Short forms.  The definition of a requantize is four float operations with a rounding each, then
-// a clamp, a truncation and a relu: 6.5 vector instructions per output with the packing, 7.75
-// without the relu, and 6 more for the sum, together several times what the matrix cores take for
-// a 1 x 1 layer.  Each of them is a function with few steps of an integer: a requantize has 127
-// thresholds (its negative half mirrors the positive one), the sum is defined on 255 x 256 pairs.
-// So whether one multiplication and one addition give the same int8 everywhere is found out by
-// looking at every threshold from both sides, or at every pair; the factor may move by some last
-// places until they do (it holds for nearly all ranges, the others keep the definition).
-//   with the relu   cvt_pk_u8(fma(acc, 2t, c)) / 2 with c = 0.5, or some 2^-18 beside it: twice the
-//                   level, rounded, in [0, 255]; the halving drops what the rounding of twice the
-//                   level and a half is off by
-//   without         fma(acc, t, 2^23 + 128) clamped to 2^23 + [1, 255]: its rounding is the
-//                   level's, and the low byte is the level + 128
-//   the sum         as the first, over fma(level, 2ta, fma(residual, 2tb, c)).  Both operands are
-//                   small integers in 16 bits, which read as half floats are that many times
-//                   2^-24: v_fma_mix_f32 takes them as they are, without a conversion
-// 3.25 instructions per output of a layer with a relu, 7 instead of 13.75 for the sum.
-constexpr float kRound = 8388608.0f + 128.0f;
-__device__ __forceinline__ uint32_t halve4(uint32_t w) { return __builtin_amdgcn_lerp(w, 0u, 0u); }
-__device__ __forceinline__ uint32_t short_relu4(int a0, int a1, int a2, int a3, float t, float c) {
-  uint32_t w = 0;
-  w = __builtin_amdgcn_cvt_pk_u8_f32(__builtin_fmaf(static_cast<float>(a0), t, c), 0, w);
-  w = __builtin_amdgcn_cvt_pk_u8_f32(__builtin_fmaf(static_cast<float>(a1), t, c), 1, w);
-  w = __builtin_amdgcn_cvt_pk_u8_f32(__builtin_fmaf(static_cast<float>(a2), t, c), 2, w);
-  w = __builtin_amdgcn_cvt_pk_u8_f32(__builtin_fmaf(static_cast<float>(a3), t, c), 3, w);
-  return halve4(w);
-}
-// the level + 128, in the low 16 bits
-__device__ __forceinline__ uint32_t short_level(int a, float t) {
-  return __float_as_uint(
-      __builtin_amdgcn_fmed3f(__builtin_fmaf(static_cast<float>(a), t, kRound), kRound - 127.0f,
-                              kRound + 127.0f));
-}
+// The short forms of mxq_forms.h, and for the sum
+//   fma(level, 2ta, fma(residual, 2tb, c)) as the form with the relu.  Both operands are small
+//   integers in 16 bits, which read as half floats are that many times 2^-24: v_fma_mix_f32 takes
+//   them as they are, without a conversion
+// 7 instructions per output instead of 13.75.
 struct SumForm {
   float ta, tb, c;  // for levels and residuals + 128, times 2^-24
 };
@@ -113,7 +86,7 @@ struct BlockForms {
   float t[3], c[3];  // factor and constant of the layers' short forms
   SumForm sum;
   int has;       // bit i: layer i has one; bit 3: the sum has
-  int pair;      // which of the tried ones that is
+  unsigned long long failed;  // of the tried pairs of factors
 };
 constexpr size_t kBlockForms = 192;
 static_assert(sizeof(BlockForms) <= kBlockForms, "room for the forms");
@@ -553,9 +526,9 @@ __global__ __launch_bounds__(256) void pack_fragments_kernel(const v4i* in, v4i*
   out[i] = ok ? in[(static_cast<size_t>(n) * taps + tap) * chunks + c] : v4i{0, 0, 0, 0};
 }
 
-// The search for the forms, in three launches: nothing found yet; work-groups 0 ... 2 each try
-// every factor and constant for a layer (layers 0 and 2 with the relu, 1 without), one per thread,
-// and the others one pair of factors each for the sum; then what the sum's found.
+// The search for the forms, in three launches: nothing found yet; work-groups 0 ... 2 each look for
+// a layer's (layers 0 and 2 with the relu, 1 without), and the others take kShares to a pair of
+// factors for the sum, each a share of the operands; then what those found.
 struct PrepareArgs {
   const char* prepared[3];
   const float* res_min;
@@ -563,13 +536,7 @@ struct PrepareArgs {
   float layer_range, sum_min, sum_max;
   BlockForms* out;
 };
-constexpr int kFactors = 64, kConstants = 16, kPairs = 49;
-__device__ __forceinline__ float moved(float v, int c) {  // 0, +1, -1, +2, ... last places away
-  return __int_as_float(__float_as_int(v) + ((c & 1) ? (c + 1) / 2 : -(c / 2)));
-}
-__device__ __forceinline__ float constant(int k) {  // likewise around 0.5, in steps of 2^-18
-  return 0.5f + static_cast<float>((k & 1) ? (k + 1) / 2 : -(k / 2)) * (1.0f / 262144.0f);
-}
+constexpr int kPairs = 49, kShares = 8;
 __device__ __forceinline__ RequantRule block_rule(const PrepareArgs& p) {
   return sum_requant_rule(dev_maxabs(-p.layer_range, p.layer_range),
                           dev_maxabs(*p.res_min, *p.res_max), p.sum_min, p.sum_max);
@@ -584,65 +551,40 @@ __device__ __forceinline__ bool pair_of_factors(const RequantRule& r, int c, flo
 }
 __global__ void clear_forms_kernel(BlockForms* out) {
   out->has = 0;
-  out->pair = kPairs;
+  out->failed = 0;
 }
 __global__ void finish_forms_kernel(PrepareArgs p) {
   BlockForms* const out = p.out;
   out->rule = block_rule(p);
+  const int pair = __builtin_ctzll(~out->failed);  // the first that has not
   float a, b;
-  pair_of_factors(out->rule, out->pair % kPairs, &a, &b);
+  const bool usable = pair_of_factors(out->rule, pair % kPairs, &a, &b);
   out->sum = sum_form(a, b);
-  if (out->pair < kPairs) out->has |= 8;
+  if (usable && pair < kPairs) out->has |= 8;
 }
 __global__ __launch_bounds__(1024) void prepare_block_kernel(PrepareArgs p) {
   const int tid = threadIdx.x;
-  __shared__ int threshold[128], first;
+  __shared__ FormSearch search;
   BlockForms* const out = p.out;
   if (blockIdx.x < 3) {
     const int layer = blockIdx.x;
     if (p.prepared[layer] == nullptr) return;
     const EpiScalars s = *reinterpret_cast<const EpiScalars*>(p.prepared[layer]);
-    // the smallest accumulator of level tid, or the largest int where none reaches it
-    if (tid < 128) {
-      int lo = 0, hi = 0x7fffffff;  // level(lo) < tid, unless tid is 0
-      while (tid > 0 && hi - lo > 1) {
-        const int at = lo + (hi - lo) / 2;
-        (epi_requant(at, s, -127.0f) >= tid ? hi : lo) = at;
-      }
-      threshold[tid] = hi;
-    }
-    if (tid == 0) first = kFactors * kConstants;
-    __syncthreads();
-    const float unit = s.in_scale * s.qscale * (layer == 1 ? 1.0f : 2.0f);
-    if (unit > 1e-30f && unit < 1e30f) {
-      const float t = moved(unit, tid / kConstants), c = constant(tid % kConstants);
-      bool same = true;
-      for (int v = 1; v < 128 && same; ++v) {
-        const int a = threshold[v];
-        for (int d = 0; d < 2; ++d) {  // the definition gives v from a on (unless a is the end)
-          const bool reached = d == 0 && epi_requant(a, s, -127.0f) >= v;
-          const int level = layer == 1
-                                ? static_cast<int>(short_level(a - d, t) & 0xffu) - 128
-                                : static_cast<int>(short_relu4(a - d, 0, 0, 0, t, c) & 0xffu);
-          same = same && (level >= v) == reached;
-        }
-      }
-      if (same) atomicMin(&first, tid);
-    }
-    __syncthreads();
+    const LayerForm f = find_form(s, layer != 1, &search);
     if (tid == 0) {
-      const int at = first % (kFactors * kConstants);
       out->s[layer] = s;
-      out->t[layer] = moved(unit, at / kConstants);
-      out->c[layer] = constant(at % kConstants);
-      if (first < kFactors * kConstants) atomicOr(&out->has, 1 << layer);
+      out->t[layer] = f.t;
+      out->c[layer] = f.c;
+      if (f.has) atomicOr(&out->has, 1 << layer);
     }
   } else {
+    // a share of the operands' pairs each
     const RequantRule r = block_rule(p);
+    const int pair = (blockIdx.x - 3) / kShares, share = (blockIdx.x - 3) % kShares;
     float a, b;
-    if (!pair_of_factors(r, blockIdx.x - 3, &a, &b)) return;
+    if (!pair_of_factors(r, pair, &a, &b)) return;
     bool differs = false;
-    for (int i = tid; i < 64 * 256; i += 1024) {
+    for (int i = share * 1024 + tid; i < 64 * 256; i += 1024 * kShares) {
       const int a0 = 4 * (i >> 8) - 127, y0 = (i & 255) - 128;  // a0 ... a0 + 3
       int x[4];
       uint32_t packed = 0;
@@ -654,8 +596,7 @@ __global__ __launch_bounds__(1024) void prepare_block_kernel(PrepareArgs p) {
       differs |= short_sum4(x[0] + 128, x[1] + 128, x[2] + 128, x[3] + 128, y, sum_form(a, b)) !=
                  sum_requant4_general<true>(packed, y, r);
     }
-    if (__syncthreads_or(differs) == 0 && tid == 0)
-      atomicMin(&out->pair, static_cast<int>(blockIdx.x) - 3);
+    if (__syncthreads_or(differs) != 0 && tid == 0) atomicOr(&out->failed, 1ULL << pair);
   }
 }
 
@@ -869,7 +810,7 @@ int mxq_prepare_block(void* stream, const void* prepared_first, const void* prep
   hipStream_t s = static_cast<hipStream_t>(stream);
   hipLaunchKernelGGL(clear_forms_kernel, dim3(1), dim3(1), 0, s, a.out);
   MXQ_LAUNCH_CHECK();
-  hipLaunchKernelGGL(prepare_block_kernel, dim3(3 + kPairs), dim3(1024), 0, s, a);
+  hipLaunchKernelGGL(prepare_block_kernel, dim3(3 + kPairs * kShares), dim3(1024), 0, s, a);
   MXQ_LAUNCH_CHECK();
   hipLaunchKernelGGL(finish_forms_kernel, dim3(1), dim3(1), 0, s, a);
   MXQ_LAUNCH_CHECK();

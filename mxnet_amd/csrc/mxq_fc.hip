@@ -13,6 +13,7 @@
 #include "mxq_common.h"
 #include "mxq_fc_args.h"
 #include "mxq_few_tiles.h"
+#include "mxq_forms.h"
 #include "mxq_resident.h"
 #include "mxq_gemm.h"
 #include "mxq_tiles.h"
@@ -207,8 +208,29 @@ __global__ __launch_bounds__(1024) void sum_pairs_kernel(float layer_range,
 __global__ __launch_bounds__(256) void prepare_layer_kernel(Epilogue e, int N, char* out) {
   const EpiScalars s = epi_scalars(e);
   const int n = blockIdx.x * 256 + threadIdx.x;
-  if (n == 0) *reinterpret_cast<EpiScalars*>(out) = s;
+  if (n == 0) {
+    *reinterpret_cast<EpiScalars*>(out) = s;
+    *reinterpret_cast<LayerForms*>(out + kFormsAt) = LayerForms{0, 0.0f, 0.0f, 0.0f};
+  }
   if (n < N) reinterpret_cast<int*>(out + kPreparedBias)[n] = epi_bias32(e, s, n);
+}
+
+// The layer's short forms into what prepare_layer_kernel wrote: a work-group each.
+__global__ __launch_bounds__(1024) void prepare_forms_kernel(char* prepared) {
+  __shared__ FormSearch search;
+  const EpiScalars s = *reinterpret_cast<const EpiScalars*>(prepared);
+  const bool relu = blockIdx.x == 0;
+  const LayerForm f = find_form(s, relu, &search);
+  if (threadIdx.x == 0 && f.has) {
+    LayerForms* const out = reinterpret_cast<LayerForms*>(prepared + kFormsAt);
+    if (relu) {
+      out->t_relu = f.t;
+      out->c_relu = f.c;
+    } else {
+      out->t_plain = f.t;
+    }
+    atomicOr(&out->has, relu ? 1 : 2);
+  }
 }
 
 // an output without elements still owes its range scalars
@@ -539,6 +561,15 @@ int mxq_prepare_layer(void* stream, const int8_t* bias, int N, const float* min_
   e.real_range = (a < b) ? b : a;
   hipLaunchKernelGGL(prepare_layer_kernel, dim3(static_cast<unsigned>(N / 256 + 1)), dim3(256), 0,
                      static_cast<hipStream_t>(stream), e, N, static_cast<char*>(prepared));
+  MXQ_LAUNCH_CHECK();
+  MXQ_API_END();
+}
+
+int mxq_prepare_forms(void* stream, void* prepared) {
+  MXQ_API_BEGIN();
+  MXQ_CHECK(prepared != nullptr && aligned16(prepared), "null or unaligned pointer");
+  hipLaunchKernelGGL(prepare_forms_kernel, dim3(2), dim3(1024), 0, static_cast<hipStream_t>(stream),
+                     static_cast<char*>(prepared));
   MXQ_LAUNCH_CHECK();
   MXQ_API_END();
 }

@@ -28,6 +28,7 @@
 
 #include "../../include/mxq.h"
 #include "mxq_common.h"
+#include "mxq_forms.h"
 #include "mxq_resident.h"
 
 namespace mxq {
@@ -53,7 +54,7 @@ constexpr int kRing = 8192;  // bytes in LDS through which a wave's weights come
 
 // 4 waves, WN of them side by side, each on 32 rows and NI times 32 columns of a tile; NS tiles of
 // operand rows in LDS, two work-groups per CU.
-template <int KS, int WN, int NI, int NS, bool GATHER>
+template <int KS, int WN, int NI, int NS, bool GATHER, bool FORMS = false>
 __device__ __forceinline__ void resident(const Args& args, const ResidentArgs& p, int group) {
   constexpr int NW = 4, THREADS = 64 * NW, WM = NW / WN, TM = 32 * WM, TN = 32 * NI, NC = WN * TN;
   constexpr int K = 32 * KS, CH = 2 * KS;
@@ -73,7 +74,7 @@ __device__ __forceinline__ void resident(const Args& args, const ResidentArgs& p
   const int wm = wave / WN, wn = wave % WN, lrow = lane & 31, lgrp = lane >> 5;
   const int n0 = group * NC;
   const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(rows));
-  auto swizzle = [](int r) { return r & 15; };
+  auto swizzle = [](int r) { return CH == 4 ? (r >> 2) & 3 : r & 15; };
 
   // the rows' way into LDS: lane's slot (row, chunk) holds chunk ^ swizzle(row) of that row
   int m_next = blockIdx.x * TM;            // first row of the tile that is fetched next
@@ -158,17 +159,20 @@ __device__ __forceinline__ void resident(const Args& args, const ResidentArgs& p
   // columns of 256 bytes); whole lines go through LDS instead, 128 bytes of 32 columns at a time.
   v4i weight[NI][KS];
   {
-    constexpr int UNITS = NI * KS / 4;
+    // pieces of up to 128 bytes of 32 columns, a few instructions each
+    constexpr int STEPS = KS < 4 ? KS : 4, RC = 2 * STEPS, ASKS = RC / 2, PARTS = KS / STEPS;
+    constexpr int UNITS = NI * PARTS;
+    static_assert(UNITS >= 2, "both places of the ring");
     const v4i rsrc = make_rsrc(p.weight, static_cast<uint32_t>(p.N) * K);
     const int first = n0 + wn * TN;
     const uint32_t ring = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(shared)) + wave * kRing;
     const v4i* const held = reinterpret_cast<const v4i*>(shared + wave * kRing);
-    auto swz8 = [](int r) { return (r ^ (r >> 2)) & 7; };
+    auto mixed = [](int r) { return RC == 4 ? (r >> 2) & 3 : (r ^ (r >> 2)) & 7; };
     auto ask = [&](int u) {
-      const int ni = u / (KS / 4), part = u % (KS / 4);
+      const int ni = u / PARTS, part = u % PARTS;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int r = i * 8 + (lane >> 3), c = (lane & 7) ^ swz8(r);
+      for (int i = 0; i < ASKS; ++i) {
+        const int r = i * (64 / RC) + lane / RC, c = (lane % RC) ^ mixed(r);
         dma_buffer(__builtin_amdgcn_readfirstlane(ring + (u % 2) * 4096 + i * 1024),
                    static_cast<uint32_t>((first + ni * 32 + r) * K + part * 128 + c * 16), rsrc);
       }
@@ -178,13 +182,13 @@ __device__ __forceinline__ void resident(const Args& args, const ResidentArgs& p
 #pragma unroll
     for (int u = 0; u < UNITS; ++u) {
       if (u + 1 < UNITS)
-        wait_vmcnt<4>();
+        wait_vmcnt<ASKS>();
       else
         wait_vmcnt<0>();
 #pragma unroll
-      for (int k = 0; k < 4; ++k)
-        weight[u / (KS / 4)][u % (KS / 4) * 4 + k] =
-            held[(u % 2) * 256 + lrow * 8 + ((k * 2 + lgrp) ^ swz8(lrow))];
+      for (int k = 0; k < STEPS; ++k)
+        weight[u / PARTS][u % PARTS * STEPS + k] =
+            held[(u % 2) * 256 + lrow * RC + ((k * 2 + lgrp) ^ mixed(lrow))];
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       if (u + 2 < UNITS) ask(u + 2);
     }
@@ -204,7 +208,9 @@ __device__ __forceinline__ void resident(const Args& args, const ResidentArgs& p
     }
     asm volatile("" : "+v"(held_bias[ni]));
   }
-  auto run = [&](auto stream, auto relu) {
+  LayerForms forms = {};
+  if constexpr (FORMS) forms = *reinterpret_cast<const LayerForms*>(p.epi.prepared + kFormsAt);
+  auto run = [&](auto stream, auto relu, auto short_form) {
     int stage = 0, ahead = NS - 1, before = -1, parity = 0;
     for (int m0 = blockIdx.x * TM; m0 < p.M; m0 += m_step) {
       asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(S + (NS - 2) * (D + S))
@@ -228,9 +234,18 @@ __device__ __forceinline__ void resident(const Args& args, const ResidentArgs& p
       for (int ni = 0; ni < NI; ++ni)
 #pragma unroll
         for (int vq = 0; vq < 4; ++vq)
-          *reinterpret_cast<uint32_t*>(to + ni * 32 + 8 * vq) =
-              epi_requant_pack<decltype(relu)::value>(acc[ni][4 * vq], acc[ni][4 * vq + 1],
-                                                      acc[ni][4 * vq + 2], acc[ni][4 * vq + 3], s);
+        {
+          const int a0 = acc[ni][4 * vq], a1 = acc[ni][4 * vq + 1], a2 = acc[ni][4 * vq + 2],
+                    a3 = acc[ni][4 * vq + 3];
+          uint32_t w;
+          if constexpr (!decltype(short_form)::value)
+            w = epi_requant_pack<decltype(relu)::value>(a0, a1, a2, a3, s);
+          else if constexpr (decltype(relu)::value)
+            w = short_relu4(a0, a1, a2, a3, forms.t_relu, forms.c_relu);
+          else
+            w = short_plain4(a0, a1, a2, a3, forms.t_plain);
+          *reinterpret_cast<uint32_t*>(to + ni * 32 + 8 * vq) = w;
+        }
       before = m0;
       parity ^= 1;
       stage = stage + 1 == NS ? 0 : stage + 1;
@@ -239,13 +254,28 @@ __device__ __forceinline__ void resident(const Args& args, const ResidentArgs& p
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
     store(before, out + (parity ^ 1) * TM * LD, stream);
   };
-  if (p.epi.stream8) {
-    if (p.epi.relu) run(std::true_type(), std::true_type());
-    else run(std::true_type(), std::false_type());
-  } else {
-    if (p.epi.relu) run(std::false_type(), std::true_type());
-    else run(std::false_type(), std::false_type());
-  }
+  typedef std::true_type Yes;
+  typedef std::false_type No;
+  auto run_form = [&](auto stream) {
+    if constexpr (FORMS) {
+      if (p.epi.relu && (forms.has & 1)) {
+        run(stream, Yes(), Yes());
+        return;
+      }
+      if (!p.epi.relu && (forms.has & 2)) {
+        run(stream, No(), Yes());
+        return;
+      }
+    }
+    if (p.epi.relu)
+      run(stream, Yes(), No());
+    else
+      run(stream, No(), No());
+  };
+  if (p.epi.stream8)
+    run_form(Yes());
+  else
+    run_form(No());
   if (blockIdx.x == 0 && group == 0 && tid == 0) epilogue_ranges<kEpiPlain>(p.epi);
 }
 
@@ -254,18 +284,24 @@ __global__ __launch_bounds__(256, 2) void resident_kernel(Args args) {
   resident<KS, WN, NI, NS, GATHER>(args, args.r, blockIdx.y);
 }
 
-// Two layers over the same rows.
+// Two layers over the same rows: the stage starts of a network, whose first layer and projection read
+// the same tensor.  Their scales stay, so the requantize takes its short form where one was found
+// (mxq_forms.h): 4 instead of 7.75 vector instructions an output without a relu, 3.25 instead of
+// 6.7 with it.  Batch 64, us, two launches / one launch / with the short forms:
+//   200704 x 64 -> 64 and 256   27.0 / - / 20.0      50176 x 256 -> 128 and 512  26.2 / 24.0 / 19.3
+//   12544 x 512 -> 256 and 1024 26.6 / 20.4 / 18.3
 struct PairArgs {
   Args a;
   ResidentArgs b;
   int first;  // column groups of the first
 };
-template <int KS, int NS, bool GATHER>
+template <int KS, int WN, int NS, bool GATHER>
 __global__ __launch_bounds__(256, 2) void resident_pair_kernel(PairArgs args) {
   const bool second = static_cast<int>(blockIdx.y) >= args.first;
   ResidentArgs r = args.a.r;
   if (second) r = args.b;
-  resident<KS, 4, 2, NS, GATHER>(args.a, r, static_cast<int>(blockIdx.y) - (second ? args.first : 0));
+  resident<KS, WN, 2, NS, GATHER, true>(args.a, r,
+                                        static_cast<int>(blockIdx.y) - (second ? args.first : 0));
 }
 
 // Work-groups along the rows, and how a tile's images follow the one before.
@@ -297,15 +333,20 @@ void launch(hipStream_t s, Args& a) {
   MXQ_LAUNCH_CHECK();
 }
 
-template <int KS, int NS>
+// Columns of a work-group and rows of a tile of a pair.
+int pair_columns(int K) { return K == 64 ? 128 : 256; }
+int pair_rows(int K) { return K == 64 ? 64 : 32; }
+
+template <int KS, int WN, int NS>
 void launch_pair(hipStream_t s, PairArgs& p) {
-  const int first = (p.a.r.N + 255) / 256, ny = first + (p.b.N + 255) / 256;
-  const int gx = row_groups(p.a, 32, ny);
+  constexpr int NC = 64 * WN;
+  const int first = (p.a.r.N + NC - 1) / NC, ny = first + (p.b.N + NC - 1) / NC;
+  const int gx = row_groups(p.a, 128 / WN, ny);
   p.first = first;
   if (p.a.r.area != 0)
-    hipLaunchKernelGGL((resident_pair_kernel<KS, NS, true>), dim3(gx, ny), dim3(256), 0, s, p);
+    hipLaunchKernelGGL((resident_pair_kernel<KS, WN, NS, true>), dim3(gx, ny), dim3(256), 0, s, p);
   else
-    hipLaunchKernelGGL((resident_pair_kernel<KS, NS, false>), dim3(gx, ny), dim3(256), 0, s, p);
+    hipLaunchKernelGGL((resident_pair_kernel<KS, WN, NS, false>), dim3(gx, ny), dim3(256), 0, s, p);
   MXQ_LAUNCH_CHECK();
 }
 
@@ -313,7 +354,7 @@ bool takes(const ResidentArgs& a, bool aligned) {
   if (!aligned || a.epi.out8 == nullptr || a.epi.out32 != nullptr || a.epi.outf != nullptr ||
       a.epi.with_sum)
     return false;
-  if ((a.K != 256 && a.K != 512) || a.N % 16 != 0) return false;
+  if (a.N % 16 != 0) return false;
   if (static_cast<long long>(a.N) * a.K >= (1LL << 31) || a.ldo >= (1 << 24)) return false;
   if (a.area != 0) {
     // what quotient() and the offsets inside a tile hold
@@ -326,7 +367,7 @@ bool takes(const ResidentArgs& a, bool aligned) {
 }  // namespace
 
 bool resident_wins(const ResidentArgs& a, bool aligned) {
-  if (!takes(a, aligned)) return false;
+  if (!takes(a, aligned) || (a.K != 256 && a.K != 512)) return false;
   const int wide = a.K == 256 && a.N <= 64 ? 64 : a.N <= 128 ? 128 : 256;  // columns of a group
   const int high = wide == 64 ? 64 : 32;                                   // rows of a tile
   const long long groups = (a.N + wide - 1) / wide, tiles = (a.M + high - 1LL) / high * groups;
@@ -336,17 +377,20 @@ bool resident_wins(const ResidentArgs& a, bool aligned) {
 
 bool resident_pair_wins(const ResidentArgs& a, const ResidentArgs& b, bool aligned) {
   if (!takes(a, aligned) || !takes(b, aligned)) return false;
-  const long long groups = (a.N + 255) / 256 + (b.N + 255) / 256;
-  if (3 * (a.N + b.N) < 2 * groups * 256) return false;
-  return (a.M + 31LL) / 32 * groups >= (a.K == 256 ? 3 : 6) * num_cus();
+  if (a.K != 64 && a.K != 256 && a.K != 512) return false;
+  const int wide = pair_columns(a.K), high = pair_rows(a.K);
+  const long long groups = (a.N + wide - 1) / wide + (b.N + wide - 1) / wide;
+  if (3 * (a.N + b.N) < 2 * groups * wide) return false;
+  return (a.M + high - 1LL) / high * groups >= (a.K == 512 ? 6 : 3) * num_cus();
 }
 
 void launch_resident_pair(hipStream_t s, const ResidentArgs& a, const ResidentArgs& b) {
   PairArgs p = {};
   p.a.r = a;
   p.b = b;
-  if (a.K == 256) launch_pair<8, 4>(s, p);
-  else launch_pair<16, 3>(s, p);
+  if (a.K == 64) launch_pair<2, 2, 3>(s, p);
+  else if (a.K == 256) launch_pair<8, 4, 4>(s, p);
+  else launch_pair<16, 4, 3>(s, p);
 }
 
 void launch_resident(hipStream_t s, const ResidentArgs& r) {

@@ -9,16 +9,25 @@ from mxnet_amd._lib import check, lib
 pytestmark = pytest.mark.gpu
 
 
-def layer(o, c, seed):
+def layer(o, c, seed, forms):
     g = torch.Generator(device="cuda").manual_seed(seed)
     draw = lambda s: torch.randint(-127, 128, s, device="cuda", generator=g, dtype=torch.int8)
     weight, bias = draw((o, c)), draw((o,))
     ranges = [torch.tensor([v], device="cuda") for v in (-3.0, 2.5, -0.5, 0.75, -1.0, 1.0)]
     prepared = torch.empty(64 + 4 * o, dtype=torch.int8, device="cuda")
-    calib = (-20.0 - seed, 18.0)
     stream = torch.cuda.current_stream().cuda_stream
-    check(lib.mxq_prepare_layer(stream, bias.data_ptr(), o, *[r.data_ptr() for r in ranges], *calib,
-                                prepared.data_ptr()))
+    for step in range(20):
+        calib = (-20.0 - seed - 0.1 * step, 18.0)
+        check(lib.mxq_prepare_layer(stream, bias.data_ptr(), o, *[r.data_ptr() for r in ranges],
+                                    *calib, prepared.data_ptr()))
+        assert prepared[32:36].view(torch.int32).item() == 0
+        if not forms:
+            break
+        check(lib.mxq_prepare_forms(stream, prepared.data_ptr()))
+        if prepared[32:36].view(torch.int32).item() == 3:  # as for nine ranges out of ten
+            break
+    else:
+        pytest.fail("no short forms for any of these ranges")
     return weight, prepared, calib
 
 
@@ -30,13 +39,16 @@ SHAPES = [(1, 14, 14, 512, 256, 1024, 1), (1, 15, 13, 512, 272, 48, 2), (1, 7, 7
           (64, 14, 14, 1024, 512, 2048, 2), (31, 9, 11, 1040, 528, 1040, 1),  # 128 x 128 tiles
           (64, 56, 56, 256, 128, 512, 2), (64, 28, 28, 512, 256, 1024, 2),    # weights in registers
           (33, 57, 29, 256, 512, 144, 1), (50, 31, 33, 512, 240, 1008, 2),
-          (64, 56, 56, 64, 64, 256, 1)]                                   # two launches
+          (64, 56, 56, 64, 64, 256, 1), (65, 57, 55, 64, 48, 208, 1),         # ... of 64 bytes
+          (64, 16, 16, 64, 64, 256, 1), (80, 14, 15, 64, 64, 240, 1),
+          (64, 56, 56, 128, 64, 256, 1)]                                  # two launches
 
 
 @pytest.mark.parametrize("shape", SHAPES)
 @pytest.mark.parametrize("relu", [(1, 0), (0, 1)])
 @pytest.mark.parametrize("off", [0, 1])  # unaligned images: two launches
-def test_pair_is_two_convolutions(shape, relu, off):
+@pytest.mark.parametrize("forms", [False, True])
+def test_pair_is_two_convolutions(shape, relu, off, forms):
     n, h, w, c, o1, o2, s = shape
     if off and n > 5:
         pytest.skip("the fallback does not depend on the size")
@@ -44,7 +56,7 @@ def test_pair_is_two_convolutions(shape, relu, off):
     data = torch.randint(-127, 128, (n * h * w * c + 16,), device="cuda", dtype=torch.int8)
     data = data[off:off + n * h * w * c]
     stream = torch.cuda.current_stream().cuda_stream
-    layers, outs, wants = [layer(o1, c, 1), layer(o2, c, 2)], [], []
+    layers, outs, wants = [layer(o1, c, 1, forms), layer(o2, c, 2, forms)], [], []
     for (weight, prepared, calib), o, r in zip(layers, (o1, o2), relu):
         # a guard behind every output
         outs.append(torch.full((m * o + 64,), 77, dtype=torch.int8, device="cuda"))
