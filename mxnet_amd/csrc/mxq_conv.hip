@@ -1681,7 +1681,7 @@ void conv_pair(void* stream, const int8_t* data, int N, int H, int W, int C, int
     e.relu = l.relu;
     const float lo = fabsf(l.min_calib), hi = fabsf(l.max_calib);
     e.real_range = (lo < hi) ? hi : lo;
-    e.stream8 = epi_stream_rows(g.M);
+    e.stream8 = 0;  // the next launches read both: 608.8 us for a ResNet-50 at batch 64, 603.3 so
     return e;
   };
   const int M = static_cast<int>(g.M);
