@@ -402,6 +402,15 @@ int mxq_quantized_conv_pair_prepared(void* stream, const int8_t* data, int N, in
                                      const void* prepared2, int O2, int8_t* out2, int relu2,
                                      float min_calib2, float max_calib2);
 
+/* A 3 x 3 convolution of stride 1 and padding 1, prepared, over 256 channels and more (a multiple),
+ * with its weights [O][3][3][C] laid out beforehand. */
+int mxq_quantized_conv3x3_fits(int N, int H, int W, int C, int O);
+size_t mxq_quantized_conv3x3_weights(int C, int O);
+int mxq_pack_conv3x3_weights(void* stream, const int8_t* in, int C, int O, int8_t* out);
+int mxq_quantized_conv3x3(void* stream, const int8_t* data, const int8_t* weights,
+                          const void* prepared, int N, int H, int W, int C, int O, int8_t* out8,
+                          int relu);
+
 /* A stem: a 4 x 4 convolution of stride 1 over 16 channels, prepared, and the 3 x 3 maximum of
  * stride 2 and padding 1 behind it in one launch; out8 is [N][pooled_h][pooled_w][O]. */
 int mxq_quantized_conv_pool_fits(int N, int H, int W, int C, int O, int KH, int KW, int pad_h,

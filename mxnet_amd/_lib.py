@@ -74,6 +74,10 @@ SIGNATURES = {
     "mxq_quantized_fc_sum_prepared": (_i, [_p] * 4 + [_i] * 3 + [_p] * 4 + [_f] * 4 +
                                       [_i, _i, _p, _p, _sz]),
     "mxq_prepare_forms": (_i, [_p, _p]),
+    "mxq_quantized_conv3x3_fits": (_i, [_i] * 5),
+    "mxq_quantized_conv3x3_weights": (_sz, [_i] * 2),
+    "mxq_pack_conv3x3_weights": (_i, [_p, _p, _i, _i, _p]),
+    "mxq_quantized_conv3x3": (_i, [_p] * 4 + [_i] * 5 + [_p, _i]),
     "mxq_quantized_conv_pool_fits": (_i, [_i] * 11),
     "mxq_quantized_conv_pool": (_i, [_p] * 4 + [_i] * 11 + [_p, _i]),
     "mxq_quantized_conv_pair_fits": (_i, [_i] * 8),

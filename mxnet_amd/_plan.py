@@ -30,7 +30,7 @@ _FLAG_OF = {torch.float32: 0, torch.float64: 1, torch.float16: 2, torch.uint8: 3
 _SIZE_OF = {0: 4, 1: 8, 2: 2, 3: 1, 4: 4, 5: 1, 6: 8, 7: 1, 12: 2}
 _FLOAT32, _INT32, _INT8 = 0, 4, 5
 (_NODE, _CONV, _FC, _FC_F32, _FC_SUM, _FC_SUM_RQ, _QUANT_NHWC, _TO_NHWC, _FROM_NHWC, _POOL, _RELU,
- _ADD, _REQUANTIZE, _BLOCK, _PAIR, _CONV_POOL) = range(16)
+ _ADD, _REQUANTIZE, _BLOCK, _PAIR, _CONV_POOL, _CONV3) = range(17)
 _NULL, _ARENA, _HELD, _FEED, _OUTPUT = range(5)
 
 
@@ -727,6 +727,10 @@ class _Builder:
                 layers, blobs = blobs, None
                 places[5:7] = [self.prepared(columns, calib, [place(r) for r in refs], True)
                                for columns, calib, refs in layers]
+            if kind == _CONV3:
+                (columns, calib, refs), blobs = blobs, None
+                places[1] = self.conv3x3_weights(ints, place(refs[1]))
+                places[2] = self.prepared(columns, calib, [place(r) for r in refs], True)
             if kind == _CONV_POOL:
                 (columns, calib, refs), blobs = blobs, None
                 places[2] = self.prepared(columns, calib, [place(r) for r in refs])
@@ -750,8 +754,7 @@ class _Builder:
         self.fuse_stem(users, gone)
         self.fuse_blocks(users, gone)
         self.pair_convs(gone)
-        if not gone:
-            return
+        self.single_convs(gone)
         self.steps = [s for at, s in enumerate(self.steps) if at not in gone]
         for b in self.buffers:
             b.first = b.last = None
@@ -836,6 +839,27 @@ class _Builder:
                               [(geo[4], calib, refs), (geo2[4], calib2, refs2)])
             gone.add(j)
             del first[id(refs2[0])]
+
+    def single_convs(self, gone):
+        """3 x 3 convolutions that are left on their own and have a kernel for that."""
+        for at, (kind, geo, calib, refs, _, _) in enumerate(self.steps):
+            if (kind == _CONV and at not in gone and geo[5:13] == (3, 3, 1, 1, 1, 1, 1, 1) and
+                    self.stays(refs) and _lib.lib.mxq_quantized_conv3x3_fits(*geo[:5])):
+                self.steps[at] = (_CONV3, geo[:5] + (geo[13],), (), [refs[0], None, None, refs[10]],
+                                  None, (geo[4], calib, refs))
+
+    def conv3x3_weights(self, ints, at):
+        what, names = self.origin[at[1]]
+
+        def make():
+            out = torch.empty(int(_lib.lib.mxq_quantized_conv3x3_weights(*ints[3:5])),
+                              dtype=torch.int8, device=self.device)
+            _lib.check(_lib.lib.mxq_pack_conv3x3_weights(
+                self.stream, self.held[at[1]].data_ptr(), int(ints[3]), int(ints[4]),
+                out.data_ptr()))
+            return out
+
+        return self.laid(("conv3x3", what), names, make).place
 
     @staticmethod
     def stays(refs):

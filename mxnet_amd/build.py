@@ -11,7 +11,7 @@ HIP_SOURCES = ["mxq_capi.hip", "mxq_cast.hip", "mxq_fc.hip", "mxq_fc_plain.hip",
                "mxq_fc_sum.hip", "mxq_fc_sum_requant.hip", "mxq_conv.hip", "mxq_conv_nchw.hip", "mxq_pool.hip",
                "mxq_eltwise.hip", "mxq_layout.hip", "mxq_histogram.hip",
                "mxq_nhwc.hip", "mxq_few_tiles.hip", "mxq_block.hip",
-               "mxq_entropy.hip", "mxq_resident.hip", "mxq_stem.hip"]
+               "mxq_entropy.hip", "mxq_resident.hip", "mxq_stem.hip", "mxq_conv3x3.hip"]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",

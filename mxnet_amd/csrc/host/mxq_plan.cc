@@ -138,6 +138,10 @@ bool Plan::run(void* stream, const std::vector<at::Tensor>& feeds,
         rc = mxq_quantized_conv_pool(stream, q(0), q(1), p(2), i(0), i(1), i(2), i(3), i(4), i(5),
                                      i(6), i(7), i(8), i(9), i(10), q(3), i(11));
         break;
+      case Kind::kConv3x3:  // refs: data, weights, what mxq_prepare_layer made, output
+        rc = mxq_quantized_conv3x3(stream, q(0), q(1), p(2), i(0), i(1), i(2), i(3), i(4), q(3),
+                                   i(5));
+        break;
       case Kind::kRequantize:
         rc = mxq_requantize(stream, static_cast<int32_t*>(p(0)), v(2), v(3), q(1), v(4), v(4) + 1,
                             static_cast<size_t>(n[0]), 1, f[0], f[1], nullptr, 0);

@@ -45,6 +45,7 @@ enum class Kind : int {
   kBlock,        // 3 x 3 convolution -> 1 x 1 -> sum (-> 1 x 1), each requantized
   kConvPair,     // two 1 x 1 convolutions of one tensor, each requantized (-> relu)
   kConvPool,     // 4 x 4 convolution, requantized (-> relu) -> 3 x 3 maximum
+  kConv3x3,      // 3 x 3 convolution over many channels, requantized (-> relu)
 };
 
 struct Step {
