@@ -114,7 +114,9 @@ extern "C" int mxq_histogram_f32(void* stream, const float* in, size_t n, const 
   const size_t cap = static_cast<size_t>(num_cus()) * (bins <= kMaxLdsBins / 2 ? 2 : 1);
   if (grid > cap) grid = cap;
   if (lds)
-    hipLaunchKernelGGL((histogram_kernel<true>), dim3(static_cast<unsigned>(grid)), dim3(kCountThreads), (2 * static_cast<size_t>(bins) + 1) * sizeof(uint32_t), s, in, n,
+    hipLaunchKernelGGL((histogram_kernel<true>), dim3(static_cast<unsigned>(grid)),
+                       dim3(kCountThreads),
+                       (2 * static_cast<size_t>(bins) + 1) * sizeof(uint32_t), s, in, n,
                        edges, bins, counts);
   else
     hipLaunchKernelGGL((histogram_kernel<false>), dim3(static_cast<unsigned>(grid)),

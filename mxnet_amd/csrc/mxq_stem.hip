@@ -11,14 +11,16 @@
 // of a 32 x 32 product that lane group g keeps in register v is pixel 14 g + v, and a row's
 // horizontal maxima are seven v_max3 on the lane's own registers.  Pixels outside the image repeat
 // the window's nearest one, which a maximum does not notice.  A convolution row shares three of its
-// four input rows with the one above: fragments of eight input rows live in registers, four of them
-// on their way; weights and bias stay there too.  No LDS but for the pooled bytes' transposition, no
-// barrier.
+// four input rows with the one above, so a wave sends each input row to a ring of seven slots of
+// its own in LDS once, four of them on their way, and reads its fragments from there; weights and
+// bias stay in registers.  No barrier: nothing but a wave's own rows and the transposition of its
+// pooled bytes goes through LDS.
 //
-// Batch 64, 224 x 224, 3 -> 64 channels: 20.6 us, where the two launches took 27.7 and 15.4.  A third
-// of it stays without the products and the requantization: a row is a chain of waiting, reading LDS
-// and sending for the next, and two waves a SIMD (the weights of 64 channels in registers) cover
-// half of it; one group of 32 channels per wave reads the input twice and is level.
+// Batch 64, 224 x 224, 3 -> 64 channels: 20.6 us, where the two launches took 27.7 and 15.4.  A
+// third of it stays without the products and the requantization: a row is a chain of waiting,
+// reading LDS and sending for the next, and two waves a SIMD (the weights of 64 channels in
+// registers) cover half of it; one group of 32 channels per wave reads the input twice and is
+// level.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
