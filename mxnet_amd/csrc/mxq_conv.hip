@@ -272,8 +272,10 @@ __global__ __launch_bounds__(Cfg::kThreads, Cfg::kMinWaves) void conv_pair_kerne
 // transposed through the patch row that has just become dead.  No barrier per K step,
 // every input row is fetched (R + 2) / R times instead of nine, and with two waves per SIMD
 // one wave's fetch and epilogue overlap the other's MFMAs.  int8 output with the fused
-// requantize only (the form the quantized graph runs with a calibrated convolution);
-// everything else takes the tiled kernels.
+// requantize (the form the quantized graph runs with a calibrated convolution), or the operator's
+// int32 planes: a register holds 32 consecutive pixels of one channel then, which leave as they
+// are, 128 bytes a channel (56 x 56 at batch 64 26.6 -> 21.1 us, the tiled kernel before).
+// Other outputs take the tiled kernels.
 constexpr int kRowsC = 64;        // input channels = bytes per pixel
 constexpr int kRowsO = 64;        // output channels
 constexpr int kRowsPitch = 60;    // patch pixels per row
@@ -284,7 +286,8 @@ constexpr int kRowsWaves = 8;
 // pitch 64 bytes) over the banks for the column-wise writes and the row-wise reads alike
 __device__ __forceinline__ int tile_swz(int row) { return (row ^ (row >> 2)) & 3; }
 
-template <int R>
+// PLANES: int32 planes instead of int8 pixels
+template <int R, bool PLANES>
 __global__ __launch_bounds__(64 * kRowsWaves, 1) void conv3x3_rows_kernel(ConvArgs p) {
   constexpr int CH = kRowsC / 16;                       // 16-byte chunks per pixel
   constexpr int kPatchPixels = (R + 2) * kRowsPitch;
@@ -395,6 +398,30 @@ __global__ __launch_bounds__(64 * kRowsWaves, 1) void conv3x3_rows_kernel(ConvAr
                 acc[mi][ni] =
                     __builtin_amdgcn_mfma_i32_32x32x32_i8(fb[ni], fa[mi], acc[mi][ni], 0, 0, 0);
           }
+      if constexpr (PLANES) {
+        // (the products' wait states stand here: none behind the masks of the stores)
+        asm volatile("s_nop 15\n\ts_nop 15"
+                     : "+v"(acc[0][0]), "+v"(acc[0][1]), "+v"(acc[1][0]), "+v"(acc[1][1]));
+        const int plane = p.OH * p.OW;
+        const auto image = __builtin_amdgcn_make_buffer_rsrc(
+            p.epi.out32 + static_cast<size_t>(n) * kRowsO * plane, 0, kRowsO * plane * 4,
+            0x00020000);
+#pragma unroll
+        for (int mi = 0; mi < 2; ++mi) {
+          const int px = mi * 32 + lrow;
+          // past the end of the row: dropped
+          const uint32_t at = px < p.OW ? ((oh0 + r) * p.OW + px + 4 * lgrp * plane) * 4u
+                                        : kOutOfRange;
+#pragma unroll
+          for (int ni = 0; ni < 2; ++ni)
+#pragma unroll
+            for (int v = 0; v < 16; ++v)
+              __builtin_amdgcn_raw_buffer_store_b32(
+                  static_cast<uint32_t>(acc[mi][ni][v]), image, at,
+                  (ni * 32 + 8 * (v / 4) + v % 4) * plane * 4, 0);
+        }
+        continue;
+      }
       // patch row r is dead now (output row r + 1 starts at patch row r + 1): the int8 tile
       // of up to 58 pixels x 64 channels is transposed through it, 64 bytes per pixel
       char* stage = reinterpret_cast<char*>(patch + r * kRowsPitch * CH);
@@ -455,8 +482,11 @@ bool conv3x3_rows_ok(const ConvArgs& a) {
   const long long data_bytes = static_cast<long long>(a.N) * a.H * a.W * a.C;
   return a.KH == 3 && a.KW == 3 && a.sh == 1 && a.sw == 1 && a.ph == 1 && a.pw == 1 &&
          a.dh == 1 && a.dw == 1 && a.C == kRowsC && a.O == kRowsO && a.W <= kRowsMaxW &&
-         a.epi.out32 == nullptr && a.epi.out8 != nullptr && aligned16(a.data) &&
-         aligned16(a.weight) && aligned16(a.epi.out8) && data_bytes < (1LL << 31);
+         aligned16(a.data) && aligned16(a.weight) && data_bytes < (1LL << 31) &&
+         (a.epi.out32 == nullptr
+              ? a.epi.out8 != nullptr && aligned16(a.epi.out8)
+              : a.epi.out8 == nullptr && a.epi.plane > 0 &&
+                    4LL * kRowsO * a.OH * a.OW < (1LL << 31));
 }
 
 void launch_conv3x3_rows(hipStream_t s, const ConvArgs& a) {
@@ -468,12 +498,10 @@ void launch_conv3x3_rows(hipStream_t s, const ConvArgs& a) {
   const long items = two ? items2 : static_cast<long>(a.N) * a.OH;
   long grid = (items + kRowsWaves - 1) / kRowsWaves;
   if (grid > cus) grid = cus;
-  if (two)
-    hipLaunchKernelGGL(conv3x3_rows_kernel<2>, dim3(static_cast<unsigned>(grid)),
-                       dim3(64 * kRowsWaves), 0, s, a);
-  else
-    hipLaunchKernelGGL(conv3x3_rows_kernel<1>, dim3(static_cast<unsigned>(grid)),
-                       dim3(64 * kRowsWaves), 0, s, a);
+  const auto kernel = a.epi.out32 != nullptr
+                          ? (two ? conv3x3_rows_kernel<2, true> : conv3x3_rows_kernel<1, true>)
+                          : (two ? conv3x3_rows_kernel<2, false> : conv3x3_rows_kernel<1, false>);
+  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(64 * kRowsWaves), 0, s, a);
   MXQ_LAUNCH_CHECK();
 }
 
@@ -1546,9 +1574,15 @@ void conv_nhwc(void* stream, const int8_t* data, const int8_t* weight, const int
     plan = plan_conv(g, aligned, unsplit);
   }
   // 61: the parked-weights row kernel (3 x 3 over 64 -> 64 channels, fused int8 output);
-  // chosen for it whenever the launch has rows for every wave of the chip
-  if (plan.cfg == 61 || (force.cfg == 0 && conv3x3_rows_ok(a) &&
-                         static_cast<long>(a.N) * a.OH >= 1L * kRowsWaves * num_cus())) {
+  // chosen for it whenever the launch has rows for every wave of the chip; with int32 planes from
+  // three rows a CU on, as the tiled kernel has the wider output to move through LDS (us, tiled and
+  // here, 56 x 56: 448 rows 7.6 / 8.4, 896 11.4 / 9.3, 1344 13.4 / 10.4, 3584 26.6 / 21.1), but
+  // not for short rows, whose products are mostly padding (28 wide, 1792 rows 11.3 / 9.7, 17 wide,
+  // 2624 rows 10.0 / 12.5, 14 wide, 3584 rows 11.0 / 13.1)
+  const bool planes = a.epi.out32 != nullptr;
+  if (plan.cfg == 61 || (force.cfg == 0 && conv3x3_rows_ok(a) && (!planes || a.W >= 24) &&
+                         static_cast<long>(a.N) * a.OH >=
+                             (planes ? 3L : 1L * kRowsWaves) * num_cus())) {
     MXQ_CHECK(conv3x3_rows_ok(a), "shape does not qualify for the parked-weights 3x3 kernel");
     MXQ_CHECK(plan.splits <= 1 || force.splits == 0, "the 3x3 row kernel has no split-K form");
     launch_conv3x3_rows(s, a);
