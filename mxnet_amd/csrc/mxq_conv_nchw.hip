@@ -768,6 +768,7 @@ struct NchwPlan {
   // NHWC view of the adapter routes
   int vC;
   int gather_mode;         // kPlanesGather: how the loader fetches a group's four pixels
+  bool loader_too;         // kPlanesPrepass: kPlanesGather does it as well, without a workspace
   int pitch, row_stride;   // kPlanesPrepass: columns per image and bytes per channel row
   bool weight_in_place;    // 1 x 1 window over C % 16 == 0 channels: OIHW is OHWI already
   size_t d_bytes, w_bytes, split_bytes;
@@ -807,7 +808,14 @@ NchwPlan plan_nchw(int N, int C, int H, int W, int O, int KH, int KW, int sh, in
     const int plane_in = H * W;
     const long long pitch = (P + 3) / 4 * 4, row = (1LL * N * pitch + 15) / 16 * 16;
     const bool prepass_ok = P < kGatherMaxPlane && 1LL * C * row < (1LL << 31);
-    const bool light = 1LL * O * C <= 256 * 1024 || !prepass_ok;
+    // Four channel tiles and more fetch the pixels that often, one stage ahead: with enough of
+    // them the ring wins there too (us, loader and ring: 256 -> 512 / 2 at 56 x 56 50.1 / 42.5,
+    // 256 -> 1024 / 2 99.5 / 68.8, 128 -> 512 / 2 38.4 / 32.0, 512 -> 512 / 2 at 28 x 28 25.9 /
+    // 20.9, 256 -> 512 / 2 17.3 / 16.2 and for 16 images, 3136 pixels, 7.2 / 8.6; 256 -> 384 / 2
+    // at 56 x 56 47.5 / 47.1, 64 -> 512 / 2 28.3 / 28.4).
+    const bool few_weights = 1LL * O * C <= 256 * 1024;
+    const bool many_tiles = O >= 512 && C >= 128 && 1LL * N * P >= 12 * 1024;
+    const bool light = (few_weights && !many_tiles) || !prepass_ok;
     int mode = kGatherBytes;
     if (sw == 2 && pl.OW % 4 == 0 && (sh * W) % 8 == 0 && plane_in % 8 == 0 && 2 * pl.OW <= W)
       mode = kGatherPair;
@@ -822,6 +830,8 @@ NchwPlan plan_nchw(int N, int C, int H, int W, int O, int KH, int KW, int sh, in
     // whose kernel has the deeper stages: 2048 -> 512 at 7 x 7 24.8 against 21.6 us)
     if (!(C >= 2048 && 1LL * N * P <= 4096)) {
       pl.route = Route::kPlanesPrepass;
+      pl.gather_mode = mode;
+      pl.loader_too = mode != kGatherBytes && few_weights;
       pl.pitch = static_cast<int>(pitch);
       pl.row_stride = static_cast<int>(row);
       pl.d_bytes = up256(static_cast<size_t>(C) * row);
@@ -890,6 +900,11 @@ void conv_nchw(void* stream, const int8_t* data, const int8_t* weight, const int
   // cfg 1 pins the adapter route; 71.. pin a tile of the NCHW kernel
   const bool aligned = aligned16(data) && aligned16(weight) && cfg != 1;
   NchwPlan pl = plan_nchw(N, C, H, W, O, KH, KW, sh, sw, ph, pw, dh, dw, aligned);
+  if (pl.loader_too && (workspace == nullptr || !aligned16(workspace) ||
+                        workspace_bytes < pl.d_bytes)) {
+    pl.route = Route::kPlanesGather;
+    pl.d_bytes = 0;
+  }
   const bool planes_route = pl.route == Route::kPlanes || pl.route == Route::kPlanesGather ||
                             pl.route == Route::kPlanesPrepass;
   MXQ_CHECK(cfg < 70 || planes_route,
@@ -970,6 +985,11 @@ void conv_nchw(void* stream, const int8_t* data, const int8_t* weight, const int
         if (pick == 73 && C >= 1024 && pl.route == Route::kPlanes && a.pitch != 0) pick = 84;
       }
     }
+    // Gathered planes of half a thousand pixels and more take the 128 x 128 tile (us, 256 x 128 and
+    // 128 x 128, 28 x 28 out: 256 -> 512 45.4 / 42.5, 512 -> 512 58.2 / 54.5; 29 x 29: 60.0 / 52.7;
+    // 128 x 64 is level with it alone, in a ResNet-50 pass ahead or 5 us behind by card), smaller
+    // ones don't (14 x 14: 512 -> 1024 98.1 / 98.6; 7 x 7: 512 -> 2048 183.5 / 186.9)
+    if (cfg < 70 && pl.route == Route::kPlanesPrepass && pick == 77 && a.P >= 512) pick = 71;
     switch (pick) {
       case 71: launch_planes<PlaneM>(s, a, gm); break;
       case 72: launch_planes<PlaneN64>(s, a, gm); break;

@@ -16,7 +16,9 @@ pytestmark = pytest.mark.gpu
                                    (70, 16, 1, 5, 16, 1, 3), (33, 32, 5, 1, 16, 2, 1),
                                    (130, 16, 1, 1, 64, 1, 1), (1, 32, 181, 181, 16, 2, 2),
                                    (2, 16, 40, 51, 32, 3, 2), (1, 16, 128, 256, 16, 1, 3),
-                                   (1, 16, 129, 256, 16, 1, 3), (9, 96, 3, 3, 16, 1, 1)])
+                                   (1, 16, 129, 256, 16, 1, 3), (9, 96, 3, 3, 16, 1, 1),
+                                   (64, 128, 28, 28, 512, 2, 2), (16, 256, 57, 57, 528, 2, 2),
+                                   (25, 272, 46, 46, 512, 2, 2)])
 def test_integers_of_the_general_path(shape):
     n, c, h, w, o, sh, sw = shape
     oh, ow = (h - 1) // sh + 1, (w - 1) // sw + 1
@@ -36,5 +38,26 @@ def test_integers_of_the_general_path(shape):
             1, *[r.data_ptr() for r in ranges], None, None, out.data_ptr(), span.data_ptr(),
             span.data_ptr() + 4, space.data_ptr(), need, cfg))
         assert (space[need:] == 55).all()
+        outs.append(out)
+    assert torch.equal(*outs)
+
+
+def test_many_tiles_without_a_workspace():
+    """Layers that gather beforehand only because it is faster do without the room for it."""
+    n, c, h, o = 64, 128, 28, 512
+    data = torch.randint(-127, 128, (n, c, h, h), device="cuda", dtype=torch.int8)
+    weight = torch.randint(-127, 128, (o, c, 1, 1), device="cuda", dtype=torch.int8)
+    ranges = [torch.tensor([v], device="cuda") for v in (-3.0, 2.5, -0.5, 0.75)]
+    span = torch.empty(2, device="cuda")
+    need = lib.mxq_quantized_conv_nchw_workspace(n, c, h, h, o, 1, 1, 2, 2, 0, 0, 1, 1, 1)
+    space, outs = torch.empty(need, dtype=torch.int8, device="cuda"), []
+    assert need >= n * c * (h // 2) ** 2
+    for room in (need, 0):
+        out = torch.full((n, o, h // 2, h // 2), 77, dtype=torch.int32, device="cuda")
+        check(lib.mxq_quantized_conv_nchw(
+            torch.cuda.current_stream().cuda_stream, data.data_ptr(), weight.data_ptr(), None, n, c,
+            h, h, o, 1, 1, 2, 2, 0, 0, 1, 1, *[r.data_ptr() for r in ranges], None, None,
+            out.data_ptr(), span.data_ptr(), span.data_ptr() + 4,
+            space.data_ptr() if room else None, room))
         outs.append(out)
     assert torch.equal(*outs)
