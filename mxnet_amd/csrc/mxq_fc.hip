@@ -279,7 +279,7 @@ void launch_fc(hipStream_t s, const int8_t* data, const int8_t* weight, int M, i
       return;
     }
   }
-  if (force.cfg == 0) {
+  if (force.cfg == 0 && (K == 256 || K == 512)) {  // its reductions
     ResidentArgs r = {};
     r.data = data;
     r.weight = weight;
