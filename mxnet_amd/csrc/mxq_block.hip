@@ -751,8 +751,12 @@ extern "C" {
 // 1.1 MB of weights that a CU takes in: 19 tiles (14 x 14 x 256 on 3 images) 15.6 us against 16.0,
 // 25 tiles 15.6 against 16.5, 98 of 32 pixels 16.6 against 23.3, 196 of 64 22.0 against 38.3.
 int mxq_quantized_block_fits(int N, int H, int W, int C, int C_mid, int C_out, int C_next) {
-  const BlockPlan b = plan_block(N, H, W, C, C_mid, C_out, C_next);
-  return b.tiles > 0 && (b.variant < 256 || b.tiles >= 20) ? 1 : 0;
+  try {
+    const BlockPlan b = plan_block(N, H, W, C, C_mid, C_out, C_next);
+    return b.tiles > 0 && (b.variant < 256 || b.tiles >= 20) ? 1 : 0;
+  } catch (...) {  // no device to ask
+    return 0;
+  }
 }
 
 size_t mxq_quantized_block_weights(int C, int C_mid, int C_out, int C_next) {

@@ -250,7 +250,11 @@ int mxq_quantized_conv3x3_fits(int N, int H, int W, int C, int O) {
   if (!conv3x3_ok(N, H, W, C, O) || O < 64) return 0;
   const long long rows = (1LL * N * H * W + kRows - 1) / kRows;
   const long long groups = rows * ((O + kColumns - 1) / kColumns);
-  return 6 * groups >= num_cus() && groups <= 2 * num_cus();
+  try {
+    return 6 * groups >= num_cus() && groups <= 2 * num_cus();
+  } catch (...) {  // no device to ask
+    return 0;
+  }
 }
 
 size_t mxq_quantized_conv3x3_weights(int C, int O) {

@@ -75,6 +75,20 @@ def test_argument_validation_needs_no_gpu():
     assert lib.mxq_dequantize(None, None, 5, p, p, None, 0) == 0
 
 
+def test_rules_that_ask_for_the_device_answer_without_one():
+    """A query whose rule counts compute units says no where there is no device, like the other
+    queries: an exception must not leave a C entry point."""
+    import subprocess
+    import sys
+    program = ("from mxnet_amd._lib import lib\n"
+               "print(lib.mxq_quantized_block_fits(1, 56, 56, 64, 64, 256, 64),"
+               " lib.mxq_quantized_conv3x3_fits(64, 7, 7, 512, 512),"
+               " lib.mxq_quantized_conv_pair_fits(64, 56, 56, 256, 128, 512, 2, 2))")
+    r = subprocess.run([sys.executable, "-c", program], cwd=ROOT, capture_output=True, text=True,
+                       timeout=240, env=dict(os.environ, HIP_VISIBLE_DEVICES="-1"))
+    assert (r.returncode, r.stdout.split()) == (0, ["0", "0", "0"]), r.stderr
+
+
 def test_no_fallback_without_library(tmp_path, monkeypatch):
     """The package refuses to import when the HIP library is missing."""
     import importlib.util
