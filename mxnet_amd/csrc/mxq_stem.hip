@@ -276,6 +276,8 @@ bool conv_pool_ok(int N, int H, int W, int C, int O, int KH, int KW, int ph, int
   if (OH <= 0 || OW <= 0 || 1LL * H * W * 16 >= (1LL << 31)) return false;
   // every window holds a pixel
   if (2LL * (PH - 1) - 1 >= OH || 2LL * (PW - 1) - 1 >= OW) return false;
+  // offsets in a pooled row, the one that drops a store behind all of them
+  if (1LL * PW * O >= (1LL << 31)) return false;
   return 1LL * N * ((PW + kColumns - 1) / kColumns) * PH < (1LL << 29);
 }
 

@@ -4,7 +4,7 @@ import threading
 import pytest
 import torch
 
-from mxnet_amd import _frontend, contrib, operator
+from mxnet_amd import _frontend, _lib, contrib, operator
 from mxnet_amd import symbol as S
 from mxnet_amd.executor import Executor, _Graph
 
@@ -114,3 +114,14 @@ def test_threads_share_a_graphs_nodes():
     ex.symbol = S.Activation(ex.symbol, act_type="relu", name="r")
     assert torch.equal(ex.forward(data=-x)[0], torch.relu(ex.params["f_bias"] + 1 - want))
     assert ex._structure() is not before and before.symbol is not ex.symbol
+
+
+# image columns (padded by 7 on either side), channels, pooled columns
+@pytest.mark.parametrize("w,o,pw,fits", [(2 ** 22 - 12, 1008, 2 ** 21, True),
+                                         (2 ** 22 - 13, 1024, 2 ** 21 - 1, True),
+                                         (2 ** 22 - 12, 1024, 2 ** 21, False),
+                                         (2 ** 23, 1024, 2 ** 22, False)])
+def test_stem_offsets_of_a_pooled_row(w, o, pw, fits):
+    """A lane stores at an offset of 32 bits in its pooled row, and one that has nothing to store at
+    2^31, which the row must not reach."""
+    assert _lib.lib.mxq_quantized_conv_pool_fits(1, 1, w, 16, o, 4, 4, 2, 7, 1, pw) == fits
