@@ -278,7 +278,9 @@ bool conv_pool_ok(int N, int H, int W, int C, int O, int KH, int KW, int ph, int
   if (2LL * (PH - 1) - 1 >= OH || 2LL * (PW - 1) - 1 >= OW) return false;
   // offsets in a pooled row, the one that drops a store behind all of them
   if (1LL * PW * O >= (1LL << 31)) return false;
-  return 1LL * N * ((PW + kColumns - 1) / kColumns) * PH < (1LL << 29);
+  // two waves a SIMD in bands, or a wave for each strip of every image: 2^32 lanes are a launch's
+  const long long strips = 1LL * N * ((PW + kColumns - 1) / kColumns);
+  return strips < (1LL << 26) - 4 && strips * PH < (1LL << 29);
 }
 
 }  // namespace

@@ -125,3 +125,9 @@ def test_stem_offsets_of_a_pooled_row(w, o, pw, fits):
     """A lane stores at an offset of 32 bits in its pooled row, and one that has nothing to store at
     2^31, which the row must not reach."""
     assert _lib.lib.mxq_quantized_conv_pool_fits(1, 1, w, 16, o, 4, 4, 2, 7, 1, pw) == fits
+
+
+@pytest.mark.parametrize("n,fits", [(2 ** 26 - 5, True), (2 ** 26 - 4, False), (2 ** 27, False)])
+def test_stem_lanes_of_a_launch(n, fits):
+    """A wave for each image of one strip: a launch has less than 2^32 lanes."""
+    assert _lib.lib.mxq_quantized_conv_pool_fits(n, 1, 1, 16, 16, 4, 4, 2, 2, 1, 1) == fits
