@@ -273,7 +273,8 @@ bool conv_pool_ok(int N, int H, int W, int C, int O, int KH, int KW, int ph, int
   if (N <= 0 || C != 16 || KH != 4 || KW != 4 || O <= 0 || O % 16 != 0 || O > 1024) return false;
   if (ph < 0 || pw < 0 || PH <= 0 || PW <= 0) return false;
   const long long OH = 1LL * H + 2 * ph - 3, OW = 1LL * W + 2 * pw - 3;
-  if (OH <= 0 || OW <= 0 || 1LL * H * W * 16 >= (1LL << 31)) return false;
+  if (OH <= 0 || OW <= 0 || OH >= (1LL << 31) || OW >= (1LL << 31)) return false;
+  if (1LL * H * W * 16 >= (1LL << 31)) return false;
   // every window holds a pixel
   if (2LL * (PH - 1) - 1 >= OH || 2LL * (PW - 1) - 1 >= OW) return false;
   // offsets in a pooled row, the one that drops a store behind all of them

@@ -131,3 +131,11 @@ def test_stem_offsets_of_a_pooled_row(w, o, pw, fits):
 def test_stem_lanes_of_a_launch(n, fits):
     """A wave for each image of one strip: a launch has less than 2^32 lanes."""
     assert _lib.lib.mxq_quantized_conv_pool_fits(n, 1, 1, 16, 16, 4, 4, 2, 2, 1, 1) == fits
+
+
+@pytest.mark.parametrize("pad,fits", [(2 ** 30, True), (2 ** 30 + 1, False), (2 ** 31 - 1, False)])
+def test_stem_extent_of_a_padded_image(pad, fits):
+    """The convolution's extents are ints: 1 + 2 * pad - 3 of them."""
+    args = [1, 1, 1, 16, 16, 4, 4, 2, 2, 1, 1]
+    for axis in (7, 8):
+        assert _lib.lib.mxq_quantized_conv_pool_fits(*args[:axis], pad, *args[axis + 1:]) == fits
