@@ -179,7 +179,10 @@ def _entropy_bounds(hists, levels):
             return None
         if not (h.min() >= 0 and h.sum(dtype=np.float64) < 2 ** 31):  # neither for a NaN
             return None
-    return capi.entropy_bounds(hists, levels)
+    try:
+        return capi.entropy_bounds(hists, levels)
+    except torch.cuda.OutOfMemoryError:  # a float per candidate and level, up to 0.5 GB a histogram
+        return None
 
 
 def _calibrate_entropy_many(problems):

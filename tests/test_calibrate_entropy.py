@@ -11,6 +11,7 @@ import numpy as np
 import pytest
 
 from mxnet_amd import quantization as Q
+from mxnet_amd._lib import MXQError
 
 f32 = np.float32
 _libm = ctypes.CDLL(ctypes.util.find_library("m"))
@@ -107,3 +108,26 @@ def test_entropy_search_without_memory_for_a_threads_scratch(tmp_path):
     env = dict(os.environ, OMP_NUM_THREADS="4")
     run = subprocess.run([program], env=env, capture_output=True, timeout=60, text=True)
     assert run.returncode == 0, (run.returncode, run.stdout, run.stderr)
+
+
+def test_entropy_search_without_device_memory_for_the_bounds(monkeypatch):
+    """Histograms of the host need no device: where the bounds find no memory there the host's own
+    do, and any other error is reported."""
+    hist = np.histogram(np.random.default_rng(3).standard_normal(5000), bins=401, range=(-4, 4))[0]
+    problem = hist, np.linspace(-4, 4, 402), 63
+    want = Q.calibrate_entropy(*problem)
+    raised = []
+
+    def bounds(hists, levels):
+        raised.append(kind)
+        raise kind("of the device")
+
+    monkeypatch.setattr(Q.torch.cuda, "is_initialized", lambda: True)
+    monkeypatch.setattr(Q.torch.cuda, "is_current_stream_capturing", lambda: False)
+    monkeypatch.setattr(Q.capi, "entropy_bounds", bounds)
+    kind = Q.torch.cuda.OutOfMemoryError
+    assert Q.calibrate_entropy(*problem) == want
+    kind = MXQError
+    with pytest.raises(MXQError):
+        Q.calibrate_entropy(*problem)
+    assert raised == [Q.torch.cuda.OutOfMemoryError, MXQError]
