@@ -389,7 +389,9 @@ int mxq_quantize_to_nhwc(void* stream, const float* in, int8_t* out, float* omin
   MXQ_CHECK(in != nullptr && out != nullptr && aligned16(out), "null or unaligned data pointer");
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (space_to_depth && C <= 4 && a.chunks == 1 && W >= 2 && N <= 65535) {
-    const dim3 grid((a.OH * a.OW + kS2dThreads - 1) / kS2dThreads, N), block(kS2dThreads);
+    // (a plane may reach to the last int)
+    const unsigned plane = static_cast<unsigned>(a.OH * a.OW);
+    const dim3 grid((plane + kS2dThreads - 1) / kS2dThreads, N), block(kS2dThreads);
     switch (C) {
       case 1: hipLaunchKernelGGL(quantize_s2d_kernel<1>, grid, block, 0, s, a); break;
       case 2: hipLaunchKernelGGL(quantize_s2d_kernel<2>, grid, block, 0, s, a); break;

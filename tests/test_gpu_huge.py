@@ -310,3 +310,26 @@ def test_conv_input_over_2gib(capi, O, ksize):
         blk = slice(n0, min(n0 + step, NB))
         part = capi.quantized_conv_nhwc(d[blk], w, b, *one, *one, *one, **kw)
         assert torch.equal(res["out8"][blk], part["out8"]), f"images from {n0}"
+
+
+def test_space_to_depth_of_a_plane_up_to_the_last_int(capi):
+    """2^31 - 2 output pixels: the groups that cover them are counted past the largest int."""
+    from mxnet_amd._lib import check, lib
+    h, w, ow = 3, (1 << 31) - 2, (1 << 30) - 1
+    x = torch.empty(h, w, device="cuda")
+    x.normal_(generator=torch.Generator(device="cuda").manual_seed(9))
+    out = torch.full((2, ow, 16), 99, dtype=torch.int8, device="cuda")
+    lo, hi = torch.empty(1, device="cuda"), torch.empty(1, device="cuda")
+    check(lib.mxq_quantize_to_nhwc(torch.cuda.current_stream().cuda_stream, x.data_ptr(),
+                                   out.data_ptr(), lo.data_ptr(), hi.data_ptr(), 1, 1, h, w, 16, 1,
+                                   0, 0, -2.5, 3.0))
+    assert (lo.item(), hi.item()) == (-3.0, 3.0)
+    for first in (0, ow // 2 - 1000, ow - 4099):
+        last = min(first + 5000, ow)
+        part = x[:, 2 * first:2 * last].contiguous()
+        q = capi.quantize_v2(part, "int8", min_calib_range=-2.5, max_calib_range=3.0)[0]
+        want = torch.zeros((4, 2 * (last - first)), dtype=torch.int8, device="cuda")
+        want[:h] = q
+        want = want.view(2, 2, last - first, 2).permute(0, 2, 1, 3).reshape(2, last - first, 4)
+        assert torch.equal(out[:, first:last, :4], want)
+        assert not out[:, first:last, 4:].any()
