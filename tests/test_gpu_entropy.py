@@ -1,7 +1,10 @@
 """The entropy calibration's bounds from the GPU: they hold for what the definition's float sums
 give, candidate by candidate, and the search that starts from them is the host's own search."""
+import time
+
 import numpy as np
 import pytest
+import torch
 
 from mxnet_amd import capi
 from mxnet_amd import quantization as Q
@@ -115,3 +118,22 @@ def test_what_stays_on_the_host():
                       (np.full(601, 2.0 ** 23, f32), 255), (np.ones(32769, f32), 255)):
         assert Q._entropy_bounds([good, h], [255, levels]) is None
     assert Q._entropy_bounds([np.ones(32767, f32)], [255]).shape == (16384 - 127, 2)
+
+
+def test_histograms_that_are_not_exact_take_no_round_trip_a_bin():
+    """Counts of 2^24 and more are added up in the order of the bins: with reads ahead of the
+    additions a quarter more than an exact histogram takes, with an access at a time three times
+    as much."""
+    bins = 8001
+    x = np.arange(bins) - bins // 2
+    exact = np.floor(60 * np.exp(-(x / 1200.0) ** 2)).astype(f32)
+    took = []
+    for h in (exact, exact * f32(5000)):
+        runs = []
+        for _ in range(8):
+            torch.cuda.synchronize()
+            start = time.perf_counter()
+            capi.entropy_bounds([h], [255])
+            runs.append(time.perf_counter() - start)
+        took.append(min(runs))
+    assert took[1] < 1.8 * took[0], took
