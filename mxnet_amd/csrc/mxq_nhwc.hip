@@ -87,27 +87,40 @@ __global__ __launch_bounds__(kThreads) void quantize_nhwc_kernel(QuantNhwcArgs a
 // looked at (clamped into the image and taken out again where they were outside).  224 x 224 x 3
 // in the head of a network's pass: batch 64 9.9 us, one image 3.2 (with the channels a variable and
 // a branch around each load 13.4 and 6.7).
+// PAIR: images of two columns and more.  FLAT: lanes run on from one image to the next, for planes
+// that leave much of a work-group's last lanes idle (60000 images of 3 x 4 x 4 29.4 us -> 6.4, 8000 of
+// 8 x 8 6.2 -> 3.6, 200 of 3 x 40 x 40 3.3 -> 3.2); else images are the grid's second axis, which saves
+// a division.
 constexpr int kS2dThreads = 128;
-template <int C>
+constexpr int kS2dFlat = 1024;  // pixels of a plane from which on images are an axis
+template <int C, bool PAIR, bool FLAT>
 __global__ __launch_bounds__(kS2dThreads) void quantize_s2d_kernel(QuantNhwcArgs a) {
-  const int pixel = blockIdx.x * kS2dThreads + threadIdx.x, plane = a.OH * a.OW;
-  if (pixel == 0 && blockIdx.y == 0) {
+  const int plane = a.OH * a.OW;
+  unsigned at = blockIdx.x * kS2dThreads + threadIdx.x, image = blockIdx.y;
+  if (at == 0 && image == 0) {
     *a.omin = -a.range;
     *a.omax = a.range;
   }
-  if (pixel >= plane) return;
+  if (FLAT) {
+    if (at >= a.pieces) return;
+    image = at / static_cast<unsigned>(plane);
+    at -= image * static_cast<unsigned>(plane);
+  } else if (at >= static_cast<unsigned>(plane)) {
+    return;
+  }
+  const int pixel = static_cast<int>(at);
   const float s = 127.0f / a.range;
   const int oh = static_cast<int>(static_cast<unsigned>(pixel) / static_cast<unsigned>(a.OW));
   const int x = 2 * (pixel - oh * a.OW) - a.off_w, y = 2 * oh - a.off_h;
-  const int from = x < 0 ? 0 : x > a.W - 2 ? a.W - 2 : x;
-  const float* const img = a.in + static_cast<size_t>(blockIdx.y) * C * a.H * a.W;
-  float v[2][C][2];
+  const int from = !PAIR || x < 0 ? 0 : x > a.W - 2 ? a.W - 2 : x;
+  const float* const img = a.in + static_cast<size_t>(image) * C * a.H * a.W;
+  float v[2][C][2] = {};
 #pragma unroll
   for (int d = 0; d < 2; ++d) {
     const int h = y + d < 0 ? 0 : y + d > a.H - 1 ? a.H - 1 : y + d;
 #pragma unroll
     for (int c = 0; c < C; ++c)
-      __builtin_memcpy(v[d][c], img + (static_cast<size_t>(c) * a.H + h) * a.W + from, 8);
+      __builtin_memcpy(v[d][c], img + (static_cast<size_t>(c) * a.H + h) * a.W + from, PAIR ? 8 : 4);
   }
   int q[16];
 #pragma unroll
@@ -132,7 +145,7 @@ __global__ __launch_bounds__(kS2dThreads) void quantize_s2d_kernel(QuantNhwcArgs
 #pragma unroll
   for (int j = 0; j < 4; ++j)
     w[j] = static_cast<int>(pack_bytes(q[4 * j], q[4 * j + 1], q[4 * j + 2], q[4 * j + 3]));
-  a.out[static_cast<size_t>(blockIdx.y) * plane + pixel] = w;
+  a.out[static_cast<size_t>(image) * plane + pixel] = w;
 }
 
 struct PoolNhwcArgs {
@@ -355,6 +368,32 @@ unsigned capped_blocks(size_t items) {
   return static_cast<unsigned>(g < cap ? g : cap);
 }
 
+// Images in as many launches as their lanes (FLAT) or the grid's second axis need.
+template <int C, bool PAIR, bool FLAT>
+void launch_s2d_as(hipStream_t s, QuantNhwcArgs a, int N) {
+  const long long plane = 1LL * a.OH * a.OW;  // up to the last int
+  const int most = FLAT ? static_cast<int>(((1LL << 31) - 1) / plane) : 65535;
+  for (int left = N; left > 0; left -= most) {
+    const int images = left < most ? left : most;
+    a.pieces = static_cast<size_t>(images) * plane;
+    const long long lanes = FLAT ? images * plane : plane;
+    const dim3 grid(static_cast<unsigned>((lanes + kS2dThreads - 1) / kS2dThreads),
+                    FLAT ? 1 : images);
+    hipLaunchKernelGGL((quantize_s2d_kernel<C, PAIR, FLAT>), grid, dim3(kS2dThreads), 0, s, a);
+    MXQ_LAUNCH_CHECK();
+    a.in += static_cast<size_t>(images) * a.C * a.H * a.W;
+    a.out += a.pieces;
+  }
+}
+template <int C>
+void launch_s2d(hipStream_t s, const QuantNhwcArgs& a, int N) {
+  const bool flat = 1LL * a.OH * a.OW < kS2dFlat;
+  if (a.W == 1)
+    flat ? launch_s2d_as<C, false, true>(s, a, N) : launch_s2d_as<C, false, false>(s, a, N);
+  else
+    flat ? launch_s2d_as<C, true, true>(s, a, N) : launch_s2d_as<C, true, false>(s, a, N);
+}
+
 }  // namespace
 }  // namespace mxq
 
@@ -388,15 +427,12 @@ int mxq_quantize_to_nhwc(void* stream, const float* in, int8_t* out, float* omin
   if (a.pieces == 0) return 0;
   MXQ_CHECK(in != nullptr && out != nullptr && aligned16(out), "null or unaligned data pointer");
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (space_to_depth && C <= 4 && a.chunks == 1 && W >= 2 && N <= 65535) {
-    // (a plane may reach to the last int)
-    const unsigned plane = static_cast<unsigned>(a.OH * a.OW);
-    const dim3 grid((plane + kS2dThreads - 1) / kS2dThreads, N), block(kS2dThreads);
+  if (space_to_depth && C <= 4 && a.chunks == 1) {
     switch (C) {
-      case 1: hipLaunchKernelGGL(quantize_s2d_kernel<1>, grid, block, 0, s, a); break;
-      case 2: hipLaunchKernelGGL(quantize_s2d_kernel<2>, grid, block, 0, s, a); break;
-      case 3: hipLaunchKernelGGL(quantize_s2d_kernel<3>, grid, block, 0, s, a); break;
-      default: hipLaunchKernelGGL(quantize_s2d_kernel<4>, grid, block, 0, s, a);
+      case 1: launch_s2d<1>(s, a, N); break;
+      case 2: launch_s2d<2>(s, a, N); break;
+      case 3: launch_s2d<3>(s, a, N); break;
+      default: launch_s2d<4>(s, a, N);
     }
   } else if (space_to_depth)
     hipLaunchKernelGGL((quantize_nhwc_kernel<true>), dim3(blocks_for(a.pieces)), dim3(kThreads),

@@ -333,3 +333,23 @@ def test_space_to_depth_of_a_plane_up_to_the_last_int(capi):
         want = want.view(2, 2, last - first, 2).permute(0, 2, 1, 3).reshape(2, last - first, 4)
         assert torch.equal(out[:, first:last, :4], want)
         assert not out[:, first:last, 4:].any()
+
+
+def test_space_to_depth_of_more_pixels_than_a_launch_counts(capi):
+    """Images of two output pixels, 2^31 + 10 of those: what one launch's lanes leave goes out in
+    another."""
+    from mxnet_amd._lib import check, lib
+    n = (1 << 30) + 5
+    x = torch.empty(n, 1, 2, 4, device="cuda")
+    x.normal_(generator=torch.Generator(device="cuda").manual_seed(11))
+    out = torch.full((n, 1, 2, 16), 99, dtype=torch.int8, device="cuda")
+    lo, hi = torch.empty(1, device="cuda"), torch.empty(1, device="cuda")
+    check(lib.mxq_quantize_to_nhwc(torch.cuda.current_stream().cuda_stream, x.data_ptr(),
+                                   out.data_ptr(), lo.data_ptr(), hi.data_ptr(), n, 1, 2, 4, 16, 1,
+                                   0, 0, -2.5, 3.0))
+    for first in (0, n // 2 - 1000, n - 2005):
+        part = x[first:first + 2005]
+        q = capi.quantize_v2(part, "int8", min_calib_range=-2.5, max_calib_range=3.0)[0]
+        want = q.view(-1, 2, 2, 2).permute(0, 2, 1, 3).reshape(-1, 1, 2, 4)
+        assert torch.equal(out[first:first + 2005, :, :, :4], want)
+        assert not out[first:first + 2005, :, :, 4:].any()

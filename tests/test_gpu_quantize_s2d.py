@@ -17,6 +17,19 @@ pytestmark = pytest.mark.gpu
                                    (1, 33, 130)])
 @pytest.mark.parametrize("off", [(0, 0), (1, 1), (0, 1), (1, 0)])
 def test_image(c, n, h, w, off):
+    check_images(c, n, h, w, off)
+
+
+# lanes that run on from image to image, single columns and rows, images past the grid's second axis
+@pytest.mark.parametrize("n,c,h,w", [(70001, 3, 4, 4), (65537, 1, 64, 64), (66000, 2, 1, 1),
+                                     (9, 3, 2047, 1), (9, 3, 2049, 1), (3, 4, 63, 66), (5, 1, 62, 65),
+                                     (40, 2, 9, 1), (130, 3, 1, 2), (1000, 1, 23, 11)])
+@pytest.mark.parametrize("off", [(0, 0), (1, 1)])
+def test_many_small_images(n, c, h, w, off):
+    check_images(c, n, h, w, off)
+
+
+def check_images(c, n, h, w, off):
     rng = np.random.default_rng(h * w + c)
     x = rng.standard_normal((n, c, h, w)).astype(np.float32) * 2
     special = [0.0, -0.0, np.nan, np.inf, -np.inf, 3.0, -3.0, 1e-30, -1e-30]
