@@ -137,3 +137,11 @@ def test_histograms_that_are_not_exact_take_no_round_trip_a_bin():
             runs.append(time.perf_counter() - start)
         took.append(min(runs))
     assert took[1] < 1.8 * took[0], took
+
+
+@pytest.mark.parametrize("bins,count,device", [([201, 201], 30, True), ([201], 30, False),
+                                               ([227], 30, False), ([229], 30, True)])
+def test_few_candidates_stay_on_the_host(bins, count, device):
+    """99 candidates and fewer, in all: the host's threads are through before the launches are."""
+    found = Q._entropy_bounds([np.ones(b, f32) for b in bins], [count] * len(bins))
+    assert (found is not None) == device
