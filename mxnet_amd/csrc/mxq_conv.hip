@@ -489,20 +489,49 @@ bool conv3x3_rows_ok(const ConvArgs& a) {
                     4LL * kRowsO * a.OH * a.OW < (1LL << 31));
 }
 
-void launch_conv3x3_rows(hipStream_t s, const ConvArgs& a) {
-  const long cus = num_cus();
+struct RowItems {
+  bool two;      // output rows per item, or one
+  long items;
+  long rounds;   // of the chip's waves over them
+};
+RowItems row_items(const ConvArgs& a) {
+  const long waves = static_cast<long>(kRowsWaves) * num_cus();
   // two output rows per item once that still gives most waves of the chip an item: a third
   // fewer input rows to fetch per output row
   const long items2 = static_cast<long>(a.N) * ((a.OH + 1) / 2);
-  const bool two = 5 * items2 >= 3 * kRowsWaves * cus;
-  const long items = two ? items2 : static_cast<long>(a.N) * a.OH;
-  long grid = (items + kRowsWaves - 1) / kRowsWaves;
+  RowItems r;
+  r.two = 5 * items2 >= 3 * waves;
+  r.items = r.two ? items2 : static_cast<long>(a.N) * a.OH;
+  r.rounds = (r.items + waves - 1) / waves;
+  return r;
+}
+
+void launch_conv3x3_rows(hipStream_t s, const ConvArgs& a) {
+  const long cus = num_cus();
+  const RowItems r = row_items(a);
+  long grid = (r.items + kRowsWaves - 1) / kRowsWaves;
   if (grid > cus) grid = cus;
+  const bool two = r.two;
   const auto kernel = a.epi.out32 != nullptr
                           ? (two ? conv3x3_rows_kernel<2, true> : conv3x3_rows_kernel<1, true>)
                           : (two ? conv3x3_rows_kernel<2, false> : conv3x3_rows_kernel<1, false>);
   hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(64 * kRowsWaves), 0, s, a);
   MXQ_LAUNCH_CHECK();
+}
+
+// Whether int32 planes leave this kernel sooner than the tiled one, which moves the wider output
+// through LDS: from three rows a CU on (us, tiled and here, 56 x 56: 448 rows 7.6 / 8.4, 896 11.4 /
+// 9.3, 1344 13.4 / 10.4, 3584 26.6 / 21.1), but not for short rows, whose products are mostly padding
+// (28 wide, 1792 rows 11.3 / 9.7, 17 wide, 2624 rows 10.0 / 12.5, 14 wide, 3584 rows 11.0 / 13.1), nor
+// for rows of less than 36 pixels where the last of several rounds leaves most waves idle (24 and
+// 28 wide, 4600 rows: 12 and 9 % behind, 29 wide 4484 rows 28.1 / 31.6; 9000 rows 2 % behind and
+// 3 % ahead), and less than five a CU (32 wide, 800 rows 11.8 / 12.9).
+bool conv3x3_rows_wins_planes(const ConvArgs& a) {
+  const long rows = static_cast<long>(a.N) * a.OH;
+  if (a.W < 24 || rows < (a.W >= 36 ? 3L : 5L) * num_cus()) return false;
+  const RowItems r = row_items(a);
+  const long room = r.rounds * kRowsWaves * num_cus();
+  return a.W >= 36 || r.rounds == 1 || 10 * room <= 16 * r.items;
 }
 
 // ---- few-tap convolution over 16 channels, straight from memory -------------------------
@@ -1574,15 +1603,13 @@ void conv_nhwc(void* stream, const int8_t* data, const int8_t* weight, const int
     plan = plan_conv(g, aligned, unsplit);
   }
   // 61: the parked-weights row kernel (3 x 3 over 64 -> 64 channels, fused int8 output);
-  // chosen for it whenever the launch has rows for every wave of the chip; with int32 planes from
-  // three rows a CU on, as the tiled kernel has the wider output to move through LDS (us, tiled and
-  // here, 56 x 56: 448 rows 7.6 / 8.4, 896 11.4 / 9.3, 1344 13.4 / 10.4, 3584 26.6 / 21.1), but
-  // not for short rows, whose products are mostly padding (28 wide, 1792 rows 11.3 / 9.7, 17 wide,
-  // 2624 rows 10.0 / 12.5, 14 wide, 3584 rows 11.0 / 13.1)
+  // chosen for it whenever the launch has rows for every wave of the chip, with int32 planes by a
+  // rule of their own
   const bool planes = a.epi.out32 != nullptr;
-  if (plan.cfg == 61 || (force.cfg == 0 && conv3x3_rows_ok(a) && (!planes || a.W >= 24) &&
-                         static_cast<long>(a.N) * a.OH >=
-                             (planes ? 3L : 1L * kRowsWaves) * num_cus())) {
+  if (plan.cfg == 61 ||
+      (force.cfg == 0 && conv3x3_rows_ok(a) &&
+       (planes ? conv3x3_rows_wins_planes(a)
+               : static_cast<long>(a.N) * a.OH >= 1L * kRowsWaves * num_cus()))) {
     MXQ_CHECK(conv3x3_rows_ok(a), "shape does not qualify for the parked-weights 3x3 kernel");
     MXQ_CHECK(plan.splits <= 1 || force.splits == 0, "the 3x3 row kernel has no split-K form");
     launch_conv3x3_rows(s, a);
