@@ -566,6 +566,10 @@ __global__ __launch_bounds__(256) void gather_planes_kernel(GatherArgs a) {
 // The four gathers of a ResNet-50 at batch 64, whose inputs come from memory: 28 x 28 x 512 / 2
 // 11.7 us -> 9.8, 14 x 14 x 1024 / 2  7.8 -> 6.6, 7 x 7 x 512  8.4 -> 5.4, 7 x 7 x 2048  8.2 -> 7.1.
 // Groups of 8 KB instead of 16 measured 11.2, 6.1, 5.3 and 6.4, of 4 KB 11.9, 7.4, 5.3 and 7.6.
+// A group is one chain, load and pick, the picked bytes four times as dear: planes whose least group
+// is a long one stay with the form above (layers of 64 channels, one image or a few, us, there and
+// here: 21 x 21 -0.5, 27 x 27 8.8 / 10.3, 35 x 35 8.8 / 13.0, 45 x 45 8.8 / 17.1; of stride 2: 35 x 35
+// -0.2, 45 x 45 +0.8).
 struct GatherLdsArgs {
   const int8_t* in;
   uint8_t* out;
@@ -576,6 +580,7 @@ struct GatherLdsArgs {
   uint32_t magic_slots, magic_row, magic_per, magic_ow;
 };
 constexpr int kGatherLds = 16 * 1024, kGatherLdsMost = 32 * 1024;
+constexpr long long kGatherChain = 40 * 1024;  // loaded bytes and four times the picked ones
 
 // n / d for n * d < 2^30, magic = 2^31 / d + 1
 __device__ __forceinline__ int quotient(int n, uint32_t magic) {
@@ -642,8 +647,8 @@ bool launch_gather_lds(hipStream_t s, const int8_t* in, int8_t* out, int N, int 
   int unit = 1;  // channels that are whole pieces
   while (unit < 16 && unit * plane_in % 16 != 0) unit *= 2;
   const long long least = unit * plane_in;
-  if (least > kGatherLdsMost || C % unit != 0 || 1LL * N * C * plane_in >= (1LL << 31) ||
-      !aligned16(in))
+  if (least > kGatherLdsMost || least + 4LL * unit * pitch > kGatherChain || C % unit != 0 ||
+      1LL * N * C * plane_in >= (1LL << 31) || !aligned16(in))
     return false;
   GatherLdsArgs a;
   a.in = in;

@@ -18,7 +18,11 @@ pytestmark = pytest.mark.gpu
                                    (2, 16, 40, 51, 32, 3, 2), (1, 16, 128, 256, 16, 1, 3),
                                    (1, 16, 129, 256, 16, 1, 3), (9, 96, 3, 3, 16, 1, 1),
                                    (64, 128, 28, 28, 512, 2, 2), (16, 256, 57, 57, 528, 2, 2),
-                                   (25, 272, 46, 46, 512, 2, 2)])
+                                   (25, 272, 46, 46, 512, 2, 2),
+                                   # the longest groups that go through LDS, and the next ones
+                                   (1, 16, 128, 256, 16, 8, 8), (2, 16, 43, 45, 32, 4, 4),
+                                   (2, 16, 43, 45, 32, 3, 4), (3, 64, 21, 21, 32, 1, 1),
+                                   (3, 64, 23, 23, 32, 1, 1), (2, 48, 35, 35, 64, 2, 2)])
 def test_integers_of_the_general_path(shape):
     n, c, h, w, o, sh, sw = shape
     oh, ow = (h - 1) // sh + 1, (w - 1) // sw + 1
