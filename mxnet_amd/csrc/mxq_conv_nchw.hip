@@ -817,9 +817,11 @@ NchwPlan plan_nchw(int N, int C, int H, int W, int O, int KH, int KW, int sh, in
     // them the ring wins there too (us, loader and ring: 256 -> 512 / 2 at 56 x 56 50.1 / 42.5,
     // 256 -> 1024 / 2 99.5 / 68.8, 128 -> 512 / 2 38.4 / 32.0, 512 -> 512 / 2 at 28 x 28 25.9 /
     // 20.9, 256 -> 512 / 2 17.3 / 16.2 and for 16 images, 3136 pixels, 7.2 / 8.6; 256 -> 384 / 2
-    // at 56 x 56 47.5 / 47.1, 64 -> 512 / 2 28.3 / 28.4).
+    // at 56 x 56 47.5 / 47.1, 64 -> 512 / 2 28.3 / 28.4).  Of a short reduction the second launch
+    // needs more pixels (128 -> 512 / 2: 12544 pixels 11.2 / 13.4, 25088 16.9 / 19.0, 37632 27.2 /
+    // 24.3).
     const bool few_weights = 1LL * O * C <= 256 * 1024;
-    const bool many_tiles = O >= 512 && C >= 128 && 1LL * N * P >= 12 * 1024;
+    const bool many_tiles = O >= 512 && C >= 128 && 1LL * N * P >= (C >= 256 ? 12 : 32) * 1024;
     const bool light = (few_weights && !many_tiles) || !prepass_ok;
     int mode = kGatherBytes;
     if (sw == 2 && pl.OW % 4 == 0 && (sh * W) % 8 == 0 && plane_in % 8 == 0 && 2 * pl.OW <= W)

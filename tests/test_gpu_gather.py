@@ -47,8 +47,9 @@ def test_integers_of_the_general_path(shape):
 
 
 def test_many_tiles_without_a_workspace():
-    """Layers that gather beforehand only because it is faster do without the room for it."""
-    n, c, h, o = 64, 128, 28, 512
+    """Layers that gather beforehand only because it is faster (256 channels, 12544 pixels of 512
+    outputs; 128 channels from 32768 pixels on) do without the room for it."""
+    n, c, h, o = 64, 256, 28, 512
     data = torch.randint(-127, 128, (n, c, h, h), device="cuda", dtype=torch.int8)
     weight = torch.randint(-127, 128, (o, c, 1, 1), device="cuda", dtype=torch.int8)
     ranges = [torch.tensor([v], device="cuda") for v in (-3.0, 2.5, -0.5, 0.75)]
@@ -65,3 +66,12 @@ def test_many_tiles_without_a_workspace():
             space.data_ptr() if room else None, room))
         outs.append(out)
     assert torch.equal(*outs)
+
+
+@pytest.mark.parametrize("n,c,gathers", [(64, 128, False), (168, 128, True), (64, 256, True),
+                                         (61, 256, False)])
+def test_which_layers_gather_beforehand(n, c, gathers):
+    """28 x 28 / 2 -> 512: where the second launch is worth it.  (Behind it the workspace holds the
+    pixels the layer reads.)"""
+    need = lib.mxq_quantized_conv_nchw_workspace(n, c, 28, 28, 512, 1, 1, 2, 2, 0, 0, 1, 1, 1)
+    assert (need >= n * c * 14 * 14) == gathers
