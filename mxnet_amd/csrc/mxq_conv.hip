@@ -1575,7 +1575,8 @@ void conv_nhwc(void* stream, const int8_t* data, const int8_t* weight, const int
   const long long data_bytes = static_cast<long long>(N) * H * W * C;
   const bool dma_ok = aligned && data_bytes < (1LL << 31) &&
                       static_cast<long long>(O) * a.K < (1LL << 31);
-  if (force.cfg == 0 && KH == 1 && KW == 1 && pad_h == 0 && pad_w == 0) {
+  // 65: 1 x 1 layers with the weights in registers, where that is the faster way
+  if ((force.cfg == 0 || force.cfg == 65) && KH == 1 && KW == 1 && pad_h == 0 && pad_w == 0) {
     ResidentArgs r = {};
     r.data = data;
     r.weight = weight;
@@ -1594,6 +1595,7 @@ void conv_nhwc(void* stream, const int8_t* data, const int8_t* weight, const int
       return;
     }
   }
+  MXQ_CHECK(force.cfg != 65, "not a layer for the kernel with the weights in registers");
   ConvPlan plan = plan_conv(g, aligned, force);
   // a split the chooser proposed is dropped when the caller brought no room for it
   if (force.splits == 0 && plan.splits > 1 &&

@@ -31,6 +31,7 @@ namespace mxq {
 //   57..59  128x64 and 64x128 with 128-byte stages, 64x64 with 256-byte stages
 //   60      256x192 with 128-byte stages (outputs whose width is a multiple of 192)
 //   61, 62  the short-K streaming kernel with 64- / 128-column strips
+//   65      the kernel with the weights in registers, where it is the faster one
 //   71      the few-tiles kernel (any shape; here `splits` is the number of waves per
 //           32 x 32 tile, negative for 16 x 16 tiles)
 // Output tile of a direct-to-LDS configuration (what a split-K work-group leaves in the
@@ -279,7 +280,7 @@ void launch_fc(hipStream_t s, const int8_t* data, const int8_t* weight, int M, i
       return;
     }
   }
-  if (force.cfg == 0 && (K == 256 || K == 512)) {  // its reductions
+  if ((force.cfg == 0 || force.cfg == 65) && (K == 256 || K == 512)) {  // its reductions
     ResidentArgs r = {};
     r.data = data;
     r.weight = weight;
@@ -293,6 +294,7 @@ void launch_fc(hipStream_t s, const int8_t* data, const int8_t* weight, int M, i
       return;
     }
   }
+  MXQ_CHECK(force.cfg != 65, "not a layer for the kernel with the weights in registers");
   FcPlan plan = plan_fc(M, N, K, aligned, fused8, force, sum, epi.sum_requant != 0);
   // a split the chooser proposed is dropped when the caller brought no room for it
   if (force.splits == 0 && plan.splits > 1 &&

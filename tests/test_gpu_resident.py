@@ -5,6 +5,7 @@ import pytest
 import torch
 
 from mxnet_amd import capi
+from mxnet_amd._lib import MXQError
 
 pytestmark = pytest.mark.gpu
 
@@ -43,12 +44,20 @@ def test_rows(k, n, relu, bias):
         got = capi.quantized_conv_nhwc(*args, **kw)
         want = capi.quantized_conv_nhwc(*args, force=(25, 1), **kw)
         same(got, want)
+        # it is this kernel that was chosen: pinned, any other choice is an error
+        flat = (x.view(m, k), w, *args[2:])
+        pinned = capi.quantized_fc(*flat, force=(65, 1, 0), **kw)
+        assert torch.equal(pinned["out8"], want["out8"].view(m, n))
+    with pytest.raises(MXQError):
+        capi.quantized_fc(x.view(m, k)[:least // 2], w, *args[2:], force=(65, 1, 0), **kw)
 
 
 # (images, height, width, strides): odd planes, images smaller than a tile, one output line
 @pytest.mark.parametrize("images,h,w,sh,sw", [(40, 57, 55, 2, 2), (3000, 9, 7, 2, 2),
                                               (9000, 5, 4, 2, 3), (26000, 2, 2, 2, 2),
-                                              (2, 301, 300, 2, 1), (3, 2, 65000, 2, 3)])
+                                              (2, 199, 299, 2, 1), (3, 2, 65000, 2, 3),
+                                              # planes the kernel leaves to the tiled ones
+                                              (2, 301, 300, 2, 1)])
 @pytest.mark.parametrize("k,n", [(256, 64), (256, 128), (256, 512), (512, 128), (512, 512)])
 def test_strided(images, h, w, sh, sw, k, n):
     oh, ow = (h - 1) // sh + 1, (w - 1) // sw + 1
@@ -59,3 +68,8 @@ def test_strided(images, h, w, sh, sw, k, n):
     got = capi.quantized_conv_nhwc(*args, **kw)
     want = capi.quantized_conv_nhwc(*args, force=(25, 1), **kw)
     same(got, want)
+    if oh * ow < 30000:
+        same(capi.quantized_conv_nhwc(*args, force=(65, 1), **kw), want)
+    else:
+        with pytest.raises(MXQError):
+            capi.quantized_conv_nhwc(*args, force=(65, 1), **kw)
