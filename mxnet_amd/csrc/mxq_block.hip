@@ -26,7 +26,9 @@
 // What bounds it: a tile's own chain.  Of the 42000 clocks of a tile of 14 x 14 x 256 -> 1024 ->
 // 256 (one per CU) 5000 go by until the patch is there, 15000 in the 3 x 3 layer (9200 of matrix
 // work), 14000 in the sum's layer (8000 of vector and 4000 of matrix work that overlap little: two
-// waves of a SIMD run in step from the barrier on), 8000 behind it.  Measured at batch 64 against
+// waves of a SIMD run in step from the barrier on), 8000 behind it.  With up to 128 channels in the
+// middle half of the waves (64 on tiles of 32 pixels: of four, two) have no column tile of the 3 x 3
+// layer, more than half of the products, and wait at the barrier behind it.  Measured at batch 64 against
 // the three launches: 22.8 us against 38.3 there, 31 / 45 for 28 x 28 x 128, 38.6 / 60 for 56 x 56 x
 // 64.  A quantized ResNet-50 at batch 64 went from 867 us to 667 with it, one image from 241 to 234.
 // Measured and not kept: a column tile's products made while the one before is finished (level, 100

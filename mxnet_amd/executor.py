@@ -22,8 +22,9 @@ from . import _frontend, _plan
 from . import operator as _operator
 
 # Input shape combinations an executor keeps a plan for, the ones used last.  A plan by itself is
-# small (1 KiB of device memory for a quantized ResNet-50); the 11 MB of laid-out weights are the
-# graph's.
+# small (1 KiB of device memory for a quantized ResNet-50); the laid-out weights are the graph's, for
+# all of its plans: 11 MB packed, and what its launches of several layers (7 MB at batch 64, 1 on one
+# image) and of 3 x 3 layers over many channels (7 MB at batch 64) read, made of those and beside them.
 _MAX_PLANS = 64
 
 
