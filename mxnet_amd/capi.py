@@ -290,22 +290,34 @@ def minmax(data):
     return out
 
 
+_ENTROPY_WS_BYTES = 1 << 30
+
+
 def entropy_bounds(hists, levels):
     """float64 [candidate, 2] on the host: bounds of what the entropy calibration's float sums give
     for every candidate of numpy histograms, one behind the other; taken on the current device."""
     dev = torch.device("cuda", torch.cuda.current_device())
-    found = []
-    for at in range(0, len(hists), 16):  # as many as a call takes
-        h, n = hists[at:at + 16], levels[at:at + 16]
-        bins, quantized = (ctypes.c_int * len(h))(*[x.size for x in h]), (ctypes.c_int * len(h))(*n)
-        data = torch.from_numpy(np.concatenate(h)).to(dev)
+    found, at = [], 0
+    while at < len(hists):
+        # as many as a call takes, while their workspace (a float per candidate and level, up to
+        # 0.5 GB a histogram) is no larger than that
+        end, wsb = at, 0
+        while end < len(hists) and end - at < 16:
+            n = end + 1 - at
+            more_bins = (ctypes.c_int * n)(*[x.size for x in hists[at:end + 1]])
+            more_levels = (ctypes.c_int * n)(*levels[at:end + 1])
+            more = lib.mxq_entropy_bounds_workspace(n, more_bins, more_levels)
+            if end > at and more > _ENTROPY_WS_BYTES:
+                break
+            end, wsb, bins, quantized = end + 1, more, more_bins, more_levels
+        data = torch.from_numpy(np.concatenate(hists[at:end])).to(dev)
         out = torch.empty(sum(b // 2 + 1 - q // 2 for b, q in zip(bins, quantized)), 2,
                           dtype=torch.float64, device=dev)
-        wsb = lib.mxq_entropy_bounds_workspace(len(h), bins, quantized)
         ws = _workspace(wsb, dev)
-        check(lib.mxq_entropy_bounds(_stream(), len(h), _ptr(data), bins, quantized, _ptr(out),
+        check(lib.mxq_entropy_bounds(_stream(), end - at, _ptr(data), bins, quantized, _ptr(out),
                                      _ptr(ws), wsb))
         found.append(out)
+        at = end
     return torch.cat(found).cpu().numpy() if len(found) > 1 else found[0].cpu().numpy()
 
 

@@ -145,3 +145,22 @@ def test_few_candidates_stay_on_the_host(bins, count, device):
     """99 candidates and fewer, in all: the host's threads are through before the launches are."""
     found = Q._entropy_bounds([np.ones(b, f32) for b in bins], [count] * len(bins))
     assert (found is not None) == device
+
+
+@pytest.mark.parametrize("room", [1, 3 << 20, 1 << 30])
+def test_histograms_beyond_a_workspace_take_further_calls(room, monkeypatch):
+    rng = np.random.default_rng(room)
+    hists = [histogram(KINDS[i % len(KINDS)], 401 + 200 * i, rng) for i in range(11)]
+    levels = [255, 3, 64] * 3 + [31, 401]
+    want = np.concatenate([capi.entropy_bounds([h], [n]) for h, n in zip(hists, levels)])
+    calls, run = [], capi.lib.mxq_entropy_bounds
+
+    def bounds(stream, count, *args):
+        calls.append((count, args[-1]))
+        return run(stream, count, *args)
+
+    monkeypatch.setattr(capi, "_ENTROPY_WS_BYTES", room)
+    monkeypatch.setattr(capi.lib, "mxq_entropy_bounds", bounds)
+    assert np.array_equal(capi.entropy_bounds(hists, levels), want)
+    assert all(count == 1 or size <= room for count, size in calls)
+    assert len(calls) == (11 if room == 1 else 1) or 1 < len(calls) < 11
