@@ -23,15 +23,20 @@
 // Rows in LDS are an odd number of 16-byte chunks apart: 16 consecutive rows' fragments hit
 // distinct bank groups without a permutation, for any channel count.
 //
-// What bounds it: a tile's own chain.  Of the 42000 clocks of a tile of 14 x 14 x 256 -> 1024 ->
-// 256 (one per CU) 5000 go by until the patch is there, 15000 in the 3 x 3 layer (9200 of matrix
-// work), 14000 in the sum's layer (8000 of vector and 4000 of matrix work that overlap little: two
-// waves of a SIMD run in step from the barrier on), 8000 behind it.  With up to 128 channels in the
-// middle half of the waves (64 on tiles of 32 pixels: of four, two) have no column tile of the 3 x 3
-// layer, more than half of the products, and wait at the barrier behind it.  Measured at batch 64 against
-// the three launches: 22.8 us against 38.3 there, 31 / 45 for 28 x 28 x 128, 38.6 / 60 for 56 x 56 x
-// 64.  A quantized ResNet-50 at batch 64 went from 867 us to 667 with it, one image from 241 to 234.
-// Measured and not kept: a column tile's products made while the one before is finished (level, 100
+// What bounds it: instruction issue.  Vector instructions and MFMAs, which overlap little (the waves
+// of a work-group run in step from each barrier on), fill 75 to 85 % of a CU's busy clocks; the sum
+// alone is 7 vector instructions per output of 64 ... 256 channels in the middle times four.  So what is
+// not arithmetic has as few as possible: a weight's place is a scalar offset and an immediate, the three
+// taps of a row are immediates where the channels are those of a kernel instance (KSB), the places of a
+// tile's pixels in the tensors come from a table, and pieces of rows are walked by carries, not divided
+// (984 -> 760 vector instructions a wave of 56 x 56 x 64, of which 550 are arithmetic).  Measured in a
+// quantized ResNet-50's pass at batch 64, before and after: 46.2 -> 40.4 us for 56 x 56 x 64 -> 256 ->
+// 64, 34.4 -> 32.3 for 28 x 28 x 128, 26.7 -> 25.4 for 14 x 14 x 256; the pass 613 -> 592.  As three
+// launches they were 60, 45 and 38 us.
+// Measured and not kept: the 3 x 3 layer's reduction shared by the waves that have no column tile of
+// it (up to 128 channels in the middle half of them), or by 16 waves: level or behind, for the sums
+// that are exchanged cost more vector instructions than the idle waves did time;
+// a column tile's products made while the one before is finished (level, 100
 // registers more), the second layer's operand held in registers (level), wave priorities (level).
 #include <hip/hip_runtime.h>
 
@@ -49,6 +54,7 @@ namespace {
 #define MXQ_INLINE __attribute__((always_inline))
 
 constexpr int kBlockLds = 160 * 1024;
+typedef unsigned int v4u __attribute__((ext_vector_type(4)));
 
 // The short forms of mxq_forms.h, and for the sum
 //   fma(level, 2ta, fma(residual, 2tb, c)) as the form with the relu.  Both operands are small
@@ -109,6 +115,8 @@ struct BlockArgs {
   int tn, th, tw, tiles_h, tiles_w;  // tiles down and across an image
   int area, across, count, rows;     // (above) and pixels of a tile, rows of its patch
   int off_patch, off_bias, off_table, off_pixel;  // bytes in LDS
+  // what NW * 64 pieces are in rows and pieces beyond them, of the shortcut's slots and of the outputs
+  int res_rows, res_rest, wide_rows, wide_rest, next_rows, next_rest;
   int parts, row_pitch;   // load instructions and bytes per row of the patch
   uint32_t magic_tiles_w, magic_tiles_h, magic_area, magic_across, magic_h2, magic_pixel, magic_res,
       magic_wide, magic_next, magic_tap;
@@ -134,8 +142,10 @@ uint32_t magic_of(int d) { return static_cast<uint32_t>((1ULL << 31) / static_ca
 // WM x WN waves, each RT row tiles of 32 pixels by one column tile of 32 channels at a time.
 // GB, GC: MFMA steps whose weights a wave requests together (the 3 x 3 layer's, and the whole
 // reduction of the second layer).
+// KSB: MFMA steps of a tap where the data has exactly 32 * KSB channels, so that the places of three
+// taps in a row are constants; 0 for any other count, where a table in LDS has them.
 // `tile` is one of p.tiles; or, of runs, the one that begins at pixel `first`.
-template <int WM, int WN, int RT, int GB, int GC>
+template <int WM, int WN, int RT, int GB, int GC, int KSB>
 __device__ __forceinline__ void block_tile(const BlockArgs& p, int tile, int first) {
   constexpr int NW = WM * WN, TM = 32 * WM * RT, GA = 8;
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -148,7 +158,7 @@ __device__ __forceinline__ void block_tile(const BlockArgs& p, int tile, int fir
                "s"(p.run), "s"(p.area), "s"(p.across), "s"(p.count), "s"(p.rows), "s"(p.off_pixel),
                "s"(p.magic_area), "s"(p.magic_across), "s"(p.magic_h2),
                "s"(p.magic_pixel), "s"(p.parts), "s"(p.row_pitch), "s"(p.magic_res),
-               "s"(p.magic_tap), "s"(p.tiles));
+               "s"(p.magic_tap), "s"(p.tiles), "s"(p.res_rows), "s"(p.res_rest));
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WN, wn = wave % WN;
@@ -178,18 +188,31 @@ __device__ __forceinline__ void block_tile(const BlockArgs& p, int tile, int fir
 
   const auto weights = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(p.weights), 0,
                                                          p.kb_all * 1024, 0x00020000);
-  // fragment number k; zeros, and nothing is fetched, from kNone on
-  constexpr int kNone = 0x100000;
-  auto fragment = [&](int k) MXQ_INLINE {
-    return __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(
-                                       weights, k * 1024 + lane * 16, 0, 0));
+  // Fragments number from ... from + G - 1, one at a time: a scalar offset and an immediate each, no
+  // vector instruction.  Where there are none, zeros, and nothing is fetched: the lane's place is past
+  // the end then, and the scalar part 0 (a buffer's bound is compared with the place alone, after the
+  // scalar part was subtracted from it).
+  const int lane16 = lane * 16;
+  struct Fragments {
+    int from, at;
+  };
+  auto fragments = [&](bool some, int from) MXQ_INLINE {
+    return Fragments{some ? from : 0, some ? lane16 : 0x40000000};
+  };
+  auto fragment = [&](const Fragments& f, int i) MXQ_INLINE {
+    return __builtin_bit_cast(v4i,
+                              __builtin_amdgcn_raw_buffer_load_b128(
+                                  weights, f.at + (i & 3) * 1024, (f.from + (i & ~3)) * 1024, 0));
+  };
+  auto load_first = [&](auto& w, const Fragments& f) MXQ_INLINE {
+#pragma unroll
+    for (int i = 0; i < static_cast<int>(sizeof(w) / sizeof(v4i)); ++i) w[i] = fragment(f, i);
   };
   const int tiles_b = (p.Cm + 31) >> 5, tiles_c = (p.Co + 31) >> 5, tiles_a = (p.Ca + 31) >> 5;
   const bool has_b = wn < tiles_b;
   v4i wb[GB];
   const int first_b = (has_b ? wn : 0) * p.kb;
-#pragma unroll
-  for (int i = 0; i < GB; ++i) wb[i] = fragment(first_b + i);
+  load_first(wb, fragments(true, first_b));
 
   // the patch: the tile's rows of every one of its images and one above and below, a column on
   // either side; zeros where they leave the image
@@ -224,25 +247,36 @@ __device__ __forceinline__ void block_tile(const BlockArgs& p, int tile, int fir
       }
     }
   }
-  // which pixel of the tensor each of the tile's is, -1 past the edges
-  int* const pixel_of = reinterpret_cast<int*>(smem + p.off_pixel);
+  // For each of the tile's pixels where it lies in the wide tensors and in the last layer's result,
+  // past their ends for those past the edges, and where the patch has its first tap.
+  constexpr int kMore = 24;  // rows a load instruction of the shortcut may go beyond the tile
+  uint32_t* const wide_of = reinterpret_cast<uint32_t*>(smem + p.off_pixel);
+  uint32_t* const next_of = wide_of + TM + kMore;
+  int* const place_of = reinterpret_cast<int*>(next_of + TM);
   if (tid < TM) {
-    const int img = quotient_any(start_at + tid, p.area, p.magic_area), rem = start_at + tid - img * p.area;
+    // rows without a pixel read the first one's; never stored
+    const int i = start_at + (tid < p.count ? tid : 0);
+    const int img = quotient_any(i, p.area, p.magic_area), rem = i - img * p.area;
     const int ty = quotient(rem, p.magic_across), tx = rem - ty * p.across;
     const int n = n0 + img, h = h0 + ty, w = w0 + tx;
     const bool ok = tid < p.count && n < p.N && h < p.H && w < p.W;
-    pixel_of[tid] = ok ? (n * p.H + h) * p.W + w : -1;
+    const uint32_t pixel = static_cast<uint32_t>((n * p.H + h) * p.W + w);
+    wide_of[tid] = ok ? pixel * p.Co : kOutOfRange;
+    next_of[tid] = ok ? pixel * p.Ca : kOutOfRange;
+    place_of[tid] = (n * H2 + h - v0) * row_pitch + tx * PP * 16;
+    if (tid < kMore) wide_of[TM + tid] = kOutOfRange;
   }
   const int* const sbias = reinterpret_cast<const int*>(smem + p.off_bias);
-  const int bias_c = (p.Cm + 255) & ~255, bias_a = bias_c + ((p.Co + 255) & ~255);
+  const int bias_c = (p.Cm + 31) & ~31, bias_a = bias_c + ((p.Co + 31) & ~31);
 #pragma unroll
   for (int layer = 0; layer < 3; ++layer) {
     const int columns = layer == 0 ? p.Cm : layer == 1 ? p.Co : p.Ca;
     const int at = layer == 0 ? 0 : layer == 1 ? bias_c : bias_a;
-    if (columns != 0) {  // whole load instructions, zeros behind the last column
+    if (columns != 0) {  // whole column tiles, zeros behind the last column
       const v4i rsrc = make_rsrc(p.prepared[layer] + kPreparedBias, 4u * columns);
       for (int it = wave; it * 256 < columns; it += NW)
-        fetch(p.off_bias + at * 4 + it * 1024, it * 1024 + lane * 16, rsrc);
+        if (it * 256 + lane * 4 < ((columns + 31) & ~31))
+          fetch(p.off_bias + at * 4 + it * 1024, it * 1024 + lane16, rsrc);
     }
   }
   const EpiScalars s_b = p.forms->s[0], s_c = p.forms->s[1], s_a = p.forms->s[2];
@@ -253,52 +287,52 @@ __device__ __forceinline__ void block_tile(const BlockArgs& p, int tile, int fir
   const int has = p.forms->has;
   // where step k of the 3 x 3 layer reads, from the pixel's place under the first tap; steps behind
   // the last one have zero weights
-  for (int k = tid; k < p.kb + 2 * GB; k += 64 * NW) {
-    const int last = 9 * p.ksb - 1, at = k < last ? k : last;
-    const int tap = quotient(at, p.magic_tap), kh = tap / 3;
-    reinterpret_cast<int*>(smem + p.off_table)[k] =
-        kh * row_pitch + (tap - 3 * kh) * PP * 16 + (at - tap * p.ksb) * 32;
+  if constexpr (KSB == 0) {
+    for (int k = tid; k < p.kb + 2 * GB; k += 64 * NW) {
+      const int last = 9 * p.ksb - 1, at = k < last ? k : last;
+      const int tap = quotient(at, p.magic_tap), kh = tap / 3;
+      reinterpret_cast<int*>(smem + p.off_table)[k] =
+          kh * row_pitch + (tap - 3 * kh) * PP * 16 + (at - tap * p.ksb) * 32;
+    }
   }
   // The shortcut, a share of it at a time while the 3 x 3 layer runs.
   const v4i res_rsrc = make_rsrc(p.res, static_cast<uint32_t>(p.N) * p.H * p.W * p.Co);
   const int res_slots = TM * PO;
   int res_at = wave;
+  int res_row = quotient(res_at * 64 + lane, p.magic_res);
+  int res_j = res_at * 64 + lane - res_row * PO;
   auto fetch_shortcut = [&]() MXQ_INLINE {
     if (res_at * 64 < res_slots) {
-      const int q = res_at * 64 + lane;
-      const int row = quotient(q, p.magic_res), j = q - row * PO;
-      const int pixel = row < TM && j < CO ? pixel_of[row] : -1;
-      fetch(res_at * 1024, pixel >= 0 ? static_cast<uint32_t>(pixel * p.Co + 16 * j) : kOutOfRange,
-            res_rsrc);
+      // (the pad of a row gets what follows the row in memory)
+      fetch(res_at * 1024, wide_of[res_row] + 16 * res_j, res_rsrc);
       res_at += NW;
+      res_row += p.res_rows;
+      res_j += p.res_rest;
+      const bool carry = res_j >= PO;
+      res_j -= carry ? PO : 0;
+      res_row += carry;
     }
   };
 
   // this lane's rows: where they begin in each of the three
   const int frow = lane & 31, fgrp = lane >> 5;
   const int row0 = wm * RT * 32 + frow;
-  int in_patch[RT];
-#pragma unroll
-  for (int rt = 0; rt < RT; ++rt) {
-    int i = row0 + 32 * rt;
-    // rows without a pixel read the first one's; never stored
-    i = start_at + (i < p.count ? i : 0);
-    const int img = quotient_any(i, p.area, p.magic_area), rem = i - img * p.area;
-    const int ty = quotient(rem, p.magic_across), tx = rem - ty * p.across;
-    in_patch[rt] = p.off_patch + ((n0 + img) * H2 + h0 + ty - v0) * row_pitch + tx * PP * 16 +
-                   fgrp * 16;
-  }
   v16i acc[RT];
-  auto read_bias = [&](const int* bias, v4i (&b)[4]) MXQ_INLINE {
+  // The bias as first accumulators.  Each row tile reads its own: registers are copied with vector
+  // instructions, which this kernel is short of, so the compiler must not see that they are the same.
+  auto start = [&](v16i (&acc)[RT], const int* bias) MXQ_INLINE {
+    int at = static_cast<int>(reinterpret_cast<uintptr_t>(bias + 4 * fgrp));
 #pragma unroll
-    for (int vq = 0; vq < 4; ++vq)
-      b[vq] = *reinterpret_cast<const v4i*>(bias + 8 * vq + 4 * fgrp);
-  };
-  auto start = [&](v16i (&acc)[RT], const v4i (&b)[4]) MXQ_INLINE {
+    for (int rt = 0; rt < RT; ++rt) {
+      asm volatile("" : "+v"(at));
+      const auto b = reinterpret_cast<const __attribute__((address_space(3))) v4i*>(at);
 #pragma unroll
-    for (int rt = 0; rt < RT; ++rt)
+      for (int vq = 0; vq < 4; ++vq) {
+        const v4i x = b[2 * vq];
 #pragma unroll
-      for (int i = 0; i < 16; ++i) acc[rt][i] = b[i / 4][i % 4];
+        for (int i = 0; i < 4; ++i) acc[rt][4 * vq + i] = x[i];
+      }
+    }
   };
   // One group of G steps.  The pixels of a step are read kAhead steps before they are multiplied,
   // and a step's weights make room for those of the same step of the next group (fragments from
@@ -313,10 +347,10 @@ __device__ __forceinline__ void block_tile(const BlockArgs& p, int tile, int fir
     for (int rt = 0; rt < RT; ++rt)
       x[rt] = *reinterpret_cast<const v4i*>(smem + base[rt] + offset);
   };
-  // offset_of(i): where step i of the group reads, for i up to G + kAhead - 1
-  auto first_pixels = [&](const int (&base)[RT], auto offset_of) MXQ_INLINE {
+  // read(i, x): the pixels of step i of the group, for i up to G + kAhead - 1
+  auto first_pixels = [&](auto read) MXQ_INLINE {
 #pragma unroll
-    for (int i = 0; i < kAhead; ++i) read_pixels(px[i], base, offset_of(i));
+    for (int i = 0; i < kAhead; ++i) read(i, px[i]);
   };
   auto multiply = [&](v16i (&acc)[RT], v4i w, const v4i (&x)[RT]) MXQ_INLINE {
 #pragma unroll
@@ -325,14 +359,14 @@ __device__ __forceinline__ void block_tile(const BlockArgs& p, int tile, int fir
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) asm volatile("" : "+v"(acc[rt]));
   };
-  auto run_group = [&](auto& w, int from, const int (&base)[RT], auto offset_of) MXQ_INLINE {
+  auto run_group = [&](auto& w, const Fragments& f, auto read) MXQ_INLINE {
     constexpr int G = sizeof(w) / sizeof(v4i);
     static_assert(G % kRing == 0, "the sets of pixels take turns");
 #pragma unroll
     for (int i = 0; i < G; ++i) {
-      read_pixels(px[(i + kAhead) % kRing], base, offset_of(i + kAhead));
+      read(i + kAhead, px[(i + kAhead) % kRing]);
       multiply(acc, w[i], px[i % kRing]);
-      w[i] = fragment(from + i);
+      w[i] = fragment(f, i);
       __builtin_amdgcn_sched_barrier(0);
     }
   };
@@ -346,31 +380,58 @@ __device__ __forceinline__ void block_tile(const BlockArgs& p, int tile, int fir
   // ---- 3 x 3 ------------------------------------------------------------------------------
   const int groups = p.kb / GB;
   if (has_b) {
-    v4i bias[4];
-    read_bias(sbias + 32 * wn, bias);
-    start(acc, bias);
-    const int* const table = reinterpret_cast<const int*>(smem + p.off_table);
-    auto read_offsets = [&](int g, int (&o)[GB]) MXQ_INLINE {
+    int in_patch[RT];
 #pragma unroll
-      for (int i = 0; i < GB; ++i) o[i] = __builtin_amdgcn_readfirstlane(table[g * GB + i]);
-    };
-    int now[GB], later[GB];
-    read_offsets(0, now);
-    read_offsets(1, later);
-    auto offset_of = [&](int i) MXQ_INLINE { return i < GB ? now[i] : later[i - GB]; };
-    first_pixels(in_patch, offset_of);
-    for (int g = 0; g < groups; ++g) {
-      fetch_shortcut();
-      run_group(wb, g + 1 < groups ? first_b + (g + 1) * GB : kNone, in_patch, offset_of);
+    for (int rt = 0; rt < RT; ++rt) in_patch[rt] = p.off_patch + place_of[row0 + 32 * rt] + fgrp * 16;
+    start(acc, sbias + 32 * wn);
+    if constexpr (KSB != 0) {
+      constexpr int kRow = 3 * KSB, kTap = odd(2 * KSB) * 16;
+      static_assert(kRow % GB == 0, "a row of taps is whole groups");
+      int below[RT];
+      // step i of the taps in a row, or of the row below
+      auto read = [&](int i, v4i (&x)[RT]) MXQ_INLINE {
+        const int k = i < kRow ? i : i - kRow;
+        read_pixels(x, i < kRow ? in_patch : below, k / KSB * kTap + k % KSB * 32);
+      };
+      first_pixels(read);
+      for (int row = 0; row < 3; ++row) {
 #pragma unroll
-      for (int i = 0; i < GB; ++i) now[i] = later[i];
-      read_offsets(g + 2, later);
+        for (int rt = 0; rt < RT; ++rt) below[rt] = in_patch[rt] + row_pitch;
+#pragma unroll
+        for (int g = 0; g < kRow / GB; ++g) {
+          fetch_shortcut();
+          run_group(wb,
+                    fragments(row < 2 || g + 1 < kRow / GB, first_b + row * kRow + (g + 1) * GB),
+                    [&](int i, v4i (&x)[RT]) MXQ_INLINE { read(g * GB + i, x); });
+        }
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) in_patch[rt] = below[rt];
+      }
+    } else {
+      const int* const table = reinterpret_cast<const int*>(smem + p.off_table);
+      auto read_offsets = [&](int g, int (&o)[GB]) MXQ_INLINE {
+#pragma unroll
+        for (int i = 0; i < GB; ++i) o[i] = __builtin_amdgcn_readfirstlane(table[g * GB + i]);
+      };
+      int now[GB], later[GB];
+      read_offsets(0, now);
+      read_offsets(1, later);
+      auto read = [&](int i, v4i (&x)[RT]) MXQ_INLINE {
+        read_pixels(x, in_patch, i < GB ? now[i] : later[i - GB]);
+      };
+      first_pixels(read);
+      for (int g = 0; g < groups; ++g) {
+        fetch_shortcut();
+        run_group(wb, fragments(g + 1 < groups, first_b + (g + 1) * GB), read);
+#pragma unroll
+        for (int i = 0; i < GB; ++i) now[i] = later[i];
+        read_offsets(g + 2, later);
+      }
     }
   }
   while (res_at * 64 < res_slots) fetch_shortcut();
   v4i wc[GC];
-#pragma unroll
-  for (int i = 0; i < GC; ++i) wc[i] = fragment(p.at_c + wn * GC + i);
+  load_first(wc, fragments(wn < tiles_c, p.at_c + wn * GC));
   // column tile t of a layer's int8 result into rows of `pitch` chunks at the patch's place
   auto finish = [&](int t, int pitch, auto pack) MXQ_INLINE {
 #pragma unroll
@@ -410,10 +471,9 @@ __device__ __forceinline__ void block_tile(const BlockArgs& p, int tile, int fir
   auto widen = [&](auto how) MXQ_INLINE {
     constexpr int F = decltype(how)::value;
     for (int t = wn; t < tiles_c; t += WN) {
-      const int from = t + WN < tiles_c ? p.at_c + (t + WN) * GC : kNone;
-      v4i bias[4];
+      const Fragments f = fragments(t + WN < tiles_c, p.at_c + (t + WN) * GC);
       uint32_t shortcut[RT][4];
-      read_bias(sbias + bias_c + 32 * t, bias);
+      start(acc, sbias + bias_c + 32 * t);
       read_pixels(px[0], in_mid, 0);
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt)
@@ -421,12 +481,11 @@ __device__ __forceinline__ void block_tile(const BlockArgs& p, int tile, int fir
         for (int vq = 0; vq < 4; ++vq)
           shortcut[rt][vq] =
               *reinterpret_cast<const uint32_t*>(smem + at_wide[rt] + 32 * t + 8 * vq);
-      start(acc, bias);
 #pragma unroll
       for (int i = 0; i < GC; ++i) {
         if (i + 1 < GC) read_pixels(px[(i + 1) & 1], in_mid, 32 * (i + 1));
         multiply(acc, wc[i], px[i & 1]);
-        wc[i] = fragment(from + i);
+        wc[i] = fragment(f, i);
         __builtin_amdgcn_sched_barrier(0);
       }
 #pragma unroll
@@ -455,60 +514,74 @@ __device__ __forceinline__ void block_tile(const BlockArgs& p, int tile, int fir
   else
     widen(std::integral_constant<int, 0>());
   v4i wa[GA];
-  if (p.Ca != 0) {
-#pragma unroll
-    for (int i = 0; i < GA; ++i) wa[i] = fragment(p.at_a + wn * p.ka + i);
-  }
+  if (p.Ca != 0) load_first(wa, fragments(wn < tiles_a, p.at_a + wn * p.ka));
   publish();
 
   // Rows of `chunks` pieces, `pitch` apart in LDS, to their pixels.  Plain stores: the next block
   // reads both outputs, and what it finds in the memory-side cache it does not fetch from memory
   // (quantized ResNet-50 at batch 64, all blocks with streaming stores / plain ones: 680 / 651 us).
-  auto leave = [&](int at, int chunks, int pitch, uint32_t magic, int8_t* out) MXQ_INLINE {
-    for (int i = tid; i < TM * chunks; i += 64 * NW) {
-      const int row = quotient(i, magic), j = i - row * chunks, pixel = pixel_of[row];
-      if (pixel >= 0)
-        *reinterpret_cast<v4i*>(out + (static_cast<size_t>(pixel) * chunks + j) * 16) =
-            *reinterpret_cast<const v4i*>(smem + at + (row * pitch + j) * 16);
+  auto leave = [&](int at, int chunks, int pitch, uint32_t magic, int rows, int rest,
+                   const uint32_t* pixel_of, int8_t* out) MXQ_INLINE {
+    const auto to = __builtin_amdgcn_make_buffer_rsrc(
+        out, 0, static_cast<uint32_t>(p.N) * p.H * p.W * chunks * 16, 0x00020000);
+    int row = quotient(tid, magic), j = tid - row * chunks, from = at + (row * pitch + j) * 16;
+    for (int left = TM * chunks; left > 0; left -= 64 * NW) {
+      // (rows past the tile's are written nowhere)
+      const uint32_t pixel = row < TM ? pixel_of[row] : kOutOfRange;
+      __builtin_amdgcn_raw_buffer_store_b128(
+          __builtin_bit_cast(v4u, *reinterpret_cast<const v4i*>(smem + from)), to, pixel + 16 * j, 0,
+          0);
+      row += rows;
+      j += rest;
+      from += (rows * pitch + rest) * 16;
+      const bool carry = j >= chunks;
+      j -= carry ? chunks : 0;
+      row += carry;
+      from += carry ? (pitch - chunks) * 16 : 0;
     }
   };
-  leave(0, CO, PO, p.magic_wide, p.out);
+  leave(0, CO, PO, p.magic_wide, p.wide_rows, p.wide_rest, wide_of, p.out);
   if (p.Ca == 0) return;
 
   // ---- the next block's first 1 x 1 ---------------------------------------------------------
   const int groups_a = p.ka / GA;
   for (int t = wn; t < tiles_a; t += WN) {
-    v4i bias[4];
-    read_bias(sbias + bias_a + 32 * t, bias);
-    start(acc, bias);
-    first_pixels(in_wide, [](int i) { return 32 * i; });
-    for (int g = 0; g < groups_a; ++g)
+    start(acc, sbias + bias_a + 32 * t);
+    first_pixels([&](int i, v4i (&x)[RT]) MXQ_INLINE { read_pixels(x, in_wide, 32 * i); });
+    int at[RT];
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) at[rt] = in_wide[rt];
+    for (int g = 0; g < groups_a; ++g) {
+      const bool last = g + 1 == groups_a;
       run_group(wa,
-                g + 1 < groups_a ? p.at_a + t * p.ka + (g + 1) * GA
-                : t + WN < tiles_a ? p.at_a + (t + WN) * p.ka : kNone,
-                in_wide, [&](int i) { return (g * GA + i) * 32; });
+                fragments(!last || t + WN < tiles_a,
+                          p.at_a + (last ? (t + WN) * p.ka : t * p.ka + (g + 1) * GA)),
+                [&](int i, v4i (&x)[RT]) MXQ_INLINE { read_pixels(x, at, 32 * i); });
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) at[rt] += 32 * GA;
+    }
     finish_layer(s_a, t_a, c_a, (has & 4) != 0, p.relu_a, t, PA);
   }
   publish();
-  leave(p.off_patch, CA, PA, p.magic_next, p.next);
+  leave(p.off_patch, CA, PA, p.magic_next, p.next_rows, p.next_rest, next_of, p.next);
 }
 
-template <int WM, int WN, int RT, int GB, int GC>
+template <int WM, int WN, int RT, int GB, int GC, int KSB>
 __global__ __launch_bounds__(64 * WM * WN, GC < 8 ? 4 : 2) void block_kernel(BlockArgs p) {
   // an XCD takes a run of neighbouring tiles: they share halo rows in its L2
   const int per = (p.tiles + 7) >> 3;
   const int tile = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
-  if (tile < p.tiles) block_tile<WM, WN, RT, GB, GC>(p, tile, tile * 32 * WM * RT);
+  if (tile < p.tiles) block_tile<WM, WN, RT, GB, GC, KSB>(p, tile, tile * 32 * WM * RT);
 }
 
 // Runs of pixels: p.tiles (a multiple of 8) of 64 and the rest in halves behind them.
-template <int GB, int GC>
+template <int GB, int GC, int KSB>
 __global__ __launch_bounds__(512, GC < 8 ? 4 : 2) void block_halves_kernel(BlockArgs p) {
   const int block = blockIdx.x;
   if (block < p.tiles)
-    block_tile<1, 8, 2, GB, GC>(p, 0, 64 * ((block & 7) * (p.tiles >> 3) + (block >> 3)));
+    block_tile<1, 8, 2, GB, GC, KSB>(p, 0, 64 * ((block & 7) * (p.tiles >> 3) + (block >> 3)));
   else
-    block_tile<1, 8, 1, GB, GC>(p, 0, 64 * p.tiles + 32 * (block - p.tiles));
+    block_tile<1, 8, 1, GB, GC, KSB>(p, 0, 64 * p.tiles + 32 * (block - p.tiles));
 }
 
 // [O][taps][C] rows -> fragments [ceil(O / 32)][steps][64 lanes][16 bytes]: lane l of step
@@ -645,9 +718,9 @@ bool fit_lds(BlockPlan* b, int C, int Cm, int Co, int Ca) {
   const int wide = up(b->tm * odd_tiles(Co / 16), 64) * 16;
   const int mid = b->tm * odd_tiles((Cm > Ca ? Cm : Ca) / 16) * 16;
   const int patch = first > mid ? static_cast<int>(first) : mid;
-  const int bias = 4 * (up(Cm, 256) + up(Co, 256) + up(Ca, 256));
+  const int bias = 4 * (up(Cm, 32) + up(Co, 32) + up(Ca, 32));
   const int table = 4 * (b->steps[0] + 2 * 8);
-  const long long lds = static_cast<long long>(wide) + patch + bias + table + 4 * b->tm;
+  const long long lds = static_cast<long long>(wide) + patch + bias + table + 4 * (3 * b->tm + 24);
   b->off_patch = wide;
   b->off_bias = wide + patch;
   b->off_table = b->off_bias + bias;
@@ -733,10 +806,31 @@ BlockPlan plan_block(int N, int H, int W, int C, int Cm, int Co, int Ca) {
 }
 
 template <int WM, int WN, int RT, int GB, int GC>
-void launch_block(hipStream_t s, const BlockArgs& a, int lds) {
-  const unsigned grid = static_cast<unsigned>((a.tiles + 7) / 8 * 8);
-  hipLaunchKernelGGL((block_kernel<WM, WN, RT, GB, GC>), dim3(grid), dim3(64 * WM * WN),
-                     static_cast<size_t>(lds), s, a);
+void launch_block(hipStream_t s, BlockArgs a, const BlockPlan& b) {
+  constexpr int n = 64 * WM * WN, ksb = GC;  // as many channels in as in the middle
+  const int pitch = odd_tiles(a.Co / 16);
+  a.res_rows = n / pitch;
+  a.res_rest = n % pitch;
+  a.wide_rows = n / (a.Co / 16);
+  a.wide_rest = n % (a.Co / 16);
+  a.next_rows = a.Ca ? n / (a.Ca / 16) : 0;
+  a.next_rest = a.Ca ? n % (a.Ca / 16) : 0;
+  const bool known = a.C == 32 * ksb;
+  if (b.halves != 0) {
+    const dim3 grid(static_cast<unsigned>(b.tiles + b.halves));
+    if constexpr (WM == 1 && WN == 8 && RT == 2) {
+      if (known)
+        hipLaunchKernelGGL((block_halves_kernel<GB, GC, ksb>), grid, dim3(n), b.lds, s, a);
+      else
+        hipLaunchKernelGGL((block_halves_kernel<GB, GC, 0>), grid, dim3(n), b.lds, s, a);
+    }
+  } else {
+    const dim3 grid(static_cast<unsigned>((a.tiles + 7) / 8 * 8));
+    if (known)
+      hipLaunchKernelGGL((block_kernel<WM, WN, RT, GB, GC, ksb>), grid, dim3(n), b.lds, s, a);
+    else
+      hipLaunchKernelGGL((block_kernel<WM, WN, RT, GB, GC, 0>), grid, dim3(n), b.lds, s, a);
+  }
   MXQ_LAUNCH_CHECK();
 }
 
@@ -882,26 +976,19 @@ int mxq_quantized_block(void* stream, const int8_t* data, const int8_t* weights,
   a.relu_a = relu_third != 0;
   a.tiles = b.tiles;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (b.halves != 0) {
-    const dim3 grid(static_cast<unsigned>(b.tiles + b.halves));
-    if (b.variant == 128)
-      hipLaunchKernelGGL((block_halves_kernel<6, 4>), grid, dim3(512), b.lds, s, a);
-    else
-      hipLaunchKernelGGL((block_halves_kernel<8, 8>), grid, dim3(512), b.lds, s, a);
-    MXQ_LAUNCH_CHECK();
-  } else if (b.tm == 32) {
+  if (b.tm == 32) {
     if (b.variant == 64)
-      launch_block<1, 4, 1, 6, 2>(s, a, b.lds);
+      launch_block<1, 4, 1, 6, 2>(s, a, b);
     else if (b.variant == 128)
-      launch_block<1, 8, 1, 6, 4>(s, a, b.lds);
+      launch_block<1, 8, 1, 6, 4>(s, a, b);
     else
-      launch_block<1, 8, 1, 8, 8>(s, a, b.lds);
+      launch_block<1, 8, 1, 8, 8>(s, a, b);
   } else if (b.variant == 64) {
-    launch_block<2, 2, 1, 6, 2>(s, a, b.lds);
+    launch_block<2, 2, 1, 6, 2>(s, a, b);
   } else if (b.variant == 128) {
-    launch_block<1, 8, 2, 6, 4>(s, a, b.lds);
+    launch_block<1, 8, 2, 6, 4>(s, a, b);
   } else {
-    launch_block<1, 8, 2, 8, 8>(s, a, b.lds);
+    launch_block<1, 8, 2, 8, 8>(s, a, b);
   }
   MXQ_API_END();
 }

@@ -121,6 +121,19 @@ def test_block_that_ends_in_halves(n, h, w, c, mid, out, after, more):
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("whole", [False, True])
+@pytest.mark.parametrize("n,h,w,c,mid,out,after", [
+    (1, 6, 11, 64, 48, 16, 16), (2, 9, 10, 64, 64, 1040, 0), (1, 5, 5, 128, 16, 16, 48),
+    (2, 9, 10, 128, 96, 208, 16), (1, 7, 10, 256, 256, 16, 32), (2, 7, 7, 256, 240, 1040, 80)])
+def test_block_whose_taps_are_constants(n, h, w, c, mid, out, after, whole):
+    """Exactly the channels that a kernel instance is made for, with one piece a row and with many."""
+    if whole:
+        n += torch.cuda.get_device_properties(0).multi_processor_count * 32 // (h * w) + 1
+    have, want, _ = blocks(n, h, w, c, mid, out, after)
+    for a, b in zip(have, want):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("relu1,relu3", [(0, 0), (1, 0), (0, 1)])
 @pytest.mark.parametrize("mid,spread", [(48, 0.02), (128, 40.0), (160, 1.0)])
 def test_block_ranges_on_whole_tiles(mid, spread, relu1, relu3):
