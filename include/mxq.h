@@ -549,12 +549,20 @@ int mxq_quantized_block(void* stream, const int8_t* data, const int8_t* weights,
  * NaN; workspace as for mxq_quantize_v2.
  * mxq_histogram_f32: counts[k] of the values with edges[k] <= x < edges[k + 1] (the last bin
  * includes its upper edge), `bins` + 1 increasing edges and `bins` counts on the device;
- * values outside and NaN are not counted; n < 2^32. */
+ * values outside and NaN are not counted; n < 2^32.
+ * mxq_symmetric_histogram_f32: both in one go, without a word from the host between them.  `out`, on
+ * the device, receives the two extreme values, 1 or 0, and the `bins` counts (of at most 2^24) over
+ * [-th, th], its edges as numpy.histogram computes them in float32; th of NaN: the larger magnitude
+ * of the two.  0 where those edges do not increase or th is not finite: the counts mean nothing
+ * then.  The workspace is 16-byte aligned. */
 size_t mxq_minmax_f32_workspace(size_t n);
 int mxq_minmax_f32(void* stream, const float* in, size_t n, float* out_min, float* out_max,
                    void* workspace, size_t workspace_bytes);
 int mxq_histogram_f32(void* stream, const float* in, size_t n, const float* edges, int bins,
                       uint32_t* counts);
+size_t mxq_symmetric_histogram_f32_workspace(size_t n, int bins);
+int mxq_symmetric_histogram_f32(void* stream, const float* in, size_t n, int bins, float th,
+                                uint32_t* out, void* workspace, size_t workspace_bytes);
 
 /* Entropy calibration: bounds [lower, upper] of what mxq_calibrate_entropy's float sums give for
  * every candidate threshold, narrowest first, of up to 16 histograms (`hist`, on the device, one

@@ -119,13 +119,31 @@ class _Values:
 
     def __init__(self, arr):
         self._device = self._host = None
+        self._range = self._counts = None
         if (isinstance(arr, torch.Tensor) and arr.is_cuda and arr.dtype == torch.float32 and
                 0 < arr.numel() < 2 ** 32):
             self._device = arr.detach().contiguous()
         else:
             self._host = _to_numpy(arr)
 
+    def measure(self, bins, th=None):
+        """Take the extreme values and the counts over [-th, th] (or over the values' own symmetric
+        range) from the device in one go: one wait for it instead of two, between which it idles.  A
+        first batch of 196608 values in 8001 bins 240 -> 100 us."""
+        if self._device is None or not 0 < bins <= 1 << 24:
+            return
+        if th is not None and not (isinstance(th, np.float32) and np.isfinite(th)):
+            return  # edges in float64, as numpy has them
+        found = capi.symmetric_histogram(self._device, bins, th).cpu().numpy()
+        lo, hi = found[:2].view(np.float32)
+        self._range = lo, hi
+        if found[2]:
+            self._counts = (max(abs(lo), abs(hi)) if th is None else th,
+                            found[3:].view(np.uint32).astype(np.int64))
+
     def extremes(self):
+        if self._range is not None:
+            return self._range
         if self._device is None:
             return np.min(self._host), np.max(self._host)
         lo, hi = capi.minmax(self._device).cpu().numpy()
@@ -133,6 +151,9 @@ class _Values:
 
     def counts(self, bins, th):
         """numpy.histogram(values, bins, range=(-th, th))[0]"""
+        if (self._counts is not None and isinstance(th, np.float32) and th == self._counts[0] and
+                bins == len(self._counts[1])):
+            return self._counts[1]
         if self._device is not None and np.isfinite(th):
             edges = np.histogram_bin_edges(np.empty(0, np.float32), bins=bins, range=(-th, th))
             if edges.dtype == np.float32 and np.all(edges[1:] > edges[:-1]):
@@ -265,8 +286,10 @@ class _LayerHistogramCollector(CalibrationCollector):
         arr = _Values(arr)
         seen = self.hist_dict.get(name)
         if seen is None:
+            arr.measure(self.num_bins)
             self.hist_dict[name] = _SymmetricHistogram.of(arr, self.num_bins).as_tuple()
         else:
+            arr.measure(len(seen[0]), seen[4])
             lo, hi = arr.extremes()
             self.hist_dict[name] = self.combine_histogram(seen, arr, lo, hi,
                                                           max(abs(lo), abs(hi)))

@@ -57,3 +57,32 @@ def test_collector_on_device_tensors_is_the_host_collector():
     for h, d in zip(on_host.hist_dict["t"], on_device.hist_dict["t"]):
         assert np.array_equal(h, d)
     assert on_host.post_collect() == on_device.post_collect()
+
+
+@pytest.mark.parametrize("bins", [1, 2, 255, 8001, 16384, 20001])
+@pytest.mark.parametrize("th", [None, 1e-33, 0.7, 1.6e38])  # bins of normal width: numpy has no others
+def test_symmetric_histogram_is_the_two_calls(bins, th):
+    """Values on numpy's edges and beside them, so that an edge one last place off would show."""
+    top = np.float32(2.7 if th is None else th)
+    edges = np.histogram_bin_edges(np.empty(0, np.float32), bins=bins, range=(-top, top))
+    assert edges.dtype == np.float32
+    x = np.concatenate([edges, np.nextafter(edges, np.float32(0)), edges[::3] * np.float32(0.3)])
+    if th is not None and top < 1e38:
+        x = np.append(x, 2 * top).astype(np.float32)
+    v = Q._Values(torch.from_numpy(x).cuda())
+    v.measure(bins, None if th is None else top)
+    assert v.extremes() == (x.min(), x.max())
+    assert v._counts is not None
+    got = v.counts(bins, top)
+    assert np.array_equal(got, Q._Values(torch.from_numpy(x).cuda()).counts(bins, top))
+    assert np.array_equal(got, np.histogram(x, bins=bins, range=(-top, top))[0])
+
+
+@pytest.mark.parametrize("value", [0.0, float("nan"), float("inf")])
+def test_symmetric_histogram_without_a_range(value):
+    x = torch.full((1000,), value, device="cuda")
+    v = Q._Values(x)
+    v.measure(101)
+    assert v._counts is None
+    lo, hi = v.extremes()
+    assert (np.isnan(lo) and np.isnan(hi)) if np.isnan(value) else (lo, hi) == (value, value)
