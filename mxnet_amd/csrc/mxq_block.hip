@@ -29,9 +29,12 @@
 // not arithmetic has as few as possible: a weight's place is a scalar offset and an immediate, the three
 // taps of a row are immediates where the channels are those of a kernel instance (KSB), the places of a
 // tile's pixels in the tensors come from a table, and pieces of rows are walked by carries, not divided
-// (984 -> 760 vector instructions a wave of 56 x 56 x 64, of which 550 are arithmetic).  Measured in a
-// quantized ResNet-50's pass at batch 64, before and after: 46.2 -> 40.4 us for 56 x 56 x 64 -> 256 ->
-// 64, 34.4 -> 32.3 for 28 x 28 x 128, 26.7 -> 25.4 for 14 x 14 x 256; the pass 613 -> 592.  As three
+// (984 -> 760 vector instructions a wave of 56 x 56 x 64, of which 550 are arithmetic); and a barrier
+// waits for what it is for, not for weights or stores on their way.  The 3 x 3 layer of 256 channels is
+// bound by the 64 bytes a clock that a CU takes in (its 590 KB of weights: 9200 clocks, as many as the
+// products take; 10000 measured), as is the time in front of it.  Measured in a quantized ResNet-50's
+// pass at batch 64, before and after: 46.2 -> 38.9 us for 56 x 56 x 64 -> 256 -> 64, 34.4 -> 30.6 for
+// 28 x 28 x 128, 26.7 -> 23.9 for 14 x 14 x 256; the pass 593 -> 566, one image 200.3 -> 193.6.  As three
 // launches they were 60, 45 and 38 us.
 // Measured and not kept: the 3 x 3 layer's reduction shared by the waves that have no column tile of
 // it (up to 128 channels in the middle half of them), or by 16 waves: level or behind, for the sums
@@ -118,8 +121,8 @@ struct BlockArgs {
   // what NW * 64 pieces are in rows and pieces beyond them, of the shortcut's slots and of the outputs
   int res_rows, res_rest, wide_rows, wide_rest, next_rows, next_rest;
   int parts, row_pitch;   // load instructions and bytes per row of the patch
-  uint32_t magic_tiles_w, magic_tiles_h, magic_area, magic_across, magic_h2, magic_pixel, magic_res,
-      magic_wide, magic_next, magic_tap;
+  uint32_t magic_tiles_w, magic_tiles_h, magic_area, magic_across, magic_h2, magic_pixel,
+      magic_res, magic_wide, magic_next, magic_tap;
   int relu_b, relu_a, tiles;
 };
 
@@ -218,32 +221,42 @@ __device__ __forceinline__ void block_tile(const BlockArgs& p, int tile, int fir
   // either side; zeros where they leave the image
   {
     const v4i rsrc = make_rsrc(p.data, static_cast<uint32_t>(p.N) * p.H * p.W * p.C);
-    // A row of the patch is a whole number of load instructions: a lane's place in the row stays as
-    // the wave goes down the rows, and a row is one scalar offset.  (A lane that finds its pixel
-    // anew for every piece, by divisions or by carries, costs 300 clocks per instruction.)
-    int j = lane, px = 0;
+    // A row of the patch is a whole number of load instructions, and a row is one scalar offset: the
+    // lanes look at a row each, all at once, and what they find is read from them row by row; a lane's
+    // place in a row moves on by carries from part to part.  Parts start at the wave behind the one that
+    // took the last row of the part before, so that all take as many.  (An instruction takes a lone wave
+    // five clocks here: looking at the row for every load, 55 instructions, 14 x 14 x 256 had 3200
+    // clocks in front of its patch, and 28 x 28 x 128 2300.)  No short circuits: a branch takes longer than
+    // what it skips.
     const int row_bytes = p.W * p.C;
-    int carry = quotient(j, p.magic_pixel);
-    j -= carry * PP;
-    px += carry;
-    const int step = quotient(64, p.magic_pixel), rest = 64 - step * PP;
-    for (int part = 0; part < p.parts; ++part) {
-      const int iw = w0 + px - 1;
-      const bool ok = j < CH && px < p.across + 2 &&
-                      static_cast<unsigned>(iw) < static_cast<unsigned>(p.W);
-      const uint32_t place = ok ? static_cast<uint32_t>(iw * p.C + 16 * j) : kOutOfRange;
-      for (int r = wave; r < p.rows; r += NW) {
-        const int n = quotient_any(v0 + r, H2, p.magic_h2), ih = v0 + r - n * H2 - 1;
-        const bool inside = n < p.N && static_cast<unsigned>(ih) < static_cast<unsigned>(p.H);
-        fetch(p.off_patch + r * row_pitch + part * 1024,
-              inside ? place + static_cast<uint32_t>((n * p.H + ih) * row_bytes) : kOutOfRange,
-              rsrc);
+    const int px_step = quotient(64, p.magic_pixel), j_rest = 64 - px_step * PP;
+    for (int first_row = 0; first_row < p.rows; first_row += 64) {
+      uint32_t row_at, row_none;
+      {
+        const int v = v0 + first_row + lane, n = quotient_any(v, H2, p.magic_h2), ih = v - n * H2 - 1;
+        const int none = (n >= p.N) | (static_cast<unsigned>(ih) >= static_cast<unsigned>(p.H));
+        row_at = static_cast<uint32_t>((n * p.H + ih) * row_bytes);
+        row_none = static_cast<uint32_t>(none) << 31;
       }
-      j += rest;
-      px += step;
-      if (j >= PP) {
-        j -= PP;
-        ++px;
+      const int rows = p.rows - first_row < 64 ? p.rows - first_row : 64;
+      int px = quotient(lane, p.magic_pixel), j = lane - px * PP, before = 0;
+      for (int part = 0; part < p.parts; ++part) {
+        const int iw = w0 + px - 1;
+        const int none = (j >= CH) | (px >= p.across + 2) |
+                         (static_cast<unsigned>(iw) >= static_cast<unsigned>(p.W));
+        const uint32_t at = static_cast<uint32_t>(__mul24(iw, p.C) + 16 * j);
+        const uint32_t outside = static_cast<uint32_t>(none) << 31;
+        for (int r = (wave - before) & (NW - 1); r < rows; r += NW)
+          fetch(p.off_patch + (first_row + r) * row_pitch + part * 1024,
+                (at + __builtin_amdgcn_readlane(row_at, r)) |
+                    (outside | __builtin_amdgcn_readlane(row_none, r)),
+                rsrc);
+        before += rows;
+        j += j_rest;
+        px += px_step;
+        const int carry = j >= PP;
+        j -= carry ? PP : 0;
+        px += carry;
       }
     }
   }
@@ -253,32 +266,38 @@ __device__ __forceinline__ void block_tile(const BlockArgs& p, int tile, int fir
   uint32_t* const wide_of = reinterpret_cast<uint32_t*>(smem + p.off_pixel);
   uint32_t* const next_of = wide_of + TM + kMore;
   int* const place_of = reinterpret_cast<int*>(next_of + TM);
-  if (tid < TM) {
+  static_assert(TM <= 64 && kMore <= TM, "one wave makes the tables");
+  if (wave == NW - 1 && lane < TM) {  // the wave that has least to fetch
     // rows without a pixel read the first one's; never stored
-    const int i = start_at + (tid < p.count ? tid : 0);
+    const int i = start_at + (lane < p.count ? lane : 0);
     const int img = quotient_any(i, p.area, p.magic_area), rem = i - img * p.area;
     const int ty = quotient(rem, p.magic_across), tx = rem - ty * p.across;
     const int n = n0 + img, h = h0 + ty, w = w0 + tx;
-    const bool ok = tid < p.count && n < p.N && h < p.H && w < p.W;
+    const bool ok = lane < p.count && n < p.N && h < p.H && w < p.W;
     const uint32_t pixel = static_cast<uint32_t>((n * p.H + h) * p.W + w);
-    wide_of[tid] = ok ? pixel * p.Co : kOutOfRange;
-    next_of[tid] = ok ? pixel * p.Ca : kOutOfRange;
-    place_of[tid] = (n * H2 + h - v0) * row_pitch + tx * PP * 16;
-    if (tid < kMore) wide_of[TM + tid] = kOutOfRange;
+    wide_of[lane] = ok ? pixel * p.Co : kOutOfRange;
+    next_of[lane] = ok ? pixel * p.Ca : kOutOfRange;
+    place_of[lane] = (n * H2 + h - v0) * row_pitch + tx * PP * 16;
+    if (lane < kMore) wide_of[TM + lane] = kOutOfRange;
   }
   const int* const sbias = reinterpret_cast<const int*>(smem + p.off_bias);
   const int bias_c = (p.Cm + 31) & ~31, bias_a = bias_c + ((p.Co + 31) & ~31);
-#pragma unroll
-  for (int layer = 0; layer < 3; ++layer) {
-    const int columns = layer == 0 ? p.Cm : layer == 1 ? p.Co : p.Ca;
-    const int at = layer == 0 ? 0 : layer == 1 ? bias_c : bias_a;
-    if (columns != 0) {  // whole column tiles, zeros behind the last column
-      const v4i rsrc = make_rsrc(p.prepared[layer] + kPreparedBias, 4u * columns);
-      for (int it = wave; it * 256 < columns; it += NW)
-        if (it * 256 + lane * 4 < ((columns + 31) & ~31))
-          fetch(p.off_bias + at * 4 + it * 1024, it * 1024 + lane16, rsrc);
+  // Whole column tiles of a layer's bias, zeros behind its last column: those of the 3 x 3 layer now,
+  // the others' while that one runs.
+  auto fetch_bias = [&](const char* prepared, int columns, int at, int i) MXQ_INLINE {
+    const v4i rsrc = make_rsrc(prepared + kPreparedBias, 4u * columns);
+    if (i * 256 + lane * 4 < ((columns + 31) & ~31))
+      fetch(p.off_bias + at * 4 + i * 1024, i * 1024 + lane16, rsrc);
+  };
+  if (wave == 0) fetch_bias(p.prepared[0], p.Cm, 0, 0);  // no more than 256
+  auto fetch_later_bias = [&]() MXQ_INLINE {
+    const int n_c = (p.Co + 255) >> 8, n_a = (p.Ca + 255) >> 8;
+    for (int it = NW - 1 - wave; it < n_c + n_a; it += NW) {
+      const bool c = it < n_c;
+      fetch_bias(c ? p.prepared[1] : p.prepared[2], c ? p.Co : p.Ca, c ? bias_c : bias_a,
+                 c ? it : it - n_c);
     }
-  }
+  };
   const EpiScalars s_b = p.forms->s[0], s_c = p.forms->s[1], s_a = p.forms->s[2];
   const RequantRule rule = p.forms->rule;
   const float t_b = p.forms->t[0], t_c = p.forms->t[1], t_a = p.forms->t[2];
@@ -370,12 +389,20 @@ __device__ __forceinline__ void block_tile(const BlockArgs& p, int tile, int fir
       __builtin_amdgcn_sched_barrier(0);
     }
   };
-  auto publish = [&]() MXQ_INLINE {  // what this wave wrote to LDS or had written there, to all of them
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+  // What this wave wrote to LDS, and what it had written there but for the newest `pending` loads, to
+  // all of them.  Only what the barrier is for is waited for: weights on their way to registers, or
+  // stores, at a barrier that publishes a result cost 1000 to 2500 clocks each.
+  auto publish = [&](auto pending) MXQ_INLINE {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(decltype(pending)::value) : "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
   };
-  publish();
+  auto publish_written = [&]() MXQ_INLINE {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  publish(std::integral_constant<int, 0>());  // the patch, the bias, the tables
 
   // ---- 3 x 3 ------------------------------------------------------------------------------
   const int groups = p.kb / GB;
@@ -400,6 +427,9 @@ __device__ __forceinline__ void block_tile(const BlockArgs& p, int tile, int fir
 #pragma unroll
         for (int g = 0; g < kRow / GB; ++g) {
           fetch_shortcut();
+          // (the last of them a latency ahead of the barrier behind the layer)
+          if constexpr (GC == 8) fetch_shortcut();
+          if (g == 0 && row == 1) fetch_later_bias();
           run_group(wb,
                     fragments(row < 2 || g + 1 < kRow / GB, first_b + row * kRow + (g + 1) * GB),
                     [&](int i, v4i (&x)[RT]) MXQ_INLINE { read(g * GB + i, x); });
@@ -422,12 +452,15 @@ __device__ __forceinline__ void block_tile(const BlockArgs& p, int tile, int fir
       first_pixels(read);
       for (int g = 0; g < groups; ++g) {
         fetch_shortcut();
+        if (g == 0) fetch_later_bias();
         run_group(wb, fragments(g + 1 < groups, first_b + (g + 1) * GB), read);
 #pragma unroll
         for (int i = 0; i < GB; ++i) now[i] = later[i];
         read_offsets(g + 2, later);
       }
     }
+  } else {
+    fetch_later_bias();
   }
   while (res_at * 64 < res_slots) fetch_shortcut();
   v4i wc[GC];
@@ -457,7 +490,7 @@ __device__ __forceinline__ void block_tile(const BlockArgs& p, int tile, int fir
   __builtin_amdgcn_s_barrier();  // every wave is through with the patch
   asm volatile("" ::: "memory");
   if (has_b) finish_layer(s_b, t_b, c_b, (has & 1) != 0, p.relu_b, wn, PM);
-  publish();
+  publish(std::integral_constant<int, GC>());  // the result, and the shortcut in front of `wc`
 
   // ---- 1 x 1 and the sum ------------------------------------------------------------------
   // where this lane's rows are read as an operand, and where its outputs of a column tile lie
@@ -515,7 +548,7 @@ __device__ __forceinline__ void block_tile(const BlockArgs& p, int tile, int fir
     widen(std::integral_constant<int, 0>());
   v4i wa[GA];
   if (p.Ca != 0) load_first(wa, fragments(wn < tiles_a, p.at_a + wn * p.ka));
-  publish();
+  publish_written();
 
   // Rows of `chunks` pieces, `pitch` apart in LDS, to their pixels.  Plain stores: the next block
   // reads both outputs, and what it finds in the memory-side cache it does not fetch from memory
@@ -562,7 +595,7 @@ __device__ __forceinline__ void block_tile(const BlockArgs& p, int tile, int fir
     }
     finish_layer(s_a, t_a, c_a, (has & 4) != 0, p.relu_a, t, PA);
   }
-  publish();
+  publish_written();
   leave(p.off_patch, CA, PA, p.magic_next, p.next_rows, p.next_rest, next_of, p.next);
 }
 
