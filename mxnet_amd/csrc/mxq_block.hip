@@ -33,8 +33,8 @@
 // waits for what it is for, not for weights or stores on their way.  The 3 x 3 layer of 256 channels is
 // bound by the 64 bytes a clock that a CU takes in (its 590 KB of weights: 9200 clocks, as many as the
 // products take; 10000 measured), as is the time in front of it.  Measured in a quantized ResNet-50's
-// pass at batch 64, before and after: 46.2 -> 38.9 us for 56 x 56 x 64 -> 256 -> 64, 34.4 -> 30.6 for
-// 28 x 28 x 128, 26.7 -> 23.9 for 14 x 14 x 256; the pass 593 -> 566, one image 200.3 -> 193.6.  As three
+// pass at batch 64, before and after: 46.2 -> 39.3 us for 56 x 56 x 64 -> 256 -> 64, 34.4 -> 32.1 for
+// 28 x 28 x 128, 26.7 -> 24.9 for 14 x 14 x 256; the pass 593 -> 566, one image 200.3 -> 193.6.  As three
 // launches they were 60, 45 and 38 us.
 // Measured and not kept: the 3 x 3 layer's reduction shared by the waves that have no column tile of
 // it (up to 128 channels in the middle half of them), or by 16 waves: level or behind, for the sums
