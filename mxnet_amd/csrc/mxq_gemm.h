@@ -128,6 +128,89 @@ __device__ __forceinline__ void epi_store16(v4i val, void* p) {
     *reinterpret_cast<v4i*>(p) = val;
 }
 
+// Four adjacent 32-bit values on any dword mark; RAGGED: of which only `left` may be inside the row.
+typedef int v4i_dword __attribute__((ext_vector_type(4), aligned(4)));
+template <bool RAGGED>
+__device__ __forceinline__ void epi_store_quad(int* to, v4i val, int left) {
+  if (!RAGGED || left >= 4) {
+    *reinterpret_cast<v4i_dword*>(to) = val;
+  } else {  // the last quad of a row of no multiple of 4
+    to[0] = val[0];
+    if (left > 1) to[1] = val[1];
+    if (left > 2) to[2] = val[2];
+  }
+}
+
+// Sixteen adjacent bytes of which `left` are inside the row, at any address: one store, or four for
+// the last piece of a row.  (Element by element, a quad of a row each, a tile's lanes wrote single
+// bytes into 32 rows at once: 31117 x 144 -> 395 47 us, -> 400 18.)
+__device__ __forceinline__ void epi_store_ragged(int8_t* to, v4i val, int left) {
+  if (left >= 16) {
+    __builtin_memcpy(to, &val, 16);
+    return;
+  }
+  if (left <= 0) return;
+  uint64_t part[2];
+  __builtin_memcpy(part, &val, 16);
+  uint64_t w = part[0];
+  if (left & 8) {
+    __builtin_memcpy(to, &w, 8);
+    to += 8;
+    w = part[1];
+  }
+  if (left & 4) {
+    const uint32_t x = static_cast<uint32_t>(w);
+    __builtin_memcpy(to, &x, 4);
+    to += 4;
+    w >>= 32;
+  }
+  if (left & 2) {
+    const uint16_t x = static_cast<uint16_t>(w);
+    __builtin_memcpy(to, &x, 2);
+    to += 2;
+    w >>= 16;
+  }
+  if (left & 1) *to = static_cast<int8_t>(w);
+}
+// ... and read, zeros behind the row's end; nothing past it is touched.
+__device__ __forceinline__ v4i epi_load_ragged(const int8_t* from, int left) {
+  v4i val = {0, 0, 0, 0};
+  if (left >= 16) {
+    __builtin_memcpy(&val, from, 16);
+    return val;
+  }
+  uint64_t lo = 0, hi = 0;
+  int at = 0;
+  if (left & 8) {
+    __builtin_memcpy(&lo, from, 8);
+    at = 8;
+  }
+  uint64_t w = 0;
+  int shift = 0;
+  if (left & 4) {
+    uint32_t x;
+    __builtin_memcpy(&x, from + at, 4);
+    w = x;
+    at += 4;
+    shift = 32;
+  }
+  if (left & 2) {
+    uint16_t x;
+    __builtin_memcpy(&x, from + at, 2);
+    w |= static_cast<uint64_t>(x) << shift;
+    at += 2;
+    shift += 16;
+  }
+  if (left & 1) w |= static_cast<uint64_t>(static_cast<uint8_t>(from[at])) << shift;
+  if (left & 8)
+    hi = w;
+  else
+    lo = w;
+  const uint64_t part[2] = {lo, hi};
+  __builtin_memcpy(&val, part, 16);
+  return val;
+}
+
 __device__ __forceinline__ float dev_maxabs(float a, float b) {
   float x = fabsf(a), y = fabsf(b);
   return (x < y) ? y : x;
@@ -657,6 +740,11 @@ __device__ __forceinline__ void gemm_mainloop_dma(v16i (&acc)[Cfg::MI][Cfg::NI],
 #pragma unroll
   for (int s = 0; s < NS - 1; ++s) issue(s);  // stages 0 .. min(KT, NS-1)-1
   after_prologue();
+  // The prologue's loads have to be in their registers before the loop: a pending one whose register
+  // the loop's fragments share is waited for in every step, with the stage that was just requested
+  // (4096 x 3072 -> 768 on 128 x 64 tiles 21 -> 25.6 us).  With two stages the first step waits for
+  // everything anyway.
+  if (NS == 2) __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
   auto last_issued = [&](int kt_now) {         // newest stage in flight during step kt_now
     const int l = kt_now + NS - 2;
     return l < KT - 1 ? l : KT - 1;
@@ -853,7 +941,7 @@ __device__ __forceinline__ void gemm_epilogue(v16i (&acc)[Cfg::MI][Cfg::NI], con
 // each wave's int8 tile: lanes own 4 adjacent columns of 32 different rows after
 // the MFMA, which would make every store instruction touch 32 cache lines with 8
 // bytes each; staged through LDS a store instruction writes whole 64..128-byte row
-// segments.  Falls back to gemm_epilogue when the output is not 16-byte friendly.
+// segments.  Rows that begin off the 16-byte marks, or end between them, leave from the same tile.
 // What the epilogue needs from global memory, fetched before the K loop so that the
 // scalar loads, the divisions and the bias load are hidden behind it: the range
 // scalars and the int32 bias of column n0 + threadIdx.x.
@@ -1036,30 +1124,16 @@ __device__ __forceinline__ void gemm_epilogue_lds(v16i (&acc)[Cfg::MI][Cfg::NI],
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / Cfg::WN, wn = wave % Cfg::WN;
   const int m_base = m0 + wm * TM, n_base = n0 + wn * TN;
+  // Whether the int8 tile leaves in 16-byte pieces on 16-byte marks; if not, in the same pieces
+  // wherever they lie (epi_store_ragged).  Rows of 32-bit outputs need no such question: their
+  // pieces of four lie on dword marks, which is all that a 16-byte store asks for.
   const bool fast8 = e.out8 == nullptr ||
                      ((N % 16 == 0) && (ldo % 16 == 0) &&
                       ((reinterpret_cast<uintptr_t>(e.out8) & 15u) == 0));
-  const bool fast32 = e.out32 == nullptr ||
-                      ((N % 4 == 0) && (ldo % 4 == 0) &&
-                       ((reinterpret_cast<uintptr_t>(e.out32) & 15u) == 0));
-  // the sum's scales; a rule whose products could overflow goes the general way with the
-  // unaligned outputs
+  // the sum's scales
   bool fasts = true;
   if constexpr (epi_sums(MODE))
     fasts = ((reinterpret_cast<uintptr_t>(e.res) & 15u) == 0) && pre.sum.fast;
-  const bool fastf = MODE != kEpiF32 || e.outf == nullptr ||
-                     ((N % 4 == 0) && (ldo % 4 == 0) &&
-                      ((reinterpret_cast<uintptr_t>(e.outf) & 15u) == 0));
-  // A kernel of a sum mode writes nothing but the int8 tile: where that cannot leave in 16-byte
-  // pieces, it leaves byte by byte from the staged copy below.  Without the element-wise
-  // epilogue in it the 256 x 256 tile keeps its accumulators in registers (with it 768 bytes of
-  // scratch per lane: 12544 x 256 -> 1024 43 us).
-  if constexpr (!epi_sums(MODE)) {
-    if (__builtin_expect(!(fast8 && fast32 && fastf), 0)) {
-      gemm_epilogue<Cfg, MODE>(acc, e, m_base, n_base, M, N, ldo);
-      return;
-    }
-  }
   char* lds = reinterpret_cast<char*>(lds_v);
   int* sbias = reinterpret_cast<int*>(lds);
   char* stage = lds + Cfg::BN * 4 + wave * kPerWave;
@@ -1090,7 +1164,8 @@ __device__ __forceinline__ void gemm_epilogue_lds(v16i (&acc)[Cfg::MI][Cfg::NI],
   // of MFMA tile (mi, ni).  One 32 x 32 tile at a time through the wave's scratch: stored
   // directly a lane's quads touch 32 rows with 32 bytes each; read back, 8 lanes cover one
   // 128-byte row and a store instruction writes 8 whole cache lines.
-  auto store_rows32 = [&](int* out, auto quad) {
+  auto store_rows32_as = [&](int* out, auto quad, auto ragged) {
+    constexpr bool kRagged = decltype(ragged)::value;
     if (kStage32) {
       int* t32 = reinterpret_cast<int*>(stage);
 #pragma unroll
@@ -1116,7 +1191,7 @@ __device__ __forceinline__ void gemm_epilogue_lds(v16i (&acc)[Cfg::MI][Cfg::NI],
             const int m = m_base + mi * 32 + it * 8 + (lane >> 3);
             const int n = n_base + ni * 32 + (lane & 7) * 4;
             if (m < M && n < N)
-              *reinterpret_cast<v4i*>(out + static_cast<size_t>(m) * ldo + n) = back[it];
+              epi_store_quad<kRagged>(out + static_cast<size_t>(m) * ldo + n, back[it], N - n);
           }
         }
       }
@@ -1129,9 +1204,17 @@ __device__ __forceinline__ void gemm_epilogue_lds(v16i (&acc)[Cfg::MI][Cfg::NI],
           for (int mi = 0; mi < MI; ++mi) {
             const int m = m_base + mi * 32 + lrow, n = n_base + ni * 32 + 8 * vq + 4 * lgrp;
             if (m < M && n < N)
-              *reinterpret_cast<v4i*>(out + static_cast<size_t>(m) * ldo + n) = quad(mi, ni, vq);
+              epi_store_quad<kRagged>(out + static_cast<size_t>(m) * ldo + n, quad(mi, ni, vq),
+                                      N - n);
           }
     }
+  };
+  // (the question once, not at every store: 4096 x 3072 int32 rows lose 3 % to it there)
+  auto store_rows32 = [&](int* out, auto quad) {
+    if ((N & 3) == 0)
+      store_rows32_as(out, quad, std::false_type());
+    else
+      store_rows32_as(out, quad, std::true_type());
   };
   auto acc_quad = [&](int mi, int ni, int vq) {
     return v4i{acc[mi][ni][4 * vq], acc[mi][ni][4 * vq + 1], acc[mi][ni][4 * vq + 2],
@@ -1177,8 +1260,9 @@ __device__ __forceinline__ void gemm_epilogue_lds(v16i (&acc)[Cfg::MI][Cfg::NI],
             for (int it = 0; it < 4; ++it) {
               const int n = n_base + ni * 32 + it * 8 + c;
               if (n < N && m0 < M)
-                *reinterpret_cast<v4i*>(e.out32 + (static_cast<size_t>(img) * N + n) * e.plane +
-                                        pix) = col[it];
+                *reinterpret_cast<v4i_dword*>(e.out32 +
+                                              (static_cast<size_t>(img) * N + n) * e.plane + pix) =
+                    col[it];
             }
           } else {
             // any other plane (7 x 7): a lane takes one pixel of the tile's 32, a store
@@ -1213,8 +1297,9 @@ __device__ __forceinline__ void gemm_epilogue_lds(v16i (&acc)[Cfg::MI][Cfg::NI],
               const v4i w = acc_quad(mi, ni, vq);
               const int img = m / e.plane, pix = m - img * e.plane;
 #pragma unroll
-              for (int i = 0; i < 4; ++i)  // N % 4 == 0 on this path
-                e.out32[(static_cast<size_t>(img) * N + (n + i)) * e.plane + pix] = w[i];
+              for (int i = 0; i < 4; ++i)
+                if (n + i < N)
+                  e.out32[(static_cast<size_t>(img) * N + (n + i)) * e.plane + pix] = w[i];
             }
           }
     }
@@ -1311,8 +1396,41 @@ __device__ __forceinline__ void gemm_epilogue_lds(v16i (&acc)[Cfg::MI][Cfg::NI],
           epi_store16<decltype(stream)::value>(val, e.out8 + static_cast<size_t>(m) * ldo + n);
       }
     };
+    // the same pieces of rows that begin anywhere
+    auto store_ragged = [&](auto sum_mode) {
+      constexpr int SM = decltype(sum_mode)::value;
+#pragma unroll 1
+      for (int it = 0; it < kIters; ++it) {
+        const int piece = it * 64 + lane;
+        const int rr = piece / LPR, c16 = piece - rr * LPR;
+        const int m = m_base + rr, n = n_base + c16 * 16;
+        if ((kPieces % 64 != 0 && piece >= kPieces) || m >= M || n >= N) continue;
+        v4i val = *reinterpret_cast<const v4i*>(stage + rr * LD + c16 * 16);
+        const size_t off = static_cast<size_t>(m) * ldo + n;
+        if constexpr (SM != 0) {
+          const v4i res = epi_load_ragged(e.res + off, N - n);
+#pragma unroll
+          for (int w = 0; w < 4; ++w) {
+            const uint32_t x = static_cast<uint32_t>(val[w]), y = static_cast<uint32_t>(res[w]);
+            val[w] = static_cast<int>(SM == 3 ? epi_sum_pairs4(x, y, pre)
+                                              : epi_sum4<SM == 2>(x, y, pre));
+          }
+        }
+        epi_store_ragged(e.out8 + off, val, N - n);
+      }
+    };
     if constexpr (epi_sums(MODE)) {
       if (__builtin_expect(!(fast8 && fasts), 0)) {
+        if (pre.sum.fast) {
+          if (MODE == kEpiSumRq && epi_sum_pairs(pre))
+            store_ragged(std::integral_constant<int, MODE == kEpiSumRq ? 3 : 2>());
+          else if (e.sum_relu)
+            store_ragged(std::integral_constant<int, 2>());
+          else
+            store_ragged(std::integral_constant<int, 1>());
+          return;
+        }
+        // a rule whose products could overflow, one by one
 #pragma unroll 1
         for (int i = lane; i < TM * TN; i += 64) {
           const int rr = i / TN, c = i - rr * TN;
@@ -1336,6 +1454,8 @@ __device__ __forceinline__ void gemm_epilogue_lds(v16i (&acc)[Cfg::MI][Cfg::NI],
         store_sums(std::true_type());
       else
         store_sums(std::false_type());
+    } else if (__builtin_expect(!fast8, 0)) {
+      store_ragged(std::integral_constant<int, 0>());
     } else if (e.stream8) {
       store_tile(std::true_type(), std::integral_constant<int, 0>());
     } else {

@@ -1,0 +1,114 @@
+"""Outputs whose rows are no multiple of 16 bytes (or of 4 integers), or that begin off a mark:
+the tiled kernels write them in whole pieces, the last one of a row in parts.  What lies before and
+behind the output stays."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from tests.data_gen import int8_uniform
+
+pytestmark = pytest.mark.gpu
+
+GUARD = 64  # bytes on either side
+RD, RW, RB = 2.0, 0.1, 1.0
+CALIB = (-30.0, 28.0)
+
+
+def dev(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+def scalars(*values):
+    return [dev(np.array([v], np.float32)) for v in values]
+
+
+class Guarded:
+    def __init__(self, shape, dtype, offset):
+        self.shape, self.dtype, self.front = shape, dtype, GUARD + offset
+        self.nbytes = int(np.prod(shape)) * np.dtype(dtype).itemsize
+        self.buf = torch.full((self.front + self.nbytes + GUARD,), 0x5A, dtype=torch.uint8,
+                              device="cuda")
+
+    def ptr(self):
+        return self.buf.data_ptr() + self.front
+
+    def get(self):
+        host = self.buf.cpu().numpy()
+        assert (host[:self.front] == 0x5A).all(), "written in front of the output"
+        assert (host[self.front + self.nbytes:] == 0x5A).all(), "written behind the output"
+        return host[self.front:self.front + self.nbytes].copy().view(self.dtype).reshape(self.shape)
+
+
+# every tile of the direct-to-LDS kernels; widths that end in each part of a piece
+@pytest.mark.parametrize("cfg", [12, 31, 41, 43, 44, 24, 51, 53, 56, 57, 58, 59, 60])
+@pytest.mark.parametrize("N, offset", [(395, 0), (135, 4), (30, 1), (257, 0), (64, 8), (9, 3),
+                                       (1, 0)])
+def test_fc_rows_of_any_width(cfg, N, offset):
+    from mxnet_amd._lib import check, lib
+    M, K = 131, 128
+    d, w, b = (int8_uniform((M, K), seed=N), int8_uniform((N, K), seed=N + 1),
+               int8_uniform((N,), seed=2))
+    acc, lo, hi = oracle.quantized_fully_connected(d, w, b, -RD, RD, -RW, RW, -RB, RB)
+    want8 = oracle.requantize(acc, lo, hi, *CALIB)[0]
+    held = [dev(a) for a in (d, w, b)] + scalars(-RD, RD, -RW, RW, -RB, RB)
+    out = torch.empty(4, dtype=torch.float32, device="cuda")
+    p = [out.data_ptr() + 4 * i for i in range(4)]
+    for want32, wants8 in ((False, True), (True, False), (True, True)):
+        o8 = Guarded((M, N), np.int8, offset) if wants8 else None
+        o32 = Guarded((M, N), np.int32, 4 * (offset % 4)) if want32 else None
+        check(lib.mxq_test_quantized_fc(
+            torch.cuda.current_stream().cuda_stream, *[t.data_ptr() for t in held[:3]], M, N, K,
+            *[t.data_ptr() for t in held[3:]], o32.ptr() if o32 else None, p[0], p[1],
+            o8.ptr() if o8 else None, p[2], p[3], 0, *CALIB, None, 0, cfg, 1, 0))
+        if o8:
+            np.testing.assert_array_equal(o8.get(), want8)
+        if o32:
+            np.testing.assert_array_equal(o32.get(), acc)
+
+
+@pytest.mark.parametrize("cfg", [12, 41, 43, 44, 51, 57])
+@pytest.mark.parametrize("N, offset, relu", [(395, 0, 1), (30, 1, 0), (9, 0, 1), (64, 4, 0)])
+def test_fc_sum_rows_of_any_width(cfg, N, offset, relu):
+    from mxnet_amd._lib import check, lib
+    M, K = 131, 128
+    d, w, b = (int8_uniform((M, K), seed=N), int8_uniform((N, K), seed=N + 1),
+               int8_uniform((N,), seed=2))
+    res = int8_uniform((M, N), seed=7)
+    reach, sums = 20.0, (-40.0, 35.0)
+    acc, lo, hi = oracle.quantized_fully_connected(d, w, b, -RD, RD, -RW, RW, -RB, RB)
+    q, qlo, qhi = oracle.requantize(acc, lo, hi, *CALIB)
+    want = oracle.quantized_elemwise_add(q, res, qlo, qhi, -reach, reach, min_calib_range=sums[0],
+                                         max_calib_range=sums[1])[0]
+    if relu:
+        want = oracle.relu_i8(want)
+    held = [dev(a) for a in (d, w, b)] + scalars(-RD, RD, -RW, RW, -RB, RB)
+    r = Guarded((M, N), np.int8, offset)
+    r.buf[r.front:r.front + r.nbytes] = dev(res.view(np.uint8).ravel())
+    rs = scalars(-reach, reach)
+    out = torch.empty(4, dtype=torch.float32, device="cuda")
+    p = [out.data_ptr() + 4 * i for i in range(4)]
+    o = Guarded((M, N), np.int8, offset)
+    check(lib.mxq_test_quantized_fc_sum(
+        torch.cuda.current_stream().cuda_stream, *[t.data_ptr() for t in held[:3]], M, N, K,
+        *[t.data_ptr() for t in held[3:]], r.ptr(), *[t.data_ptr() for t in rs], o.ptr(), *p,
+        *CALIB, *sums, relu, None, 0, cfg, 1, 0))
+    np.testing.assert_array_equal(o.get(), want)
+
+
+@pytest.mark.parametrize("cfg", [11, 22, 24, 25, 31, 33, 36, 37, 38, 39])
+@pytest.mark.parametrize("O, H", [(57, 6), (30, 7), (131, 8)])
+def test_conv_rows_and_planes_of_any_channel_count(cfg, O, H):
+    from mxnet_amd import capi
+    N, C = 3, 16
+    d, w, b = (int8_uniform((N, C, H, H), seed=O), int8_uniform((O, C, 3, 3), seed=1),
+               int8_uniform((O,), seed=2))
+    acc, lo, hi = oracle.quantized_conv(d, w, b, -RD, RD, -RW, RW, -RB, RB, (1, 1), (1, 1))
+    want8 = oracle.requantize(acc, lo, hi, *CALIB)[0]
+    s = scalars(-RD, RD, -RW, RW, -RB, RB)
+    got = capi.quantized_conv_nhwc(dev(d.transpose(0, 2, 3, 1)), dev(w.transpose(0, 2, 3, 1)),
+                                   dev(b), *s, pad=(1, 1), want_int32=False, calib=CALIB,
+                                   relu=False, force=(cfg, 1))
+    np.testing.assert_array_equal(got["out8"].cpu().numpy().transpose(0, 3, 1, 2), want8)
+    planes = capi.quantized_conv_nchw(dev(d), dev(w), dev(b), *s, pad=(1, 1))
+    np.testing.assert_array_equal(planes["out32"].cpu().numpy(), acc)
