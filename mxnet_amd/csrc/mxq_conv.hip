@@ -998,31 +998,75 @@ void launch_cfg(hipStream_t s, const ConvArgs& a, bool aligned) {
 }
 
 // ---- layout adapters ------------------------------------------------------------
-// A second, small transpose that rides along in the launch of a large one: the weights of
-// a convolution ([O][C][taps] -> [O][taps][C]) next to its data.  A launch of its own costs
-// 4.6-5.9 us inside a network however little it moves (launch, then a cold round trip to
-// memory), which for four 3 x 3 layers was 20 us of a 520 us pass.  [B][R][S] -> [B][S][R]
-// with 16 | R and S small: a thread gathers 16 bytes S apart and stores them as one piece.
-struct SmallJob {
+// A transpose [B][R][S] -> [B][S][RP] of bytes, 16 | RP, zeros in positions R ... RP - 1, that asks
+// nothing of R, S or the input's address: a lane gathers 16 bytes S apart and stores them as one
+// piece.  The lanes run along S, so that a load instruction of a wave reads whole lines, whatever S is
+// (along the pieces of a row, as it was, it read 64 lines for 64 bytes: the weights of 7 x 7 x 512
+// -> 512, 3 x 3).  Where a row has four pieces and more, the four waves of a work-group take four of
+// them, 64 bytes that leave through one L2.
+// Two of them fit a launch, or one rides along in another's: the weights of a convolution
+// ([O][C][taps] -> [O][taps][C]) next to its data.  A launch of its own costs 4.6-5.9 us inside a
+// network however little it moves (launch, then a cold round trip to memory).
+struct GatherJob {
   const uint8_t* in;
   uint8_t* out;
-  int R, S;
-  unsigned pieces;   // B * S * R / 16; 0 = no job
+  int R, S, RP;
+  unsigned tiles_s, tiles_k;  // of 64 columns and 4 pieces; 0: pieces one behind the other
+  unsigned pieces;            // B * S * RP / 16, or what covers it in tiles
+  unsigned blocks;            // work-groups' worth of pieces; 0: no job
 };
 
-__device__ __forceinline__ void small_transpose_job(const SmallJob& j, unsigned block,
-                                                    unsigned nblocks) {
+GatherJob no_job() { return GatherJob{nullptr, nullptr, 0, 1, 16, 0, 0, 0, 0}; }
+
+bool gather_job_ok(const void* out, long long B, long long S, long long RP) {
+  return RP % 16 == 0 && aligned16(out) && B * S * RP > 0 &&
+         B * (S + 64) * (RP / 16 + 4) < (1LL << 31);
+}
+GatherJob gather_job(const void* in, void* out, int B, int R, int S, int RP) {
+  GatherJob j = {static_cast<const uint8_t*>(in), static_cast<uint8_t*>(out), R, S, RP, 0, 0, 0, 0};
+  const unsigned per_row = static_cast<unsigned>(RP) >> 4;
+  if (S >= 64 && per_row >= 4) {
+    j.tiles_s = (static_cast<unsigned>(S) + 63u) / 64u;
+    j.tiles_k = (per_row + 3u) / 4u;
+    j.blocks = static_cast<unsigned>(B) * j.tiles_s * j.tiles_k;
+    j.pieces = j.blocks * 256u;
+  } else {
+    j.pieces = static_cast<unsigned>(B) * static_cast<unsigned>(S) * per_row;
+    j.blocks = (j.pieces + 255u) / 256u;
+  }
+  return j;
+}
+
+__device__ __forceinline__ void gather_job_run(const GatherJob& j, unsigned block,
+                                               unsigned nblocks) {
   typedef uint32_t u4 __attribute__((ext_vector_type(4)));
-  const unsigned per_row = static_cast<unsigned>(j.R) >> 4;     // pieces per output row [b][s]
-  for (unsigned t = block * 256u + threadIdx.x; t < j.pieces; t += nblocks * 256u) {
-    const unsigned row = t / per_row, k = t - row * per_row;    // row = b * S + s
-    const unsigned b = row / static_cast<unsigned>(j.S), s = row - b * j.S;
-    const uint8_t* src = j.in + (static_cast<size_t>(b) * j.R + 16 * k) * j.S + s;
+  const unsigned per_row = static_cast<unsigned>(j.RP) >> 4, S = static_cast<unsigned>(j.S);
+  for (unsigned item = block; item < j.blocks; item += nblocks) {
+    unsigned b, k, s;
+    if (j.tiles_s != 0) {
+      const unsigned rest = item / j.tiles_s;
+      b = rest / j.tiles_k;
+      s = (item - rest * j.tiles_s) * 64u + (threadIdx.x & 63u);
+      k = (rest - b * j.tiles_k) * 4u + (threadIdx.x >> 6);
+      if (s >= S || k >= per_row) continue;
+    } else {
+      const unsigned t = item * 256u + threadIdx.x;
+      if (t >= j.pieces) continue;
+      const unsigned rest = t / S;
+      s = t - rest * S;
+      b = rest / per_row;
+      k = rest - b * per_row;
+    }
+    const int rows = j.R - static_cast<int>(16 * k);  // of the input under this piece
+    const int last = rows > 0 ? (rows < 16 ? rows - 1 : 15) : 0;
+    const uint8_t* src = j.in + (static_cast<size_t>(b) * j.R + (rows > 0 ? 16 * k : 0)) * S + s;
     uint32_t w[4] = {0, 0, 0, 0};
 #pragma unroll
-    for (int i = 0; i < 16; ++i)
-      w[i >> 2] |= static_cast<uint32_t>(src[static_cast<size_t>(i) * j.S]) << (8 * (i & 3));
-    *reinterpret_cast<u4*>(j.out + static_cast<size_t>(row) * j.R + 16 * k) =
+    for (int i = 0; i < 16; ++i) {
+      const uint32_t x = src[static_cast<size_t>(i < last ? i : last) * S];
+      w[i >> 2] |= (i < rows ? x : 0u) << (8 * (i & 3));
+    }
+    *reinterpret_cast<u4*>(j.out + (static_cast<size_t>(b) * S + s) * j.RP + 16 * k) =
         u4{w[0], w[1], w[2], w[3]};
   }
 }
@@ -1058,12 +1102,12 @@ __global__ __launch_bounds__(256) void transpose_kernel(const T* __restrict__ in
 // (a wave writes 1 KiB contiguous when the group covers all RP positions of its rows).
 __global__ __launch_bounds__(256) void transpose_i8_kernel(const uint8_t* __restrict__ in,
                                                            uint8_t* __restrict__ out, int R,
-                                                           int S, int RP, int B, SmallJob job) {
+                                                           int S, int RP, int B, GatherJob job) {
   constexpr int kPitch = 17;  // dwords per transposed row: 64 bytes + 4 of padding
   __shared__ uint32_t tile[128 * kPitch];
   if (static_cast<int>(blockIdx.z) >= B) {   // the extra z slices carry the riding job
     const unsigned per_z = gridDim.x * gridDim.y;
-    small_transpose_job(job, (blockIdx.z - B) * per_z + blockIdx.y * gridDim.x + blockIdx.x,
+    gather_job_run(job, (blockIdx.z - B) * per_z + blockIdx.y * gridDim.x + blockIdx.x,
                         (gridDim.z - B) * per_z);
     return;
   }
@@ -1123,12 +1167,12 @@ template <int PIECE>
 __global__ __launch_bounds__(256) void transpose_i8_wide_kernel(const uint8_t* __restrict__ in,
                                                                 uint8_t* __restrict__ out,
                                                                 int R, int S, int RP,
-                                                                WideOrder o, SmallJob job) {
+                                                                WideOrder o, GatherJob job) {
   typedef uint32_t u4 __attribute__((ext_vector_type(4)));
   constexpr int kPitch = 33;  // dwords per transposed row: 128 bytes + 4 of padding
   __shared__ uint32_t tile[128 * kPitch];
   if (blockIdx.x >= o.grid) {   // blocks past the tile grid carry the riding job
-    small_transpose_job(job, blockIdx.x - o.grid, gridDim.x - o.grid);
+    gather_job_run(job, blockIdx.x - o.grid, gridDim.x - o.grid);
     return;
   }
   // the tile sequence runs along S first, then R, then the batch; with o.per_xcd != 0 the
@@ -1199,15 +1243,12 @@ __global__ __launch_bounds__(256) void copy16_kernel(const uint8_t* __restrict__
     reinterpret_cast<u4*>(out)[q] = reinterpret_cast<const u4*>(in)[q];
 }
 
-// Small tensors with a thin inner extent on their own (7 x 7 planes of up to 4 MiB, or a
-// weight tensor whose data took a kernel that carries no rider): the job body as a kernel,
-// up to two jobs per launch.
-__global__ __launch_bounds__(256) void small_transpose_kernel(SmallJob first, SmallJob second,
-                                                              unsigned first_blocks) {
-  if (blockIdx.x < first_blocks)
-    small_transpose_job(first, blockIdx.x, first_blocks);
+// Whatever the kernels above do not take, up to two jobs per launch.
+__global__ __launch_bounds__(256) void gather_transpose_kernel(GatherJob first, GatherJob second) {
+  if (blockIdx.x < first.blocks)
+    gather_job_run(first, blockIdx.x, first.blocks);
   else
-    small_transpose_job(second, blockIdx.x - first_blocks, gridDim.x - first_blocks);
+    gather_job_run(second, blockIdx.x - first.blocks, gridDim.x - first.blocks);
 }
 
 // A thin extent (at most 64 bytes, e.g. 7 x 7 planes) beside a long one that is a multiple of
@@ -1256,15 +1297,11 @@ __global__ __launch_bounds__(256) void s2d_nhwc_kernel(const int8_t* __restrict_
 // 14.3 -> 12.1 us).  Rows on the marks lose 10 % that way (64 x 64 planes: 25.6 -> 28.9 us) and
 // the way back to planes gains nothing reliably, so those keep the plain order.
 // work-groups a riding job gets: enough to be done when the carrier is
-inline unsigned job_blocks(const SmallJob& job) {
-  if (job.pieces == 0) return 0;
-  const unsigned want = (job.pieces + 255u) / 256u;
-  return want < 1024u ? want : 1024u;
-}
+inline unsigned job_blocks(const GatherJob& job) { return job.blocks < 1024u ? job.blocks : 1024u; }
 
 template <int PIECE>
 void launch_wide(hipStream_t s, const void* in, void* out, int B, int R, int S, int RP,
-                 const SmallJob& job) {
+                 const GatherJob& job) {
   WideOrder o;
   o.tiles_s = static_cast<unsigned>((S + 127) / 128);
   o.tiles_r = static_cast<unsigned>((RP + 127) / 128);
@@ -1279,18 +1316,25 @@ void launch_wide(hipStream_t s, const void* in, void* out, int B, int R, int S, 
   MXQ_LAUNCH_CHECK();
 }
 
-// [B][R][S] -> [B][S][RP].  `rider`, when given, is a small job the launch carries along if
-// its kernel can (then rider->pieces is cleared); the caller launches what is left.
+// [B][R][S] -> [B][S][RP].  `rider`, when given, is a job the launch carries along if
+// its kernel can (then rider->blocks is cleared); the caller launches what is left.
 template <typename T>
 void launch_transpose(hipStream_t s, const void* in, void* out, int B, int R, int S, int RP,
-                      SmallJob* rider = nullptr) {
+                      GatherJob* rider = nullptr) {
   if (B == 0 || RP == 0 || S == 0) return;
   MXQ_CHECK(RP >= R, "padded extent below the extent");
-  SmallJob none = {nullptr, nullptr, 16, 1, 0};
-  SmallJob job = rider != nullptr ? *rider : none;
+  const GatherJob job = rider != nullptr ? *rider : no_job();
   auto carried = [&]() {
-    if (rider != nullptr) rider->pieces = 0;
+    if (rider != nullptr) rider->blocks = 0;
   };
+  auto gather = [&]() {
+    const GatherJob me = gather_job(in, out, B, R, S, RP);
+    hipLaunchKernelGGL(gather_transpose_kernel, dim3(me.blocks + job_blocks(job)), dim3(256), 0, s,
+                       me, job);
+    MXQ_LAUNCH_CHECK();
+    carried();
+  };
+  const bool gathers = sizeof(T) == 1 && R > 0 && gather_job_ok(out, B, S, RP);
   // only the kernels that put batches and row tiles on grid.y / grid.z have their limit
   auto check_yz = [&]() {
     MXQ_CHECK(B < 65535 && (RP + 63) / 64 <= 65535, "transpose grid too large");
@@ -1322,16 +1366,9 @@ void launch_transpose(hipStream_t s, const void* in, void* out, int B, int R, in
     carried();
     return;
   }
-  if (sizeof(T) == 1 && RP == R && R % 16 == 0 && S > 1 && S <= 64 && aligned16(out) &&
-      static_cast<long long>(B) * R * S <= (4LL << 20)) {
+  if (gathers && S > 1 && S <= 64 && static_cast<long long>(B) * RP * S <= (4LL << 20)) {
     // a small tensor with a thin inner extent (3 x 3 weights, 7 x 7 planes)
-    SmallJob me = {static_cast<const uint8_t*>(in), static_cast<uint8_t*>(out), R, S,
-                   static_cast<unsigned>(static_cast<long long>(B) * S * (R / 16))};
-    const unsigned mine = (me.pieces + 255u) / 256u;
-    hipLaunchKernelGGL(small_transpose_kernel, dim3(mine + job_blocks(job)), dim3(256), 0, s, me,
-                       job, mine);
-    MXQ_LAUNCH_CHECK();
-    carried();
+    gather();
     return;
   }
   if (sizeof(T) == 1 && RP == R && aligned16(in) && aligned16(out)) {
@@ -1362,6 +1399,10 @@ void launch_transpose(hipStream_t s, const void* in, void* out, int B, int R, in
       MXQ_LAUNCH_CHECK();
       return;
     }
+  }
+  if (gathers) {
+    gather();
+    return;
   }
   check_yz();
   dim3 grid((S + 63) / 64, (RP + 63) / 64, B);
@@ -1812,16 +1853,14 @@ void nchw_to_nhwc_pair(hipStream_t s, const int8_t* data, int8_t* d_out, int N, 
                        int W, int Cp, const int8_t* weight, int8_t* w_out, int O, int KH, int KW) {
   MXQ_CHECK(static_cast<long long>(H) * W < (1LL << 31), "image too large");
   const int taps = KH * KW;
-  const long long wpieces = static_cast<long long>(O) * taps * (C / 16);
-  SmallJob job = {reinterpret_cast<const uint8_t*>(weight), reinterpret_cast<uint8_t*>(w_out), C,
-                  taps, 0};
-  const bool rides = w_out != nullptr && Cp == C && C % 16 == 0 && taps > 1 && taps <= 64 &&
-                     aligned16(w_out) && wpieces < (1LL << 31);
-  if (rides) job.pieces = static_cast<unsigned>(wpieces);
+  GatherJob job = no_job();
+  if (w_out != nullptr && gather_job_ok(w_out, O, taps, Cp))
+    job = gather_job(weight, w_out, O, C, taps, Cp);
+  const bool rides = job.blocks != 0;
   if (static_cast<long long>(N) * Cp * H * W != 0)
     launch_transpose<int8_t>(s, data, d_out, N, C, H * W, Cp, &job);
   if (w_out == nullptr) return;
-  if (rides && job.pieces == 0) return;   // carried
+  if (rides && job.blocks == 0) return;   // carried
   launch_transpose<int8_t>(s, weight, w_out, O, C, taps, Cp);
 }
 
