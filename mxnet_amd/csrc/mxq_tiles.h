@@ -79,6 +79,15 @@ inline Tile choose_tile(long M, long N, long K, long cus, bool gather = false,
     if (sp > 4) sp = 4;
     if (sp >= 2) *splits = static_cast<int>(sp);
   };
+  // Gathered operands (a convolution) of at most 64 columns: an address is made per 16 bytes of
+  // pixels and stage, so 128-byte stages and tiles of 128 pixels pay from a reduction of 512 on
+  // (140544 x 1584 -> 57 56.6 -> 38.4 us, 50176 x 2304 -> 32 24.9 -> 21.8, 50176 x 576 -> 48 14.6 ->
+  // 13.6), with less than a tile per CU the tiles of 64 (25088 x 1152 -> 64 14.4 -> 13.6, 12544 x
+  // 2304 -> 48 17.1 -> 15.8; 25088 x 576 -> 64 is level and stays).
+  if (gather && N <= 64 && K >= 512 && K < 4096) {
+    if (tiles(128, 64) >= cus) return Tile::kR128K2;
+    if (K >= 1024) return Tile::kS64K2;
+  }
   if (N <= 64) {
     if (K >= 4096) few_tile_splits();
     return (K >= 4096) ? Tile::kS64x4 : Tile::kS64x2;
@@ -90,8 +99,11 @@ inline Tile choose_tile(long M, long N, long K, long cus, bool gather = false,
   // 392 tiles of 64 x 128 against 17.6 us on 784 tiles of 64 x 64.  From K = 4096 on the
   // 64 x 64 tile with 256-byte stages is the better of the two unless the half-size tiles
   // still come two to a CU (512 x 4096 -> 4096: 18.3 us against 19.8 us on 256 tiles).
+  // Gathered operands whose 64 x 64 tiles are more than two per CU take them at any length: what
+  // does not fit at once waits for the 256-byte stages' LDS (12544 x 4608 -> 200 39.4 -> 32.0 us, 3600 x
+  // 8624 -> 528 62.9 -> 49.1; 2880 x 8624 -> 528, 405 tiles of 64 x 64, 39.1 and 49.0).
   const long tq = tiles(64, 128), tr = tiles(128, 64);
-  const long need = (K >= 4096) ? 2 * cus : cus;
+  const long need = (K >= 4096 && !(gather && tiles(64, 64) > 2 * cus)) ? 2 * cus : cus;
   if (tq >= need || tr >= need) {
     const bool q_fits = tq >= need && N % 128 == 0, r_fits = tr >= need;
     if (q_fits && (gather || !r_fits)) return Tile::kQ128K2;
