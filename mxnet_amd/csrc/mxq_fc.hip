@@ -145,10 +145,13 @@ FcPlan plan_fc(int M, int N, int K, bool aligned, bool fused8, const GemmForce& 
 // Rows that are no multiple of 16 bytes: the few-tiles kernel reads them as they are, but a
 // shape of many tiles is better copied into padded rows and given to the tiled kernels, where the
 // caller brought room for the copies (K = 1237: 1024 x 1024 13.5 us against 11.2 with the copies,
-// 256 x 2048 9.2 against 10.6).
+// 256 x 2048 9.2 against 10.6).  Below 64 bytes a row there is little to read and the copies cost as much,
+// so twice as many tiles are asked for (28717 x 18 -> 352, 9878 tiles, 38.9 us against 16.8; 136367 x 13
+// -> 8, 4262 tiles, 19.7 against 15.5; 9245 x 58 -> 239, 2312 tiles, 16.7 against 12.6; 1813 x 19 -> 544,
+// 969 tiles, 10.9 against 11.3).
 int fc_padded_k(int M, int N, int K) {
   const int Kp = (K + 15) / 16 * 16;
-  const bool wanted = Kp != K && K >= 64 && few_tiles_count(M, N) > 3L * num_cus() &&
+  const bool wanted = Kp != K && few_tiles_count(M, N) > (K >= 64 ? 3L : 6L) * num_cus() &&
                       static_cast<long long>(M) * Kp < (1LL << 31) &&
                       static_cast<long long>(N) * Kp < (1LL << 31);
   return wanted ? Kp : 0;

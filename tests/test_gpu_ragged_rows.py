@@ -112,3 +112,36 @@ def test_conv_rows_and_planes_of_any_channel_count(cfg, O, H):
     np.testing.assert_array_equal(got["out8"].cpu().numpy().transpose(0, 3, 1, 2), want8)
     planes = capi.quantized_conv_nchw(dev(d), dev(w), dev(b), *s, pad=(1, 1))
     np.testing.assert_array_equal(planes["out32"].cpu().numpy(), acc)
+
+
+# reductions below 64 bytes on either side of the tiles from which the rows are padded first
+@pytest.mark.parametrize("M, K, N", [(1569, 13, 1024), (1537, 13, 1024), (1536, 13, 1024),
+                                     (3000, 1, 600), (2048, 63, 1001), (50000, 11, 14)])
+def test_fc_short_rows_of_many_tiles(M, K, N):
+    from mxnet_amd import capi
+    d, w, b = (int8_uniform((M, K), seed=N), int8_uniform((N, K), seed=N + 1),
+               int8_uniform((N,), seed=2))
+    acc, lo, hi = oracle.quantized_fully_connected(d, w, b, -RD, RD, -RW, RW, -RB, RB)
+    want8 = oracle.requantize(acc, lo, hi, *CALIB)[0]
+    got = capi.quantized_fc(dev(d), dev(w), dev(b), *scalars(-RD, RD, -RW, RW, -RB, RB),
+                            want_int32=True, calib=CALIB)
+    np.testing.assert_array_equal(got["out32"].cpu().numpy(), acc)
+    np.testing.assert_array_equal(got["out8"].cpu().numpy(), want8)
+
+
+# convolutions on either side of the lines between the tiles of 64 and 128 pixels
+@pytest.mark.parametrize("M_side, C, O, k, N", [
+    (16, 64, 57, 3, 127), (16, 64, 57, 3, 129), (16, 128, 30, 3, 130), (16, 128, 30, 3, 16),
+    (12, 176, 132, 5, 40)])
+def test_conv_of_few_channels_out(M_side, C, O, k, N):
+    from mxnet_amd import capi
+    d, w, b = (int8_uniform((N, C, M_side, M_side), seed=O), int8_uniform((O, C, k, k), seed=1),
+               int8_uniform((O,), seed=2))
+    r = (-RD, RD, -RW, RW, -RB, RB)
+    x, y, z = (dev(a) for a in (d.transpose(0, 2, 3, 1), w.transpose(0, 2, 3, 1), b))
+    got = capi.quantized_conv_nhwc(x, y, z, *scalars(*r), pad=(k // 2, k // 2), want_int32=True)
+    want = capi.quantized_conv_nhwc(x, y, z, *scalars(*r), pad=(k // 2, k // 2), want_int32=True,
+                                    force=(25, 1))
+    assert torch.equal(got["out32"], want["out32"])
+    few = oracle.quantized_conv(d[:1], w, b, *r, (1, 1), (k // 2, k // 2))[0]
+    np.testing.assert_array_equal(got["out32"][:1].cpu().numpy().transpose(0, 3, 1, 2), few)
