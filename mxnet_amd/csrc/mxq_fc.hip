@@ -94,6 +94,7 @@ FcPlan plan_fc(int M, int N, int K, bool aligned, bool fused8, const GemmForce& 
         case Tile::kQ128K2: plan.cfg = 58; break;
         case Tile::kS64K4: plan.cfg = 59; break;
         case Tile::kW192K2: plan.cfg = 60; break;
+        case Tile::kW64x2: plan.cfg = 42; break;  // not proposed for plain operands
       }
     } else {
       if (tiles(256, 256) >= cus)

@@ -35,7 +35,8 @@ enum class Tile {
   kS64K4,   // 64 x 64, 256-byte stages, 2-stage ring
   kR128K2,  // 128 x 64, 128-byte stages, 2-stage ring
   kQ128K2,  // 64 x 128, 128-byte stages, 2-stage ring
-  kW192K2   // 256 x 192, 128-byte stages, 2-stage ring
+  kW192K2,  // 256 x 192, 128-byte stages, 2-stage ring
+  kW64x2    // 256 x 64, 64-byte stages, 2-stage ring
 };
 
 // M x N outputs, reduction length K, `cus` compute units.  Distilled from sweeps over
@@ -82,12 +83,20 @@ inline Tile choose_tile(long M, long N, long K, long cus, bool gather = false,
   // Gathered operands (a convolution) of at most 64 columns: an address is made per 16 bytes of
   // pixels and stage, so 128-byte stages and tiles of 128 pixels pay from a reduction of 512 on
   // (140544 x 1584 -> 57 56.6 -> 38.4 us, 50176 x 2304 -> 32 24.9 -> 21.8, 50176 x 576 -> 48 14.6 ->
-  // 13.6), with less than a tile per CU the tiles of 64 (25088 x 1152 -> 64 14.4 -> 13.6, 12544 x
-  // 2304 -> 48 17.1 -> 15.8; 25088 x 576 -> 64 is level and stays).
-  if (gather && N <= 64 && K >= 512 && K < 4096) {
+  // 13.6, 57600 x 10400 -> 64 123.5 -> 70.5), with less than a tile per CU the tiles of 64 (25088 x 1152
+  // -> 64 14.4 -> 13.6, 12544 x 2304 -> 48 17.1 -> 15.8; 25088 x 576 -> 64 is level and stays), on
+  // 256-byte stages where they are many (27648 x 20384 -> 64 108.9 -> 72.7, 4732 x 5200 -> 36 28.5 ->
+  // 22.9).  Short ones take 256 pixels once there are two such tiles per CU and more (529803 x 144 -> 41
+  // 40.2 -> 31.2, 192000 x 432 -> 48 24.0 -> 18.7; 131072 x 432 -> 46, two exactly, is level).
+  if (gather && N <= 64 && K >= 512) {
     if (tiles(128, 64) >= cus) return Tile::kR128K2;
+    if (K >= 4096) {
+      few_tile_splits();
+      return Tile::kS64K4;
+    }
     if (K >= 1024) return Tile::kS64K2;
   }
+  if (gather && N <= 64 && K < 512 && tiles(256, 64) > 2 * cus) return Tile::kW64x2;
   if (N <= 64) {
     if (K >= 4096) few_tile_splits();
     return (K >= 4096) ? Tile::kS64x4 : Tile::kS64x2;

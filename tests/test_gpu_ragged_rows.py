@@ -132,7 +132,8 @@ def test_fc_short_rows_of_many_tiles(M, K, N):
 # convolutions on either side of the lines between the tiles of 64 and 128 pixels
 @pytest.mark.parametrize("M_side, C, O, k, N", [
     (16, 64, 57, 3, 127), (16, 64, 57, 3, 129), (16, 128, 30, 3, 130), (16, 128, 30, 3, 16),
-    (12, 176, 132, 5, 40)])
+    (12, 176, 132, 5, 40), (16, 512, 20, 3, 20), (32, 512, 33, 3, 33), (7, 208, 9, 9, 3),
+    (64, 16, 41, 3, 33), (64, 16, 24, 3, 32)])
 def test_conv_of_few_channels_out(M_side, C, O, k, N):
     from mxnet_amd import capi
     d, w, b = (int8_uniform((N, C, M_side, M_side), seed=O), int8_uniform((O, C, k, k), seed=1),
