@@ -1209,7 +1209,7 @@ __device__ __forceinline__ void gemm_epilogue_lds(v16i (&acc)[Cfg::MI][Cfg::NI],
           }
     }
   };
-  // (the question once, not at every store: 4096 x 3072 int32 rows lose 3 % to it there)
+  // (asked once, not at every store: 31117 x 144 -> 400 in int32 21.4 us there, 20.5 here)
   auto store_rows32 = [&](int* out, auto quad) {
     if ((N & 3) == 0)
       store_rows32_as(out, quad, std::false_type());
