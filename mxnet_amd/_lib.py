@@ -124,7 +124,8 @@ for _name, (_res, _args) in SIGNATURES.items():
 
 # test-only twins of the FC and convolution entry points (tests/mxq_test_hooks.h, not part
 # of include/mxq.h): the same arguments followed by the tile configuration, the split-K
-# factor and, for the FC, the streaming kernel's work-groups per CU (0 = choose)
+# factor and, for the FC, the streaming kernel's work-groups per CU (0 = choose); and what a block's
+# launch reads of LDS
 TEST_HOOKS = {
     "mxq_test_quantized_fc": (_i, SIGNATURES["mxq_quantized_fc"][1] + [_i, _i, _i]),
     "mxq_test_quantized_fc_sum": (_i, SIGNATURES["mxq_quantized_fc_sum"][1] + [_i, _i, _i]),
@@ -133,6 +134,7 @@ TEST_HOOKS = {
     "mxq_test_quantized_fc_f32": (_i, SIGNATURES["mxq_quantized_fc_f32"][1] + [_i, _i]),
     "mxq_test_quantized_conv_nhwc": (_i, SIGNATURES["mxq_quantized_conv_nhwc"][1] + [_i, _i]),
     "mxq_test_quantized_conv_nchw": (_i, SIGNATURES["mxq_quantized_conv_nchw"][1] + [_i]),
+    "mxq_test_block_lds": (_i, [_i] * 8 + [ctypes.POINTER(_i)] * 2),
 }
 for _name, (_res, _args) in TEST_HOOKS.items():
     _fn = getattr(lib, _name)

@@ -130,6 +130,31 @@ __host__ __device__ constexpr int odd(int chunks) { return chunks | 1; }
 // ... of rows that are written in whole column tiles of 32 channels
 __host__ __device__ constexpr int odd_tiles(int chunks) { return ((chunks + 1) & ~1) | 1; }
 
+// A lane's pieces of rows that leave the launch: `chunks` pieces a row, rows `pitch` pieces apart in LDS
+// from `at` on; the next one is `rows` rows and `rest` pieces further.
+struct Pieces {
+  int row, j, from;
+  __host__ __device__ void begin(int first_row, int first_j, int at, int pitch) {
+    row = first_row;
+    j = first_j;
+    from = at + (row * pitch + j) * 16;
+  }
+  __host__ __device__ void next(int rows, int rest, int chunks, int pitch) {
+    row += rows;
+    j += rest;
+    from += (rows * pitch + rest) * 16;
+    const bool carry = j >= chunks;
+    j -= carry ? chunks : 0;
+    row += carry;
+    from += carry ? (pitch - chunks) * 16 : 0;
+  }
+  // what is read of LDS: where the lanes are more than the pieces, no more than there is of it
+  __host__ __device__ int place(int tile_rows, int at) const { return row < tile_rows ? from : at; }
+};
+// From a row of the patch to the one below it, for the taps in row `row` of three.  The last of them
+// has none below; what is read ahead there is not used.
+__host__ __device__ inline int row_below(int row, int row_pitch) { return row < 2 ? row_pitch : 0; }
+
 // floor(n / d) for n * d < 2^30, magic = 2^31 / d + 1: (2n + 1) / 2d is never an integer, and no
 // case (d = 1) needs a branch, behind which the compiler would load the next argument
 __device__ __forceinline__ int quotient(int n, uint32_t magic) {
@@ -423,7 +448,7 @@ __device__ __forceinline__ void block_tile(const BlockArgs& p, int tile, int fir
       first_pixels(read);
       for (int row = 0; row < 3; ++row) {
 #pragma unroll
-        for (int rt = 0; rt < RT; ++rt) below[rt] = in_patch[rt] + row_pitch;
+        for (int rt = 0; rt < RT; ++rt) below[rt] = in_patch[rt] + row_below(row, row_pitch);
 #pragma unroll
         for (int g = 0; g < kRow / GB; ++g) {
           fetch_shortcut();
@@ -557,20 +582,16 @@ __device__ __forceinline__ void block_tile(const BlockArgs& p, int tile, int fir
                    const uint32_t* pixel_of, int8_t* out) MXQ_INLINE {
     const auto to = __builtin_amdgcn_make_buffer_rsrc(
         out, 0, static_cast<uint32_t>(p.N) * p.H * p.W * chunks * 16, 0x00020000);
-    int row = quotient(tid, magic), j = tid - row * chunks, from = at + (row * pitch + j) * 16;
+    Pieces piece;
+    const int first = quotient(tid, magic);
+    piece.begin(first, tid - first * chunks, at, pitch);
     for (int left = TM * chunks; left > 0; left -= 64 * NW) {
       // (rows past the tile's are written nowhere)
-      const uint32_t pixel = row < TM ? pixel_of[row] : kOutOfRange;
+      const uint32_t pixel = piece.row < TM ? pixel_of[piece.row] : kOutOfRange;
       __builtin_amdgcn_raw_buffer_store_b128(
-          __builtin_bit_cast(v4u, *reinterpret_cast<const v4i*>(smem + from)), to, pixel + 16 * j, 0,
-          0);
-      row += rows;
-      j += rest;
-      from += (rows * pitch + rest) * 16;
-      const bool carry = j >= chunks;
-      j -= carry ? chunks : 0;
-      row += carry;
-      from += carry ? (pitch - chunks) * 16 : 0;
+          __builtin_bit_cast(v4u, *reinterpret_cast<const v4i*>(smem + piece.place(TM, at))), to,
+          pixel + 16 * piece.j, 0, 0);
+      piece.next(rows, rest, chunks, pitch);
     }
   };
   leave(0, CO, PO, p.magic_wide, p.wide_rows, p.wide_rest, wide_of, p.out);
@@ -1025,5 +1046,49 @@ int mxq_quantized_block(void* stream, const int8_t* data, const int8_t* weights,
   }
   MXQ_API_END();
 }
+
+#ifdef MXQ_TEST_HOOKS
+// The bytes of LDS that a tile of `tile` pixels has, and how far the reads of the outputs' pieces, of
+// the 1 x 1 layers' operands and of the constant taps reach.
+int mxq_test_block_lds(int N, int H, int W, int C, int C_mid, int C_out, int C_next, int tile,
+                       int* lds, int* reach) {
+  MXQ_API_BEGIN();
+  MXQ_CHECK((tile == 32 || tile == 64) && lds != nullptr && reach != nullptr, "bad arguments");
+  *lds = *reach = 0;
+  const BlockPlan b = plan_tiles(N, H, W, C, C_mid, C_out, C_next, tile);
+  if (b.tiles == 0) return 0;
+  *lds = b.lds;
+  const int lanes = b.variant == 64 ? 256 : 512;
+  auto read = [&](int place) { *reach = place + 16 > *reach ? place + 16 : *reach; };
+  auto leave = [&](int at, int chunks) {
+    const int pitch = odd_tiles(chunks);
+    for (int tid = 0; tid < lanes && chunks != 0; ++tid) {
+      Pieces piece;
+      piece.begin(tid / chunks, tid % chunks, at, pitch);
+      for (int left = tile * chunks; left > 0; left -= lanes) {
+        read(piece.place(tile, at));
+        piece.next(lanes / chunks, lanes % chunks, chunks, pitch);
+      }
+    }
+  };
+  leave(0, C_out / 16);
+  leave(b.off_patch, C_next / 16);
+  // the last row of each operand, whole steps and what is read ahead of them
+  const int ahead = b.variant == 256 && tile == 64 ? 3 : 1;
+  read(b.off_patch + (tile - 1) * odd_tiles(C_mid / 16) * 16 + 16 + 32 * (b.steps[1] - 1));
+  if (C_next != 0)
+    read((tile - 1) * odd_tiles(C_out / 16) * 16 + 16 + 32 * (b.steps[2] - 1 + ahead));
+  if (C == b.variant) {  // constant taps: from the last of the tile's pixels that has a place
+    const int pixel = odd(C / 16) * 16;
+    int at = b.off_patch + (b.rows - 3) * b.row_pitch + (b.tw - 1) * pixel + 16;
+    for (int row = 0; row < 3; ++row) {
+      read(at + 2 * pixel + C - 32);
+      read(at + row_below(row, b.row_pitch) + 32 * (ahead - 1));
+      at += b.row_pitch;
+    }
+  }
+  MXQ_API_END();
+}
+#endif  // MXQ_TEST_HOOKS
 
 }  // extern "C"

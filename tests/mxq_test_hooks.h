@@ -88,6 +88,12 @@ int mxq_test_quantized_conv_nchw(void* stream, const int8_t* data, const int8_t*
                                  const float* max_bias, int32_t* out32, float* omin, float* omax,
                                  void* workspace, size_t workspace_bytes, int cfg);
 
+/* How a block's launch on tiles of 32 or 64 pixels (mxq_quantized_block) uses LDS: the bytes that a
+ * work-group has and the end of the furthest read of the outputs' pieces, of the 1 x 1 layers' operands and
+ * of constant taps, both 0 where there is no such launch. */
+int mxq_test_block_lds(int N, int H, int W, int C, int C_mid, int C_out, int C_next, int tile,
+                       int* lds, int* reach);
+
 #ifdef __cplusplus
 }
 #endif
