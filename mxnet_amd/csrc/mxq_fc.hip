@@ -153,6 +153,8 @@ FcPlan plan_fc(int M, int N, int K, bool aligned, bool fused8, const GemmForce& 
 int fc_padded_k(int M, int N, int K) {
   const int Kp = (K + 15) / 16 * 16;
   const bool wanted = Kp != K && few_tiles_count(M, N) > (K >= 64 ? 3L : 6L) * num_cus() &&
+                      // (the copies read 16 bytes at once)
+                      static_cast<long long>(M) * K >= 16 && static_cast<long long>(N) * K >= 16 &&
                       static_cast<long long>(M) * Kp < (1LL << 31) &&
                       static_cast<long long>(N) * Kp < (1LL << 31);
   return wanted ? Kp : 0;

@@ -146,3 +146,32 @@ def test_conv_of_few_channels_out(M_side, C, O, k, N):
     assert torch.equal(got["out32"], want["out32"])
     few = oracle.quantized_conv(d[:1], w, b, *r, (1, 1), (k // 2, k // 2))[0]
     np.testing.assert_array_equal(got["out32"][:1].cpu().numpy().transpose(0, 3, 1, 2), few)
+
+
+# more than six tiles a CU over weights, or data, of fewer than the 16 bytes that a padding copy reads at
+# once, and of 16 exactly
+@pytest.mark.parametrize("M, K, N", [(50000, 3, 4), (50000, 1, 8), (50000, 13, 1), (50000, 15, 1),
+                                     (50000, 2, 8), (50000, 3, 6), (1, 3, 60000), (5, 3, 60000),
+                                     (6, 3, 60000)])
+def test_fc_operands_of_a_few_bytes(M, K, N):
+    from mxnet_amd import capi
+    d, w, b = (int8_uniform((M, K), seed=N), int8_uniform((N, K), seed=N + 1),
+               int8_uniform((N,), seed=2))
+    acc, lo, hi = oracle.quantized_fully_connected(d, w, b, -RD, RD, -RW, RW, -RB, RB)
+    want8 = oracle.requantize(acc, lo, hi, *CALIB)[0]
+    got = capi.quantized_fc(dev(d), dev(w), dev(b), *scalars(-RD, RD, -RW, RW, -RB, RB),
+                            want_int32=True, calib=CALIB)
+    np.testing.assert_array_equal(got["out32"].cpu().numpy(), acc)
+    np.testing.assert_array_equal(got["out8"].cpu().numpy(), want8)
+
+
+@pytest.mark.parametrize("O", [3, 4, 5, 6])
+def test_conv_1x1_of_an_image_to_a_few_channels(O):
+    from mxnet_amd import capi
+    d, w, b = (int8_uniform((1, 3, 224, 224), seed=O), int8_uniform((O, 3, 1, 1), seed=1),
+               int8_uniform((O,), seed=2))
+    r = (-RD, RD, -RW, RW, -RB, RB)
+    want = oracle.quantized_conv(d, w, b, *r, (1, 1), (0, 0))[0]
+    got = capi.quantized_conv_nhwc(dev(d.transpose(0, 2, 3, 1)), dev(w.transpose(0, 2, 3, 1)),
+                                   dev(b), *scalars(*r), want_int32=True)
+    np.testing.assert_array_equal(got["out32"].cpu().numpy().transpose(0, 3, 1, 2), want)
