@@ -1357,13 +1357,13 @@ void launch_transpose(hipStream_t s, const void* in, void* out, int B, int R, in
     check_yz();
     const unsigned per_z = static_cast<unsigned>((S + 127) / 128) * ((RP + 63) / 64);
     const unsigned extra_z = (job_blocks(job) + per_z - 1) / per_z;
-    MXQ_CHECK(B + extra_z <= 65535u, "transpose grid too large");
-    dim3 grid128((S + 127) / 128, (RP + 63) / 64, B + extra_z);
+    const bool fits = B + extra_z <= 65535u;  // the rider, else a launch of its own
+    dim3 grid128((S + 127) / 128, (RP + 63) / 64, fits ? B + extra_z : B);
     hipLaunchKernelGGL(transpose_i8_kernel, grid128, dim3(256), 0, s,
                        static_cast<const uint8_t*>(in), static_cast<uint8_t*>(out), R, S, RP, B,
                        job);
     MXQ_LAUNCH_CHECK();
-    carried();
+    if (fits) carried();
     return;
   }
   if (gathers && S > 1 && S <= 64 && static_cast<long long>(B) * RP * S <= (4LL << 20)) {

@@ -51,3 +51,16 @@ def test_data_and_weights_in_one_launch(N, C, H, O, k):
                                    *[dev(np.array([v], np.float32)) for v in r],
                                    pad=(k // 2, k // 2))
     np.testing.assert_array_equal(got["out32"].cpu().numpy(), want)
+
+
+# images that fill a launch's third extent leave no room in it for the weights
+@pytest.mark.parametrize("N", [65532, 65533, 65534])
+def test_weights_stay_behind_where_images_fill_the_grid(N):
+    from mxnet_amd import capi
+    d, w, b = (int8_uniform((N, 3, 2, 2), seed=1), int8_uniform((64, 3, 3, 3), seed=2),
+               int8_uniform((64,), seed=3))
+    r = (-2.0, 2.0, -0.1, 0.1, -1.0, 1.0)
+    want = oracle.quantized_conv(d, w, b, *r, (1, 1), (1, 1))[0]
+    got = capi.quantized_conv_nchw(dev(d), dev(w), dev(b),
+                                   *[dev(np.array([v], np.float32)) for v in r], pad=(1, 1))
+    np.testing.assert_array_equal(got["out32"].cpu().numpy(), want)
