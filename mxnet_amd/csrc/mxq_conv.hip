@@ -1014,25 +1014,41 @@ struct GatherJob {
   unsigned tiles_s, tiles_k;  // of 64 columns and 4 pieces; 0: pieces one behind the other
   unsigned pieces;            // B * S * RP / 16, or what covers it in tiles
   unsigned blocks;            // work-groups' worth of pieces; 0: no job
+  // of the two extents that a place is divided by: tiles_s and tiles_k, or S and the pieces of a row
+  unsigned magic_s, magic_k;
 };
 
-GatherJob no_job() { return GatherJob{nullptr, nullptr, 0, 1, 16, 0, 0, 0, 0}; }
+GatherJob no_job() { return GatherJob{nullptr, nullptr, 0, 1, 16, 0, 0, 0, 0, 0, 0}; }
+
+// floor(n / d) for n < 2^31, magic = 2^31 / d + 1: the product is at most one too large.  (A division
+// by a value that the compiler does not know is a dozen instructions.  A launch of a few work-groups
+// waits for its rider, 37 x 32 x 9 weights beside 5 images of 12 x 12: 3.12 us with the divisions and
+// all pieces clamped, 2.96 without the clamping, 2.80 without both.)
+unsigned gather_magic(unsigned d) { return static_cast<unsigned>((1ull << 31) / d + 1); }
+__device__ __forceinline__ unsigned gather_quotient(unsigned n, unsigned d, unsigned magic) {
+  const unsigned q = __umulhi(2u * n + 1u, magic);
+  return q - (q * d > n);
+}
 
 bool gather_job_ok(const void* out, long long B, long long S, long long RP) {
   return RP % 16 == 0 && aligned16(out) && B * S * RP > 0 &&
          B * (S + 64) * (RP / 16 + 4) < (1LL << 31);
 }
 GatherJob gather_job(const void* in, void* out, int B, int R, int S, int RP) {
-  GatherJob j = {static_cast<const uint8_t*>(in), static_cast<uint8_t*>(out), R, S, RP, 0, 0, 0, 0};
+  GatherJob j = {static_cast<const uint8_t*>(in), static_cast<uint8_t*>(out), R, S, RP, 0, 0, 0, 0, 0, 0};
   const unsigned per_row = static_cast<unsigned>(RP) >> 4;
   if (S >= 64 && per_row >= 4) {
     j.tiles_s = (static_cast<unsigned>(S) + 63u) / 64u;
     j.tiles_k = (per_row + 3u) / 4u;
     j.blocks = static_cast<unsigned>(B) * j.tiles_s * j.tiles_k;
     j.pieces = j.blocks * 256u;
+    j.magic_s = gather_magic(j.tiles_s);
+    j.magic_k = gather_magic(j.tiles_k);
   } else {
     j.pieces = static_cast<unsigned>(B) * static_cast<unsigned>(S) * per_row;
     j.blocks = (j.pieces + 255u) / 256u;
+    j.magic_s = gather_magic(static_cast<unsigned>(S));
+    j.magic_k = gather_magic(per_row);
   }
   return j;
 }
@@ -1044,27 +1060,34 @@ __device__ __forceinline__ void gather_job_run(const GatherJob& j, unsigned bloc
   for (unsigned item = block; item < j.blocks; item += nblocks) {
     unsigned b, k, s;
     if (j.tiles_s != 0) {
-      const unsigned rest = item / j.tiles_s;
-      b = rest / j.tiles_k;
+      const unsigned rest = gather_quotient(item, j.tiles_s, j.magic_s);
+      b = gather_quotient(rest, j.tiles_k, j.magic_k);
       s = (item - rest * j.tiles_s) * 64u + (threadIdx.x & 63u);
       k = (rest - b * j.tiles_k) * 4u + (threadIdx.x >> 6);
       if (s >= S || k >= per_row) continue;
     } else {
       const unsigned t = item * 256u + threadIdx.x;
       if (t >= j.pieces) continue;
-      const unsigned rest = t / S;
+      const unsigned rest = gather_quotient(t, S, j.magic_s);
       s = t - rest * S;
-      b = rest / per_row;
+      b = gather_quotient(rest, per_row, j.magic_k);
       k = rest - b * per_row;
     }
     const int rows = j.R - static_cast<int>(16 * k);  // of the input under this piece
-    const int last = rows > 0 ? (rows < 16 ? rows - 1 : 15) : 0;
     const uint8_t* src = j.in + (static_cast<size_t>(b) * j.R + (rows > 0 ? 16 * k : 0)) * S + s;
     uint32_t w[4] = {0, 0, 0, 0};
+    // whole pieces without the clamping (64 x 16 x 113 x 113 9.6 -> 7.2 us), where all lanes have them
+    if (__all(rows >= 16)) {
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const uint32_t x = src[static_cast<size_t>(i < last ? i : last) * S];
-      w[i >> 2] |= (i < rows ? x : 0u) << (8 * (i & 3));
+      for (int i = 0; i < 16; ++i)
+        w[i >> 2] |= static_cast<uint32_t>(src[static_cast<size_t>(i) * S]) << (8 * (i & 3));
+    } else {
+      const int last = rows > 0 ? rows - 1 : 0;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const uint32_t x = src[static_cast<size_t>(i < last ? i : last) * S];
+        w[i >> 2] |= (i < rows ? x : 0u) << (8 * (i & 3));
+      }
     }
     *reinterpret_cast<u4*>(j.out + (static_cast<size_t>(b) * S + s) * j.RP + 16 * k) =
         u4{w[0], w[1], w[2], w[3]};

@@ -40,7 +40,8 @@ def test_planes_to_padded_pixels(N, C, H, W, padded, offset):
 # 3 x 3, 5 x 5, 8 x 8 and 9 x 9 windows (64 and 81 taps), over planes of each kernel that carries them
 @pytest.mark.parametrize("N, C, H, O, k", [
     (2, 47, 16, 46, 3), (2, 7, 29, 35, 3), (1, 9, 21, 33, 5), (3, 130, 9, 20, 3), (2, 200, 20, 24, 3),
-    (1, 65, 12, 5, 8), (1, 20, 13, 6, 9), (2, 13, 11, 8, 1), (1, 1, 5, 1, 3)])
+    (1, 65, 12, 5, 8), (1, 20, 13, 6, 9), (2, 13, 11, 8, 1), (1, 1, 5, 1, 3),
+    (2, 32, 12, 37, 3), (1, 16, 16, 70, 5), (1, 48, 8, 3, 9)])  # whole pieces only
 def test_data_and_weights_in_one_launch(N, C, H, O, k):
     from mxnet_amd import capi
     d, w, b = (int8_uniform((N, C, H, H), seed=C), int8_uniform((O, C, k, k), seed=O),
