@@ -31,10 +31,14 @@ __global__ __launch_bounds__(kThreads) void zero_counts_kernel(uint32_t* counts,
 // that a work-group filled, hence few work-groups with many values each.  196608 values in 8001
 // bins 10 us; with the edges in memory and one value at a time 36, on the host 700.
 // LDS: bins are counted there.  VALUES: of a lane in flight; with one, edges stay in memory.
+// `holds`, where there is one, is 0 for edges that do not increase: between those a value would be
+// moved on bin by bin through all of them, and nothing is counted.
 template <bool LDS, int THREADS, int VALUES>
 __global__ __launch_bounds__(THREADS) void histogram_kernel(const float* __restrict__ in, size_t n,
                                                             const float* __restrict__ edges,
-                                                            int bins, uint32_t* counts) {
+                                                            int bins, uint32_t* counts,
+                                                            const uint32_t* holds) {
+  if (holds != nullptr && *holds == 0) return;
   constexpr bool HELD = VALUES > 1;  // the edges, in LDS
   extern __shared__ uint32_t local[];
   float* const edge_lds = reinterpret_cast<float*>(local + bins);
@@ -119,7 +123,7 @@ __global__ __launch_bounds__(1024) void symmetric_edges_kernel(const float* rang
 }
 
 void launch_histogram(hipStream_t s, const float* in, size_t n, const float* edges, int bins,
-                      uint32_t* counts) {
+                      uint32_t* counts, const uint32_t* holds) {
   if (n == 0) return;
   const bool lds = bins <= kMaxLdsBins;
   // Eight values a lane and the edges in LDS where there are values for them (us, one value / eight:
@@ -136,7 +140,7 @@ void launch_histogram(hipStream_t s, const float* in, size_t n, const float* edg
   const auto kernel = eight ? histogram_kernel<true, 1024, 8>
                             : lds ? histogram_kernel<true, 512, 1> : histogram_kernel<false, 512, 1>;
   hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(threads),
-                     words * sizeof(uint32_t), s, in, n, edges, bins, counts);
+                     words * sizeof(uint32_t), s, in, n, edges, bins, counts, holds);
   MXQ_LAUNCH_CHECK();
 }
 
@@ -158,7 +162,7 @@ int mxq_histogram_f32(void* stream, const float* in, size_t n, const float* edge
                      s, counts, bins);
   MXQ_LAUNCH_CHECK();
   if (n == 0) return 0;
-  launch_histogram(s, in, n, edges, bins, counts);
+  launch_histogram(s, in, n, edges, bins, counts, nullptr);
   MXQ_API_END();
 }
 
@@ -186,7 +190,7 @@ int mxq_symmetric_histogram_f32(void* stream, const float* in, size_t n, int bin
   hipLaunchKernelGGL(symmetric_edges_kernel, dim3(1), dim3(1024), 0, s, range, th, bins, edges,
                      out + 2, out + 3);
   MXQ_LAUNCH_CHECK();
-  launch_histogram(s, in, n, edges, bins, out + 3);
+  launch_histogram(s, in, n, edges, bins, out + 3, out + 2);
   MXQ_API_END();
 }
 

@@ -86,3 +86,16 @@ def test_symmetric_histogram_without_a_range(value):
     assert v._counts is None
     lo, hi = v.extremes()
     assert (np.isnan(lo) and np.isnan(hi)) if np.isnan(value) else (lo, hi) == (value, value)
+
+
+@pytest.mark.parametrize("bins", [101, 8001, 20001])
+@pytest.mark.parametrize("value, th", [(0.0, None), (1e-44, None), (0.5, np.float32(0)),
+                                       (0.5, np.float32(1e-44))])
+def test_nothing_is_counted_without_edges(bins, value, th):
+    """Edges that do not increase: looking for a bin between them would walk through all of them, so
+    no value is looked at."""
+    x = torch.full((70001,), value, device="cuda")
+    x[::2] *= -1
+    found = capi.symmetric_histogram(x, bins, th).cpu().numpy()
+    assert tuple(found[:2].view(np.float32)) == (-np.float32(value), np.float32(value))
+    assert found[2] == 0 and not found[3:].any()
