@@ -553,8 +553,9 @@ int mxq_quantized_block(void* stream, const int8_t* data, const int8_t* weights,
  * mxq_symmetric_histogram_f32: both in one go, without a word from the host between them.  `out`, on
  * the device, receives the two extreme values, 1 or 0, and the `bins` counts (of at most 2^24) over
  * [-th, th], its edges as numpy.histogram computes them in float32; th of NaN: the larger magnitude
- * of the two.  0 where those edges do not increase or th is not finite: the counts mean nothing
- * then.  The workspace is 16-byte aligned. */
+ * of the two.  0 where those edges do not increase or th is not finite: nothing is counted then.  The
+ * workspace is 16-byte aligned.
+ * mxq_symmetric_histogram_inside_f32: the same, but 0 as well where a value lies beyond th. */
 size_t mxq_minmax_f32_workspace(size_t n);
 int mxq_minmax_f32(void* stream, const float* in, size_t n, float* out_min, float* out_max,
                    void* workspace, size_t workspace_bytes);
@@ -563,6 +564,8 @@ int mxq_histogram_f32(void* stream, const float* in, size_t n, const float* edge
 size_t mxq_symmetric_histogram_f32_workspace(size_t n, int bins);
 int mxq_symmetric_histogram_f32(void* stream, const float* in, size_t n, int bins, float th,
                                 uint32_t* out, void* workspace, size_t workspace_bytes);
+int mxq_symmetric_histogram_inside_f32(void* stream, const float* in, size_t n, int bins, float th,
+                                       uint32_t* out, void* workspace, size_t workspace_bytes);
 
 /* Entropy calibration: bounds [lower, upper] of what mxq_calibrate_entropy's float sums give for
  * every candidate threshold, narrowest first, of up to 16 histograms (`hist`, on the device, one

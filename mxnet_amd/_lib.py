@@ -109,6 +109,7 @@ SIGNATURES = {
     "mxq_histogram_f32": (_i, [_p, _p, _sz, _p, _i, _p]),
     "mxq_symmetric_histogram_f32_workspace": (_sz, [_sz, _i]),
     "mxq_symmetric_histogram_f32": (_i, [_p, _p, _sz, _i, _f, _p, _p, _sz]),
+    "mxq_symmetric_histogram_inside_f32": (_i, [_p, _p, _sz, _i, _f, _p, _p, _sz]),
     "mxq_entropy_bounds_workspace": (_sz, [_i, ctypes.POINTER(_i), ctypes.POINTER(_i)]),
     "mxq_entropy_bounds": (_i, [_p, _i, _p, ctypes.POINTER(_i), ctypes.POINTER(_i), _p, _p, _sz]),
     "mxq_nchw_to_nhwc_i8": (_i, [_p, _p, _p, _i, _i, _i, _i]),

@@ -332,16 +332,16 @@ def histogram(data, edges):
     return counts
 
 
-def symmetric_histogram(data, bins, th=None):
+def symmetric_histogram(data, bins, th=None, inside=False):
     """(smallest value, largest value, whether the counts hold, int32 counts over [-th, th]) of a
     float32 tensor as one int32 device tensor, the values by their bits; without `th` over the larger
-    magnitude of the two."""
+    magnitude of the two.  With `inside` nothing is counted where a value lies beyond `th`."""
     assert data.dtype == torch.float32
     n = data.numel()
     out = torch.empty(3 + bins, dtype=torch.int32, device=data.device)
     wsb = lib.mxq_symmetric_histogram_f32_workspace(n, bins)
     ws = _workspace(wsb, data.device)
-    check(lib.mxq_symmetric_histogram_f32(_stream(), _ptr(data), n, bins,
-                                          float("nan") if th is None else float(th), _ptr(out),
-                                          _ptr(ws), wsb))
+    take = lib.mxq_symmetric_histogram_inside_f32 if inside else lib.mxq_symmetric_histogram_f32
+    check(take(_stream(), _ptr(data), n, bins, float("nan") if th is None else float(th),
+               _ptr(out), _ptr(ws), wsb))
     return out

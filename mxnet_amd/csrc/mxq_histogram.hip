@@ -97,19 +97,16 @@ __global__ __launch_bounds__(THREADS) void histogram_kernel(const float* __restr
 // The edges of `bins` equal bins over [-t, t], each as numpy computes it in float32 (index times
 // step plus start, rounded twice; the last one t), and whether they increase and t is finite; the
 // counts of the histogram that follows cleared.  t: the larger magnitude of range[0 ... 1], or `th`
-// where that is no NaN.  (On the host the edges, their copy and a second wait for the device were
+// where that is no NaN; with `inside`, a range that reaches beyond it counts as one without edges.  (On the host the edges, their copy and a second wait for the device were
 // 100 us of the 240 that a tensor took.)
 __global__ __launch_bounds__(1024) void symmetric_edges_kernel(const float* range, float th,
-                                                               int bins, float* edges,
+                                                               bool inside, int bins, float* edges,
                                                                uint32_t* increase,
                                                                uint32_t* counts) {
-  float t = th;
-  if (th != th) {
-    const float x = fabsf(range[0]), y = fabsf(range[1]);
-    t = (x < y) ? y : x;
-  }
+  const float x = fabsf(range[0]), y = fabsf(range[1]), reach = (x < y) ? y : x;
+  const float t = th != th ? reach : th;
   const float step = (t + t) / static_cast<float>(bins);
-  bool ok = t < INFINITY;
+  bool ok = t < INFINITY && !(inside && reach > t);
   for (int i = threadIdx.x; i < bins; i += 1024) {
     const float edge = static_cast<float>(i) * step - t;
     const float next = i + 1 < bins ? static_cast<float>(i + 1) * step - t : t;
@@ -149,10 +146,34 @@ void launch_histogram(hipStream_t s, const float* in, size_t n, const float* edg
 
 using namespace mxq;
 
+static int symmetric_histogram(void* stream, const float* in, size_t n, int bins, float th,
+                               bool inside, uint32_t* out, void* workspace,
+                               size_t workspace_bytes) {
+  MXQ_API_BEGIN();
+  MXQ_CHECK(bins > 0 && bins <= (1 << 24), "a histogram needs at least one bin, and at most 2^24");
+  MXQ_CHECK(n > 0 && n <= 0xffffffffu, "counts are 32 bits wide, and no value has no range");
+  MXQ_CHECK(in != nullptr && out != nullptr && workspace != nullptr, "null pointer");
+  const size_t extremes = mxq_minmax_f32_workspace(n);
+  MXQ_CHECK(workspace_bytes >= mxq_symmetric_histogram_f32_workspace(n, bins) &&
+                (reinterpret_cast<uintptr_t>(workspace) & 15u) == 0,
+            "workspace too small or unaligned");
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  char* const ws = static_cast<char*>(workspace);
+  float* const range = reinterpret_cast<float*>(out);
+  float* const edges = reinterpret_cast<float*>(ws + extremes);
+  const int status = mxq_minmax_f32(stream, in, n, range, range + 1, ws, extremes);
+  if (status != 0) return status;
+  hipLaunchKernelGGL(symmetric_edges_kernel, dim3(1), dim3(1024), 0, s, range, th, inside, bins,
+                     edges, out + 2, out + 3);
+  MXQ_LAUNCH_CHECK();
+  launch_histogram(s, in, n, edges, bins, out + 3, out + 2);
+  MXQ_API_END();
+}
+
 extern "C" {
 
-int mxq_histogram_f32(void* stream, const float* in, size_t n, const float* edges,
-                                 int bins, uint32_t* counts) {
+int mxq_histogram_f32(void* stream, const float* in, size_t n, const float* edges, int bins,
+                      uint32_t* counts) {
   MXQ_API_BEGIN();
   MXQ_CHECK(bins > 0, "a histogram needs at least one bin");
   MXQ_CHECK(n <= 0xffffffffu, "counts are 32 bits wide");
@@ -173,25 +194,12 @@ size_t mxq_symmetric_histogram_f32_workspace(size_t n, int bins) {
 
 int mxq_symmetric_histogram_f32(void* stream, const float* in, size_t n, int bins, float th,
                                 uint32_t* out, void* workspace, size_t workspace_bytes) {
-  MXQ_API_BEGIN();
-  MXQ_CHECK(bins > 0 && bins <= (1 << 24), "a histogram needs at least one bin, and at most 2^24");
-  MXQ_CHECK(n > 0 && n <= 0xffffffffu, "counts are 32 bits wide, and no value has no range");
-  MXQ_CHECK(in != nullptr && out != nullptr && workspace != nullptr, "null pointer");
-  const size_t extremes = mxq_minmax_f32_workspace(n);
-  MXQ_CHECK(workspace_bytes >= mxq_symmetric_histogram_f32_workspace(n, bins) &&
-                (reinterpret_cast<uintptr_t>(workspace) & 15u) == 0,
-            "workspace too small or unaligned");
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  char* const ws = static_cast<char*>(workspace);
-  float* const range = reinterpret_cast<float*>(out);
-  float* const edges = reinterpret_cast<float*>(ws + extremes);
-  const int status = mxq_minmax_f32(stream, in, n, range, range + 1, ws, extremes);
-  if (status != 0) return status;
-  hipLaunchKernelGGL(symmetric_edges_kernel, dim3(1), dim3(1024), 0, s, range, th, bins, edges,
-                     out + 2, out + 3);
-  MXQ_LAUNCH_CHECK();
-  launch_histogram(s, in, n, edges, bins, out + 3, out + 2);
-  MXQ_API_END();
+  return symmetric_histogram(stream, in, n, bins, th, false, out, workspace, workspace_bytes);
+}
+
+int mxq_symmetric_histogram_inside_f32(void* stream, const float* in, size_t n, int bins, float th,
+                                       uint32_t* out, void* workspace, size_t workspace_bytes) {
+  return symmetric_histogram(stream, in, n, bins, th, true, out, workspace, workspace_bytes);
 }
 
 }  // extern "C"

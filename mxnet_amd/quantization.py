@@ -126,15 +126,16 @@ class _Values:
         else:
             self._host = _to_numpy(arr)
 
-    def measure(self, bins, th=None):
+    def measure(self, bins, th=None, inside=False):
         """Take the extreme values and the counts over [-th, th] (or over the values' own symmetric
         range) from the device in one go: one wait for it instead of two, between which it idles.  A
-        first batch of 196608 values in 8001 bins 240 -> 100 us."""
+        first batch of 196608 values in 8001 bins 125 -> 65 us.  With `inside` there are counts only
+        if no value lies beyond `th`."""
         if self._device is None or not 0 < bins <= 1 << 24:
             return
         if th is not None and not (isinstance(th, np.float32) and np.isfinite(th)):
             return  # edges in float64, as numpy has them
-        found = capi.symmetric_histogram(self._device, bins, th).cpu().numpy()
+        found = capi.symmetric_histogram(self._device, bins, th, inside).cpu().numpy()
         lo, hi = found[:2].view(np.float32)
         self._range = lo, hi
         if found[2]:
@@ -289,7 +290,8 @@ class _LayerHistogramCollector(CalibrationCollector):
             arr.measure(self.num_bins)
             self.hist_dict[name] = _SymmetricHistogram.of(arr, self.num_bins).as_tuple()
         else:
-            arr.measure(len(seen[0]), seen[4])
+            # a batch that reaches further grows the histogram and is counted in the grown one
+            arr.measure(len(seen[0]), seen[4], inside=True)
             lo, hi = arr.extremes()
             self.hist_dict[name] = self.combine_histogram(seen, arr, lo, hi,
                                                           max(abs(lo), abs(hi)))

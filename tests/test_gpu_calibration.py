@@ -99,3 +99,18 @@ def test_nothing_is_counted_without_edges(bins, value, th):
     found = capi.symmetric_histogram(x, bins, th).cpu().numpy()
     assert tuple(found[:2].view(np.float32)) == (-np.float32(value), np.float32(value))
     assert found[2] == 0 and not found[3:].any()
+
+
+@pytest.mark.parametrize("bins", [101, 8001, 20001])
+@pytest.mark.parametrize("value, counted", [(0.5, True), (np.nextafter(np.float32(0.5), 1), False),
+                                            (-0.6, False), (np.inf, False)])
+def test_nothing_is_counted_of_a_batch_that_reaches_further(bins, value, counted):
+    x = np.random.default_rng(bins).uniform(-0.5, 0.5, 70001).astype(np.float32)
+    x[777] = value
+    t = torch.from_numpy(x).cuda()
+    found = capi.symmetric_histogram(t, bins, np.float32(0.5), inside=True).cpu().numpy()
+    assert tuple(found[:2].view(np.float32)) == (x.min(), x.max())
+    assert found[2] == counted
+    plain = capi.symmetric_histogram(t, bins, np.float32(0.5)).cpu().numpy()
+    assert plain[2] == 1 and plain[3:].sum() == 70001 - (not counted)
+    assert np.array_equal(found[3:], plain[3:] if counted else 0 * plain[3:])
