@@ -111,6 +111,20 @@ def _to_numpy(arr):
     return arr.detach().cpu().numpy() if isinstance(arr, torch.Tensor) else np.asarray(arr)
 
 
+def _edges_in_float32():
+    """Whether the installed numpy computes a float32 histogram's edges in float32 (from its version 2
+    on; before, in float64 and rounded), as the device does."""
+    th, bins = np.float32(2.7), 8001
+    asked = np.histogram_bin_edges(np.empty(0, np.float32), bins=bins, range=(-th, th))
+    step = np.float32(th + th) / np.float32(bins)
+    made = np.arange(bins + 1, dtype=np.float32) * step - th
+    made[-1] = th
+    return asked.dtype == np.float32 and np.array_equal(asked, made)
+
+
+_EDGES_IN_FLOAT32 = _edges_in_float32()
+
+
 class _Values:
     """A collected tensor as the collectors look at it: its extreme values and its counts over
     given bins, as numpy has them.  A float32 tensor on the device is reduced and counted
@@ -131,7 +145,7 @@ class _Values:
         range) from the device in one go: one wait for it instead of two, between which it idles.  A
         first batch of 196608 values in 8001 bins 125 -> 65 us.  With `inside` there are counts only
         if no value lies beyond `th`."""
-        if self._device is None or not 0 < bins <= 1 << 24:
+        if self._device is None or not 0 < bins <= 1 << 24 or not _EDGES_IN_FLOAT32:
             return
         if th is not None and not (isinstance(th, np.float32) and np.isfinite(th)):
             return  # edges in float64, as numpy has them
