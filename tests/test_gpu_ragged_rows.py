@@ -96,7 +96,7 @@ def test_fc_sum_rows_of_any_width(cfg, N, offset, relu):
     np.testing.assert_array_equal(o.get(), want)
 
 
-@pytest.mark.parametrize("cfg", [11, 22, 24, 25, 31, 33, 36, 37, 38, 39])
+@pytest.mark.parametrize("cfg", [11, 22, 23, 24, 25, 31, 33, 36, 37, 38, 39])
 @pytest.mark.parametrize("O, H", [(57, 6), (30, 7), (131, 8)])
 def test_conv_rows_and_planes_of_any_channel_count(cfg, O, H):
     from mxnet_amd import capi
@@ -140,12 +140,21 @@ def test_conv_of_few_channels_out(M_side, C, O, k, N):
                int8_uniform((O,), seed=2))
     r = (-RD, RD, -RW, RW, -RB, RB)
     x, y, z = (dev(a) for a in (d.transpose(0, 2, 3, 1), w.transpose(0, 2, 3, 1), b))
-    got = capi.quantized_conv_nhwc(x, y, z, *scalars(*r), pad=(k // 2, k // 2), want_int32=True)
+    got = capi.quantized_conv_nhwc(x, y, z, *scalars(*r), pad=(k // 2, k // 2), want_int32=True,
+                                   calib=CALIB)
     want = capi.quantized_conv_nhwc(x, y, z, *scalars(*r), pad=(k // 2, k // 2), want_int32=True,
                                     force=(25, 1))
     assert torch.equal(got["out32"], want["out32"])
-    few = oracle.quantized_conv(d[:1], w, b, *r, (1, 1), (k // 2, k // 2))[0]
-    np.testing.assert_array_equal(got["out32"][:1].cpu().numpy().transpose(0, 3, 1, 2), few)
+    acc = got["out32"].cpu().numpy()
+    some = [0, N - 1]
+    few, lo, hi = oracle.quantized_conv(d[some], w, b, *r, (1, 1), (k // 2, k // 2))
+    np.testing.assert_array_equal(acc[some].transpose(0, 3, 1, 2), few)
+    # the bytes of all images, with int32 rows beside them and alone
+    want8 = oracle.requantize(acc, lo, hi, *CALIB)[0]
+    alone = capi.quantized_conv_nhwc(x, y, z, *scalars(*r), pad=(k // 2, k // 2), want_int32=False,
+                                     calib=CALIB)
+    for out in (got, alone):
+        np.testing.assert_array_equal(out["out8"].cpu().numpy(), want8)
 
 
 # more than six tiles a CU over weights, or data, of fewer than the 16 bytes that a padding copy reads at
