@@ -286,24 +286,41 @@ __device__ __forceinline__ void block_tile(const BlockArgs& p, int tile, int fir
     }
   }
   // For each of the tile's pixels where it lies in the wide tensors and in the last layer's result,
-  // past their ends for those past the edges, and where the patch has its first tap.
-  constexpr int kMore = 24;  // rows a load instruction of the shortcut may go beyond the tile
+  // past their ends for those past the edges, and where the patch has its first tap.  With more than
+  // 128 channels in the middle LDS has no room for three tables where it had for one (7 x 7 x 128 -> 256
+  // -> 2048 -> 256 is 352 bytes short): every wave finds its own rows' first taps, while the patch is on
+  // its way, and the last layer's places take those of the first one's bias, behind that layer.
+  constexpr bool kOneTable = GC == 8;
   uint32_t* const wide_of = reinterpret_cast<uint32_t*>(smem + p.off_pixel);
-  uint32_t* const next_of = wide_of + TM + kMore;
-  int* const place_of = reinterpret_cast<int*>(next_of + TM);
-  static_assert(TM <= 64 && kMore <= TM, "one wave makes the tables");
-  if (wave == NW - 1 && lane < TM) {  // the wave that has least to fetch
+  uint32_t* const next_of =
+      kOneTable ? reinterpret_cast<uint32_t*>(smem + p.off_bias) : wide_of + TM;
+  int* const place_of = reinterpret_cast<int*>(wide_of + 2 * TM);
+  struct Pixel {
+    int n, h, w, tx;
+  };
+  auto pixel_at = [&](int row) MXQ_INLINE {
     // rows without a pixel read the first one's; never stored
-    const int i = start_at + (lane < p.count ? lane : 0);
+    const int i = start_at + (row < p.count ? row : 0);
     const int img = quotient_any(i, p.area, p.magic_area), rem = i - img * p.area;
     const int ty = quotient(rem, p.magic_across), tx = rem - ty * p.across;
-    const int n = n0 + img, h = h0 + ty, w = w0 + tx;
-    const bool ok = lane < p.count && n < p.N && h < p.H && w < p.W;
-    const uint32_t pixel = static_cast<uint32_t>((n * p.H + h) * p.W + w);
+    return Pixel{n0 + img, h0 + ty, w0 + tx, tx};
+  };
+  auto place_at = [&](const Pixel& x) MXQ_INLINE {
+    return (x.n * H2 + x.h - v0) * row_pitch + x.tx * PP * 16;
+  };
+  static_assert(TM <= 64, "one wave makes the tables");
+  const bool makes_tables = wave == NW - 1 && lane < TM;  // the wave that has least to fetch
+  uint32_t next_at = kOutOfRange;
+  if (makes_tables) {
+    const Pixel x = pixel_at(lane);
+    const bool ok = lane < p.count && x.n < p.N && x.h < p.H && x.w < p.W;
+    const uint32_t pixel = static_cast<uint32_t>((x.n * p.H + x.h) * p.W + x.w);
     wide_of[lane] = ok ? pixel * p.Co : kOutOfRange;
-    next_of[lane] = ok ? pixel * p.Ca : kOutOfRange;
-    place_of[lane] = (n * H2 + h - v0) * row_pitch + tx * PP * 16;
-    if (lane < kMore) wide_of[TM + lane] = kOutOfRange;
+    next_at = ok ? pixel * p.Ca : kOutOfRange;
+    if constexpr (!kOneTable) {
+      next_of[lane] = next_at;
+      place_of[lane] = place_at(x);
+    }
   }
   const int* const sbias = reinterpret_cast<const int*>(smem + p.off_bias);
   const int bias_c = (p.Cm + 31) & ~31, bias_a = bias_c + ((p.Co + 31) & ~31);
@@ -347,8 +364,10 @@ __device__ __forceinline__ void block_tile(const BlockArgs& p, int tile, int fir
   int res_j = res_at * 64 + lane - res_row * PO;
   auto fetch_shortcut = [&]() MXQ_INLINE {
     if (res_at * 64 < res_slots) {
-      // (the pad of a row gets what follows the row in memory)
-      fetch(res_at * 1024, wide_of[res_row] + 16 * res_j, res_rsrc);
+      // (the pad of a row gets what follows the row in memory; tiles of 32 do not end on a whole load
+      // instruction, and get their last row again behind it)
+      const int row = TM % 64 == 0 || res_row < TM ? res_row : TM - 1;
+      fetch(res_at * 1024, wide_of[row] + 16 * res_j, res_rsrc);
       res_at += NW;
       res_row += p.res_rows;
       res_j += p.res_rest;
@@ -361,6 +380,12 @@ __device__ __forceinline__ void block_tile(const BlockArgs& p, int tile, int fir
   // this lane's rows: where they begin in each of the three
   const int frow = lane & 31, fgrp = lane >> 5;
   const int row0 = wm * RT * 32 + frow;
+  int in_patch[RT];
+  if constexpr (kOneTable) {
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+      in_patch[rt] = p.off_patch + place_at(pixel_at(row0 + 32 * rt)) + fgrp * 16;
+  }
   v16i acc[RT];
   // The bias as first accumulators.  Each row tile reads its own: registers are copied with vector
   // instructions, which this kernel is short of, so the compiler must not see that they are the same.
@@ -432,9 +457,11 @@ __device__ __forceinline__ void block_tile(const BlockArgs& p, int tile, int fir
   // ---- 3 x 3 ------------------------------------------------------------------------------
   const int groups = p.kb / GB;
   if (has_b) {
-    int in_patch[RT];
+    if constexpr (!kOneTable) {
 #pragma unroll
-    for (int rt = 0; rt < RT; ++rt) in_patch[rt] = p.off_patch + place_of[row0 + 32 * rt] + fgrp * 16;
+      for (int rt = 0; rt < RT; ++rt)
+        in_patch[rt] = p.off_patch + place_of[row0 + 32 * rt] + fgrp * 16;
+    }
     start(acc, sbias + 32 * wn);
     if constexpr (KSB != 0) {
       constexpr int kRow = 3 * KSB, kTap = odd(2 * KSB) * 16;
@@ -515,6 +542,7 @@ __device__ __forceinline__ void block_tile(const BlockArgs& p, int tile, int fir
   __builtin_amdgcn_s_barrier();  // every wave is through with the patch
   asm volatile("" ::: "memory");
   if (has_b) finish_layer(s_b, t_b, c_b, (has & 1) != 0, p.relu_b, wn, PM);
+  if (kOneTable && makes_tables) next_of[lane] = next_at;
   publish(std::integral_constant<int, GC>());  // the result, and the shortcut in front of `wc`
 
   // ---- 1 x 1 and the sum ------------------------------------------------------------------
@@ -774,7 +802,8 @@ bool fit_lds(BlockPlan* b, int C, int Cm, int Co, int Ca) {
   const int patch = first > mid ? static_cast<int>(first) : mid;
   const int bias = 4 * (up(Cm, 32) + up(Co, 32) + up(Ca, 32));
   const int table = 4 * (b->steps[0] + 2 * 8);
-  const long long lds = static_cast<long long>(wide) + patch + bias + table + 4 * (3 * b->tm + 24);
+  const long long lds = static_cast<long long>(wide) + patch + bias + table +
+                        4 * b->tm * (b->variant == 256 ? 1 : 3);
   b->off_patch = wide;
   b->off_bias = wide + patch;
   b->off_table = b->off_bias + bias;

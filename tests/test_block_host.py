@@ -27,3 +27,13 @@ def test_block_reads_only_the_lds_it_has(n, h, w, tile):
                     assert reach <= have, (c, mid, out, after)
                     some += have > 0
     assert some > 100
+
+
+# within 608 bytes of what a tile of 64 pixels may have: of all LDS, and of half of it
+@pytest.mark.parametrize("shape, most", [
+    ((64, 7, 7, 128, 256, 2048, 256), 160 * 1024), ((64, 15, 15, 96, 192, 2048, 0), 160 * 1024),
+    ((64, 10, 10, 1232, 112, 768, 0), 160 * 1024), ((64, 4, 4, 704, 256, 512, 256), 160 * 1024),
+    ((64, 11, 11, 528, 112, 512, 0), 80 * 1024), ((64, 17, 17, 320, 128, 256, 0), 160 * 1024 // 3)])
+def test_block_tables_take_no_more_lds_than_a_word_a_pixel(shape, most):
+    have, reach = lds(*shape, 64)
+    assert 0 < have <= most and reach <= have

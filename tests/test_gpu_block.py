@@ -134,6 +134,18 @@ def test_block_whose_taps_are_constants(n, h, w, c, mid, out, after, whole):
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("n,h,w,c,mid,out,after", [
+    (1, 7, 7, 128, 256, 2048, 256), (1, 8, 8, 96, 192, 2048, 0), (2, 10, 10, 1232, 112, 768, 0),
+    (1, 4, 4, 704, 256, 512, 256), (1, 11, 11, 528, 112, 512, 0)])
+@pytest.mark.parametrize("whole", [False, True])
+def test_block_that_lds_just_holds(n, h, w, c, mid, out, after, whole):
+    if whole:
+        n += torch.cuda.get_device_properties(0).multi_processor_count * 32 // (h * w) + 1
+    have, want, _ = blocks(n, h, w, c, mid, out, after)
+    for a, b in zip(have, want):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("relu1,relu3", [(0, 0), (1, 0), (0, 1)])
 @pytest.mark.parametrize("mid,spread", [(48, 0.02), (128, 40.0), (160, 1.0)])
 def test_block_ranges_on_whole_tiles(mid, spread, relu1, relu3):
