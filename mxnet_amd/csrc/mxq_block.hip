@@ -490,14 +490,18 @@ __device__ __forceinline__ void block_tile(const BlockArgs& p, int tile, int fir
         for (int rt = 0; rt < RT; ++rt) in_patch[rt] = below[rt];
       }
     } else {
-      const int* const table = reinterpret_cast<const int*>(smem + p.off_table);
-      auto read_offsets = [&](int g, int (&o)[GB]) MXQ_INLINE {
+      // A group's places come with one read, a lane each, that is on its way while a group is multiplied
+      // (pair by pair behind it, waited for each time: 10 x 10 x 1232 -> 112 25.7 us, 22.0 when all were
+      // asked for at once, 20.6 so).
+      const int* table =
+          reinterpret_cast<const int*>(smem + p.off_table) + (lane < GB ? lane : 0);
+      auto take_offsets = [&](int x, int (&o)[GB]) MXQ_INLINE {
 #pragma unroll
-        for (int i = 0; i < GB; ++i) o[i] = __builtin_amdgcn_readfirstlane(table[g * GB + i]);
+        for (int i = 0; i < GB; ++i) o[i] = __builtin_amdgcn_readlane(x, i);
       };
       int now[GB], later[GB];
-      read_offsets(0, now);
-      read_offsets(1, later);
+      take_offsets(table[0], now);
+      take_offsets(table[GB], later);
       auto read = [&](int i, v4i (&x)[RT]) MXQ_INLINE {
         read_pixels(x, in_patch, i < GB ? now[i] : later[i - GB]);
       };
@@ -505,10 +509,12 @@ __device__ __forceinline__ void block_tile(const BlockArgs& p, int tile, int fir
       for (int g = 0; g < groups; ++g) {
         fetch_shortcut();
         if (g == 0) fetch_later_bias();
+        const int ahead = table[2 * GB];
+        table += GB;
         run_group(wb, fragments(g + 1 < groups, first_b + (g + 1) * GB), read);
 #pragma unroll
         for (int i = 0; i < GB; ++i) now[i] = later[i];
-        read_offsets(g + 2, later);
+        take_offsets(ahead, later);
       }
     }
   } else {
