@@ -24,18 +24,20 @@
 // distinct bank groups without a permutation, for any channel count.
 //
 // What bounds it: instruction issue.  Vector instructions and MFMAs, which overlap little (the waves
-// of a work-group run in step from each barrier on), fill 75 to 85 % of a CU's busy clocks; the sum
-// alone is 7 vector instructions per output of 64 ... 256 channels in the middle times four.  So what is
-// not arithmetic has as few as possible: a weight's place is a scalar offset and an immediate, the three
-// taps of a row are immediates where the channels are those of a kernel instance (KSB), the places of a
-// tile's pixels in the tensors come from a table, and pieces of rows are walked by carries, not divided
-// (984 -> 760 vector instructions a wave of 56 x 56 x 64, of which 550 are arithmetic); and a barrier
-// waits for what it is for, not for weights or stores on their way.  The 3 x 3 layer of 256 channels is
-// bound by the 64 bytes a clock that a CU takes in (its 590 KB of weights: 9200 clocks, as many as the
-// products take; 10000 measured), as is the time in front of it.  Measured in a quantized ResNet-50's
-// pass at batch 64, before and after: 46.2 -> 39.3 us for 56 x 56 x 64 -> 256 -> 64, 34.4 -> 32.1 for
-// 28 x 28 x 128, 26.7 -> 24.9 for 14 x 14 x 256; the pass 593 -> 566, one image 200.3 -> 193.6.  As three
-// launches they were 60, 45 and 38 us.
+// of a work-group run in step from each barrier on), take 81 % of a CU's busy clocks in 56 x 56 x 64 and
+// 69 % in 28 x 28 x 128 and 14 x 14 x 256 (counters, batch 64); the sum alone is 7 vector instructions
+// per output of 64 ... 256 channels in the middle times four.  So what is not arithmetic has as few as
+// possible: a weight's place is a scalar offset and an immediate, the three taps of a row are immediates
+// where the channels are those of a kernel instance (KSB), the places of a tile's pixels in the tensors
+// come from a table, and pieces of rows are walked by carries, not divided (947 -> 822 vector instructions
+// a wave of 56 x 56 x 64, 1007 -> 892 and 2035 -> 1594 of the others); and a barrier waits for what it is for,
+// not for weights or stores on their way.  The 3 x 3 layer of 256 channels takes in 590 KB of weights, 9200
+// clocks at the 64 bytes a clock of a CU and as many as its products.  Measured in a quantized
+// ResNet-50's pass at batch 64, before and after: 45.0 -> 39.9 us for 56 x 56 x 64 -> 256 -> 64, 33.9 ->
+// 32.2 for 28 x 28 x 128, 26.6 -> 25.0 for 14 x 14 x 256; the pass's kernels 629 -> 603, one image's 210 ->
+// 204.  Channels that no instance is made for, the block alone: 56 x 56 x 48 -> 192 -> 48 38.3 -> 37.7, 28
+// x 28 x 96 -> 384 -> 96 31.5 -> 30.1, 14 x 14 x 192 -> 768 -> 192 18.5 -> 17.1.  As three launches, alone: 67,
+// 53 and 43 us against 49, 30 and 28.
 // Measured and not kept: the 3 x 3 layer's reduction shared by the waves that have no column tile of
 // it (up to 128 channels in the middle half of them), or by 16 waves: level or behind, for the sums
 // that are exchanged cost more vector instructions than the idle waves did time;
@@ -249,10 +251,9 @@ __device__ __forceinline__ void block_tile(const BlockArgs& p, int tile, int fir
     // A row of the patch is a whole number of load instructions, and a row is one scalar offset: the
     // lanes look at a row each, all at once, and what they find is read from them row by row; a lane's
     // place in a row moves on by carries from part to part.  Parts start at the wave behind the one that
-    // took the last row of the part before, so that all take as many.  (An instruction takes a lone wave
-    // five clocks here: looking at the row for every load, 55 instructions, 14 x 14 x 256 had 3200
-    // clocks in front of its patch, and 28 x 28 x 128 2300.)  No short circuits: a branch takes longer than
-    // what it skips.
+    // took the last row of the part before, so that all take as many.  (The waves have little else to do
+    // here, so each of the 55 instructions that looking at the row for every load takes is waited for.)  No
+    // short circuits: a branch takes longer than what it skips.
     const int row_bytes = p.W * p.C;
     const int px_step = quotient(64, p.magic_pixel), j_rest = 64 - px_step * PP;
     for (int first_row = 0; first_row < p.rows; first_row += 64) {
@@ -441,7 +442,7 @@ __device__ __forceinline__ void block_tile(const BlockArgs& p, int tile, int fir
   };
   // What this wave wrote to LDS, and what it had written there but for the newest `pending` loads, to
   // all of them.  Only what the barrier is for is waited for: weights on their way to registers, or
-  // stores, at a barrier that publishes a result cost 1000 to 2500 clocks each.
+  // stores, at a barrier that publishes a result would cost a round trip to memory each.
   auto publish = [&](auto pending) MXQ_INLINE {
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(decltype(pending)::value) : "memory");
     __builtin_amdgcn_s_barrier();
@@ -831,8 +832,10 @@ BlockPlan plan_tiles(int N, int H, int W, int C, int Cm, int Co, int Ca, int tm)
   // A run of pixels in the tensor's order wastes no row of a tile, but its patch is three to five
   // times the tile: 36 KB for 64 pixels of a 56 x 56 plane over 64 channels where 8 x 8 of them need
   // 10, and LDS is what limits the work-groups a CU holds.  So runs where a CU holds one anyway or
-  // where it still holds two; rectangles elsewhere.  (Batch 64, runs / rectangles: 56 x 56 x 64 43.4 /
-  // 39.0 us, 28 x 28 x 128 31.6 / 32.0, 14 x 14 x 256 23.2 / 24.6.)
+  // where it still holds two; rectangles elsewhere.  (Batch 64, runs / rectangles: 56 x 56 x 64 63.1 /
+  // 49.3 us, 30 x 30 x 64 20.7 / 19.2, 28 x 28 x 128 30.4 / 32.0, 17 x 17 x 128 13.9 / 16.1, 40 x 40 x 128, where
+  // a CU does not hold two, 54.0 / 53.4, 14 x 14 x 256 27.6 / 29.5, 24 x 24 x 256 73.7 / 79.8.  On tiles of 32
+  // rectangles are ahead by up to 5 %: 28 x 28 x 128 on one image 7.6 / 7.2.)
   if (b.variant > 64) {
     b.run = 1;
     // its rows, one above and below, two more for every image boundary inside
@@ -878,10 +881,11 @@ BlockPlan plan_tiles(int N, int H, int W, int C, int Cm, int Co, int Ca, int tm)
 
 // Tiles of 64 pixels: a CU then multiplies a weight as long as it takes in the next one.  Where they
 // would leave half of the CUs idle, of 32: a tile's chain is shorter by half of its products and its
-// vector work (28 x 28 x 128 on one image 10.7 us -> 9.2, on 8 images 13 -> 9.6; 14 x 14 x 256 on
-// 4 images 18.9 -> 15.6).  And where a few runs are left over when every CU has had as many, those
-// go in halves, so that fewer CUs end with a whole tile more than the others (784 tiles of 28 x 28 x
-// 128 on 256 CUs, four blocks in a network's pass: 2 us less each).
+// vector work (28 x 28 x 128 on one image 9.3 us -> 7.5, on 8 images 10.1 -> 8.4; 14 x 14 x 256 on
+// 4 images 22.7 -> 16.9, on 32 24.4 -> 18.9; 56 x 56 x 64 on two, 98 tiles, 8.4 -> 6.7).  And where a few
+// runs are left over when every CU has had as many, those go in halves, so that fewer CUs end with a
+// whole tile more than the others (28 x 28 x 128 at batch 64, 784 tiles on 256 CUs, 30.8 -> 29.2; at batch
+// 24 15.9 -> 14.4, at 32, 136 left over, 17.3 and 17.6).
 BlockPlan plan_block(int N, int H, int W, int C, int Cm, int Co, int Ca) {
   BlockPlan b = plan_tiles(N, H, W, C, Cm, Co, Ca, 64);
   const int cus = num_cus(), over = b.tiles % cus;
@@ -931,10 +935,12 @@ using namespace mxq;
 extern "C" {
 
 // Whether it is also the faster way.  It is from one image on with up to 128 channels in the middle
-// (56 x 56 x 64: 7.4 us against 14.1 in three launches on one image, 38.6 against 60.2 on 64;
-// 28 x 28 x 128 9.2 / 14.0 and 30.4 / 45.2).  Above that a tile alone takes 15 us, most of it the
-// 1.1 MB of weights that a CU takes in: 19 tiles (14 x 14 x 256 on 3 images) 15.6 us against 16.0,
-// 25 tiles 15.6 against 16.5, 98 of 32 pixels 16.6 against 23.3, 196 of 64 22.0 against 38.3.
+// (56 x 56 x 64: 6.5 us against 14.7 in three launches on one image, 49 against 67 on 64; 28 x 28 x 128 7.6
+// / 15.0 and 30 / 53).  Above that a tile alone takes 16 us, most of it the 1.1 MB of weights that a CU
+// takes in: 7 tiles (7 x 7 x 256 on 4 images) 16.2 us against 14.7, 13 tiles 16.5 against 16.1 ... 16.5, 25 tiles
+// 16.8 against 19.4, 98 of 32 pixels 18.9 against 30.0, 196 of 64 27.6 against 42.7.  (The line was drawn
+// where an earlier form of the kernel met the three launches; this one would already be ahead at 19
+// tiles, 16.8 against 18.9.)
 int mxq_quantized_block_fits(int N, int H, int W, int C, int C_mid, int C_out, int C_next) {
   try {
     const BlockPlan b = plan_block(N, H, W, C, C_mid, C_out, C_next);

@@ -149,7 +149,9 @@ FcPlan plan_fc(int M, int N, int K, bool aligned, bool fused8, const GemmForce& 
 // 256 x 2048 9.2 against 10.6).  Below 64 bytes a row there is little to read and the copies cost as much,
 // so twice as many tiles are asked for (28717 x 18 -> 352, 9878 tiles, 38.9 us against 16.8; 136367 x 13
 // -> 8, 4262 tiles, 19.7 against 15.5; 9245 x 58 -> 239, 2312 tiles, 16.7 against 12.6; 1813 x 19 -> 544,
-// 969 tiles, 10.9 against 11.3).
+// 969 tiles, 10.9 against 11.3).  However short they are: a copy sixteen times as large as rows of one
+// byte is no larger than that of fifteen (60000 x 1 -> 16, 1875 tiles, 9.3 against 7.7, x 15 9.4 against 7.6; 60000 x 1
+// -> 300 54 against 16.5, x 15 60 against 16.2).
 int fc_padded_k(int M, int N, int K) {
   const int Kp = (K + 15) / 16 * 16;
   const bool wanted = Kp != K && few_tiles_count(M, N) > (K >= 64 ? 3L : 6L) * num_cus() &&

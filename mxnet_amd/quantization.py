@@ -143,8 +143,8 @@ class _Values:
     def measure(self, bins, th=None, inside=False):
         """Take the extreme values and the counts over [-th, th] (or over the values' own symmetric
         range) from the device in one go: one wait for it instead of two, between which it idles.  A
-        first batch of 196608 values in 8001 bins 125 -> 65 us.  With `inside` there are counts only
-        if no value lies beyond `th`."""
+        batch of 196608 values in 8001 bins 133 -> 67 us.  With `inside` there are counts only if no
+        value lies beyond `th`; such a batch is waited for twice as before, and costs 155 us, not 147."""
         if self._device is None or not 0 < bins <= 1 << 24 or not _EDGES_IN_FLOAT32:
             return
         if th is not None and not (isinstance(th, np.float32) and np.isfinite(th)):
