@@ -114,6 +114,19 @@ def test_conv_rows_and_planes_of_any_channel_count(cfg, O, H):
     np.testing.assert_array_equal(planes["out32"].cpu().numpy(), acc)
 
 
+# tiles whose stages are too small to turn a 32-bit tile round: stored as they lie
+@pytest.mark.parametrize("O", [112, 113, 114, 115])
+@pytest.mark.parametrize("H", [33, 40])
+def test_conv_planes_from_small_tiles(O, H):
+    from mxnet_amd import capi
+    d, w, b = (int8_uniform((8, 3, H, H), seed=O), int8_uniform((O, 3, 3, 3), seed=1),
+               int8_uniform((O,), seed=2))
+    acc = oracle.quantized_conv(d, w, b, -RD, RD, -RW, RW, -RB, RB, (2, 2), (1, 1))[0]
+    planes = capi.quantized_conv_nchw(dev(d), dev(w), dev(b), *scalars(-RD, RD, -RW, RW, -RB, RB),
+                                      stride=(2, 2), pad=(1, 1))
+    np.testing.assert_array_equal(planes["out32"].cpu().numpy(), acc)
+
+
 # reductions below 64 bytes on either side of the tiles from which the rows are padded first
 @pytest.mark.parametrize("M, K, N", [(1569, 13, 1024), (1537, 13, 1024), (1536, 13, 1024),
                                      (3000, 1, 600), (2048, 63, 1001), (50000, 11, 14)])
