@@ -610,9 +610,10 @@ __device__ __forceinline__ void block_tile(const BlockArgs& p, int tile, int fir
   if (p.Ca != 0) load_first(wa, fragments(wn < tiles_a, p.at_a + wn * p.ka));
   publish_written();
 
-  // Rows of `chunks` pieces, `pitch` apart in LDS, to their pixels.  Plain stores: the next block
-  // reads both outputs, and what it finds in the memory-side cache it does not fetch from memory
-  // (quantized ResNet-50 at batch 64, all blocks with streaming stores / plain ones: 680 / 651 us).
+  // Rows of `chunks` pieces, `pitch` apart in LDS, to their pixels.  No streaming stores: the
+  // next block reads both outputs, and what it finds in the memory-side cache it does not fetch from
+  // memory (quantized ResNet-50 at batch 64, all blocks with streaming stores / plain ones / written
+  // through: 573 / 544 / 534 us; plain ones leave up to 32 MB of dirty lines to the launch's end).
   auto leave = [&](int at, int chunks, int pitch, uint32_t magic, int rows, int rest,
                    const uint32_t* pixel_of, int8_t* out) MXQ_INLINE {
     const auto to = __builtin_amdgcn_make_buffer_rsrc(
@@ -625,7 +626,7 @@ __device__ __forceinline__ void block_tile(const BlockArgs& p, int tile, int fir
       const uint32_t pixel = piece.row < TM ? pixel_of[piece.row] : kOutOfRange;
       __builtin_amdgcn_raw_buffer_store_b128(
           __builtin_bit_cast(v4u, *reinterpret_cast<const v4i*>(smem + piece.place(TM, at))), to,
-          pixel + 16 * piece.j, 0, 0);
+          pixel + 16 * piece.j, 0, kDeviceScope);
       piece.next(rows, rest, chunks, pitch);
     }
   };

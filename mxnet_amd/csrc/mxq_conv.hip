@@ -686,7 +686,7 @@ __global__ __launch_bounds__(256, KS > 5 ? 3 : 4) void conv_taps_kernel(TapArgs 
       const v4i val = *reinterpret_cast<const v4i*>(stage + rr * LD + c16 * 16);
       __builtin_amdgcn_raw_buffer_store_b128(
           val, out, o < p.O ? static_cast<uint32_t>(rr * p.O + o) : kOutOfRange, 0,
-          decltype(stream)::value ? 2 /* nt */ : 0);
+          decltype(stream)::value ? 2 /* nt */ : kDeviceScope);
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_wave_barrier();

@@ -254,7 +254,7 @@ __global__ __launch_bounds__(256, 2) void fc_stream_kernel(FcArgs p, int bn, int
         }
       }
       __builtin_amdgcn_raw_buffer_store_b128(val, out, rr * p.ldo + n_begin + s0 + c16 * 16, 0,
-                                             decltype(stream)::value ? kNonTemporal : 0);
+                                             decltype(stream)::value ? kNonTemporal : kDeviceScope);
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_wave_barrier();

@@ -147,7 +147,7 @@ __device__ __forceinline__ void resident(const Args& args, const ResidentArgs& p
       const uint32_t at =
           n0 + c * 16 < p.N ? static_cast<uint32_t>(row * p.ldo + c * 16) : kOutOfRange;
       __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, at, 0,
-                                             decltype(stream)::value ? kNonTemporal : 0);
+                                             decltype(stream)::value ? kNonTemporal : kDeviceScope);
     }
   };
 

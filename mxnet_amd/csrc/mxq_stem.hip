@@ -119,7 +119,7 @@ __global__ __launch_bounds__(256, 2) void conv_pool_kernel(StemArgs p) {
     asm volatile("" ::: "memory");
     const int px = piece_px < kColumns ? piece_px : 0;
     const v4i v = *reinterpret_cast<const v4i*>(stage + px * kPitch + piece_c * 16);
-    __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, piece_at, 0, 0);
+    __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, piece_at, 0, kDeviceScope);
     asm volatile("" ::: "memory");
   };
   // Everything that the walk starts with goes out at once: the bias, the weights, seven rows (and
