@@ -495,6 +495,8 @@ int mxq_quantized_conv_nchw(void* stream, const int8_t* data, const int8_t* weig
  * bias keep them zero through every layer).
  * mxq_quantize_to_nhwc: calibrated quantize_v2 (int8) of a float NCHW image straight into that
  * layout; space_to_depth != 0 into the layout of mxq_nchw_to_s2d_nhwc_i8.
+ * mxq_quantize_to_s2d: that, with H2 and W2 given; each may be one more than that layout's, the
+ * last row or column then holds zeros alone.
  * mxq_quantized_pooling_nhwc: mxq_quantized_pooling_nchw's windows and rounding on int8 of that
  * layout (C a multiple of 16); the range passes through and is left to the caller.
  * mxq_pack_weight: OIHW int8 -> [O_padded,KH,KW,C_padded] with zeros, or the weight of the
@@ -503,6 +505,9 @@ int mxq_quantized_conv_nchw(void* stream, const int8_t* data, const int8_t* weig
 int mxq_quantize_to_nhwc(void* stream, const float* in, int8_t* out, float* omin, float* omax,
                          int N, int C, int H, int W, int C_padded, int space_to_depth, int off_h,
                          int off_w, float min_calib, float max_calib);
+int mxq_quantize_to_s2d(void* stream, const float* in, int8_t* out, float* omin, float* omax,
+                        int N, int C, int H, int W, int C_padded, int off_h, int off_w, int H2,
+                        int W2, float min_calib, float max_calib);
 int mxq_quantized_pooling_nhwc(void* stream, const int8_t* in, int N, int H, int W, int C,
                                int kernel_h, int kernel_w, int stride_h, int stride_w, int pad_h,
                                int pad_w, int OH, int OW, int pool_type, int count_include_pad,

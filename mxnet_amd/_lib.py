@@ -95,6 +95,7 @@ SIGNATURES = {
     "mxq_quantized_conv_nchw": (_i, [_p, _p, _p, _p] + [_i] * 13 + [_p] * 6 +
                                 [_p, _p, _p, _p, _sz]),
     "mxq_quantize_to_nhwc": (_i, [_p] * 5 + [_i] * 8 + [_f, _f]),
+    "mxq_quantize_to_s2d": (_i, [_p] * 5 + [_i] * 9 + [_f, _f]),
     "mxq_quantized_pooling_nhwc": (_i, [_p, _p] + [_i] * 14 + [_p]),
     "mxq_pack_weight": (_i, [_p, _p, _p] + [_i] * 7),
     "mxq_quantized_block_fits": (_i, [_i] * 7),

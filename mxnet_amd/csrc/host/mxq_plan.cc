@@ -102,8 +102,12 @@ bool Plan::run(void* stream, const std::vector<at::Tensor>& feeds,
         break;
       }
       case Kind::kQuantNhwc:
-        rc = mxq_quantize_to_nhwc(stream, v(0), q(1), v(2), v(2) + 1, i(0), i(1), i(2), i(3),
-                                  i(4), i(5), i(6), i(7), f[0], f[1]);
+        if (i(5))
+          rc = mxq_quantize_to_s2d(stream, v(0), q(1), v(2), v(2) + 1, i(0), i(1), i(2), i(3),
+                                   i(4), i(6), i(7), i(8), i(9), f[0], f[1]);
+        else
+          rc = mxq_quantize_to_nhwc(stream, v(0), q(1), v(2), v(2) + 1, i(0), i(1), i(2), i(3),
+                                    i(4), 0, 0, 0, f[0], f[1]);
         break;
       case Kind::kToNhwc:
         rc = mxq_nchw_to_nhwc_pad_i8(stream, q(0), q(1), i(0), i(1), i(2), i(3), i(4));

@@ -394,17 +394,10 @@ void launch_s2d(hipStream_t s, const QuantNhwcArgs& a, int N) {
     flat ? launch_s2d_as<C, true, true>(s, a, N) : launch_s2d_as<C, true, false>(s, a, N);
 }
 
-}  // namespace
-}  // namespace mxq
-
-using namespace mxq;
-
-extern "C" {
-
-int mxq_quantize_to_nhwc(void* stream, const float* in, int8_t* out, float* omin, float* omax,
-                         int N, int C, int H, int W, int C_padded, int space_to_depth, int off_h,
-                         int off_w, float min_calib, float max_calib) {
-  MXQ_API_BEGIN();
+// One row or column of the space-to-depth form more than the image has: `more_h`, `more_w`.
+void quantize_to_nhwc(void* stream, const float* in, int8_t* out, float* omin, float* omax, int N,
+                      int C, int H, int W, int C_padded, bool space_to_depth, int off_h, int off_w,
+                      int more_h, int more_w, float min_calib, float max_calib) {
   MXQ_CHECK(N >= 0 && C > 0 && H > 0 && W > 0, "bad shape");
   MXQ_CHECK(C_padded % 16 == 0 && C_padded >= (space_to_depth ? 4 : 1) * C, "bad C_padded");
   MXQ_CHECK((off_h == 0 || off_h == 1) && (off_w == 0 || off_w == 1), "offsets are 0 or 1");
@@ -415,8 +408,8 @@ int mxq_quantize_to_nhwc(void* stream, const float* in, int8_t* out, float* omin
   a.omin = omin;
   a.omax = omax;
   a.C = C; a.H = H; a.W = W;
-  a.OH = space_to_depth ? (H + off_h + 1) / 2 : H;
-  a.OW = space_to_depth ? (W + off_w + 1) / 2 : W;
+  a.OH = space_to_depth ? (H + off_h + 1) / 2 + more_h : H;
+  a.OW = space_to_depth ? (W + off_w + 1) / 2 + more_w : W;
   a.chunks = C_padded / 16;
   a.off_h = off_h;
   a.off_w = off_w;
@@ -424,7 +417,7 @@ int mxq_quantize_to_nhwc(void* stream, const float* in, int8_t* out, float* omin
   a.range = (x < y) ? y : x;
   MXQ_CHECK(static_cast<long long>(a.OH) * a.OW < (1LL << 31), "image too large");
   a.pieces = static_cast<size_t>(N) * a.OH * a.OW * a.chunks;
-  if (a.pieces == 0) return 0;
+  if (a.pieces == 0) return;
   MXQ_CHECK(in != nullptr && out != nullptr && aligned16(out), "null or unaligned data pointer");
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (space_to_depth && C <= 4 && a.chunks == 1) {
@@ -441,6 +434,34 @@ int mxq_quantize_to_nhwc(void* stream, const float* in, int8_t* out, float* omin
     hipLaunchKernelGGL((quantize_nhwc_kernel<false>), dim3(blocks_for(a.pieces)), dim3(kThreads),
                        0, s, a);
   MXQ_LAUNCH_CHECK();
+}
+
+}  // namespace
+}  // namespace mxq
+
+using namespace mxq;
+
+extern "C" {
+
+int mxq_quantize_to_nhwc(void* stream, const float* in, int8_t* out, float* omin, float* omax,
+                         int N, int C, int H, int W, int C_padded, int space_to_depth, int off_h,
+                         int off_w, float min_calib, float max_calib) {
+  MXQ_API_BEGIN();
+  quantize_to_nhwc(stream, in, out, omin, omax, N, C, H, W, C_padded, space_to_depth != 0, off_h,
+                   off_w, 0, 0, min_calib, max_calib);
+  MXQ_API_END();
+}
+
+int mxq_quantize_to_s2d(void* stream, const float* in, int8_t* out, float* omin, float* omax,
+                        int N, int C, int H, int W, int C_padded, int off_h, int off_w, int H2,
+                        int W2, float min_calib, float max_calib) {
+  MXQ_API_BEGIN();
+  MXQ_CHECK(H > 0 && W > 0, "bad shape");
+  const long long more_h = H2 - (1LL * H + off_h + 1) / 2, more_w = W2 - (1LL * W + off_w + 1) / 2;
+  MXQ_CHECK((more_h == 0 || more_h == 1) && (more_w == 0 || more_w == 1),
+            "rows and columns that the image does not give");
+  quantize_to_nhwc(stream, in, out, omin, omax, N, C, H, W, C_padded, true, off_h, off_w,
+                   static_cast<int>(more_h), static_cast<int>(more_w), min_calib, max_calib);
   MXQ_API_END();
 }
 
