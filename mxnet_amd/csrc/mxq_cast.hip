@@ -132,7 +132,7 @@ __device__ __forceinline__ float to_float(int32_t x) { return static_cast<float>
 template <typename SrcT, typename Rule, bool PRE>
 __device__ __forceinline__ void narrow_stream(const SrcT* __restrict__ in,
                                               uint8_t* __restrict__ out, size_t n, Rule rule,
-                                              float pre, bool rev = false) {
+                                              float pre, unsigned groups, bool rev = false) {
   typedef SrcT Vec4 __attribute__((ext_vector_type(4)));
   const size_t nquad = n >> 2;  // groups of 4 elements
   const Vec4* in4 = reinterpret_cast<const Vec4*>(in);
@@ -144,7 +144,7 @@ __device__ __forceinline__ void narrow_stream(const SrcT* __restrict__ in,
     out4 += nquad - 1;
   }
   const ptrdiff_t dir = rev ? -1 : 1;
-  const size_t stride = size_t(gridDim.x) * kThreads;
+  const size_t stride = size_t(groups) * kThreads;
   size_t q = size_t(blockIdx.x) * kThreads + threadIdx.x;
   // main loop: kUnroll segments, each `stride` quads apart
   for (; q + size_t(kUnroll - 1) * stride < nquad; q += size_t(kUnroll) * stride) {
@@ -194,8 +194,8 @@ __device__ __forceinline__ void narrow_stream(const SrcT* __restrict__ in,
 template <typename SrcT, typename Rule, bool PRE>
 __device__ __forceinline__ void narrow_scalar(const SrcT* __restrict__ in,
                                               uint8_t* __restrict__ out, size_t n, Rule rule,
-                                              float pre) {
-  const size_t stride = size_t(gridDim.x) * kThreads;
+                                              float pre, unsigned groups) {
+  const size_t stride = size_t(groups) * kThreads;
   for (size_t i = size_t(blockIdx.x) * kThreads + threadIdx.x; i < n; i += stride) {
     float f = to_float(in[i]);
     if (PRE) f = f * pre;
@@ -295,7 +295,7 @@ __global__ __launch_bounds__(kThreads) void quantize_kernel(const float* __restr
                                                             const float* __restrict__ dlo,
                                                             const float* __restrict__ dhi,
                                                             const uint32_t* __restrict__ parts,
-                                                            int nparts, int rev) {
+                                                            int nparts, int rev, unsigned groups) {
   if (dlo != nullptr) {
     lo = *dlo;
     hi = *dhi;
@@ -307,9 +307,9 @@ __global__ __launch_bounds__(kThreads) void quantize_kernel(const float* __restr
     rule.lo = lo;
     rule.s = static_cast<float>((255.0 - 0.0) / static_cast<double>(hi - lo));
     if (VEC)
-      narrow_stream<float, QuantU8, false>(in, out, n, rule, 0.f, rev != 0);
+      narrow_stream<float, QuantU8, false>(in, out, n, rule, 0.f, groups, rev != 0);
     else
-      narrow_scalar<float, QuantU8, false>(in, out, n, rule, 0.f);
+      narrow_scalar<float, QuantU8, false>(in, out, n, rule, 0.f, groups);
     if (blockIdx.x == 0 && threadIdx.x == 0) {
       *omin = lo;
       *omax = hi;
@@ -319,9 +319,9 @@ __global__ __launch_bounds__(kThreads) void quantize_kernel(const float* __restr
     QuantI8 rule;
     rule.s = 127.0f / r;
     if (VEC)
-      narrow_stream<float, QuantI8, false>(in, out, n, rule, 0.f, rev != 0);
+      narrow_stream<float, QuantI8, false>(in, out, n, rule, 0.f, groups, rev != 0);
     else
-      narrow_scalar<float, QuantI8, false>(in, out, n, rule, 0.f);
+      narrow_scalar<float, QuantI8, false>(in, out, n, rule, 0.f, groups);
     if (blockIdx.x == 0 && threadIdx.x == 0) {
       *omin = -r;
       *omax = r;
@@ -336,15 +336,15 @@ template <bool VEC>
 __global__ __launch_bounds__(kThreads) void quantize_asym_kernel(
     const float* __restrict__ in, uint8_t* __restrict__ out, float* __restrict__ oscale,
     float* __restrict__ oshift, size_t n, float lo, float hi, const uint32_t* __restrict__ parts,
-    int nparts, int rev) {
+    int nparts, int rev, unsigned groups) {
   if (parts != nullptr) load_range_f32(parts, nparts, lo, hi);
   QuantAsym rule;
   rule.scale = 255.0f / (hi - lo);
   rule.shift = 255.0f - hi * rule.scale;
   if (VEC)
-    narrow_stream<float, QuantAsym, false>(in, out, n, rule, 0.f, rev != 0);
+    narrow_stream<float, QuantAsym, false>(in, out, n, rule, 0.f, groups, rev != 0);
   else
-    narrow_scalar<float, QuantAsym, false>(in, out, n, rule, 0.f);
+    narrow_scalar<float, QuantAsym, false>(in, out, n, rule, 0.f, groups);
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     *oscale = rule.scale;
     *oshift = rule.shift;
@@ -358,8 +358,8 @@ __global__ __launch_bounds__(kThreads) void asym_bytes_kernel(const uint8_t* __r
                                                               uint8_t* __restrict__ out,
                                                               float* __restrict__ oscale,
                                                               float* __restrict__ oshift,
-                                                              size_t n, int vec) {
-  const size_t stride = size_t(gridDim.x) * kThreads;
+                                                              size_t n, int vec, unsigned groups) {
+  const size_t stride = size_t(groups) * kThreads;
   const size_t t0 = size_t(blockIdx.x) * kThreads + threadIdx.x;
   size_t done = 0;
   if (vec) {
@@ -389,7 +389,7 @@ __global__ __launch_bounds__(kThreads) void requantize_kernel(
     const int32_t* __restrict__ in, uint8_t* __restrict__ out, float* __restrict__ omin,
     float* __restrict__ omax, size_t n, const float* __restrict__ imin,
     const float* __restrict__ imax, float real_range, const uint32_t* __restrict__ parts,
-    int nparts, int rev) {
+    int nparts, int rev, unsigned groups) {
   const float in_scale = maxabs(*imin, *imax) / 2147483648.0f;
   if (parts != nullptr) {
     float lo, hi;
@@ -399,9 +399,9 @@ __global__ __launch_bounds__(kThreads) void requantize_kernel(
   QuantI8 rule;
   rule.s = 127.0f / maxabs(-real_range, real_range);
   if (VEC)
-    narrow_stream<int32_t, QuantI8, true>(in, out, n, rule, in_scale, rev != 0);
+    narrow_stream<int32_t, QuantI8, true>(in, out, n, rule, in_scale, groups, rev != 0);
   else
-    narrow_scalar<int32_t, QuantI8, true>(in, out, n, rule, in_scale);
+    narrow_scalar<int32_t, QuantI8, true>(in, out, n, rule, in_scale, groups);
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     *omin = -real_range;
     *omax = real_range;
@@ -486,7 +486,8 @@ template <bool UNSIGNED, bool VEC>
 __global__ __launch_bounds__(kThreads) void dequantize_kernel(const uint8_t* __restrict__ in,
                                                               float* __restrict__ out, size_t n,
                                                               const float* __restrict__ imin,
-                                                              const float* __restrict__ imax) {
+                                                              const float* __restrict__ imax,
+                                                              unsigned groups) {
   const float lo = *imin, hi = *imax;
   const float scale = UNSIGNED ? (hi - lo) / (255.0f - 0.0f) : maxabs(hi, lo) / 127.0f;
   auto conv = [&](uint32_t byte) -> float {
@@ -505,7 +506,7 @@ __global__ __launch_bounds__(kThreads) void dequantize_kernel(const uint8_t* __r
     y.w = conv(w >> 24);
     return y;
   };
-  const size_t stride = size_t(gridDim.x) * kThreads;
+  const size_t stride = size_t(groups) * kThreads;
   if (VEC) {
     const size_t nquad = n >> 2;
     const uint32_t* in4 = reinterpret_cast<const uint32_t*>(in);
@@ -515,7 +516,7 @@ __global__ __launch_bounds__(kThreads) void dequantize_kernel(const uint8_t* __r
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     for (size_t r = size_t(blockIdx.x) * kWaves + wave; r < runs;
-         r += size_t(gridDim.x) * kWaves) {
+         r += size_t(groups) * kWaves) {
       const uint32_t* src = in4 + r * kDeqRunQuads;
       uint32_t w[kPer];
 #pragma unroll
@@ -600,7 +601,8 @@ __device__ __forceinline__ void block_fold(T& mn, T& mx) {
 // NaN is detected through the largest |x| bit pattern (> 0x7f800000).
 template <bool VEC>
 __global__ __launch_bounds__(kThreads) void minmax_f32_kernel(const float* __restrict__ in,
-                                                              size_t n, uint32_t* parts) {
+                                                              size_t n, uint32_t* parts,
+                                                              unsigned groups) {
   float mn = INFINITY, mx = -INFINITY;
   uint32_t amax = 0;
   auto fold = [&](float x) {
@@ -609,7 +611,7 @@ __global__ __launch_bounds__(kThreads) void minmax_f32_kernel(const float* __res
     uint32_t a = __builtin_bit_cast(uint32_t, x) & 0x7fffffffu;
     amax = a > amax ? a : amax;
   };
-  const size_t stride = size_t(gridDim.x) * kThreads;
+  const size_t stride = size_t(groups) * kThreads;
   if (VEC) {
     const size_t nquad = n >> 2;
     const f4* in4 = reinterpret_cast<const f4*>(in);
@@ -656,13 +658,14 @@ __global__ __launch_bounds__(kThreads) void minmax_f32_kernel(const float* __res
 // int32 min / max of the whole tensor in one pass.
 template <bool VEC>
 __global__ __launch_bounds__(kThreads) void minmax_i32_kernel(const int32_t* __restrict__ in,
-                                                              size_t n, uint32_t* parts) {
+                                                              size_t n, uint32_t* parts,
+                                                              unsigned groups) {
   int mn = INT32_MAX, mx = INT32_MIN;
   auto fold = [&](int x) {
     mn = x < mn ? x : mn;
     mx = x > mx ? x : mx;
   };
-  const size_t stride = size_t(gridDim.x) * kThreads;
+  const size_t stride = size_t(groups) * kThreads;
   if (VEC) {
     const size_t nquad = n >> 2;
     const i4* in4 = reinterpret_cast<const i4*>(in);
@@ -709,8 +712,9 @@ __global__ __launch_bounds__(kThreads) void relu_i8_kernel(const int8_t* __restr
                                                            const float* __restrict__ imin,
                                                            const float* __restrict__ imax,
                                                            float* __restrict__ omin,
-                                                           float* __restrict__ omax, bool vec) {
-  const size_t stride = size_t(gridDim.x) * kThreads;
+                                                           float* __restrict__ omax, bool vec,
+                                                           unsigned groups) {
+  const size_t stride = size_t(groups) * kThreads;
   const size_t t0 = size_t(blockIdx.x) * kThreads + threadIdx.x;
   auto relu4 = [](uint32_t w) -> uint32_t {
     // a byte is negative iff its top bit is set: build a per-byte keep mask
@@ -812,13 +816,13 @@ template <int KIND, int PIECES>
 __global__ __launch_bounds__(kWholeThreads) void whole_cast_kernel(
     const void* __restrict__ in, uint8_t* __restrict__ out, float* __restrict__ omin,
     float* __restrict__ omax, int n, const float* __restrict__ imin,
-    const float* __restrict__ imax) {
+    const float* __restrict__ imax, int threads) {
   constexpr bool INT = KIND == kWholeRequant;
   typedef std::conditional_t<INT, int, float> T;
   typedef T Vec4 __attribute__((ext_vector_type(4)));
   const T* const src = static_cast<const T*>(in);
   const Vec4* const src4 = static_cast<const Vec4*>(in);
-  const int nquad = n >> 2, threads = blockDim.x, tid = threadIdx.x;
+  const int nquad = n >> 2, tid = threadIdx.x;
   float in_scale = 0.0f;
   if (INT) in_scale = maxabs(*imin, *imax) / 2147483648.0f;
   Vec4 x[PIECES];
@@ -994,7 +998,7 @@ void launch_whole(hipStream_t s, const void* in, uint8_t* out, float* omin, floa
   const int count = static_cast<int>(n);
 #define MXQ_W(PIECES)                                                                             \
   hipLaunchKernelGGL((whole_cast_kernel<KIND, PIECES>), dim3(1), dim3(threads), 0, s, in, out,   \
-                     omin, omax, count, imin, imax)
+                     omin, omax, count, imin, imax, static_cast<int>(threads))
   if (quads <= kWholeThreads)
     MXQ_W(1);
   else
@@ -1012,7 +1016,7 @@ void launch_quantize(hipStream_t s, const float* in, void* out, float* omin, flo
 #define MXQ_Q(U, V) \
   hipLaunchKernelGGL((quantize_kernel<U, V>), dim3(grid), dim3(kThreads), 0, s, in, o, omin, \
                      omax, n, lo, hi, dlo, dhi, parts, nparts,                           \
-                     parts != nullptr ? 1 : 0)
+                     parts != nullptr ? 1 : 0, static_cast<unsigned>(grid))
   if (out_type == MXQ_UINT8) {
     if (vec) MXQ_Q(true, true); else MXQ_Q(true, false);
   } else {
@@ -1062,10 +1066,10 @@ int mxq_quantize_v2(void* stream, const float* in, void* out, float* omin, float
     const int grid = reduce_grid(n);
     if (aligned16(in))
       hipLaunchKernelGGL((minmax_f32_kernel<true>), dim3(grid), dim3(kThreads), 0, s, in, n,
-                         parts);
+                         parts, static_cast<unsigned>(grid));
     else
       hipLaunchKernelGGL((minmax_f32_kernel<false>), dim3(grid), dim3(kThreads), 0, s, in, n,
-                         parts);
+                         parts, static_cast<unsigned>(grid));
     MXQ_LAUNCH_CHECK();
     launch_quantize(s, in, out, omin, omax, n, out_type, 0.f, 0.f, nullptr, nullptr, parts,
                     grid);
@@ -1112,9 +1116,11 @@ int mxq_minmax_f32(void* stream, const float* in, size_t n, float* out_min, floa
   uint32_t* parts = carve(workspace, workspace_bytes);
   const int grid = reduce_grid(n);
   if (aligned16(in))
-    hipLaunchKernelGGL((minmax_f32_kernel<true>), dim3(grid), dim3(kThreads), 0, s, in, n, parts);
+    hipLaunchKernelGGL((minmax_f32_kernel<true>), dim3(grid), dim3(kThreads), 0, s, in, n, parts,
+                       static_cast<unsigned>(grid));
   else
-    hipLaunchKernelGGL((minmax_f32_kernel<false>), dim3(grid), dim3(kThreads), 0, s, in, n, parts);
+    hipLaunchKernelGGL((minmax_f32_kernel<false>), dim3(grid), dim3(kThreads), 0, s, in, n, parts,
+                       static_cast<unsigned>(grid));
   hipLaunchKernelGGL(minmax_result_kernel, dim3(1), dim3(kThreads), 0, s, parts, grid, out_min,
                      out_max);
   MXQ_LAUNCH_CHECK();
@@ -1140,10 +1146,10 @@ int mxq_quantize_asym(void* stream, const void* in, int in_type, uint8_t* out, f
     const uint8_t* i8 = static_cast<const uint8_t*>(in);
     if (in_type == MXQ_INT8)
       hipLaunchKernelGGL((asym_bytes_kernel<true>), dim3(grid), dim3(kThreads), 0, s, i8, out,
-                         oscale, oshift, n, vec);
+                         oscale, oshift, n, vec, static_cast<unsigned>(grid));
     else
       hipLaunchKernelGGL((asym_bytes_kernel<false>), dim3(grid), dim3(kThreads), 0, s, i8, out,
-                         oscale, oshift, n, vec);
+                         oscale, oshift, n, vec, static_cast<unsigned>(grid));
     MXQ_LAUNCH_CHECK();
     return 0;
   }
@@ -1158,9 +1164,11 @@ int mxq_quantize_asym(void* stream, const void* in, int in_type, uint8_t* out, f
     }
     nparts = reduce_grid(n);
     if (aligned16(in))
-      hipLaunchKernelGGL((minmax_f32_kernel<true>), dim3(nparts), dim3(kThreads), 0, s, f, n, ws);
+      hipLaunchKernelGGL((minmax_f32_kernel<true>), dim3(nparts), dim3(kThreads), 0, s, f, n, ws,
+                         static_cast<unsigned>(nparts));
     else
-      hipLaunchKernelGGL((minmax_f32_kernel<false>), dim3(nparts), dim3(kThreads), 0, s, f, n, ws);
+      hipLaunchKernelGGL((minmax_f32_kernel<false>), dim3(nparts), dim3(kThreads), 0, s, f, n, ws,
+                         static_cast<unsigned>(nparts));
     MXQ_LAUNCH_CHECK();
     parts = ws;
   }
@@ -1169,11 +1177,11 @@ int mxq_quantize_asym(void* stream, const void* in, int in_type, uint8_t* out, f
   if (vec)
     hipLaunchKernelGGL((quantize_asym_kernel<true>), dim3(grid), dim3(kThreads), 0, s, f, out,
                        oscale, oshift, n, min_calib, max_calib, parts, nparts,
-                       parts != nullptr ? 1 : 0);
+                       parts != nullptr ? 1 : 0, static_cast<unsigned>(grid));
   else
     hipLaunchKernelGGL((quantize_asym_kernel<false>), dim3(grid), dim3(kThreads), 0, s, f, out,
                        oscale, oshift, n, min_calib, max_calib, parts, nparts,
-                       parts != nullptr ? 1 : 0);
+                       parts != nullptr ? 1 : 0, static_cast<unsigned>(grid));
   MXQ_LAUNCH_CHECK();
   MXQ_API_END();
 }
@@ -1230,21 +1238,21 @@ int mxq_requantize(void* stream, const int32_t* in, const float* imin, const flo
     nparts = reduce_grid(n);
     if (aligned16(in))
       hipLaunchKernelGGL((minmax_i32_kernel<true>), dim3(nparts), dim3(kThreads), 0, s, in, n,
-                         ws);
+                         ws, static_cast<unsigned>(nparts));
     else
       hipLaunchKernelGGL((minmax_i32_kernel<false>), dim3(nparts), dim3(kThreads), 0, s, in, n,
-                         ws);
+                         ws, static_cast<unsigned>(nparts));
     MXQ_LAUNCH_CHECK();
     parts = ws;
   }
   if (vec)
     hipLaunchKernelGGL((requantize_kernel<true>), dim3(grid), dim3(kThreads), 0, s, in, o, omin,
                        omax, n, imin, imax, real_range, parts, nparts,
-                       parts != nullptr ? 1 : 0);
+                       parts != nullptr ? 1 : 0, static_cast<unsigned>(grid));
   else
     hipLaunchKernelGGL((requantize_kernel<false>), dim3(grid), dim3(kThreads), 0, s, in, o,
                        omin, omax, n, imin, imax, real_range, parts, nparts,
-                       parts != nullptr ? 1 : 0);
+                       parts != nullptr ? 1 : 0, static_cast<unsigned>(grid));
   MXQ_LAUNCH_CHECK();
   MXQ_API_END();
 }
@@ -1267,7 +1275,8 @@ int mxq_quantized_relu(void* stream, const int8_t* in, const float* imin, const 
   }
   const int grid = stream_grid(n == 0 ? 1 : (vec ? (n + 15) / 16 : n), n);
   hipLaunchKernelGGL(relu_i8_kernel, dim3(grid), dim3(kThreads), 0,
-                     static_cast<hipStream_t>(stream), in, out, n, imin, imax, omin, omax, vec);
+                     static_cast<hipStream_t>(stream), in, out, n, imin, imax, omin, omax, vec,
+                     static_cast<unsigned>(grid));
   MXQ_LAUNCH_CHECK();
   MXQ_API_END();
 }
@@ -1299,7 +1308,7 @@ int mxq_dequantize(void* stream, const void* in, int in_type, const float* imin,
   }
 #define MXQ_D(U, V) \
   hipLaunchKernelGGL((dequantize_kernel<U, V>), dim3(grid), dim3(kThreads), 0, s, i8, out, n, \
-                     imin, imax)
+                     imin, imax, static_cast<unsigned>(grid))
   if (in_type == MXQ_UINT8) {
     if (vec) MXQ_D(true, true); else MXQ_D(true, false);
   } else {

@@ -54,6 +54,13 @@ struct Error : public std::runtime_error {
   }                                          \
   return 0;
 
+// A launch of a small kernel is host time, and that depends on its arguments: up to 112 bytes of them take
+// 2.65 us, 128 and more 3.1 to 3.4 (3000 launches in a row, in three of four processes; in the others 2.35
+// whatever there is).  A kernel that asks for gridDim or blockDim takes 72 bytes of hidden ones, so the
+// kernels that small operator calls end in are told how many work-groups they are (`groups`).  480
+// elements, without the Python call: dequantize 3.55 -> 2.9 us, quantize 3.5 -> 3.4, which is then what the
+// GPU takes.
+
 // Compute units of the calling thread's current device (cached per thread and device).
 int num_cus();
 

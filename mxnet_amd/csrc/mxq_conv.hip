@@ -1018,6 +1018,11 @@ struct GatherJob {
   unsigned magic_s, magic_k;
 };
 
+// work-groups a riding job gets: enough to be done when the carrier is
+__host__ __device__ inline unsigned job_blocks(const GatherJob& job) {
+  return job.blocks < 1024u ? job.blocks : 1024u;
+}
+
 GatherJob no_job() { return GatherJob{nullptr, nullptr, 0, 1, 16, 0, 0, 0, 0, 0, 0}; }
 
 // floor(n / d) for n < 2^31, magic = 2^31 / d + 1: the product is at most one too large.  (A division
@@ -1125,13 +1130,13 @@ __global__ __launch_bounds__(256) void transpose_kernel(const T* __restrict__ in
 // (a wave writes 1 KiB contiguous when the group covers all RP positions of its rows).
 __global__ __launch_bounds__(256) void transpose_i8_kernel(const uint8_t* __restrict__ in,
                                                            uint8_t* __restrict__ out, int R,
-                                                           int S, int RP, int B, GatherJob job) {
+                                                           int S, int RP, int B, GatherJob job,
+                                                           unsigned riders) {
   constexpr int kPitch = 17;  // dwords per transposed row: 64 bytes + 4 of padding
   __shared__ uint32_t tile[128 * kPitch];
   if (static_cast<int>(blockIdx.z) >= B) {   // the extra z slices carry the riding job
-    const unsigned per_z = gridDim.x * gridDim.y;
-    gather_job_run(job, (blockIdx.z - B) * per_z + blockIdx.y * gridDim.x + blockIdx.x,
-                        (gridDim.z - B) * per_z);
+    const unsigned wide = (S + 127) >> 7, high = (RP + 63) >> 6;
+    gather_job_run(job, ((blockIdx.z - B) * high + blockIdx.y) * wide + blockIdx.x, riders);
     return;
   }
   const size_t b = blockIdx.z;
@@ -1195,7 +1200,7 @@ __global__ __launch_bounds__(256) void transpose_i8_wide_kernel(const uint8_t* _
   constexpr int kPitch = 33;  // dwords per transposed row: 128 bytes + 4 of padding
   __shared__ uint32_t tile[128 * kPitch];
   if (blockIdx.x >= o.grid) {   // blocks past the tile grid carry the riding job
-    gather_job_run(job, blockIdx.x - o.grid, gridDim.x - o.grid);
+    gather_job_run(job, blockIdx.x - o.grid, job_blocks(job));
     return;
   }
   // the tile sequence runs along S first, then R, then the batch; with o.per_xcd != 0 the
@@ -1271,7 +1276,7 @@ __global__ __launch_bounds__(256) void gather_transpose_kernel(GatherJob first, 
   if (blockIdx.x < first.blocks)
     gather_job_run(first, blockIdx.x, first.blocks);
   else
-    gather_job_run(second, blockIdx.x - first.blocks, gridDim.x - first.blocks);
+    gather_job_run(second, blockIdx.x - first.blocks, job_blocks(second));
 }
 
 // A thin extent (at most 64 bytes, e.g. 7 x 7 planes) beside a long one that is a multiple of
@@ -1319,8 +1324,6 @@ __global__ __launch_bounds__(256) void s2d_nhwc_kernel(const int8_t* __restrict_
 // work-group ids over the XCDs is undone (64 x 256 x 56 x 56: 22.6 -> 21.1 us, 64 x 512 x 28 x 28:
 // 14.3 -> 12.1 us).  Rows on the marks lose 10 % that way (64 x 64 planes: 25.6 -> 28.9 us) and
 // the way back to planes gains nothing reliably, so those keep the plain order.
-// work-groups a riding job gets: enough to be done when the carrier is
-inline unsigned job_blocks(const GatherJob& job) { return job.blocks < 1024u ? job.blocks : 1024u; }
 
 template <int PIECE>
 void launch_wide(hipStream_t s, const void* in, void* out, int B, int R, int S, int RP,
@@ -1384,7 +1387,7 @@ void launch_transpose(hipStream_t s, const void* in, void* out, int B, int R, in
     dim3 grid128((S + 127) / 128, (RP + 63) / 64, fits ? B + extra_z : B);
     hipLaunchKernelGGL(transpose_i8_kernel, grid128, dim3(256), 0, s,
                        static_cast<const uint8_t*>(in), static_cast<uint8_t*>(out), R, S, RP, B,
-                       job);
+                       job, fits ? extra_z * per_z : 0u);
     MXQ_LAUNCH_CHECK();
     if (fits) carried();
     return;

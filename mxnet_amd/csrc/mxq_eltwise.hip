@@ -257,9 +257,9 @@ __global__ __launch_bounds__(kAddChunkThreads) void add32_chunk_kernel(AddArgs a
 }
 
 template <int OUT, bool LU, bool RU>
-__global__ __launch_bounds__(kThreads) void add_kernel(AddArgs a) {
+__global__ __launch_bounds__(kThreads) void add_kernel(AddArgs a, unsigned groups) {
   const AddRule<OUT, LU, RU> r = add_rule<OUT, LU, RU>(a);
-  const size_t stride = size_t(gridDim.x) * kThreads;
+  const size_t stride = size_t(groups) * kThreads;
   const size_t t0 = size_t(blockIdx.x) * kThreads + threadIdx.x;
   size_t done = 0;
   if (a.vec_ok) {
@@ -278,7 +278,7 @@ __global__ __launch_bounds__(kThreads) void add_kernel(AddArgs a) {
       const int lane = threadIdx.x & 63;
       const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
       for (size_t run = size_t(blockIdx.x) * kWaves + wave; run < runs;
-           run += size_t(gridDim.x) * kWaves) {
+           run += size_t(groups) * kWaves) {
         uint32_t x[kPer], y[kPer];
 #pragma unroll
         for (int j = 0; j < kPer; ++j) {
@@ -778,10 +778,10 @@ __device__ __forceinline__ int sbyte(uint32_t w, int k) {
 // fit int8 the reference's conversion is undefined; this takes the low byte of the
 // truncated int32, which is what the x86 build of the reference's loop produces.
 template <int OUT>
-__global__ __launch_bounds__(kThreads) void mul_kernel(MulArgs a) {
+__global__ __launch_bounds__(kThreads) void mul_kernel(MulArgs a, unsigned groups) {
   float omin = 0.f, omax = 0.f;
   const float scale = mul_scale<OUT>(a, omin, omax);
-  const size_t stride = size_t(gridDim.x) * kThreads;
+  const size_t stride = size_t(groups) * kThreads;
   const size_t t0 = size_t(blockIdx.x) * kThreads + threadIdx.x;
   size_t done = 0;
   if (a.vec_ok) {
@@ -1119,7 +1119,8 @@ int mxq_quantized_elemwise_add(void* stream, const void* lhs, int lhs_type, cons
   hipStream_t s = static_cast<hipStream_t>(stream);
   const bool lu = lhs_type == MXQ_UINT8, ru = rhs_type == MXQ_UINT8;
 #define MXQ_ADD(O, L, R) \
-  hipLaunchKernelGGL((add_kernel<O, L, R>), dim3(grid), dim3(kThreads), 0, s, a)
+  hipLaunchKernelGGL((add_kernel<O, L, R>), dim3(grid), dim3(kThreads), 0, s, a, \
+                     static_cast<unsigned>(grid))
   if (out_type == MXQ_INT32 && a.vec_ok && n >= kAddChunkMinElements) {
     const size_t per = size_t(kAddChunkPieces) * kAddChunkThreads;
     const size_t chunks = ((n >> 2) + per - 1) / per;
@@ -1304,11 +1305,14 @@ int mxq_quantized_elemwise_mul(void* stream, const int8_t* lhs, const int8_t* rh
   const int grid = grid_for(a.vec_ok ? (n + per_lane - 1) / per_lane : n);
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (out_type == MXQ_INT8)
-    hipLaunchKernelGGL((mul_kernel<MXQ_INT8>), dim3(grid), dim3(kThreads), 0, s, a);
+    hipLaunchKernelGGL((mul_kernel<MXQ_INT8>), dim3(grid), dim3(kThreads), 0, s, a,
+                       static_cast<unsigned>(grid));
   else if (out_type == MXQ_INT32)
-    hipLaunchKernelGGL((mul_kernel<MXQ_INT32>), dim3(grid), dim3(kThreads), 0, s, a);
+    hipLaunchKernelGGL((mul_kernel<MXQ_INT32>), dim3(grid), dim3(kThreads), 0, s, a,
+                       static_cast<unsigned>(grid));
   else
-    hipLaunchKernelGGL((mul_kernel<MXQ_FLOAT32>), dim3(grid), dim3(kThreads), 0, s, a);
+    hipLaunchKernelGGL((mul_kernel<MXQ_FLOAT32>), dim3(grid), dim3(kThreads), 0, s, a,
+                       static_cast<unsigned>(grid));
   MXQ_LAUNCH_CHECK();
   MXQ_API_END();
 }

@@ -81,11 +81,11 @@ struct EmbedArgs {
 };
 
 template <typename IT, bool VEC>
-__global__ __launch_bounds__(kThreads) void embedding_kernel(EmbedArgs a) {
+__global__ __launch_bounds__(kThreads) void embedding_kernel(EmbedArgs a, unsigned groups) {
   const int g = threadIdx.x & (a.group - 1);
   const size_t rows_per_block = kThreads >> a.shift;
   size_t row = size_t(blockIdx.x) * rows_per_block + (threadIdx.x >> a.shift);
-  const size_t step = size_t(gridDim.x) * rows_per_block;
+  const size_t step = size_t(groups) * rows_per_block;
   for (; row < a.n; row += step) {
     const int64_t j = clipped_index<IT>(a.idx, row, a.K);
     copy_row<VEC>(a.weight + static_cast<size_t>(j) * a.D, a.out + row * a.D, a.D, g, a.group);
@@ -100,9 +100,11 @@ template <typename IT>
 void launch_embedding(hipStream_t s, const EmbedArgs& a, bool vec) {
   const int grid = grid_for_rows(a.n, a.group);
   if (vec)
-    hipLaunchKernelGGL((embedding_kernel<IT, true>), dim3(grid), dim3(kThreads), 0, s, a);
+    hipLaunchKernelGGL((embedding_kernel<IT, true>), dim3(grid), dim3(kThreads), 0, s, a,
+                       static_cast<unsigned>(grid));
   else
-    hipLaunchKernelGGL((embedding_kernel<IT, false>), dim3(grid), dim3(kThreads), 0, s, a);
+    hipLaunchKernelGGL((embedding_kernel<IT, false>), dim3(grid), dim3(kThreads), 0, s, a,
+                       static_cast<unsigned>(grid));
   MXQ_LAUNCH_CHECK();
 }
 

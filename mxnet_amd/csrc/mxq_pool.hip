@@ -421,8 +421,8 @@ __global__ __launch_bounds__(256) void copy_bytes_kernel(const uint8_t* __restri
                                                          uint8_t* __restrict__ out, size_t n,
                                                          int vec_ok, const float* imin,
                                                          const float* imax, float* omin,
-                                                         float* omax) {
-  const size_t stride = static_cast<size_t>(gridDim.x) * 256;
+                                                         float* omax, unsigned groups) {
+  const size_t stride = static_cast<size_t>(groups) * 256;
   const size_t t = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x;
   if (t == 0 && omin != nullptr) {  // the range goes with the data (null: it is in place)
     *omin = *imin;
@@ -610,7 +610,8 @@ int mxq_quantized_flatten(void* stream, const void* in, const float* imin, const
     if (g < 1) g = 1;
     hipLaunchKernelGGL(copy_bytes_kernel, dim3(static_cast<unsigned>(g)), dim3(256), 0, s,
                        static_cast<const uint8_t*>(in), static_cast<uint8_t*>(out), n_bytes,
-                       vec_ok, imin, imax, range_moves ? omin : nullptr, omax);
+                       vec_ok, imin, imax, range_moves ? omin : nullptr, omax,
+                       static_cast<unsigned>(g));
     MXQ_LAUNCH_CHECK();
   } else if (range_moves) {
     hipLaunchKernelGGL(copy_range_kernel, dim3(1), dim3(1), 0, s, imin, imax, omin, omax);
