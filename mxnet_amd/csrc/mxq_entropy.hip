@@ -18,6 +18,7 @@
 
 #include <cmath>
 #include <cstdint>
+#include <type_traits>
 
 #include "../../include/mxq.h"
 #include "mxq_common.h"
@@ -38,6 +39,7 @@ struct Problem {
 };
 struct Info {     // of a candidate
   float first, last, p_take, q_take, p_sum, q_sum;
+  float q_least;  // the least level that is not 0, smoothed
   int state;      // 0: bounded, 1: infinite, 2: unknown (the host's chain reports what is wrong)
 };
 struct Args {
@@ -46,6 +48,7 @@ struct Args {
   int *counts, *filled, *seen;  // prefix sums of the integer parts, of them that are not 0, of bins
   float* head;                  // float sums from the first bin on
   int* exact;                   // per problem: every partial sum of counts is exact
+  float* least;                 // ... the least bin that is not 0, 0 where one is below
   float* levels;                // [candidate][level], not smoothed
   Info* info;
   double* bounds;               // [candidate][2]
@@ -88,15 +91,20 @@ __global__ __launch_bounds__(1024) void entropy_prefix_kernel(Args a) {
   __syncthreads();
   int s[3] = {0, 0, 0};
   bool whole = true;
+  float least = INFINITY;
   for (int j = from; j < to; ++j) {
     const int n = static_cast<int>(h[j]);
     whole = whole && static_cast<float>(n) == h[j];
+    if (h[j] != 0.0f) least = fminf(least, h[j]);
     s[0] += n;
     s[1] += n != 0;
     s[2] += h[j] != 0.0f;
   }
   for (int k = 0; k < 3; ++k) sums[k][tid] = s[k];
   whole = __syncthreads_and(whole) != 0;
+  __shared__ float leasts[16];
+  for (int d = 1; d < 64; d *= 2) least = fminf(least, __shfl_xor(least, d));
+  if ((tid & 63) == 0) leasts[tid >> 6] = least;
   for (int step = 1; step < 1024; step *= 2) {
     int add[3];
     for (int k = 0; k < 3; ++k) add[k] = tid >= step ? sums[k][tid - step] : 0;
@@ -119,7 +127,11 @@ __global__ __launch_bounds__(1024) void entropy_prefix_kernel(Args a) {
   }
   if (tid == 1023)
     for (int k = 0; k < 3; ++k) out[k][p.bins] = sums[k][1023];
-  if (tid == 0) a.exact[blockIdx.x] = exact;
+  if (tid == 0) {
+    a.exact[blockIdx.x] = exact;
+    for (int k = 1; k < 16; ++k) least = fminf(least, leasts[k]);
+    a.least[blockIdx.x] = fmaxf(least, 0.0f);
+  }
   if (exact) return;
   __syncthreads();
   if (tid == 0) chain(0.0f, h, 0, p.bins, [&](int j, float sum) { h[j] = sum; });
@@ -161,6 +173,7 @@ __global__ __launch_bounds__(256) void entropy_levels_kernel(Args a) {
     return lo < hi ? sum[hi] - sum[lo] : 0;
   };
   int p_entries = 0, q_entries = 0;
+  float least = INFINITY;
   float* const levels = a.levels + p.level + static_cast<long long>(s) * p.levels;
   for (int j = lane; j < p.levels; j += 64) {
     const int lo = j * merged, end = j + 1 == p.levels ? width : lo + merged;
@@ -176,11 +189,14 @@ __global__ __launch_bounds__(256) void entropy_levels_kernel(Args a) {
     const int to = end + start < stop - 1 ? end + start : stop - 1;
     const int entries = between(seen, from, to);
     p_entries += entries;
-    if (level != 0.0f)
+    if (level != 0.0f) {
       q_entries += entries + (j == 0 && first != 0.0f) + (j + 1 == p.levels && last != 0.0f);
+      least = fminf(least, level);
+    }
   }
   p_entries = wave_sum(p_entries) + (first != 0.0f) + (last != 0.0f);
   q_entries = wave_sum(q_entries);
+  for (int d = 1; d < 64; d *= 2) least = fminf(least, __shfl_xor(least, d));
   if (lane == 0) {
     Info r = {};
     r.first = first;
@@ -189,83 +205,263 @@ __global__ __launch_bounds__(256) void entropy_levels_kernel(Args a) {
       r.state = 1;
     else if (!smoothing(width, p_entries, &r.p_take))
       r.state = 2;
+    r.q_least = least - r.q_take;
     a.info[p.candidate + s] = r;
   }
 }
 
-// The two float chains of a candidate, a lane each, of two waves; the histogram in LDS.
-// Neighbouring candidates step through their bins side by side, one bin apart.  A chain's pace is
-// what one wave issues and what it waits for LDS: 195 us for the three histograms above (both
-// chains in one wave, 4 bins read at a time: 264).
+// The two float chains of a candidate, a lane each, of two waves; neighbouring candidates side by
+// side.  A chain's pace is what its wave issues, an instruction every four clocks, and what it waits for,
+// so a bin is an entry, one instruction that smooths it and the addition:
+//   the distribution itself: every lane at the same bin, which a scalar load brings.  Smoothed it is
+//     max(bin - take, kEps) where no bin but 0 is that small;
+//   the levels: every lane at the same place of its own levels, which are as long as each other's or a
+//     bin longer; in LDS a bin is infinity, or kEps where it is 0, and min(bin, level) is what it adds
+//     where no level is below kEps.
+// Where that does not hold a comparison and a selection smooth a bin, and each lane goes its own way
+// through its levels.
+// (For three histograms of 8001 bins: 165 us with both from LDS, smoothed by a comparison and a
+// selection, and a level asked for one level ahead; 80 us so, and 122 for 135 where lanes go their own
+// way, at 40 levels.)
+typedef const __attribute__((address_space(4))) float* ScalarFloats;
+constexpr int kMarksBehind = 64;  // what is read ahead past a lane's last bin
+
+__device__ __forceinline__ float smoothed(float v, float take) {
+  return v != 0.0f ? v - take : kEps;
+}
+// bins `from` ... `to` - 1 of the distribution, where the lane's own are from `mine` up to `last`
+template <bool ALL, bool LARGE>
+__device__ __forceinline__ void add_bins(float& sum, ScalarFloats h, int from, int to, int mine,
+                                         int last, float take) {
+  auto add = [&](int j, float v) {
+    const float next = sum + (LARGE ? fmaxf(v - take, kEps) : smoothed(v, take));
+    sum = ALL || (j >= mine && j < last) ? next : sum;
+  };
+  // two sets of bins take turns
+  constexpr int B = 16;
+  float x[B], y[B];
+  auto read = [&](float (&v)[B], int j) {
+#pragma unroll
+    for (int k = 0; k < B; ++k) v[k] = h[j + k];
+  };
+  int j = from;
+  if (j + 2 * B <= to) {
+    read(x, j);
+    for (; j + 2 * B <= to; j += 2 * B) {
+      read(y, j + B);
+#pragma unroll
+      for (int k = 0; k < B; ++k) add(j + k, x[k]);
+      if (j + 3 * B <= to) read(x, j + 2 * B);
+#pragma unroll
+      for (int k = 0; k < B; ++k) add(j + B + k, y[k]);
+    }
+  }
+  for (; j < to; j += 8) {
+    float z[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) z[k] = h[j + k < to ? j + k : to - 1];
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+      if (j + k < to) add(j + k, z[k]);
+  }
+}
+template <bool LARGE>
+__device__ __forceinline__ float p_chain(const Args& a, const Problem& p, const Info& r, int i) {
+  const float take = r.p_take;
+  float sum = smoothed(r.first, take);
+  const int start = p.zero - i, stop = p.zero + i + 1;
+  // the bins of lane 0, the widest, around those of the last lane, which are everyone's
+  const int widest = __builtin_amdgcn_readfirstlane(i);
+  const int narrowest = __builtin_amdgcn_readlane(i, 63);
+  const int begin = p.zero - widest + 1, end = p.zero + widest;
+  const int in = p.zero - narrowest + 1, out = p.zero + narrowest;
+  const ScalarFloats h = reinterpret_cast<ScalarFloats>(
+      reinterpret_cast<uintptr_t>(a.hist + p.hist));
+  add_bins<false, LARGE>(sum, h, begin, in, start + 1, stop - 1, take);
+  add_bins<true, LARGE>(sum, h, in, out, 0, 0, take);
+  add_bins<false, LARGE>(sum, h, out, end, start + 1, stop - 1, take);
+  return sum + smoothed(r.last, take);
+}
+// (positive floats are ordered as their bits are; fminf would have every mark made canonical first)
+__device__ __forceinline__ float marked(int mark, float q) {
+  const int level = __float_as_int(q);
+  return __int_as_float(mark < level ? mark : level);
+}
+// Levels of 16 * k + REST bins (LONG: k > 0) in every lane, a bin longer where `more`.  A level's bins are
+// added in a piece of REST, pieces of 16 and that bin, each read while what is before it is added.
+template <int REST, bool LONG>
+__device__ __forceinline__ float q_chain(const Problem& p, const Info& r, const float* levels,
+                                         const int* marks, int width, int each, bool more) {
+  const float take = r.q_take;
+  const int step = each + static_cast<int>(more), full = each / 16;
+  const int first = __float_as_int(r.first != 0.0f ? INFINITY : kEps);
+  const int* v = marks;
+  int x[16], y[16], last;
+#pragma unroll
+  for (int k = 0; k < REST; ++k) x[k] = k == 0 ? first : v[k];
+#pragma unroll
+  for (int k = 0; k < 16; ++k) y[k] = LONG ? (REST + k == 0 ? first : v[REST + k]) : 0;
+  last = v[each];
+  float sum = 0.0f;
+  constexpr int B = 8;  // levels on their way
+  float next[B];
+#pragma unroll
+  for (int k = 0; k < B; ++k) next[k] = levels[k < p.levels ? k : p.levels - 1];
+  for (int j = 0; j < p.levels - 1; j += B) {
+    float now[B];
+#pragma unroll
+    for (int k = 0; k < B; ++k) now[k] = smoothed(next[k], take);
+#pragma unroll
+    for (int k = 0; k < B; ++k)
+      next[k] = levels[j + B + k < p.levels ? j + B + k : p.levels - 1];
+    const int count = p.levels - 1 - j < B ? p.levels - 1 - j : B;
+    for (int l = 0; l < count; ++l) {
+      const float q = now[0];
+#pragma unroll
+      for (int k = 0; k + 1 < B; ++k) now[k] = now[k + 1];
+#pragma unroll
+      for (int k = 0; k < REST; ++k) sum += marked(x[k], q);
+      __builtin_amdgcn_sched_barrier(0);
+      const int* at = v + REST;
+      v += step;
+#pragma unroll
+      for (int k = 0; k < REST; ++k) x[k] = v[k];
+      if (LONG) {
+        int left = full;
+        do {
+          at = --left > 0 ? at + 16 : v + REST;
+#pragma unroll
+          for (int half = 0; half < 16; half += 8) {
+#pragma unroll
+            for (int k = half; k < half + 8; ++k) sum += marked(y[k], q);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int k = half; k < half + 8; ++k) y[k] = at[k];
+          }
+        } while (left > 0);
+      }
+      sum = more ? sum + marked(last, q) : sum;
+      last = v[each];
+    }
+  }
+  // the last level is as long as it is
+  const float q = smoothed(levels[p.levels - 1], take);
+  const int mine = width - 1 - (p.levels - 1) * step;
+  int longest = mine;
+  for (int d = 1; d < 64; d *= 2) {
+    const int other = __shfl_xor(longest, d);
+    longest = other > longest ? other : longest;
+  }
+  longest = __builtin_amdgcn_readfirstlane(longest);
+  for (int o = 0; o < longest; o += 16) {
+#pragma unroll
+    for (int k = 0; k < 16; ++k) y[k] = v[o + k < mine ? o + k : mine];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) sum = o + k < mine ? sum + marked(y[k], q) : sum;
+  }
+  return sum + (r.last != 0.0f ? q : kEps);
+}
+template <int REST = 0>
+__device__ __forceinline__ float q_chain_of(const Problem& p, const Info& r, const float* levels,
+                                            const int* marks, int width, int each, bool more) {
+  if constexpr (REST == 16) {
+    return 0.0f;
+  } else {
+    if (each % 16 != REST)
+      return q_chain_of<REST + 1>(p, r, levels, marks, width, each, more);
+    return each < 16 ? q_chain<REST, false>(p, r, levels, marks, width, each, more)
+                     : q_chain<REST, true>(p, r, levels, marks, width, each, more);
+  }
+}
 __global__ __launch_bounds__(128) void entropy_chains_kernel(Args a) {
-  extern __shared__ float hist[];
+  extern __shared__ int marks[];
   const Problem p = a.p[blockIdx.y];
   if (static_cast<int>(blockIdx.x) * 64 >= p.candidates) return;
-  for (int j = threadIdx.x; j < p.bins; j += 128) hist[j] = a.hist[p.hist + j];
+  for (int j = threadIdx.x; j < p.bins; j += 128 * 16) {
+    float v[16];
+#pragma unroll
+    for (int k = 0; k < 16; ++k)
+      v[k] = a.hist[p.hist + (j + 128 * k < p.bins ? j + 128 * k : p.bins - 1)];
+#pragma unroll
+    for (int k = 0; k < 16; ++k)
+      if (j + 128 * k < p.bins)
+        marks[j + 128 * k] = __float_as_int(v[k] != 0.0f ? INFINITY : kEps);
+  }
   __syncthreads();
-  // the widest first: a wave of them takes longest
-  const int s = p.candidates - 1 - (blockIdx.x * 64 + (threadIdx.x & 63));
-  if (s < 0) return;
+  // the widest first: a wave of them takes longest; lanes without a candidate take the narrowest
+  const int at = p.candidates - 1 - (blockIdx.x * 64 + (threadIdx.x & 63));
+  const int s = at < 0 ? 0 : at;
   Info* const info = a.info + p.candidate + s;
-  if (info->state != 0) return;
-  const int i = p.half + s, width = 2 * i + 1, merged = width / p.levels;
-  const float* const h = hist + p.zero - i;
-  const float first = info->first, last = info->last;
-  float sum = 0.0f;
+  const Info r = *info;
+  if (__all(r.state != 0)) return;
+  const int i = p.half + s, width = 2 * i + 1;
   if (threadIdx.x < 64) {
-    const float take = info->p_take;
-    auto add = [&](float v) { sum += v != 0.0f ? v - take : kEps; };
-    add(first);
-    int o = 1;
-    for (; o + 16 < width; o += 16) {
-      float v[16];
-#pragma unroll
-      for (int k = 0; k < 16; ++k) v[k] = h[o + k];
-#pragma unroll
-      for (int k = 0; k < 16; ++k) add(v[k]);
-    }
-    for (; o + 1 < width; ++o) add(h[o]);
-    add(last);
-    info->p_sum = sum;
+    const float sum = __all(r.state != 0 || a.least[blockIdx.y] - r.p_take >= kEps)
+                          ? p_chain<true>(a, p, r, i)
+                          : p_chain<false>(a, p, r, i);
+    if (r.state == 0 && at >= 0) info->p_sum = sum;
     return;
   }
-  const float take = info->q_take;
   const float* const levels = a.levels + p.level + static_cast<long long>(s) * p.levels;
-  float level = levels[0];
-  auto smoothed = [&](float v) { return v != 0.0f ? v - take : kEps; };
-  auto add = [&](float v, float q) { sum += v != 0.0f ? q : kEps; };
-  add(first, smoothed(level));
-  for (int j = 0; j < p.levels; ++j) {
-    const float q = smoothed(level);
-    const bool end = j + 1 == p.levels;
-    if (!end) level = levels[j + 1];
-    const int to = end ? width - 1 : (j + 1) * merged;
-    int o = j == 0 ? 1 : j * merged;
-    for (; o + 8 <= to; o += 8) {
-      float v[8];
+  const int merged = width / p.levels, each = __builtin_amdgcn_readlane(merged, 63);
+  const int most = __builtin_amdgcn_readfirstlane(merged);
+  const int* const mine = marks + p.zero - i;
+  float sum;
+  if (most <= each + 1 && __all(r.state != 0 || r.q_least >= kEps)) {
+    sum = q_chain_of(p, r, levels, mine, width, each, merged > each);
+  } else {
+    float level = levels[0], q = smoothed(level, r.q_take);
+    sum = r.first != 0.0f ? q : kEps;
+    for (int j = 0; j < p.levels; ++j) {
+      q = smoothed(level, r.q_take);
+      const bool end = j + 1 == p.levels;
+      if (!end) level = levels[j + 1];
+      const int to = end ? width - 1 : (j + 1) * merged;
+      int o = j == 0 ? 1 : j * merged;
+      for (; o + 8 <= to; o += 8) {
+        int v[8];
 #pragma unroll
-      for (int k = 0; k < 8; ++k) v[k] = h[o + k];
+        for (int k = 0; k < 8; ++k) v[k] = mine[o + k];
 #pragma unroll
-      for (int k = 0; k < 8; ++k) add(v[k], q);
+        for (int k = 0; k < 8; ++k) sum += v[k] == __float_as_int(kEps) ? kEps : q;
+      }
+      if (o < to) {  // fewer than 8, read in one go as well
+        int v[7];
+#pragma unroll
+        for (int k = 0; k < 7; ++k) v[k] = mine[o + k < to ? o + k : o];
+#pragma unroll
+        for (int k = 0; k < 7; ++k)
+          if (o + k < to) sum += v[k] == __float_as_int(kEps) ? kEps : q;
+      }
     }
-    if (o < to) {  // fewer than 8, read in one go as well
-      float v[7];
-#pragma unroll
-      for (int k = 0; k < 7; ++k) v[k] = h[o + k < to ? o + k : o];
-#pragma unroll
-      for (int k = 0; k < 7; ++k)
-        if (o + k < to) add(v[k], q);
-    }
-    if (end) add(last, q);
+    sum += r.last != 0.0f ? q : kEps;
   }
-  info->q_sum = sum;
+  if (r.state == 0 && at >= 0) info->q_sum = sum;
 }
 
-// The bounds, a wave per candidate, 4 bins in a row per lane.  With u = 2^-24, a term of the float
+// RN(a / b) from RN(1 / b): a quotient that is off by less than two last places and one correction
+// by its exact remainder (Markstein's division)
+__device__ __forceinline__ float quotient(float a, float b, float reciprocal) {
+  const float q = a * reciprocal;
+  return __builtin_fmaf(__builtin_fmaf(-q, b, a), reciprocal, q);
+}
+// The natural logarithm of a normal positive number: the instruction's, a last place of log2, times
+// ln 2 in two parts.
+__device__ __forceinline__ float natural_log(float x) {
+  constexpr float hi = 0x1.62e42ep-1f, lo = 0x1.efa39ep-25f;
+  const float y = __builtin_amdgcn_logf(x), z = y * hi;
+  return z + __builtin_fmaf(y, lo, __builtin_fmaf(y, hi, -z));
+}
+
+// The bounds, a wave per candidate, 16 bins in a row per lane.  With u = 2^-24, a term of the float
 // chain carries a logarithm of at most a last place (2u) and a product's rounding, a term here a
-// logarithm of at most two (4u) and an exact product; a sum of the chain carries u of itself.
-// (135 us for the three histograms above; with logarithms in double and a bin per lane 314.)
+// logarithm of at most two (4u; 2.71u is the most over 2^30 arguments) and an exact product; a sum of the
+// chain carries u of itself.  The factors add up to one, and a last place of theirs (should a quotient
+// miss it, which none of 2^30 did) to u.
+// (Vector instructions bound it: 136 us for the three histograms above with the compiler's divisions and
+// logarithm and 4 bins in a row, a scan of the wave for every 256 bins; 95 us so.)
 __global__ __launch_bounds__(256) void entropy_bounds_kernel(Args a) {
+  constexpr int B = 16;
   const Problem p = a.p[blockIdx.y];
   const int lane = threadIdx.x & 63, s = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (s >= p.candidates) return;
@@ -278,30 +474,40 @@ __global__ __launch_bounds__(256) void entropy_bounds_kernel(Args a) {
   const int i = p.half + s, start = p.zero - i, width = 2 * i + 1, merged = width / p.levels;
   const float* const h = a.hist + p.hist + start;
   const float* const levels = a.levels + p.level + static_cast<long long>(s) * p.levels;
+  const float p_once = 1.0f / r.p_sum, q_once = 1.0f / r.q_sum;
   const float p_zero = kEps / r.p_sum, q_zero = kEps / r.q_sum;
   const double zero_term = static_cast<double>(p_zero) * static_cast<double>(logf(p_zero / q_zero));
-  double sum = 0.0, magnitude = 0.0, sums = 0.0;  // the first the same in every lane
+  double sum = 0.0;  // the same in every lane
+  float magnitude = 0.0f, sums = 0.0f;
   bool bad = false;
-  for (int base = 0; base < width; base += 256) {
-    const int from = base + 4 * lane;
+  for (int base = 0; base < width; base += 64 * B) {
+    const int from = base + B * lane;
     int j = from / merged, rest = from - j * merged;
-    double t[4], all = 0.0;
+    float v[B];
+    double t[B];
+    if (from + B <= width) {
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
+      for (int k = 0; k < B; k += 4) __builtin_memcpy(v + k, h + from + k, 16);
+    } else {
+#pragma unroll
+      for (int k = 0; k < B; ++k) v[k] = from + k < width ? h[from + k] : 0.0f;
+    }
+    double all = 0.0;
+#pragma unroll
+    for (int k = 0; k < B; ++k) {
       const int o = from + k;
-      t[k] = 0.0;
-      if (o < width) {
-        const float v = o == 0 ? r.first : o + 1 == width ? r.last : h[o];
-        t[k] = zero_term;
-        if (v != 0.0f) {
-          const float level = levels[j < p.levels ? j : p.levels - 1];
-          const float q = level != 0.0f ? level - r.q_take : kEps;
-          const float pn = (v - r.p_take) / r.p_sum, qn = q / r.q_sum;
-          bad = bad || !(pn > 0.0f) || !(qn > 0.0f);
-          t[k] = static_cast<double>(pn) * static_cast<double>(logf(pn / qn));
-        }
-      }
-      magnitude += fabs(t[k]);
+      const float x = o == 0 ? r.first : o + 1 == width ? r.last : v[k];
+      const float level = levels[j < p.levels ? j : p.levels - 1];
+      const float q = level != 0.0f ? level - r.q_take : kEps;
+      const float pn = quotient(x - r.p_take, r.p_sum, p_once), qn = quotient(q, r.q_sum, q_once);
+      // pn / qn, but for the last place of 1 / qn
+      const float once = __builtin_amdgcn_rcpf(qn);
+      const double term =
+          static_cast<double>(pn) * static_cast<double>(natural_log(quotient(pn, qn, once)));
+      const bool filled = x != 0.0f && o < width;
+      bad = bad || (filled && (!(pn > 0.0f) || !(qn > 0.0f)));
+      t[k] = filled ? term : o < width ? zero_term : 0.0;
+      magnitude += fabsf(static_cast<float>(t[k]));
       all += t[k];
       if (++rest == merged) {
         ++j;
@@ -317,9 +523,9 @@ __global__ __launch_bounds__(256) void entropy_bounds_kernel(Args a) {
     sum = __shfl(before, 63);
     before -= all;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
+    for (int k = 0; k < B; ++k) {
       before += t[k];
-      sums += from + k < width ? fabs(before) : 0.0;
+      sums += from + k < width ? fabsf(static_cast<float>(before)) : 0.0f;
     }
   }
   for (int d = 1; d < 64; d *= 2) {
@@ -328,7 +534,8 @@ __global__ __launch_bounds__(256) void entropy_bounds_kernel(Args a) {
   }
   bad = __any(bad);
   const double u = 1.0 / 16777216.0;
-  const double margin = 1.05 * u * (8 * magnitude + sums) + 1e-12;
+  // (5 % for what is summed up in float here)
+  const double margin = 1.05 * u * (8.0 * magnitude + 1.0 + sums) + 1e-12;
   if (lane == 0) {
     const bool known = !bad && isfinite(sum) && isfinite(margin);
     out[0] = known ? sum - margin : -INFINITY;
@@ -341,7 +548,7 @@ size_t up256(size_t x) { return (x + 255) / 256 * 256; }
 // Where the parts of the workspace lie, and the problems' descriptions.
 struct Layout {
   size_t prefix = 0, candidates = 0, levels = 0, hist = 0;  // elements
-  size_t bytes = 0, at[7];
+  size_t bytes = 0, at[8];
   Layout(int count, const int* bins, const int* num_levels, Problem* out) {
     for (int i = 0; i < count; ++i) {
       MXQ_CHECK(bins[i] % 2 == 1 && bins[i] <= kMaxBins && num_levels[i] >= 3 &&
@@ -363,9 +570,9 @@ struct Layout {
       levels += static_cast<size_t>(p.candidates) * p.levels;
       if (out != nullptr) out[i] = p;
     }
-    const size_t parts[7] = {prefix * 4, prefix * 4, prefix * 4, prefix * 4, kMaxProblems * 4,
-                             levels * 4, candidates * sizeof(Info)};
-    for (int k = 0; k < 7; ++k) {
+    const size_t parts[8] = {prefix * 4, prefix * 4, prefix * 4, prefix * 4, kMaxProblems * 4,
+                             levels * 4, candidates * sizeof(Info), kMaxProblems * 4};
+    for (int k = 0; k < 8; ++k) {
       at[k] = bytes;
       bytes += up256(parts[k]);
     }
@@ -409,6 +616,7 @@ int mxq_entropy_bounds(void* stream, int count, const float* hist, const int* bi
   a.exact = reinterpret_cast<int*>(ws + l.at[4]);
   a.levels = reinterpret_cast<float*>(ws + l.at[5]);
   a.info = reinterpret_cast<Info*>(ws + l.at[6]);
+  a.least = reinterpret_cast<float*>(ws + l.at[7]);
   a.bounds = bounds;
   int most = 0, widest = 0;
   for (int i = 0; i < count; ++i) {
@@ -423,7 +631,7 @@ int mxq_entropy_bounds(void* stream, int count, const float* hist, const int* bi
   hipLaunchKernelGGL(entropy_levels_kernel, dim3((most + 3) / 4, n), dim3(256), 0, s, a);
   MXQ_LAUNCH_CHECK();
   hipLaunchKernelGGL(entropy_chains_kernel, dim3((most + 63) / 64, n), dim3(128),
-                     static_cast<size_t>(widest) * 4, s, a);
+                     static_cast<size_t>(widest + kMarksBehind) * 4, s, a);
   MXQ_LAUNCH_CHECK();
   hipLaunchKernelGGL(entropy_bounds_kernel, dim3((most + 3) / 4, n), dim3(256), 0, s, a);
   MXQ_LAUNCH_CHECK();
