@@ -1510,7 +1510,6 @@ ConvPlan plan_conv(const ConvGeometry& g, bool aligned, const GemmForce& force) 
         case Tile::kM128x2: plan.cfg = 24; break;
         case Tile::kM128K2: plan.cfg = 33; break;
         case Tile::kS64x2: plan.cfg = 25; break;
-        case Tile::kS64x4: plan.cfg = 15; break;  // not proposed for gathered operands
         case Tile::kS64K2: plan.cfg = 31; break;
         case Tile::kR128K2: plan.cfg = 37; break;
         case Tile::kQ128K2: plan.cfg = 38; break;

@@ -733,8 +733,9 @@ typedef PlaneCfg<64, 128, 128, 2, 2> PlaneP64k2;
 // 14 x 14 256 -> 1024 16.4 / 16.6 / 20.4).  Up to two small tiles a CU wait for memory at every step, and
 // what is under way is then what counts: 64 x 64 tiles, 1024 -> 512 / 2 at 14 x 14 11.0 / 9.8 / 8.6, and of
 // 8 images 1024 -> 256 at 14 x 14 12.3 / 8.2 / 7.4, 512 -> 128 at 28 x 28 8.9 / 6.9 / 6.8; of 4 images, four
-// to seven steps, 256 -> 1024 5.5 / 5.1 / 5.7, of 7 images 320 -> 640 at 20 x 20 6.4 / 5.9 / 6.0.  So is it for 128 x
-// 64 tiles, small ones as well, of any grid (256 -> 64 at 56 x 56 behind other layers 23.4 / 21.6 / 24.4).
+// to seven steps, 256 -> 1024 5.5 / 5.1 / 5.7, of 7 images 320 -> 640 at 20 x 20 6.4 / 5.9 / 6.0.  So is it
+// for 128 x 64 tiles, small ones as well, of any grid (256 -> 64 at 56 x 56 behind other layers 23.4 / 21.6 /
+// 24.4).
 template <class Cfg>
 int plane_stages(int steps, long long groups) {
   if (steps < 3) return 2;

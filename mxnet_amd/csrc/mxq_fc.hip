@@ -88,7 +88,6 @@ FcPlan plan_fc(int M, int N, int K, bool aligned, bool fused8, const GemmForce& 
         case Tile::kM128x2: plan.cfg = 43; break;
         case Tile::kM128K2: plan.cfg = 53; break;
         case Tile::kS64x2: plan.cfg = 44; break;
-        case Tile::kS64x4: plan.cfg = 24; break;
         case Tile::kS64K2: plan.cfg = 51; break;
         case Tile::kR128K2: plan.cfg = 57; break;
         case Tile::kQ128K2: plan.cfg = 58; break;

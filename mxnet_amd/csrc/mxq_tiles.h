@@ -30,7 +30,6 @@ enum class Tile {
   kM128x2,  // 128 x 128, 64-byte stages, 2-stage ring
   kM128K2,  // 128 x 128, 128-byte stages, 2-stage ring
   kS64x2,   // 64 x 64, 64-byte stages, 2-stage ring
-  kS64x4,   // 64 x 64, 64-byte stages, 4-stage ring, pinned pipeline
   kS64K2,   // 64 x 64, 128-byte stages, 2-stage ring
   kS64K4,   // 64 x 64, 256-byte stages, 2-stage ring
   kR128K2,  // 128 x 64, 128-byte stages, 2-stage ring
@@ -49,12 +48,13 @@ enum class Tile {
 //    CU, and one group's epilogue overlaps another's K loop.  A K step costs a barrier and
 //    a round of DMA latency whatever its size, so from K = 512 on the stages are 128 bytes
 //    deep (half as many steps: 10-20 % on every mid-size shape measured); below that the
-//    deeper stage would mostly be padding or leave too few steps to overlap;
+//    deeper stage would mostly be padding or leave too few steps to overlap.  Small tiles with
+//    little company on their CU take them from K = 256 on, and deeper ones (below);
 //  * 256 x 128 from 0.75 tiles per CU (fewer, larger stores per loaded byte), 128 x 128
-//    once it fills the chip, then 128 x 64 / 64 x 128, else 64 x 64 keeps every CU busy.
+//    once it fills the chip, then 64 x 128, else 64 x 64 keeps every CU busy.
 // `gather` says that the left operand is gathered pixel by pixel (convolution): the 64-row
 // tile then issues half as many gathers per wave and measures a few per cent ahead of the
-// 128-row one, which in turn is ahead for plain row-major operands.
+// 128-row one.
 inline Tile choose_tile(long M, long N, long K, long cus, bool gather = false,
                         int* splits = nullptr) {
   if (splits != nullptr) *splits = 1;
@@ -80,52 +80,69 @@ inline Tile choose_tile(long M, long N, long K, long cus, bool gather = false,
     if (sp > 4) sp = 4;
     if (sp >= 2) *splits = static_cast<int>(sp);
   };
+  // Tiles of 64 x 64 on 256-byte stages keep 64 KB under way on a CU, two of them at a time: up to two a
+  // CU every step waits for memory, and bytes under way are what counts (the operands from HBM, us, 64-
+  // and 128-byte stages and these: 1024 x 448 -> 1024 6.0 / 5.2 / 4.8, 2048 x 512 -> 1024 6.9 / 6.4 / 5.9,
+  // 16384 x 1024 -> 64 12.1 / 11.0 / 9.9, 32768 x 512 -> 64 10.6 / 10.0 / 9.2, 12351 x 3872 -> 64 49.4 / - /
+  // 25.1; 128 x 64 and these: 2048 x 512 -> 1024 7.1 / 5.9, 2048 x 2048 -> 1024 13.1 / 11.0).
+  // From the third tile a CU on they wait for LDS (3000 x 512 -> 1024, 752 tiles, 7.8 / 6.8 / 8.7, 65536 x
+  // 2048 -> 64, 1024 tiles, 56.7 / 53.0 / 51.3).
+  const long t64 = tiles(64, 64);
+  const bool two_a_cu = t64 <= 2 * cus;
   // Gathered operands (a convolution) of at most 64 columns: an address is made per 16 bytes of
   // pixels and stage, so 128-byte stages and tiles of 128 pixels pay from a reduction of 512 on
   // (140544 x 1584 -> 57 56.6 -> 38.4 us, 50176 x 2304 -> 32 24.9 -> 21.8, 50176 x 576 -> 48 14.6 ->
-  // 13.6, 57600 x 10400 -> 64 123.5 -> 70.5), with less than a tile per CU the tiles of 64 (25088 x 1152
-  // -> 64 14.4 -> 13.6, 12544 x 2304 -> 48 17.1 -> 15.8; 25088 x 576 -> 64 is level and stays), on
-  // 256-byte stages where they are many (27648 x 20384 -> 64 108.9 -> 72.7, 4732 x 5200 -> 36 28.5 ->
-  // 22.9).  Short ones take 256 pixels once there are two such tiles per CU and more (529803 x 144 -> 41
-  // 40.2 -> 31.2, 192000 x 432 -> 48 24.0 -> 18.7; 131072 x 432 -> 46, two exactly, is level).
+  // 13.6, 57600 x 10400 -> 64 123.5 -> 70.5), with less than a tile per CU the tiles of 64 (25088 x 576
+  // -> 64 8.0 -> 6.8, 25088 x 720 -> 40 9.1 -> 8.0), on 256-byte stages from four of them on (6272 x 2304
+  // -> 48 13.4 -> 10.5, 12544 x 2304 -> 64 13.8 -> 10.9, 25600 x 1152 -> 64 9.8 -> 9.7, 27648 x 20384 -> 64
+  // 108.9 -> 72.7).  Short ones take 256 pixels once there are two such tiles per CU and more (529803 x
+  // 144 -> 41 40.2 -> 31.2, 192000 x 432 -> 48 24.0 -> 18.7; 131072 x 432 -> 46, two exactly, is level).
   if (gather && N <= 64 && K >= 512) {
     if (tiles(128, 64) >= cus) return Tile::kR128K2;
-    if (K >= 4096) {
-      few_tile_splits();
-      return Tile::kS64K4;
-    }
-    if (K >= 1024) return Tile::kS64K2;
-  }
-  if (gather && N <= 64 && K < 512 && tiles(256, 64) > 2 * cus) return Tile::kW64x2;
-  if (N <= 64) {
+    if (K < 1024) return Tile::kS64K2;
     if (K >= 4096) few_tile_splits();
-    return (K >= 4096) ? Tile::kS64x4 : Tile::kS64x2;
+    return Tile::kS64K4;
+  }
+  if (gather && N <= 64)
+    return tiles(256, 64) > 2 * cus ? Tile::kW64x2 : Tile::kS64x2;
+  // Plain operands: 128-byte stages where there are more than two tiles a CU (65536 x 512 -> 64 17.9 ->
+  // 16.3, 200704 x 1024 -> 64 75.5 -> 71.8, 65536 x 256 -> 64 10.4 -> 9.7)
+  if (N <= 64) {
+    if (K < 256) return Tile::kS64x2;
+    if (K < 512 || !two_a_cu) return Tile::kS64K2;
+    if (K >= 4096) few_tile_splits();
+    return Tile::kS64K4;
   }
   if (4 * tiles(256, 128) >= 3 * cus) return (K >= 512) ? Tile::kW128K2 : Tile::kW128x2;
   if (tiles(128, 128) >= cus) return (K >= 256) ? Tile::kM128K2 : Tile::kM128x2;
-  if (K < 512) return Tile::kS64x2;
-  // half-size tiles while they still give every CU one: 12544 x 2304 -> 256 takes 14.1 us on
-  // 392 tiles of 64 x 128 against 17.6 us on 784 tiles of 64 x 64.  From K = 4096 on the
-  // 64 x 64 tile with 256-byte stages is the better of the two unless the half-size tiles
-  // still come two to a CU (512 x 4096 -> 4096: 18.3 us against 19.8 us on 256 tiles).
-  // Gathered operands whose 64 x 64 tiles are more than two per CU take them at any length: what
-  // does not fit at once waits for the 256-byte stages' LDS (12544 x 4608 -> 200 39.4 -> 32.0 us, 3600 x
-  // 8624 -> 528 62.9 -> 49.1; 2880 x 8624 -> 528, 405 tiles of 64 x 64, 39.1 and 49.0).
-  const long tq = tiles(64, 128), tr = tiles(128, 64);
-  const long need = (K >= 4096 && !(gather && tiles(64, 64) > 2 * cus)) ? 2 * cus : cus;
-  if (tq >= need || tr >= need) {
-    const bool q_fits = tq >= need && N % 128 == 0, r_fits = tr >= need;
-    if (q_fits && (gather || !r_fits)) return Tile::kQ128K2;
-    return r_fits ? Tile::kR128K2 : Tile::kQ128K2;
+  if (K < 256) return Tile::kS64x2;
+  if (two_a_cu) {
+    if (gather) {
+      // A stage that is partly padding is an address for each 16 bytes of it all the same: 256-byte
+      // stages from 768 on or where they are whole (3600 x 720 -> 128 7.0 -> 6.4, 3136 x 512 -> 512 7.3 ->
+      // 6.8, but 3136 x 576 -> 512 7.0 -> 7.5), 128-byte ones where no more than a fifth of them is not
+      // (3136 x 384 -> 192 6.1 -> 5.6, 6272 x 432 -> 256 7.0 -> 6.8, but 12544 x 288 -> 128 6.2 -> 6.3)
+      if (K < 768 && K % 256 != 0)
+        return K >= 512 || 5 * ((K + 127) / 128 * 128 - K) <= K ? Tile::kS64K2 : Tile::kS64x2;
+      if (K < 512) return Tile::kS64K2;
+    }
+    if (K >= 4096) few_tile_splits();
+    return Tile::kS64K4;
   }
-  // Fewer than two 64 x 64 tiles per CU are left: 256-byte stages once K leaves them four
-  // steps (3136 x 4608 -> 512: 15.8 us against 19.8 us).  With so few work-groups per CU a
-  // deeper stage is what keeps bytes in flight, which counts most when the operands come
-  // from HBM: inside the 19-layer ResNet stack (every layer reads operands last touched
-  // 300 us earlier) 3136 x 2048 -> 512 is 3.6 us and the strided 3136 x 1024 -> 512 2.4 us
-  // faster this way, and level with 128-byte stages when the operands are cache-warm.
-  if (K >= 4096) few_tile_splits();
-  return (K >= 1024) ? Tile::kS64K4 : Tile::kS64K2;
+  // More tiles than that: half-size ones.  12544 x 2304 -> 256 takes 14.1 us on 392 tiles of 64 x 128
+  // against 17.6 us on 784 tiles of 64 x 64, 12544 x 432 -> 256 8.0 against 8.8 (of a width between,
+  // 7840 x 432 -> 316, 8.9 against 8.4).
+  if (gather) {
+    if (K < (N % 128 == 0 ? 384 : 512)) return Tile::kS64x2;
+    return N % 128 == 0 ? Tile::kQ128K2 : Tile::kR128K2;
+  }
+  // Plain operands of a short reduction stay on the small ones (us, 64 x 64, 64 x 128, 128 x 64: 6272 x
+  // 512 -> 512 6.7 / 6.6 / 7.0, 25088 x 512 -> 128 9.5 / 9.8 / 9.8, 4096 x 512 -> 768 7.4 / 7.5 / 8.2,
+  // 1000 x 1024 -> 2500 9.2 / 9.3 / 9.3; 12544 x 2048 -> 256 20.4 / 20.7 / 22.2, 3000 x 2048 -> 1024 15.2 /
+  // 14.7 / 16.1, 3000 x 3072 -> 1024 20.1 / 19.4 / 19.7, 12544 x 4096 -> 256 38.5 / 37.6 / 39.8; of widths
+  // between, 8303 x 2608 -> 300 21.9 / 20.6 / 22.0, 5718 x 4400 -> 346 32.5 / 30.8 / 30.6, 28600 x 2352 ->
+  // 66 31.6 / 22.0 / 21.2).
+  return K < 2048 ? Tile::kS64K2 : Tile::kQ128K2;
 }
 
 }  // namespace mxq
