@@ -84,7 +84,7 @@ FcPlan plan_fc(int M, int N, int K, bool aligned, bool fused8, const GemmForce& 
       switch (choose_tile(M, N, K, cus, false, &auto_splits)) {
         case Tile::kL8: plan.cfg = glb_ok ? 12 : 31; break;
         case Tile::kW128x2: plan.cfg = 41; break;
-        case Tile::kW128K2: plan.cfg = 56; break;
+        case Tile::kW128K2: plan.cfg = 56; break;  // not proposed for plain operands
         case Tile::kM128x2: plan.cfg = 43; break;
         case Tile::kM128K2: plan.cfg = 53; break;
         case Tile::kS64x2: plan.cfg = 44; break;

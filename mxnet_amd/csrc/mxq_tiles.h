@@ -50,8 +50,9 @@ enum class Tile {
 //    deep (half as many steps: 10-20 % on every mid-size shape measured); below that the
 //    deeper stage would mostly be padding or leave too few steps to overlap.  Small tiles with
 //    little company on their CU take them from K = 256 on, and deeper ones (below);
-//  * 256 x 128 from 0.75 tiles per CU (fewer, larger stores per loaded byte), 128 x 128
-//    once it fills the chip, then 64 x 128, else 64 x 64 keeps every CU busy.
+//  * the 256 x 256 tile holds a CU alone, the 128 x 128 tile comes two to a CU and the 256 x 128
+//    tile on 64-byte stages and the 64 x 128 tile three: which of them is ahead is a matter of
+//    how many rounds the grid takes.  Once 128 x 128 tiles no longer fill the chip, 64 x 64 ones.
 // `gather` says that the left operand is gathered pixel by pixel (convolution): the 64-row
 // tile then issues half as many gathers per wave and measures a few per cent ahead of the
 // 128-row one.
@@ -65,7 +66,19 @@ inline Tile choose_tile(long M, long N, long K, long cus, bool gather = false,
   if (!gather && K >= 512 && N % 192 == 0 && tiles(256, 192) <= cus &&
       4 * tiles(256, 192) >= 3 * cus && tiles(256, 192) > tiles(256, 256))
     return Tile::kW192K2;
-  if (K > 256 && N > 128 && 16 * tiles(256, 256) >= 9 * cus) return Tile::kL8;
+  // A round of 256 x 256 tiles is as long as 1.6 of 128 x 128 tiles, two to a CU.  A few tiles into its
+  // second round it is behind (us, 256 x 256 and 128 x 128: 4352 x 1024 -> 4352, 289 tiles, 38.2 / 32.2, 17000 x
+  // 4096 -> 1024, 268, 110.8 / 91.4, 95000 x 1024 -> 256, 372, 57.6 / 50.6, but 5120 x 1024 -> 5120, 400, 39.4 /
+  // 42.7), and so it is where ragged edges leave 128 x 128 tiles a single one (20000 x 1024 -> 300, 158 and
+  // 471 tiles, 21.5 / 17.0; the convolutions 12544 x 512 -> 640 15.3 / 11.5, 19220 x 720 -> 300 18.2 / 14.0).
+  // Gathered operands come closer: from 1.35 rounds of the smaller tiles in one of these on the larger are
+  // ahead (38400 x 2592 -> 640, 1.46, 90.0 / 104.8, 36800 x 2592 -> 640, 1.41, 83.2 / 85.0, 41600 x 2592 -> 512, 1.27,
+  // 81.6 / 83.7, 68992 x 864 -> 256, 1.05, 38.2 / 33.0).
+  const long t256 = tiles(256, 256), t128 = tiles(128, 128);
+  const long rounds256 = (t256 + cus - 1) / cus, rounds128 = (t128 + 2 * cus - 1) / (2 * cus);
+  const bool larger = gather && rounds256 > 1 ? 10 * t128 >= 27 * cus * rounds256
+                                              : 5 * rounds128 >= 8 * rounds256;
+  if (K > 256 && N > 128 && 16 * t256 >= 9 * cus && larger) return Tile::kL8;
   // Split-K: an output of few 64 x 64 tiles under a very long reduction (a fully-connected
   // layer at small batch: 256 x 8192 -> 800, 64 x 25088 -> 4096) leaves most CUs idle and
   // each tile walks thousands of K bytes alone.  Up to four work-groups share a tile then
@@ -113,8 +126,25 @@ inline Tile choose_tile(long M, long N, long K, long cus, bool gather = false,
     if (K >= 4096) few_tile_splits();
     return Tile::kS64K4;
   }
-  if (4 * tiles(256, 128) >= 3 * cus) return (K >= 512) ? Tile::kW128K2 : Tile::kW128x2;
-  if (tiles(128, 128) >= cus) return (K >= 256) ? Tile::kM128K2 : Tile::kM128x2;
+  if (t128 >= cus) {
+    if (K < 256) return 4 * tiles(256, 128) >= 3 * cus ? Tile::kW128x2 : Tile::kM128x2;
+    // One round of 128 x 128 tiles, two to a CU (us, 256 x 128 on 128-byte stages, which hold a CU alone,
+    // and these: 16384 x 2048 -> 512 33.5 / 30.8, 28000 x 1024 -> 256 15.2 / 13.8, 2048 x 768 -> 4096 into int32
+    // 15.6 / 14.5; on 64-byte stages 8192 x 256 -> 1024 into int32 12.1 / 11.1).
+    // Very long reductions of gathered operands are ahead on the former (the convolutions 16000 x 6000 ->
+    // 413 62.1 / 69.3, 7840 x 7600 -> 787 64.2 / 69.1, but 12544 x 4608 -> 512 38.7 / 37.8).
+    if (t128 <= 2 * cus)
+      return gather && K >= 5120 && 4 * tiles(256, 128) >= 3 * cus ? Tile::kW128K2 : Tile::kM128K2;
+    // More of them: short reductions and gathered operands on 256 x 128 tiles, three to a CU, unless these
+    // are wide and long or very long (128-byte stages, 256 x 128, 128 x 128: the convolutions 200704 x 576 ->
+    // 128 45.5 / 33.8 / 41.0, 102400 x 864 -> 128 27.2 / 22.5 / 25.8, 72128 x 1296 -> 128 33.0 / 26.4 / 30.2, 102400 x
+    // 2304 -> 128 52.4 / 46.8 / 50.0, 94080 x 4608 -> 100 83.7 / 74.8 / 71.7, 41600 x 2592 -> 512 82.3 / 91.2 / 83.7;
+    // 131072 x 320 -> 128 25.5 / 20.5 / 24.6)
+    if (K < 512 || (gather && K < (N > 128 ? 1024 : 4096))) return Tile::kW128x2;
+    // else what comes out even of 64 x 128, three to a CU, and 128 x 128 (33000 x 512 -> 200, 516 of the
+    // latter, 14.4 / 18.3, 90000 x 2048 -> 128, 704, 69.1 / 72.3, 131072 x 1024 -> 128, 1024, 60.6 / 58.1)
+    return !gather && t128 <= 3 * cus ? Tile::kQ128K2 : Tile::kM128K2;
+  }
   if (K < 256) return Tile::kS64x2;
   if (two_a_cu) {
     if (gather) {
@@ -136,13 +166,13 @@ inline Tile choose_tile(long M, long N, long K, long cus, bool gather = false,
     if (K < (N % 128 == 0 ? 384 : 512)) return Tile::kS64x2;
     return N % 128 == 0 ? Tile::kQ128K2 : Tile::kR128K2;
   }
-  // Plain operands of a short reduction stay on the small ones (us, 64 x 64, 64 x 128, 128 x 64: 6272 x
-  // 512 -> 512 6.7 / 6.6 / 7.0, 25088 x 512 -> 128 9.5 / 9.8 / 9.8, 4096 x 512 -> 768 7.4 / 7.5 / 8.2,
-  // 1000 x 1024 -> 2500 9.2 / 9.3 / 9.3; 12544 x 2048 -> 256 20.4 / 20.7 / 22.2, 3000 x 2048 -> 1024 15.2 /
-  // 14.7 / 16.1, 3000 x 3072 -> 1024 20.1 / 19.4 / 19.7, 12544 x 4096 -> 256 38.5 / 37.6 / 39.8; of widths
-  // between, 8303 x 2608 -> 300 21.9 / 20.6 / 22.0, 5718 x 4400 -> 346 32.5 / 30.8 / 30.6, 28600 x 2352 ->
-  // 66 31.6 / 22.0 / 21.2).
-  return K < 2048 ? Tile::kS64K2 : Tile::kQ128K2;
+  // Plain operands of a short reduction stay on the small ones up to three of them a CU (us, 64 x 64, 128 x
+  // 64, 64 x 128: 4096 x 768 -> 768 from memory 9.3 / 10.0 / 9.4, again 7.6 / 8.1 / 8.2, 3000 x 512 -> 1024 6.8 / 7.2 / -
+  // and 6.6 / 7.2 / 7.1; a few more, 12544 x 1024 -> 256, 784, 12.3 / 13.2 / 12.6 and 10.4 / 9.4 / 9.6).  Long ones
+  // take 64 x 128 (12544 x 2048 -> 256 20.4 / 22.2 / 20.7 and 16.4 / 15.8 / 15.0, 3000 x 2048 -> 1024 15.2 / 16.1 / 14.7
+  // and 13.3 / 13.3 / 12.9, 8303 x 2608 -> 300 21.9 / 22.0 / 20.6).
+  if (K >= 2048) return Tile::kQ128K2;
+  return t64 <= 3 * cus && K < 1536 ? Tile::kS64K2 : Tile::kR128K2;
 }
 
 }  // namespace mxq

@@ -38,6 +38,17 @@ def test_fully_connected(capi, M, N, K):
          d.double() @ w.double().t().contiguous())
 
 
+# one round of 128 x 128 tiles (two to a CU of 256) and a little more, 256 x 256 tiles of one round, a
+# little and much more
+@pytest.mark.parametrize("M,N", [(8192, 1024), (8193, 1020), (33000, 200), (70000, 100), (131072, 72),
+                                 (4352, 4351), (5120, 5120)])
+@pytest.mark.parametrize("K", [256, 272, 512, 1040])
+def test_fully_connected_of_larger_tiles(capi, M, N, K):
+    d, w = operands((M, K), (N, K))
+    same(lambda **kw: capi.quantized_fc(d, w, None, *ranges(), **kw), (44, 1, 0),
+         d.double() @ w.double().t().contiguous())
+
+
 @pytest.mark.parametrize("M,K,N", [(8192, 8192, 33), (4096, 8208, 64), (700, 4112, 900)])
 def test_long_reductions_of_few_tiles(capi, M, K, N):
     d, w = operands((M, K), (N, K))
@@ -48,7 +59,9 @@ def test_long_reductions_of_few_tiles(capi, M, K, N):
 @pytest.mark.parametrize("n,h,c,o", [(16, 14, 32, 512), (16, 14, 48, 512), (16, 14, 64, 512),
                                      (16, 14, 80, 512), (16, 14, 96, 500), (16, 28, 48, 256),
                                      (16, 28, 48, 270), (16, 28, 64, 270), (32, 28, 64, 64),
-                                     (32, 28, 80, 40), (16, 25, 128, 64), (16, 25, 464, 40)])
+                                     (32, 28, 80, 40), (16, 25, 128, 64), (16, 25, 464, 40),
+                                     (23, 56, 32, 128), (23, 56, 32, 100), (28, 40, 64, 300),
+                                     (20, 31, 80, 300), (24, 40, 128, 276), (23, 40, 288, 640)])
 def test_convolution(capi, n, h, c, o):
     d, w = operands((n, h, h, c), (o, 3, 3, c))
     columns = torch.nn.functional.unfold(d.permute(0, 3, 1, 2).float(), 3, padding=1)  # n, c * 9, h * h
