@@ -247,6 +247,42 @@ __global__ __launch_bounds__(Cfg::kThreads, NS <= 2 ? Cfg::kMinWaves : 1) void c
   conv_dma<Cfg, NS, PIPE>(p, blockIdx.x);
 }
 
+// Tiles on eight waves (gemm_mainloop_sliced).
+template <class Cfg, int NS>
+__device__ __forceinline__ void conv_sliced(const ConvArgs& p, int block) {
+  typedef typename Cfg::Tile Tile;
+  __shared__ __attribute__((aligned(16))) v4i lds[NS * Cfg::STAGE_SLOTS];
+  const int tiles_m = (p.M + Cfg::BM - 1) / Cfg::BM, tiles_n = (p.O + Cfg::BN - 1) / Cfg::BN;
+  int tm, tn, tile = 0, z = 0;
+  if (__builtin_expect(p.sk.splits > 1, 0))
+    tile_coords_split(block, tiles_m, tiles_n, p.sk.splits, tm, tn, tile, z);
+  else
+    tile_coords(block, tiles_m, tiles_n, tm, tn);
+  const int m0 = tm * Cfg::BM, n0 = tn * Cfg::BN;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  EpiPreOf<kEpiPlain> pre;
+  auto prefetch = [&]() { pre = epi_prefetch<Tile>(p.epi, n0, p.O); };
+  const int kt_all = (p.K + Cfg::BK - 1) / Cfg::BK;
+  const int kt0 = z * p.sk.kt_per_split;
+  const int KT = (kt_all - kt0) < p.sk.kt_per_split ? (kt_all - kt0) : p.sk.kt_per_split;
+  ConvIssuer<Cfg, Cfg::A_CHUNKS> ai;
+  RowIssuerBuffer<Cfg, Cfg::B_CHUNKS> bi;
+  ai.init(p, m0, wave, lane, kt0 * Cfg::BK);
+  bi.init(p.weight, n0, p.O, p.K, wave, lane, kt0 * Cfg::BK);
+  if (block == 0 && threadIdx.x == 0) epilogue_ranges(p.epi);
+  v16i acc[1][1];
+  if (!gemm_mainloop_sliced<Cfg, NS>(acc, ai, bi, KT, lds, prefetch)) return;
+  if (__builtin_expect(p.sk.splits > 1, 0) && !splitk_gather<Tile>(acc, p.sk, tile, z)) return;
+  gemm_epilogue_lds<Tile, NS * Cfg::STAGE_SLOTS * 16>(acc, p.epi, pre, m0, n0, p.M, p.O,
+                                                      static_cast<size_t>(p.O), lds);
+}
+
+template <class Cfg, int NS>
+__global__ __launch_bounds__(Cfg::kThreads, 4) void conv_sliced_kernel(ConvArgs p) {
+  conv_sliced<Cfg, NS>(p, blockIdx.x);
+}
+
 // Two convolutions of the same images in one launch.
 struct ConvPair {
   ConvArgs a, b;
@@ -976,6 +1012,17 @@ void launch_dma(hipStream_t s, ConvArgs a, int splits, const Workspace& ws) {
   MXQ_LAUNCH_CHECK();
 }
 
+template <class Cfg, int NS>
+void launch_sliced(hipStream_t s, ConvArgs a, int splits, const Workspace& ws) {
+  const long tiles =
+      static_cast<long>((a.M + Cfg::BM - 1) / Cfg::BM) * ((a.O + Cfg::BN - 1) / Cfg::BN);
+  splitk_setup<typename Cfg::Tile>(s, a.sk, tiles, a.K, splits, ws.ptr, ws.bytes);
+  hipLaunchKernelGGL((conv_sliced_kernel<Cfg, NS>),
+                     dim3(static_cast<unsigned>(tiles * a.sk.splits)), dim3(Cfg::kThreads), 0, s,
+                     a);
+  MXQ_LAUNCH_CHECK();
+}
+
 template <class Cfg>
 void launch_pair(hipStream_t s, const ConvArgs& a, const ConvArgs& b) {
   auto tiles = [](const ConvArgs& x) {
@@ -1448,6 +1495,8 @@ bool conv_cfg_tile(int cfg, int& bm, int& bn) {
     case 15: case 25: case 31: case 32: case 39: bm = 64; bn = 64; return true;
     case 37: bm = 128; bn = 64; return true;
     case 38: bm = 64; bn = 128; return true;
+    case 40: bm = 64; bn = 64; return true;
+    case 41: bm = 128; bn = 32; return true;
     default: return false;
   }
 }
@@ -1497,13 +1546,15 @@ ConvPlan plan_conv(const ConvGeometry& g, bool aligned, const GemmForce& force) 
       return static_cast<long>((M + bm - 1) / bm) * ((O + bn - 1) / bn);
     };
     int auto_splits = 1;
-    if (dma_ok && few_tiles_wins(M, O, K, cus) && few_tiles_conv_ok(g.C, K, g.KH, g.KW)) {
+    const bool may_split = force.splits != 1;
+    if (dma_ok && few_tiles_wins(M, O, K, cus, may_split) &&
+        few_tiles_conv_ok(g.C, K, g.KH, g.KW)) {
       plan.cfg = 63;
       plan.splits = 1;
       return plan;
     }
     if (dma_ok) {
-      switch (choose_tile(M, O, K, cus, true, &auto_splits)) {
+      switch (choose_tile(M, O, K, cus, true, may_split ? &auto_splits : nullptr)) {
         case Tile::kL8: plan.cfg = 11; break;
         case Tile::kW128x2: plan.cfg = 22; break;
         case Tile::kW128K2: plan.cfg = 36; break;
@@ -1515,6 +1566,8 @@ ConvPlan plan_conv(const ConvGeometry& g, bool aligned, const GemmForce& force) 
         case Tile::kQ128K2: plan.cfg = 38; break;
         case Tile::kS64K4: plan.cfg = 39; break;
         case Tile::kW64x2: plan.cfg = 23; break;
+        case Tile::kS64S4: plan.cfg = 40; break;
+        case Tile::kN32S3: plan.cfg = 41; break;
         case Tile::kW192K2: plan.cfg = 11; break;  // not proposed for gathered operands
       }
     } else if (O > 128 && tiles(256, 256) >= cus) {
@@ -1737,6 +1790,8 @@ void conv_nhwc(void* stream, const int8_t* data, const int8_t* weight, const int
     case 37: launch_dma<CfgRK, 2, 0>(s, a, sp, ws); break;
     case 38: launch_dma<CfgQK, 2, 0>(s, a, sp, ws); break;
     case 39: launch_dma<CfgSK2, 2, 0>(s, a, sp, ws); break;
+    case 40: launch_sliced<SlicedCfg<64, 64, 256>, 4>(s, a, sp, ws); break;
+    case 41: launch_sliced<SlicedCfg<128, 32, 256>, 3>(s, a, sp, ws); break;
     case 22: launch_dma<CfgW128, 2, 0>(s, a, sp, ws); break;
     case 23: launch_dma<CfgW64, 2, 0>(s, a, sp, ws); break;
     case 24: launch_dma<CfgM, 2, 0>(s, a, sp, ws); break;

@@ -42,7 +42,7 @@ bool fc_cfg_tile(int cfg, int& bm, int& bn) {
     case 21: case 41: case 56: bm = 256; bn = 128; return true;
     case 22: case 42: bm = 256; bn = 64; return true;
     case 23: case 43: case 53: case 54: bm = 128; bn = 128; return true;
-    case 24: case 44: case 51: case 52: case 59: bm = 64; bn = 64; return true;
+    case 24: case 44: case 51: case 52: case 59: case 33: bm = 64; bn = 64; return true;
     case 57: bm = 128; bn = 64; return true;
     case 58: bm = 64; bn = 128; return true;
     case 60: bm = 256; bn = 192; return true;
@@ -73,7 +73,8 @@ FcPlan plan_fc(int M, int N, int K, bool aligned, bool fused8, const GemmForce& 
       return static_cast<long>((M + bm - 1) / bm) * ((N + bn - 1) / bn);
     };
     int auto_splits = 1;
-    if ((buf_ok && few_tiles_wins(M, N, K, cus)) ||
+    const bool may_split = force.splits != 1;
+    if ((buf_ok && few_tiles_wins(M, N, K, cus, may_split)) ||
         (!aligned && few_tiles_count(M, N) < (1L << 31) && static_cast<long long>(M) * K >= 16 &&
          static_cast<long long>(N) * K >= 16)) {
       plan.cfg = 71;
@@ -81,7 +82,7 @@ FcPlan plan_fc(int M, int N, int K, bool aligned, bool fused8, const GemmForce& 
       return plan;
     }
     if (buf_ok) {
-      switch (choose_tile(M, N, K, cus, false, &auto_splits)) {
+      switch (choose_tile(M, N, K, cus, false, may_split ? &auto_splits : nullptr)) {
         case Tile::kL8: plan.cfg = glb_ok ? 12 : 31; break;
         case Tile::kW128x2: plan.cfg = 41; break;
         case Tile::kW128K2: plan.cfg = 56; break;  // not proposed for plain operands
@@ -93,7 +94,9 @@ FcPlan plan_fc(int M, int N, int K, bool aligned, bool fused8, const GemmForce& 
         case Tile::kQ128K2: plan.cfg = 58; break;
         case Tile::kS64K4: plan.cfg = 59; break;
         case Tile::kW192K2: plan.cfg = 60; break;
+        case Tile::kS64S4: plan.cfg = 33; break;
         case Tile::kW64x2: plan.cfg = 42; break;  // not proposed for plain operands
+        case Tile::kN32S3: plan.cfg = 33; break;  // nor these
       }
     } else {
       if (tiles(256, 256) >= cus)

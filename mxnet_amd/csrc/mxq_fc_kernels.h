@@ -93,6 +93,37 @@ __global__ __launch_bounds__(Cfg::kThreads, NS <= 2 ? Cfg::kMinWaves : 1) void f
                                                            static_cast<size_t>(p.ldo), lds);
 }
 
+// A tile on eight waves (gemm_mainloop_sliced).
+template <class Cfg, int NS, int MODE>
+__global__ __launch_bounds__(Cfg::kThreads, 4) void fc_sliced_kernel(FcArgs p) {
+  typedef typename Cfg::Tile Tile;
+  __shared__ __attribute__((aligned(16))) v4i lds[NS * Cfg::STAGE_SLOTS];
+  const int tiles_m = (p.M + Cfg::BM - 1) / Cfg::BM, tiles_n = (p.N + Cfg::BN - 1) / Cfg::BN;
+  int tm, tn, tile = 0, z = 0;
+  if (__builtin_expect(p.sk.splits > 1, 0))
+    tile_coords_split(blockIdx.x, tiles_m, tiles_n, p.sk.splits, tm, tn, tile, z);
+  else
+    tile_coords(blockIdx.x, tiles_m, tiles_n, tm, tn);
+  const int m0 = tm * Cfg::BM, n0 = tn * Cfg::BN;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  EpiPreOf<MODE> pre;
+  auto prefetch = [&]() { pre = epi_prefetch<Tile, MODE>(p.epi, n0, p.N); };
+  const int kt_all = (p.K + Cfg::BK - 1) / Cfg::BK;
+  const int kt0 = z * p.sk.kt_per_split;
+  const int KT = (kt_all - kt0) < p.sk.kt_per_split ? (kt_all - kt0) : p.sk.kt_per_split;
+  RowIssuerBuffer<Cfg, Cfg::A_CHUNKS> ai;
+  RowIssuerBuffer<Cfg, Cfg::B_CHUNKS> bi;
+  ai.init(p.data, m0, p.M, p.K, wave, lane, kt0 * Cfg::BK);
+  bi.init(p.weight, n0, p.N, p.K, wave, lane, kt0 * Cfg::BK);
+  if (blockIdx.x == 0 && threadIdx.x == 0) epilogue_ranges<MODE>(p.epi);
+  v16i acc[1][1];
+  if (!gemm_mainloop_sliced<Cfg, NS>(acc, ai, bi, KT, lds, prefetch)) return;
+  if (__builtin_expect(p.sk.splits > 1, 0) && !splitk_gather<Tile>(acc, p.sk, tile, z)) return;
+  gemm_epilogue_lds<Tile, NS * Cfg::STAGE_SLOTS * 16, MODE>(acc, p.epi, pre, m0, n0, p.M, p.N,
+                                                            static_cast<size_t>(p.ldo), lds);
+}
+
 typedef GemmCfg<256, 256, 64, 2, 4> CfgL8;    // 8 waves, wave tile 128 x 64
 typedef GemmCfg<256, 256, 64, 2, 2> CfgL4;    // 4 waves, wave tile 128 x 128
 typedef GemmCfg<256, 128, 64, 4, 2> CfgW128;  // 8 waves, wave tile 64 x 64
@@ -330,6 +361,16 @@ void launch_dma(hipStream_t s, FcArgs a, int splits, const Workspace& ws) {
   MXQ_LAUNCH_CHECK();
 }
 
+template <class Cfg, int NS, int MODE>
+void launch_sliced(hipStream_t s, FcArgs a, int splits, const Workspace& ws) {
+  const long tiles = static_cast<long>((a.M + Cfg::BM - 1) / Cfg::BM) * ((a.N + Cfg::BN - 1) / Cfg::BN);
+  splitk_setup<typename Cfg::Tile>(s, a.sk, tiles, a.K, splits, ws.ptr, ws.bytes);
+  hipLaunchKernelGGL((fc_sliced_kernel<Cfg, NS, MODE>),
+                     dim3(static_cast<unsigned>(tiles * a.sk.splits)), dim3(Cfg::kThreads), 0, s,
+                     a);
+  MXQ_LAUNCH_CHECK();
+}
+
 template <class Cfg, int MODE>
 void launch_cfg(hipStream_t s, const FcArgs& a, bool aligned) {
   const int tiles = ((a.M + Cfg::BM - 1) / Cfg::BM) * ((a.N + Cfg::BN - 1) / Cfg::BN);
@@ -389,6 +430,7 @@ void fc_launch_mode(hipStream_t s, const FcArgs& a, const FcLaunch& how, const W
     case 58: launch_dma<CfgQK, 2, 0, true, MODE>(s, a, sp, ws); break;
     case 59: launch_dma<CfgSK2, 2, 0, true, MODE>(s, a, sp, ws); break;
     case 60: launch_dma<CfgW192K, 2, 0, true, MODE>(s, a, sp, ws); break;
+    case 33: launch_sliced<SlicedCfg<64, 64, 256>, 4, MODE>(s, a, sp, ws); break;
     case 31: launch_dma<CfgL8, 4, 2, true, MODE>(s, a, sp, ws); break;
     case 32: launch_dma<CfgL4, 4, 2, true, MODE>(s, a, sp, ws); break;
     default: MXQ_CHECK(false, "unknown fc tile configuration " << cfg);

@@ -819,6 +819,129 @@ __device__ __forceinline__ void gemm_mainloop_dma(v16i (&acc)[Cfg::MI][Cfg::NI],
   }
 }
 
+// ---- sliced main loop ----------------------------------------------------------------
+// A tile of 4096 outputs whose stages are shared by eight waves: a wave multiplies 64 rows with 32
+// columns (one half of the tile) over a quarter of each stage's reduction (its slice).
+//
+// For grids of no more than a tile a CU.  Four waves of 32 x 32 are one a SIMD there, and a wave's loads,
+// reads of LDS and products stand one behind the other: 0.70 us a step of 256 bytes, whether two, three or
+// four stages are under way.  Two waves a SIMD overlap them, and 64 x 32 outputs a wave take 48 KB of LDS
+// reads a step instead of 64; with four stages a step takes 0.48 us (14400 x 25088 -> 32, 225 tiles, 67.6 -> 50.6
+// us, 1024 x 4096 -> 1024, 256 tiles, 14.0 -> 11.4).  On two stages, one under way, it is level with the four
+// waves (66.4), on three 49.4.  What bounds it now is what a CU takes in: 32 KB in 0.48 us, as fast as two
+// four-wave work-groups do together, with which it is level where a grid has two tiles a CU.  The
+// partial sums of the slices pass through the ring once, 48 KB written and read, about 0.5 us.
+template <int BM_, int BN_, int BK_>
+struct SlicedCfg {
+  static constexpr int BM = BM_, BN = BN_, BK = BK_, CH = BK / 16, KS = BK / 32;
+  static constexpr bool kWide = BN == 64;  // halves are columns; else rows
+  // what the epilogue sees: the four waves that stay
+  typedef GemmCfg<BM, BN, BK, BM / 32, BN / 32> Tile;
+  static constexpr int kSlices = 4, kThreads = 512;
+  static constexpr int A_CHUNKS = BM * CH / kThreads, B_CHUNKS = BN * CH / kThreads;
+  static constexpr int STAGE_SLOTS = (BM + BN) * CH;
+  static_assert((BM == 64 && BN == 64) || (BM == 128 && BN == 32), "two halves of 64 x 32");
+  static_assert(KS % kSlices == 0 && (BN * CH) % kThreads == 0, "whole steps and loads a wave");
+};
+
+// Returns true in the four waves that hold the tile's sums, as those of SlicedCfg::Tile; the others
+// are to return (a barrier waits for the waves that are left).
+template <class Cfg, int NS, class AIssuer, class BIssuer, class AfterPrologue>
+__device__ __forceinline__ bool gemm_mainloop_sliced(v16i (&acc)[1][1], AIssuer& ai, BIssuer& bi,
+                                                     int KT, v4i* lds,
+                                                     AfterPrologue&& after_prologue) {
+  constexpr int CH = Cfg::CH, NW = Cfg::kThreads / 64;
+  constexpr int AI = Cfg::A_CHUNKS, BI = Cfg::B_CHUNKS, CPT = AI + BI;
+  constexpr int STEPS = Cfg::KS / Cfg::kSlices;
+  constexpr int STAGE_BYTES = Cfg::STAGE_SLOTS * 16;
+  // three quarters of the partial sums pass through the ring
+  static_assert(NS * STAGE_BYTES >= 12 * 4096, "ring too small for the partial sums");
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // Wave w < 4 is to end with the tile's rows 32 * (w / Tile::WN) and columns 32 * (w % Tile::WN): those
+  // of its half that its slice's number says
+  const int half = Cfg::kWide ? wave & 1 : wave >> 1 & 1;
+  const int slice = Cfg::kWide ? wave >> 1 : (wave >> 2) * 2 + (wave & 1);
+  const int row0 = Cfg::kWide ? 0 : 64 * half, col0 = Cfg::kWide ? 32 * half : 0;
+  const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds));
+  auto issue = [&](int stage) {
+    if (stage >= KT) return;
+    const uint32_t sb = lds0 + static_cast<uint32_t>(stage % NS) * STAGE_BYTES;
+#pragma unroll
+    for (int j = 0; j < AI; ++j) ai.issue(j, stage, sb + (j * NW + wave) * 1024);
+#pragma unroll
+    for (int j = 0; j < BI; ++j)
+      bi.issue(j, stage, sb + Cfg::BM * CH * 16 + (j * NW + wave) * 1024);
+    ai.stage_done();
+    bi.stage_done();
+  };
+  const int frow = lane & 31, fgrp = lane >> 5;
+  int fa0[STEPS], fb0[STEPS];  // rows 32 further are 32 * CH slots further (swz() does not see them)
+#pragma unroll
+  for (int i = 0; i < STEPS; ++i) {
+    const int chunk = ((slice + Cfg::kSlices * i) * 2 + fgrp) ^ swz<CH>(frow);
+    fa0[i] = (row0 + frow) * CH + chunk;
+    fb0[i] = (Cfg::BM + col0 + frow) * CH + chunk;
+  }
+  v16i part[2];
+#pragma unroll
+  for (int mi = 0; mi < 2; ++mi)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) part[mi][v] = 0;
+#pragma unroll
+  for (int s = 0; s < NS - 1; ++s) issue(s);
+  after_prologue();
+  if (NS == 2) __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0), as in gemm_mainloop_dma
+  for (int kt = 0; kt < KT; ++kt) {
+    const int last = kt + NS - 2 < KT - 1 ? kt + NS - 2 : KT - 1;
+    wait_ahead<CPT, NS - 2>(last - kt);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // ... and what it read of stage kt - 1
+    __builtin_amdgcn_s_barrier();
+    const v4i* st = lds + (kt % NS) * Cfg::STAGE_SLOTS;
+    v4i fa[STEPS][2], fb[STEPS];
+#pragma unroll
+    for (int i = 0; i < STEPS; ++i) {
+      fa[i][0] = st[fa0[i]];
+      fb[i] = st[fb0[i]];
+      fa[i][1] = st[fa0[i] + 32 * CH];
+    }
+    issue(kt + NS - 1);
+#pragma unroll
+    for (int i = 0; i < STEPS; ++i)
+#pragma unroll
+      for (int mi = 0; mi < 2; ++mi)
+        part[mi] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fb[i], fa[i][mi], part[mi], 0, 0, 0);
+  }
+  // The sums of rows 32 * mi of a half go to its wave of slice mi.
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();  // the ring's last stages are read
+  auto give = [&](int mi, int from) {
+    v4i* to = lds + ((mi * 2 + half) * 3 + from) * 256 + lane;
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      to[q * 64] = v4i{part[mi][4 * q], part[mi][4 * q + 1], part[mi][4 * q + 2],
+                       part[mi][4 * q + 3]};
+  };
+  if (slice != 0) give(0, slice - 1);
+  if (slice != 1) give(1, slice == 0 ? 0 : slice - 1);
+  __syncthreads();
+  if (slice >= 2) return false;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) acc[0][0][v] = slice == 0 ? part[0][v] : part[1][v];
+  const v4i* from = lds + (slice * 2 + half) * 3 * 256 + lane;
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const v4i w = from[k * 256 + q * 64];
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        acc[0][0][4 * q + i] = static_cast<int>(static_cast<uint32_t>(acc[0][0][4 * q + i]) +
+                                                static_cast<uint32_t>(w[i]));
+    }
+  return true;
+}
+
 // Stores one wave's accumulators.  m_base/n_base: origin of the wave tile.
 // What a kernel's epilogue is built for besides the int32 and int8 outputs.  Only the
 // fully-connected kernels are built with the extras, each as an instantiation of its own:

@@ -35,7 +35,9 @@ enum class Tile {
   kR128K2,  // 128 x 64, 128-byte stages, 2-stage ring
   kQ128K2,  // 64 x 128, 128-byte stages, 2-stage ring
   kW192K2,  // 256 x 192, 128-byte stages, 2-stage ring
-  kW64x2    // 256 x 64, 64-byte stages, 2-stage ring
+  kW64x2,   // 256 x 64, 64-byte stages, 2-stage ring
+  kS64S4,   // 64 x 64 on eight waves, 256-byte stages, 4-stage ring
+  kN32S3    // 128 x 32 on eight waves, 256-byte stages, 3-stage ring
 };
 
 // M x N outputs, reduction length K, `cus` compute units.  Distilled from sweeps over
@@ -79,20 +81,37 @@ inline Tile choose_tile(long M, long N, long K, long cus, bool gather = false,
   const bool larger = gather && rounds256 > 1 ? 10 * t128 >= 27 * cus * rounds256
                                               : 5 * rounds128 >= 8 * rounds256;
   if (K > 256 && N > 128 && 16 * t256 >= 9 * cus && larger) return Tile::kL8;
-  // Split-K: an output of few 64 x 64 tiles under a very long reduction (a fully-connected
-  // layer at small batch: 256 x 8192 -> 800, 64 x 25088 -> 4096) leaves most CUs idle and
-  // each tile walks thousands of K bytes alone.  Up to four work-groups share a tile then
-  // (18.3 -> 12.9 us and 63.5 -> 27 us on those two).  The price is a counter-clearing
-  // launch and the partial sums' round trip through memory (about 2 us plus 1 us per 4 MB),
-  // which is why shapes with more tiles or a shorter K are left alone: on the ResNet-50 and
-  // BERT layers every split measured slower than the unsplit kernel.
-  auto few_tile_splits = [&]() {
-    const long t = tiles(64, 64);
-    if (splits == nullptr || K < 8192 || 2 * t > cus) return;
-    long sp = cus / t;
-    if (sp > 4) sp = 4;
-    if (sp >= 2) *splits = static_cast<int>(sp);
+  // Up to one 64 x 64 tile a CU: eight waves share each of its stages, and three stages are under way.
+  // With a wave a SIMD the tile's loads, reads of LDS and products were issued one behind the other
+  // whatever the ring (us, four waves on two stages and eight on four: the convolutions 14400 x 25088 -> 32
+  // 67.6 / 50.6, 850 x 5328 -> 922 20.7 / 16.3, 9216 x 3168 -> 51 12.3 / 10.8, 1125 x 1600 -> 330 9.3 / 9.0, 3971 x 784 -> 193
+  // 9.3 / 9.4; plain operands 1024 x 4096 -> 1024 14.0 / 11.4, 100 x 7776 -> 6096 24.2 / 18.3, 78 x 1680 -> 7489 10.1 /
+  // 9.7, 252 x 1376 -> 1562 7.4 / 7.6).  From the second tile a CU on two of the small work-groups are level
+  // or ahead (7680 x 3200 -> 72, 386 tiles, 16.1 / 21.5).
+  // Split-K: where such tiles leave CUs idle and the reduction is long, as many work-groups share one as
+  // there are CUs for, each with 1536 of it and more.  The price is a counter-clearing launch and the partial
+  // sums' round trip through memory, about 3 us (unsplit and split: 1152 x 15680 -> 336 32.1 / 23.4 on two,
+  // 2401 x 3920 -> 147 14.1 / 13.9, 765 x 3728 -> 512 11.6 / 12.1; 54 tiles 1681 x 13328 -> 98 27.9 / 16.3 on four;
+  // 6 tiles 121 x 34800 -> 153 on 6, 8, 12 and 16 19.5 / 17.7 / 17.5 / 18.3).
+  // Gathered operands of at most 32 columns take 128 x 32 tiles, half as many of which are padding, with
+  // one of these a CU (20172 x 11760 -> 11, 158, 41.6 on four waves, 30.4 so, 28512 x 2000 -> 27 12.8 / 11.0) or
+  // split over a long reduction (64 x 64 tiles split and these: 14400 x 25088 -> 32 50.6 / 36.4, 7744 x 14112 -> 11
+  // 21.9 / 18.6, 12500 x 6272 -> 19 17.3 / 15.9, but 14336 x 4000 -> 18 12.5 / 13.6).
+  const long t64 = tiles(64, 64), t32 = tiles(128, 32);
+  auto shared = [&](long t, long slice) {
+    long sp = cus / t < K / slice ? cus / t : K / slice;
+    if (sp > 12) sp = 12;
+    if (splits != nullptr && sp >= 2) *splits = static_cast<int>(sp);
   };
+  if (gather && N <= 32 && t32 <= cus &&
+      (2 * t32 > cus ? K >= 1536 : K >= 6144 && splits != nullptr)) {
+    shared(t32, 2048);
+    return Tile::kN32S3;
+  }
+  if (t64 <= cus && K >= (gather ? 1024 : 1536)) {
+    if (K >= 4096) shared(t64, 1536);
+    return Tile::kS64S4;
+  }
   // Tiles of 64 x 64 on 256-byte stages keep 64 KB under way on a CU, two of them at a time: up to two a
   // CU every step waits for memory, and bytes under way are what counts (the operands from HBM, us, 64-
   // and 128-byte stages and these: 1024 x 448 -> 1024 6.0 / 5.2 / 4.8, 2048 x 512 -> 1024 6.9 / 6.4 / 5.9,
@@ -100,7 +119,6 @@ inline Tile choose_tile(long M, long N, long K, long cus, bool gather = false,
   // 25.1; 128 x 64 and these: 2048 x 512 -> 1024 7.1 / 5.9, 2048 x 2048 -> 1024 13.1 / 11.0).
   // From the third tile a CU on they wait for LDS (3000 x 512 -> 1024, 752 tiles, 7.8 / 6.8 / 8.7, 65536 x
   // 2048 -> 64, 1024 tiles, 56.7 / 53.0 / 51.3).
-  const long t64 = tiles(64, 64);
   const bool two_a_cu = t64 <= 2 * cus;
   // Gathered operands (a convolution) of at most 64 columns: an address is made per 16 bytes of
   // pixels and stage, so 128-byte stages and tiles of 128 pixels pay from a reduction of 512 on
@@ -112,9 +130,7 @@ inline Tile choose_tile(long M, long N, long K, long cus, bool gather = false,
   // 144 -> 41 40.2 -> 31.2, 192000 x 432 -> 48 24.0 -> 18.7; 131072 x 432 -> 46, two exactly, is level).
   if (gather && N <= 64 && K >= 512) {
     if (tiles(128, 64) >= cus) return Tile::kR128K2;
-    if (K < 1024) return Tile::kS64K2;
-    if (K >= 4096) few_tile_splits();
-    return Tile::kS64K4;
+    return K < 1024 ? Tile::kS64K2 : Tile::kS64K4;
   }
   if (gather && N <= 64)
     return tiles(256, 64) > 2 * cus ? Tile::kW64x2 : Tile::kS64x2;
@@ -123,7 +139,6 @@ inline Tile choose_tile(long M, long N, long K, long cus, bool gather = false,
   if (N <= 64) {
     if (K < 256) return Tile::kS64x2;
     if (K < 512 || !two_a_cu) return Tile::kS64K2;
-    if (K >= 4096) few_tile_splits();
     return Tile::kS64K4;
   }
   if (t128 >= cus) {
@@ -156,7 +171,6 @@ inline Tile choose_tile(long M, long N, long K, long cus, bool gather = false,
         return K >= 512 || 5 * ((K + 127) / 128 * 128 - K) <= K ? Tile::kS64K2 : Tile::kS64x2;
       if (K < 512) return Tile::kS64K2;
     }
-    if (K >= 4096) few_tile_splits();
     return Tile::kS64K4;
   }
   // More tiles than that: half-size ones.  12544 x 2304 -> 256 takes 14.1 us on 392 tiles of 64 x 128
