@@ -1000,6 +1000,7 @@ typedef GemmCfg<64, 64, 128, 2, 2> CfgSK;
 typedef GemmCfg<128, 64, 128, 2, 2> CfgRK;
 typedef GemmCfg<64, 128, 128, 2, 2> CfgQK;
 typedef GemmCfg<64, 64, 256, 2, 2> CfgSK2;
+typedef GemmCfg<128, 32, 128, 4, 1> CfgNK;
 
 template <class Cfg, int NS, int PIPE>
 void launch_dma(hipStream_t s, ConvArgs a, int splits, const Workspace& ws) {
@@ -1496,7 +1497,7 @@ bool conv_cfg_tile(int cfg, int& bm, int& bn) {
     case 37: bm = 128; bn = 64; return true;
     case 38: bm = 64; bn = 128; return true;
     case 40: bm = 64; bn = 64; return true;
-    case 41: bm = 128; bn = 32; return true;
+    case 41: case 42: bm = 128; bn = 32; return true;
     default: return false;
   }
 }
@@ -1568,6 +1569,7 @@ ConvPlan plan_conv(const ConvGeometry& g, bool aligned, const GemmForce& force) 
         case Tile::kW64x2: plan.cfg = 23; break;
         case Tile::kS64S4: plan.cfg = 40; break;
         case Tile::kN32S3: plan.cfg = 41; break;
+        case Tile::kN32K2: plan.cfg = 42; break;
         case Tile::kW192K2: plan.cfg = 11; break;  // not proposed for gathered operands
       }
     } else if (O > 128 && tiles(256, 256) >= cus) {
@@ -1792,6 +1794,7 @@ void conv_nhwc(void* stream, const int8_t* data, const int8_t* weight, const int
     case 39: launch_dma<CfgSK2, 2, 0>(s, a, sp, ws); break;
     case 40: launch_sliced<SlicedCfg<64, 64, 256>, 4>(s, a, sp, ws); break;
     case 41: launch_sliced<SlicedCfg<128, 32, 256>, 3>(s, a, sp, ws); break;
+    case 42: launch_dma<CfgNK, 2, 0>(s, a, sp, ws); break;
     case 22: launch_dma<CfgW128, 2, 0>(s, a, sp, ws); break;
     case 23: launch_dma<CfgW64, 2, 0>(s, a, sp, ws); break;
     case 24: launch_dma<CfgM, 2, 0>(s, a, sp, ws); break;

@@ -96,7 +96,7 @@ FcPlan plan_fc(int M, int N, int K, bool aligned, bool fused8, const GemmForce& 
         case Tile::kW192K2: plan.cfg = 60; break;
         case Tile::kS64S4: plan.cfg = 33; break;
         case Tile::kW64x2: plan.cfg = 42; break;  // not proposed for plain operands
-        case Tile::kN32S3: plan.cfg = 33; break;  // nor these
+        case Tile::kN32S3: case Tile::kN32K2: plan.cfg = 33; break;  // nor these
       }
     } else {
       if (tiles(256, 256) >= cus)

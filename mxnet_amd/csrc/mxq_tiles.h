@@ -37,7 +37,8 @@ enum class Tile {
   kW192K2,  // 256 x 192, 128-byte stages, 2-stage ring
   kW64x2,   // 256 x 64, 64-byte stages, 2-stage ring
   kS64S4,   // 64 x 64 on eight waves, 256-byte stages, 4-stage ring
-  kN32S3    // 128 x 32 on eight waves, 256-byte stages, 3-stage ring
+  kN32S3,   // 128 x 32 on eight waves, 256-byte stages, 3-stage ring
+  kN32K2    // 128 x 32, 128-byte stages, 2-stage ring
 };
 
 // M x N outputs, reduction length K, `cus` compute units.  Distilled from sweeps over
@@ -128,7 +129,14 @@ inline Tile choose_tile(long M, long N, long K, long cus, bool gather = false,
   // -> 48 13.4 -> 10.5, 12544 x 2304 -> 64 13.8 -> 10.9, 25600 x 1152 -> 64 9.8 -> 9.7, 27648 x 20384 -> 64
   // 108.9 -> 72.7).  Short ones take 256 pixels once there are two such tiles per CU and more (529803 x
   // 144 -> 41 40.2 -> 31.2, 192000 x 432 -> 48 24.0 -> 18.7; 131072 x 432 -> 46, two exactly, is level).
+  // At most 32 columns: 128 x 32 tiles, half of 64 columns would be padding (83824 x 2800 -> 19 33.1 -> 29.2,
+  // 169756 x 3920 -> 10 63.3 -> 52.2, 68600 x 784 -> 23 14.2 -> 12.2, 60543 x 576 -> 28 9.2 -> 8.1, 178475 x 432 -> 12
+  // 17.0 -> 15.2, 26244 x 784 -> 25 9.7 -> 9.1, but 163607 x 288 -> 16 11.0 -> 11.7).
+  if (gather && N <= 32 && K >= 432 && 4 * t32 >= 3 * cus) return Tile::kN32K2;
   if (gather && N <= 64 && K >= 512) {
+    // (tiles of 256 pixels, many of them, up to 800: 338724 x 576 -> 57 36.3 / 30.2, 159048 x 784 -> 45 24.4 /
+    // 21.0, 467046 x 784 -> 34 60.8 / 47.5; 205379 x 864 -> 42 27.9 / 31.9)
+    if (K < 800 && tiles(256, 64) > 2 * cus) return Tile::kW64x2;
     if (tiles(128, 64) >= cus) return Tile::kR128K2;
     return K < 1024 ? Tile::kS64K2 : Tile::kS64K4;
   }
@@ -143,6 +151,10 @@ inline Tile choose_tile(long M, long N, long K, long cus, bool gather = false,
   }
   if (t128 >= cus) {
     if (K < 256) return 4 * tiles(256, 128) >= 3 * cus ? Tile::kW128x2 : Tile::kM128x2;
+    // Gathered operands whose last 128 columns are half empty, on 128 x 64 tiles where these are one
+    // round as well (16940 x 11760 -> 136, 266 and 399 tiles, 96.4 / 67.9, 18496 x 23520 -> 190, 290 and 435, 163.7 /
+    // 135.0, 12138 x 2352 -> 269, 285 and 475, 24.2 / 20.6, but 14045 x 1872 -> 294, 330 and 550, 22.2 / 24.3)
+    if (gather && K >= 1024 && tiles(128, 64) < 2 * cus) return Tile::kR128K2;
     // One round of 128 x 128 tiles, two to a CU (us, 256 x 128 on 128-byte stages, which hold a CU alone,
     // and these: 16384 x 2048 -> 512 33.5 / 30.8, 28000 x 1024 -> 256 15.2 / 13.8, 2048 x 768 -> 4096 into int32
     // 15.6 / 14.5; on 64-byte stages 8192 x 256 -> 1024 into int32 12.1 / 11.1).

@@ -1,4 +1,4 @@
-"""Tiles on eight waves that share each stage's reduction: at the lines of the rules
+"""Tiles on eight waves that share each stage's reduction, and tiles of 32 columns: at the lines of the rules
 that choose them, at their edges and split over work-groups, against float64 products (exact for these lengths)
 and, requantized, against the smallest tile pinned."""
 import pytest
@@ -72,7 +72,7 @@ def test_convolution(capi, n, h, c, o, k, s):
     want = torch.cat([x.t().double() @ weight.t().contiguous() for x in columns]).reshape(n, oh, oh, o)
     same(lambda **kw: capi.quantized_conv_nhwc(d, w, None, *ranges(), pad=(k // 2, k // 2), stride=(s, s), **kw),
          (25, 1), want)
-    for cfg in (40, 41):
+    for cfg in (40, 41, 42):
         for splits in (1, 2, 5):
             got = capi.quantized_conv_nhwc(d, w, None, *ranges(), pad=(k // 2, k // 2), stride=(s, s),
                                            want_int32=True, force=(cfg, splits))["out32"]
