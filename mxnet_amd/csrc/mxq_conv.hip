@@ -271,7 +271,7 @@ __device__ __forceinline__ void conv_sliced(const ConvArgs& p, int block) {
   ai.init(p, m0, wave, lane, kt0 * Cfg::BK);
   bi.init(p.weight, n0, p.O, p.K, wave, lane, kt0 * Cfg::BK);
   if (block == 0 && threadIdx.x == 0) epilogue_ranges(p.epi);
-  v16i acc[1][1];
+  v16i acc[1][Cfg::NI];
   if (!gemm_mainloop_sliced<Cfg, NS>(acc, ai, bi, KT, lds, prefetch)) return;
   if (__builtin_expect(p.sk.splits > 1, 0) && !splitk_gather<Tile>(acc, p.sk, tile, z)) return;
   gemm_epilogue_lds<Tile, NS * Cfg::STAGE_SLOTS * 16>(acc, p.epi, pre, m0, n0, p.M, p.O,
@@ -279,7 +279,7 @@ __device__ __forceinline__ void conv_sliced(const ConvArgs& p, int block) {
 }
 
 template <class Cfg, int NS>
-__global__ __launch_bounds__(Cfg::kThreads, 4) void conv_sliced_kernel(ConvArgs p) {
+__global__ __launch_bounds__(Cfg::kThreads, 2) void conv_sliced_kernel(ConvArgs p) {
   conv_sliced<Cfg, NS>(p, blockIdx.x);
 }
 
@@ -1498,6 +1498,7 @@ bool conv_cfg_tile(int cfg, int& bm, int& bn) {
     case 38: bm = 64; bn = 128; return true;
     case 40: bm = 64; bn = 64; return true;
     case 41: case 42: bm = 128; bn = 32; return true;
+    case 43: bm = 128; bn = 128; return true;
     default: return false;
   }
 }
@@ -1570,6 +1571,7 @@ ConvPlan plan_conv(const ConvGeometry& g, bool aligned, const GemmForce& force) 
         case Tile::kS64S4: plan.cfg = 40; break;
         case Tile::kN32S3: plan.cfg = 41; break;
         case Tile::kN32K2: plan.cfg = 42; break;
+        case Tile::kM128S3: plan.cfg = 43; break;
         case Tile::kW192K2: plan.cfg = 11; break;  // not proposed for gathered operands
       }
     } else if (O > 128 && tiles(256, 256) >= cus) {
@@ -1794,6 +1796,7 @@ void conv_nhwc(void* stream, const int8_t* data, const int8_t* weight, const int
     case 39: launch_dma<CfgSK2, 2, 0>(s, a, sp, ws); break;
     case 40: launch_sliced<SlicedCfg<64, 64, 256>, 4>(s, a, sp, ws); break;
     case 41: launch_sliced<SlicedCfg<128, 32, 256>, 3>(s, a, sp, ws); break;
+    case 43: launch_sliced<SlicedCfg<128, 128, 128>, 3>(s, a, sp, ws); break;
     case 42: launch_dma<CfgNK, 2, 0>(s, a, sp, ws); break;
     case 22: launch_dma<CfgW128, 2, 0>(s, a, sp, ws); break;
     case 23: launch_dma<CfgW64, 2, 0>(s, a, sp, ws); break;

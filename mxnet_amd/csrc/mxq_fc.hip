@@ -41,7 +41,7 @@ bool fc_cfg_tile(int cfg, int& bm, int& bn) {
     case 11: case 12: case 14: case 16: case 31: case 32: case 55: bm = 256; bn = 256; return true;
     case 21: case 41: case 56: bm = 256; bn = 128; return true;
     case 22: case 42: bm = 256; bn = 64; return true;
-    case 23: case 43: case 53: case 54: bm = 128; bn = 128; return true;
+    case 23: case 43: case 53: case 54: case 34: bm = 128; bn = 128; return true;
     case 24: case 44: case 51: case 52: case 59: case 33: bm = 64; bn = 64; return true;
     case 57: bm = 128; bn = 64; return true;
     case 58: bm = 64; bn = 128; return true;
@@ -95,6 +95,7 @@ FcPlan plan_fc(int M, int N, int K, bool aligned, bool fused8, const GemmForce& 
         case Tile::kS64K4: plan.cfg = 59; break;
         case Tile::kW192K2: plan.cfg = 60; break;
         case Tile::kS64S4: plan.cfg = 33; break;
+        case Tile::kM128S3: plan.cfg = 34; break;
         case Tile::kW64x2: plan.cfg = 42; break;  // not proposed for plain operands
         case Tile::kN32S3: case Tile::kN32K2: plan.cfg = 33; break;  // nor these
       }

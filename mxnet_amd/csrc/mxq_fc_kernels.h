@@ -95,7 +95,7 @@ __global__ __launch_bounds__(Cfg::kThreads, NS <= 2 ? Cfg::kMinWaves : 1) void f
 
 // A tile on eight waves (gemm_mainloop_sliced).
 template <class Cfg, int NS, int MODE>
-__global__ __launch_bounds__(Cfg::kThreads, 4) void fc_sliced_kernel(FcArgs p) {
+__global__ __launch_bounds__(Cfg::kThreads, 2) void fc_sliced_kernel(FcArgs p) {
   typedef typename Cfg::Tile Tile;
   __shared__ __attribute__((aligned(16))) v4i lds[NS * Cfg::STAGE_SLOTS];
   const int tiles_m = (p.M + Cfg::BM - 1) / Cfg::BM, tiles_n = (p.N + Cfg::BN - 1) / Cfg::BN;
@@ -117,7 +117,7 @@ __global__ __launch_bounds__(Cfg::kThreads, 4) void fc_sliced_kernel(FcArgs p) {
   ai.init(p.data, m0, p.M, p.K, wave, lane, kt0 * Cfg::BK);
   bi.init(p.weight, n0, p.N, p.K, wave, lane, kt0 * Cfg::BK);
   if (blockIdx.x == 0 && threadIdx.x == 0) epilogue_ranges<MODE>(p.epi);
-  v16i acc[1][1];
+  v16i acc[1][Cfg::NI];
   if (!gemm_mainloop_sliced<Cfg, NS>(acc, ai, bi, KT, lds, prefetch)) return;
   if (__builtin_expect(p.sk.splits > 1, 0) && !splitk_gather<Tile>(acc, p.sk, tile, z)) return;
   gemm_epilogue_lds<Tile, NS * Cfg::STAGE_SLOTS * 16, MODE>(acc, p.epi, pre, m0, n0, p.M, p.N,
@@ -431,6 +431,7 @@ void fc_launch_mode(hipStream_t s, const FcArgs& a, const FcLaunch& how, const W
     case 59: launch_dma<CfgSK2, 2, 0, true, MODE>(s, a, sp, ws); break;
     case 60: launch_dma<CfgW192K, 2, 0, true, MODE>(s, a, sp, ws); break;
     case 33: launch_sliced<SlicedCfg<64, 64, 256>, 4, MODE>(s, a, sp, ws); break;
+    case 34: launch_sliced<SlicedCfg<128, 128, 128>, 3, MODE>(s, a, sp, ws); break;
     case 31: launch_dma<CfgL8, 4, 2, true, MODE>(s, a, sp, ws); break;
     case 32: launch_dma<CfgL4, 4, 2, true, MODE>(s, a, sp, ws); break;
     default: MXQ_CHECK(false, "unknown fc tile configuration " << cfg);

@@ -820,49 +820,67 @@ __device__ __forceinline__ void gemm_mainloop_dma(v16i (&acc)[Cfg::MI][Cfg::NI],
 }
 
 // ---- sliced main loop ----------------------------------------------------------------
-// A tile of 4096 outputs whose stages are shared by eight waves: a wave multiplies 64 rows with 32
-// columns (one half of the tile) over a quarter of each stage's reduction (its slice).
+// A tile whose stages are shared by eight waves: each multiplies 64 rows with 32 or 64 of the columns
+// over a quarter or a half of the stage's reduction (its slice).
 //
-// For grids of no more than a tile a CU.  Four waves of 32 x 32 are one a SIMD there, and a wave's loads,
-// reads of LDS and products stand one behind the other: 0.70 us a step of 256 bytes, whether two, three or
-// four stages are under way.  Two waves a SIMD overlap them, and 64 x 32 outputs a wave take 48 KB of LDS
-// reads a step instead of 64; with four stages a step takes 0.48 us (14400 x 25088 -> 32, 225 tiles, 67.6 -> 50.6
-// us, 1024 x 4096 -> 1024, 256 tiles, 14.0 -> 11.4).  On two stages, one under way, it is level with the four
-// waves (66.4), on three 49.4.  What bounds it now is what a CU takes in: 32 KB in 0.48 us, as fast as two
-// four-wave work-groups do together, with which it is level where a grid has two tiles a CU.  The
-// partial sums of the slices pass through the ring once, 48 KB written and read, about 0.5 us.
+// For grids of no more than a tile a CU.  Four waves are one a SIMD there, and a wave's loads, reads of LDS
+// and products stand one behind the other: with 64 x 64 tiles 0.70 us a step of 256 bytes, whether two,
+// three or four stages are under way.  Two waves a SIMD overlap them, and 64 x 32 outputs a wave take 48 KB
+// of LDS reads a step instead of 64; with four stages a step takes 0.48 us (14400 x 25088 -> 32, 225 tiles,
+// 67.6 -> 50.6 us, 1024 x 4096 -> 1024, 256 tiles, 14.0 -> 11.4).  On two stages, one under way, it is level
+// with the four waves (66.4), on three 49.4.  What bounds it now is what a CU takes in: 32 KB in 0.48 us, as
+// fast as two four-wave work-groups do together, with which it is level where a grid has two tiles a CU.
+// 128 x 128 tiles take in as much for four times the products, 0.65 us a step of 128 bytes on three stages or
+// four against 0.78 on four waves, and 0.75 on eight waves of 32 x 64 that share no stage (741 x 6352 ->
+// 4954, 234 tiles, 52.0 -> 40.1 us; 2646 x 23200 -> 931, 168, 136.3 -> 108.8).
+// The partial sums of the slices pass through the ring once, 48 or 64 KB written and read, about 0.5 us.
+//
+// A wave's parts of the tile: 64 rows from row0 on, 32 * NI columns from col0 on, over one of the slices.
 template <int BM_, int BN_, int BK_>
 struct SlicedCfg {
   static constexpr int BM = BM_, BN = BN_, BK = BK_, CH = BK / 16, KS = BK / 32;
-  static constexpr bool kWide = BN == 64;  // halves are columns; else rows
-  // what the epilogue sees: the four waves that stay
-  typedef GemmCfg<BM, BN, BK, BM / 32, BN / 32> Tile;
-  static constexpr int kSlices = 4, kThreads = 512;
+  static constexpr int kThreads = 512;
+  static constexpr int NI = BN == 128 ? 2 : 1;                // columns of a wave, in 32s
+  static constexpr int kPlaces = BM * BN / (64 * 32 * NI);    // waves that share out a slice
+  static constexpr int kSlices = 8 / kPlaces;
+  // what the epilogue sees: the waves of two slices, 32 rows each
+  typedef GemmCfg<BM, BN, BK, BM / 32, BN / (32 * NI)> Tile;
   static constexpr int A_CHUNKS = BM * CH / kThreads, B_CHUNKS = BN * CH / kThreads;
   static constexpr int STAGE_SLOTS = (BM + BN) * CH;
-  static_assert((BM == 64 && BN == 64) || (BM == 128 && BN == 32), "two halves of 64 x 32");
+  static_assert((BM == 64 && BN == 64) || (BM == 128 && (BN == 32 || BN == 128)), "places below");
   static_assert(KS % kSlices == 0 && (BN * CH) % kThreads == 0, "whole steps and loads a wave");
+  // Wave w of the tile's ends with the rows 32 * (w / Tile::WN): those of its 64 that its slice's number
+  // says, so the slice is part of w / Tile::WN.
+  __device__ __forceinline__ static int slice(int w) {
+    if (BN == 128) return w >> 1 & 1;
+    return BN == 64 ? w >> 1 : (w >> 2) * 2 + (w & 1);
+  }
+  __device__ __forceinline__ static int row0(int w) {
+    if (BN == 128) return 64 * (w >> 2);
+    return BN == 64 ? 0 : 64 * (w >> 1 & 1);
+  }
+  __device__ __forceinline__ static int col0(int w) {
+    if (BN == 128) return 64 * (w & 1);
+    return BN == 64 ? 32 * (w & 1) : 0;
+  }
 };
 
-// Returns true in the four waves that hold the tile's sums, as those of SlicedCfg::Tile; the others
-// are to return (a barrier waits for the waves that are left).
+// Returns true in the waves that hold the tile's sums, as those of SlicedCfg::Tile; the others are to
+// return (a barrier waits for the waves that are left).
 template <class Cfg, int NS, class AIssuer, class BIssuer, class AfterPrologue>
-__device__ __forceinline__ bool gemm_mainloop_sliced(v16i (&acc)[1][1], AIssuer& ai, BIssuer& bi,
-                                                     int KT, v4i* lds,
+__device__ __forceinline__ bool gemm_mainloop_sliced(v16i (&acc)[1][Cfg::NI], AIssuer& ai,
+                                                     BIssuer& bi, int KT, v4i* lds,
                                                      AfterPrologue&& after_prologue) {
-  constexpr int CH = Cfg::CH, NW = Cfg::kThreads / 64;
+  constexpr int CH = Cfg::CH, NW = Cfg::kThreads / 64, NI = Cfg::NI, SLICES = Cfg::kSlices;
   constexpr int AI = Cfg::A_CHUNKS, BI = Cfg::B_CHUNKS, CPT = AI + BI;
-  constexpr int STEPS = Cfg::KS / Cfg::kSlices;
+  constexpr int STEPS = Cfg::KS / SLICES;
   constexpr int STAGE_BYTES = Cfg::STAGE_SLOTS * 16;
-  // three quarters of the partial sums pass through the ring
-  static_assert(NS * STAGE_BYTES >= 12 * 4096, "ring too small for the partial sums");
+  // what the waves give away passes through the ring
+  static_assert(NS * STAGE_BYTES >= Cfg::kPlaces * 2 * (SLICES - 1) * NI * 4096,
+                "ring too small for the partial sums");
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  // Wave w < 4 is to end with the tile's rows 32 * (w / Tile::WN) and columns 32 * (w % Tile::WN): those
-  // of its half that its slice's number says
-  const int half = Cfg::kWide ? wave & 1 : wave >> 1 & 1;
-  const int slice = Cfg::kWide ? wave >> 1 : (wave >> 2) * 2 + (wave & 1);
-  const int row0 = Cfg::kWide ? 0 : 64 * half, col0 = Cfg::kWide ? 32 * half : 0;
+  const int slice = Cfg::slice(wave), row0 = Cfg::row0(wave), col0 = Cfg::col0(wave);
   const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds));
   auto issue = [&](int stage) {
     if (stage >= KT) return;
@@ -879,30 +897,32 @@ __device__ __forceinline__ bool gemm_mainloop_sliced(v16i (&acc)[1][1], AIssuer&
   int fa0[STEPS], fb0[STEPS];  // rows 32 further are 32 * CH slots further (swz() does not see them)
 #pragma unroll
   for (int i = 0; i < STEPS; ++i) {
-    const int chunk = ((slice + Cfg::kSlices * i) * 2 + fgrp) ^ swz<CH>(frow);
+    const int chunk = ((slice + SLICES * i) * 2 + fgrp) ^ swz<CH>(frow);
     fa0[i] = (row0 + frow) * CH + chunk;
     fb0[i] = (Cfg::BM + col0 + frow) * CH + chunk;
   }
-  v16i part[2];
+  v16i part[2][NI];
 #pragma unroll
   for (int mi = 0; mi < 2; ++mi)
 #pragma unroll
-    for (int v = 0; v < 16; ++v) part[mi][v] = 0;
+    for (int ni = 0; ni < NI; ++ni)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) part[mi][ni][v] = 0;
 #pragma unroll
   for (int s = 0; s < NS - 1; ++s) issue(s);
   after_prologue();
-  if (NS == 2) __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0), as in gemm_mainloop_dma
   for (int kt = 0; kt < KT; ++kt) {
     const int last = kt + NS - 2 < KT - 1 ? kt + NS - 2 : KT - 1;
     wait_ahead<CPT, NS - 2>(last - kt);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // ... and what it read of stage kt - 1
     __builtin_amdgcn_s_barrier();
     const v4i* st = lds + (kt % NS) * Cfg::STAGE_SLOTS;
-    v4i fa[STEPS][2], fb[STEPS];
+    v4i fa[STEPS][2], fb[STEPS][NI];
 #pragma unroll
     for (int i = 0; i < STEPS; ++i) {
       fa[i][0] = st[fa0[i]];
-      fb[i] = st[fb0[i]];
+#pragma unroll
+      for (int ni = 0; ni < NI; ++ni) fb[i][ni] = st[fb0[i] + ni * 32 * CH];
       fa[i][1] = st[fa0[i] + 32 * CH];
     }
     issue(kt + NS - 1);
@@ -910,35 +930,49 @@ __device__ __forceinline__ bool gemm_mainloop_sliced(v16i (&acc)[1][1], AIssuer&
     for (int i = 0; i < STEPS; ++i)
 #pragma unroll
       for (int mi = 0; mi < 2; ++mi)
-        part[mi] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fb[i], fa[i][mi], part[mi], 0, 0, 0);
+#pragma unroll
+        for (int ni = 0; ni < NI; ++ni)
+          part[mi][ni] =
+              __builtin_amdgcn_mfma_i32_32x32x32_i8(fb[i][ni], fa[i][mi], part[mi][ni], 0, 0, 0);
   }
-  // The sums of rows 32 * mi of a half go to its wave of slice mi.
+  // The sums of rows 32 * mi of a place go to its wave of slice mi.
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();  // the ring's last stages are read
-  auto give = [&](int mi, int from) {
-    v4i* to = lds + ((mi * 2 + half) * 3 + from) * 256 + lane;
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-      to[q * 64] = v4i{part[mi][4 * q], part[mi][4 * q + 1], part[mi][4 * q + 2],
-                       part[mi][4 * q + 3]};
+  const int place = row0 / 64 * (Cfg::BN / (32 * NI)) + col0 / (32 * NI);
+  auto given = [&](int mi, int from) {
+    return lds + ((place * 2 + mi) * (SLICES - 1) + from) * NI * 256 + lane;
   };
-  if (slice != 0) give(0, slice - 1);
-  if (slice != 1) give(1, slice == 0 ? 0 : slice - 1);
+#pragma unroll
+  for (int mi = 0; mi < 2; ++mi) {
+    if (slice == mi) continue;
+    v4i* to = given(mi, slice - (slice > mi));
+#pragma unroll
+    for (int ni = 0; ni < NI; ++ni)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        to[(ni * 4 + q) * 64] = v4i{part[mi][ni][4 * q], part[mi][ni][4 * q + 1],
+                                    part[mi][ni][4 * q + 2], part[mi][ni][4 * q + 3]};
+  }
   __syncthreads();
   if (slice >= 2) return false;
 #pragma unroll
-  for (int v = 0; v < 16; ++v) acc[0][0][v] = slice == 0 ? part[0][v] : part[1][v];
-  const v4i* from = lds + (slice * 2 + half) * 3 * 256 + lane;
+  for (int ni = 0; ni < NI; ++ni)
 #pragma unroll
-  for (int q = 0; q < 4; ++q)
+    for (int v = 0; v < 16; ++v) acc[0][ni][v] = slice == 0 ? part[0][ni][v] : part[1][ni][v];
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      const v4i w = from[k * 256 + q * 64];
+  for (int k = 0; k < SLICES - 1; ++k) {
+    const v4i* from = given(slice, k);
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        acc[0][0][4 * q + i] = static_cast<int>(static_cast<uint32_t>(acc[0][0][4 * q + i]) +
-                                                static_cast<uint32_t>(w[i]));
-    }
+    for (int ni = 0; ni < NI; ++ni)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const v4i w = from[(ni * 4 + q) * 64];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          acc[0][ni][4 * q + i] = static_cast<int>(static_cast<uint32_t>(acc[0][ni][4 * q + i]) +
+                                                   static_cast<uint32_t>(w[i]));
+      }
+  }
   return true;
 }
 

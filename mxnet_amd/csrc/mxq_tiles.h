@@ -38,7 +38,8 @@ enum class Tile {
   kW64x2,   // 256 x 64, 64-byte stages, 2-stage ring
   kS64S4,   // 64 x 64 on eight waves, 256-byte stages, 4-stage ring
   kN32S3,   // 128 x 32 on eight waves, 256-byte stages, 3-stage ring
-  kN32K2    // 128 x 32, 128-byte stages, 2-stage ring
+  kN32K2,   // 128 x 32, 128-byte stages, 2-stage ring
+  kM128S3   // 128 x 128 on eight waves, 128-byte stages, 3-stage ring
 };
 
 // M x N outputs, reduction length K, `cus` compute units.  Distilled from sweeps over
@@ -99,19 +100,18 @@ inline Tile choose_tile(long M, long N, long K, long cus, bool gather = false,
   // split over a long reduction (64 x 64 tiles split and these: 14400 x 25088 -> 32 50.6 / 36.4, 7744 x 14112 -> 11
   // 21.9 / 18.6, 12500 x 6272 -> 19 17.3 / 15.9, but 14336 x 4000 -> 18 12.5 / 13.6).
   const long t64 = tiles(64, 64), t32 = tiles(128, 32);
-  auto shared = [&](long t, long slice) {
-    long sp = cus / t < K / slice ? cus / t : K / slice;
-    if (sp > 12) sp = 12;
-    if (splits != nullptr && sp >= 2) *splits = static_cast<int>(sp);
+  auto sharing = [&](long t, long slice) {
+    if (splits == nullptr || t == 0) return 1L;  // (an output without elements has no tile)
+    const long sp = cus / t < K / slice ? cus / t : K / slice;
+    return sp > 12 ? 12L : sp < 1 ? 1L : sp;
+  };
+  auto shared = [&](long sp) {
+    if (splits != nullptr) *splits = static_cast<int>(sp);
   };
   if (gather && N <= 32 && t32 <= cus &&
       (2 * t32 > cus ? K >= 1536 : K >= 6144 && splits != nullptr)) {
-    shared(t32, 2048);
+    shared(sharing(t32, 2048));
     return Tile::kN32S3;
-  }
-  if (t64 <= cus && K >= (gather ? 1024 : 1536)) {
-    if (K >= 4096) shared(t64, 1536);
-    return Tile::kS64S4;
   }
   // Tiles of 64 x 64 on 256-byte stages keep 64 KB under way on a CU, two of them at a time: up to two a
   // CU every step waits for memory, and bytes under way are what counts (the operands from HBM, us, 64-
@@ -121,6 +121,25 @@ inline Tile choose_tile(long M, long N, long K, long cus, bool gather = false,
   // From the third tile a CU on they wait for LDS (3000 x 512 -> 1024, 752 tiles, 7.8 / 6.8 / 8.7, 65536 x
   // 2048 -> 64, 1024 tiles, 56.7 / 53.0 / 51.3).
   const bool two_a_cu = t64 <= 2 * cus;
+  // From half a 64 x 64 tile a CU to two of them and a long reduction: 128 x 128 tiles, which take in half
+  // as much an output, split over the chip where that leaves few CUs idle (64 x 64 tiles and these: 1176 x
+  // 45472 -> 653, 209 and 60 on four, 87.1 / 64.6, 720 x 15680 -> 799, 156 and 42 on six, 33.2 / 28.4, 475 x 29008 ->
+  // 1145, 144 and 36 on seven, 52.5 / 37.8, but 1568 x 12000 -> 493, 200 and 52 on four, 27.4 / 28.8, 6758 x 6176 ->
+  // 113, 212 and 53, 19.0 / 20.9; with a second of the former on a CU 9408 x 11600 -> 71, 294 and 74 on three,
+  // 39.8 / 30.9, 784 x 6272 -> 1387, 286 and 77, 25.6 / 22.7, 699 x 8160 -> 2429, 418 and 114 on two, 35.9 / 30.7, but
+  // 3831 x 6848 -> 404, 420 and 120 on two, 24.3 / 25.8, 1701 x 6768 -> 862, 378 and 98, 27.1 / 27.7).
+  if (N > 64 && 2 * t64 > cus && two_a_cu) {
+    const long sp = sharing(t128, 1536);
+    if (sp >= 2 && 5 * sp * t128 >= 4 * cus &&
+        K >= (t64 <= cus ? 14336 : sp >= 3 ? 6144 : 8000)) {
+      shared(sp);
+      return Tile::kM128S3;
+    }
+  }
+  if (t64 <= cus && K >= (gather ? 1024 : 1536)) {
+    if (K >= 4096) shared(sharing(t64, 1536));
+    return Tile::kS64S4;
+  }
   // Gathered operands (a convolution) of at most 64 columns: an address is made per 16 bytes of
   // pixels and stage, so 128-byte stages and tiles of 128 pixels pay from a reduction of 512 on
   // (140544 x 1584 -> 57 56.6 -> 38.4 us, 50176 x 2304 -> 32 24.9 -> 21.8, 50176 x 576 -> 48 14.6 ->
@@ -149,12 +168,21 @@ inline Tile choose_tile(long M, long N, long K, long cus, bool gather = false,
     if (K < 512 || !two_a_cu) return Tile::kS64K2;
     return Tile::kS64K4;
   }
+  // Up to one 128 x 128 tile a CU, more than two of 64 x 64: eight waves on it, two stages under way (us, 64 x
+  // 128, 128 x 64 or 128 x 128 tiles on four, whichever is first, and these: 741 x 6352 -> 4954, 234 tiles, 49.5 /
+  // 40.1, 321 x 7248 -> 5932, 141, 47.0 / 40.7, 7853 x 2832 -> 441, 248, 23.8 / 21.3, 2048 x 2048 -> 2048, 256, 14.8 /
+  // 14.5, 4096 x 3072 -> 768, 192, 18.2 / 17.7, 4096 x 768 -> 768 7.7 / 8.3; the convolutions 5203 x 22400 -> 701, 246,
+  // 111.7 / 106.6, 15884 x 3136 -> 204, 250, 22.5 / 22.2, 9522 x 2016 -> 380, 225, 17.9 / 17.2, but 12544 x 2304 -> 256, 196
+  // tiles without a ragged edge, 15.4 / 16.0).
+  if (!two_a_cu && t128 <= cus && K >= 1536 && !(gather && N % 128 == 0 && K < 4096))
+    return Tile::kM128S3;
   if (t128 >= cus) {
     if (K < 256) return 4 * tiles(256, 128) >= 3 * cus ? Tile::kW128x2 : Tile::kM128x2;
     // Gathered operands whose last 128 columns are half empty, on 128 x 64 tiles where these are one
     // round as well (16940 x 11760 -> 136, 266 and 399 tiles, 96.4 / 67.9, 18496 x 23520 -> 190, 290 and 435, 163.7 /
-    // 135.0, 12138 x 2352 -> 269, 285 and 475, 24.2 / 20.6, but 14045 x 1872 -> 294, 330 and 550, 22.2 / 24.3)
-    if (gather && K >= 1024 && tiles(128, 64) < 2 * cus) return Tile::kR128K2;
+    // 135.0, 12138 x 2352 -> 269, 285 and 475, 24.2 / 20.6, 18963 x 288 -> 134, 298 and 447, 9.9 / 8.6, but 14045 x 1872 -> 294, 330
+    // and 550, 22.2 / 24.3)
+    if (gather && tiles(128, 64) < 2 * cus) return Tile::kR128K2;
     // One round of 128 x 128 tiles, two to a CU (us, 256 x 128 on 128-byte stages, which hold a CU alone,
     // and these: 16384 x 2048 -> 512 33.5 / 30.8, 28000 x 1024 -> 256 15.2 / 13.8, 2048 x 768 -> 4096 into int32
     // 15.6 / 14.5; on 64-byte stages 8192 x 256 -> 1024 into int32 12.1 / 11.1).
@@ -194,11 +222,8 @@ inline Tile choose_tile(long M, long N, long K, long cus, bool gather = false,
   }
   // Plain operands of a short reduction stay on the small ones up to three of them a CU (us, 64 x 64, 128 x
   // 64, 64 x 128: 4096 x 768 -> 768 from memory 9.3 / 10.0 / 9.4, again 7.6 / 8.1 / 8.2, 3000 x 512 -> 1024 6.8 / 7.2 / -
-  // and 6.6 / 7.2 / 7.1; a few more, 12544 x 1024 -> 256, 784, 12.3 / 13.2 / 12.6 and 10.4 / 9.4 / 9.6).  Long ones
-  // take 64 x 128 (12544 x 2048 -> 256 20.4 / 22.2 / 20.7 and 16.4 / 15.8 / 15.0, 3000 x 2048 -> 1024 15.2 / 16.1 / 14.7
-  // and 13.3 / 13.3 / 12.9, 8303 x 2608 -> 300 21.9 / 22.0 / 20.6).
-  if (K >= 2048) return Tile::kQ128K2;
-  return t64 <= 3 * cus && K < 1536 ? Tile::kS64K2 : Tile::kR128K2;
+  // and 6.6 / 7.2 / 7.1; a few more, 12544 x 1024 -> 256, 784, 12.3 / 13.2 / 12.6 and 10.4 / 9.4 / 9.6).
+  return t64 <= 3 * cus ? Tile::kS64K2 : Tile::kR128K2;
 }
 
 }  // namespace mxq
