@@ -27,16 +27,13 @@ inline long few_tiles_count(long M, long N) { return ((M + 31) / 32) * ((N + 31)
 // Where the kernel is chosen for aligned operands: no more 32 x 32 tiles than CUs, so that the
 // 64 x 64 tiles of the other kernels would leave most of the chip idle (196 x 1024 -> 1024, 224
 // tiles: 4.1 us against 5.2; 784 x 1024 -> 512, 400 tiles: 5.7 against 5.2), and a reduction of
-// at least two blocks (at 64 bytes the tiled kernels are level or ahead).  A long reduction is ahead on
-// 64 x 64 tiles that several work-groups share, where the caller brought room for that: from 6144 on
-// with more than a quarter of the tiles (us, here and there: 592 x 6304 -> 281, 171 tiles, 14.6 / 12.4, 358 x
-// 8112 -> 200, 84, 13.9 / 12.0, but 186 x 5856 -> 515, 102, 11.4 / 12.4, 896 x 4352 -> 253, 224, 11.0 / 11.2), from
-// 24576 on with any (192 x 25088 -> 81 16.2 / 15.4, 48 x 33200 -> 686 23.5 / 18.2, but 272 x 23520 -> 81 16.1 /
-// 16.7, 512 x 17248 -> 106 13.8 / 15.5).
+// at least two blocks (at 64 bytes the tiled kernels are level or ahead).  From 8192 on
+// the tiled kernels split the reduction over work-groups and keep all but the smallest outputs, from 32768 on
+// these too where the caller brought room for it (us, here and there: 121 x 34800 -> 153 23.2 / 17.5, 48 x
+// 33200 -> 686 23.5 / 18.2, but 192 x 25088 -> 81 16.2 / 15.4, 512 x 17248 -> 106 13.8 / 15.5).
 inline bool few_tiles_wins(long M, long N, long K, long cus, bool may_split = false) {
-  const long most = may_split ? (K < 6144 ? cus : K < 24576 ? cus / 4 : 0)
-                              : (K < 8192 ? cus : cus / 4);
-  return K >= 256 && few_tiles_count(M, N) <= most;
+  return K >= 256 && few_tiles_count(M, N) <= (K < 8192 ? cus : cus / 4) &&
+         !(may_split && K >= 32768);
 }
 
 // Waves that share one tile's reduction of K bytes: 2, 4, 8 or 16 for a 32 x 32 tile, -4 or -8

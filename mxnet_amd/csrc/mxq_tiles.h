@@ -91,14 +91,16 @@ inline Tile choose_tile(long M, long N, long K, long cus, bool gather = false,
   // 9.7, 252 x 1376 -> 1562 7.4 / 7.6).  From the second tile a CU on two of the small work-groups are level
   // or ahead (7680 x 3200 -> 72, 386 tiles, 16.1 / 21.5).
   // Split-K: where such tiles leave CUs idle and the reduction is long, as many work-groups share one as
-  // there are CUs for, each with 1536 of it and more.  The price is a counter-clearing launch and the partial
-  // sums' round trip through memory, about 3 us (unsplit and split: 1152 x 15680 -> 336 32.1 / 23.4 on two,
-  // 2401 x 3920 -> 147 14.1 / 13.9, 765 x 3728 -> 512 11.6 / 12.1; 54 tiles 1681 x 13328 -> 98 27.9 / 16.3 on four;
-  // 6 tiles 121 x 34800 -> 153 on 6, 8, 12 and 16 19.5 / 17.7 / 17.5 / 18.3).
+  // there are CUs for, each with 1536 of it and more (unsplit and split: 1152 x 15680 -> 336 32.1 / 23.4 on two,
+  // 1681 x 13328 -> 98, 54 tiles, 27.9 / 16.3 on four, 121 x 34800 -> 153, 6 tiles, on 6, 8, 12 and 16 19.5 / 17.7 /
+  // 17.5 / 18.3).  The price is a counter-clearing launch and the partial sums' round trip through memory, about
+  // 3 us, and as much of the host's time, which is what a caller of small layers waits for: below 8192 it gains
+  // no more than that (2500 x 4704 -> 114, 80 tiles, 15.1 / 13.3, 5396 x 8144 -> 58, 85, 19.2 / 17.2, 765 x 3728 -> 512,
+  // 96, 11.6 / 12.1).
   // Gathered operands of at most 32 columns take 128 x 32 tiles, half as many of which are padding, with
   // one of these a CU (20172 x 11760 -> 11, 158, 41.6 on four waves, 30.4 so, 28512 x 2000 -> 27 12.8 / 11.0) or
   // split over a long reduction (64 x 64 tiles split and these: 14400 x 25088 -> 32 50.6 / 36.4, 7744 x 14112 -> 11
-  // 21.9 / 18.6, 12500 x 6272 -> 19 17.3 / 15.9, but 14336 x 4000 -> 18 12.5 / 13.6).
+  // 21.9 / 18.6, 15876 x 12400 -> 8 27.3 / 23.3; 14336 x 4000 -> 18 12.5 / 13.6).
   const long t64 = tiles(64, 64), t32 = tiles(128, 32);
   auto sharing = [&](long t, long slice) {
     if (splits == nullptr || t == 0) return 1L;  // (an output without elements has no tile)
@@ -109,7 +111,7 @@ inline Tile choose_tile(long M, long N, long K, long cus, bool gather = false,
     if (splits != nullptr) *splits = static_cast<int>(sp);
   };
   if (gather && N <= 32 && t32 <= cus &&
-      (2 * t32 > cus ? K >= 1536 : K >= 6144 && splits != nullptr)) {
+      (2 * t32 > cus ? K >= 1536 : K >= 8192 && splits != nullptr)) {
     shared(sharing(t32, 2048));
     return Tile::kN32S3;
   }
@@ -137,7 +139,7 @@ inline Tile choose_tile(long M, long N, long K, long cus, bool gather = false,
     }
   }
   if (t64 <= cus && K >= (gather ? 1024 : 1536)) {
-    if (K >= 4096) shared(sharing(t64, 1536));
+    if (K >= 8192) shared(sharing(t64, 1536));
     return Tile::kS64S4;
   }
   // Gathered operands (a convolution) of at most 64 columns: an address is made per 16 bytes of

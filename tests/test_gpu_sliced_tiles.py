@@ -29,9 +29,9 @@ def same(call, pinned, want):
         assert torch.equal(call(**kw)["out8"], call(force=pinned, **kw)["out8"])
 
 
-# 256 tiles of 64 x 64, a ragged 255, 36, 6 and one; one work-group a tile below 4096, 2 ... 12 from there on
+# 256 tiles of 64 x 64, a ragged 255, 36, 6 and one; one work-group a tile below 8192, 2 ... 12 from there on
 @pytest.mark.parametrize("M,N", [(1024, 1024), (961, 1023), (1090, 79), (300, 385), (121, 153), (33, 17)])
-@pytest.mark.parametrize("K", [1536, 1552, 1776, 4096, 6160, 8208, 24592])
+@pytest.mark.parametrize("K", [1536, 1552, 1776, 4096, 8192, 8208, 32784])
 def test_fully_connected(capi, M, N, K):
     d, w = operands((M, K), (N, K))
     want = d.double() @ w.double().t().contiguous()
