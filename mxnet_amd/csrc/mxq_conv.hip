@@ -789,6 +789,177 @@ void launch_conv_taps(hipStream_t s, const ConvArgs& a) {
 #undef MXQ_TAPS
 }
 
+// ---- convolution over 16 channels, window and pixels resident in LDS ---------------------
+// A pixel of 16 channels is one 16-byte piece, and the implicit GEMM brings it into LDS once per tap, with
+// an address for each: 140 KB for 128 pixels of a 7 x 7 window and 32 channels out.  Here a work-group
+// takes BM consecutive output pixels (in (n, oh, ow) order, regardless of where a row or an image
+// ends) and BN output channels, brings the input rows the pixels touch into LDS once, "virtual rows" of
+// H + 2 pad an image with pad columns left and right, and all taps of its channels, and forms the
+// activation fragments by addresses: two taps of 32 pixels an MFMA, the pixels one behind the other.
+// What bounds it is a work-group's one unhidden prologue, 2 to 3 us, and for many columns the weights that
+// every work-group brings (25 KB for 7 x 7 and 32 channels), then LDS reads (2 KB an MFMA on 128 pixels, 1.5
+// on 256).  Fused, implicit GEMM and this (us): 50176 pixels -> 29, 5 x 5, 9.6 / 6.4, 16928 -> 87, 7 x 7, 11.8 /
+// 8.2, 97600 -> 24, 3 x 3, 9.1 / 6.4.
+struct WindowArgs {
+  ConvArgs c;
+  int pixels_w, rows_h;  // columns of a patch row, virtual rows of an image
+  int steps, pitch;      // MFMA steps; 16-byte pieces between the weights of two channels
+  int off_patch, off_taps;
+};
+
+template <class Cfg>
+__global__ __launch_bounds__(256, 2) void conv_window_kernel(WindowArgs t) {
+  static_assert(Cfg::WN == 1 && Cfg::kThreads == 256, "four waves below each other");
+  constexpr int MI = Cfg::MI, NI = Cfg::NI;
+  extern __shared__ __attribute__((aligned(16))) char window_lds[];
+  const ConvArgs& p = t.c;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lrow = lane & 31, lgrp = lane >> 5;
+  const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(window_lds));
+  int tm, tn;
+  tile_coords(blockIdx.x, (p.M + Cfg::BM - 1) / Cfg::BM, (p.O + Cfg::BN - 1) / Cfg::BN, tm, tn);
+  const int m0 = tm * Cfg::BM, n0 = tn * Cfg::BN, taps = p.KH * p.KW, plane = p.OH * p.OW;
+  // the first virtual row under output pixel m
+  auto row_of = [&](int m) {
+    const int n = m / plane, oh = (m - n * plane) / p.OW;
+    return n * t.rows_h + oh * p.sh;
+  };
+  const int v0 = row_of(m0);
+  {
+    const int last = m0 + Cfg::BM < p.M ? m0 + Cfg::BM - 1 : p.M - 1;
+    const int pieces = (row_of(last) + (p.KH - 1) * p.dh + 1 - v0) * t.pixels_w;
+    const v4i rsrc = make_rsrc(p.data, static_cast<uint32_t>(p.N) * p.H * p.W * 16);
+    for (int i = wave * 64; i < pieces; i += 256) {
+      const int at = i + lane, row = at / t.pixels_w, v = v0 + row, n = v / t.rows_h;
+      const int ih = v - n * t.rows_h - p.ph, iw = at - row * t.pixels_w - p.pw;
+      const bool ok = at < pieces && n < p.N &&
+                      static_cast<unsigned>(ih) < static_cast<unsigned>(p.H) &&
+                      static_cast<unsigned>(iw) < static_cast<unsigned>(p.W);
+      dma_buffer(lds0 + t.off_patch + i * 16,
+                 ok ? static_cast<uint32_t>(((n * p.H + ih) * p.W + iw) * 16) : kOutOfRange, rsrc);
+    }
+  }
+  {
+    const v4i rsrc = make_rsrc(p.weight, static_cast<uint32_t>(p.O) * taps * 16);
+    for (int i = wave * 64; i < Cfg::BN * t.pitch; i += 256) {
+      const int at = i + lane, o = at / t.pitch, c = at - o * t.pitch;
+      const bool ok = o < Cfg::BN && n0 + o < p.O && c < taps;  // zeros meet taps past the last
+      dma_buffer(lds0 + i * 16,
+                 ok ? static_cast<uint32_t>(((n0 + o) * taps + c) * 16) : kOutOfRange, rsrc);
+    }
+  }
+  int* const tap_at = reinterpret_cast<int*>(window_lds + t.off_taps);
+  for (int i = tid; i < 2 * t.steps; i += 256) {
+    const int kh = i / p.KW, kw = i - kh * p.KW;
+    tap_at[i] = i < taps ? (kh * p.dh * t.pixels_w + kw * p.dw) * 16 : 0;
+  }
+  const EpiPreOf<kEpiPlain> pre = epi_prefetch<Cfg>(p.epi, n0, p.O);
+  const char* pixel[MI];
+#pragma unroll
+  for (int mi = 0; mi < MI; ++mi) {
+    int m = m0 + wave * Cfg::TM + mi * 32 + lrow;
+    m = m < p.M ? m : p.M - 1;  // never stored
+    pixel[mi] = window_lds + t.off_patch + ((row_of(m) - v0) * t.pixels_w + m % p.OW * p.sw) * 16;
+  }
+  const char* const weights = window_lds + (lrow * t.pitch + lgrp) * 16;
+  v16i acc[MI][NI];
+#pragma unroll
+  for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+    for (int ni = 0; ni < NI; ++ni)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[mi][ni][v] = 0;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+#pragma unroll 4
+  for (int ks = 0; ks < t.steps; ++ks) {
+    const int at = tap_at[2 * ks + lgrp];
+    v4i fa[MI], fb[NI];
+#pragma unroll
+    for (int mi = 0; mi < MI; ++mi) fa[mi] = *reinterpret_cast<const v4i*>(pixel[mi] + at);
+#pragma unroll
+    for (int ni = 0; ni < NI; ++ni)
+      fb[ni] = *reinterpret_cast<const v4i*>(weights + (ni * 32 * t.pitch + 2 * ks) * 16);
+#pragma unroll
+    for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+      for (int ni = 0; ni < NI; ++ni)
+        acc[mi][ni] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fb[ni], fa[mi], acc[mi][ni], 0, 0, 0);
+  }
+  if (blockIdx.x == 0 && tid == 0) epilogue_ranges(p.epi);
+  gemm_epilogue_lds<Cfg, EpiScratch<Cfg>::kNeed32>(acc, p.epi, pre, m0, n0, p.M, p.O,
+                                                   static_cast<size_t>(p.O),
+                                                   reinterpret_cast<v4i*>(window_lds));
+}
+
+// The layout of a launch in LDS, and how much of it there is; 0 where the kernel does not take the shape.
+template <class Cfg>
+size_t window_layout(const ConvArgs& a, WindowArgs& t) {
+  const long long data_bytes = static_cast<long long>(a.N) * a.H * a.W * a.C;
+  const int taps = a.KH * a.KW;
+  if (a.C != 16 || taps < 2 || taps > 64 || a.M <= 0 || data_bytes >= (1LL << 31) ||
+      static_cast<long long>(a.O) * taps * 16 >= (1LL << 31) || !aligned16(a.data) ||
+      !aligned16(a.weight))
+    return 0;
+  const long long pixels_w = a.W + 2LL * a.pw, rows_h = a.H + 2LL * a.ph;
+  if (a.N * rows_h >= (1LL << 30)) return 0;
+  // Most virtual rows under BM consecutive pixels: a step down for every output row they can touch
+  // behind the first, a jump for every image.
+  const long long down = (Cfg::BM - 2 + a.OW) / a.OW;
+  const long long images = (Cfg::BM - 2) / (static_cast<long long>(a.OH) * a.OW) + 1;
+  const long long jump = rows_h - static_cast<long long>(a.OH) * a.sh;
+  const long long rows = down * a.sh + (a.N > 1 && jump > 0 ? images * jump : 0) +
+                         (a.KH - 1LL) * a.dh + 1;
+  t.c = a;
+  t.steps = (taps + 1) / 2;
+  t.pitch = (2 * t.steps) | 1;
+  auto up = [](long long pieces) { return (pieces + 63) / 64 * 1024; };  // whole load instructions
+  const long long weights = up(static_cast<long long>(Cfg::BN) * t.pitch);
+  const long long all = weights + up(rows * pixels_w) + 2 * t.steps * 4;
+  if (all > 80 * 1024) return 0;
+  t.pixels_w = static_cast<int>(pixels_w);
+  t.rows_h = static_cast<int>(rows_h);
+  t.off_patch = static_cast<int>(weights);
+  t.off_taps = static_cast<int>(all - 2 * t.steps * 4);
+  const size_t epilogue = EpiScratch<Cfg>::kNeed32;
+  return static_cast<size_t>(all) > epilogue ? static_cast<size_t>(all) : epilogue;
+}
+
+typedef GemmCfg<128, 32, 128, 4, 1> CfgWindow;
+typedef GemmCfg<256, 32, 128, 4, 1> CfgWindow2;
+
+// Which of the two takes a convolution that the few-tiles kernel does not; 0 for neither.  Up to 32 channels
+// out both are ahead of the implicit GEMM, 256 pixels from three tiles of 128 a CU on (us, implicit GEMM, 128,
+// 256: 97600 -> 24, 3 x 3, 763 tiles, 9.1 / 6.4 / 6.6, 143748 -> 13, 3 x 3, 1124, 10.4 / 8.3 / 7.7).  More channels
+// bring the pixels again for every 32: they pay under windows of 16 taps and more, to two tiles of 128 a CU
+// (9604 -> 76, 5 x 5, 225, 7.2 / 5.8, 6075 -> 232, 5 x 5, 384, 7.4 / 6.4), of 256 to six (60984 -> 75, 5 x 5, 1431,
+// 12.2 / 12.7 / 11.1, but into int32 20631 -> 393, 7 x 7, 2106, 26.1 / 24.0 / 27.1, 242064 -> 86, 5 x 5, 5676, 35.7 /
+// 43.6 / 46.6), and under smaller ones to one (4800 -> 108, 3 x 3, 152, 5.1 / 4.8, but 52983 -> 37, 3 x 3, 828, 7.3 /
+// 7.8 / 7.3).  Strided windows read every second piece of LDS and pay from 49 taps on (7605 -> 88, 7 x 7 by 2,
+// 9.4 / 7.6, but 25281 -> 37, 5 x 5 by 2 into int32, 7.4 / 8.2).
+int window_cfg(const ConvArgs& a) {
+  const int taps = a.KH * a.KW;
+  if (a.C != 16 || taps < 9 || (a.sh * a.sw != 1 && taps < 49)) return 0;
+  const long cus = num_cus(), t = (a.M + 127L) / 128 * ((a.O + 31) / 32);
+  if (a.O <= 32) return t <= 3 * cus ? 66 : 67;
+  if (taps < 16) return t <= cus ? 66 : 0;
+  return t <= 2 * cus ? 66 : t <= 6 * cus ? 67 : 0;
+}
+
+template <class Cfg>
+bool launch_window(hipStream_t s, const ConvArgs& a) {
+  WindowArgs t;
+  const size_t lds = window_layout<Cfg>(a, t);
+  if (lds == 0) return false;
+  const long tiles =
+      static_cast<long>((a.M + Cfg::BM - 1) / Cfg::BM) * ((a.O + Cfg::BN - 1) / Cfg::BN);
+  hipLaunchKernelGGL((conv_window_kernel<Cfg>), dim3(static_cast<unsigned>(tiles)), dim3(256), lds,
+                     s, t);
+  MXQ_LAUNCH_CHECK();
+  return true;
+}
+
 // ---- 3 x 3 convolution with the input patch resident in LDS -------------------------
 // The implicit GEMM above stages every input pixel nine times, once per tap, through the
 // CU's 64 bytes per clock from L1 into LDS, which is what bounds every tile below 256 x 256.
@@ -1758,6 +1929,14 @@ void conv_nhwc(void* stream, const int8_t* data, const int8_t* weight, const int
     MXQ_CHECK(plan.splits <= 1 || force.splits == 0, "the patch kernel has no split-K form");
     launch_conv3x3_patch(s, a);
     return;
+  }
+  // 66, 67: the window kernel on 128 and 256 pixels
+  const int window = force.cfg == 66 || force.cfg == 67 ? force.cfg
+                     : force.cfg == 0 && plan.cfg != 63 && dma_ok ? window_cfg(a) : 0;
+  if (window != 0) {
+    MXQ_CHECK(dma_ok && force.splits <= 1, "shape does not qualify for the window kernel");
+    if (window == 66 ? launch_window<CfgWindow>(s, a) : launch_window<CfgWindow2>(s, a)) return;
+    MXQ_CHECK(force.cfg == 0, "shape does not qualify for the window kernel");
   }
   const int cfg = plan.cfg, sp = plan.splits;
   if (cfg == 63) {  // the few-tiles kernel; `splits` is the number of waves per tile
