@@ -799,7 +799,9 @@ void launch_conv_taps(hipStream_t s, const ConvArgs& a) {
 // What bounds it is a work-group's one unhidden prologue, 2 to 3 us, and for many columns the weights that
 // every work-group brings (25 KB for 7 x 7 and 32 channels), then LDS reads (2 KB an MFMA on 128 pixels, 1.5
 // on 256).  Fused, implicit GEMM and this (us): 50176 pixels -> 29, 5 x 5, 9.6 / 6.4, 16928 -> 87, 7 x 7, 11.8 /
-// 8.2, 97600 -> 24, 3 x 3, 9.1 / 6.4.
+// 8.2, 97600 -> 24, 3 x 3, 9.1 / 6.4.  Over more channels, pixels an odd number of pieces apart, it is ahead only
+// over 32 into 32 and fewer (200704 -> 32, 3 x 3, 15.0 / 11.7, 83655 -> 17, 5 x 5, 11.2 / 10.8) and level or behind over
+// 48 and 64 (11250 -> 11, 5 x 5, 8.4 / 8.4, 200704 -> 64, 3 x 3, 15.1 / 30.9): left at 16.
 struct WindowArgs {
   ConvArgs c;
   int pixels_w, rows_h;  // columns of a patch row, virtual rows of an image
