@@ -439,8 +439,13 @@ __global__ __launch_bounds__(128) void entropy_chains_kernel(Args a) {
   if (r.state == 0 && at >= 0) info->q_sum = sum;
 }
 
-// RN(a / b) from RN(1 / b): a quotient that is off by less than two last places and one correction
-// by its exact remainder (Markstein's division)
+// a / b from a reciprocal, the first guess and one correction by its remainder (Markstein's division).
+// With RN(1 / b) it is RN(a / b) while nothing leaves the normal range: in units of the quotient's last
+// place u the guess is off by less than 1.5, so the remainder is rounded by no more than 1 / b of u 2^-23 and
+// the correction misses a / b by less than 3.5 u 2^-24, while a quotient that is no midpoint of two floats is
+// u 2^-24 n / b from the next one for a whole n.  That leaves those with n of up to 7, and a test goes
+// through all of them.  With a reciprocal a last place off it is that, or where a / b is as close to a midpoint,
+// the float on its other side.
 __device__ __forceinline__ float quotient(float a, float b, float reciprocal) {
   const float q = a * reciprocal;
   return __builtin_fmaf(__builtin_fmaf(-q, b, a), reciprocal, q);
@@ -455,9 +460,9 @@ __device__ __forceinline__ float natural_log(float x) {
 
 // The bounds, a wave per candidate, 16 bins in a row per lane.  With u = 2^-24, a term of the float
 // chain carries a logarithm of at most a last place (2u) and a product's rounding, a term here a
-// logarithm of at most two (4u; 2.71u is the most over 2^30 arguments) and an exact product; a sum of the
-// chain carries u of itself.  The factors add up to one, and a last place of theirs (should a quotient
-// miss it, which none of 2^30 did) to u.
+// logarithm of at most two (4u; a test measures it on every normal number) and an exact product; a sum
+// of the chain carries u of itself.  The factors are the chain's, and add up to one; the logarithms'
+// arguments are its own or the next float, 2u of the logarithm.
 // (Vector instructions bound it: 136 us for the three histograms above with the compiler's divisions and
 // logarithm and 4 bins in a row, a scan of the wave for every 256 bins; 95 us so.)
 __global__ __launch_bounds__(256) void entropy_bounds_kernel(Args a) {
@@ -478,7 +483,7 @@ __global__ __launch_bounds__(256) void entropy_bounds_kernel(Args a) {
   const float p_zero = kEps / r.p_sum, q_zero = kEps / r.q_sum;
   const double zero_term = static_cast<double>(p_zero) * static_cast<double>(logf(p_zero / q_zero));
   double sum = 0.0;  // the same in every lane
-  float magnitude = 0.0f, sums = 0.0f;
+  double magnitude = 0.0, sums = 0.0;
   bool bad = false;
   for (int base = 0; base < width; base += 64 * B) {
     const int from = base + B * lane;
@@ -500,14 +505,13 @@ __global__ __launch_bounds__(256) void entropy_bounds_kernel(Args a) {
       const float level = levels[j < p.levels ? j : p.levels - 1];
       const float q = level != 0.0f ? level - r.q_take : kEps;
       const float pn = quotient(x - r.p_take, r.p_sum, p_once), qn = quotient(q, r.q_sum, q_once);
-      // pn / qn, but for the last place of 1 / qn
       const float once = __builtin_amdgcn_rcpf(qn);
       const double term =
           static_cast<double>(pn) * static_cast<double>(natural_log(quotient(pn, qn, once)));
       const bool filled = x != 0.0f && o < width;
       bad = bad || (filled && (!(pn > 0.0f) || !(qn > 0.0f)));
       t[k] = filled ? term : o < width ? zero_term : 0.0;
-      magnitude += fabsf(static_cast<float>(t[k]));
+      magnitude += fabs(t[k]);
       all += t[k];
       if (++rest == merged) {
         ++j;
@@ -525,7 +529,7 @@ __global__ __launch_bounds__(256) void entropy_bounds_kernel(Args a) {
 #pragma unroll
     for (int k = 0; k < B; ++k) {
       before += t[k];
-      sums += from + k < width ? fabsf(static_cast<float>(before)) : 0.0f;
+      sums += from + k < width ? fabs(before) : 0.0;
     }
   }
   for (int d = 1; d < 64; d *= 2) {
@@ -534,14 +538,26 @@ __global__ __launch_bounds__(256) void entropy_bounds_kernel(Args a) {
   }
   bad = __any(bad);
   const double u = 1.0 / 16777216.0;
-  // (5 % for what is summed up in float here)
-  const double margin = 1.05 * u * (8.0 * magnitude + 1.0 + sums) + 1e-12;
+  // (5 % for what is of second order, the factors' sum among it)
+  const double margin = 1.05 * u * (8.0 * magnitude + 2.0 + sums) + 1e-12;
   if (lane == 0) {
     const bool known = !bad && isfinite(sum) && isfinite(margin);
     out[0] = known ? sum - margin : -INFINITY;
     out[1] = known ? sum + margin : INFINITY;
   }
 }
+
+#ifdef MXQ_TEST_HOOKS
+__global__ __launch_bounds__(256) void entropy_functions_kernel(const float* a, const float* b,
+                                                                size_t n, float* exact, float* near,
+                                                                float* logs) {
+  const size_t i = blockIdx.x * size_t(256) + threadIdx.x;
+  if (i >= n) return;
+  if (exact != nullptr) exact[i] = quotient(a[i], b[i], 1.0f / b[i]);
+  if (near != nullptr) near[i] = quotient(a[i], b[i], __builtin_amdgcn_rcpf(b[i]));
+  if (logs != nullptr) logs[i] = natural_log(a[i]);
+}
+#endif
 
 size_t up256(size_t x) { return (x + 255) / 256 * 256; }
 
@@ -637,5 +653,20 @@ int mxq_entropy_bounds(void* stream, int count, const float* hist, const int* bi
   MXQ_LAUNCH_CHECK();
   MXQ_API_END();
 }
+
+#ifdef MXQ_TEST_HOOKS
+// tests/mxq_test_hooks.h
+int mxq_test_entropy_functions(void* stream, const float* a, const float* b, size_t n, float* exact,
+                               float* near, float* logs) {
+  MXQ_API_BEGIN();
+  if (n == 0) return 0;
+  MXQ_CHECK(n <= (size_t(1) << 31), "too many numbers");
+  MXQ_CHECK(a != nullptr && (b != nullptr || (exact == nullptr && near == nullptr)), "null pointer");
+  hipLaunchKernelGGL(entropy_functions_kernel, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256),
+                     0, static_cast<hipStream_t>(stream), a, b, n, exact, near, logs);
+  MXQ_LAUNCH_CHECK();
+  MXQ_API_END();
+}
+#endif  // MXQ_TEST_HOOKS
 
 }  // extern "C"

@@ -94,6 +94,11 @@ int mxq_test_quantized_conv_nchw(void* stream, const int8_t* data, const int8_t*
 int mxq_test_block_lds(int N, int H, int W, int C, int C_mid, int C_out, int C_next, int tile,
                        int* lds, int* reach);
 
+/* What the entropy bounds (mxq_entropy_bounds) compute with, on n floats: a / b from the rounded reciprocal
+ * and from the instruction's, and the logarithm of a; outputs may be null. */
+int mxq_test_entropy_functions(void* stream, const float* a, const float* b, size_t n, float* exact,
+                               float* near, float* logs);
+
 #ifdef __cplusplus
 }
 #endif
