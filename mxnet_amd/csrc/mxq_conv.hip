@@ -1092,6 +1092,7 @@ __global__ __launch_bounds__(512, 2) void conv3x3_patch_kernel(ConvArgs p) {
       const int newest = (kt + NS - 2) < (KT - 1) ? (kt + NS - 2) : (KT - 1);
       wait_ahead<BI, NS - 2>(newest - kt);
     }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // ... and what it read of stage kt - 1
     __builtin_amdgcn_s_barrier();
     issue(kt + NS - 1);
     const v4i* sbw = reinterpret_cast<const v4i*>(ring + (kt % NS) * STAGE_BYTES);

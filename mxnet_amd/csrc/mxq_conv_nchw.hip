@@ -330,6 +330,7 @@ __global__ __launch_bounds__(Cfg::kThreads, 2) void conv1x1_planes_kernel(PlaneA
     for (int kt = 0; kt < KT; ++kt) {
       const int newest = (kt + NS - 2) < (KT - 1) ? (kt + NS - 2) : (KT - 1);
       wait_ahead<CPT, NS - 2>(newest - kt);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // ... and what it read of stage kt - 1
       __builtin_amdgcn_s_barrier();
       issue(kt + NS - 1);
       compute(kt);

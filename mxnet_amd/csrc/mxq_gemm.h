@@ -763,6 +763,8 @@ __device__ __forceinline__ void gemm_mainloop_dma(v16i (&acc)[Cfg::MI][Cfg::NI],
   if (PIPE == 0) {
     for (int kt = 0; kt < KT; ++kt) {
       wait_ahead<CPT, NS - 2>(last_issued(kt) - kt);  // this wave's part of stage kt landed
+      // ... and what it read of stage kt-1 (its products may be scheduled on either side)
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       __builtin_amdgcn_s_barrier();                    // ... everybody's; stage kt-1 is free
       issue(kt + NS - 1);
 #pragma unroll
