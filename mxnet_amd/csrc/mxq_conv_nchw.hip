@@ -731,18 +731,22 @@ typedef PlaneCfg<64, 128, 128, 2, 2> PlaneP64k2;
 // Stages of the ring.  Two, whatever the reduction, where a CU has work-groups enough: one's loads are
 // under way while another multiplies, and three or four stages leave room for fewer of them (64 images,
 // us with two / three / four: 28 x 28 128 -> 512 27.7 / 30.2 / 32.4, 56 x 56 64 -> 256 47.5 / 48.1 / 47.5,
-// 14 x 14 256 -> 1024 16.4 / 16.6 / 20.4).  Up to two small tiles a CU wait for memory at every step, and
-// what is under way is then what counts: 64 x 64 tiles, 1024 -> 512 / 2 at 14 x 14 11.0 / 9.8 / 8.6, and of
-// 8 images 1024 -> 256 at 14 x 14 12.3 / 8.2 / 7.4, 512 -> 128 at 28 x 28 8.9 / 6.9 / 6.8; of 4 images, four
-// to seven steps, 256 -> 1024 5.5 / 5.1 / 5.7, of 7 images 320 -> 640 at 20 x 20 6.4 / 5.9 / 6.0.  So is it
-// for 128 x 64 tiles, small ones as well, of any grid (256 -> 64 at 56 x 56 behind other layers 23.4 / 21.6 /
-// 24.4).
+// 14 x 14 256 -> 1024 16.4 / 16.6 / 20.4).  Up to two 64 x 64 tiles a CU wait for memory at every step, and
+// what is under way is then what counts: 1024 -> 512 / 2 at 14 x 14 11.0 / 9.8 / 8.6, and of 8 images
+// 1024 -> 256 at 14 x 14 12.3 / 8.2 / 7.4, 512 -> 128 at 28 x 28 8.9 / 6.9 / 6.8; of 4 images, four to
+// seven steps, 256 -> 1024 5.5 / 5.1 / 5.7, of 7 images 320 -> 640 at 20 x 20 6.4 / 5.9 / 6.0.  59 drawn
+// layers are 1.15 times as fast on three stages (0.95 to 1.39).  64 x 128 tiles, one to two a CU, are level with
+// them (51 drawn layers 0.997, 0.94 to 1.06) and stay on two.
+// 128 x 64 tiles take three, whatever the grid: up to one a CU the operands from memory 1.00 to 1.05 times as fast
+// at three to five steps, 1.1 at eight, 1.2 from sixteen on (16 images, 1536 -> 20 at 12 x 12, 13.0 / 10.8), past
+// that level to 6 % behind alone (256 -> 64 at 56 x 56 22.2 / 23.0), that layer behind others 23.4 / 21.6 /
+// 24.4.  Operands of less than the L2, read again and again, are the exception: 5 % behind at three steps, 22 at 28.
 template <class Cfg>
 int plane_stages(int steps, long long groups) {
-  if (steps < 3) return 2;
-  if (Cfg::BP == 128 && Cfg::BO == 64) return 3;
-  if (Cfg::BP * Cfg::BO > 64 * 128 || Cfg::BK != 64 || groups > 2 * num_cus()) return 2;
-  return Cfg::BO == 64 && steps >= 8 ? 4 : 3;
+  if (steps < 3 || Cfg::BO != 64 || Cfg::BK != 64) return 2;
+  if (Cfg::BP == 128) return 3;
+  if (groups > 2 * num_cus()) return 2;
+  return steps >= 8 ? 4 : 3;
 }
 
 template <class Cfg>
@@ -763,8 +767,8 @@ void launch_planes(hipStream_t s, PlaneArgs a, int gm) {
   } else {
     const int stages = plane_stages<Cfg>((a.C + Cfg::BK - 1) / Cfg::BK, total);
     // (only the tiles that plane_stages tells apart have the longer rings)
-    constexpr bool longer = Cfg::BK == 64 && Cfg::BP * Cfg::BO <= 128 * 64;
-    constexpr int three = longer ? 3 : 2, four = longer && Cfg::BO == 64 && Cfg::BP == 64 ? 4 : 2;
+    constexpr bool longer = Cfg::BK == 64 && Cfg::BO == 64;
+    constexpr int three = longer ? 3 : 2, four = longer && Cfg::BP == 64 ? 4 : 2;
     if (stages == 4)
       hipLaunchKernelGGL((conv1x1_planes_kernel<Cfg, four, kNative>), grid, block, 0, s, a);
     else if (stages == 3)
