@@ -127,7 +127,7 @@ for _name, (_res, _args) in SIGNATURES.items():
 # test-only twins of the FC and convolution entry points (tests/mxq_test_hooks.h, not part
 # of include/mxq.h): the same arguments followed by the tile configuration, the split-K
 # factor and, for the FC, the streaming kernel's work-groups per CU (0 = choose); what a block's
-# launch reads of LDS; and the functions that the entropy bounds are made of
+# launch reads of LDS; what is chosen for a layer; and the functions that the entropy bounds are made of
 TEST_HOOKS = {
     "mxq_test_quantized_fc": (_i, SIGNATURES["mxq_quantized_fc"][1] + [_i, _i, _i]),
     "mxq_test_quantized_fc_sum": (_i, SIGNATURES["mxq_quantized_fc_sum"][1] + [_i, _i, _i]),
@@ -137,6 +137,8 @@ TEST_HOOKS = {
     "mxq_test_quantized_conv_nhwc": (_i, SIGNATURES["mxq_quantized_conv_nhwc"][1] + [_i, _i]),
     "mxq_test_quantized_conv_nchw": (_i, SIGNATURES["mxq_quantized_conv_nchw"][1] + [_i]),
     "mxq_test_block_lds": (_i, [_i] * 8 + [ctypes.POINTER(_i)] * 2),
+    "mxq_test_fc_plan": (_i, [_i] * 6 + [_p, _sz] + [ctypes.POINTER(_i)] * 2),
+    "mxq_test_conv_plan": (_i, [_i] * 13 + [_p, _sz] + [ctypes.POINTER(_i)] * 2),
     "mxq_test_entropy_functions": (_i, [_p, _p, _p, _sz, _p, _p, _p]),
 }
 for _name, (_res, _args) in TEST_HOOKS.items():

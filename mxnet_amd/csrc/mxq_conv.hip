@@ -1746,7 +1746,8 @@ ConvPlan plan_conv(const ConvGeometry& g, bool aligned, const GemmForce& force) 
         case Tile::kN32S3: plan.cfg = 41; break;
         case Tile::kN32K2: plan.cfg = 42; break;
         case Tile::kM128S3: plan.cfg = 43; break;
-        case Tile::kW192K2: plan.cfg = 11; break;  // not proposed for gathered operands
+        case Tile::kW192K2:
+          MXQ_CHECK(false, "a tile of plain operands proposed for gathered ones");
       }
     } else if (O > 128 && tiles(256, 256) >= cus) {
       plan.cfg = 1;
@@ -1789,6 +1790,18 @@ size_t conv_plan_workspace(const ConvPlan& plan, const ConvGeometry& g) {
   if (plan.splits <= 1 || !conv_cfg_tile(plan.cfg, bm, bn)) return 0;
   const long tiles = static_cast<long>((g.M + bm - 1) / bm) * ((g.O + bn - 1) / bn);
   return splitk_workspace_bytes(tiles, plan.splits, bm, bn);
+}
+
+// ... with the workspace at hand: a split that the chooser proposed is dropped without room for it.
+ConvPlan plan_conv_within(const ConvGeometry& g, bool aligned, const GemmForce& force,
+                          const Workspace& ws) {
+  const ConvPlan plan = plan_conv(g, aligned, force);
+  if (force.splits != 0 || plan.splits <= 1 ||
+      (ws.ptr != nullptr && aligned16(ws.ptr) && ws.bytes >= conv_plan_workspace(plan, g)))
+    return plan;
+  GemmForce unsplit = force;
+  unsplit.splits = 1;
+  return plan_conv(g, aligned, unsplit);
 }
 
 // Both C entry points: `planar` writes out32 as [N][O][OH][OW] instead of [N][OH][OW][O].
@@ -1894,14 +1907,7 @@ void conv_nhwc(void* stream, const int8_t* data, const int8_t* weight, const int
     }
   }
   MXQ_CHECK(force.cfg != 65, "not a layer for the kernel with the weights in registers");
-  ConvPlan plan = plan_conv(g, aligned, force);
-  // a split the chooser proposed is dropped when the caller brought no room for it
-  if (force.splits == 0 && plan.splits > 1 &&
-      (ws.ptr == nullptr || !aligned16(ws.ptr) || ws.bytes < conv_plan_workspace(plan, g))) {
-    GemmForce unsplit = force;
-    unsplit.splits = 1;
-    plan = plan_conv(g, aligned, unsplit);
-  }
+  const ConvPlan plan = plan_conv_within(g, aligned, force, ws);
   // 61: the parked-weights row kernel (3 x 3 over 64 -> 64 channels, fused int8 output);
   // chosen for it whenever the launch has rows for every wave of the chip, with int32 planes by a
   // rule of their own
@@ -2242,6 +2248,33 @@ int mxq_test_quantized_conv_nhwc(void* stream, const int8_t* data, const int8_t*
   conv_nhwc(stream, data, weight, bias, N, H, W, C, O, KH, KW, stride_h, stride_w, pad_h, pad_w,
             dilate_h, dilate_w, min_data, max_data, min_weight, max_weight, min_bias, max_bias,
             out32, omin, omax, out8, rmin, rmax, relu, min_calib, max_calib, false, force, ws);
+  MXQ_API_END();
+}
+
+// tests/mxq_test_hooks.h
+int mxq_test_conv_plan(int N, int H, int W, int C, int O, int KH, int KW, int stride_h, int stride_w,
+                       int pad_h, int pad_w, int dilate_h, int dilate_w, void* workspace,
+                       size_t workspace_bytes, int* cfg, int* splits) {
+  MXQ_API_BEGIN();
+  MXQ_CHECK(C % 16 == 0 && cfg != nullptr && splits != nullptr, "whole pieces of channels");
+  const ConvGeometry g = conv_geometry(N, H, W, C, O, KH, KW, stride_h, stride_w, pad_h, pad_w,
+                                       dilate_h, dilate_w);
+  Workspace ws;
+  ws.ptr = workspace;
+  ws.bytes = workspace_bytes;
+  const ConvPlan plan = plan_conv_within(g, true, GemmForce(), ws);
+  ConvArgs a = {};
+  a.N = N; a.H = H; a.W = W; a.C = C; a.O = O; a.KH = KH; a.KW = KW;
+  a.sh = stride_h; a.sw = stride_w; a.ph = pad_h; a.pw = pad_w; a.dh = dilate_h; a.dw = dilate_w;
+  a.OH = g.OH; a.OW = g.OW;
+  a.M = static_cast<int>(g.M);
+  a.K = static_cast<int>(g.K);
+  const int window = plan.cfg != 63 ? window_cfg(a) : 0;
+  WindowArgs t;
+  const bool fits = window == 66   ? window_layout<CfgWindow>(a, t) != 0
+                    : window == 67 ? window_layout<CfgWindow2>(a, t) != 0 : false;
+  *cfg = fits ? window : plan.cfg;
+  *splits = fits ? 1 : plan.splits;
   MXQ_API_END();
 }
 #endif  // MXQ_TEST_HOOKS

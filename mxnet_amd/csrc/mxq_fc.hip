@@ -26,6 +26,7 @@ namespace mxq {
 //   14, 16  direct-to-LDS 256x256, 4 waves: compiler-scheduled / pinned pipeline
 //   21..24  direct-to-LDS buffer-load kernels 256x128, 256x64, 128x128, 64x64
 //   31, 32  as 12 / 16 with buffer loads (K % 16 == 0 instead of K % 64 == 0)
+//   33, 34  64x64 and 128x128 on eight waves
 //   41..44  as 21..24 with a 2-stage ring (short K)
 //   51..56  128-byte stages: 64x64 (2, 3 stages), 128x128 (2, 3), 256x256 (2), 256x128 (2)
 //   57..59  128x64 and 64x128 with 128-byte stages, 64x64 with 256-byte stages
@@ -34,6 +35,8 @@ namespace mxq {
 //   65      the kernel with the weights in registers, where it is the faster one
 //   71      the few-tiles kernel (any shape; here `splits` is the number of waves per
 //           32 x 32 tile, negative for 16 x 16 tiles)
+// plan_fc proposes 1, 3, 4, 12, 31, 33, 34, 41, 43, 44, 51, 53, 57..62 and 71, and 55 for a residual sum;
+// the others are there for who pins them.
 // Output tile of a direct-to-LDS configuration (what a split-K work-group leaves in the
 // workspace); false for every other configuration.
 bool fc_cfg_tile(int cfg, int& bm, int& bn) {
@@ -85,7 +88,6 @@ FcPlan plan_fc(int M, int N, int K, bool aligned, bool fused8, const GemmForce& 
       switch (choose_tile(M, N, K, cus, false, may_split ? &auto_splits : nullptr)) {
         case Tile::kL8: plan.cfg = glb_ok ? 12 : 31; break;
         case Tile::kW128x2: plan.cfg = 41; break;
-        case Tile::kW128K2: plan.cfg = 56; break;  // not proposed for plain operands
         case Tile::kM128x2: plan.cfg = 43; break;
         case Tile::kM128K2: plan.cfg = 53; break;
         case Tile::kS64x2: plan.cfg = 44; break;
@@ -96,8 +98,8 @@ FcPlan plan_fc(int M, int N, int K, bool aligned, bool fused8, const GemmForce& 
         case Tile::kW192K2: plan.cfg = 60; break;
         case Tile::kS64S4: plan.cfg = 33; break;
         case Tile::kM128S3: plan.cfg = 34; break;
-        case Tile::kW64x2: plan.cfg = 42; break;  // not proposed for plain operands
-        case Tile::kN32S3: case Tile::kN32K2: plan.cfg = 33; break;  // nor these
+        case Tile::kW128K2: case Tile::kW64x2: case Tile::kN32S3: case Tile::kN32K2:
+          MXQ_CHECK(false, "a tile of gathered operands proposed for plain ones");
       }
     } else {
       if (tiles(256, 256) >= cus)
@@ -114,7 +116,9 @@ FcPlan plan_fc(int M, int N, int K, bool aligned, bool fused8, const GemmForce& 
     // they cover 0.56 of the CUs (12544 x 256 -> 1024: -1.9 us per layer) and 128 x 128
     // tiles otherwise (50176 x 128 -> 512: -1.2 us per layer).
     // The requantized sum is another third of arithmetic: 128 x 128 tiles throughout (12544 x 256
-    // -> 1024 15.8 us against 16.8, 50176 x 128 -> 512 22.6 against 27.7).
+    // -> 1024 15.8 us against 16.8, 50176 x 128 -> 512 22.6 against 27.7).  (Where one round of 128 x 128 tiles
+    // is proposed, on 128-byte stages, either form is level with 64-byte ones: 8192 x 320 -> 1024 10.5 and 11.0 us
+    // against 10.7 and 11.1, 12544 x 320 -> 512 10.3 and 10.8 against 10.2 and 10.8.)
     if (sum && plan.cfg == 41) {
       if (!requant && K >= 256 && N > 128 && 16 * tiles(256, 256) >= 9 * cus)
         plan.cfg = 55;
@@ -174,6 +178,18 @@ size_t fc_plan_workspace(const FcPlan& plan, int M, int N) {
   if (plan.splits <= 1 || !fc_cfg_tile(plan.cfg, bm, bn)) return 0;
   const long tiles = static_cast<long>((M + bm - 1) / bm) * ((N + bn - 1) / bn);
   return splitk_workspace_bytes(tiles, plan.splits, bm, bn);
+}
+
+// ... with the workspace at hand: a split that the chooser proposed is dropped without room for it.
+FcPlan plan_fc_within(int M, int N, int K, bool aligned, bool fused8, const GemmForce& force,
+                      bool sum, bool requant, const Workspace& ws) {
+  const FcPlan plan = plan_fc(M, N, K, aligned, fused8, force, sum, requant);
+  if (force.splits != 0 || plan.splits <= 1 ||
+      (ws.ptr != nullptr && aligned16(ws.ptr) && ws.bytes >= fc_plan_workspace(plan, M, N)))
+    return plan;
+  GemmForce unsplit = force;
+  unsplit.splits = 1;
+  return plan_fc(M, N, K, aligned, fused8, unsplit, sum, requant);
 }
 
 // Looks for a short form of the requantized sum over given ranges (SumPairs): the products of the
@@ -306,14 +322,8 @@ void launch_fc(hipStream_t s, const int8_t* data, const int8_t* weight, int M, i
     }
   }
   MXQ_CHECK(force.cfg != 65, "not a layer for the kernel with the weights in registers");
-  FcPlan plan = plan_fc(M, N, K, aligned, fused8, force, sum, epi.sum_requant != 0);
-  // a split the chooser proposed is dropped when the caller brought no room for it
-  if (force.splits == 0 && plan.splits > 1 &&
-      (ws.ptr == nullptr || !aligned16(ws.ptr) || ws.bytes < fc_plan_workspace(plan, M, N))) {
-    GemmForce unsplit = force;
-    unsplit.splits = 1;
-    plan = plan_fc(M, N, K, aligned, fused8, unsplit, sum, epi.sum_requant != 0);
-  }
+  const FcPlan plan =
+      plan_fc_within(M, N, K, aligned, fused8, force, sum, epi.sum_requant != 0, ws);
   const int cfg = plan.cfg;
   if (cfg >= 11 && cfg <= 16) MXQ_CHECK(glb_ok, "shape does not qualify for the DMA kernels");
   if (cfg == 61 || cfg == 62) {
@@ -497,6 +507,21 @@ int mxq_test_quantized_fc(void* stream, const int8_t* data, const int8_t* weight
   fc_entry(stream, data, weight, bias, M, N, K, min_data, max_data, min_weight, max_weight,
            min_bias, max_bias, out32, omin, omax, out8, nullptr, rmin, rmax, relu, min_calib,
            max_calib, workspace, workspace_bytes, force);
+  MXQ_API_END();
+}
+
+// tests/mxq_test_hooks.h
+int mxq_test_fc_plan(int M, int N, int K, int fused_int8, int sum, int requant, void* workspace,
+                     size_t workspace_bytes, int* cfg, int* splits) {
+  MXQ_API_BEGIN();
+  MXQ_CHECK(M > 0 && N > 0 && K > 0 && cfg != nullptr && splits != nullptr, "bad arguments");
+  Workspace ws;
+  ws.ptr = workspace;
+  ws.bytes = workspace_bytes;
+  const FcPlan plan = plan_fc_within(M, N, K, K % 16 == 0, fused_int8 != 0, GemmForce(), sum != 0,
+                                     requant != 0, ws);
+  *cfg = plan.cfg;
+  *splits = plan.splits;
   MXQ_API_END();
 }
 #endif  // MXQ_TEST_HOOKS

@@ -94,6 +94,16 @@ int mxq_test_quantized_conv_nchw(void* stream, const int8_t* data, const int8_t*
 int mxq_test_block_lds(int N, int H, int W, int C, int C_mid, int C_out, int C_next, int tile,
                        int* lds, int* reach);
 
+/* What the entry points choose, host code alone (a device is asked for its compute units): the tile
+ * configuration and the work-groups per output tile of a fully-connected layer whose operands are aligned and
+ * whose reduction is taken as it is, and of a convolution's tiled kernels and its window kernel.  `workspace`
+ * is looked at for its alignment only. */
+int mxq_test_fc_plan(int M, int N, int K, int fused_int8, int sum, int requant, void* workspace,
+                     size_t workspace_bytes, int* cfg, int* splits);
+int mxq_test_conv_plan(int N, int H, int W, int C, int O, int KH, int KW, int stride_h, int stride_w,
+                       int pad_h, int pad_w, int dilate_h, int dilate_w, void* workspace,
+                       size_t workspace_bytes, int* cfg, int* splits);
+
 /* What the entropy bounds (mxq_entropy_bounds) compute with, on n floats: a / b from the rounded reciprocal
  * and from the instruction's, and the logarithm of a; outputs may be null. */
 int mxq_test_entropy_functions(void* stream, const float* a, const float* b, size_t n, float* exact,
