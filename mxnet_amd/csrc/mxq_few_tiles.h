@@ -30,7 +30,8 @@ inline long few_tiles_count(long M, long N) { return ((M + 31) / 32) * ((N + 31)
 // at least two blocks (at 64 bytes the tiled kernels are level or ahead).  From 8192 on
 // the tiled kernels split the reduction over work-groups and keep all but the smallest outputs, from 32768 on
 // these too where the caller brought room for it (us, here and there: 121 x 34800 -> 153 23.2 / 17.5, 48 x
-// 33200 -> 686 23.5 / 18.2, but 192 x 25088 -> 81 16.2 / 15.4, 512 x 17248 -> 106 13.8 / 15.5).
+// 33200 -> 686 23.5 / 18.2, 192 x 25088 -> 81 16.2 / 15.4, but 512 x 17248 -> 106 13.8 / 15.5; drawn convolutions,
+// the operands from memory, 11 of 32768 and more 1.7 to 4.1 times as fast, 11 of 16384 ... 32768 0.95 to 2.1).
 inline bool few_tiles_wins(long M, long N, long K, long cus, bool may_split = false) {
   return K >= 256 && few_tiles_count(M, N) <= (K < 8192 ? cus : cus / 4) &&
          !(may_split && K >= 32768);

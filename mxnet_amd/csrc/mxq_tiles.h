@@ -91,12 +91,13 @@ inline Tile choose_tile(long M, long N, long K, long cus, bool gather = false,
   // 9.7, 252 x 1376 -> 1562 7.4 / 7.6).  From the second tile a CU on two of the small work-groups are level
   // or ahead (7680 x 3200 -> 72, 386 tiles, 16.1 / 21.5).
   // Split-K: where such tiles leave CUs idle and the reduction is long, as many work-groups share one as
-  // there are CUs for, each with 1536 of it and more (unsplit and split: 1152 x 15680 -> 336 32.1 / 23.4 on two,
-  // 1681 x 13328 -> 98, 54 tiles, 27.9 / 16.3 on four, 121 x 34800 -> 153, 6 tiles, on 6, 8, 12 and 16 19.5 / 17.7 /
-  // 17.5 / 18.3).  The price is a counter-clearing launch and the partial sums' round trip through memory, about
-  // 3 us, and as much of the host's time, which is what a caller of small layers waits for: below 8192 it gains
-  // no more than that (2500 x 4704 -> 114, 80 tiles, 15.1 / 13.3, 5396 x 8144 -> 58, 85, 19.2 / 17.2, 765 x 3728 -> 512,
-  // 96, 11.6 / 12.1).
+  // there are CUs for, each with 1536 of it and more (convolutions, unsplit on four waves, on eight, and split: 1152 x
+  // 15680 -> 336 42.0 / 30.3 / 22.2 on two, 1681 x 13328 -> 98, 54 tiles, 36.4 / 26.7 / 16.6 on four, 121 x 34800 ->
+  // 153, 6 tiles, 87.8 / 57.8 / 17.0 on 12; on 6, 8 and 16 19.5 / 17.7 / 18.3).  The price is a counter-clearing
+  // launch and the partial sums' round trip through memory, about 3 us, and as much of the host's time, which is
+  // what a caller of small layers waits for: below 8192 it gains no more than that, with any tile (2500 x 4704 ->
+  // 114, 80 tiles, 15.1 / 13.3, 5396 x 8144 -> 58, 85, 19.2 / 17.2, 765 x 3728 -> 512, 96, 11.6 / 12.1; 128 x 128
+  // tiles below).
   // Gathered operands of at most 32 columns take 128 x 32 tiles, half as many of which are padding, with
   // one of these a CU (20172 x 11760 -> 11, 158, 41.6 on four waves, 30.4 so, 28512 x 2000 -> 27 12.8 / 11.0) or
   // split over a long reduction (64 x 64 tiles split and these: 14400 x 25088 -> 32 50.6 / 36.4, 7744 x 14112 -> 11
@@ -124,16 +125,18 @@ inline Tile choose_tile(long M, long N, long K, long cus, bool gather = false,
   // 2048 -> 64, 1024 tiles, 56.7 / 53.0 / 51.3).
   const bool two_a_cu = t64 <= 2 * cus;
   // From half a 64 x 64 tile a CU to two of them and a long reduction: 128 x 128 tiles, which take in half
-  // as much an output, split over the chip where that leaves few CUs idle (64 x 64 tiles and these: 1176 x
-  // 45472 -> 653, 209 and 60 on four, 87.1 / 64.6, 720 x 15680 -> 799, 156 and 42 on six, 33.2 / 28.4, 475 x 29008 ->
-  // 1145, 144 and 36 on seven, 52.5 / 37.8, but 1568 x 12000 -> 493, 200 and 52 on four, 27.4 / 28.8, 6758 x 6176 ->
-  // 113, 212 and 53, 19.0 / 20.9; with a second of the former on a CU 9408 x 11600 -> 71, 294 and 74 on three,
-  // 39.8 / 30.9, 784 x 6272 -> 1387, 286 and 77, 25.6 / 22.7, 699 x 8160 -> 2429, 418 and 114 on two, 35.9 / 30.7, but
-  // 3831 x 6848 -> 404, 420 and 120 on two, 24.3 / 25.8, 1701 x 6768 -> 862, 378 and 98, 27.1 / 27.7).
+  // as much an output, split over the chip where that leaves few CUs idle (64 x 64 tiles, on eight waves up to one a
+  // CU, and these: 1176 x 45472 -> 653, 209 and 60 on four, 87.1 / 64.6, 720 x 15680 -> 799, 156 and 42 on six,
+  // 33.2 / 28.4, 475 x 29008 -> 1145, 144 and 36 on seven, 53.6 / 37.4, but 1568 x 12000 -> 493, 200 and 52 on four,
+  // 27.4 / 28.8; with a second of the former on a CU, on four waves, 9408 x 11600 -> 71, 294 and 74 on three, 39.8 /
+  // 30.9, 925 x 11712 -> 1712, 405 and 112 on two, 39.9 / 34.7).  90 drawn FC layers and 50 convolutions of that are
+  // 1.2 times as fast on three and more from 8192 on, 1.04 below, some of them behind (2512 x 6624 -> 387 20.2 / 22.0,
+  // 784 x 6272 -> 1387 19.5 / 20.7), and on two 1.05 up to 10000, 1.09 from there, some level or behind (1150 x 12544 ->
+  // 1656 39.7 / 41.3).
   if (N > 64 && 2 * t64 > cus && two_a_cu) {
     const long sp = sharing(t128, 1536);
     if (sp >= 2 && 5 * sp * t128 >= 4 * cus &&
-        K >= (t64 <= cus ? 14336 : sp >= 3 ? 6144 : 8000)) {
+        K >= (t64 <= cus ? 14336 : 8192)) {
       shared(sp);
       return Tile::kM128S3;
     }
@@ -156,7 +159,8 @@ inline Tile choose_tile(long M, long N, long K, long cus, bool gather = false,
   if (gather && N <= 32 && K >= 432 && 4 * t32 >= 3 * cus) return Tile::kN32K2;
   if (gather && N <= 64 && K >= 512) {
     // (tiles of 256 pixels, many of them, up to 800: 338724 x 576 -> 57 36.3 / 30.2, 159048 x 784 -> 45 24.4 /
-    // 21.0, 467046 x 784 -> 34 60.8 / 47.5; 205379 x 864 -> 42 27.9 / 31.9)
+    // 21.0, 467046 x 784 -> 34 60.8 / 47.5; 205379 x 864 -> 42 27.9 / 31.9, though of eight drawn of 800 ... 1008 none
+    // is behind)
     if (K < 800 && tiles(256, 64) > 2 * cus) return Tile::kW64x2;
     if (tiles(128, 64) >= cus) return Tile::kR128K2;
     return K < 1024 ? Tile::kS64K2 : Tile::kS64K4;
@@ -175,7 +179,8 @@ inline Tile choose_tile(long M, long N, long K, long cus, bool gather = false,
   // 40.1, 321 x 7248 -> 5932, 141, 47.0 / 40.7, 7853 x 2832 -> 441, 248, 23.8 / 21.3, 2048 x 2048 -> 2048, 256, 14.8 /
   // 14.5, 4096 x 3072 -> 768, 192, 18.2 / 17.7, 4096 x 768 -> 768 7.7 / 8.3; the convolutions 5203 x 22400 -> 701, 246,
   // 111.7 / 106.6, 15884 x 3136 -> 204, 250, 22.5 / 22.2, 9522 x 2016 -> 380, 225, 17.9 / 17.2, but 12544 x 2304 -> 256, 196
-  // tiles without a ragged edge, 15.4 / 16.0).
+  // tiles without a ragged edge, 14.8 / 14.9, 12544 x 2880 -> 256 18.4 / 18.6; others of such widths would be ahead, 10192 x
+  // 3744 -> 384 26.9 / 23.3).
   if (!two_a_cu && t128 <= cus && K >= 1536 && !(gather && N % 128 == 0 && K < 4096))
     return Tile::kM128S3;
   if (t128 >= cus) {
@@ -186,8 +191,12 @@ inline Tile choose_tile(long M, long N, long K, long cus, bool gather = false,
     // and 550, 22.2 / 24.3)
     if (gather && tiles(128, 64) < 2 * cus) return Tile::kR128K2;
     // One round of 128 x 128 tiles, two to a CU (us, 256 x 128 on 128-byte stages, which hold a CU alone,
-    // and these: 16384 x 2048 -> 512 33.5 / 30.8, 28000 x 1024 -> 256 15.2 / 13.8, 2048 x 768 -> 4096 into int32
-    // 15.6 / 14.5; on 64-byte stages 8192 x 256 -> 1024 into int32 12.1 / 11.1).
+    // and these, into int32: 16384 x 2048 -> 512 33.5 / 30.8, 9464 x 1920 -> 715 31.2 / 26.2, 2048 x 768 -> 4096 15.6 /
+    // 14.5; on 64-byte stages 8192 x 256 -> 1024 12.1 / 11.1).  18 drawn layers are 1.09 times as fast into
+    // int32 (0.97 to 1.19).  Into int8 they are 1.05 times as fast while the former are 0.75 to 0.9 a CU (55 layers,
+    // 0.93 to 1.35; 8176 x 3376 -> 728 44.1 / 32.7) and 0.99 where those come out at nearly one (23, 0.91 to 1.13;
+    // 832 x 2704 -> 7890 29.1 / 33.4, 16384 x 1968 -> 512 23.9 / 25.5, but 8656 x 5392 -> 883 67.3 / 59.7).
+    // With a residual sum 8192 x 1024 -> 1024 16.1 / 16.7, 3136 x 512 -> 2048 12.0 / 11.0.
     // Very long reductions of gathered operands are ahead on the former (the convolutions 16000 x 6000 ->
     // 413 62.1 / 69.3, 7840 x 7600 -> 787 64.2 / 69.1, but 12544 x 4608 -> 512 38.7 / 37.8).
     if (t128 <= 2 * cus)

@@ -42,9 +42,11 @@ def test_fully_connected(capi, M, N, K):
                                              force=(cfg, splits, 0))["out32"].double(), want)
 
 
-# 128 x 128 tiles: 256 of them, a ragged 176, 133, and few enough of them to be shared by two ... five
+# 128 x 128 tiles: 256 of them, a ragged 176, 133; just below the lengths from which they are split (64 x 64 tiles
+# there, split once); and shared by two, three, five and six
 @pytest.mark.parametrize("M,N,K", [(2048, 2048, 1536), (2048, 2040, 1552), (1300, 1999, 1664), (2400, 833, 2064),
-                                   (699, 2429, 6160), (784, 1387, 6272), (1000, 470, 8208), (450, 1101, 12304)])
+                                   (699, 2429, 6160), (784, 1387, 6272), (1000, 470, 8208), (450, 1101, 12304),
+                                   (699, 2429, 8208), (784, 1387, 8208), (700, 900, 14352), (720, 799, 15696)])
 def test_fully_connected_of_larger_tiles(capi, M, N, K):
     d, w = operands((M, K), (N, K))
     same(lambda **kw: capi.quantized_fc(d, w, None, *ranges(), **kw), (44, 1, 0),

@@ -38,7 +38,9 @@ FULLY_CONNECTED = [(1024, 1520, 1024, (59, 1), (59, 1)), (1024, 1536, 1024, (33,
                    (121, 8208, 153, (71, 0), (71, 0)), (121, 32752, 153, (71, 0), (71, 0)),
                    (121, 32784, 153, (33, 12), (71, 0)),
                    (720, 14320, 799, (33, 1), (33, 1)), (720, 15680, 799, (34, 6), (33, 1)),
-                   (475, 29008, 1145, (34, 7), (33, 1)),
+                   (475, 29008, 1145, (34, 7), (33, 1)), (784, 8176, 1387, (59, 1), (59, 1)),
+                   (784, 8192, 1387, (34, 3), (59, 1)), (699, 8176, 2429, (59, 1), (59, 1)),
+                   (699, 8192, 2429, (34, 2), (59, 1)),
                    (2048, 1520, 2048, (53, 1), (53, 1)), (2048, 1536, 2048, (34, 1), (34, 1))]
 
 
