@@ -24,8 +24,8 @@
 // distinct bank groups without a permutation, for any channel count.
 //
 // What bounds it: instruction issue.  Vector instructions and MFMAs, which overlap little (the waves
-// of a work-group run in step from each barrier on), take 81 % of a CU's busy clocks in 56 x 56 x 64 and
-// 69 % in 28 x 28 x 128 and 14 x 14 x 256 (counters, batch 64); the sum alone is 7 vector instructions
+// of a work-group run in step from each barrier on), take 80 % of a CU's busy clocks in 56 x 56 x 64 and
+// 66 % in 28 x 28 x 128 and 14 x 14 x 256 (counters, batch 64); the sum alone is 7 vector instructions
 // per output of 64 ... 256 channels in the middle times four.  So what is not arithmetic has as few as
 // possible: a weight's place is a scalar offset and an immediate, the three taps of a row are immediates
 // where the channels are those of a kernel instance (KSB), the places of a tile's pixels in the tensors
@@ -612,8 +612,9 @@ __device__ __forceinline__ void block_tile(const BlockArgs& p, int tile, int fir
 
   // Rows of `chunks` pieces, `pitch` apart in LDS, to their pixels.  No streaming stores: the
   // next block reads both outputs, and what it finds in the memory-side cache it does not fetch from
-  // memory (quantized ResNet-50 at batch 64, all blocks with streaming stores / plain ones / written
-  // through: 573 / 544 / 534 us; plain ones leave up to 32 MB of dirty lines to the launch's end).
+  // memory (quantized ResNet-50 at batch 64, all blocks with streaming stores 5 % behind plain ones;
+  // written through, kDeviceScope, a block is 1.5 to 2.3 us ahead of those, which leave up to 32 MB of
+  // dirty lines to the launch's end).
   auto leave = [&](int at, int chunks, int pitch, uint32_t magic, int rows, int rest,
                    const uint32_t* pixel_of, int8_t* out) MXQ_INLINE {
     const auto to = __builtin_amdgcn_make_buffer_rsrc(

@@ -939,7 +939,8 @@ typedef GemmCfg<256, 32, 128, 4, 1> CfgWindow2;
 // 12.2 / 12.7 / 11.1, but into int32 20631 -> 393, 7 x 7, 2106, 26.1 / 24.0 / 27.1, 242064 -> 86, 5 x 5, 5676, 35.7 /
 // 43.6 / 46.6), and under smaller ones to one (4800 -> 108, 3 x 3, 152, 5.1 / 4.8, but 52983 -> 37, 3 x 3, 828, 7.3 /
 // 7.8 / 7.3).  Strided windows read every second piece of LDS and pay from 49 taps on (7605 -> 88, 7 x 7 by 2,
-// 9.4 / 7.6, but 25281 -> 37, 5 x 5 by 2 into int32, 7.4 / 8.2).
+// 9.4 / 7.6, but 25281 -> 37, 5 x 5 by 2 into int32, 7.4 / 8.2).  Where the rows under 256 pixels find no room,
+// 128 pixels are not tried, though theirs may (11 images of 40 x 236 -> 20, 7 x 7, 16.6 / 14.4).
 int window_cfg(const ConvArgs& a) {
   const int taps = a.KH * a.KW;
   if (a.C != 16 || taps < 9 || (a.sh * a.sw != 1 && taps < 49)) return 0;

@@ -739,8 +739,8 @@ typedef PlaneCfg<64, 128, 128, 2, 2> PlaneP64k2;
 // them (51 drawn layers 0.997, 0.94 to 1.06) and stay on two.
 // 128 x 64 tiles take three, whatever the grid: up to one a CU the operands from memory 1.00 to 1.05 times as fast
 // at three to five steps, 1.1 at eight, 1.2 from sixteen on (16 images, 1536 -> 20 at 12 x 12, 13.0 / 10.8), past
-// that level to 6 % behind alone (256 -> 64 at 56 x 56 22.2 / 23.0), that layer behind others 23.4 / 21.6 /
-// 24.4.  Operands of less than the L2, read again and again, are the exception: 5 % behind at three steps, 22 at 28.
+// that level to 6 % behind alone (256 -> 64 at 56 x 56 22.2 / 23.0), but that layer's pass with 18 others behind
+// requantize and relu is 1.3 us of 727 ahead.  Operands of less than the L2, read again and again, are the exception: 5 % behind at three steps, 22 at 28.
 template <class Cfg>
 int plane_stages(int steps, long long groups) {
   if (steps < 3 || Cfg::BO != 64 || Cfg::BK != 64) return 2;

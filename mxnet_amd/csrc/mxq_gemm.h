@@ -118,11 +118,12 @@ constexpr int kEpiStreamRows = 8192;
 inline int epi_stream_rows(long long rows) { return rows >= kEpiStreamRows ? 1 : 0; }
 
 // The cache policy of int8 tiles that are not streamed: sc1, written through the XCD's L2.  A plain
-// store leaves a dirty line there, and a launch ends when the last of them is written back: a
-// quantized ResNet-50 at batch 64, whose blocks, pairs and last stage write 800 MB like that, 544 us with
-// plain stores and 523 so (the blocks alone 534), 40 images of 200 x 200 through 48 ... 192 channels
-// 226.6 and 219.6, one image level; the 19 layers on operands of their own 237.9 and 235.5.  (Int32
-// planes stay plain: the same layers behind NCHW operators 730 us, written through 754.)
+// store leaves a dirty line there, and a launch ends when the last of them is written back: passes of a
+// quantized ResNet-50 at batch 64, whose blocks, pairs and last stage write 570 MB like that, 577 us with
+// plain stores and 558 so (its 29 kernels, traced, 612 and 572: 1.5 to 3.7 us each of the larger ones, the same
+// bytes), 40 images of 200 x 200 through 48 ... 192 channels 226.6 and 219.6, one image and the 19 layers on
+// operands of their own level (195.0 / 194.5, 264.2 / 264.8).  (Int32 planes stay plain: the same layers behind
+// NCHW operators 730 us, written through 754.)
 constexpr int kDeviceScope = 16;  // sc1 in the buffer instructions' cache policy
 
 // 16 bytes of the int8 output tile.  The flavour is a compile-time parameter and callers
