@@ -36,7 +36,7 @@ namespace mxq {
 //   71      the few-tiles kernel (any shape; here `splits` is the number of waves per
 //           32 x 32 tile, negative for 16 x 16 tiles)
 // plan_fc proposes 1, 3, 4, 12, 31, 33, 34, 41, 43, 44, 51, 53, 57..62 and 71, and 55 for a residual sum;
-// the others are there for who pins them.
+// the others are built with the test entries alone, for the tests that pin them.
 // Output tile of a direct-to-LDS configuration (what a split-K work-group leaves in the
 // workspace); false for every other configuration.
 bool fc_cfg_tile(int cfg, int& bm, int& bn) {

@@ -405,27 +405,15 @@ void fc_launch_mode(hipStream_t s, const FcArgs& a, const FcLaunch& how, const W
   }
   switch (cfg) {
     case 1: launch_cfg<CfgL8, MODE>(s, a, how.aligned); break;
-    case 2: launch_cfg<CfgL4, MODE>(s, a, how.aligned); break;
     case 3: launch_cfg<CfgM, MODE>(s, a, how.aligned); break;
     case 4: launch_cfg<CfgS, MODE>(s, a, how.aligned); break;
-    case 11: launch_dma<CfgL8, 4, 0, false, MODE>(s, a, sp, ws); break;
     case 12: launch_dma<CfgL8, 4, 2, false, MODE>(s, a, sp, ws); break;
-    case 14: launch_dma<CfgL4, 4, 0, false, MODE>(s, a, sp, ws); break;
-    case 16: launch_dma<CfgL4, 4, 2, false, MODE>(s, a, sp, ws); break;
-    case 21: launch_dma<CfgW128, 4, 2, true, MODE>(s, a, sp, ws); break;
-    case 22: launch_dma<CfgW64, 4, 2, true, MODE>(s, a, sp, ws); break;
-    case 23: launch_dma<CfgM, 4, 2, true, MODE>(s, a, sp, ws); break;
-    case 24: launch_dma<CfgS, 4, 2, true, MODE>(s, a, sp, ws); break;
     case 41: launch_dma<CfgW128, 2, 0, true, MODE>(s, a, sp, ws); break;
-    case 42: launch_dma<CfgW64, 2, 0, true, MODE>(s, a, sp, ws); break;
     case 43: launch_dma<CfgM, 2, 0, true, MODE>(s, a, sp, ws); break;
     case 44: launch_dma<CfgS, 2, 0, true, MODE>(s, a, sp, ws); break;
     case 51: launch_dma<CfgSK, 2, 0, true, MODE>(s, a, sp, ws); break;
-    case 52: launch_dma<CfgSK, 3, 0, true, MODE>(s, a, sp, ws); break;
     case 53: launch_dma<CfgMK, 2, 0, true, MODE>(s, a, sp, ws); break;
-    case 54: launch_dma<CfgMK, 3, 0, true, MODE>(s, a, sp, ws); break;
     case 55: launch_dma<CfgL8K, 2, 0, true, MODE>(s, a, sp, ws); break;
-    case 56: launch_dma<CfgW128K, 2, 0, true, MODE>(s, a, sp, ws); break;
     case 57: launch_dma<CfgRK, 2, 0, true, MODE>(s, a, sp, ws); break;
     case 58: launch_dma<CfgQK, 2, 0, true, MODE>(s, a, sp, ws); break;
     case 59: launch_dma<CfgSK2, 2, 0, true, MODE>(s, a, sp, ws); break;
@@ -433,7 +421,21 @@ void fc_launch_mode(hipStream_t s, const FcArgs& a, const FcLaunch& how, const W
     case 33: launch_sliced<SlicedCfg<64, 64, 256>, 4, MODE>(s, a, sp, ws); break;
     case 34: launch_sliced<SlicedCfg<128, 128, 128>, 3, MODE>(s, a, sp, ws); break;
     case 31: launch_dma<CfgL8, 4, 2, true, MODE>(s, a, sp, ws); break;
+#ifdef MXQ_TEST_HOOKS  // nothing proposes these
+    case 2: launch_cfg<CfgL4, MODE>(s, a, how.aligned); break;
+    case 11: launch_dma<CfgL8, 4, 0, false, MODE>(s, a, sp, ws); break;
+    case 14: launch_dma<CfgL4, 4, 0, false, MODE>(s, a, sp, ws); break;
+    case 16: launch_dma<CfgL4, 4, 2, false, MODE>(s, a, sp, ws); break;
+    case 21: launch_dma<CfgW128, 4, 2, true, MODE>(s, a, sp, ws); break;
+    case 22: launch_dma<CfgW64, 4, 2, true, MODE>(s, a, sp, ws); break;
+    case 23: launch_dma<CfgM, 4, 2, true, MODE>(s, a, sp, ws); break;
+    case 24: launch_dma<CfgS, 4, 2, true, MODE>(s, a, sp, ws); break;
+    case 42: launch_dma<CfgW64, 2, 0, true, MODE>(s, a, sp, ws); break;
+    case 52: launch_dma<CfgSK, 3, 0, true, MODE>(s, a, sp, ws); break;
+    case 54: launch_dma<CfgMK, 3, 0, true, MODE>(s, a, sp, ws); break;
+    case 56: launch_dma<CfgW128K, 2, 0, true, MODE>(s, a, sp, ws); break;
     case 32: launch_dma<CfgL4, 4, 2, true, MODE>(s, a, sp, ws); break;
+#endif
     default: MXQ_CHECK(false, "unknown fc tile configuration " << cfg);
   }
 }
